@@ -25,6 +25,7 @@ SOURCES = [
     "ffi_plan.hip",
     "ffi_util.hip",
     "ffi_wide.hip",
+    "ffi_sliced.hip",
     "ffi_bf16.hip",
     "ffi_loss.hip",
     "ffi_sparse_grad.hip",

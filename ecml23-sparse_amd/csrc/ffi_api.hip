@@ -617,6 +617,7 @@ int ffi_set_option(const char* name, int value) {
         {"plan_weights_in_lds", &ffi::Options::plan_weights_in_lds, -1, 1},
         {"workgroups_per_cu", &ffi::Options::workgroups_per_cu, 0, 16},
         {"plan_sorted_columns", &ffi::Options::plan_sorted_columns, -1, 1},
+        {"wide_ranges", &ffi::Options::wide_ranges, 0, 4},
     };
     for (const auto& t : table) {
         if (std::strcmp(name, t.name) != 0) continue;

@@ -30,6 +30,7 @@ struct Options {
     int fwd_lane64 = 0;             // -1: never the 64-sample forward kernel
     int plan_weights_in_lds = 0;    // -1: never / 1: whenever the tile fits
     int workgroups_per_cu = 0;      // upper limit for the kernel that walks a tiled plan
+    int wide_ranges = 0;            // column ranges of the sliced forward kernel
     int plan_sorted_columns = 0;    // -1: never / 1: always (in the weights-in-LDS form) the plans that hand the columns to the walking kernel's threads tile by tile, by length
 };
 extern Options g_options;
@@ -65,7 +66,7 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 void workspace_clear(int device);
 size_t workspace_bytes(int device);

@@ -27,92 +27,6 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// ---- forward ------------------------------------------------------------------------------------
-// grid (label blocks, batch passes).  A wavefront walks 16 labels one after the other; per
-// connection it loads one 512-byte piece of row idx[j,k] of xT and does two multiply-adds per lane.
-// Results go through LDS so that out is written in 256-byte rows.
-// TWO == false (batch <= 64): lanes own one batch entry each, the loads and multiply-adds of the second half are left out.
-template <bool TWO>
-__global__ __launch_bounds__(kWideThreads) void fwd_wide_kernel(const float* __restrict__ xT,
-                                                                const int32_t* __restrict__ idx,
-                                                                const float* __restrict__ w,
-                                                                const float* __restrict__ bias, float* __restrict__ out,
-                                                                int B, int N, int L, int K, int ldb) {
-    __shared__ float tile[kWideLabels * kWideStride];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int j0 = blockIdx.x * kWideLabels;
-    const int bc0 = blockIdx.y * kWideBatch;
-    const buffer_rsrc xr = make_rsrc(xT, (size_t)N * (size_t)ldb * sizeof(float));
-    const unsigned lane_off0 = (unsigned)(bc0 + lane) * 4u, lane_off1 = lane_off0 + 256u;
-    const unsigned row_bytes = (unsigned)ldb * 4u;
-    for (int q = 0; q < kWideLabels / 4; ++q) {
-        const int jl = wave * (kWideLabels / 4) + q;
-        const int j = j0 + jl;
-        float acc0 = 0.f, acc1 = 0.f;
-        if (j < L) {                                            // wave-uniform
-            const int32_t* irow = idx + (size_t)j * K;
-            const float* wrow = w + (size_t)j * K;
-            for (int k0 = 0; k0 < K; k0 += 64) {
-                const int kn = min(64, K - k0);
-                // one connection per lane, handed out below as wave-uniform scalars
-                const unsigned iv = (lane < kn) ? (unsigned)irow[k0 + lane] : 0u;
-                const float wv = (lane < kn) ? wrow[k0 + lane] : 0.f;
-                int k = 0;
-                for (; k + kWideInflight <= kn; k += kWideInflight) {
-                    float x0[kWideInflight], x1[kWideInflight], ws[kWideInflight];
-#pragma unroll
-                    for (int u = 0; u < kWideInflight; ++u) {
-                        const unsigned n = (unsigned)__builtin_amdgcn_readlane((int)iv, k + u);
-                        ws[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wv), k + u));
-                        x0[u] = buffer_load_f32(xr, lane_off0, n * row_bytes);
-                        x1[u] = TWO ? buffer_load_f32(xr, lane_off1, n * row_bytes) : 0.f;
-                    }
-#pragma unroll
-                    for (int u = 0; u < kWideInflight; ++u) {
-                        acc0 = fmaf(ws[u], x0[u], acc0);
-                        if (TWO) acc1 = fmaf(ws[u], x1[u], acc1);
-                    }
-                }
-                if (k < kn) {
-                    // the last, partly filled group, its gathers in flight together like the others: connections behind
-                    // the end repeat the last one and are left out of the sum (one gather at a time cost 40 % at fan-in 12)
-                    float x0[kWideInflight], x1[kWideInflight], ws[kWideInflight];
-#pragma unroll
-                    for (int u = 0; u < kWideInflight; ++u) {
-                        const int kk = min(k + u, kn - 1);
-                        const unsigned n = (unsigned)__builtin_amdgcn_readlane((int)iv, kk);
-                        const float wk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wv), kk));
-                        ws[u] = wk;
-                        x0[u] = buffer_load_f32(xr, lane_off0, n * row_bytes);
-                        x1[u] = TWO ? buffer_load_f32(xr, lane_off1, n * row_bytes) : 0.f;
-                    }
-#pragma unroll
-                    for (int u = 0; u < kWideInflight; ++u) {
-                        if (k + u < kn) {                       // wave-uniform
-                            acc0 = fmaf(ws[u], x0[u], acc0);
-                            if (TWO) acc1 = fmaf(ws[u], x1[u], acc1);
-                        }
-                    }
-                }
-            }
-        }
-        tile[jl * kWideStride + lane] = acc0;
-        tile[jl * kWideStride + 64 + lane] = acc1;
-    }
-    __syncthreads();
-    // out[b, j0 .. j0+63]: one wavefront writes one 256-byte row per step
-    const int jl = threadIdx.x & 63;
-    if (j0 + jl < L) {
-        const bool has_bias = bias != nullptr;
-        const float bj = has_bias ? bias[j0 + jl] : 0.f;
-        for (int bb = threadIdx.x >> 6; bb < (TWO ? kWideBatch : kWideBatch / 2); bb += kWideThreads / 64) {
-            const int b = bc0 + bb;
-            const float v = tile[jl * kWideStride + bb];
-            if (b < B) out[(size_t)b * L + j0 + jl] = has_bias ? v + bj : v;
-        }
-    }
-}
-
 // ---- weight gradient ----------------------------------------------------------------------------
 // grid (label blocks).  Per batch pass the workgroup brings g[b, j0..j0+63] into LDS (coalesced
 // along labels), then every wavefront handles 16 labels: per connection one 512-byte piece of the
@@ -320,20 +234,6 @@ int wide_features(const float* x, const Dims& d, hipStream_t s, const float** xT
 }
 
 }  // namespace
-
-int launch_forward_wide(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
-                        hipStream_t s) {
-    if (!wide_offsets_fit(d.N, d.B)) return FFI_ERR_TOO_LARGE;
-    const float* xT = nullptr;
-    int ldb = 0;
-    FFI_TRY(wide_features(x, d, s, &xT, &ldb));
-    dim3 grid((d.L + kWideLabels - 1) / kWideLabels, (d.B + kWideBatch - 1) / kWideBatch);
-    if (grid.y > 65535u) return FFI_ERR_TOO_LARGE;
-    if (d.B > 64) hipLaunchKernelGGL(fwd_wide_kernel<true>, grid, dim3(kWideThreads), 0, s, xT, idx, w, bias, out, d.B, d.N, d.L, d.K, ldb);
-    else hipLaunchKernelGGL(fwd_wide_kernel<false>, grid, dim3(kWideThreads), 0, s, xT, idx, w, bias, out, d.B, d.N, d.L, d.K, ldb);
-    FFI_HIP_TRY(hipGetLastError());
-    return FFI_OK;
-}
 
 int launch_weight_grad_wide(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
                             hipStream_t s) {

@@ -1,0 +1,44 @@
+"""Inputs whose tile does not fit in LDS (more than 1,216 columns): the kernels that gather from sample-sliced tables, at
+the sizes where they change form, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from conftest import load_package, reference_law_inputs, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ffi():
+    return load_package()
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# (B, N, L, K): slices of 4, 8, 16 and 32 samples and their edges; several slices per list and one; label blocks and
+# chunks of connections with remainders; rows on and off 16-byte boundaries
+FORWARD_SHAPES = [(1, 1217, 300, 1), (4, 2000, 257, 16), (5, 1217, 129, 17), (8, 3000, 128, 40), (9, 1300, 65, 33), (16, 2500, 130, 64),
+                  (17, 4000, 63, 3), (33, 1300, 64, 72), (100, 40_000, 200, 65), (130, 1500, 97, 130), (64, 70_000, 150, 36)]
+
+
+@pytest.mark.parametrize("ranges", [0, 1, 2, 3, 4])
+def test_forward_of_wide_inputs(ffi, ranges):
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_ranges", ranges) == 0
+    try:
+        for B, N, L, K in FORWARD_SHAPES:
+            x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + N)
+            ref = oracle.forward(x, lookup, w, transposed=False)
+            bias = np.linspace(-1, 1, L).astype(np.float32)
+            for tp in (False, True):
+                dx = dev(x.T if tp else x)
+                fwd = ffi.fan_in_sparse_matmul_tp if tp else ffi.fan_in_sparse_matmul
+                assert rel_err(fwd(dx, dev(lookup), dev(w)).cpu().numpy(), ref) <= 1e-5, (B, N, L, K, tp)
+            out = ffi.fan_in_sparse_matmul_bias(dev(x), dev(lookup), dev(w), dev(bias)).cpu().numpy()
+            assert rel_err(out, ref + bias) <= 1e-5, (B, N, L, K)
+    finally:
+        lib.ffi_set_option(b"wide_ranges", 0)
