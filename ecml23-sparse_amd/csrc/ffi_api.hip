@@ -2,6 +2,7 @@
 // No arithmetic lives here.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
+#include "ffi_sliced.h"
 
 #include <algorithm>
 #include <climits>
@@ -138,10 +139,17 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     ffi_plan* p = find_cached_plan(lookup, d, dev);
+    bool zeroed = false;
+    auto passes = [&](const unsigned long long* verdict) -> int {
+        // (the global form's walk has both operands of a connection at hand: one walk for both gradients)
+        if (!p->tiled && wg.features != nullptr)
+            return launch_backward_wide(p, wg.features, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d.B, d.tp, s);
+        FFI_TRY(between(p));
+        return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, verdict, &zeroed);
+    };
     if (!p) {
         FFI_TRY(create_cached_plan(lookup, d, dev, s, &p));
-        FFI_TRY(between(p));
-        return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s);
+        return passes(nullptr);
     }
     bool seen = false, current = true;
     unsigned long long bad = 0;
@@ -151,13 +159,10 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         // the build fingerprints the present content, so this call needs no check
         const int st = plan_build(p, lookup, s);
         if (st != FFI_OK) { drop_cached_plan(p); return st; }
-        FFI_TRY(between(p));
-        return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s);
+        return passes(nullptr);
     }
     FFI_TRY(plan_guard_enqueue(p, lookup, s));
-    FFI_TRY(between(p));
-    bool zeroed = false;
-    FFI_TRY(launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, p->d_guard + kGuardVerdict, &zeroed));
+    FFI_TRY(passes(p->d_guard + kGuardVerdict));
     return launch_backward_if_outdated(p->d_guard + kGuardVerdict, wg.features, lookup, weights, out_grad, feature_grad,
                                        wg.weight_grad, wg.bias_grad, d, s, zeroed);
 }
@@ -647,11 +652,11 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
     if (check_dims(batch, num_features, num_units, fan_in, transposed, &d) != FFI_OK) return 0;
     const size_t B = (size_t)d.B, N = (size_t)d.N, L = (size_t)d.L, K = (size_t)d.K;
     const bool narrow = tile_path_fits(d.N) && d.L < (1 << 25);
-    const size_t ldw = (B + 31) / 32 * 32;                         // row stride of the wide kernels' own copies
+    const size_t slice = 4 * (size_t)slice_lanes(d.B, 4), slice_pad = (B + slice - 1) / slice * slice;      // samples of the sliced copies
     // the batch-major copy of the features (one slot, shared by the passes and by the permuted weights below)
     size_t features_slot = 0;
     if (narrow) features_slot = d.tp ? 0 : N * B * 4;
-    else features_slot = (d.tp && ldw == B) ? 0 : N * ldw * 4;
+    else features_slot = N * slice_pad * 4;
     size_t total = 0, partial_slot = 0;
     if (passes & FFI_PASS_BACKWARD) {
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;
@@ -683,10 +688,15 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
             }
             if (tile_path_fits(d.N) && d.N < (1 << kArrIdBits)) total += arranged_words((long long)(L * ((K + 31) / 32))) * 2;   // idx16
         } else {
-            const size_t nblocks = (L + 65535) / 65536;
-            total += L * K * 4 + (nblocks * N + 1) * 4;                                 // perm, col_ptr
-            partial_slot = L * ldw * 4;                                                 // out_grad, batch-major
-            if (!d.tp) features_slot = std::max(features_slot, N * B * 4);
+            const size_t labels = (size_t)plan_block_labels(d.N, d.K, d.L), nblocks = (L + labels - 1) / labels, lists = nblocks * N;
+            const double mu = (double)L * (double)K / (double)lists;                    // connections per list, Poisson-like
+            const size_t slots = (size_t)((double)lists * (mu + 3.5 * (1.0 - std::exp(-mu)) + std::max(0.0, 4.0 - mu) * (1.0 - std::exp(-mu))));
+            int gl, slices, m, streams, per_stream;
+            walk_shape(d.N, d.B, d.L, (int)nblocks, &gl, &slices, &m, &streams, &per_stream);
+            total += slots * 6 + (lists + 1) * 4;                                       // slot_pos, slot_lab, oct_ptr
+            total += slots * 4 * (1 + (size_t)slices);                                  // weights and weight gradients in slot order
+            partial_slot = (L + N * (size_t)streams) * slice_pad * 4;                   // out_grad in slices, sums per stream
+            features_slot = std::max(features_slot, N * slice_pad * 4);
         }
     }
     return total + features_slot + partial_slot;

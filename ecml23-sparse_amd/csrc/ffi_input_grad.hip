@@ -625,8 +625,7 @@ int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* 
         }
         return FFI_OK;
     }
-    if (!p->perm || !p->col_ptr) return FFI_ERR_BAD_ARGUMENT;
-    return launch_input_grad_wide(p, w, g, gx, B, tp, s);
+    return launch_backward_wide(p, nullptr, w, g, gx, nullptr, nullptr, B, tp, s);
 }
 
 }  // namespace ffi

@@ -66,7 +66,7 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 void workspace_clear(int device);
 size_t workspace_bytes(int device);
@@ -207,9 +207,10 @@ int launch_rewire(int32_t* lookup, const float* w, float* const* arrays, int n_a
 // padding slots: a fixed order, but not the ascending-position order in which the reference's CPU
 // kernel accumulates (tfsparse/cc/kernels/backward.cpp:64-72).
 //
-// tiled == false (any shape): a CSC per block of `block_labels` labels.  perm[e] = flat position of
-// the e-th connection in (label block, column, position) order;
-// col_ptr[blk*N + n] .. col_ptr[blk*N + n + 1] are the connections of column n inside block blk.
+// tiled == false (any shape): the connections grouped by (block of `block_labels` labels, column), positions ascending, every
+// list padded to whole octs of slots: list blk * N + n is octs oct_ptr[blk * N + n] .. oct_ptr[blk * N + n + 1] - 1.
+// slot_pos = flat position of the slot's connection (-1: padding), slot_lab = its label inside the block (kNoLabel: padding),
+// pos_slot = slot_pos the other way round.
 struct ffi_plan {
     int device = -1;
     int L = 0, K = 0, N = 0;
@@ -240,10 +241,13 @@ struct ffi_plan {
     // quarter by quarter (ffi::arranged_quarter_offset), so that the 64 lanes of a wavefront load 1 KB in one piece
     unsigned short* idx16 = nullptr;
     // blocked global form
-    int block_labels = 0;     // labels per block (bounds the part of out_grad that is live at a time)
+    int block_labels = 0;     // labels per block (<= 65535: bounds the part of out_grad that is live at a time)
     int nblocks = 0;
-    int32_t* perm = nullptr;
-    int32_t* col_ptr = nullptr;
+    long long slots = 0;
+    unsigned* oct_ptr = nullptr;         // [nblocks * N + 1]
+    int32_t* slot_pos = nullptr;
+    unsigned short* slot_lab = nullptr;
+    unsigned* pos_slot = nullptr;        // [L * K] slot of each flat position
     unsigned long long* d_scratch = nullptr;  // counters of the build, fingerprint partial sums (device)
     unsigned long long* h_scratch = nullptr;  // pinned mirror
     hipEvent_t fp_done = nullptr;             // recorded behind the fingerprint kernel and its copy to h_scratch
@@ -277,6 +281,7 @@ struct ffi_plan {
 };
 
 namespace ffi {
+constexpr unsigned short kNoLabel = 0xffff;  // slot_lab of a padding slot
 constexpr int kPlanTileLabels = 1024;     // a [1024+1][32] fp32 tile fits LDS
 constexpr unsigned kPadPos = 0xffffu;      // pos16 of a padding slot; real positions are below it (tile_labels * K <= 0xffff)
 // LDS of the kernel that walks the tiled form: the tile's rows of out_grad (per bank half: half the tile plus some room
@@ -326,6 +331,7 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
+int plan_block_labels(int N, int K, int L);
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s);
 // Content fingerprint of `lookup` (and the count of ids outside [0,N)).  _begin enqueues the kernel
 // on `s` and returns; _end waits for that kernel only, not for what the caller enqueued on `s`
@@ -358,7 +364,10 @@ int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* 
 bool input_grad_unplanned_fits(int N, int K);
 int launch_input_grad_unplanned(const unsigned long long* verdict, const int32_t* idx, const float* w, const float* g, float* gx,
                                 const Dims& d, hipStream_t s);
-int launch_input_grad_wide(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp, hipStream_t s);
+// Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.
+void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, int* streams, int* blocks_per_stream);
+int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
+                         bool tp, hipStream_t s);
 }  // namespace ffi
 
 #endif  // FFI_INTERNAL_H

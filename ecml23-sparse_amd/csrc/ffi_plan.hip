@@ -11,6 +11,7 @@
 #include <functional>
 
 #include <rocprim/device/device_radix_sort.hpp>
+#include <rocprim/device/device_scan.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
 
 namespace ffi {
@@ -679,7 +680,7 @@ void free_arrays(ffi_plan* p, bool keep = false) {
     }
     p->owned.clear();
     p->rowpos = nullptr;
-    p->perm = nullptr; p->col_ptr = nullptr; p->slice_off = nullptr; p->lab16 = nullptr; p->pos16 = nullptr; p->slot32 = nullptr; p->idx16 = nullptr; p->colperm = nullptr;
+    p->oct_ptr = nullptr; p->slot_pos = nullptr; p->slot_lab = nullptr; p->pos_slot = nullptr; p->slots = 0; p->slice_off = nullptr; p->lab16 = nullptr; p->pos16 = nullptr; p->slot32 = nullptr; p->idx16 = nullptr; p->colperm = nullptr;
     p->tiled = false; p->w_in_lds = false; p->total_rows = 0; p->bytes = 0;
 }
 
@@ -726,6 +727,15 @@ void dev_release(ffi_plan* p, void* ptr) {
 }
 
 }  // namespace
+
+// Labels per block of the global form: the block's rows of one slice of out_grad (128 bytes each) take five eighths of an
+// XCD's L2 -- shared by as many blocks as the workgroups of that many columns leave room for at a time -- unless the
+// lists of a block's columns would then hold fewer than eight connections.
+int plan_block_labels(int N, int K, int L) {
+    const double resident = 20480.0 * std::min(1.0, (double)N / 4096.0), filled = 8.0 * (double)N / (double)K;
+    const int labels = (int)std::min(65535.0, std::max(1024.0, std::max(resident, filled)));
+    return std::min(labels, L);
+}
 
 // Labels per tile of the tiled form, and whether the walking kernel keeps the tile's weights in LDS (then the tiles
 // are smaller).
@@ -902,49 +912,90 @@ __global__ __launch_bounds__(kBlock) void block_key_kernel(const int32_t* __rest
     key[p] = (unsigned)(j / block_labels) * (unsigned)N + (unsigned)idx[p];
 }
 
-constexpr int kPlanBlockLabels = 65536;
+// octs[n] = octs of slots that list n takes; the last entry (a list of its own behind the lists) is 0
+__global__ __launch_bounds__(kBlock) void oct_count_kernel(const int32_t* __restrict__ ptr, int nkeys, unsigned* __restrict__ octs) {
+    const int n = blockIdx.x * kBlock + threadIdx.x;
+    if (n > nkeys) return;
+    octs[n] = n < nkeys ? (unsigned)(ptr[n + 1] - ptr[n] + 7) / 8u : 0u;
+}
+
+__global__ __launch_bounds__(kBlock) void slot_clear_kernel(int32_t* __restrict__ slot_pos, unsigned short* __restrict__ slot_lab, size_t slots) {
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= slots) return;
+    slot_pos[i] = -1;
+    slot_lab[i] = kNoLabel;
+}
+
+__global__ __launch_bounds__(kBlock) void slot_fill_kernel(const unsigned* __restrict__ sorted_keys, const int32_t* __restrict__ sorted_pos,
+                                                           const int32_t* __restrict__ ptr, const unsigned* __restrict__ oct_ptr, int total,
+                                                           int K, int N, int block_labels, int32_t* __restrict__ slot_pos,
+                                                           unsigned short* __restrict__ slot_lab, unsigned* __restrict__ pos_slot) {
+    const int e = blockIdx.x * kBlock + threadIdx.x;
+    if (e >= total) return;
+    const unsigned key = sorted_keys[e];
+    const size_t slot = (size_t)oct_ptr[key] * 8 + (size_t)(e - ptr[key]);
+    const int pos = sorted_pos[e];
+    slot_pos[slot] = pos;
+    pos_slot[pos] = (unsigned)slot;
+    slot_lab[slot] = (unsigned short)(pos / K - (int)(key / (unsigned)N) * block_labels);
+}
 
 int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     const int total = p->L * p->K;  // validated to fit int32 by the caller
-    const int nblocks = (p->L + kPlanBlockLabels - 1) / kPlanBlockLabels;
+    const int block_labels = plan_block_labels(p->N, p->K, p->L);
+    const int nblocks = (p->L + block_labels - 1) / block_labels;
     const long long nkeys = (long long)nblocks * p->N;
-    if (nkeys >= (1ll << 31)) return FFI_ERR_TOO_LARGE;
-    if (!dev_alloc(p, &p->perm, (size_t)total) || !dev_alloc(p, &p->col_ptr, (size_t)nkeys + 1)) return FFI_ERR_OUT_OF_MEMORY;
-    unsigned* keys = nullptr;
-    unsigned* sorted_keys = nullptr;
+    if (nkeys >= (1ll << 31) - 1) return FFI_ERR_TOO_LARGE;
+    if (!dev_alloc(p, &p->oct_ptr, (size_t)nkeys + 1)) return FFI_ERR_OUT_OF_MEMORY;
+    unsigned *keys = nullptr, *sorted_keys = nullptr, *octs = nullptr;
+    int32_t *sorted_pos = nullptr, *ptr = nullptr;
     void* temp = nullptr;
-    size_t temp_bytes = 0;
+    size_t temp_bytes = 0, scan_bytes = 0;
     const int end_bit = bits_for((unsigned)(nkeys - 1));
     rocprim::counting_iterator<int32_t> positions(0);
     auto cleanup = [&]() {
-        if (keys) (void)hipFree(keys);
-        if (sorted_keys) (void)hipFree(sorted_keys);
-        if (temp) (void)hipFree(temp);
+        for (void* q : {(void*)keys, (void*)sorted_keys, (void*)octs, (void*)sorted_pos, (void*)ptr, temp})
+            if (q) (void)hipFree(q);
     };
     // stable LSD radix sort of ((block, column), flat position): positions stay ascending inside a column
-    hipError_t e = rocprim::radix_sort_pairs(nullptr, temp_bytes, keys, sorted_keys, positions, p->perm, (unsigned)total, 0,
-                                             end_bit, s);
+    hipError_t e = rocprim::radix_sort_pairs(nullptr, temp_bytes, keys, sorted_keys, positions, sorted_pos, (unsigned)total, 0, end_bit, s);
+    if (e == hipSuccess) e = rocprim::exclusive_scan(nullptr, scan_bytes, octs, p->oct_ptr, 0u, (size_t)nkeys + 1, rocprim::plus<unsigned>(), s);
     if (e != hipSuccess) return hip_fail(e);
+    temp_bytes = std::max<size_t>(std::max(temp_bytes, scan_bytes), 4);
     if (hipMalloc(&keys, (size_t)total * sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&sorted_keys, (size_t)total * sizeof(unsigned)) != hipSuccess ||
-        hipMalloc(&temp, temp_bytes ? temp_bytes : 4) != hipSuccess) {
+        hipMalloc(&sorted_pos, (size_t)total * sizeof(int32_t)) != hipSuccess ||
+        hipMalloc(&ptr, ((size_t)nkeys + 1) * sizeof(int32_t)) != hipSuccess ||
+        hipMalloc(&octs, ((size_t)nkeys + 1) * sizeof(unsigned)) != hipSuccess || hipMalloc(&temp, temp_bytes) != hipSuccess) {
         (void)hipGetLastError();
         cleanup();
         return FFI_ERR_OUT_OF_MEMORY;
     }
-    hipLaunchKernelGGL(block_key_kernel, dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, s, lookup, total, p->K, p->N,
-                       kPlanBlockLabels, keys);
-    e = rocprim::radix_sort_pairs(temp, temp_bytes, keys, sorted_keys, positions, p->perm, (unsigned)total, 0, end_bit, s);
+    auto grid = [](size_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); };
+    hipLaunchKernelGGL(block_key_kernel, grid((size_t)total), dim3(kBlock), 0, s, lookup, total, p->K, p->N, block_labels, keys);
+    e = rocprim::radix_sort_pairs(temp, temp_bytes, keys, sorted_keys, positions, sorted_pos, (unsigned)total, 0, end_bit, s);
     if (e != hipSuccess) { cleanup(); return hip_fail(e); }
-    hipLaunchKernelGGL(col_ptr_kernel, dim3((unsigned)((nkeys + 1 + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, sorted_keys,
-                       total, (int)nkeys, p->col_ptr);
+    hipLaunchKernelGGL(col_ptr_kernel, grid((size_t)nkeys + 1), dim3(kBlock), 0, s, sorted_keys, total, (int)nkeys, ptr);
+    hipLaunchKernelGGL(oct_count_kernel, grid((size_t)nkeys + 1), dim3(kBlock), 0, s, ptr, (int)nkeys, octs);
+    e = rocprim::exclusive_scan(temp, temp_bytes, octs, p->oct_ptr, 0u, (size_t)nkeys + 1, rocprim::plus<unsigned>(), s);
+    unsigned total_octs = 0;
+    if (e == hipSuccess) e = hipMemcpyAsync(&total_octs, p->oct_ptr + nkeys, sizeof(unsigned), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) { cleanup(); return hip_fail(e); }
+    const size_t slots = (size_t)total_octs * 8;
+    if (slots >= (1ull << 32)) { cleanup(); return FFI_ERR_TOO_LARGE; }
+    if (!dev_alloc(p, &p->slot_pos, slots) || !dev_alloc(p, &p->slot_lab, slots) || !dev_alloc(p, &p->pos_slot, (size_t)total)) { cleanup(); return FFI_ERR_OUT_OF_MEMORY; }
+    hipLaunchKernelGGL(slot_clear_kernel, grid(slots), dim3(kBlock), 0, s, p->slot_pos, p->slot_lab, slots);
+    hipLaunchKernelGGL(slot_fill_kernel, grid((size_t)total), dim3(kBlock), 0, s, sorted_keys, sorted_pos, ptr, p->oct_ptr, total, p->K, p->N,
+                       block_labels, p->slot_pos, p->slot_lab, p->pos_slot);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     cleanup();
     if (e != hipSuccess) return hip_fail(e);
-    p->block_labels = kPlanBlockLabels;
+    p->block_labels = block_labels;
     p->nblocks = nblocks;
-    p->bytes += (size_t)total * sizeof(int32_t) + ((size_t)nkeys + 1) * sizeof(int32_t);
+    p->slots = (long long)slots;
+    p->bytes += slots * (sizeof(int32_t) + sizeof(unsigned short)) + ((size_t)nkeys + 1 + (size_t)total) * sizeof(unsigned);
     return FFI_OK;
 }
 

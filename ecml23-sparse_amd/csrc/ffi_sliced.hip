@@ -13,27 +13,47 @@ constexpr int kSlThreads = 256;
 constexpr int kSlInflight = 8;            // gathers a lane has in flight
 
 // ---- slice tables -------------------------------------------------------------------------------------------------
-// [B, rows] -> [slice][row][sl]: 64 x 64 tiles through LDS, whole lines on both sides.
+// [B, rows] -> [slice][row][sl]: 64 x 64 tiles through LDS, four elements per load and store (of rows at any alignment: the
+// memory system serves them), a tile's loads all in flight together.  One element at a time moved 3.0 TB/s.
+template <typename T> struct Quad { T v[4]; };
+
 template <typename T>
 __global__ __launch_bounds__(256) void slices_from_batch_major_kernel(const T* __restrict__ src, T* __restrict__ dst, int rows, int B,
                                                                       int sl) {
-    __shared__ T tile[64][64 + 4 / sizeof(T)];
+    __shared__ T tile[64][65];                            // [row][sample]
     const int r0 = blockIdx.x * 64, b0 = blockIdx.y * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int r4 = (threadIdx.x & 15) * 4, ty = threadIdx.x >> 4;
+    Quad<T> q[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int b = b0 + ty + 4 * i, r = r0 + tx;
-        tile[ty + 4 * i][tx] = (b < B && r < rows) ? src[(size_t)b * rows + r] : (T)0;
+    for (int i = 0; i < 4; ++i) {
+        const int b = b0 + ty + 16 * i, r = r0 + r4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[i].v[e] = (T)0;
+        if (b < B) {
+            if (r + 4 <= rows) q[i] = *reinterpret_cast<const Quad<T>*>(src + (size_t)b * rows + r);
+            else
+                for (int e = 0; e < 4; ++e)
+                    if (r + e < rows) q[i].v[e] = src[(size_t)b * rows + r + e];
+        }
     }
-    __syncthreads();
-    const int padded = (B + sl - 1) / sl * sl;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tile[r4 + e][ty + 16 * i] = q[i].v[e];
+    __syncthreads();
+    const int padded = (B + sl - 1) / sl * sl, width = sl < 64 ? sl : 64, quads = width / 4;      // (a slice inside the tile)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        // consecutive threads run over a slice's samples, then its rows, then the slices
         const int e = (int)threadIdx.x + 256 * i;
-        // (slices narrower than the tile: consecutive threads run over a slice's samples, then its rows)
-        const int width = sl < 64 ? sl : 64;
-        const int in = e % width, r = r0 + (e / width) % 64, b = b0 + e / (width * 64) * width + in;
-        if (r < rows && b < padded) dst[((size_t)(b / sl) * rows + r) * sl + b % sl] = tile[b - b0][r - r0];
+        const int in = e % quads * 4, r = e / quads % 64, t = e / (quads * 64) * width + in;
+        const int b = b0 + t;
+        if (r0 + r < rows && b < padded) {
+            Quad<T> o;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o.v[c] = tile[r][t + c];
+            *reinterpret_cast<Quad<T>*>(dst + ((size_t)(b / sl) * rows + r0 + r) * sl + b % sl) = o;
+        }
     }
 }
 

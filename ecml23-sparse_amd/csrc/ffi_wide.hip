@@ -9,6 +9,7 @@
 // connection moves B*4 bytes.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
+#include "ffi_sliced.h"
 
 #include <algorithm>
 
@@ -124,86 +125,289 @@ __global__ __launch_bounds__(kWideThreads) void wgrad_wide_kernel(const float* _
     if (bias_grad != nullptr && threadIdx.x < kWideLabels && j0 + (int)threadIdx.x < L) bias_grad[j0 + threadIdx.x] = bres[threadIdx.x];
 }
 
-// ---- input gradient -----------------------------------------------------------------------------
-// One wavefront per (column n, batch pass).  The plan lists the connections of a column, grouped by
-// label block and in ascending position; the wavefront walks them in that order (64 at a time: one
-// per lane, then handed out as scalars), gathering one 512-byte piece of row j of gT per
-// connection.  No atomics, fixed order: reproducible.  Label blocks bound the part of gT that is
-// live at any time, so the gathers are served by the last-level cache.
-template <bool TWO>
-__global__ __launch_bounds__(kWideThreads) void igrad_wide_kernel(const int32_t* __restrict__ perm,
-                                                                  const int32_t* __restrict__ col_ptr,
-                                                                  const float* __restrict__ w,
-                                                                  const float* __restrict__ gT, float* __restrict__ gxT,
-                                                                  int B, int N, int L, int K, int nblocks,
-                                                                  unsigned kdiv_mul, unsigned kdiv_shift, int ldb) {
+// ---- input gradient and weight gradient over the plan's global form ------------------------------------------------
+// Column n's gradient sums w * g[label] over its connections; the weight gradient of a connection is the dot product of
+// x[n] and g[label].  Both need row `label` of out_grad, so one walk over the lists of the plan gathers it once: GL lanes of
+// 16 bytes hold a row of a slice of out_grad (ffi_sliced.h), a wavefront owns M x (64 / GL) columns -- their sums stay in
+// LDS -- and goes through the label blocks of its stream in order.  All workgroups of an XCD do so
+// at the same pace, so the block's rows of out_grad (a few MB) are what the L2 holds.
+//
+// A lane group copies its list through LDS, a window of a few octs of slots at a time, the next window on its way while it
+// walks.  Weight gradients leave in the order of the plan's slots
+// (weight_grads_in_place_kernel moves them).
+//
+// What bounds it: L2 delivery of the gathered rows (31 TB/s at most) and, with DOT, the instructions beside it (per oct and
+// lane 64 multiply-adds, 21 for the sums over the lanes, 8 gathers).
+constexpr int kWalkThreads = 1024;
+constexpr int kWalkMaxM = 4;
+// octs per window of a lane group, quads of it that a lane brings, and the window's place in LDS (16-byte words, one more
+// than it holds: the groups read from different banks)
+constexpr int walk_octs(int gl) { return gl >= 4 ? 4 : gl; }
+constexpr int walk_quads(int gl) { return walk_octs(gl) * 2 / gl; }
+constexpr int walk_stride(int gl) { return walk_octs(gl) * 4 + 1; }
+
+// v + (v of the lane that CTRL pairs with this one)
+template <int CTRL> __device__ __forceinline__ float dpp_add(float keep, float send) {
+    return keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, send), CTRL, 0xf, 0xf, true));
+}
+
+// Sums eight values over the GL lanes of a group; lane `sub` is left with values sub * (8 / GL) ... of them, in p[0 ... 8 / GL).
+template <int GL> __device__ __forceinline__ void group_sums(float (&p)[8], int sub) {
+    constexpr int kHalfMirror = 0x141, kQuadMirror = 0x1b, kQuadSwap = 0xb1;    // lanes i <-> 7 - i, 3 - i, i ^ 1
+    if constexpr (GL == 8) {
+        const bool up = (sub & 4) != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = dpp_add<kHalfMirror>(up ? p[i + 4] : p[i], up ? p[i] : p[i + 4]);
+    }
+    if constexpr (GL >= 4) {
+        constexpr int n = GL == 8 ? 2 : 4;
+        const bool up = (sub & 2) != 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) p[i] = dpp_add<kQuadMirror>(up ? p[i + n] : p[i], up ? p[i] : p[i + n]);
+    }
+    if constexpr (GL >= 2) {
+        constexpr int n = GL == 8 ? 1 : GL == 4 ? 2 : 4;
+        const bool up = (sub & 1) != 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) p[i] = dpp_add<kQuadSwap>(up ? p[i + n] : p[i], up ? p[i] : p[i + n]);
+    }
+}
+
+template <int GL, bool DOT>
+__global__ __launch_bounds__(kWalkThreads) void walk_columns_kernel(const float* __restrict__ gtab, const float* __restrict__ xtab,
+                                                                    const unsigned* __restrict__ oct_ptr,
+                                                                    const unsigned short* __restrict__ slot_lab,
+                                                                    const float* __restrict__ slot_w, float* __restrict__ gx_part,
+                                                                    float* __restrict__ gw_slots, int add_gw, size_t slots, int N, int L,
+                                                                    int nblocks, int block_labels, int blocks_per_stream, int col_chunks,
+                                                                    int units, int M) {
+    constexpr int kGroups = 64 / GL;
+    constexpr unsigned kRow = GL * 16u;
+    constexpr unsigned kNoRow = 0xffffff00u;
+    constexpr int kOcts = walk_octs(GL), kQuads = walk_quads(GL);
+    // per wavefront: its groups' windows of (row offset, weight) pairs, two per entry, and the sums of its M x 64 lanes
+    extern __shared__ __align__(16) uint4 walk_mem[];
+    const int u = xcd_unit(blockIdx.x, units);
+    if (u < 0) return;
+    const int chunk = u % col_chunks, stream = u / col_chunks;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n = blockIdx.x * (kWideThreads / 64) + wave;
-    if (n >= N) return;                                         // wave-uniform
-    const int bc0 = blockIdx.y * kWideBatch;
-    const buffer_rsrc gr = make_rsrc(gT, (size_t)L * (size_t)ldb * sizeof(float));
-    const unsigned lane_off0 = (unsigned)(bc0 + lane) * 4u, lane_off1 = lane_off0 + 256u;
-    float acc0 = 0.f, acc1 = 0.f;
-    for (int blk = 0; blk < nblocks; ++blk) {
-        const int beg = col_ptr[(size_t)blk * N + n], end = col_ptr[(size_t)blk * N + n + 1];
-        for (int e0 = beg; e0 < end; e0 += 64) {
-            const int cnt = min(64, end - e0);
-            int p = 0;
-            float wv = 0.f;
-            if (lane < cnt) { p = perm[e0 + lane]; wv = w[p]; }
-            // label of the connection: p / K by multiply-high and shift (exact for p < 2^31)
-            const unsigned jv = kdiv_mul ? (__umulhi((unsigned)p, kdiv_mul) >> kdiv_shift) : (unsigned)p;
-            int i = 0;
-            for (; i + kWideInflight <= cnt; i += kWideInflight) {
-                float a[kWideInflight], b[kWideInflight], ws[kWideInflight];
+    const int sub = lane & (GL - 1), grp = lane / GL;
+    const int n0 = (chunk * (kWalkThreads / 64) + wave) * M * kGroups;     // first column of this wavefront
+    if (n0 >= N) return;                                                    // (the barriers below count the wavefronts that are left)
+    uint4* const wave_mem = walk_mem + wave * (kGroups * walk_stride(GL) + 64 * M);
+    uint4* list = wave_mem + grp * walk_stride(GL);
+    float4* sums = reinterpret_cast<float4*>(wave_mem + kGroups * walk_stride(GL)) + lane;
+    const unsigned lane_off = (unsigned)sub * 16u;
+    for (int m = 0; m < M; ++m) sums[64 * m] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int blk_end = min((stream + 1) * blocks_per_stream, nblocks);
+    int blk = stream * blocks_per_stream;
+    // octs of this lane group's list of (blk, m), and its column's row of x (fetched anew for every block: held for all m
+    // it would cost a wavefront per SIMD); columns behind the last have no octs
+    auto list_of = [&](int b, int m, unsigned& begin, unsigned& end, float4& x) {
+        const size_t at = (size_t)b * N;
+        const int n = n0 + m * kGroups + grp;
+        begin = oct_ptr[at + min(n, N)];
+        end = oct_ptr[at + min(n + 1, N)];
+        if (DOT) x = *reinterpret_cast<const float4*>(xtab + (size_t)min(n, N - 1) * (GL * 4) + sub * 4);
+    };
+    uint4 next_w[kQuads];
+    uint2 next_lab[kQuads];
+    auto fetch = [&](unsigned oct) {                                        // (behind the plan's end: its last quad)
 #pragma unroll
-                for (int u = 0; u < kWideInflight; ++u) {
-                    const unsigned j = (unsigned)__builtin_amdgcn_readlane((int)jv, i + u);
-                    ws[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wv), i + u));
-                    // rows of gT are ldb*4 bytes; L*ldb*4 < 2^32 is checked by the launcher
-                    a[u] = buffer_load_f32(gr, lane_off0, j * (unsigned)ldb * 4u);
-                    b[u] = TWO ? buffer_load_f32(gr, lane_off1, j * (unsigned)ldb * 4u) : 0.f;
+        for (int v = 0; v < kQuads; ++v) {
+            const size_t at = min((size_t)oct * 8 + 4 * (v * GL + sub), slots - 4);
+            next_w[v] = *reinterpret_cast<const uint4*>(slot_w + at);
+            next_lab[v] = *reinterpret_cast<const uint2*>(slot_lab + at);
+        }
+    };
+    unsigned begin = 0, end = 0;
+    float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (blk < blk_end) {
+        list_of(blk, 0, begin, end, xv);
+        fetch(begin);
+    }
+    for (; blk < blk_end; ++blk) {
+        __syncthreads();
+        const int label0 = blk * block_labels;
+        const buffer_rsrc rsrc = make_rsrc(gtab + (size_t)label0 * (GL * 4), (size_t)min(block_labels, L - label0) * kRow);
+#pragma unroll 1
+        for (int m = 0; m < M; ++m) {
+            float4 acc = sums[64 * m];
+            int longest = (int)(end - begin);
+#pragma unroll
+            for (int off = 32; off >= GL; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+            longest = __builtin_amdgcn_readfirstlane(longest);
+            unsigned after_begin = 0, after_end = 0;                        // the lists that follow
+            float4 after_x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (m + 1 < M) list_of(blk, m + 1, after_begin, after_end, after_x);
+            else if (blk + 1 < blk_end) list_of(blk + 1, 0, after_begin, after_end, after_x);
+            for (int w0 = 0; w0 < longest || w0 == 0; w0 += kOcts) {
+                __builtin_amdgcn_wave_barrier();                            // (the windows are the wavefront's own: LDS serves it in order)
+                const unsigned at = begin + (unsigned)w0;
+                const int here = min(kOcts, (int)(end - at));               // octs of this group's list in this window (<= 0: none)
+                float4 gw_old[DOT ? kQuads : 1];
+#pragma unroll
+                for (int v = 0; v < kQuads; ++v) {
+                    const int q = v * GL + sub;
+                    const uint2 lab = next_lab[v];
+                    const unsigned l0 = lab.x & 0xffffu, l1 = lab.x >> 16, l2 = lab.y & 0xffffu, l3 = lab.y >> 16;
+                    list[2 * q] = make_uint4(l0 == kNoLabel ? kNoRow : l0 * kRow, next_w[v].x, l1 == kNoLabel ? kNoRow : l1 * kRow, next_w[v].y);
+                    list[2 * q + 1] = make_uint4(l2 == kNoLabel ? kNoRow : l2 * kRow, next_w[v].z, l3 == kNoLabel ? kNoRow : l3 * kRow, next_w[v].w);
+                    if (DOT) {
+                        gw_old[v] = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (add_gw && q < 2 * here) gw_old[v] = *reinterpret_cast<const float4*>(gw_slots + (size_t)at * 8 + 4 * q);
+                    }
                 }
+                fetch(w0 + kOcts < longest ? at + kOcts : after_begin);
+                __builtin_amdgcn_wave_barrier();
+                const int steps = min(kOcts, longest - w0);
+#pragma unroll 1
+                for (int i = 0; i < steps; ++i) {
+                    if (i < here) {
+                        uint4 e[4], x[8];
 #pragma unroll
-                for (int u = 0; u < kWideInflight; ++u) {
-                    acc0 = fmaf(ws[u], a[u], acc0);
-                    if (TWO) acc1 = fmaf(ws[u], b[u], acc1);
+                        for (int v = 0; v < 4; ++v) e[v] = list[4 * i + v];
+#pragma unroll
+                        for (int v = 0; v < 8; ++v)
+                            x[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((v & 1) ? e[v / 2].z : e[v / 2].x) + lane_off, 0, 0));
+                        float p[8];
+#pragma unroll
+                        for (int v = 0; v < 8; ++v) {
+                            const float wv = __uint_as_float((v & 1) ? e[v / 2].w : e[v / 2].y);
+                            const float r0 = __uint_as_float(x[v].x), r1 = __uint_as_float(x[v].y), r2 = __uint_as_float(x[v].z), r3 = __uint_as_float(x[v].w);
+                            acc.x = fmaf(wv, r0, acc.x); acc.y = fmaf(wv, r1, acc.y);
+                            acc.z = fmaf(wv, r2, acc.z); acc.w = fmaf(wv, r3, acc.w);
+                            if (DOT) p[v] = fmaf(xv.w, r3, fmaf(xv.z, r2, fmaf(xv.y, r1, xv.x * r0)));
+                        }
+                        if (DOT) {
+                            group_sums<GL>(p, sub);
+#pragma unroll
+                            for (int v = 0; v < 8 / GL; ++v) reinterpret_cast<float*>(list + 4 * i)[sub * (8 / GL) + v] = p[v];   // (in place of the oct)
+                        }
+                    }
                 }
-            }
-            if (i < cnt) {
-                // (the last, partly filled group: in flight together, what lies behind the end is left out of the sum)
-                float a[kWideInflight], b[kWideInflight], ws[kWideInflight];
+                if (DOT) {
+                    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int u = 0; u < kWideInflight; ++u) {
-                    const int ii = min(i + u, cnt - 1);
-                    const unsigned j = (unsigned)__builtin_amdgcn_readlane((int)jv, ii);
-                    const float wk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wv), ii));
-                    ws[u] = wk;
-                    a[u] = buffer_load_f32(gr, lane_off0, j * (unsigned)ldb * 4u);
-                    b[u] = TWO ? buffer_load_f32(gr, lane_off1, j * (unsigned)ldb * 4u) : 0.f;
-                }
-#pragma unroll
-                for (int u = 0; u < kWideInflight; ++u) {
-                    if (i + u < cnt) {                          // wave-uniform
-                        acc0 = fmaf(ws[u], a[u], acc0);
-                        if (TWO) acc1 = fmaf(ws[u], b[u], acc1);
+                    for (int v = 0; v < kQuads; ++v) {
+                        const int q = v * GL + sub;
+                        if (q < 2 * here) {
+                            const float4 d = *reinterpret_cast<const float4*>(list + 4 * (q >> 1) + (q & 1));
+                            *reinterpret_cast<float4*>(gw_slots + (size_t)at * 8 + 4 * q) =
+                                make_float4(gw_old[v].x + d.x, gw_old[v].y + d.y, gw_old[v].z + d.z, gw_old[v].w + d.w);
+                        }
                     }
                 }
             }
+            sums[64 * m] = acc;
+            begin = after_begin; end = after_end; xv = after_x;
         }
     }
-    if (bc0 + lane < B) gxT[(size_t)n * B + bc0 + lane] = acc0;
-    if (TWO && bc0 + 64 + lane < B) gxT[(size_t)n * B + bc0 + 64 + lane] = acc1;
+    for (int m = 0; m < M; ++m) {
+        const int n = n0 + m * kGroups + grp;
+        if (n < N)
+            *reinterpret_cast<float4*>(gx_part + ((size_t)stream * N + n) * (GL * 4) + sub * 4) = sums[64 * m];
+    }
 }
 
-// floor(p / d) for 0 <= p < 2^31 as (p * mul) >> (32 + shift)
-void magic_divisor(unsigned d, unsigned* mul, unsigned* shift) {
-    if (d == 1) { *mul = 0; *shift = 0; return; }               // mul == 0 means: quotient = p
-    unsigned s = 0;
-    while ((1ull << s) < d) ++s;                                   // s = ceil(log2 d)
-    const unsigned long long m = ((1ull << (32 + s - 1)) + d - 1) / d;   // fits 32 bits, error < 2^-31
-    *mul = (unsigned)m;
-    *shift = s - 1;
+// slot_w[slot] = the weight of the slot's connection (0 in padding).  Slots are dealt to the XCDs in eight consecutive
+// ranges: an XCD reads the weights of one label block after the other, which its L2 holds.
+__global__ __launch_bounds__(256) void slot_weights_kernel(const float* __restrict__ w, const int32_t* __restrict__ slot_pos,
+                                                           float* __restrict__ slot_w, size_t slots, int units) {
+    const int u = xcd_unit(blockIdx.x, units);
+    if (u < 0) return;
+    const size_t q = (size_t)u * 256 + threadIdx.x;
+    if (q * 4 >= slots) return;
+    const int4 at = reinterpret_cast<const int4*>(slot_pos)[q];
+    float4 v;
+    v.x = w[max(at.x, 0)]; v.y = w[max(at.y, 0)]; v.z = w[max(at.z, 0)]; v.w = w[max(at.w, 0)];
+    if (at.x < 0) v.x = 0.f;
+    if (at.y < 0) v.y = 0.f;
+    if (at.z < 0) v.z = 0.f;
+    if (at.w < 0) v.w = 0.f;
+    reinterpret_cast<float4*>(slot_w)[q] = v;
+}
+
+// gw[pos] = gw_slots[pos_slot[pos]]; positions are dealt to the XCDs like the slots above.  (Reads at random places: the same
+// permutation as scattered writes, from the slots' side, took twice as long.)
+__global__ __launch_bounds__(256) void weight_grads_in_place_kernel(const float* __restrict__ gw_slots, const unsigned* __restrict__ pos_slot,
+                                                                    float* __restrict__ gw, size_t count, int units) {
+    const int u = xcd_unit(blockIdx.x, units);
+    if (u < 0) return;
+    const size_t p0 = ((size_t)u * 256 + threadIdx.x / 64 * 64) * 4 + (threadIdx.x & 63);
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = gw_slots[pos_slot[min(p0 + 64 * i, count - 1)]];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (p0 + 64 * i < count) gw[p0 + 64 * i] = v[i];
+}
+
+// gx ([N,B] or [B,N]) = sum over the streams of part[slice][stream][n][sl], ascending; 32 columns x 32 samples per workgroup
+template <bool TP>
+__global__ __launch_bounds__(256) void gather_gx_kernel(const float* __restrict__ part, float* __restrict__ gx, int N, int B, int sl,
+                                                        int streams) {
+    __shared__ float tile[32][33];
+    const int n0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int i = ty; i < 32; i += 8) {
+        const int n = n0 + i, b = b0 + tx;
+        float v = 0.f;
+        if (n < N && b < B)
+            for (int t = 0; t < streams; ++t) v += part[(((size_t)(b / sl) * streams + t) * N + n) * sl + b % sl];
+        if (TP) {
+            if (n < N && b < B) gx[(size_t)n * B + b] = v;
+        } else {
+            tile[i][tx] = v;
+        }
+    }
+    if (TP) return;
+    __syncthreads();
+    for (int i = ty; i < 32; i += 8) {
+        const int n = n0 + tx, b = b0 + i;
+        if (n < N && b < B) gx[(size_t)b * N + n] = tile[tx][i];
+    }
+}
+
+// bias_grad[j] = sum over the samples of g[b, j]: 64 labels per workgroup, four partial sums added in order
+__global__ __launch_bounds__(256) void column_sums_kernel(const float* __restrict__ g, float* __restrict__ bias_grad, int B, int L) {
+    __shared__ float part[4][64];
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int j = blockIdx.x * 64 + tx;
+    float v = 0.f;
+    if (j < L)
+        for (int b = ty; b < B; b += 4) v += g[(size_t)b * L + j];
+    part[ty][tx] = v;
+    __syncthreads();
+    if (ty == 0 && j < L) bias_grad[j] = ((part[0][tx] + part[1][tx]) + part[2][tx]) + part[3][tx];
+}
+
+struct WalkArgs {
+    const float *gtab, *xtab, *slot_w;
+    float *gx_part, *gw_slots;
+    bool add_gw;
+    int streams, blocks_per_stream;
+};
+
+template <int GL, bool DOT>
+int launch_walk(int m, const ffi_plan* p, const WalkArgs& a, hipStream_t s) {
+    const int wg_cols = kWalkThreads / 64 * m * (64 / GL), col_chunks = (p->N + wg_cols - 1) / wg_cols;
+    const int units = col_chunks * a.streams;
+    const size_t lds = (size_t)(kWalkThreads / 64) * (64 / GL * walk_stride(GL) + 64 * m) * sizeof(uint4);
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)walk_columns_kernel<GL, DOT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((walk_columns_kernel<GL, DOT>), dim3(xcd_grid(units)), dim3(kWalkThreads), lds, s, a.gtab, a.xtab, p->oct_ptr,
+                       p->slot_lab, a.slot_w, a.gx_part, a.gw_slots, a.add_gw ? 1 : 0, (size_t)p->slots, p->N, p->L, p->nblocks,
+                       p->block_labels, a.blocks_per_stream, col_chunks, units, m);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
+template <bool DOT>
+int launch_walk_gl(int gl, int m, const ffi_plan* p, const WalkArgs& a, hipStream_t s) {
+    if (gl == 1) return launch_walk<1, DOT>(m, p, a, s);
+    if (gl == 2) return launch_walk<2, DOT>(m, p, a, s);
+    if (gl == 4) return launch_walk<4, DOT>(m, p, a, s);
+    return launch_walk<8, DOT>(m, p, a, s);
 }
 
 }  // namespace
@@ -255,26 +459,66 @@ int launch_weight_grad_wide(const float* x, const int32_t* idx, const float* g, 
     return FFI_OK;
 }
 
-int launch_input_grad_wide(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp, hipStream_t s) {
-    if (!wide_offsets_fit(p->L, B)) return FFI_ERR_TOO_LARGE;
-    const int ldb = wide_row_stride(B);
-    float* gT = nullptr;
-    FFI_TRY(workspace_get(s, kWsPartials, (size_t)p->L * ldb * sizeof(float), (void**)&gT));
-    FFI_TRY(launch_transpose(g, gT, B, p->L, s, p->L, ldb));      // [B,L] -> [L,ldb]
-    float* gxT = gx;
-    if (!tp) FFI_TRY(workspace_get(s, kWsFeaturesT, (size_t)p->N * B * sizeof(float), (void**)&gxT));
-    unsigned mul = 0, shift = 0;
-    magic_divisor((unsigned)p->K, &mul, &shift);
-    dim3 grid((p->N + kWideThreads / 64 - 1) / (kWideThreads / 64), (B + kWideBatch - 1) / kWideBatch);
-    if (grid.y > 65535u) return FFI_ERR_TOO_LARGE;
-    if (B > 64)
-        hipLaunchKernelGGL(igrad_wide_kernel<true>, grid, dim3(kWideThreads), 0, s, p->perm, p->col_ptr, w, gT, gxT, B, p->N, p->L,
-                           p->K, p->nblocks, mul, shift, ldb);
-    else
-        hipLaunchKernelGGL(igrad_wide_kernel<false>, grid, dim3(kWideThreads), 0, s, p->perm, p->col_ptr, w, gT, gxT, B, p->N,
-                           p->L, p->K, p->nblocks, mul, shift, ldb);
+// How the walk is cut: columns per lane group (m) and streams of label blocks, so that about 16 wavefronts per CU are in
+// flight: as many columns per group as that allows (a walk of all blocks each), else several streams whose sums are added.
+void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, int* streams, int* blocks_per_stream) {
+    *gl = slice_lanes(B, 4);
+    *slices = (B + *gl * 4 - 1) / (*gl * 4);
+    const long long target = device_cu_count();                             // workgroups
+    const int group_cols = kWalkThreads / *gl;                              // columns per workgroup and m
+    *m = kWalkMaxM;
+    while (*m > 1 && (long long)(N + group_cols * *m - 1) / (group_cols * *m) < target) *m /= 2;
+    const long long wgs = (N + group_cols * *m - 1) / (group_cols * *m);
+    const int want = (int)std::min<long long>(nblocks, std::max<long long>(1, target / wgs));
+    *blocks_per_stream = (nblocks + want - 1) / want;
+    *streams = (nblocks + *blocks_per_stream - 1) / *blocks_per_stream;
+}
+
+int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
+                         bool tp, hipStream_t s) {
+    if (!p->oct_ptr || !p->slot_pos || !p->slot_lab) return FFI_ERR_BAD_ARGUMENT;
+    const bool dot = gw != nullptr;
+    int gl, slices, m;
+    WalkArgs a{};
+    walk_shape(p->N, B, p->L, p->nblocks, &gl, &slices, &m, &a.streams, &a.blocks_per_stream);
+    const int sl = gl * 4;
+    const size_t slots = (size_t)p->slots, count = (size_t)p->L * p->K, gslice = (size_t)p->L * sl, part = (size_t)p->N * sl * a.streams;
+    float* ws = nullptr;
+    FFI_TRY(workspace_get(s, kWsPartials, (gslice + part) * slices * sizeof(float), (void**)&ws));
+    float* slot_w = nullptr;
+    FFI_TRY(workspace_get(s, kWsSlots, slots * sizeof(float), (void**)&slot_w));
+    FFI_TRY(launch_slices_f32(g, ws, p->L, B, sl, false, s));
+    float* const parts = ws + gslice * slices;
+    float* xtab = nullptr;
+    if (dot) {
+        FFI_TRY(workspace_get(s, kWsFeaturesT, (size_t)p->N * sl * slices * sizeof(float), (void**)&xtab));
+        FFI_TRY(launch_slices_f32(x, xtab, p->N, B, sl, tp, s));
+        FFI_TRY(workspace_get(s, kWsWeightParts, slots * sizeof(float), (void**)&a.gw_slots));
+    }
+    const int slot_units = (int)((slots / 4 + 255) / 256);
+    hipLaunchKernelGGL(slot_weights_kernel, dim3(xcd_grid(slot_units)), dim3(256), 0, s, w, p->slot_pos, slot_w, slots, slot_units);
     FFI_HIP_TRY(hipGetLastError());
-    if (!tp) FFI_TRY(launch_transpose(gxT, gx, p->N, B, s));      // [N,B] -> [B,N]
+    // one slice after the other: their weight gradients add up in place
+    a.slot_w = slot_w;
+    for (int q = 0; q < slices; ++q) {
+        a.gtab = ws + gslice * q; a.gx_part = parts + part * q; a.add_gw = q > 0;
+        a.xtab = dot ? xtab + (size_t)p->N * sl * q : nullptr;
+        FFI_TRY(dot ? launch_walk_gl<true>(gl, m, p, a, s) : launch_walk_gl<false>(gl, m, p, a, s));
+    }
+    if (dot) {
+        const int units = (int)((count + 1023) / 1024);
+        hipLaunchKernelGGL(weight_grads_in_place_kernel, dim3(xcd_grid(units)), dim3(256), 0, s, a.gw_slots, p->pos_slot, gw, count, units);
+        FFI_HIP_TRY(hipGetLastError());
+    }
+    if (bias_grad != nullptr) {
+        hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((p->L + 63) / 64)), dim3(256), 0, s, g, bias_grad, B, p->L);
+        FFI_HIP_TRY(hipGetLastError());
+    }
+    const dim3 grid((unsigned)((p->N + 31) / 32), (unsigned)((B + 31) / 32));
+    if (grid.y > 65535u) return FFI_ERR_TOO_LARGE;
+    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
+    else hipLaunchKernelGGL(gather_gx_kernel<false>, grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
+    FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 

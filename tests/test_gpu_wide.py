@@ -42,3 +42,31 @@ def test_forward_of_wide_inputs(ffi, ranges):
             assert rel_err(out, ref + bias) <= 1e-5, (B, N, L, K)
     finally:
         lib.ffi_set_option(b"wide_ranges", 0)
+
+
+# (B, N, L, K): lane groups of 1, 2, 4 and 8; lists that are empty, shorter and longer than a window; several label blocks,
+# streams and slices; one column
+BACKWARD_SHAPES = [(1, 1217, 900, 3), (4, 2000, 30_000, 9), (5, 1217, 129, 17), (8, 3000, 3000, 40), (9, 1300, 65, 33), (16, 2500, 5000, 64),
+                   (17, 40_000, 63, 3), (33, 1300, 9000, 72), (100, 40_000, 200, 65), (130, 1500, 97, 130), (64, 30_000, 3000, 36)]
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_backward_of_wide_inputs(ffi, transposed):
+    for B, N, L, K in BACKWARD_SHAPES:
+        x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B + N)
+        if (B, N) == (33, 1300):
+            lookup[::3] = 7                                     # one column holds a third of all connections
+        ref_gx, ref_gw = oracle.backward(np.ascontiguousarray(x.T) if transposed else x, lookup, w, g, transposed=transposed)
+        dx, dl, dw, dg = dev(x.T if transposed else x), dev(lookup), dev(w), dev(g)
+        bwd = ffi.fan_in_sparse_matmul_grad_tp if transposed else ffi.fan_in_sparse_matmul_grad
+        first = None
+        for _ in range(2):                                      # the call that builds the plan, and one behind a check of it
+            gx, gw = bwd(dx, dl, dw, dg)
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4, (B, N, L, K)
+            assert rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4, (B, N, L, K)
+            assert first is None or torch.equal(first, gx)
+            first = gx
+        if not transposed:
+            bias = torch.zeros(L, device="cuda", requires_grad=True)
+            gb, = torch.autograd.grad(ffi.fan_in_sparse_matmul_bias(dx.requires_grad_(True), dl, dw, bias), [bias], dg)
+            assert rel_err(gb.cpu().numpy(), g.astype(np.float64).sum(0)) <= 1e-5
