@@ -26,7 +26,7 @@ SOURCES = [
     "ffi_util.hip",
     "ffi_wide.hip",
     "ffi_sliced.hip",
-    "ffi_bf16.hip",
+    "ffi_topk.hip",
     "ffi_loss.hip",
     "ffi_sparse_grad.hip",
     "ffi_optimizer.hip",

@@ -287,7 +287,8 @@ int ffi_forward_topk_bf16(const uint16_t* features, const int32_t* lookup, const
     if (!features || !lookup || !weights || !topk_values || !topk_indices) return FFI_ERR_NULL_POINTER;
     Dims d;
     FFI_TRY(check_dims(batch, num_features, num_units, fan_in, transposed, &d));
-    return launch_forward_topk_bf16(features, lookup, weights, topk_values, topk_indices, k, d, (hipStream_t)stream);
+    if (k < 1 || k > 8) return FFI_ERR_BAD_ARGUMENT;
+    return launch_forward_topk_sliced(features, lookup, weights, nullptr, true, TopkArgs{k, topk_values, topk_indices}, d, (hipStream_t)stream);
 }
 
 int ffi_topk_f32(const float* scores, int64_t batch, int64_t num_units, int k, float* topk_values, int32_t* topk_indices,
@@ -622,7 +623,7 @@ int ffi_set_option(const char* name, int value) {
         {"plan_weights_in_lds", &ffi::Options::plan_weights_in_lds, -1, 1},
         {"workgroups_per_cu", &ffi::Options::workgroups_per_cu, 0, 16},
         {"plan_sorted_columns", &ffi::Options::plan_sorted_columns, -1, 1},
-        {"wide_ranges", &ffi::Options::wide_ranges, 0, 4},
+        {"wide_phases", &ffi::Options::wide_phases, -1, 1},
     };
     for (const auto& t : table) {
         if (std::strcmp(name, t.name) != 0) continue;

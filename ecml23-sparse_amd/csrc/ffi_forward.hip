@@ -6,7 +6,7 @@
 //                      takes its x operand from LDS; the LDS delivers 128 bytes per clock per CU,
 //                      which bounds the kernel (4 bytes per multiply-add), so the layout is chosen
 //                      to keep the gathers free of bank conflicts and the instruction count low.
-// Other shapes go to the wide-input kernel (ffi_wide.hip).
+// Batches of at most 16 samples and wide inputs go to the kernels of ffi_sliced.hip.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 #include "ffi_loss.h"
@@ -85,8 +85,7 @@ constexpr int kTopkPark = 24;           // candidates per (workgroup, batch row)
 // those >= tau[b]; every such (label, score) is appended to the sample's candidate list, a few hundred to a
 // few thousand entries out of all labels, and a small kernel selects the k best afterwards.
 struct FwdTopk {
-    const float* tau;     // tau[b * tau_stride]
-    int tau_stride;
+    const float* tau;     // [B]
     int* count;           // [B] candidates appended so far (may run past cap: the list is then incomplete)
     float* cand_val;      // [B][cap]
     int* cand_idx;        // [B][cap]
@@ -157,7 +156,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     stage_rows32<kTileThreads, 8>(xs, xT, N, B, b0);       // (eight loads in flight per thread: the tile arrives in one round trip at 768 rows)
     if (TOPK && threadIdx.x < kTileBatch) local_count[threadIdx.x] = 0;
     if (TOPK && threadIdx.x < kTileBatch)          // rows past the batch never qualify
-        tau_s[threadIdx.x] = b0 + (int)threadIdx.x < B ? ft.tau[(size_t)(b0 + threadIdx.x) * ft.tau_stride] : __builtin_inff();
+        tau_s[threadIdx.x] = b0 + (int)threadIdx.x < B ? ft.tau[b0 + threadIdx.x] : __builtin_inff();
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const unsigned skewbase = (unsigned)(size_t)(__attribute__((address_space(3))) float*)xs + (unsigned)(lane & 7) * 16u;
@@ -272,7 +271,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
                                 if (lslot < kTopkPark) {
                                     local_cand[b * kTopkPark + lslot] = make_int2(j, __float_as_int(acc[b]));
                                 } else {
-                                    const int slot = atomicAdd(&ft.count[b0 + b], 1);
+                                    const int slot = atomicAdd(&ft.count[(size_t)(b0 + b) * kTopkCountStep], 1);
                                     if (slot < ft.cap) {
                                         ft.cand_val[(size_t)(b0 + b) * ft.cap + slot] = acc[b];
                                         ft.cand_idx[(size_t)(b0 + b) * ft.cap + slot] = j;
@@ -330,7 +329,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
         __syncthreads();
         if (threadIdx.x < kTileBatch) {
             const int n = min(local_count[threadIdx.x], kTopkPark);
-            local_base[threadIdx.x] = n ? atomicAdd(&ft.count[b0 + threadIdx.x], n) : 0;
+            local_base[threadIdx.x] = n ? atomicAdd(&ft.count[(size_t)(b0 + threadIdx.x) * kTopkCountStep], n) : 0;
         }
         __syncthreads();
         for (int e = threadIdx.x; e < kTileBatch * kTopkPark; e += kTileThreads) {
@@ -618,27 +617,19 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
     FwdLoss fl{gout, nullptr, nullptr, 0.f, 0, 0};
     FwdTopk ft{};
     const bool topk = tk != nullptr;
-    int* count = nullptr;
+    TopkCandidates tc{};
     size_t lds_topk = lds;
     if (topk) {
         // thresholds: the k-th best score of every sample among kTopkSample evenly spaced labels
         const int S = std::min(kTopkSample, d.L);
-        const size_t cand = (size_t)d.B * kTopkCap;
-        unsigned char* ws = nullptr;
-        const size_t bytes = ((size_t)d.B * S + 2 * (size_t)d.B * 8 + (size_t)d.B + 2 * cand) * 4;
-        FFI_TRY(workspace_get(s, kWsTopk, bytes, (void**)&ws));
-        float* sample_scores = reinterpret_cast<float*>(ws);
-        float* tau_val = sample_scores + (size_t)d.B * S;
-        int* tau_idx = reinterpret_cast<int*>(tau_val + (size_t)d.B * 8);
-        count = tau_idx + (size_t)d.B * 8;
-        float* cand_val = reinterpret_cast<float*>(count + d.B);
-        int* cand_idx = reinterpret_cast<int*>(cand_val + cand);
-        hipLaunchKernelGGL(fwd_sample_kernel, dim3(S), dim3(256), 0, s, xT, idx, w, bias, d.B, d.N, d.L, d.K, S, sample_scores);
+        void* ws = nullptr;
+        FFI_TRY(workspace_get(s, kWsTopk, topk_candidate_bytes(d.B, S), &ws));
+        tc = topk_candidates_at(ws, d.B, S);
+        hipLaunchKernelGGL(fwd_sample_kernel, dim3(S), dim3(256), 0, s, xT, idx, w, bias, d.B, d.N, d.L, d.K, S, tc.sample);
         FFI_HIP_TRY(hipGetLastError());
-        FFI_TRY(launch_topk_f32(sample_scores, d.B, S, tk->k, tau_val, tau_idx, s));
-        FFI_TRY(launch_topk_candidates_init(count, cand_idx, d.B, kTopkCap, s));
+        FFI_TRY(launch_topk_threshold(tc.sample, (size_t)S, 1, S, tk->k, tc, d.B, s));
         // LDS behind the tile of x holds the workgroup's candidates until the end of the kernel
-        ft = FwdTopk{tau_val + (tk->k - 1), tk->k, count, cand_val, cand_idx, kTopkCap};
+        ft = FwdTopk{tc.tau, tc.count, tc.val, tc.idx, kTopkCap};
         lds_topk = lds + (size_t)kTileBatch * kTopkPark * sizeof(int2);
     }
     int npartial = 0;
@@ -661,8 +652,8 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         // (a sample with more candidates than its list holds: its row once more, from the score matrix if there is one)
         TopkRowSource src;
         if (epi == kEpiScores || epi == kEpiLossGradAndScores) src.scores = out;
-        src.xT = xT; src.idx = idx; src.w = w; src.bias = bias; src.N = d.N; src.L = d.L; src.K = d.K;
-        FFI_TRY(launch_topk_candidates_select(ft.cand_val, ft.cand_idx, count, d.B, kTopkCap, tk->k, tk->values, tk->indices, s, src));
+        src.x = xT; src.tp = true; src.idx = idx; src.w = w; src.bias = bias; src.N = d.N; src.L = d.L; src.K = d.K;
+        FFI_TRY(launch_topk_select(tc, d.B, *tk, src, s));
     }
     if (epi != kEpiLossGrad && epi != kEpiLossGradAndScores) return FFI_OK;
     // the listed label positions: from the score matrix when it was written, else recomputed from x ([N,B] here)
@@ -678,7 +669,7 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
 int launch_forward(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                    hipStream_t s) {
     // (the kernel reaches the 32 rows of out of a batch tile through 32-bit byte offsets)
-    if (tile_path_fits(d.N) && d.L < (1 << 25)) return forward_tiles(x, idx, w, bias, out, nullptr, kEpiScores, nullptr, nullptr, d, s);
+    if (tile_path_fits(d.N) && d.L < (1 << 25) && !few_samples(d)) return forward_tiles(x, idx, w, bias, out, nullptr, kEpiScores, nullptr, nullptr, d, s);
     return launch_forward_wide(x, idx, w, bias, out, d, s);
 }
 
@@ -698,13 +689,12 @@ int launch_forward_loss(const float* x, const int32_t* idx, const float* w, cons
 
 int launch_forward_topk(const float* x, const int32_t* idx, const float* w, const float* bias, float* scores, const TopkArgs& tk,
                         const Dims& d, hipStream_t s) {
-    if (tile_path_fits(d.N) && d.L < (1 << 25))
+    if (tile_path_fits(d.N) && d.L < (1 << 25) && (scores != nullptr || !few_samples(d)))
         return forward_tiles(x, idx, w, bias, scores, nullptr, scores ? kEpiScores : kEpiNone, nullptr, &tk, d, s);
-    // wide inputs: the score matrix (the caller's, or a workspace), then its top-k
-    float* sc = scores;
-    if (sc == nullptr) FFI_TRY(workspace_get(s, kWsScores, (size_t)d.B * d.L * sizeof(float), (void**)&sc));
-    FFI_TRY(launch_forward_wide(x, idx, w, bias, sc, d, s));
-    return launch_topk_f32(sc, d.B, d.L, tk.k, tk.values, tk.indices, s);
+    // wide inputs: candidates as the scores are formed, or the score matrix the caller wants, then its top-k
+    if (scores == nullptr) return launch_forward_topk_sliced(x, idx, w, bias, false, tk, d, s);
+    FFI_TRY(launch_forward_wide(x, idx, w, bias, scores, d, s));
+    return launch_topk_f32(scores, d.B, d.L, tk.k, tk.values, tk.indices, s);
 }
 
 // ---- forward pass for callers that cannot allocate ------------------------------------------------

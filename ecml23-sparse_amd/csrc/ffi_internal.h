@@ -30,7 +30,7 @@ struct Options {
     int fwd_lane64 = 0;             // -1: never the 64-sample forward kernel
     int plan_weights_in_lds = 0;    // -1: never / 1: whenever the tile fits
     int workgroups_per_cu = 0;      // upper limit for the kernel that walks a tiled plan
-    int wide_ranges = 0;            // column ranges of the sliced forward kernel
+    int wide_phases = 0;            // -1: never / 1: wherever it can: the forward kernel in phases for wide inputs
     int plan_sorted_columns = 0;    // -1: never / 1: always (in the weights-in-LDS form) the plans that hand the columns to the walking kernel's threads tile by tile, by length
 };
 extern Options g_options;
@@ -75,8 +75,6 @@ int device_cu_count();
 // inference variant: bf16 features / weights (raw 16-bit patterns), fp32 accumulation
 int launch_forward_bf16(const unsigned short* features, const int32_t* idx, const unsigned short* w, float* out,
                         const Dims& d, hipStream_t s);
-int launch_forward_topk_bf16(const unsigned short* features, const int32_t* idx, const unsigned short* w, float* values,
-                             int32_t* indices, int k, const Dims& d, hipStream_t s);
 int launch_topk_f32(const float* scores, int B, int L, int k, float* values, int32_t* indices, hipStream_t s);
 
 // dst[c][r] = src[r][c] for a row-major [rows, cols] matrix.
@@ -133,25 +131,43 @@ int launch_forward_loss(const float* x, const int32_t* idx, const float* w, cons
 // forward pass with per-sample top-k; the score matrix is written only if `scores` is given
 int launch_forward_topk(const float* x, const int32_t* idx, const float* w, const float* bias, float* scores, const TopkArgs& tk,
                         const Dims& d, hipStream_t s);
-// Candidate lists for a threshold-based top-k: count[B] appended entries, cand_val / cand_idx [B][kTopkCap].
-constexpr int kTopkCap = 8192;          // candidate slots per sample (a multiple of 8)
-int launch_topk_candidates_init(int* count, int* cand_idx, int B, int cap, hipStream_t s);
+int launch_forward_wide_bf16(const unsigned short* x, const int32_t* idx, const unsigned short* w, float* out, const Dims& d, hipStream_t s);
+int launch_forward_topk_wide_bf16(const unsigned short* x, const int32_t* idx, const unsigned short* w, const TopkArgs& tk, const Dims& d, hipStream_t s);
+// Top-k by a threshold (ffi_topk.hip): scores of a sample of the labels, the threshold of every sample of the batch, and the
+// candidates that reach it.  In a workspace of topk_candidate_bytes.
+constexpr int kTopkCap = 8192;          // candidate slots per sample
+constexpr int kTopkCountStep = 32;      // ints between the samples' counters: a cache line each
+struct TopkCandidates {
+    float* sample;     // [B][S]
+    float* tau;        // [B]
+    int* count;        // [B] candidates appended so far (may run past the cap: the list is then incomplete)
+    float* val;        // [B][kTopkCap]
+    int* idx;
+};
+size_t topk_candidate_bytes(int B, int sample);
+TopkCandidates topk_candidates_at(void* ws, int B, int sample);
+// tau and count from sample scores: scores[b * row + i * step], i < S
+int launch_topk_threshold(const float* scores, size_t row, int step, int S, int k, const TopkCandidates& c, int B, hipStream_t s);
 // Where the scores of a whole row come from when a sample's candidate list has overflowed: the score matrix [B,L],
-// or (scores == null) the layer itself, features as xT [N][B].
+// or (scores == null) the layer itself.
 struct TopkRowSource {
     const float* scores = nullptr;
-    const float* xT = nullptr;
+    const void* x = nullptr;
     const int32_t* idx = nullptr;
-    const float* w = nullptr;
+    const void* w = nullptr;
     const float* bias = nullptr;
     int N = 0, L = 0, K = 0;
+    bool tp = false, bf16 = false;
 };
-// the k best candidates of every sample; a sample whose count exceeds cap is answered from its whole row (src)
-int launch_topk_candidates_select(const float* cand_val, const int* cand_idx, const int* count, int B, int cap, int k,
-                                  float* values, int32_t* indices, hipStream_t s, const TopkRowSource& src);
-// the k best of nlists * 8 (score, label) candidates per sample (label -1 = empty slot)
-int launch_topk_merge(const float* part_val, const int* part_idx, int B, int nlists, int k, float* values, int32_t* indices,
-                      hipStream_t s);
+// the k best candidates of every sample; a sample whose count exceeds the cap is answered from its whole row (src)
+int launch_topk_select(const TopkCandidates& c, int B, const TopkArgs& tk, const TopkRowSource& src, hipStream_t s);
+
+// ---- forward pass over sample slices (ffi_sliced.hip): any shape, fp32 or bf16 ------------------------------------
+// top-k without the score matrix
+int launch_forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, bool bf16, const TopkArgs& tk, const Dims& d,
+                               hipStream_t s);
+// whether the narrow forward pass (scores, top-k) of so few samples is better off there than on a 32-sample tile
+bool few_samples(const Dims& d);
 
 // ---- backward pass over the non-zero entries of out_grad only (ffi_sparse_grad.hip) -------------
 // words[t][j]: bit i set <=> out_grad[32 t + i, j] may be non-zero

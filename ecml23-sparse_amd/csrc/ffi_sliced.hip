@@ -107,10 +107,15 @@ template <int GL> struct SlicedShape {
 __host__ __device__ constexpr int list_stride(int chunk) { return chunk + 2; }
 constexpr unsigned kNoRow = 0xffffff00u;
 
+typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
+
 template <bool BF16> struct LaneAcc;
 template <> struct LaneAcc<false> {
+    using Element = float;
     static constexpr int kSamples = 4;
     float a[4];
+    __device__ __forceinline__ void add2(uint4 x, uint4 y, unsigned wx, unsigned wy) { add(x, wx); add(y, wy); }
+    __device__ __forceinline__ void add_pair(uint4 x, uint4 y, const unsigned* w) { add(x, w[0]); add(y, w[1]); }
     __device__ __forceinline__ void add(uint4 x, unsigned w) {
         const float wv = __uint_as_float(w);
         a[0] = fmaf(wv, __uint_as_float(x.x), a[0]); a[1] = fmaf(wv, __uint_as_float(x.y), a[1]);
@@ -118,24 +123,64 @@ template <> struct LaneAcc<false> {
     }
 };
 template <> struct LaneAcc<true> {
+    using Element = unsigned short;
     static constexpr int kSamples = 8;
     float a[8];
-    __device__ __forceinline__ void add(uint4 x, unsigned w) {
-        const float wv = __uint_as_float(w);
-        const unsigned v[4] = {x.x, x.y, x.z, x.w};
+    // two connections at a time: their values of a sample side by side, one dot product with both weights (two instructions
+    // per multiply-add where unpacking to fp32 takes four; the products are exact either way)
+    __device__ __forceinline__ void add2(uint4 x, uint4 y, unsigned wx, unsigned wy) {
+        const unsigned w = __builtin_amdgcn_perm(wy, wx, 0x07060302u);
+        add_pair(x, y, &w);
+    }
+    __device__ __forceinline__ void add_pair(uint4 x, uint4 y, const unsigned* w) {
+        const bf16_pair wv = __builtin_bit_cast(bf16_pair, *w);
+        const unsigned u[4] = {x.x, x.y, x.z, x.w}, v[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            a[2 * i] = fmaf(wv, __uint_as_float(v[i] << 16), a[2 * i]);
-            a[2 * i + 1] = fmaf(wv, __uint_as_float(v[i] & 0xffff0000u), a[2 * i + 1]);
+            a[2 * i] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16_pair, __builtin_amdgcn_perm(v[i], u[i], 0x05040100u)), wv, a[2 * i], false);
+            a[2 * i + 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16_pair, __builtin_amdgcn_perm(v[i], u[i], 0x07060302u)), wv, a[2 * i + 1], false);
         }
     }
 };
+
+// Where a forward kernel that keeps no scores puts those at or above their sample's threshold.
+struct TopkSink {
+    const float* tau;              // [B]; null: the kernel stores scores
+    int* count;                    // [B] entries appended
+    float* val;                    // [B][cap]
+    int* idx;
+    int cap;
+};
+
+// The lane's scores of label j for samples b0 ...: few reach their threshold, so each takes its place with an atomic.
+template <int PER>
+__device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&a)[PER], const float (&tau)[PER], int b0, int j, bool valid) {
+    bool hit = false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) hit |= a[i] >= tau[i];
+    if (!valid || !hit) return;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (a[i] >= tau[i]) {
+            const int slot = atomicAdd(&sink.count[(size_t)(b0 + i) * kTopkCountStep], 1);
+            if (slot < sink.cap) {
+                sink.val[(size_t)(b0 + i) * sink.cap + slot] = a[i];
+                sink.idx[(size_t)(b0 + i) * sink.cap + slot] = j;
+            }
+        }
+    }
+}
+template <int PER>
+__device__ __forceinline__ void topk_thresholds(const TopkSink& sink, int b0, int B, float (&tau)[PER]) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) tau[i] = b0 + i < B ? sink.tau[b0 + i] : __builtin_inff();
+}
 
 template <int GL, bool BF16, int SLICES, bool QUADS>
 __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __restrict__ table, const int32_t* __restrict__ idx,
                                                                 const void* __restrict__ w, const float* __restrict__ bias,
                                                                 float* __restrict__ out, int B, int N, int L, int K, int slices, int chunk,
-                                                                int label_blocks, int units, int add_to_out) {
+                                                                int label_blocks, int units, const TopkSink sink) {
     using S = SlicedShape<GL>;
     constexpr int kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer;
     constexpr unsigned kRow = GL * 16u;
@@ -253,16 +298,34 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
                     for (int v = 0; v < kSlInflight; ++v)
                         x[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc[p], ((v & 1) ? e[v / 2].z : e[v / 2].x) + lane_off, 0, 0));
 #pragma unroll
-                    for (int v = 0; v < kSlInflight; ++v) acc[q][p].add(x[v], (v & 1) ? e[v / 2].w : e[v / 2].y);
+                    for (int v = 0; v < kSlInflight / 2; ++v) acc[q][p].add2(x[2 * v], x[2 * v + 1], e[v].y, e[v].w);
                 }
             }
             if (last) break;
             k0 += chunk;
         }
     }
+    if (sink.tau != nullptr) {
+#pragma unroll
+        for (int p = 0; p < SLICES; ++p) {
+            const int b0 = (slice0 + p) * kSl + sub * kPer;                // (beyond the last slice: no threshold is reached)
+            float tau[kPer];
+            topk_thresholds(sink, b0, B, tau);
+#pragma unroll
+            for (int q = 0; q < S::kRounds; ++q) {
+                const int j = first_label(q) + grp;
+                if (bias != nullptr) {
+                    const float bj = bias[min(j, L - 1)];
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) acc[q][p].a[i] += bj;
+                }
+                topk_append(sink, acc[q][p].a, tau, b0, j, j < L);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int p = 0; p < SLICES; ++p) {
-        if (slice0 + p >= slices) break;
         if (p > 0) __syncthreads();
 #pragma unroll
         for (int q = 0; q < S::kRounds; ++q)
@@ -271,32 +334,219 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
                 tile[(sub * kPer + i) * (S::kLabels + 1) + q * S::kRound + wave * S::kGroups + grp] = acc[q][p].a[i];
         __syncthreads();
         // rows of out, 64 labels (256 bytes) per wavefront and step
-        const int b0 = (slice0 + p) * kSl, nb = min(kSl, B - b0);
+        const int b0 = (slice0 + p) * kSl, nb = min(kSl, B - b0);         // (<= 0 beyond the last slice)
         constexpr int kCols = S::kLabels / 64;
         for (int e = wave; e < nb * kCols; e += kSlThreads / 64) {
             const int bb = e / kCols, jl = (e - bb * kCols) * 64 + lane, j = j0 + jl;
             if (j < L) {
                 const size_t at = (size_t)(b0 + bb) * L + j;
                 float v = tile[bb * (S::kLabels + 1) + jl];
-                if (add_to_out) v += out[at];
-                else if (bias != nullptr) v += bias[j];
+                if (bias != nullptr) v += bias[j];
                 __builtin_nontemporal_store(v, out + at);     // (past the L2, which the tables need: 435 -> 371 us at 128 x 4,096 x 670,000 x 32)
             }
         }
     }
 }
 
+// ---- forward, slice in LDS ----------------------------------------------------------------------------------------
+// For slices that fit in LDS beside the lists: narrow inputs with few samples or in bf16.  The workgroup brings its slice, then
+// its wavefronts take blocks of consecutive labels (every row_step-th row of the layer) -- one round of lane groups after the other, as in fwd_sliced_kernel,
+// the rows read from LDS -- and write their rows of out in pieces of that many labels.
+//
+// What bounds it: for one to four samples the stream of ids and weights from memory; from there on LDS delivery (a row of
+// 16 GL bytes and half a list entry of 16 per connection and lane group).
+typedef unsigned lds_v4u __attribute__((ext_vector_type(4)));
+constexpr int kLdThreads = 1024;
+constexpr size_t kLdBudget = 160 * 1024 - 512;
+
+template <int GL> struct LdsShape {
+    static constexpr int kGroups = 64 / GL;
+    static constexpr int kRounds = GL / 2;
+    static constexpr int kWaveLabels = kGroups * kRounds;                 // 32
+    static constexpr int kChunk = GL == 8 ? 32 : 16;
+    static constexpr int kQuads = (kGroups * kChunk + 255) / 256;
+    static constexpr int kStride = kChunk + 2;
+    static constexpr int kWaveBytes = kGroups * kStride * 8;              // (also holds 8 samples of a wavefront's labels)
+};
+template <int GL> inline size_t lds_kernel_bytes(int N) { return (size_t)(N + 1) * GL * 16 + (size_t)(kLdThreads / 64) * LdsShape<GL>::kWaveBytes; }
+
+template <int GL, bool BF16, bool QUADS>
+__global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restrict__ features, const int32_t* __restrict__ idx,
+                                                             const void* __restrict__ w, const float* __restrict__ bias,
+                                                             float* __restrict__ out, int B, int N, int L, int K, int tp, int row_step,
+                                                             int slices, int streams, int chunk, const TopkSink sink) {
+    using S = LdsShape<GL>;
+    constexpr int kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer, kWaves = kLdThreads / 64;
+    constexpr unsigned kRow = GL * 16u;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int u = xcd_contiguous_block(blockIdx.x, gridDim.x);            // (the slices of a stream share ids and weights in an L2)
+    const int slice = u % slices, stream = u / slices;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane & (GL - 1), grp = lane / GL;
+    {
+        // four samples of a column per thread and step: from a row of [N,B], or from four rows of [B,N]
+        using T = typename LaneAcc<BF16>::Element;
+        const T* x = static_cast<const T*>(features);
+        Quad<T>* dst = reinterpret_cast<Quad<T>*>(smem);
+        constexpr int kQ = kSl / 4;
+#pragma unroll 4
+        for (int e = threadIdx.x; e < N * kQ; e += kLdThreads) {
+            const int n = tp ? e / kQ : e % N, c = tp ? e % kQ : e / N;
+            Quad<T> q;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int b = slice * kSl + 4 * c + i;
+                const size_t at = tp ? (size_t)n * B + min(b, B - 1) : (size_t)min(b, B - 1) * N + n;
+                q.v[i] = b < B ? x[at] : (T)0;
+            }
+            dst[n * kQ + c] = q;
+        }
+        if (threadIdx.x < GL) reinterpret_cast<uint4*>(smem)[N * GL + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);    // what entries behind a list's end name
+    }
+    __syncthreads();
+    unsigned char* const mine = smem + (size_t)(N + 1) * kRow + (size_t)wave * S::kWaveBytes;
+    uint2* list = reinterpret_cast<uint2*>(mine);
+    // (raw LDS addresses: what a column id beyond the slice names is outside the LDS and reads as zero, or some of the LDS)
+    const unsigned rows = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem + (unsigned)sub * 16u;
+    const unsigned no_row = (unsigned)N * kRow;
+    const unsigned* w32 = reinterpret_cast<const unsigned*>(w);
+    const unsigned short* w16 = reinterpret_cast<const unsigned short*>(w);
+    const int blocks = (L + S::kWaveLabels - 1) / S::kWaveLabels, step = streams * kWaves;
+    const int b0 = slice * kSl, nb = min(kSl, B - b0);
+    float tau[kPer];
+    if (sink.tau != nullptr) topk_thresholds(sink, b0 + sub * kPer, B, tau);
+
+    uint4 ids[S::kQuads], ws[S::kQuads];
+    auto place = [&](unsigned f, int n, int& l, int& k) {
+        l = (int)((f * (65536u / (unsigned)n + 1u)) >> 16);               // f / n for f < 1,024 and n <= 32
+        k = (int)f - l * n;
+    };
+    auto fetch = [&](int blk, int q, int k0) {
+        const int kc = min(chunk, K - k0), j = blk * S::kWaveLabels + q * S::kGroups;
+#pragma unroll
+        for (int v = 0; v < S::kQuads; ++v) {
+            int l, k;
+            if (QUADS) {
+                place((unsigned)(64 * v + lane), kc / 4, l, k);
+                const size_t at = (size_t)min(j + min(l, S::kGroups - 1), L - 1) * row_step * K + k0 + 4 * k;
+                ids[v] = *reinterpret_cast<const uint4*>(idx + at);
+                if (BF16) {
+                    const uint2 h = *reinterpret_cast<const uint2*>(w16 + at);
+                    ws[v] = make_uint4(h.x << 16, h.x & 0xffff0000u, h.y << 16, h.y & 0xffff0000u);
+                } else {
+                    ws[v] = *reinterpret_cast<const uint4*>(w32 + at);
+                }
+            } else {
+                unsigned* id4 = &ids[v].x;
+                unsigned* w4 = &ws[v].x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    place((unsigned)(64 * (4 * v + e) + lane), kc, l, k);
+                    const size_t at = (size_t)min(j + min(l, S::kGroups - 1), L - 1) * row_step * K + k0 + k;
+                    id4[e] = (unsigned)idx[at];
+                    w4[e] = BF16 ? (unsigned)w16[at] << 16 : w32[at];
+                }
+            }
+        }
+    };
+    auto put = [&](int k0) {
+        const int kc = min(chunk, K - k0);
+#pragma unroll
+        for (int v = 0; v < S::kQuads; ++v) {
+            int l, k;
+            if (QUADS) {
+                place((unsigned)(64 * v + lane), kc / 4, l, k);
+                if (l < S::kGroups) {
+                    uint4* p = reinterpret_cast<uint4*>(list + l * S::kStride + 4 * k);
+                    p[0] = make_uint4(ids[v].x * kRow, ws[v].x, ids[v].y * kRow, ws[v].y);
+                    p[1] = make_uint4(ids[v].z * kRow, ws[v].z, ids[v].w * kRow, ws[v].w);
+                }
+            } else {
+                const unsigned id4[4] = {ids[v].x, ids[v].y, ids[v].z, ids[v].w}, w4[4] = {ws[v].x, ws[v].y, ws[v].z, ws[v].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    place((unsigned)(64 * (4 * v + e) + lane), kc, l, k);
+                    if (l < S::kGroups) list[l * S::kStride + k] = make_uint2(id4[e] * kRow, w4[e]);
+                }
+            }
+        }
+        if ((kc & 3) != 0 && lane < S::kGroups)                           // the walk takes four at a time
+            for (int k = kc; k < (kc + 3) / 4 * 4; ++k) list[lane * S::kStride + k] = make_uint2(no_row, 0u);
+    };
+    const uint4* mylist = reinterpret_cast<const uint4*>(list + grp * S::kStride);
+    int blk = stream * kWaves + wave;
+    if (blk >= blocks) return;
+    fetch(blk, 0, 0);
+    for (; blk < blocks; blk += step) {
+        LaneAcc<BF16> acc[S::kRounds];
+        const int jb = blk * S::kWaveLabels;
+#pragma unroll
+        for (int q = 0; q < S::kRounds; ++q) {
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) acc[q].a[i] = 0.f;
+            for (int k0 = 0; k0 < K; k0 += chunk) {
+                __builtin_amdgcn_wave_barrier();                          // (the list is the wavefront's own, and LDS serves it in order)
+                put(k0);
+                if (k0 + chunk < K) fetch(blk, q, k0 + chunk);
+                else if (q + 1 < S::kRounds) fetch(blk, q + 1, 0);
+                else fetch(min(blk + step, blocks - 1), 0, 0);
+                __builtin_amdgcn_wave_barrier();
+                const int n = min(chunk, K - k0);
+#pragma unroll 2
+                for (int i = 0; i < n; i += 4) {
+                    uint4 e[2], x[4];
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) e[v] = mylist[i / 2 + v];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) x[v] = __builtin_bit_cast(uint4, *(const lds_v4u __attribute__((address_space(3)))*)(size_t)(rows + ((v & 1) ? e[v / 2].z : e[v / 2].x)));
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) acc[q].add2(x[2 * v], x[2 * v + 1], e[v].y, e[v].w);
+                }
+            }
+        }
+        if (sink.tau != nullptr) {
+#pragma unroll
+            for (int q = 0; q < S::kRounds; ++q) {
+                const int j = jb + q * S::kGroups + grp;
+                if (bias != nullptr) {
+                    const float bj = bias[(size_t)min(j, L - 1) * row_step];
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) acc[q].a[i] += bj;
+                }
+                topk_append(sink, acc[q].a, tau, b0 + sub * kPer, j, j < L);
+            }
+            continue;
+        }
+        float* tile = reinterpret_cast<float*>(mine);                     // eight samples (or what a lane holds of four) x the labels
+        constexpr int kPitch = S::kWaveLabels + 1, kTake = kSl < 8 ? kSl : 8, kRowsPerStep = 64 / S::kWaveLabels;
+        static_assert(kTake * kPitch * 4 <= S::kWaveBytes, "the tile lies in the list's place");
+        const int jl = lane % S::kWaveLabels, j = jb + jl;
+        const float bj = (bias != nullptr && j < L) ? bias[(size_t)j * row_step] : 0.f;
+        for (int s0 = 0; s0 < nb; s0 += kTake) {
+            __builtin_amdgcn_wave_barrier();
+            if (sub * kPer >= s0 && sub * kPer < s0 + kTake) {
+#pragma unroll
+                for (int q = 0; q < S::kRounds; ++q)
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) tile[(sub * kPer + i - s0) * kPitch + q * S::kGroups + grp] = acc[q].a[i];
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int e = lane / S::kWaveLabels; e < kTake && s0 + e < nb; e += kRowsPerStep)
+                if (j < L) out[(size_t)(b0 + s0 + e) * L + j] = bias != nullptr ? tile[e * kPitch + jl] + bj : tile[e * kPitch + jl];
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 // ---- rows put in order of column range ----------------------------------------------------------------------------
 // Every row's connections in the order of `ranges` equal column ranges, positions ascending inside a range, padded to whole
-// quads with connections that name no column (the gather of one returns zero without touching memory).  The row is then
-// cut into `ranges` parts of equal length, quads [Q r / ranges, Q (r + 1) / ranges) of its Q, and part r of all rows is
-// stored in one piece.  Equal parts and not the ranges themselves: the lists of the lane groups stay equally long, and the
-// few connections that a row has too many or too few (5 % at fan-in 72 and two ranges) merely miss the L2.
-// A lane holds four entries, a row a group of Q neighbouring lanes: Q <= 64.  Both sides go through the wavefront's part
-// of LDS, so that memory is read and written in whole lines.
-constexpr int kMaxRanges = 4;
+// octs with connections that name no column (the gather of one returns zero without touching memory).  Oct r of all rows --
+// part r -- is stored in one piece.  Octs of the ordered row and not the ranges themselves: the lists of the lane groups are
+// equally long, and the columns of a part still lie close together.
+// A lane holds four entries, a row a group of 2 Q neighbouring lanes: at most 256 connections.  Both sides go through the
+// wavefront's part of LDS, so that memory is read and written in whole lines.
+constexpr int kMaxRanges = 16;
 constexpr int kMaxRangedFanIn = 256;
-__host__ __device__ constexpr int part_begin(int quads, int ranges, int r) { return quads * r / ranges; }
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __restrict__ idx, const void* __restrict__ w,
@@ -306,7 +556,7 @@ __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __res
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned* sid = mem[wave][0];
     unsigned* sw = mem[wave][1];
-    const int gs = (K + 3) / 4, rows = 64 / gs;                          // lanes per row, rows per wavefront
+    const int octs = (K + 7) / 8, gs = 2 * octs, rows = 64 / gs;         // lanes per row, rows per wavefront
     const long long row0 = ((long long)blockIdx.x * 4 + wave) * rows;
     const int nrows = (int)min((long long)rows, (long long)L - row0);    // (may be <= 0)
     const int total = nrows * K;
@@ -352,12 +602,10 @@ __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __res
             if (range[e] != 0xffu) { sid[4 * r * gs + to[e]] = id[e]; sw[4 * r * gs + to[e]] = wv[e]; }
     }
     __builtin_amdgcn_wave_barrier();
-    for (int q = 0; q < ranges; ++q) {
-        const int begin_q = part_begin(gs, ranges, q), n = part_begin(gs, ranges, q + 1) - begin_q;
-        if (n == 0) continue;
-        const size_t base = (size_t)begin_q * L + (size_t)row0 * n;      // (in quads)
-        for (int f = lane; f < nrows * n; f += 64) {
-            const int fr = f / n, from = fr * gs + begin_q + f - fr * n;
+    for (int q = 0; q < octs; ++q) {
+        const size_t base = (size_t)q * 2 * L + (size_t)row0 * 2;        // (in quads)
+        for (int f = lane; f < nrows * 2; f += 64) {
+            const int from = (f >> 1) * gs + 2 * q + (f & 1);
             reinterpret_cast<uint4*>(idx_out)[base + f] = reinterpret_cast<const uint4*>(sid)[from];
             const uint4 v = reinterpret_cast<const uint4*>(sw)[from];
             if (BF16) reinterpret_cast<uint2*>(w_out)[base + f] = make_uint2(v.x | v.y << 16, v.z | v.w << 16);
@@ -366,15 +614,175 @@ __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __res
     }
 }
 
+// ---- forward in phases --------------------------------------------------------------------------------------------
+// For slices that do not fit an XCD's L2: a workgroup of 16 wavefronts takes 128 M labels -- their sums stay in registers -- and
+// goes through the parts of their rows (above: one oct of connections per label and part) in order, a barrier behind each.
+// All workgroups of an XCD begin at the same time and do the same work, so the gathers of a phase hit the few MB of the
+// slice that its part of the rows names.
+//
+// The gathers of a step (eight labels, an oct each) are issued before the sums of the step before them, so that a wavefront
+// always has eight in flight.  The lists of a part are written two parts, its ids and weights asked for three parts ahead of
+// their use at the latest: loads return in order, and a load from memory in front of the gathers would hold them up.
+//
+// What bounds it: L2 delivery, as in fwd_sliced_kernel.
+constexpr int kPhThreads = 1024;
+
+template <bool BF16> struct PhasedShape {
+    static constexpr int kM = 4;                                  // labels per lane group: 64 lanes bring the 32 labels' octs, a quad each
+    static constexpr int kWaveLabels = 8 * kM;
+    static constexpr int kLabels = kWaveLabels * (kPhThreads / 64);
+    static constexpr int kOctWords = 5;                           // 16-byte words per label in LDS: four, and one against bank conflicts
+    static constexpr size_t kListBytes = (size_t)2 * kLabels * kOctWords * 16;
+};
+
+template <bool BF16>
+__global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __restrict__ table, const unsigned* __restrict__ idx,
+                                                                const void* __restrict__ w, const float* __restrict__ bias,
+                                                                float* __restrict__ out, int B, int N, int L, int octs, int label_blocks,
+                                                                int units, const TopkSink sink) {
+    using S = PhasedShape<BF16>;
+    constexpr int GL = 8, kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer, M = S::kM;
+    constexpr unsigned kRow = 128u;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int u = xcd_unit(blockIdx.x, units);
+    if (u < 0) return;
+    const int slice = u / label_blocks;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane & (GL - 1), grp = lane / GL;
+    const int jw = (u % label_blocks) * S::kLabels + wave * S::kWaveLabels;             // first label of this wavefront
+    uint4* const lists = reinterpret_cast<uint4*>(smem) + wave * (2 * S::kWaveLabels * S::kOctWords);
+    const size_t slice_bytes = (size_t)N * kRow;
+    const buffer_rsrc rows = make_rsrc((const char*)table + (size_t)slice * slice_bytes, slice_bytes);
+    const unsigned lane_off = (unsigned)sub * 16u;
+    LaneAcc<BF16> acc[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) acc[m].a[i] = 0.f;
+
+    // lane f brings quad f & 1 of label f / 2 (of every 32 labels).  Labels behind the last read zeros: a gather of row 0 with
+    // weight zero.
+    uint4 ids, ws;
+    auto fetch = [&](int r) {
+        const size_t base = (size_t)min(r, octs - 1) * 8 * L;                            // (behind the last part: the last again)
+        const buffer_rsrc ri = make_rsrc(idx + base, (size_t)L * 32), rw = make_rsrc((const char*)w + base * (BF16 ? 2 : 4), (size_t)L * (BF16 ? 16 : 32));
+        ids = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ri, lane * 16u, (unsigned)jw * 32u, 0));
+        if (BF16) {
+            const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rw, lane * 8u, (unsigned)jw * 16u, 0));
+            ws.x = h.x; ws.y = h.y;
+        } else {
+            ws = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, (unsigned)jw * 32u, 0));
+        }
+    };
+    auto put = [&](int r) {
+        uint4* list = lists + (r & 1) * (S::kWaveLabels * S::kOctWords) + (lane >> 1) * S::kOctWords + (lane & 1) * 2;
+        if (BF16) {                                      // (the weights of two connections share a word)
+            list[0] = make_uint4(ids.x * kRow, ids.y * kRow, ids.z * kRow, ids.w * kRow);
+            reinterpret_cast<uint2*>(list)[2] = make_uint2(ws.x, ws.y);
+        } else {
+            list[0] = make_uint4(ids.x * kRow, ws.x, ids.y * kRow, ws.y);
+            list[1] = make_uint4(ids.z * kRow, ws.z, ids.w * kRow, ws.w);
+        }
+    };
+    uint4 x[2][8];
+    constexpr int kWt = BF16 ? 4 : 8;
+    unsigned wt[2][kWt];
+    auto gather = [&](int r, int m, uint4 (&xs)[8], unsigned (&wv)[kWt]) {
+        const uint4* list = lists + (r & 1) * (S::kWaveLabels * S::kOctWords) + (m * 8 + grp) * S::kOctWords;
+        unsigned at[8];
+        if (BF16) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint4 e = list[2 * h];
+                const uint2 f = reinterpret_cast<const uint2*>(list + 2 * h)[2];
+                at[4 * h] = e.x; at[4 * h + 1] = e.y; at[4 * h + 2] = e.z; at[4 * h + 3] = e.w;
+                wv[2 * h] = f.x; wv[2 * h + 1] = f.y;
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const uint4 e = list[v];
+                at[2 * v] = e.x; at[2 * v + 1] = e.z;
+                wv[(2 * v) % kWt] = e.y; wv[(2 * v + 1) % kWt] = e.w;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 8; ++v)
+            xs[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, at[v] + lane_off, 0, 0));
+    };
+    // (the lists are the wavefront's own, and LDS serves it in order)
+    fetch(0);
+    put(0);
+    fetch(1);
+    __builtin_amdgcn_wave_barrier();
+    gather(0, 0, x[0], wt[0]);
+    for (int r = 0; r < octs; ++r) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            if (m == 0) {
+                put(r + 1);
+                __builtin_amdgcn_wave_barrier();
+            }
+            if (m + 1 < M) gather(r, m + 1, x[(m + 1) & 1], wt[(m + 1) & 1]);
+            else gather(r + 1, 0, x[(m + 1) & 1], wt[(m + 1) & 1]);
+            if (m == 0) fetch(r + 2);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[m].add_pair(x[m & 1][2 * v], x[m & 1][2 * v + 1], &wt[m & 1][v * (kWt / 4)]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_barrier();                    // (for the pace: nothing is shared)
+    }
+    __syncthreads();
+    const int b0 = slice * kSl;
+    if (sink.tau != nullptr) {
+        float tau[kPer];
+        topk_thresholds(sink, b0 + sub * kPer, B, tau);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int j = jw + m * 8 + grp;
+            if (bias != nullptr) {
+                const float bj = bias[min(j, L - 1)];
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) acc[m].a[i] += bj;
+            }
+            topk_append(sink, acc[m].a, tau, b0 + sub * kPer, j, j < L);
+        }
+        return;
+    }
+    // a wavefront's labels are consecutive: rows of out leave in pieces of 8 M labels, through the wavefront's part of LDS
+    constexpr int kPitch = S::kWaveLabels + 1, kStep = 2 * S::kWaveLabels * S::kOctWords * 4 / kPitch;       // samples that fit there
+    float* tile = reinterpret_cast<float*>(lists);
+    const int nb = min(kSl, B - b0);
+    static_assert(kStep >= 8, "a lane's samples at a time");
+    constexpr int kTake = kStep >= kSl ? kSl : kStep >= kSl / 2 ? kSl / 2 : kSl / 4;
+    for (int s0 = 0; s0 < nb; s0 += kTake) {
+        __builtin_amdgcn_wave_barrier();
+        if (sub * kPer >= s0 && sub * kPer < s0 + kTake) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) tile[(sub * kPer + i - s0) * kPitch + m * 8 + grp] = acc[m].a[i];
+        }
+        __builtin_amdgcn_wave_barrier();
+        constexpr int kRowsPerStep = 64 / S::kWaveLabels;
+        const int jl = lane % S::kWaveLabels, j = jw + jl;
+        const float bj = (bias != nullptr && j < L) ? bias[j] : 0.f;
+        for (int e = lane / S::kWaveLabels; e < kTake && s0 + e < nb; e += kRowsPerStep)
+            if (j < L) __builtin_nontemporal_store(bias != nullptr ? tile[e * kPitch + jl] + bj : tile[e * kPitch + jl], out + (size_t)(b0 + s0 + e) * L + j);
+    }
+}
+
 struct FwdSliced {
-    const void* table;
+    const void* table;             // the slices; the caller's features where the kernel makes them in LDS
     const int32_t* idx;
     const void* w;
     const float* bias;
     float* out;
     int slices, per_group;         // slices; how many of them a workgroup serves with one list
-    int K;                         // connections per row
-    bool quads, add_to_out;
+    int row_step;                  // (kernel with the slice in LDS only) row of label j: j * row_step
+    bool quads;
+    TopkSink sink;
 };
 
 template <int GL, bool BF16, int SLICES>
@@ -383,17 +791,17 @@ int launch_fwd_sliced(const FwdSliced& a, const Dims& d, hipStream_t s) {
     const int label_blocks = (d.L + S::kLabels - 1) / S::kLabels, groups = (a.slices + SLICES - 1) / SLICES;
     if ((long long)label_blocks * groups > (1ll << 28)) return FFI_ERR_TOO_LARGE;
     const int units = label_blocks * groups;
-    const int chunks = (a.K + S::kChunk - 1) / S::kChunk;
-    const int chunk = ((a.K + chunks - 1) / chunks + 7) / 8 * 8;
+    const int chunks = (d.K + S::kChunk - 1) / S::kChunk;
+    const int chunk = ((d.K + chunks - 1) / chunks + 7) / 8 * 8;
     const size_t lds = (size_t)GL * LaneAcc<BF16>::kSamples * (S::kLabels + 1) * sizeof(float) / 16 * 16 + 16 +
                        (size_t)S::kRound * list_stride(chunk) * sizeof(uint2);
     const dim3 grid(xcd_grid(units)), block(kSlThreads);
     if (a.quads)
         hipLaunchKernelGGL((fwd_sliced_kernel<GL, BF16, SLICES, true>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L,
-                           a.K, a.slices, chunk, label_blocks, units, a.add_to_out ? 1 : 0);
+                           d.K, a.slices, chunk, label_blocks, units, a.sink);
     else
         hipLaunchKernelGGL((fwd_sliced_kernel<GL, BF16, SLICES, false>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L,
-                           a.K, a.slices, chunk, label_blocks, units, a.add_to_out ? 1 : 0);
+                           d.K, a.slices, chunk, label_blocks, units, a.sink);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
@@ -417,15 +825,113 @@ int launch_fwd_sliced_lanes(int gl, const FwdSliced& a, const Dims& d, hipStream
     }
 }
 
-// `rows`: [ids][weights], each 4 L quads long
-template <bool BF16>
-int launch_rows_by_range(const int32_t* idx, const void* w, unsigned* rows, int L, int K, int N, int ranges, hipStream_t s) {
-    const int quads = (K + 3) / 4, rows_per_block = 4 * (64 / quads);
-    const unsigned range_cols = (unsigned)((N + ranges - 1) / ranges);
-    hipLaunchKernelGGL((rows_by_range_kernel<BF16>), dim3((unsigned)((L + rows_per_block - 1) / rows_per_block)), dim3(256), 0, s, idx, w, rows,
-                       rows + (size_t)L * quads * 4, L, K, range_cols, ranges);
+template <int GL, bool BF16>
+int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
+    using S = LdsShape<GL>;
+    const int chunks = (d.K + S::kChunk - 1) / S::kChunk, chunk = ((d.K + chunks - 1) / chunks + 3) / 4 * 4;
+    const int blocks = (d.L + S::kWaveLabels - 1) / S::kWaveLabels, waves = kLdThreads / 64;
+    const int streams = std::max(1, std::min((blocks + waves - 1) / waves, device_cu_count() / a.slices));
+    const size_t lds = lds_kernel_bytes<GL>(d.N);
+    const dim3 grid((unsigned)(streams * a.slices)), block(kLdThreads);
+    if (a.quads) {
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lds_kernel<GL, BF16, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL((fwd_lds_kernel<GL, BF16, true>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0,
+                           a.row_step, a.slices, streams, chunk, a.sink);
+    } else {
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lds_kernel<GL, BF16, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL((fwd_lds_kernel<GL, BF16, false>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0,
+                           a.row_step, a.slices, streams, chunk, a.sink);
+    }
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
+}
+
+template <bool BF16>
+int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
+    using S = PhasedShape<BF16>;
+    const int octs = (d.K + 7) / 8, rows_per_block = 4 * (64 / (2 * octs)), value = BF16 ? 2 : 4;
+    const int ranges = std::min(kMaxRanges, octs);
+    // [ids][weights], part by part
+    unsigned* rows = nullptr;
+    FFI_TRY(workspace_get(s, kWsRows, (size_t)d.L * octs * 8 * (4 + value), (void**)&rows));
+    void* row_w = rows + (size_t)d.L * octs * 8;
+    hipLaunchKernelGGL((rows_by_range_kernel<BF16>), dim3((unsigned)((d.L + rows_per_block - 1) / rows_per_block)), dim3(256), 0, s, a.idx, a.w,
+                       rows, row_w, d.L, d.K, (unsigned)((d.N + ranges - 1) / ranges), ranges);
+    FFI_HIP_TRY(hipGetLastError());
+    const int label_blocks = (d.L + S::kLabels - 1) / S::kLabels, units = label_blocks * a.slices;
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_phased_kernel<BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kListBytes));
+    hipLaunchKernelGGL((fwd_phased_kernel<BF16>), dim3(xcd_grid(units)), dim3(kPhThreads), S::kListBytes, s, a.table, rows, row_w, a.bias, a.out,
+                       d.B, d.N, d.L, octs, label_blocks, units, a.sink);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
+// The phased kernel or the plain one, for slices of 128-byte rows.  Per label, in time of 1 TB/s; the rates are what the kernels
+// reach at 300,000 to 670,091 labels: plain 20 inside L2 and 5.8 over the share that misses it, in phases 18, ordering the rows
+// 3.2.  fp32, 128 samples, 65,536 columns, fan-in 72: 2.18 ms plain, 1.56 in phases; 32 samples, fan-in 32 there: 245 and 295 us;
+// bf16, 512 samples, 100,000 columns, fan-in 64: 4.1 and 2.6 ms.
+bool takes_phases(size_t slice_bytes, int gl, int slices, int K, int value_bytes) {
+    if (gl != 8 || K > kMaxRangedFanIn) return false;
+    if (g_options.wide_phases != 0) return g_options.wide_phases > 0;
+    if (K <= 8) return false;
+    const double gathered = 128.0 * slices * K, miss = std::max(0.0, 1.0 - (double)kXcdL2Bytes / (double)slice_bytes);
+    const double plain = gathered / (miss > 0.0 ? std::min(20.0, 5.8 / miss) : 20.0);
+    return gathered / 18.0 + 2.0 * K * (4 + value_bytes) / 3.2 < plain;
+}
+
+// How a forward pass over slices runs: lanes per row, number of slices, and whether a slice lies in LDS (then with as many
+// lanes per row as fit; eight otherwise for more than 16 (fp32) or 32 (bf16) samples).
+struct SlicedForm {
+    int gl, sl, slices;
+    bool in_lds;
+};
+template <bool BF16>
+SlicedForm sliced_form(int B, int N) {
+    constexpr int kPer = LaneAcc<BF16>::kSamples;
+    SlicedForm f;
+    f.gl = slice_lanes(B, kPer);
+    // (two lanes per row at least: with one the lists of a wavefront are as long as its ids are short of a line; one sample,
+    // 670,091 labels: 98 us against 51)
+    auto fits = [&](int gl) { return (gl == 8 ? lds_kernel_bytes<8>(N) : gl == 4 ? lds_kernel_bytes<4>(N) : lds_kernel_bytes<2>(N)) <= kLdBudget; };
+    f.in_lds = fits(std::max(f.gl, 2));
+    if (f.in_lds) f.gl = std::max(f.gl, 2);
+    else if (f.gl == 8 && fits(4)) { f.gl = 4; f.in_lds = true; }
+    f.sl = f.gl * kPer;
+    f.slices = (B + f.sl - 1) / f.sl;
+    return f;
+}
+
+// the features in slices, in the stream's workspace
+template <bool BF16>
+int make_table(const void* x, const Dims& d, hipStream_t s, const void** table) {
+    const SlicedForm f = sliced_form<BF16>(d.B, d.N);
+    if (f.in_lds) { *table = x; return FFI_OK; }
+    const size_t slice_bytes = (size_t)d.N * f.gl * 16;
+    if (slice_bytes >= 0xffffff00ull) return FFI_ERR_TOO_LARGE;
+    void* ws = nullptr;
+    FFI_TRY(workspace_get(s, kWsFeaturesT, slice_bytes * f.slices, &ws));
+    *table = ws;
+    if (BF16) return launch_slices((const unsigned short*)x, (unsigned short*)ws, d.N, d.B, f.sl, d.tp, s);
+    return launch_slices((const float*)x, (float*)ws, d.N, d.B, f.sl, d.tp, s);
+}
+
+template <bool BF16>
+int forward_wide(const void* table, const int32_t* idx, const void* w, const float* bias, float* out, const TopkSink& sink, const Dims& d,
+                 hipStream_t s, int row_step = 1) {
+    const SlicedForm f = sliced_form<BF16>(d.B, d.N);
+    const size_t slice_bytes = (size_t)d.N * f.gl * 16;
+    const bool quads = d.K % 4 == 0 && ((uintptr_t)idx & 15) == 0 && ((uintptr_t)w & (BF16 ? 7 : 15)) == 0;
+    const int per_group = (int)std::min<size_t>((size_t)f.slices, kXcdL2Bytes / slice_bytes);
+    const FwdSliced a{table, idx, w, bias, out, f.slices, per_group, row_step, quads, sink};
+    if (f.in_lds) {
+        switch (f.gl) {
+            case 2: return launch_fwd_lds<2, BF16>(a, d, s);
+            case 4: return launch_fwd_lds<4, BF16>(a, d, s);
+            default: return launch_fwd_lds<8, BF16>(a, d, s);
+        }
+    }
+    if (takes_phases(slice_bytes, f.gl, f.slices, d.K, BF16 ? 2 : 4)) return launch_fwd_phased<BF16>(a, d, s);
+    return launch_fwd_sliced_lanes<BF16>(f.gl, a, d, s);
 }
 
 }  // namespace
@@ -437,53 +943,80 @@ int launch_slices_bf16(const unsigned short* src, unsigned short* dst, int rows,
     return launch_slices(src, dst, rows, B, sl, tp, s);
 }
 
-// Passes over the columns, each over a range whose part of the slice fits an XCD's L2: they save what the gathers lose
-// outside L2, and cost the rows put in order first and, from the second pass on, a read and a write of the scores.  Per
-// label, in time of 1 TB/s; the rates are what the kernels reach at 300,000 to 670,091 labels: gathers 20 inside L2 (17 in
-// several passes), 5.8 over the share that misses it, ordering 3.6, scores 5.5.  128 samples, 65,536 columns, fan-in 72:
-// 2.26 ms in one pass, 1.73 in two; 32 samples and fan-in 32 there: 250 us in one, 320 in two.
-static int sliced_ranges(size_t slice_bytes, int B, int K, int value_bytes) {
-    if (K > kMaxRangedFanIn) return 1;
-    if (g_options.wide_ranges > 0) return g_options.wide_ranges;
-    int best = 1;
-    double best_cost = 1e30;
-    for (int r = 1; r <= kMaxRanges; ++r) {
-        const double part = (double)slice_bytes / r, miss = std::max(0.0, 1.0 - (double)kXcdL2Bytes / part);
-        const double inside = r > 1 ? 17.0 : 20.0, rate = miss > 0.0 ? std::min(inside, 5.8 / miss) : inside;
-        const double cost = (double)B * K * value_bytes / rate + (r > 1 ? (double)K * 2 * (4 + value_bytes) / 3.6 + 8.0 * B * (r - 1) / 5.5 : 0.0);
-        if (cost < best_cost) { best_cost = cost; best = r; }
-    }
-    return best;
-}
-
 int launch_forward_wide(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                         hipStream_t s) {
-    const int gl = slice_lanes(d.B, 4), sl = gl * 4, slices = (d.B + sl - 1) / sl;
-    const size_t slice_bytes = (size_t)d.N * sl * sizeof(float);
-    if (slice_bytes >= 0xffffff00ull) return FFI_ERR_TOO_LARGE;
-    float* table = nullptr;
-    FFI_TRY(workspace_get(s, kWsFeaturesT, slice_bytes * slices, (void**)&table));
-    FFI_TRY(launch_slices_f32(x, table, d.N, d.B, sl, d.tp, s));
-    const bool quads = d.K % 4 == 0 && (((uintptr_t)idx | (uintptr_t)w) & 15) == 0;
-    const int per_group = (int)std::min<size_t>((size_t)slices, kXcdL2Bytes / slice_bytes);
-    const int ranges = sliced_ranges(slice_bytes, d.B, d.K, 4);
-    FwdSliced a{table, idx, w, bias, out, slices, per_group, d.K, quads, false};
-    if (ranges == 1) return launch_fwd_sliced_lanes<false>(gl, a, d, s);
-    const int row_quads = (d.K + 3) / 4;
-    unsigned* rows = nullptr;
-    FFI_TRY(workspace_get(s, kWsRows, (size_t)d.L * row_quads * 32, (void**)&rows));
-    FFI_TRY(launch_rows_by_range<false>(idx, w, rows, d.L, d.K, d.N, ranges, s));
-    a.quads = true;
-    for (int r = 0; r < ranges; ++r) {
-        const int begin = part_begin(row_quads, ranges, r);
-        a.K = 4 * (part_begin(row_quads, ranges, r + 1) - begin);
-        if (a.K == 0) continue;
-        a.idx = (const int32_t*)rows + (size_t)begin * 4 * d.L;
-        a.w = rows + ((size_t)row_quads + begin) * 4 * d.L;
-        FFI_TRY(launch_fwd_sliced_lanes<false>(gl, a, d, s));
-        a.add_to_out = true;
+    const void* table = nullptr;
+    FFI_TRY(make_table<false>(x, d, s, &table));
+    return forward_wide<false>(table, idx, w, bias, out, TopkSink{}, d, s);
+}
+
+int launch_forward_bf16(const unsigned short* x, const int32_t* idx, const unsigned short* w, float* out, const Dims& d, hipStream_t s) {
+    const void* table = nullptr;
+    FFI_TRY(make_table<true>(x, d, s, &table));
+    return forward_wide<true>(table, idx, w, nullptr, out, TopkSink{}, d, s);
+}
+
+// Narrow inputs, fp32: up to 16 samples half or more of a 32-sample tile would be computed for nothing (768 x 670,091 x 32, one to
+// 16 samples: 58 -> 50 us, with top-k 110 -> 75; 100 x 500,000 x 17: 36 -> 28; 20 samples and more: no faster than the tile).
+bool few_samples(const Dims& d) { return d.B <= 16; }
+
+// ---- top-k without the scores -------------------------------------------------------------------------------------
+namespace {
+
+constexpr int kTopkSampleLabels = 16384;
+
+// the rows of every step-th label
+template <typename T>
+__global__ __launch_bounds__(256) void sample_rows_kernel(const int32_t* __restrict__ idx, const T* __restrict__ w, const float* __restrict__ bias,
+                                                          int32_t* __restrict__ idx_out, T* __restrict__ w_out, float* __restrict__ bias_out,
+                                                          int step, int K, int S) {
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t i = t / (unsigned)K;
+    if (i >= (size_t)S) return;
+    const size_t j = i * step, at = j * K + (t - i * K);
+    idx_out[t] = idx[at];
+    w_out[t] = w[at];
+    if (bias != nullptr && t == i * K) bias_out[i] = bias[j];
+}
+
+// The k-th best of a sample of the labels is a threshold that k labels reach; the same kernel scores the sample and all
+// labels, so that a label's score is the same number in both.
+template <bool BF16>
+int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, const TopkArgs& tk, const Dims& d, hipStream_t s) {
+    using T = typename LaneAcc<BF16>::Element;
+    const int step = std::max(1, d.L / kTopkSampleLabels), S = std::min(d.L, (d.L + step - 1) / step);
+    const size_t rows = (size_t)S * d.K, rows_bytes = (rows * (4 + sizeof(T)) + (size_t)S * 4 + 32) / 16 * 16;
+    const bool in_lds = sliced_form<BF16>(d.B, d.N).in_lds;
+    unsigned char* ws = nullptr;
+    FFI_TRY(workspace_get(s, kWsTopk, topk_candidate_bytes(d.B, S) + 16 + (in_lds ? 0 : rows_bytes), (void**)&ws));
+    const TopkCandidates c = topk_candidates_at(ws, d.B, S);
+    const void* table = nullptr;
+    FFI_TRY(make_table<BF16>(x, d, s, &table));
+    Dims ds = d;
+    ds.L = S;
+    if (in_lds) {
+        FFI_TRY(forward_wide<BF16>(table, idx, w, bias, c.sample, TopkSink{}, ds, s, step));
+    } else {
+        int32_t* sample_idx = reinterpret_cast<int32_t*>(ws + (topk_candidate_bytes(d.B, S) + 15) / 16 * 16);
+        T* sample_w = reinterpret_cast<T*>(sample_idx + (rows + 3) / 4 * 4);
+        float* sample_bias = reinterpret_cast<float*>(sample_w + (rows + 3) / 4 * 4);
+        hipLaunchKernelGGL(sample_rows_kernel<T>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, idx, (const T*)w, bias, sample_idx,
+                           sample_w, sample_bias, step, d.K, S);
+        FFI_HIP_TRY(hipGetLastError());
+        FFI_TRY(forward_wide<BF16>(table, sample_idx, sample_w, bias ? sample_bias : nullptr, c.sample, TopkSink{}, ds, s));
     }
-    return FFI_OK;
+    FFI_TRY(launch_topk_threshold(c.sample, (size_t)S, 1, S, tk.k, c, d.B, s));
+    FFI_TRY(forward_wide<BF16>(table, idx, w, bias, nullptr, TopkSink{c.tau, c.count, c.val, c.idx, kTopkCap}, d, s));
+    TopkRowSource src;
+    src.x = x; src.tp = d.tp; src.bf16 = BF16; src.idx = idx; src.w = w; src.bias = bias; src.N = d.N; src.L = d.L; src.K = d.K;
+    return launch_topk_select(c, d.B, tk, src, s);
+}
+
+}  // namespace
+
+int launch_forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, bool bf16, const TopkArgs& tk, const Dims& d,
+                               hipStream_t s) {
+    return bf16 ? forward_topk_sliced<true>(x, idx, w, bias, tk, d, s) : forward_topk_sliced<false>(x, idx, w, bias, tk, d, s);
 }
 
 }  // namespace ffi

@@ -1,0 +1,317 @@
+// Per-sample top-k (k <= 8): of a score matrix, and the two ends of the forward passes that keep candidates instead of
+// scores.  No counterpart in the reference, which has tf.nn.top_k inside a Keras metric (sparse/metrics.py:19); equal scores
+// go to the lower label, as there.
+//
+// Long rows take a threshold: the k best of the maxima of disjoint groups of a sample of the labels are scores of k labels,
+// so the least of them is a bound that the k best scores of the row reach.  One pass collects the few scores at or above it
+// (about k L / S of L labels for a sample of S), and the k best of those are the answer.  Exact; a sample whose candidates
+// do not fit its list (thousands of labels tied at the top) is answered from its whole row.
+#include "ffi_internal.h"
+
+#include <algorithm>
+
+namespace ffi {
+namespace {
+
+constexpr int kTopMax = 8;                 // list length kept per thread (k <= 8)
+constexpr int kNoId = 0x7fffffff;
+
+// (score descending, label ascending) order
+__device__ __forceinline__ bool better(float v, int id, float w, int wid) { return v > w || (v == w && id < wid); }
+
+struct TopList {
+    float v[kTopMax];
+    int id[kTopMax];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int s = 0; s < kTopMax; ++s) { v[s] = -__builtin_inff(); id[s] = kNoId; }
+    }
+    __device__ __forceinline__ void offer(float nv, int nid) {
+        if (!better(nv, nid, v[kTopMax - 1], id[kTopMax - 1])) return;
+#pragma unroll
+        for (int s = kTopMax - 1; s >= 0; --s) {
+            const bool keep = !better(nv, nid, v[s], id[s]);                       // element s stays where it is
+            const bool prev_keep = s == 0 || !better(nv, nid, v[s - (s > 0)], id[s - (s > 0)]);
+            const float ov = s > 0 ? v[s - (s > 0)] : nv;
+            const int oi = s > 0 ? id[s - (s > 0)] : nid;
+            v[s] = keep ? v[s] : (prev_keep ? nv : ov);
+            id[s] = keep ? id[s] : (prev_keep ? nid : oi);
+        }
+    }
+    __device__ __forceinline__ void pop() {
+#pragma unroll
+        for (int t = 0; t + 1 < kTopMax; ++t) { v[t] = v[t + 1]; id[t] = id[t + 1]; }
+        v[kTopMax - 1] = -__builtin_inff();
+        id[kTopMax - 1] = kNoId;
+    }
+};
+
+// The 64 lanes hold sorted lists; kTopMax rounds in which the best head (found with shuffles) is taken by lane `round` and
+// popped by its owner.  Afterwards lane s < 8 holds the s-th best in out_*.
+__device__ __forceinline__ void wave_topk(TopList& l, int rounds, float& out_v, int& out_i) {
+    const int lane = threadIdx.x & 63;
+    out_v = -__builtin_inff();
+    out_i = kNoId;
+    for (int s = 0; s < rounds; ++s) {
+        float bv = l.v[0];
+        int bi = l.id[0];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const float ov = __shfl_xor(bv, off, 64);
+            const int oi = __shfl_xor(bi, off, 64);
+            if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+        }
+        if (lane == s) { out_v = bv; out_i = bi; }
+        if (bi != kNoId && l.id[0] == bi && l.v[0] == bv) l.pop();
+    }
+}
+
+// The workgroup's lists down to one; afterwards lane s < rounds of wavefront 0 holds the s-th best.  One barrier.
+template <int WAVES>
+__device__ __forceinline__ void block_topk(TopList& l, int rounds, float& out_v, int& out_i) {
+    __shared__ float lv[WAVES][kTopMax];
+    __shared__ int li[WAVES][kTopMax];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    wave_topk(l, rounds, out_v, out_i);
+    if (lane < kTopMax) { lv[wave][lane] = out_v; li[wave][lane] = out_i; }
+    __syncthreads();
+    if (wave != 0) return;
+    l.clear();
+    if (lane < WAVES) {
+#pragma unroll
+        for (int s = 0; s < kTopMax; ++s) { l.v[s] = lv[lane][s]; l.id[s] = li[lane][s]; }
+    }
+    wave_topk(l, rounds, out_v, out_i);
+}
+
+// Lists of a score matrix scores[B,L]: grid (splits, B); each thread scans a strided share of the split (coalesced, eight scores
+// in flight), each wavefront then reduces its 64 lists to one: four lists of eight per split (label -1 = empty slot).
+__global__ __launch_bounds__(256) void topk_scan_kernel(const float* __restrict__ scores, int L, int labels_per_split,
+                                                        float* __restrict__ part_val, int* __restrict__ part_idx, int nlists) {
+    const int b = blockIdx.y;
+    const int begin = blockIdx.x * labels_per_split, end = min(begin + labels_per_split, L);
+    TopList l;
+    l.clear();
+    const float* row = scores + (size_t)b * L;
+    for (int j0 = begin + (int)threadIdx.x; j0 < end; j0 += 256 * 8) {
+        float v8[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v8[u] = row[min(j0 + 256 * u, end - 1)];      // clamped, not predicated: the eight loads issue back to back
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j0 + 256 * u < end) l.offer(v8[u], j0 + 256 * u);
+    }
+    float ov;
+    int oi;
+    wave_topk(l, kTopMax, ov, oi);
+    const int lane = threadIdx.x & 63;
+    if (lane < kTopMax) {
+        const int list = blockIdx.x * 4 + (threadIdx.x >> 6);
+        part_val[((size_t)b * nlists + list) * kTopMax + lane] = ov;
+        part_idx[((size_t)b * nlists + list) * kTopMax + lane] = oi != kNoId ? oi : -1;
+    }
+}
+
+// The threshold of every sample and its empty candidate list: 1,024 groups of a sample of S scores (scores[b * row + i * step],
+// step > 1: straight from a score matrix), the k-th best of the groups' maxima.
+__global__ __launch_bounds__(1024) void topk_threshold_kernel(const float* __restrict__ scores, size_t row, int step, int S, int k,
+                                                              float* __restrict__ tau, int* __restrict__ count) {
+    const int b = blockIdx.x;
+    TopList l;
+    l.clear();
+    float best = -__builtin_inff();
+    for (int i0 = threadIdx.x; i0 < S; i0 += 1024 * 4) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = scores[(size_t)b * row + (size_t)min(i0 + 1024 * u, S - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i0 + 1024 * u < S) best = fmaxf(best, v[u]);      // (each score in one group only)
+    }
+    l.v[0] = best;
+    l.id[0] = (int)threadIdx.x < S ? (int)threadIdx.x : kNoId;
+    float ov;
+    int oi;
+    block_topk<16>(l, k, ov, oi);
+    if ((int)threadIdx.x == k - 1) tau[b] = ov;
+    if (threadIdx.x == 0) count[(size_t)b * kTopkCountStep] = 0;
+}
+
+// Every score at or above its row's threshold goes to the row's candidate list.  Such scores are a tiny share of the
+// row, so the scan is a plain stream: eight loads in flight per thread, one wave-wide test, the appends on the side.
+__global__ __launch_bounds__(256) void topk_filter_kernel(const float* __restrict__ scores, int L, int labels_per_split,
+                                                          const float* __restrict__ tau, int* __restrict__ count,
+                                                          float* __restrict__ cand_val, int* __restrict__ cand_idx, int cap) {
+    constexpr int kPark = 1024;                       // hits a workgroup parks in LDS before it appends them to the row's list
+    __shared__ int park_count;
+    __shared__ float park_val[kPark];
+    __shared__ int park_idx[kPark];
+    const int b = blockIdx.y;
+    const int begin = blockIdx.x * labels_per_split, end = min(begin + labels_per_split, L);
+    const float t = tau[b];
+    const float* row = scores + (size_t)b * L;
+    if (threadIdx.x == 0) park_count = 0;
+    __syncthreads();
+    for (int j0 = begin + (int)threadIdx.x; j0 < end; j0 += 256 * 8) {
+        float v8[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v8[u] = row[min(j0 + 256 * u, end - 1)];
+        bool hit = false;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) hit |= (j0 + 256 * u < end) && v8[u] >= t;
+        if (__ballot(hit)) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int j = j0 + 256 * u;
+                if (j < end && v8[u] >= t) {
+                    const int p = atomicAdd(&park_count, 1);          // an LDS counter: no round trip to memory
+                    if (p < kPark) {
+                        park_val[p] = v8[u];
+                        park_idx[p] = j;
+                    } else {
+                        const int slot = atomicAdd(&count[(size_t)b * kTopkCountStep], 1);
+                        if (slot < cap) {
+                            cand_val[(size_t)b * cap + slot] = v8[u];
+                            cand_idx[(size_t)b * cap + slot] = j;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int n = min(park_count, kPark);
+    __shared__ int first_slot;
+    if (threadIdx.x == 0) first_slot = n ? atomicAdd(&count[(size_t)b * kTopkCountStep], n) : 0;      // one reservation for the whole workgroup
+    __syncthreads();
+    for (int e = threadIdx.x; e < n; e += 256) {
+        const int slot = first_slot + e;
+        if (slot < cap) {
+            cand_val[(size_t)b * cap + slot] = park_val[e];
+            cand_idx[(size_t)b * cap + slot] = park_idx[e];
+        }
+    }
+}
+
+template <typename T> __device__ __forceinline__ float as_float(T v);
+template <> __device__ __forceinline__ float as_float<float>(float v) { return v; }
+template <> __device__ __forceinline__ float as_float<unsigned short>(unsigned short v) { return __uint_as_float((unsigned)v << 16); }
+
+// The k best of a sample's candidates, or, where they did not fit the list, of its whole row: the stored scores, or scores
+// formed anew from the layer (k ascending, bias last); every thread keeps the best eight of its share.
+template <typename T>
+__global__ __launch_bounds__(256) void topk_select_kernel(const float* __restrict__ cand_val, const int* __restrict__ cand_idx,
+                                                          const int* __restrict__ count, int cap, int k, const TopkRowSource src, int B,
+                                                          float* __restrict__ values, int* __restrict__ indices) {
+    const int b = blockIdx.x;
+    TopList l;
+    l.clear();
+    const int n = count != nullptr ? count[(size_t)b * kTopkCountStep] : cap;
+    if (n <= cap) {
+        const float* pv = cand_val + (size_t)b * cap;
+        const int* pi = cand_idx + (size_t)b * cap;
+        for (int c0 = threadIdx.x; c0 < n; c0 += 256 * 4) {           // four candidates per thread in flight
+            float v4[4];
+            int i4[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int c = min(c0 + 256 * u, n - 1);
+                i4[u] = c0 + 256 * u < n ? pi[c] : -1;
+                v4[u] = pv[c];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i4[u] >= 0) l.offer(v4[u], i4[u]);
+        }
+    } else {
+        const T* x = static_cast<const T*>(src.x);
+        const T* w = static_cast<const T*>(src.w);
+        for (int j = threadIdx.x; j < src.L; j += 256) {
+            float v = 0.f;
+            if (src.scores != nullptr) {
+                v = src.scores[(size_t)b * src.L + j];
+            } else {
+                for (int c = 0; c < src.K; ++c) {
+                    const unsigned id = min((unsigned)src.idx[(size_t)j * src.K + c], (unsigned)src.N - 1u);
+                    v = fmaf(as_float(w[(size_t)j * src.K + c]), as_float(src.tp ? x[(size_t)id * B + b] : x[(size_t)b * src.N + id]), v);
+                }
+                if (src.bias != nullptr) v += src.bias[j];
+            }
+            l.offer(v, j);
+        }
+    }
+    float ov;
+    int oi;
+    block_topk<4>(l, k, ov, oi);
+    if ((int)threadIdx.x < k) {
+        values[(size_t)b * k + threadIdx.x] = ov;
+        indices[(size_t)b * k + threadIdx.x] = oi != kNoId ? oi : -1;
+    }
+}
+
+constexpr int kTopkRowSample = 4096;
+
+}  // namespace
+
+// Thresholds, counters and candidates begin on cache lines of their own: counters that shared one with the thresholds, which
+// every workgroup reads, tripled the time of a sweep (43 -> 146 us at 12 x 3,000 x 300,000 x 32).
+static size_t line_floats(size_t n) { return (n + 31) / 32 * 32; }
+size_t topk_candidate_bytes(int B, int sample) {
+    return (line_floats((size_t)B * sample) + line_floats(B) + (size_t)B * kTopkCountStep + 2 * (size_t)B * kTopkCap) * 4;
+}
+TopkCandidates topk_candidates_at(void* ws, int B, int sample) {
+    TopkCandidates c;
+    c.sample = static_cast<float*>(ws);
+    c.tau = c.sample + line_floats((size_t)B * sample);
+    c.count = reinterpret_cast<int*>(c.tau + line_floats(B));
+    c.val = reinterpret_cast<float*>(c.count + (size_t)B * kTopkCountStep);
+    c.idx = reinterpret_cast<int*>(c.val + (size_t)B * kTopkCap);
+    return c;
+}
+
+int launch_topk_threshold(const float* scores, size_t row, int step, int S, int k, const TopkCandidates& c, int B, hipStream_t s) {
+    hipLaunchKernelGGL(topk_threshold_kernel, dim3(B), dim3(1024), 0, s, scores, row, step, S, k, c.tau, c.count);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
+int launch_topk_select(const TopkCandidates& c, int B, const TopkArgs& tk, const TopkRowSource& src, hipStream_t s) {
+    if (src.bf16) hipLaunchKernelGGL(topk_select_kernel<unsigned short>, dim3(B), dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, tk.values, tk.indices);
+    else hipLaunchKernelGGL(topk_select_kernel<float>, dim3(B), dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, tk.values, tk.indices);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
+int launch_topk_f32(const float* scores, int B, int L, int k, float* values, int32_t* indices, hipStream_t s) {
+    if (k < 1 || k > kTopMax) return FFI_ERR_BAD_ARGUMENT;
+    if (B > 65535) return FFI_ERR_TOO_LARGE;
+    // enough workgroups to fill the GPU (8 per CU), each with at least 2048 scores to scan
+    int splits = std::max(1, std::min((L + 2047) / 2048, (8 * device_cu_count() + B - 1) / std::max(1, B)));
+    const int per = (L + splits - 1) / splits;
+    splits = (L + per - 1) / per;
+    const TopkArgs tk{k, values, indices};
+    if (L <= 16 * kTopkRowSample) {
+        // rows too short to be worth a threshold: every thread keeps a list, the wavefronts reduce them
+        const int entries = splits * 4 * kTopMax;
+        char* part = nullptr;
+        const size_t list_bytes = (size_t)B * entries * 4;
+        FFI_TRY(workspace_get(s, kWsPartials, 2 * list_bytes, (void**)&part));
+        float* pv = (float*)part;
+        int* pi = (int*)(part + list_bytes);
+        hipLaunchKernelGGL(topk_scan_kernel, dim3(splits, B), dim3(256), 0, s, scores, L, per, pv, pi, splits * 4);
+        hipLaunchKernelGGL(topk_select_kernel<float>, dim3(B), dim3(256), 0, s, pv, pi, (const int*)nullptr, entries, k, TopkRowSource{}, B, values, indices);
+        FFI_HIP_TRY(hipGetLastError());
+        return FFI_OK;
+    }
+    void* ws = nullptr;
+    FFI_TRY(workspace_get(s, kWsTopk, topk_candidate_bytes(B, 0), &ws));
+    const TopkCandidates c = topk_candidates_at(ws, B, 0);
+    FFI_TRY(launch_topk_threshold(scores, (size_t)L, L / kTopkRowSample, kTopkRowSample, k, c, B, s));
+    hipLaunchKernelGGL(topk_filter_kernel, dim3(splits, B), dim3(256), 0, s, scores, L, per, c.tau, c.count, c.val, c.idx, kTopkCap);
+    FFI_HIP_TRY(hipGetLastError());
+    TopkRowSource src;
+    src.scores = scores; src.L = L;
+    return launch_topk_select(c, B, tk, src, s);
+}
+
+}  // namespace ffi

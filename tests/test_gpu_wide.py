@@ -25,10 +25,10 @@ FORWARD_SHAPES = [(1, 1217, 300, 1), (4, 2000, 257, 16), (5, 1217, 129, 17), (8,
                   (17, 4000, 63, 3), (33, 1300, 64, 72), (100, 40_000, 200, 65), (130, 1500, 97, 130), (64, 70_000, 150, 36)]
 
 
-@pytest.mark.parametrize("ranges", [0, 1, 2, 3, 4])
-def test_forward_of_wide_inputs(ffi, ranges):
+@pytest.mark.parametrize("phases", [0, 1, -1])
+def test_forward_of_wide_inputs(ffi, phases):
     lib = ffi._lib.lib()
-    assert lib.ffi_set_option(b"wide_ranges", ranges) == 0
+    assert lib.ffi_set_option(b"wide_phases", phases) == 0
     try:
         for B, N, L, K in FORWARD_SHAPES:
             x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + N)
@@ -41,7 +41,7 @@ def test_forward_of_wide_inputs(ffi, ranges):
             out = ffi.fan_in_sparse_matmul_bias(dev(x), dev(lookup), dev(w), dev(bias)).cpu().numpy()
             assert rel_err(out, ref + bias) <= 1e-5, (B, N, L, K)
     finally:
-        lib.ffi_set_option(b"wide_ranges", 0)
+        lib.ffi_set_option(b"wide_phases", 0)
 
 
 # (B, N, L, K): lane groups of 1, 2, 4 and 8; lists that are empty, shorter and longer than a window; several label blocks,
@@ -70,3 +70,48 @@ def test_backward_of_wide_inputs(ffi, transposed):
             bias = torch.zeros(L, device="cuda", requires_grad=True)
             gb, = torch.autograd.grad(ffi.fan_in_sparse_matmul_bias(dx.requires_grad_(True), dl, dw, bias), [bias], dg)
             assert rel_err(gb.cpu().numpy(), g.astype(np.float64).sum(0)) <= 1e-5
+
+
+# Narrow inputs whose slice of samples lies in LDS: (B, N, L, K) with slices of 4 to 64 samples, label blocks and lists with
+# remainders, the largest slice that fits, rows on and off 16-byte boundaries
+LDS_SHAPES = [(1, 1, 1, 1), (3, 12, 33, 5), (5, 768, 130, 16), (8, 500, 1025, 24), (16, 1216, 300, 33), (9, 64, 2000, 7),
+              (33, 100, 65, 17), (64, 1000, 257, 8), (65, 1144, 100, 130)]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_forward_from_slices_in_lds(ffi, bf16, transposed):
+    for B, N, L, K in LDS_SHAPES:
+        x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + N)
+        tx, tw = torch.from_numpy(x), torch.from_numpy(w)
+        if bf16:
+            tx, tw = tx.bfloat16(), tw.bfloat16()
+        ref = oracle.forward(tx.float().numpy(), lookup, tw.float().numpy(), transposed=False)
+        xd = (tx.t().contiguous() if transposed else tx).cuda()
+        if bf16:
+            out = ffi.fan_in_sparse_matmul_bf16(xd, dev(lookup), tw.cuda(), transposed=transposed)
+        else:
+            out = (ffi.fan_in_sparse_matmul_tp if transposed else ffi.fan_in_sparse_matmul)(xd, dev(lookup), tw.cuda())
+        assert rel_err(out.cpu().numpy(), ref) <= 1e-5, (B, N, L, K)
+
+
+# Top-k without the scores: every label in the sample that sets the threshold and a part of them; ties across the whole layer,
+# more than a candidate list holds
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,L,K", [(1, 768, 40_000, 8), (12, 3000, 9_001, 4), (20, 1300, 17_000, 3), (3, 500, 7, 5), (33, 1217, 16_385, 2)])
+@pytest.mark.parametrize("tied", [False, True])
+def test_topk_by_threshold(ffi, bf16, B, N, L, K, tied):
+    x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + N)
+    dx, dw = dev(x), dev(np.zeros_like(w) if tied else w)
+    k = min(5, L)
+    if bf16:
+        dx, dw = dx.bfloat16(), dw.bfloat16()
+        scores = ffi.fan_in_sparse_matmul_bf16(dx, dev(lookup), dw)
+        val, idx = ffi.fan_in_sparse_topk_bf16(dx, dev(lookup), dw, k=k)
+    else:
+        scores = ffi.fan_in_sparse_matmul(dx, dev(lookup), dw)
+        val, idx = ffi.fan_in_sparse_topk(dx, dev(lookup), dw, k=k)
+    assert torch.equal(val, torch.topk(scores, k, dim=1).values)
+    assert torch.equal(torch.gather(scores, 1, idx.long()), val)
+    if tied:
+        assert torch.equal(idx.cpu().long(), torch.arange(k).expand(B, k))
