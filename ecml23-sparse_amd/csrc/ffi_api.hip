@@ -300,6 +300,16 @@ int ffi_topk_f32(const float* scores, int64_t batch, int64_t num_units, int k, f
     return launch_topk_f32(scores, (int)batch, (int)num_units, k, topk_values, topk_indices, (hipStream_t)stream);
 }
 
+int ffi_topk_hits_f32(const int32_t* top_labels, int64_t batch, int64_t row_stride, int k, const int64_t* label_indices,
+                      const float* label_values, int64_t nnz, const float* also_read, double* host_result, ffi_stream_t stream) {
+    StreamCall call_lock((hipStream_t)stream);
+    if (!top_labels || !host_result || (nnz > 0 && !label_indices)) return FFI_ERR_NULL_POINTER;
+    if (batch <= 0 || nnz < 0) return FFI_ERR_BAD_SHAPE;
+    if (k < 1 || k > 8 || row_stride < k) return FFI_ERR_BAD_ARGUMENT;
+    if (batch >= INT32_MAX || nnz >= INT32_MAX || row_stride >= INT32_MAX) return FFI_ERR_TOO_LARGE;
+    return topk_hits(top_labels, (int)batch, (int)row_stride, k, label_indices, label_values, (int)nnz, also_read, host_result, (hipStream_t)stream);
+}
+
 static int check_loss_args(const int64_t* label_indices, int64_t nnz, int loss_kind, int64_t batch, int64_t num_units) {
     if (nnz < 0) return FFI_ERR_BAD_SHAPE;
     if (nnz > 0 && !label_indices) return FFI_ERR_NULL_POINTER;

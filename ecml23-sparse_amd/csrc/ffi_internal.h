@@ -66,8 +66,10 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10, kWsHostWords = 11 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
+// 128 bytes of pinned host memory of the stream, for results that the host waits for
+int host_words_get(hipStream_t s, void** out);
 void workspace_clear(int device);
 size_t workspace_bytes(int device);
 int device_cu_count();
@@ -75,6 +77,9 @@ int device_cu_count();
 // inference variant: bf16 features / weights (raw 16-bit patterns), fp32 accumulation
 int launch_forward_bf16(const unsigned short* features, const int32_t* idx, const unsigned short* w, float* out,
                         const Dims& d, hipStream_t s);
+// Label values at the k best labels, summed per rank, to result[0, k) on the host, and *also, if given, to result[k]; waits for the stream.
+int topk_hits(const int32_t* top, int B, int top_stride, int k, const int64_t* label_indices, const float* label_values, int nnz,
+              const float* also, double* result, hipStream_t s);
 int launch_topk_f32(const float* scores, int B, int L, int k, float* values, int32_t* indices, hipStream_t s);
 
 // dst[c][r] = src[r][c] for a row-major [rows, cols] matrix.

@@ -111,11 +111,29 @@ int workspace_get(hipStream_t s, int slot, size_t bytes, void** out) {
     return FFI_OK;
 }
 
+int host_words_get(hipStream_t s, void** out) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    for (WsEntry& e : g_ws) {
+        if (e.device == dev && e.stream == s && e.slot == kWsHostWords) {
+            *out = e.ptr;
+            return FFI_OK;
+        }
+    }
+    WsEntry e{dev, s, kWsHostWords, nullptr, 0};                  // (bytes: of device memory)
+    if (hipHostMalloc(&e.ptr, 128) != hipSuccess) { (void)hipGetLastError(); return FFI_ERR_OUT_OF_MEMORY; }
+    g_ws.push_back(e);
+    *out = e.ptr;
+    return FFI_OK;
+}
+
 void workspace_clear(int device) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     for (size_t i = 0; i < g_ws.size();) {
         if (g_ws[i].device == device) {
-            (void)hipFree(g_ws[i].ptr);
+            if (g_ws[i].slot == kWsHostWords) (void)hipHostFree(g_ws[i].ptr);
+            else (void)hipFree(g_ws[i].ptr);
             g_ws.erase(g_ws.begin() + i);
         } else {
             ++i;

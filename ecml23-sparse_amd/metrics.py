@@ -11,6 +11,8 @@ the tensors.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -106,11 +108,30 @@ def forward_loss(features, lookup, weights, bias, y_true, kind, grad_scale=None,
     return result + (top,) if topk else result
 
 
+_unit_gradients = {}      # device -> a scalar one that nobody writes to
+
+
+def unit_gradient(loss):
+    """What ``loss.backward()`` starts from, as a tensor that the loss functions below recognise: where it reaches them
+    unchanged they need not multiply their ``[B,L]`` gradient by it."""
+    if loss.dim() != 0 or loss.dtype != torch.float32 or not loss.is_cuda:
+        return None
+    one = _unit_gradients.get(loss.device)
+    if one is None:
+        one = torch.ones((), dtype=torch.float32, device=loss.device)
+        torch.cuda.current_stream(loss.device).synchronize()        # (once per device: other streams will read it)
+        one = _unit_gradients.setdefault(loss.device, one)
+    return one
+
+
 def _upstream_is_one(upstream):
     """True where the factor autograd hands to ``backward`` is known ON THE HOST to be 1: reading a device scalar
     here would make every training step wait for the GPU."""
     if not isinstance(upstream, torch.Tensor):
         return float(upstream) == 1.0
+    one = _unit_gradients.get(upstream.device)
+    if one is not None and upstream.data_ptr() == one.data_ptr():
+        return True
     return upstream.device.type == "cpu" and upstream.numel() == 1 and float(upstream) == 1.0
 
 
@@ -227,6 +248,23 @@ def topk_as_matrix(data, k):
     return indices, torch.ones(indices.shape[0], dtype=torch.float32, device=data.device), tuple(data.shape)
 
 
+MAX_TOPK = 8       # ranks that the library's top-k and hit counts hold
+
+
+def topk_hits(top_labels, k, y_true, also_read=None):
+    """Sum over the samples of the label value at rank ``r < k`` of ``top_labels`` (``[B, >=k]`` int32), as a list of ``k``
+    Python floats, followed by the value of the float32 device scalar ``also_read`` if one is given: one launch and one
+    wait for the stream."""
+    indices, values = _labels(y_true, top_labels.device)
+    result = (ctypes.c_double * (k + 1))()
+    with torch.cuda.device(top_labels.device):
+        _lib.check(_lib.lib().ffi_topk_hits_f32(
+            top_labels.data_ptr(), top_labels.shape[0], top_labels.stride(0), k, indices.data_ptr() if indices.numel() else None,
+            values.data_ptr() if values is not None and values.numel() else None, indices.shape[0],
+            also_read.data_ptr() if also_read is not None else None, result, _stream_handle(top_labels.device)))
+    return result[:k + 1] if also_read is not None else result[:k]
+
+
 class PrecisionAtK:
     """Fraction of the k best-scored labels of each sample that are true labels, accumulated over
     ``update_state`` calls (sparse/metrics.py:31-71: label values at the top-k positions are summed,
@@ -248,8 +286,11 @@ class PrecisionAtK:
 
     def update_from_topk(self, y_true, top_labels, num_units):
         """As ``update_state`` for callers that already hold the top-k labels ``[B, >=k]``."""
-        indices, values = _labels(y_true, top_labels.device)
         batch = top_labels.shape[0]
+        if (top_labels.is_cuda and top_labels.dtype == torch.int32 and top_labels.dim() == 2 and batch
+                and self._k <= min(MAX_TOPK, top_labels.shape[1]) and top_labels.stride(1) == 1 and top_labels.stride(0) >= self._k):
+            return self._add_hits(topk_hits(top_labels, self._k, y_true), batch)
+        indices, values = _labels(y_true, top_labels.device)
         top = top_labels[:, :self._k].to(torch.int64)
         if indices.shape[0]:
             keys = indices[:, 0] * num_units + indices[:, 1]
@@ -261,6 +302,10 @@ class PrecisionAtK:
             pos = torch.searchsorted(keys, want).clamp_(max=keys.numel() - 1)
             hit = (keys[pos] == want) & (top.reshape(-1) >= 0)
             self._correct += float((vals[pos] * hit).sum())
+        self._total += float(batch * self._k)
+
+    def _add_hits(self, hits_per_rank, batch):
+        self._correct += sum(hits_per_rank[:self._k])
         self._total += float(batch * self._k)
 
     def result(self):

@@ -9,7 +9,8 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .fixed_fan_in_ops import _stream_handle
+from . import metrics as metrics_mod
+from .fixed_fan_in_ops import _stream_handle, topk_scores
 
 
 def adam_step(variable, m, v, gradient, learning_rate, beta_1, beta_2, epsilon, step):
@@ -112,16 +113,35 @@ class SparseOptWrapper(torch.nn.Module):
             o.zero_grad()
         y_pred = self.base_model(x)
         loss = self.loss(y, y_pred)
-        loss.backward()
+        loss.backward(metrics_mod.unit_gradient(loss))
         for o in self.optimizers:
             o.step()
         self.handle_sparse_layers()
-        results = {"loss": float(loss.detach())}
         with torch.no_grad():
+            loss, y_pred = loss.detach(), y_pred.detach()
+            hits, loss_value = self._shared_hits(y, y_pred, loss)
+            results = {"loss": float(loss) if loss_value is None else loss_value}
             for m in self.metrics:
-                m.update_state(y, y_pred.detach())
+                if hits is not None and type(m) is metrics_mod.PrecisionAtK:
+                    m._add_hits(hits, y_pred.shape[0])
+                else:
+                    m.update_state(y, y_pred)
                 results[getattr(m, "name", type(m).__name__)] = m.result()
         return results
+
+    def _shared_hits(self, y, y_pred, loss):
+        """``(hits per rank, loss)`` of the step for all its ``PrecisionAtK``: the best labels of the largest k begin with those
+        of every smaller one, so one top-k, one count and one wait serve them all, and the loss comes with them."""
+        ks = [m._k for m in self.metrics if type(m) is metrics_mod.PrecisionAtK]
+        if not ks or not y_pred.is_cuda or y_pred.dim() != 2 or y_pred.dtype != torch.float32 or not y_pred.shape[0]:
+            return None, None
+        k = max(ks)
+        if min(ks) < 1 or k > metrics_mod.MAX_TOPK:
+            return None, None
+        _, top = topk_scores(y_pred, k)
+        along = loss if loss.device == y_pred.device and loss.dtype == torch.float32 and loss.numel() == 1 else None
+        hits = metrics_mod.topk_hits(top, k, y, along)
+        return hits[:k], hits[k] if along is not None else None
 
     def handle_sparse_layers(self):
         if self.rewire_interval > 0 and self.optimizer.iterations % self.rewire_interval == 1:

@@ -274,6 +274,15 @@ int ffi_topk_f32(const float* scores, int64_t batch, int64_t num_units, int k,
                  float* topk_values, int32_t* topk_indices, ffi_stream_t stream);
 
 /*
+ * Precision counts: host_result[r], r < k (1..8), becomes the sum over the samples of the label value at the sample's r-th best
+ * label (top_labels[b * row_stride + r]; values of one if label_values is null, zero where the pair is not listed, the first
+ * position where it is listed more than once).  If also_read (a device scalar, such as the loss of the step) is given, its value
+ * goes to host_result[k].  Waits for the stream.
+ */
+int ffi_topk_hits_f32(const int32_t* top_labels, int64_t batch, int64_t row_stride, int k, const int64_t* label_indices,
+                      const float* label_values, int64_t nnz, const float* also_read, double* host_result, ffi_stream_t stream);
+
+/*
  * The loss the reference trains the layer with, and its gradient with respect to the scores: the
  * producer of out_grad.  Restates SparseLossBase.call (sparse/metrics.py:136-139) on top of
  * dense_sparse_cwise_op (sparse/utils.py:11-17): every (b,j) is charged loss(score, 0), except the
