@@ -26,6 +26,7 @@ SOURCES = [
     "ffi_util.hip",
     "ffi_wide.hip",
     "ffi_sliced.hip",
+    "ffi_small.hip",
     "ffi_topk.hip",
     "ffi_loss.hip",
     "ffi_sparse_grad.hip",

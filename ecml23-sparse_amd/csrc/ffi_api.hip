@@ -100,6 +100,8 @@ struct PlannedWeightGrad {
     float* bias_grad = nullptr;
 };
 
+constexpr int kGuardHostBadIds = 1;     // the word of a plan's pinned mirror that the kernels for small layers write
+
 // The library's own in-place editors of a lookup matrix (ffi_rewire_f32, ffi_arrange_connections_f32) tell the cache:
 // every cached plan built from that buffer on this device is marked outdated on the host, so the next backward call
 // rebuilds it before it enqueues anything (no walk of an outdated plan, no recomputing kernels, reproducible sums).
@@ -147,9 +149,24 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         FFI_TRY(between(p));
         return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, verdict, &zeroed);
     };
+    // small layers read the lookup itself: of the plan they need that its build has found every id in range
+    const bool small = takes_small_backward(d);
+    auto small_pass = [&]() -> int {
+        unsigned long long* bad = nullptr;
+        FFI_HIP_TRY(hipHostGetDevicePointer((void**)&bad, p->h_guard + kGuardHostBadIds, 0));
+        if (wg.features == nullptr) FFI_TRY(between(p));       // (nothing, or a weight gradient formed without the plan)
+        return launch_backward_small(wg.features, lookup, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d, s, bad);
+    };
     if (!p) {
         FFI_TRY(create_cached_plan(lookup, d, dev, s, &p));
-        return passes(nullptr);
+        return small ? small_pass() : passes(nullptr);
+    }
+    if (small) {
+        if (p->edited_by_library || __atomic_exchange_n(p->h_guard + kGuardHostBadIds, 0ull, __ATOMIC_ACQ_REL) != 0) {
+            const int st = plan_build(p, lookup, s);
+            if (st != FFI_OK) { drop_cached_plan(p); return st; }
+        }
+        return small_pass();
     }
     bool seen = false, current = true;
     unsigned long long bad = 0;
@@ -633,6 +650,7 @@ int ffi_set_option(const char* name, int value) {
         {"plan_weights_in_lds", &ffi::Options::plan_weights_in_lds, -1, 1},
         {"workgroups_per_cu", &ffi::Options::workgroups_per_cu, 0, 16},
         {"plan_sorted_columns", &ffi::Options::plan_sorted_columns, -1, 1},
+        {"small_path", &ffi::Options::small_path, -1, 1},
         {"wide_phases", &ffi::Options::wide_phases, -1, 1},
     };
     for (const auto& t : table) {

@@ -668,6 +668,7 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
 
 int launch_forward(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                    hipStream_t s) {
+    if (takes_small_forward(d)) return launch_forward_small(x, idx, w, bias, out, d, s);
     // (the kernel reaches the 32 rows of out of a batch tile through 32-bit byte offsets)
     if (tile_path_fits(d.N) && d.L < (1 << 25) && !few_samples(d)) return forward_tiles(x, idx, w, bias, out, nullptr, kEpiScores, nullptr, nullptr, d, s);
     return launch_forward_wide(x, idx, w, bias, out, d, s);
@@ -742,6 +743,7 @@ extern "C" int ffi_forward_noalloc_f32(const float* features, const int32_t* loo
     if (!tile_path_fits((int)num_features) || num_units >= (1 << 25)) return FFI_ERR_TOO_LARGE;
     if ((uint64_t)batch * (uint64_t)num_features > kNoAllocFloats) return FFI_ERR_TOO_LARGE;
     const Dims d{(int)batch, (int)num_features, (int)num_units, (int)fan_in, transposed != 0};
+    if (takes_small_forward(d)) return launch_forward_small(features, lookup, weights, nullptr, result, d, (hipStream_t)stream);
     float* xt = nullptr;
     if (!d.tp) FFI_TRY(scratch_address(&xt));
     return forward_tiles(features, lookup, weights, nullptr, result, nullptr, kEpiScores, nullptr, nullptr, d, (hipStream_t)stream, xt);

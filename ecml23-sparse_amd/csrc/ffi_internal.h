@@ -31,6 +31,7 @@ struct Options {
     int plan_weights_in_lds = 0;    // -1: never / 1: whenever the tile fits
     int workgroups_per_cu = 0;      // upper limit for the kernel that walks a tiled plan
     int wide_phases = 0;            // -1: never / 1: wherever it can: the forward kernel in phases for wide inputs
+    int small_path = 0;             // -1: never / 1: wherever they can: the two launches for small layers
     int plan_sorted_columns = 0;    // -1: never / 1: always (in the weights-in-LDS form) the plans that hand the columns to the walking kernel's threads tile by tile, by length
 };
 extern Options g_options;
@@ -66,10 +67,13 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10, kWsHostWords = 11 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10, kWsHostWords = 11, kWsTickets = 12 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 // 128 bytes of pinned host memory of the stream, for results that the host waits for
 int host_words_get(hipStream_t s, void** out);
+// 4,096 counters of the stream that are zero between launches (a kernel that counts in them puts them back)
+constexpr int kTicketCount = 4096;
+int tickets_get(hipStream_t s, void** out);
 void workspace_clear(int device);
 size_t workspace_bytes(int device);
 int device_cu_count();
@@ -130,6 +134,13 @@ struct TopkArgs {
     float* values;
     int32_t* indices;
 };
+// small layers (ffi_small.hip): one launch forward, one for the gradients (gx or gw and gb may be null); *bad, in pinned host
+// memory, becomes 1 where an id is out of range
+bool takes_small_forward(const Dims& d);
+bool takes_small_backward(const Dims& d);
+int launch_forward_small(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s);
+int launch_backward_small(const float* x, const int32_t* idx, const float* w, const float* g, float* gx, float* gw, float* gb, const Dims& d,
+                          hipStream_t s, unsigned long long* bad);
 // forward pass whose epilogue turns the scores into loss gradients (scores may be null; tk may be null)
 int launch_forward_loss(const float* x, const int32_t* idx, const float* w, const float* bias, const LossArgs& la,
                         float* scores, float* g, const TopkArgs* tk, const Dims& d, hipStream_t s);

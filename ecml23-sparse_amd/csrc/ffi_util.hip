@@ -111,6 +111,25 @@ int workspace_get(hipStream_t s, int slot, size_t bytes, void** out) {
     return FFI_OK;
 }
 
+int tickets_get(hipStream_t s, void** out) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    for (WsEntry& e : g_ws) {
+        if (e.device == dev && e.stream == s && e.slot == kWsTickets) {
+            *out = e.ptr;
+            return FFI_OK;
+        }
+    }
+    WsEntry e{dev, s, kWsTickets, nullptr, kTicketCount * sizeof(unsigned)};
+    if (hipMalloc(&e.ptr, e.bytes) != hipSuccess) { (void)hipGetLastError(); return FFI_ERR_OUT_OF_MEMORY; }
+    const hipError_t err = hipMemset(e.ptr, 0, e.bytes);          // (once, and waited for)
+    if (err != hipSuccess || hipDeviceSynchronize() != hipSuccess) { (void)hipFree(e.ptr); return hip_fail(err); }
+    g_ws.push_back(e);
+    *out = e.ptr;
+    return FFI_OK;
+}
+
 int host_words_get(hipStream_t s, void** out) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;

@@ -111,7 +111,8 @@ def test_topk_by_threshold(ffi, bf16, B, N, L, K, tied):
     else:
         scores = ffi.fan_in_sparse_matmul(dx, dev(lookup), dw)
         val, idx = ffi.fan_in_sparse_topk(dx, dev(lookup), dw, k=k)
-    assert torch.equal(val, torch.topk(scores, k, dim=1).values)
-    assert torch.equal(torch.gather(scores, 1, idx.long()), val)
+    best = torch.topk(scores, k, dim=1).values                # (possibly summed in another order)
+    assert float((val - best).abs().max()) <= 1e-5 * float(best.abs().max())
+    assert float((torch.gather(scores, 1, idx.long()) - val).abs().max()) <= 1e-5 * float(best.abs().max())
     if tied:
         assert torch.equal(idx.cpu().long(), torch.arange(k).expand(B, k))
