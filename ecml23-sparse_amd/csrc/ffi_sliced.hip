@@ -661,17 +661,20 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
         for (int i = 0; i < kPer; ++i) acc[m].a[i] = 0.f;
 
     // lane f brings quad f & 1 of label f / 2 (of every 32 labels).  Labels behind the last read zeros: a gather of row 0 with
-    // weight zero.
+    // weight zero.  The resource begins at the wavefront's first label and ends with the part (the scalar offset of a buffer
+    // load is not part of its bounds check in every form): a wavefront behind the last label has an empty one.
     uint4 ids, ws;
+    const int jf = min(jw, L);
+    const size_t left = (size_t)(L - jf);
     auto fetch = [&](int r) {
-        const size_t base = (size_t)min(r, octs - 1) * 8 * L;                            // (behind the last part: the last again)
-        const buffer_rsrc ri = make_rsrc(idx + base, (size_t)L * 32), rw = make_rsrc((const char*)w + base * (BF16 ? 2 : 4), (size_t)L * (BF16 ? 16 : 32));
-        ids = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ri, lane * 16u, (unsigned)jw * 32u, 0));
+        const size_t base = ((size_t)min(r, octs - 1) * L + jf) * 8;                     // (behind the last part: the last again)
+        const buffer_rsrc ri = make_rsrc(idx + base, left * 32), rw = make_rsrc((const char*)w + base * (BF16 ? 2 : 4), left * (BF16 ? 16 : 32));
+        ids = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ri, lane * 16u, 0, 0));
         if (BF16) {
-            const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rw, lane * 8u, (unsigned)jw * 16u, 0));
+            const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rw, lane * 8u, 0, 0));
             ws.x = h.x; ws.y = h.y;
         } else {
-            ws = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, (unsigned)jw * 32u, 0));
+            ws = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, 0, 0));
         }
     };
     auto put = [&](int r) {

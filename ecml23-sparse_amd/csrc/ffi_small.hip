@@ -190,6 +190,7 @@ SmallShape small_shape(const Dims& d) {
 // 320, at 8 M 48 to 75 against 44 to 205; 4 M sums of gx take 55 to 60 us against 92.
 bool takes_small_forward(const Dims& d) {
     const long long sums = (long long)d.B * d.L * d.K;
+    if (d.B > 65535 * kSmSamples) return false;            // (groups of samples are the grid's second dimension)
     if (g_options.small_path != 0) return g_options.small_path > 0 && sums < (1ll << 30);
     return sums <= (4ll << 20);
 }

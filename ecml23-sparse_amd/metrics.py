@@ -117,6 +117,8 @@ def unit_gradient(loss):
     if loss.dim() != 0 or loss.dtype != torch.float32 or not loss.is_cuda:
         return None
     one = _unit_gradients.get(loss.device)
+    if one is not None and one._version:                           # (a hook wrote into it: it is no constant)
+        return None
     if one is None:
         one = torch.ones((), dtype=torch.float32, device=loss.device)
         torch.cuda.current_stream(loss.device).synchronize()        # (once per device: other streams will read it)
@@ -130,7 +132,7 @@ def _upstream_is_one(upstream):
     if not isinstance(upstream, torch.Tensor):
         return float(upstream) == 1.0
     one = _unit_gradients.get(upstream.device)
-    if one is not None and upstream.data_ptr() == one.data_ptr():
+    if one is not None and not one._version and upstream.data_ptr() == one.data_ptr():
         return True
     return upstream.device.type == "cpu" and upstream.numel() == 1 and float(upstream) == 1.0
 
