@@ -1009,13 +1009,23 @@ int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
 // connections); entry i of a unit = (connection inside the chunk << 11) | column id; units are
 // numbered chunk-major (u = chunk * L + label) so that consecutive lanes work on consecutive labels, and stored in
 // blocks of 64 (arranged_quarter_offset).
-// A wavefront takes 64 consecutive units (one block of the stored layout): their ids pass through LDS so that both
-// the loads (128 contiguous bytes of a row per half wavefront) and the stores (the block's 4 KB in one piece) are
-// coalesced; a thread per unit would read its row with a stride of a whole row between lanes (measured at
-// 670,091 labels x fan-in 32: 0.95 ms, against 0.1 ms this way).
+// Half a wavefront takes a unit, a lane a connection: the connections of either role are a ballot, and a connection's place
+// follows from the bits below its own.  So the ids are loaded in pieces of 128 bytes and nothing is looked at twice; a wavefront
+// forms 64 consecutive units (one block of the stored layout) in LDS and stores the block's 4 KB in one piece.
+// (670,091 labels x fan-in 32, beside the plan build's other kernels: a thread per unit, walking its 32 ids twice, 673 us; this 96.)
+
+// The place of a lane's connection among the connections of its unit, which are those of `unit` (a mask of neighbouring lanes)
+// with `on` set; called by whole wavefronts.
+__device__ __forceinline__ unsigned arranged_place(bool on, int id, unsigned role, unsigned long long unit) {
+    const bool first = ((unsigned)id & 1u) == role;               // (role: the parity taken at even places)
+    const unsigned long long firsts = __ballot(on && first) & unit, seconds = __ballot(on && !first) & unit;
+    const unsigned m = min((unsigned)__popcll(firsts), (unsigned)__popcll(seconds));
+    const unsigned t = (unsigned)__popcll((first ? firsts : seconds) & ((1ull << (threadIdx.x & 63)) - 1ull));
+    return t < m ? 2u * t + (first ? 0u : 1u) : 2u * m + (t - m);
+}
+
 __global__ __launch_bounds__(kBlock) void arrange_units_kernel(const int32_t* __restrict__ idx, int L, int K, int nchunks,
                                                                 unsigned short* __restrict__ out) {
-    __shared__ int in[kBlock / 64][64][33];
     __shared__ __align__(16) unsigned short outb[kBlock / 64][2048];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long total = (long long)L * nchunks;
@@ -1023,46 +1033,31 @@ __global__ __launch_bounds__(kBlock) void arrange_units_kernel(const int32_t* __
     if (u0 >= total) return;                              // (whole wavefronts; no workgroup barrier below)
     // (chunk and label of the wavefront's first unit by one division; the units behind it by stepping)
     const int c0 = (int)(u0 / L), j0 = (int)(u0 - (long long)c0 * L);
-    {
-        const int k = lane & 31;
-#pragma unroll 4
-        for (int r = 0; r < 32; ++r) {
-            const int q = 2 * r + (lane >> 5);
-            int c = c0, j = j0 + q;
+    const int k = lane & 31;
+    const unsigned long long unit = 0xffffffffull << (lane & 32);
+    unsigned short* ob = outb[wave];
+    constexpr int kStep = 8;                              // loads in flight
+    for (int r0 = 0; r0 < 32; r0 += kStep) {
+        int id[kStep];
+        bool on[kStep];
+        unsigned role[kStep];
+#pragma unroll
+        for (int i = 0; i < kStep; ++i) {
+            int c = c0, j = j0 + 2 * (r0 + i) + (lane >> 5);
             while (j >= L) { j -= L; ++c; }
-            int v = -1;
-            if (c < nchunks && c * 32 + k < K) v = idx[(size_t)j * K + c * 32 + k];
-            in[wave][q][k] = v;
+            on[i] = c < nchunks && c * 32 + k < K;
+            id[i] = on[i] ? idx[(size_t)j * K + c * 32 + k] : 0;
+            role[i] = ((unsigned)j >> 3) & 1u;
         }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    {
-        const long long u = u0 + lane;
-        const int* row = in[wave][lane];
-        unsigned short* ob = outb[wave];
-        auto dst = [&](unsigned pos) -> unsigned short& { return ob[(pos >> 3) * 512 + (unsigned)lane * 8 + (pos & 7u)]; };
-        int kn = 0;
-        if (u < total) {
-            int c = c0, j = j0 + lane;
-            while (j >= L) { j -= L; ++c; }
-            kn = min(32, K - c * 32);
-            const unsigned role = ((unsigned)j >> 3) & 1u;        // parity taken at even positions
-            unsigned nfirst = 0;
-            for (int k = 0; k < kn; ++k) nfirst += (((unsigned)row[k] & 1u) == role) ? 1u : 0u;
-            const unsigned m = min(nfirst, (unsigned)kn - nfirst);
-            unsigned tf = 0, ts = 0;
-            for (int k = 0; k < kn; ++k) {
-                const unsigned id = (unsigned)row[k];
-                const bool first = (id & 1u) == role;
-                const unsigned t = first ? tf++ : ts++;
-                const unsigned pos = t < m ? 2u * t + (first ? 0u : 1u) : 2u * m + (t - m);
-                dst(pos) = (unsigned short)(((unsigned)k << kArrIdBits) | id);
-            }
+#pragma unroll
+        for (int i = 0; i < kStep; ++i) {
+            const unsigned place = arranged_place(on[i], id[i], role[i], unit);
+            // a chunk the fan-in does not fill (and the units behind the last one, which pad the array to whole blocks): the
+            // rest points at connection 31, which such a chunk never stores
+            const unsigned pos = on[i] ? place : (unsigned)k;
+            ob[(pos >> 3) * 512 + (unsigned)(2 * (r0 + i) + (lane >> 5)) * 8 + (pos & 7u)] =
+                (unsigned short)(on[i] ? ((unsigned)k << kArrIdBits) | (unsigned)id[i] : 31u << kArrIdBits);
         }
-        // a chunk the fan-in does not fill (and the units behind the last one, which pad the array to whole blocks): the
-        // rest points at connection 31, which such a chunk never stores
-        for (int k = kn; k < 32; ++k) dst((unsigned)k) = (unsigned short)(31u << kArrIdBits);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1072,35 +1067,35 @@ __global__ __launch_bounds__(kBlock) void arrange_units_kernel(const int32_t* __
     for (int i = 0; i < 4; ++i) o4[i * 64 + lane] = b4[i * 64 + lane];
 }
 
-// The same reordering applied in place to the lookup matrix itself and to up to four float
-// matrices of its shape (weights, optimizer state): one thread per (label, chunk of 32).
+// The same reordering applied in place to the lookup matrix itself and to up to four float matrices of its shape (weights,
+// optimizer state): 2^lg lanes per (label, chunk of 32).  A unit whose connections are in place already is left alone: after a
+// rewiring that is most of them, and then the pass is one of reading ids.  Bound by memory: all four matrices moved at 670,091
+// labels x fan-in 32 are 690 MB.  (There, after one per cent of the connections was redrawn: a thread per unit with its ids and
+// places in scratch memory 1,100 us; this 70.)
 struct ArrangeArrays { float* a[4]; };
 __global__ __launch_bounds__(kBlock) void arrange_in_place_kernel(int32_t* __restrict__ idx, ArrangeArrays arr, int L, int K,
-                                                                   int nchunks) {
-    const long long u = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (u >= (long long)L * nchunks) return;
-    const int c = (int)(u / L), j = (int)(u - (long long)c * L);
-    const int k0 = c * 32, kn = min(32, K - k0);
-    int32_t* row = idx + (size_t)j * K + k0;
-    const unsigned role = ((unsigned)j >> 3) & 1u;
-    int32_t ids[32];
-    unsigned char pos[32];
-    unsigned nfirst = 0;
-    for (int k = 0; k < kn; ++k) { ids[k] = row[k]; nfirst += (((unsigned)ids[k] & 1u) == role) ? 1u : 0u; }
-    const unsigned m = min(nfirst, (unsigned)kn - nfirst);
-    unsigned tf = 0, ts = 0;
-    for (int k = 0; k < kn; ++k) {
-        const bool first = ((unsigned)ids[k] & 1u) == role;
-        const unsigned t = first ? tf++ : ts++;
-        pos[k] = (unsigned char)(t < m ? 2u * t + (first ? 0u : 1u) : 2u * m + (t - m));
-    }
-    for (int k = 0; k < kn; ++k) row[pos[k]] = ids[k];
-    for (int a = 0; a < 4; ++a) {
-        if (arr.a[a] == nullptr) continue;
-        float* frow = arr.a[a] + (size_t)j * K + k0;
-        float v[32];
-        for (int k = 0; k < kn; ++k) v[k] = frow[k];
-        for (int k = 0; k < kn; ++k) frow[pos[k]] = v[k];
+                                                                   int nchunks, int lg) {
+    const int lane = threadIdx.x & 63, width = 1 << lg, k = lane & (width - 1);
+    const unsigned long long group = (lg == 5 ? 0xffffffffull : (1ull << width) - 1ull) << (lane - k);
+    const long long total = (long long)L * nchunks, step = (long long)gridDim.x * kBlock >> lg;
+    for (long long u = ((long long)blockIdx.x * kBlock + threadIdx.x) >> lg; u < total; u += step) {
+        const int j = nchunks == 1 ? (int)u : (int)(u / nchunks), c = (int)(u - (long long)j * nchunks);
+        const bool on = c * 32 + k < K;
+        const size_t from = (size_t)j * K + c * 32 + k;
+        const int32_t id = on ? idx[from] : 0;
+        const unsigned pos = arranged_place(on, id, ((unsigned)j >> 3) & 1u, group);
+        if (!on || !(__ballot(on && pos != (unsigned)k) & group)) continue;
+        const size_t to = from - k + pos;
+        float v[4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) v[a] = arr.a[a] != nullptr ? arr.a[a][from] : 0.f;
+        // (every lane's loads are in before any lane stores: one wavefront, one instruction stream)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        idx[to] = id;
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+            if (arr.a[a] != nullptr) arr.a[a][to] = v[a];
     }
 }
 
@@ -1109,10 +1104,10 @@ __global__ __launch_bounds__(kBlock) void arrange_in_place_kernel(int32_t* __res
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s) {
     ArrangeArrays arr{{nullptr, nullptr, nullptr, nullptr}};
     for (int i = 0; i < n_arrays && i < 4; ++i) arr.a[i] = arrays[i];
-    const int nchunks = (K + 31) / 32;
-    const long long units = (long long)L * nchunks;
-    hipLaunchKernelGGL(arrange_in_place_kernel, dim3((unsigned)((units + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, lookup, arr,
-                       L, K, nchunks);
+    const int nchunks = (K + 31) / 32, lg = K <= 8 ? 3 : K <= 16 ? 4 : 5;
+    const long long units = (long long)L * nchunks, blocks = ((units << lg) + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(arrange_in_place_kernel, dim3((unsigned)std::min(blocks, 1ll << 20)), dim3(kBlock), 0, s, lookup, arr,
+                       L, K, nchunks, lg);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
