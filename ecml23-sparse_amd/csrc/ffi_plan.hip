@@ -474,22 +474,30 @@ __global__ void tile_fill_kernel(const int32_t* __restrict__ idx, const unsigned
 // connections of the same bank half in ascending flat position: the order tile_fill_kernel produces), so the slots
 // are written by threads <-> connections, not by a column's thread scanning for them.  Padding goes to the slots no
 // connection takes (a column's thread knows them from its two totals).  A label that lists one column twice sets one
-// bit for two connections: such a tile is placed by its columns' threads instead (see below), several times slower.
-// Measured at 670,091 labels x fan-in 32 over 768 columns: 6.2 ms -> 0.19 ms without such labels, 1.3 ms with some in every tile.
+// bit for two connections -- sources drawn with replacement do so all the time, two labels in five at fan-in 32 over 768
+// columns.  The connections that find their bit set are kept in chains, one per column: a connection's rank then counts the
+// chain's entries with lower labels too, and, where its own label is among them, the equal ids in front of it in its row.
+// A chain is 0.5 entries on average there; beyond dup_cap entries in a tile (four per column, or what LDS is left) the
+// columns' threads place the tile (see below).
+// Measured at 670,091 labels x fan-in 32 over 768 columns: 6.2 ms by the scan of all pairs, 0.83 ms by the columns' threads
+// (0.19 without labels that list a column twice), 0.26 by chains.
 __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
                                         int tile_labels, int zero_row, const unsigned* __restrict__ slice_off,
                                         unsigned short* __restrict__ lab16, unsigned short* __restrict__ pos16, unsigned pad_pos,
                                         unsigned* __restrict__ slot32, int words, int col_lo,
-                                        const unsigned short* __restrict__ colperm) {
+                                        const unsigned short* __restrict__ colperm, unsigned dup_cap) {
     extern __shared__ __align__(16) unsigned fill_lds[];
     const int t = blockIdx.x, nthreads = blockDim.x;
     unsigned* bm = fill_lds;                                                   // [nthreads][words] (words odd: no bank conflicts)
     unsigned* pm = bm + (size_t)nthreads * words;                              // [words] labels staged in odd LDS rows
-    unsigned short* pre = reinterpret_cast<unsigned short*>(pm + words);       // [nthreads][words + 1][2] labels before word w, even / odd rows
-    unsigned short* rows_of = pre + (size_t)nthreads * (words + 1) * 2;        // [tile_labels]
+    unsigned* heads = pm + words;                                              // [nthreads] first entry of the column's chain
+    unsigned* chain = heads + nthreads;                                        // [dup_cap] label | next entry << 16
+    unsigned short* pre = reinterpret_cast<unsigned short*>(chain + dup_cap);  // [nthreads][words][2] labels before word w, even / odd rows
+    unsigned short* rows_of = pre + (size_t)nthreads * words * 2;              // [tile_labels]
     unsigned short* ids = rows_of + ((tile_labels + 1) & ~1);                  // [tile_labels * K]
     unsigned short* thread_of = ids + (((size_t)tile_labels * K + 1) & ~(size_t)1);   // [nthreads] the thread that walks each column
-    __shared__ unsigned duplicate;
+    __shared__ unsigned duplicates;
+    constexpr unsigned kNoEntry = 0xffffu;
     // (bitmap and prefix counts are kept per column; slices, lanes and slot parities belong to threads)
     const unsigned mycol = colperm != nullptr ? colperm[(size_t)blockIdx.x * blockDim.x + threadIdx.x] : threadIdx.x;
     thread_of[mycol] = (unsigned short)threadIdx.x;
@@ -498,7 +506,8 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
     const int* src = idx + (size_t)j0 * K;
     const int total = nl * K;
     const int nslices = nthreads >> 6;
-    if (threadIdx.x == 0) duplicate = 0u;
+    if (threadIdx.x == 0) duplicates = 0u;
+    heads[threadIdx.x] = kNoEntry;
     for (int i = threadIdx.x; i < nthreads * words; i += nthreads) bm[i] = 0u;
     for (int i = threadIdx.x; i < words; i += nthreads) pm[i] = 0u;
     for (int i = threadIdx.x; i < nl; i += nthreads) rows_of[i] = rowpos[j0 + i];
@@ -517,16 +526,18 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
             const unsigned c = ids[e];
             if (c < (unsigned)nthreads) {
                 const unsigned bit = 1u << (l & 31);
-                if (atomicOr(&bm[(size_t)c * words + (l >> 5)], bit) & bit) duplicate = 1u;
+                if (atomicOr(&bm[(size_t)c * words + (l >> 5)], bit) & bit) {
+                    const unsigned at = atomicAdd(&duplicates, 1u);
+                    if (at < dup_cap) chain[at] = (unsigned)l | atomicExch(&heads[c], at) << 16;
+                }
             }
             l += dl; k += dk;
             if (k >= K) { k -= K; ++l; }
         }
     }
     __syncthreads();
-    if (duplicate) {
-        // (uniform) a label lists a column twice -- rewiring draws such labels all the time -- and the bitmap has one bit
-        // for the two connections: here the column's thread walks its bitmap row in ascending label order and scans each
+    if (duplicates > dup_cap) {
+        // (uniform) more such connections than the chains hold: the column's thread walks its bitmap row in ascending label order and scans each
         // label found for the matching connections, which yields every connection, in ascending flat position
         const unsigned mine = mycol;
         const size_t sl = (size_t)t * nslices + (threadIdx.x >> 6);
@@ -584,7 +595,7 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
     {
         const unsigned mine = mycol;
         const unsigned* my = bm + (size_t)mine * words;
-        unsigned short* mp = pre + (size_t)mine * (words + 1) * 2;
+        unsigned short* mp = pre + (size_t)mine * words * 2;
         unsigned ev = 0, od = 0;
         for (int wd = 0; wd < words; ++wd) {
             mp[2 * wd] = (unsigned short)ev; mp[2 * wd + 1] = (unsigned short)od;
@@ -596,6 +607,12 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
         const unsigned rows = slice_off[sl + 1] - slice_off[sl];
         const size_t at = row0 * 64 + (threadIdx.x & 63);
         const unsigned first = parity_first(threadIdx.x);
+        for (unsigned h = heads[mine]; h != kNoEntry;) {
+            const unsigned entry = chain[h];
+            if (rows_of[entry & 0xffffu] & 1u) ++od;
+            else ++ev;
+            h = entry >> 16;
+        }
         const unsigned cnt[2] = {ev, od};
         for (unsigned r = 0; r < rows; ++r) {
             const unsigned par = (r & 1u) ^ first;          // bank half this slot belongs to
@@ -619,7 +636,16 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
                 const int wd = l >> 5;
                 const unsigned o = pm[wd];
                 const unsigned same = bm[(size_t)c * words + wd] & (par ? o : ~o) & ((1u << (l & 31)) - 1u);
-                const unsigned rank = pre[((size_t)c * (words + 1) + wd) * 2 + par] + __builtin_popcount(same);
+                unsigned rank = pre[((size_t)c * words + wd) * 2 + par] + __builtin_popcount(same);
+                bool again = false;
+                for (unsigned h = heads[c]; h != kNoEntry;) {
+                    const unsigned entry = chain[h], other = entry & 0xffffu;
+                    if (other < (unsigned)l && (rows_of[other] & 1u) == par) ++rank;
+                    again |= other == (unsigned)l;
+                    h = entry >> 16;
+                }
+                if (again)
+                    for (int i = 1; i <= k; ++i) rank += ids[e - i] == c ? 1u : 0u;
                 const unsigned thr = thread_of[c];
                 const unsigned slot = 2u * rank + (par ^ parity_first(thr));
                 const size_t at = (size_t)slice_off[(size_t)t * nslices + (thr >> 6)] * 64 + (thr & 63u) + (size_t)slot * 64;
@@ -632,13 +658,13 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
     }
 }
 
-// LDS the bitmap form needs, and may have
+// LDS the bitmap form needs without its chains' entries, and may have
 constexpr size_t kFillLdsLimit = 160 * 1024 - 64;
 inline size_t tile_fill_bitmap_lds(int threads, int tile_labels, int K, int* words_out) {
     const int words = ((tile_labels + 31) / 32) | 1;
     *words_out = words;
     return (size_t)threads * words * sizeof(unsigned) + (size_t)words * sizeof(unsigned) +
-           (size_t)threads * (words + 1) * 2 * sizeof(unsigned short) + (size_t)((tile_labels + 1) & ~1) * sizeof(unsigned short) +
+           (size_t)threads * words * 2 * sizeof(unsigned short) + (size_t)threads * sizeof(unsigned) + (size_t)((tile_labels + 1) & ~1) * sizeof(unsigned short) +
            (((size_t)tile_labels * K + 1) & ~(size_t)1) * sizeof(unsigned short) + (size_t)threads * sizeof(unsigned short);
 }
 
@@ -879,13 +905,15 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     }
     {
         int words = 0;
-        const size_t fill_lds = tile_fill_bitmap_lds(threads, TL, p->K, &words);
+        size_t fill_lds = tile_fill_bitmap_lds(threads, TL, p->K, &words);
         const unsigned pad_pos = w_in_lds ? (unsigned)TL * (unsigned)p->K : kPadPos;
         if (fill_lds <= kFillLdsLimit) {
+            const unsigned dup_cap = (unsigned)std::min<size_t>((size_t)threads * 4, (kFillLdsLimit - fill_lds) / sizeof(unsigned));
+            fill_lds += dup_cap * sizeof(unsigned);
             hipError_t ea = hipFuncSetAttribute((const void*)tile_fill_bitmap_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds);
             if (ea != hipSuccess) return hip_fail(ea);
             hipLaunchKernelGGL(tile_fill_bitmap_kernel, dim3(tiles), dim3(threads), fill_lds, s, lookup, p->rowpos, p->L, p->K, TL, 2 * cap,
-                               p->slice_off, p->lab16, p->pos16, pad_pos, p->slot32, words, p->col_lo, p->colperm);
+                               p->slice_off, p->lab16, p->pos16, pad_pos, p->slot32, words, p->col_lo, p->colperm, dup_cap);
         } else {
             hipLaunchKernelGGL(tile_fill_kernel, dim3(tiles), dim3(threads), 0, s, lookup, p->rowpos, p->L, p->K, TL, 2 * cap, p->slice_off,
                                p->lab16, p->pos16, pad_pos, p->slot32, p->col_lo, p->colperm);

@@ -356,6 +356,18 @@ def test_labels_that_list_a_column_twice(ffi):
     assert rel_err(hip_forward(ffi, x, lookup, w, False), oracle.forward(x, lookup, w)) <= FWD_RTOL
 
 
+# chains of a tile's repeated columns: none, some, one label in every tile that repeats most of its columns, three and more
+# times a column, and more than the chains hold (fan-in 32 over 40 columns); one-, two- and many-wavefront workgroups
+@pytest.mark.parametrize("N,L,K,B", [(768, 9000, 32, 128), (768, 9000, 32, 20), (512, 5000, 64, 40), (100, 3000, 8, 33), (40, 3000, 32, 33), (1100, 3000, 24, 64)])
+def test_plan_of_sources_drawn_with_replacement(ffi, N, L, K, B):
+    x, _, w, g = reference_law_inputs(B, N, L, K, seed=N + K)
+    lookup = np.random.default_rng(N).integers(0, N, size=(L, K)).astype(np.int32)
+    lookup[::250, : K // 2] = N - 1
+    gx, gw = hip_backward(ffi, x, lookup, w, g, False)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    assert rel_err(gx, o_gx) <= GRAD_RTOL and rel_err(gw, o_gw) <= GRAD_RTOL
+
+
 def test_skewed_lookup_uses_the_global_plan(ffi):
     # every connection points at one of two columns: the padded tiled plan would explode, the
     # library must fall back to the global column order and still be exact to tolerance
