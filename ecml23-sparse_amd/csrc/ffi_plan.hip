@@ -183,6 +183,15 @@ __device__ __forceinline__ unsigned column_slots(unsigned thread, unsigned even,
     return max(first ? 2u * first - 1u : 0u, 2u * second);
 }
 
+// The sum of v over the 64 lanes, in a scalar register.
+__device__ __forceinline__ int wave_total(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);         // lane ^ 1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);         // lane ^ 2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);        // 7 - lane within eight
+    v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);        // 15 - lane within sixteen
+    return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) + (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
+}
+
 // Which LDS row of the walking kernel's tile each label is staged into (rowpos[j], inside the label's tile).
 // The bank half a row lies in is the parity of its row number, and a column is walked fastest when its labels
 // split evenly between the halves (see above: every hole costs a slot).  The label's own parity would split a
@@ -253,43 +262,74 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         return (int)((ids3[jl * W + q] >> (10 * (k - 3 * q))) & 1023u);
     };
     int placed[2] = {0, 0};
+    // What bounds the kernel is the chain from one label's adds to the next label's decision: an LDS round trip and the sum
+    // over the lanes, by DPP (through the LDS crossbar, six round trips more: 615 us at 670,091 labels x fan-in 32; 317 so).
+    // With at most 64 connections a lane has one: its column is asked for two labels ahead, the column's weight one.
+    const bool one_each = K <= 64;
+    const unsigned* const my_ids = ids3 + (lane < K ? lane / 3 : 0);
+    const int my_shift = 10 * (lane % 3);
+    auto word_of = [&](int jl) { return my_ids[min(jl, nl - 1) * W]; };
+    int col1 = 0, w0 = 0;
+    unsigned word2 = 0;
+    auto column = [&](unsigned word) { return (int)((word >> my_shift) & 1023u); };
+    auto begin = [&]() {
+        col1 = column(word_of(0));
+        word2 = word_of(1);
+        w0 = lane < K ? (int)wt[col1] : 0;
+    };
+    // the balance that label jl asks for, after `back` (0: nothing) is added to its columns; then `decide` says what is added
+    auto step = [&](int jl, int back, auto decide) {
+        if (one_each) {
+            const int c = col1, w = w0;
+            if (back != 0 && lane < K) atomicAdd(&imb[c], back);
+            const int v = imb[c];
+            col1 = column(word2);
+            word2 = word_of(jl + 2);
+            w0 = lane < K ? (int)wt[col1] : 0;
+            const int delta = decide(wave_total(w * v));
+            if (lane < K) atomicAdd(&imb[c], delta);                                // (a column may occur twice in a label)
+        } else {
+            if (back != 0)
+                for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], back);
+            int sum = 0;
+            for (int k = lane; k < K; k += 64) { const int c = id_of(jl, k); sum += wt[c] * imb[c]; }
+            const int delta = decide(wave_total(sum));
+            for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], delta);
+        }
+    };
+    begin();
     for (int jl = 0; jl < nl; ++jl) {
-        int sum = 0;
-        for (int k = lane; k < K; k += 64) { const int c = id_of(jl, k); sum += wt[c] * imb[c]; }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        int color = sum > 0 ? 1 : (sum < 0 ? 0 : (placed[1] < placed[0] ? 1 : 0));
-        if (placed[color] >= cap) color ^= 1;
-        const int delta = color ? -1 : 1;
-        for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], delta);   // a column may occur twice in a label
-        if (lane == 0) half[jl] = (unsigned char)color;
-        ++placed[color];
+        step(jl, 0, [&](int sum) {
+            int color = sum > 0 ? 1 : (sum < 0 ? 0 : (placed[1] < placed[0] ? 1 : 0));
+            if (placed[color] >= cap) color ^= 1;
+            if (lane == 0) half[jl] = (unsigned char)color;
+            ++placed[color];
+            return color ? -1 : 1;
+        });
     }
     // Second sweep: every label is taken out and put back into the half its columns now ask for -- the first sweep placed
     // the early labels knowing nothing of the later ones.  (Measured on uniformly drawn ids, 586-label tiles of fan-in 32
     // over 768 columns: slot rows 1.528 -> 1.514 per connection, where columns of unconstrained order would need 1.490.)
+    begin();
+    int next_old = half[0];                               // (written by lane 0 above; LDS accesses of a wavefront are in order)
     for (int jl = 0; jl < nl; ++jl) {
-        const int old = half[jl];                         // (written by lane 0 above; LDS accesses of a wavefront are in order)
-        const int back = old ? 1 : -1;
-        for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], back);
-        int sum = 0;
-        for (int k = lane; k < K; k += 64) { const int c = id_of(jl, k); sum += wt[c] * imb[c]; }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        int color = sum > 0 ? 1 : (sum < 0 ? 0 : old);
-        if (color != old && placed[color] >= cap) color = old;
-        const int delta = color ? -1 : 1;
-        for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], delta);
-        if (color != old) { --placed[old]; ++placed[color]; if (lane == 0) half[jl] = (unsigned char)color; }
+        const int old = __builtin_amdgcn_readfirstlane(next_old);
+        next_old = half[min(jl + 1, nl - 1)];
+        step(jl, old ? 1 : -1, [&](int sum) {
+            int color = sum > 0 ? 1 : (sum < 0 ? 0 : old);
+            if (color != old && placed[color] >= cap) color = old;
+            if (color != old) { --placed[old]; ++placed[color]; if (lane == 0) half[jl] = (unsigned char)color; }
+            return color ? -1 : 1;
+        });
     }
     // rows of a half are handed out in ascending label order
-    if (lane == 0) {
-        int next[2] = {0, 0};
-        for (int jl = 0; jl < nl; ++jl) {
-            const int color = half[jl];
-            rowpos[j0 + jl] = (unsigned short)(2 * next[color] + color);
-            ++next[color];
-        }
+    int next[2] = {0, 0};
+    for (int l0 = 0; l0 < nl; l0 += 64) {
+        const bool on = l0 + lane < nl, odd = on && half[min(l0 + lane, nl - 1)] != 0;
+        const unsigned long long odds = __ballot(odd), evens = __ballot(on && !odd), before = (1ull << lane) - 1ull;
+        if (on) rowpos[j0 + l0 + lane] = (unsigned short)(2 * (next[odd] + __popcll((odd ? odds : evens) & before)) + (odd ? 1 : 0));
+        next[0] += __popcll(evens);
+        next[1] += __popcll(odds);
     }
 }
 
