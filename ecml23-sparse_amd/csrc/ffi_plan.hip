@@ -4,6 +4,7 @@
 // lookup[j,k] == n.  The plan lists those connections column by column so that they can be walked
 // sequentially, without atomics, in an order that never changes from run to run.
 #include "ffi_internal.h"
+#include "ffi_scan.h"
 #include "ffi_lds_tile.h"
 
 #include <algorithm>
@@ -333,6 +334,30 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     }
 }
 
+// Adds a tile's connections to cnt[half of the label's row][column].  Eight ids and the rows of their labels are on their way
+// at a time; labels by stepping, not division.
+__device__ __forceinline__ void count_halves(const int32_t* __restrict__ src, const unsigned short* __restrict__ row_of, int total, int K,
+                                             int col_lo, unsigned* cnt) {
+    constexpr int kInflight = 8;
+    const int nthreads = blockDim.x, dl = nthreads / K, dk = nthreads - dl * K;
+    int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
+    for (int e0 = threadIdx.x; e0 < total; e0 += nthreads * kInflight) {
+        unsigned c[kInflight], row[kInflight];
+#pragma unroll
+        for (int i = 0; i < kInflight; ++i) {
+            const bool on = e0 + i * nthreads < total;
+            c[i] = on ? (unsigned)(src[e0 + i * nthreads] - col_lo) : ~0u;
+            row[i] = on ? row_of[l] : 0u;
+            l += dl;
+            k += dk;
+            if (k >= K) { k -= K; ++l; }
+        }
+#pragma unroll
+        for (int i = 0; i < kInflight; ++i)
+            if (c[i] < (unsigned)nthreads) atomicAdd(&cnt[(row[i] & 1u) * nthreads + c[i]], 1u);
+    }
+}
+
 // Which column each thread of the walking kernel takes in each tile (plans with `colperm`).  A wavefront walks as many
 // slot rows as the longest of its 64 columns needs, so with thread t <-> column t every slice pays for its longest
 // column (about 1.5 slot rows per connection for ids drawn uniformly); here the tile's columns are sorted by the slots
@@ -340,7 +365,8 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
 // blocks dealt to the wavefronts so that the wavefronts of a SIMD (wave, wave + 4, wave + 8, ...) have about the same
 // rows in total: longest block first, each to the SIMD with the least so far that still has a wavefront free.
 // One workgroup per tile, one thread per column (columns up to the workgroup size exist for this purpose: the ones
-// beyond the input's width have no connections).  Also stores the slot rows of each slice, as tile_count_kernel does
+// beyond the input's width have no connections).  Bound by the comparison of every column with every other (two instructions
+// each) and the dealing, which four lanes do for the four SIMDs: 670,091 labels over 768 columns 157 -> 83 us.  Also stores the slot rows of each slice, as tile_count_kernel does
 // for plans without the permutation.  LDS: counts [2][threads], keys [threads].
 __global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
                                  int tile_labels, int col_lo, unsigned short* __restrict__ colperm, unsigned* __restrict__ slice_len) {
@@ -355,43 +381,41 @@ __global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned
     cnt[nthreads + threadIdx.x] = 0;
     __syncthreads();
     const int j0 = t * tile_labels;
-    const int nl = min(tile_labels, L - j0);
-    const int* src = idx + (size_t)j0 * K;
-    const int total = nl * K;
-    for (int e = threadIdx.x; e < total; e += nthreads) {
-        const unsigned c = (unsigned)(src[e] - col_lo);
-        if (c < (unsigned)nthreads) atomicAdd(&cnt[(rowpos[j0 + e / K] & 1u) * nthreads + c], 1u);
-    }
+    count_halves(idx + (size_t)j0 * K, rowpos + j0, min(tile_labels, L - j0) * K, K, col_lo, cnt);
     __syncthreads();
     // (the slots a column needs depend by one on the lane it gets; the larger of the two)
-    const unsigned mine = 2u * max(cnt[threadIdx.x], cnt[nthreads + threadIdx.x]);
+    // (with the column below it, so that no two keys are equal: columns of equal length stay in index order)
+    const unsigned mine = 2u * max(cnt[threadIdx.x], cnt[nthreads + threadIdx.x]) * 1024u + (1023u - threadIdx.x);
     key[threadIdx.x] = mine;
     __syncthreads();
-    // place among the columns in descending order of the key: columns with a larger key, and equal ones before this one
+    // place among the columns in descending order of the key
     unsigned place = 0;
+#pragma unroll 4
     for (int c0 = 0; c0 < nthreads; c0 += 4) {
         const uint4 k4 = *reinterpret_cast<const uint4*>(key + c0);       // (the same address in every lane: one broadcast read)
-        place += (k4.x > mine || (k4.x == mine && c0 + 0 < (int)threadIdx.x)) ? 1u : 0u;
-        place += (k4.y > mine || (k4.y == mine && c0 + 1 < (int)threadIdx.x)) ? 1u : 0u;
-        place += (k4.z > mine || (k4.z == mine && c0 + 2 < (int)threadIdx.x)) ? 1u : 0u;
-        place += (k4.w > mine || (k4.w == mine && c0 + 3 < (int)threadIdx.x)) ? 1u : 0u;
+        place += k4.x > mine ? 1u : 0u;
+        place += k4.y > mine ? 1u : 0u;
+        place += k4.z > mine ? 1u : 0u;
+        place += k4.w > mine ? 1u : 0u;
     }
     __syncthreads();
     // key[] now by place: the first of each block of 64 is the block's longest column
-    key[place] = mine;
+    key[place] = mine / 1024u;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned sum[4] = {0u, 0u, 0u, 0u};
-        int used[4] = {0, 0, 0, 0};
+    if (threadIdx.x < 64) {
+        // (four lanes are the SIMDs: their sums so far, wavefronts handed out)
+        unsigned sum = 0u;
+        int used = 0;
+        const int q = (int)threadIdx.x;
         for (int b = 0; b < nslices; ++b) {
-            int best = -1;
-            for (int q = 0; q < 4; ++q) {
-                if (q + 4 * used[q] >= nslices) continue;                 // no wavefront left on that SIMD
-                if (best < 0 || sum[q] < sum[best]) best = q;
+            unsigned best = (q < 4 && q + 4 * used < nslices) ? sum * 4u + (unsigned)q : ~0u;       // (none left on that SIMD: not taken)
+            best = min(best, (unsigned)__shfl_xor((int)best, 1, 64));
+            best = min(best, (unsigned)__shfl_xor((int)best, 2, 64));
+            if (q < 4 && (best & 3u) == (unsigned)q) {
+                wave_of_block[b] = (unsigned short)(q + 4 * used);
+                sum += (used == 0 ? 3u : 1u) * key[b * 64];              // (a SIMD's longest wavefront ends up walking alone)
+                ++used;
             }
-            wave_of_block[b] = (unsigned short)(best + 4 * used[best]);
-            sum[best] += (used[best] == 0 ? 3u : 1u) * key[b * 64];      // (a SIMD's longest wavefront ends up walking alone)
-            ++used[best];
         }
     }
     __syncthreads();
@@ -414,13 +438,7 @@ __global__ void tile_count_kernel(const int32_t* __restrict__ idx, const unsigne
     cnt[nthreads + threadIdx.x] = 0;
     __syncthreads();
     const int j0 = t * tile_labels;
-    const int nl = min(tile_labels, L - j0);
-    const int* src = idx + (size_t)j0 * K;
-    const int total = nl * K;
-    for (int e = threadIdx.x; e < total; e += nthreads) {
-        const unsigned c = (unsigned)(src[e] - col_lo);
-        if (c < (unsigned)nthreads) atomicAdd(&cnt[(rowpos[j0 + e / K] & 1u) * nthreads + c], 1u);
-    }
+    count_halves(idx + (size_t)j0 * K, rowpos + j0, min(tile_labels, L - j0) * K, K, col_lo, cnt);
     __syncthreads();
     const unsigned even = cnt[threadIdx.x], odd = cnt[nthreads + threadIdx.x];
     unsigned c = column_slots(threadIdx.x, even, odd);
@@ -429,25 +447,20 @@ __global__ void tile_count_kernel(const int32_t* __restrict__ idx, const unsigne
     if ((threadIdx.x & 63) == 0) slice_len[(size_t)t * (nthreads >> 6) + (threadIdx.x >> 6)] = c;
 }
 
-// Exclusive prefix sum of n values into off[0..n] by one workgroup (n is a few thousand).
+// Exclusive prefix sum of n values into off[0..n] by one workgroup (n is a few thousand); 25 us with the
+// threads' sums added up by one of them, 15 so).
 __global__ __launch_bounds__(1024) void slice_scan_kernel(const unsigned* __restrict__ len, unsigned* __restrict__ off,
                                                            int n, unsigned long long* __restrict__ total_out) {
-    __shared__ unsigned long long part[1024];
     const int per = (n + 1023) / 1024;
-    const int b = threadIdx.x * per, e = min(b + per, n);
-    unsigned long long sum = 0;
+    const int b = min((int)threadIdx.x * per, n), e = min(b + per, n);
+    unsigned long long sum = 0, total = 0;
     for (int i = b; i < e; ++i) sum += len[i];
-    part[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long run = 0;
-        for (int i = 0; i < 1024; ++i) { const unsigned long long v = part[i]; part[i] = run; run += v; }
-        *total_out = run;
-    }
-    __syncthreads();
-    unsigned long long run = part[threadIdx.x];
+    unsigned long long run = block_sum_below<1024>(sum, &total);
     for (int i = b; i < e; ++i) { off[i] = (unsigned)run; run += len[i]; }
-    if (threadIdx.x == 1023) off[n] = (unsigned)(part[1023] + sum);
+    if (threadIdx.x == 1023) {
+        off[n] = (unsigned)total;
+        *total_out = total;
+    }
 }
 
 // One workgroup per label tile, one thread per column n.  The tile's column ids pass through LDS
