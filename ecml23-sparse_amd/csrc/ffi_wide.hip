@@ -310,6 +310,9 @@ __global__ __launch_bounds__(kWalkThreads) void walk_columns_kernel(const float*
     }
 }
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
 // slot_w[slot] = the weight of the slot's connection (0 in padding).  Slots are dealt to the XCDs in eight consecutive
 // ranges: an XCD reads the weights of one label block after the other, which its L2 holds.
 __global__ __launch_bounds__(256) void slot_weights_kernel(const float* __restrict__ w, const int32_t* __restrict__ slot_pos,
@@ -318,14 +321,15 @@ __global__ __launch_bounds__(256) void slot_weights_kernel(const float* __restri
     if (u < 0) return;
     const size_t q = (size_t)u * 256 + threadIdx.x;
     if (q * 4 >= slots) return;
-    const int4 at = reinterpret_cast<const int4*>(slot_pos)[q];
-    float4 v;
+    // (what is touched once goes past the L2, which the gathered array needs: 395 -> 369 us at 670,091 labels x fan-in 72)
+    const v4i at = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(slot_pos) + q);
+    v4f v;
     v.x = w[max(at.x, 0)]; v.y = w[max(at.y, 0)]; v.z = w[max(at.z, 0)]; v.w = w[max(at.w, 0)];
     if (at.x < 0) v.x = 0.f;
     if (at.y < 0) v.y = 0.f;
     if (at.z < 0) v.z = 0.f;
     if (at.w < 0) v.w = 0.f;
-    reinterpret_cast<float4*>(slot_w)[q] = v;
+    __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(slot_w) + q);
 }
 
 // gw[pos] = gw_slots[pos_slot[pos]]; positions are dealt to the XCDs like the slots above.  (Reads at random places: the same
@@ -337,10 +341,10 @@ __global__ __launch_bounds__(256) void weight_grads_in_place_kernel(const float*
     const size_t p0 = ((size_t)u * 256 + threadIdx.x / 64 * 64) * 4 + (threadIdx.x & 63);
     float v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = gw_slots[pos_slot[min(p0 + 64 * i, count - 1)]];
+    for (int i = 0; i < 4; ++i) v[i] = gw_slots[__builtin_nontemporal_load(pos_slot + min(p0 + 64 * i, count - 1))];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (p0 + 64 * i < count) gw[p0 + 64 * i] = v[i];
+        if (p0 + 64 * i < count) __builtin_nontemporal_store(v[i], gw + p0 + 64 * i);
 }
 
 // gx ([N,B] or [B,N]) = sum over the streams of part[slice][stream][n][sl], ascending; 32 columns x 32 samples per workgroup
