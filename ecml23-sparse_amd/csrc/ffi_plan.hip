@@ -447,7 +447,7 @@ __global__ void tile_count_kernel(const int32_t* __restrict__ idx, const unsigne
     if ((threadIdx.x & 63) == 0) slice_len[(size_t)t * (nthreads >> 6) + (threadIdx.x >> 6)] = c;
 }
 
-// Exclusive prefix sum of n values into off[0..n] by one workgroup (n is a few thousand); 25 us with the
+// Exclusive prefix sum of n values into off[0..n] by one workgroup (n is a few thousand; 25 us with the
 // threads' sums added up by one of them, 15 so).
 __global__ __launch_bounds__(1024) void slice_scan_kernel(const unsigned* __restrict__ len, unsigned* __restrict__ off,
                                                            int n, unsigned long long* __restrict__ total_out) {
@@ -528,12 +528,12 @@ __global__ void tile_fill_kernel(const int32_t* __restrict__ idx, const unsigned
 // are written by threads <-> connections, not by a column's thread scanning for them.  Padding goes to the slots no
 // connection takes (a column's thread knows them from its two totals).  A label that lists one column twice sets one
 // bit for two connections -- sources drawn with replacement do so all the time, two labels in five at fan-in 32 over 768
-// columns.  The connections that find their bit set are kept in chains, one per column: a connection's rank then counts the
-// chain's entries with lower labels too, and, where its own label is among them, the equal ids in front of it in its row.
-// A chain is 0.5 entries on average there; beyond dup_cap entries in a tile (four per column, or what LDS is left) the
-// columns' threads place the tile (see below).
+// columns.  The connections that find their bit set are kept in chains, one per column, and a connection's rank then counts
+// the chain's entries in front of it too.  A chain is 0.5 entries on average there; beyond dup_cap entries in a tile (four per
+// column, or what LDS is left) the columns' threads place the tile (see below).
 // Measured at 670,091 labels x fan-in 32 over 768 columns: 6.2 ms by the scan of all pairs, 0.83 ms by the columns' threads
-// (0.19 without labels that list a column twice), 0.26 by chains.
+// (0.19 without labels that list a column twice), 0.21 by chains (0.26 where every connection looked through its label's row
+// for the equal ids in front of it); 501,070 labels x fan-in 64 over 512 columns: 0.66 by chains (0.97).
 __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
                                         int tile_labels, int zero_row, const unsigned* __restrict__ slice_off,
                                         unsigned short* __restrict__ lab16, unsigned short* __restrict__ pos16, unsigned pad_pos,
@@ -544,13 +544,14 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
     unsigned* bm = fill_lds;                                                   // [nthreads][words] (words odd: no bank conflicts)
     unsigned* pm = bm + (size_t)nthreads * words;                              // [words] labels staged in odd LDS rows
     unsigned* heads = pm + words;                                              // [nthreads] first entry of the column's chain
-    unsigned* chain = heads + nthreads;                                        // [dup_cap] label | next entry << 16
+    unsigned* chain = heads + nthreads;                                        // [dup_cap] connection | half of its label's row << 16 | next entry << 17
     unsigned short* pre = reinterpret_cast<unsigned short*>(chain + dup_cap);  // [nthreads][words][2] labels before word w, even / odd rows
     unsigned short* rows_of = pre + (size_t)nthreads * words * 2;              // [tile_labels]
     unsigned short* ids = rows_of + ((tile_labels + 1) & ~1);                  // [tile_labels * K]
     unsigned short* thread_of = ids + (((size_t)tile_labels * K + 1) & ~(size_t)1);   // [nthreads] the thread that walks each column
     __shared__ unsigned duplicates;
-    constexpr unsigned kNoEntry = 0xffffu;
+    __shared__ unsigned deep;
+    constexpr unsigned kNoEntry = 0x7fffu, kColumn = 0x3ffu, kMaxRank = 61u;
     // (bitmap and prefix counts are kept per column; slices, lanes and slot parities belong to threads)
     const unsigned mycol = colperm != nullptr ? colperm[(size_t)blockIdx.x * blockDim.x + threadIdx.x] : threadIdx.x;
     thread_of[mycol] = (unsigned short)threadIdx.x;
@@ -559,7 +560,7 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
     const int* src = idx + (size_t)j0 * K;
     const int total = nl * K;
     const int nslices = nthreads >> 6;
-    if (threadIdx.x == 0) duplicates = 0u;
+    if (threadIdx.x == 0) { duplicates = 0u; deep = 0u; }
     heads[threadIdx.x] = kNoEntry;
     for (int i = threadIdx.x; i < nthreads * words; i += nthreads) bm[i] = 0u;
     for (int i = threadIdx.x; i < words; i += nthreads) pm[i] = 0u;
@@ -581,7 +582,7 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
                 const unsigned bit = 1u << (l & 31);
                 if (atomicOr(&bm[(size_t)c * words + (l >> 5)], bit) & bit) {
                     const unsigned at = atomicAdd(&duplicates, 1u);
-                    if (at < dup_cap) chain[at] = (unsigned)l | atomicExch(&heads[c], at) << 16;
+                    if (at < dup_cap) chain[at] = (unsigned)e | (rows_of[l] & 1u) << 16 | atomicExch(&heads[c], at) << 17;
                 }
             }
             l += dl; k += dk;
@@ -589,7 +590,28 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
         }
     }
     __syncthreads();
-    if (duplicates > dup_cap) {
+    // The rank of a chained connection among the equal ones of its label: one of them is not in the chain (which one, the order
+    // of the atomics decides), so the label's row is looked through.  It is kept, plus one, above the ten bits of its column.
+    // The one that is not chained finds all that are in front of it in the chain.
+    const bool chained = duplicates <= dup_cap;
+    if (chained) {
+        for (unsigned i = threadIdx.x; i < duplicates; i += nthreads) {
+            const unsigned e = chain[i] & 0xffffu, l = e / (unsigned)K, c = ids[e];
+            const unsigned short* row_ids = ids + l * K;
+            unsigned before = 0;
+#pragma unroll 8
+            for (unsigned q = 0; q < e - l * K; ++q) before += (row_ids[q] & kColumn) == c ? 1u : 0u;
+            if (before > kMaxRank) deep = 1u;
+            else ids[e] = (unsigned short)(c | (before + 1u) << 10);
+        }
+    }
+    __syncthreads();
+    if (deep) {
+        for (int e = threadIdx.x; e < total; e += nthreads)
+            if (ids[e] != 0xffffu) ids[e] &= kColumn;
+        __syncthreads();
+    }
+    if (!chained || deep) {
         // (uniform) more such connections than the chains hold: the column's thread walks its bitmap row in ascending label order and scans each
         // label found for the matching connections, which yields every connection, in ascending flat position
         const unsigned mine = mycol;
@@ -662,9 +684,9 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
         const unsigned first = parity_first(threadIdx.x);
         for (unsigned h = heads[mine]; h != kNoEntry;) {
             const unsigned entry = chain[h];
-            if (rows_of[entry & 0xffffu] & 1u) ++od;
+            if (entry & 0x10000u) ++od;
             else ++ev;
-            h = entry >> 16;
+            h = entry >> 17;
         }
         const unsigned cnt[2] = {ev, od};
         for (unsigned r = 0; r < rows; ++r) {
@@ -682,23 +704,21 @@ __global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const u
         int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
         const int dl = nthreads / K, dk = nthreads - dl * K;
         for (int e = threadIdx.x; e < total; e += nthreads) {
-            const unsigned c = ids[e];
-            if (c < (unsigned)nthreads) {
+            const unsigned id = ids[e], c = id & kColumn;
+            if (id != 0xffffu) {
                 const unsigned row = rows_of[l];
                 const unsigned par = row & 1u;
                 const int wd = l >> 5;
                 const unsigned o = pm[wd];
                 const unsigned same = bm[(size_t)c * words + wd] & (par ? o : ~o) & ((1u << (l & 31)) - 1u);
                 unsigned rank = pre[((size_t)c * words + wd) * 2 + par] + __builtin_popcount(same);
-                bool again = false;
+                const unsigned in_label = id >> 10, front = in_label ? (unsigned)(e - k) : (unsigned)e;
                 for (unsigned h = heads[c]; h != kNoEntry;) {
-                    const unsigned entry = chain[h], other = entry & 0xffffu;
-                    if (other < (unsigned)l && (rows_of[other] & 1u) == par) ++rank;
-                    again |= other == (unsigned)l;
-                    h = entry >> 16;
+                    const unsigned entry = chain[h];
+                    rank += ((entry & 0xffffu) < front && (entry >> 16 & 1u) == par) ? 1u : 0u;
+                    h = entry >> 17;
                 }
-                if (again)
-                    for (int i = 1; i <= k; ++i) rank += ids[e - i] == c ? 1u : 0u;
+                rank += in_label ? in_label - 1u : 0u;
                 const unsigned thr = thread_of[c];
                 const unsigned slot = 2u * rank + (par ^ parity_first(thr));
                 const size_t at = (size_t)slice_off[(size_t)t * nslices + (thr >> 6)] * 64 + (thr & 63u) + (size_t)slot * 64;

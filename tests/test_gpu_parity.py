@@ -368,6 +368,18 @@ def test_plan_of_sources_drawn_with_replacement(ffi, N, L, K, B):
     assert rel_err(gx, o_gx) <= GRAD_RTOL and rel_err(gw, o_gw) <= GRAD_RTOL
 
 
+@pytest.mark.parametrize("repeats", [2, 62, 63, 100])
+def test_plan_of_a_label_that_repeats_a_column_often(ffi, repeats):
+    # (62 equal ids are what the slot placement ranks in place; a tile with more goes to the slow one)
+    B, N, L, K = 33, 256, 1500, 128
+    x, _, w, g = reference_law_inputs(B, N, L, K, seed=repeats)
+    lookup = np.argsort(np.random.default_rng(5).random((L, N)), axis=1)[:, :K].astype(np.int32)
+    lookup[700, K - repeats:] = 3
+    gx, gw = hip_backward(ffi, x, lookup, w, g, False)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    assert rel_err(gx, o_gx) <= GRAD_RTOL and rel_err(gw, o_gw) <= GRAD_RTOL
+
+
 def test_skewed_lookup_uses_the_global_plan(ffi):
     # every connection points at one of two columns: the padded tiled plan would explode, the
     # library must fall back to the global column order and still be exact to tolerance
