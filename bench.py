@@ -35,9 +35,9 @@ PASS_KERNELS = {
     "input_grad": "igrad_permute_weights_kernel + igrad_tile_kernel + igrad_reduce_kernel",
 }
 WIDE_PASS_KERNELS = {
-    "forward": "fwd_wide_kernel",
-    "weight_grad": "wgrad_wide_kernel",
-    "input_grad": "transpose_kernel + igrad_wide_kernel",
+    "forward": "slices_from_*_kernel + rows_by_range_kernel + fwd_phased_kernel, or fwd_sliced_kernel",
+    "weight_grad": "wgrad_wide_kernel alone, walk_columns_kernel<DOT> + weight_grads_in_place_kernel in a whole backward pass",
+    "input_grad": "slices_from_*_kernel + slot_weights_kernel + walk_columns_kernel + gather_gx_kernel",
 }
 
 
@@ -325,7 +325,7 @@ def bench_inference(args, pkg, synth, cfg):
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
         "config": {"workload": f"{cfg.name}: FFI layer forward + top-5 per sample, bf16 features and weights with fp32 accumulation, "
                                f"batch {B}, {N} inputs, {L} labels, fan-in {K} (sorted rows), features [N,B]"},
-        "roofline": {"bound": "hbm", "kernel": "forward pass (fwd_bf16_topk_kernel + topk_merge_kernel)", "achieved": round(achieved, 2),
+        "roofline": {"bound": "hbm", "kernel": "forward pass (rows_by_range_kernel + fwd_phased_kernel + topk_select_kernel)", "achieved": round(achieved, 2),
                      "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "traffic": traffic.get("forward"), "traffic_source": source, "algorithmic_bytes": alg,
                      "kernel_ms": {"forward": round(kernel_ms, 4)},

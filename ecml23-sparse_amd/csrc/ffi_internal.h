@@ -147,8 +147,6 @@ int launch_forward_loss(const float* x, const int32_t* idx, const float* w, cons
 // forward pass with per-sample top-k; the score matrix is written only if `scores` is given
 int launch_forward_topk(const float* x, const int32_t* idx, const float* w, const float* bias, float* scores, const TopkArgs& tk,
                         const Dims& d, hipStream_t s);
-int launch_forward_wide_bf16(const unsigned short* x, const int32_t* idx, const unsigned short* w, float* out, const Dims& d, hipStream_t s);
-int launch_forward_topk_wide_bf16(const unsigned short* x, const int32_t* idx, const unsigned short* w, const TopkArgs& tk, const Dims& d, hipStream_t s);
 // Top-k by a threshold (ffi_topk.hip): scores of a sample of the labels, the threshold of every sample of the batch, and the
 // candidates that reach it.  In a workspace of topk_candidate_bytes.
 constexpr int kTopkCap = 8192;          // candidate slots per sample

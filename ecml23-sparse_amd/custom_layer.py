@@ -190,13 +190,22 @@ class StratifiedRewireLayerV2(torch.nn.Module):
         returns ``other_vars`` (e.g. Adam moments, sparse/optimizer.py:14-23) with the entries at
         the rewired locations set to zero.  The index buffer is edited in place and the library is
         told so: it rebuilds its plan before the next backward call."""
-        other_vars = [] if other_vars is None else list(other_vars)
+        outputs = [] if other_vars is None else [other.clone().contiguous() for other in other_vars]
+        self._rewire_in_place(outputs)
+        return outputs
+
+    def rewires_in_place(self):
+        """Whether ``rewire`` does what it does here: a caller that would copy its result back over the variables may then
+        have them edited where they are (two copies of 86 MB each at 670,091 units of fan-in 32)."""
+        return type(self).rewire is StratifiedRewireLayerV2.rewire and "rewire" not in self.__dict__
+
+    @torch.no_grad()
+    def _rewire_in_place(self, variables):
         self._rewire_count += 1
         if hasattr(self.rewire_selector, "threshold_tensor"):
             # selection, redraw and clearing in the library: one threshold (radix select), one pass over the variables
             threshold = self.rewire_selector.threshold_tensor(self.kernel_weights.detach())
-            outputs = [other.clone().contiguous() for other in other_vars]
-            ops.rewire_connections(self.kernel_indices, self.kernel_weights.detach().contiguous(), [o.view(-1) for o in outputs],
+            ops.rewire_connections(self.kernel_indices, self.kernel_weights.detach().contiguous(), [v.view(-1) for v in variables],
                                    self.input_dim, threshold, self._rewire_seed + self._rewire_count)
         else:
             # a selector that only offers a boolean mask: the same steps as torch index operations
@@ -205,14 +214,10 @@ class StratifiedRewireLayerV2(torch.nn.Module):
                 self.kernel_indices[locations] = self._random_sources(locations.numel(), self.kernel_indices.device)
             if self.kernel_indices.is_cuda:
                 ops.lookup_edited(self.kernel_indices)
-            outputs = []
-            for other in other_vars:
-                new_v = other.clone()
-                new_v.reshape(-1)[locations] = 0
-                outputs.append(new_v)
+            for v in variables:
+                v.view(-1)[locations] = 0
         if self.arrange:
-            self.arrange_connections(outputs)
-        return outputs
+            self.arrange_connections(variables)
 
 
 class StratifiedRewireLayer(StratifiedRewireLayerV2):

@@ -62,7 +62,11 @@ class SparseAdam:
     def update_sparse(self, layer):
         if self.update_moments:
             i = self._index_of(layer.sparse_weights)
-            new_m, new_v = layer.rewire([self._momentums[i], self._velocities[i]])
+            moments = [self._momentums[i], self._velocities[i]]
+            if getattr(layer, "rewires_in_place", bool)() and all(m.is_contiguous() for m in moments):
+                layer._rewire_in_place(moments)
+                return
+            new_m, new_v = layer.rewire(moments)
             self._momentums[i].copy_(new_m)
             self._velocities[i].copy_(new_v)
         else:

@@ -151,3 +151,25 @@ def test_fused_train_step_follows_the_unfused_loop(ffi):
     assert np.allclose(l0, l1, rtol=1e-5)
     assert rel_err(w1, w0) <= 1e-5 and rel_err(b1, b0) <= 1e-5
     assert l0[2] < l0[0]
+
+
+def test_moments_are_rewired_in_place_or_through_an_override(ffi):
+    # the optimizer edits its moments where they are, unless the layer's rewire is not the library's
+    class Overridden(ffi.StratifiedRewireLayerV2):
+        def rewire(self, other_vars=None):
+            return super().rewire(other_vars)
+
+    results = []
+    for kind in (ffi.StratifiedRewireLayerV2, Overridden):
+        gen = torch.Generator(device="cuda").manual_seed(3)
+        layer = kind(units=300, input_dim=64, connections=300 * 24, generator=gen, rewire_selector=ffi.FixedFractionSelector(0.2))
+        opt = ffi.SparseAdam(list(layer.parameters()), learning_rate=0.01)
+        i = opt._index_of(layer.kernel_weights)
+        m, v = opt._momentums[i], opt._velocities[i]
+        m.normal_(generator=gen)
+        v.uniform_(generator=gen)
+        opt.update_sparse(layer)
+        assert opt._momentums[i] is m and int((m == 0).sum()) == 300 * 24 // 5
+        results.append((layer.kernel_indices, layer.kernel_weights.detach(), m, v))
+    assert layer.rewires_in_place() is False
+    assert all(torch.equal(a, b) for a, b in zip(*results))
