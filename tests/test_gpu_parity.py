@@ -380,6 +380,24 @@ def test_plan_of_a_label_that_repeats_a_column_often(ffi, repeats):
     assert rel_err(gx, o_gx) <= GRAD_RTOL and rel_err(gw, o_gw) <= GRAD_RTOL
 
 
+# the sums of many label streams: one to four samples per lane group of the split reduction, and one batch too large for it
+@pytest.mark.parametrize("B", [1, 32, 33, 64, 65, 128, 129])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_input_gradient_of_many_label_streams(ffi, B, transposed):
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        x, lookup, w, g = reference_law_inputs(B, 60, 40_000, 4, seed=B)
+        xin = np.ascontiguousarray(x.T) if transposed else x
+        gx, gw = hip_backward(ffi, xin, lookup, w, g, transposed)
+        o_gx, o_gw = oracle.backward(xin, lookup, w, g, transposed=transposed)
+        assert rel_err(gx, o_gx) <= GRAD_RTOL and rel_err(gw, o_gw) <= GRAD_RTOL
+        again, _ = hip_backward(ffi, xin, lookup, w, g, transposed)
+        assert np.array_equal(gx, again)
+    finally:
+        lib.ffi_set_option(b"small_path", 0)
+
+
 def test_skewed_lookup_uses_the_global_plan(ffi):
     # every connection points at one of two columns: the padded tiled plan would explode, the
     # library must fall back to the global column order and still be exact to tolerance
