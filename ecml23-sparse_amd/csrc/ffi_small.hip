@@ -128,9 +128,17 @@ __global__ __launch_bounds__(kSbThreads) void bwd_small_kernel(const float* __re
         if (!is_last) return;
         const unsigned* sums = partial + (size_t)unit * parts * window;
         for (int c = threadIdx.x; c < n; c += threads) {
-            float t = 0.f;
-#pragma unroll 8
-            for (int i = 0; i < parts; ++i) t += __uint_as_float(__hip_atomic_load(&sums[(size_t)i * window + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            // (eight running sums: one of up to 512 parts was further from the 64-bit result than the larger layers' path, 3.9e-7
+            // against 2.7e-7 at 1 x 768 x 131,072 x 32)
+            float t8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            for (int i0 = 0; i0 < parts; i0 += 8) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float v = __uint_as_float(__hip_atomic_load(&sums[(size_t)min(i0 + i, parts - 1) * window + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    t8[i] += i0 + i < parts ? v : 0.f;
+                }
+            }
+            const float t = ((t8[0] + t8[1]) + (t8[2] + t8[3])) + ((t8[4] + t8[5]) + (t8[6] + t8[7]));
             gx[tp ? (size_t)(n0 + c) * B + b : (size_t)b * N + n0 + c] = t;
         }
         return;
