@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     const int b0 = bt * kTileBatch;
     stage_rows32<kTileThreads, 8>(xs, xT, N, B, b0);       // (eight loads in flight per thread: the tile arrives in one round trip at 768 rows)
     if (TOPK && threadIdx.x < kTileBatch) local_count[threadIdx.x] = 0;
-    if (TOPK && threadIdx.x < kTileBatch)          // rows past the batch never qualify
+    if (TOPK && threadIdx.x < kTileBatch)          // (rows past the batch: a bound that few scores reach; +inf does, so the appends are bounded by nrows)
         tau_s[threadIdx.x] = b0 + (int)threadIdx.x < B ? ft.tau[b0 + threadIdx.x] : __builtin_inff();
     __syncthreads();
     const int lane = threadIdx.x & 63;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
                 if (__ballot(hit)) {
 #pragma unroll
                     for (int b = 8 * grp; b < 8 * grp + 8; ++b) {
-                        const bool h = valid && acc[b] >= tv[b];
+                        const bool h = valid && b < nrows && acc[b] >= tv[b];
                         if (__ballot(h)) {
                             if (h) {
                                 // parked in the workgroup's LDS segment of the sample (an LDS counter answers in a few dozen

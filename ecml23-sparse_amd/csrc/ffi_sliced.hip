@@ -152,16 +152,17 @@ struct TopkSink {
     int cap;
 };
 
-// The lane's scores of label j for samples b0 ...: few reach their threshold, so each takes its place with an atomic.
+// The lane's scores of label j for samples b0 ... b0 + n - 1: few reach their threshold, so each takes its place with an atomic.
+// n bounds the samples, not a threshold that no score reaches: +inf reaches every threshold.
 template <int PER>
-__device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&a)[PER], const float (&tau)[PER], int b0, int j, bool valid) {
+__device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&a)[PER], const float (&tau)[PER], int b0, int n, int j, bool valid) {
     bool hit = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) hit |= a[i] >= tau[i];
     if (!valid || !hit) return;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        if (a[i] >= tau[i]) {
+        if (i < n && a[i] >= tau[i]) {
             const int slot = atomicAdd(&sink.count[(size_t)(b0 + i) * kTopkCountStep], 1);
             if (slot < sink.cap) {
                 sink.val[(size_t)(b0 + i) * sink.cap + slot] = a[i];
@@ -170,10 +171,11 @@ __device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&
         }
     }
 }
+// the thresholds of the n samples (n may be <= 0) from b0 on; for the rest of the lane's one that few scores reach
 template <int PER>
-__device__ __forceinline__ void topk_thresholds(const TopkSink& sink, int b0, int B, float (&tau)[PER]) {
+__device__ __forceinline__ void topk_thresholds(const TopkSink& sink, int b0, int n, float (&tau)[PER]) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) tau[i] = b0 + i < B ? sink.tau[b0 + i] : __builtin_inff();
+    for (int i = 0; i < PER; ++i) tau[i] = i < n ? sink.tau[b0 + i] : __builtin_inff();
 }
 
 template <int GL, bool BF16, int SLICES, bool QUADS>
@@ -308,9 +310,10 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
     if (sink.tau != nullptr) {
 #pragma unroll
         for (int p = 0; p < SLICES; ++p) {
-            const int b0 = (slice0 + p) * kSl + sub * kPer;                // (beyond the last slice: no threshold is reached)
+            if (slice0 + p >= slices) break;                               // (a workgroup's surplus slices repeat the last one)
+            const int b0 = (slice0 + p) * kSl + sub * kPer;
             float tau[kPer];
-            topk_thresholds(sink, b0, B, tau);
+            topk_thresholds(sink, b0, B - b0, tau);
 #pragma unroll
             for (int q = 0; q < S::kRounds; ++q) {
                 const int j = first_label(q) + grp;
@@ -319,7 +322,7 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) acc[q][p].a[i] += bj;
                 }
-                topk_append(sink, acc[q][p].a, tau, b0, j, j < L);
+                topk_append(sink, acc[q][p].a, tau, b0, B - b0, j, j < L);
             }
         }
         return;
@@ -414,7 +417,8 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
     const int blocks = (L + S::kWaveLabels - 1) / S::kWaveLabels, step = streams * kWaves;
     const int b0 = slice * kSl, nb = min(kSl, B - b0);
     float tau[kPer];
-    if (sink.tau != nullptr) topk_thresholds(sink, b0 + sub * kPer, B, tau);
+    const int mine0 = b0 + sub * kPer;                                    // first sample of this lane
+    if (sink.tau != nullptr) topk_thresholds(sink, mine0, B - mine0, tau);
 
     uint4 ids[S::kQuads], ws[S::kQuads];
     auto place = [&](unsigned f, int n, int& l, int& k) {
@@ -513,7 +517,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) acc[q].a[i] += bj;
                 }
-                topk_append(sink, acc[q].a, tau, b0 + sub * kPer, j, j < L);
+                topk_append(sink, acc[q].a, tau, mine0, B - mine0, j, j < L);
             }
             continue;
         }
@@ -739,8 +743,9 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
     __syncthreads();
     const int b0 = slice * kSl;
     if (sink.tau != nullptr) {
+        const int mine0 = b0 + sub * kPer;               // first sample of this lane
         float tau[kPer];
-        topk_thresholds(sink, b0 + sub * kPer, B, tau);
+        topk_thresholds(sink, mine0, B - mine0, tau);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             const int j = jw + m * 8 + grp;
@@ -749,7 +754,7 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) acc[m].a[i] += bj;
             }
-            topk_append(sink, acc[m].a, tau, b0 + sub * kPer, j, j < L);
+            topk_append(sink, acc[m].a, tau, mine0, B - mine0, j, j < L);
         }
         return;
     }

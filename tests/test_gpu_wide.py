@@ -116,3 +116,51 @@ def test_topk_by_threshold(ffi, bf16, B, N, L, K, tied):
     assert float((torch.gather(scores, 1, idx.long()) - val).abs().max()) <= 1e-5 * float(best.abs().max())
     if tied:
         assert torch.equal(idx.cpu().long(), torch.arange(k).expand(B, k))
+
+
+# Scores that are infinite or no number, in every kernel that collects candidates: samples behind the batch's end and slices
+# behind the last (three where a workgroup serves two or four) reach no list.  (B, N, L, K, wide_phases): slices in LDS, gathered
+# from L2, in phases; the 32-sample tile
+NONFINITE_SHAPES = [(5, 768, 20_000, 8, 0), (96, 4096, 9_001, 5, 0), (33, 1300, 17_000, 6, 0), (160, 4096, 9_001, 12, 0), (70, 5000, 3_000, 20, 1),
+                    (130, 2000, 5_000, 16, 1), (40, 768, 20_000, 12, 0)]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("shape", NONFINITE_SHAPES)
+@pytest.mark.parametrize("n_inf", [2, 40])
+def test_topk_of_scores_that_are_not_finite(ffi, bf16, shape, n_inf):
+    B, N, L, K, phases = shape
+    k = 5
+    x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + N)
+    x = np.abs(x) + 0.5                                        # (a weight of +inf gives +inf, and one of -inf gives -inf)
+    rng = np.random.default_rng(L)
+    special = rng.permutation(L)
+    bias = np.zeros(L, np.float32)
+    at = w if bf16 else bias                                   # (no bias beside bf16 scores)
+    for labels, value in ((special[:n_inf], np.inf), (special[n_inf:n_inf + L // 3], -np.inf), (special[-L // 10:], np.nan)):
+        if bf16: at[labels, 0] = value
+        else: at[labels] = value
+    dx, dl, dw, db = dev(x), dev(lookup), dev(w), dev(bias)
+    print(f"case {shape} bf16={bf16} n_inf={n_inf}", flush=True)
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_phases", phases) == 0
+    try:
+        if bf16:
+            dx, dw = dx.bfloat16(), dw.bfloat16()
+            scores = ffi.fan_in_sparse_matmul_bf16(dx, dl, dw)
+            val, idx = ffi.fan_in_sparse_topk_bf16(dx, dl, dw, k=k)
+        else:
+            scores = ffi.fan_in_sparse_matmul_bias(dx, dl, dw, db)
+            val, idx = ffi.fan_in_sparse_topk(dx, dl, dw, db, k=k)
+    finally:
+        lib.ffi_set_option(b"wide_phases", 0)
+    scores, val, idx = scores.cpu().numpy(), val.cpu().numpy(), idx.cpu().numpy()
+    infinite = np.sort(special[:n_inf])[:k]
+    assert np.isposinf(scores[:, special[:n_inf]]).all() and np.isnan(scores).sum() == B * len(special[-L // 10:])
+    n = len(infinite)
+    assert np.isposinf(val[:, :n]).all() and (idx[:, :n] == infinite).all()
+    # the finite rest: the best of the scores without NaN (possibly summed in another order)
+    rest = np.where(np.isfinite(scores), scores, -np.inf)
+    best = -np.sort(-rest, axis=1)[:, :k - n]
+    assert np.abs(val[:, n:] - best).max(initial=0.0) <= 1e-5 * np.abs(rest[np.isfinite(rest)]).max()
+    assert np.abs(np.take_along_axis(scores, idx[:, n:].astype(np.int64), 1) - val[:, n:]).max(initial=0.0) <= 1e-5 * np.abs(rest[np.isfinite(rest)]).max()
