@@ -86,6 +86,7 @@ constexpr int kTopkPark = 24;           // candidates per (workgroup, batch row)
 // few thousand entries out of all labels, and a small kernel selects the k best afterwards.
 struct FwdTopk {
     const float* tau;     // [B]
+    int* tie;             // [B] see TopkCandidates
     int* count;           // [B] candidates appended so far (may run past cap: the list is then incomplete)
     float* cand_val;      // [B][cap]
     int* cand_idx;        // [B][cap]
@@ -264,14 +265,16 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
                     for (int b = 8 * grp; b < 8 * grp + 8; ++b) {
                         const bool h = valid && b < nrows && acc[b] >= tv[b];
                         if (__ballot(h)) {
-                            if (h) {
+                            int tie = kTopkListFull;
+                            if (h) tie = ft.tie[b0 + b];
+                            if (h && topk_reaches(acc[b], j, tv[b], tie)) {
                                 // parked in the workgroup's LDS segment of the sample (an LDS counter answers in a few dozen
                                 // clocks, a global one in microseconds); a full segment sends the entry to memory directly
                                 const int lslot = atomicAdd(&local_count[b], 1);
                                 if (lslot < kTopkPark) {
                                     local_cand[b * kTopkPark + lslot] = make_int2(j, __float_as_int(acc[b]));
                                 } else {
-                                    const int slot = atomicAdd(&ft.count[(size_t)(b0 + b) * kTopkCountStep], 1);
+                                    const int slot = topk_slot(acc[b], j, tv[b], tie, &ft.tie[b0 + b], &ft.count[(size_t)(b0 + b) * kTopkCountStep], ft.cap);
                                     if (slot < ft.cap) {
                                         ft.cand_val[(size_t)(b0 + b) * ft.cap + slot] = acc[b];
                                         ft.cand_idx[(size_t)(b0 + b) * ft.cap + slot] = j;
@@ -533,14 +536,14 @@ bool lane64_fits(const Dims& d) {
 
 namespace {
 
-constexpr int kTopkSample = 4096;      // labels whose scores set the per-sample thresholds
+constexpr int kTopkSampleBits = 12, kTopkSample = 1 << kTopkSampleBits;      // labels whose scores set the per-sample thresholds
 
-// scores of every (L / S)-th label for all samples: sample_scores[b][i] (the thresholds' raw material)
+// scores of S labels, evenly spaced, for all samples: sample_scores[b][i] (the thresholds' raw material)
 __global__ __launch_bounds__(256) void fwd_sample_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
                                                          const float* __restrict__ w, const float* __restrict__ bias, int B, int N,
-                                                         int L, int K, int S, float* __restrict__ sample_scores) {
+                                                         int K, int S, TopkSampleLabels labels, float* __restrict__ sample_scores) {
     const int i = blockIdx.x;
-    const int j = (int)(((long long)i * L) / S);
+    const int j = (int)(((long long)i * labels.num) >> labels.shift);
     const int32_t* irow = idx + (size_t)j * K;
     const float* wrow = w + (size_t)j * K;
     for (int b = threadIdx.x; b < B; b += 256) {
@@ -622,14 +625,15 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
     if (topk) {
         // thresholds: the k-th best score of every sample among kTopkSample evenly spaced labels
         const int S = std::min(kTopkSample, d.L);
+        const TopkSampleLabels labels = d.L > S ? TopkSampleLabels{d.L, kTopkSampleBits} : TopkSampleLabels{1, 0};
         void* ws = nullptr;
         FFI_TRY(workspace_get(s, kWsTopk, topk_candidate_bytes(d.B, S), &ws));
         tc = topk_candidates_at(ws, d.B, S);
-        hipLaunchKernelGGL(fwd_sample_kernel, dim3(S), dim3(256), 0, s, xT, idx, w, bias, d.B, d.N, d.L, d.K, S, tc.sample);
+        hipLaunchKernelGGL(fwd_sample_kernel, dim3(S), dim3(256), 0, s, xT, idx, w, bias, d.B, d.N, d.K, S, labels, tc.sample);
         FFI_HIP_TRY(hipGetLastError());
-        FFI_TRY(launch_topk_threshold(tc.sample, (size_t)S, 1, S, tk->k, tc, d.B, s));
+        FFI_TRY(launch_topk_threshold(tc.sample, (size_t)S, 1, S, labels, tk->k, tc, d.B, s));
         // LDS behind the tile of x holds the workgroup's candidates until the end of the kernel
-        ft = FwdTopk{tc.tau, tc.count, tc.val, tc.idx, kTopkCap};
+        ft = FwdTopk{tc.tau, tc.tie, tc.count, tc.val, tc.idx, kTopkCap};
         lds_topk = lds + (size_t)kTileBatch * kTopkPark * sizeof(int2);
     }
     int npartial = 0;

@@ -153,15 +153,33 @@ constexpr int kTopkCap = 8192;          // candidate slots per sample
 constexpr int kTopkCountStep = 32;      // ints between the samples' counters: a cache line each
 struct TopkCandidates {
     float* sample;     // [B][S]
-    float* tau;        // [B]
-    int* count;        // [B] candidates appended so far (may run past the cap: the list is then incomplete)
+    float* tau;        // [B] the threshold is the pair (tau, tie): scores above tau reach it, and scores of tau of labels up to tie
+    int* tie;          // [B]
+    int* count;        // [B] candidates appended so far (may run past the cap: the list is then incomplete); the int behind each
+                       // counts the workgroups that have scanned the row of such a sample
     float* val;        // [B][kTopkCap]
     int* idx;
 };
+#if defined(__HIPCC__)
+__device__ __forceinline__ bool topk_reaches(float score, int label, float tau, int tie) { return score > tau || (score == tau && label <= tie); }
+// A place in a sample's candidate list for a score of at least tau, or one behind its end (none).  Whoever finds the list full
+// leaves a mark in place of the threshold's label, in `known` and in memory, where those that load it later see it: a full
+// list's counter is asked about once per lane, not for every label.  `known` is loaded beside tau, ahead of the scores: a load in
+// front of the append, of this word or of the counter, took 33 and 60 us of 2,560 at 512 x 100,000 x 670,091 x 64 in bf16.
+constexpr int kTopkListFull = -1;
+__device__ __forceinline__ int topk_slot(float score, int label, float tau, int& known, int* tie, int* count, int cap) {
+    if (known == kTopkListFull || !topk_reaches(score, label, tau, known)) return cap;
+    const int slot = atomicAdd(count, 1);
+    if (slot >= cap) { known = kTopkListFull; *tie = kTopkListFull; }
+    return slot;
+}
+#endif
 size_t topk_candidate_bytes(int B, int sample);
 TopkCandidates topk_candidates_at(void* ws, int B, int sample);
-// tau and count from sample scores: scores[b * row + i * step], i < S
-int launch_topk_threshold(const float* scores, size_t row, int step, int S, int k, const TopkCandidates& c, int B, hipStream_t s);
+// threshold and count from sample scores: scores[b * row + i * step], i < S
+struct TopkSampleLabels { int num, shift; };      // label of sample i: (i * num) >> shift
+int launch_topk_threshold(const float* scores, size_t row, int step, int S, TopkSampleLabels labels, int k, const TopkCandidates& c, int B,
+                          hipStream_t s);
 // Where the scores of a whole row come from when a sample's candidate list has overflowed: the score matrix [B,L],
 // or (scores == null) the layer itself.
 struct TopkRowSource {

@@ -146,6 +146,7 @@ template <> struct LaneAcc<true> {
 // Where a forward kernel that keeps no scores puts those at or above their sample's threshold.
 struct TopkSink {
     const float* tau;              // [B]; null: the kernel stores scores
+    int* tie;                      // [B] see TopkCandidates
     int* count;                    // [B] entries appended
     float* val;                    // [B][cap]
     int* idx;
@@ -155,15 +156,16 @@ struct TopkSink {
 // The lane's scores of label j for samples b0 ... b0 + n - 1: few reach their threshold, so each takes its place with an atomic.
 // n bounds the samples, not a threshold that no score reaches: +inf reaches every threshold.
 template <int PER>
-__device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&a)[PER], const float (&tau)[PER], int b0, int n, int j, bool valid) {
+__device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&a)[PER], const float (&tau)[PER], int* tie, int b0, int n, int j, bool valid) {
     bool hit = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) hit |= a[i] >= tau[i];
     if (!valid || !hit) return;
+    asm volatile("" : "+v"(b0));              // keeps the samples' addresses from being formed ahead of the label loop (48 registers in bf16: spilled, 5 x 22 x 60,520 x 5 took 15 us, now 8)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         if (i < n && a[i] >= tau[i]) {
-            const int slot = atomicAdd(&sink.count[(size_t)(b0 + i) * kTopkCountStep], 1);
+            const int slot = topk_slot(a[i], j, tau[i], tie[i], &sink.tie[b0 + i], &sink.count[(size_t)(b0 + i) * kTopkCountStep], sink.cap);
             if (slot < sink.cap) {
                 sink.val[(size_t)(b0 + i) * sink.cap + slot] = a[i];
                 sink.idx[(size_t)(b0 + i) * sink.cap + slot] = j;
@@ -171,11 +173,17 @@ __device__ __forceinline__ void topk_append(const TopkSink& sink, const float (&
         }
     }
 }
-// the thresholds of the n samples (n may be <= 0) from b0 on; for the rest of the lane's one that few scores reach
+// The thresholds of the samples from b0 on, four per load; nothing is done with them here, so that nobody waits for them.
+// (Behind the batch's end: of samples that are not there, see topk_candidates_at.)
 template <int PER>
-__device__ __forceinline__ void topk_thresholds(const TopkSink& sink, int b0, int n, float (&tau)[PER]) {
+__device__ __forceinline__ void topk_thresholds(const TopkSink& sink, int b0, float (&tau)[PER], int (&tie)[PER]) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) tau[i] = i < n ? sink.tau[b0 + i] : __builtin_inff();
+    for (int i = 0; i < PER; i += 4) {
+        const float4 t = *reinterpret_cast<const float4*>(sink.tau + b0 + i);
+        const int4 e = *reinterpret_cast<const int4*>(sink.tie + b0 + i);
+        tau[i] = t.x; tau[i + 1] = t.y; tau[i + 2] = t.z; tau[i + 3] = t.w;
+        tie[i] = e.x; tie[i + 1] = e.y; tie[i + 2] = e.z; tie[i + 3] = e.w;
+    }
 }
 
 template <int GL, bool BF16, int SLICES, bool QUADS>
@@ -313,7 +321,8 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
             if (slice0 + p >= slices) break;                               // (a workgroup's surplus slices repeat the last one)
             const int b0 = (slice0 + p) * kSl + sub * kPer;
             float tau[kPer];
-            topk_thresholds(sink, b0, B - b0, tau);
+            int tie[kPer];
+            topk_thresholds(sink, b0, tau, tie);
 #pragma unroll
             for (int q = 0; q < S::kRounds; ++q) {
                 const int j = first_label(q) + grp;
@@ -322,7 +331,7 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) acc[q][p].a[i] += bj;
                 }
-                topk_append(sink, acc[q][p].a, tau, b0, B - b0, j, j < L);
+                topk_append(sink, acc[q][p].a, tau, tie, b0, B - b0, j, j < L);
             }
         }
         return;
@@ -360,7 +369,8 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
 // 16 GL bytes and half a list entry of 16 per connection and lane group).
 typedef unsigned lds_v4u __attribute__((ext_vector_type(4)));
 constexpr int kLdThreads = 1024;
-constexpr size_t kLdBudget = 160 * 1024 - 512;
+constexpr size_t kLdThresholdBytes = 512;       // (behind the rest: thresholds of up to 64 samples, which would take 16 registers through the label loop)
+constexpr size_t kLdBudget = 160 * 1024 - kLdThresholdBytes;
 
 template <int GL> struct LdsShape {
     static constexpr int kGroups = 64 / GL;
@@ -406,6 +416,12 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
         }
         if (threadIdx.x < GL) reinterpret_cast<uint4*>(smem)[N * GL + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);    // what entries behind a list's end name
     }
+    float* const slice_tau = reinterpret_cast<float*>(smem + (size_t)(N + 1) * kRow + (size_t)kWaves * S::kWaveBytes);
+    int* const slice_tie = reinterpret_cast<int*>(slice_tau + kSl);
+    if (sink.tau != nullptr && threadIdx.x < kSl) {
+        slice_tau[threadIdx.x] = sink.tau[slice * kSl + threadIdx.x];
+        slice_tie[threadIdx.x] = sink.tie[slice * kSl + threadIdx.x];
+    }
     __syncthreads();
     unsigned char* const mine = smem + (size_t)(N + 1) * kRow + (size_t)wave * S::kWaveBytes;
     uint2* list = reinterpret_cast<uint2*>(mine);
@@ -416,9 +432,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
     const unsigned short* w16 = reinterpret_cast<const unsigned short*>(w);
     const int blocks = (L + S::kWaveLabels - 1) / S::kWaveLabels, step = streams * kWaves;
     const int b0 = slice * kSl, nb = min(kSl, B - b0);
-    float tau[kPer];
     const int mine0 = b0 + sub * kPer;                                    // first sample of this lane
-    if (sink.tau != nullptr) topk_thresholds(sink, mine0, B - mine0, tau);
 
     uint4 ids[S::kQuads], ws[S::kQuads];
     auto place = [&](unsigned f, int n, int& l, int& k) {
@@ -509,6 +523,9 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
             }
         }
         if (sink.tau != nullptr) {
+            float tau[kPer];
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) tau[i] = slice_tau[sub * kPer + i];
 #pragma unroll
             for (int q = 0; q < S::kRounds; ++q) {
                 const int j = jb + q * S::kGroups + grp;
@@ -517,7 +534,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) acc[q].a[i] += bj;
                 }
-                topk_append(sink, acc[q].a, tau, mine0, B - mine0, j, j < L);
+                topk_append(sink, acc[q].a, tau, slice_tie + sub * kPer, mine0, B - mine0, j, j < L);
             }
             continue;
         }
@@ -745,7 +762,8 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
     if (sink.tau != nullptr) {
         const int mine0 = b0 + sub * kPer;               // first sample of this lane
         float tau[kPer];
-        topk_thresholds(sink, mine0, B - mine0, tau);
+        int tie[kPer];
+        topk_thresholds(sink, mine0, tau, tie);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             const int j = jw + m * 8 + grp;
@@ -754,7 +772,7 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) acc[m].a[i] += bj;
             }
-            topk_append(sink, acc[m].a, tau, mine0, B - mine0, j, j < L);
+            topk_append(sink, acc[m].a, tau, tie, mine0, B - mine0, j, j < L);
         }
         return;
     }
@@ -839,7 +857,8 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
     const int chunks = (d.K + S::kChunk - 1) / S::kChunk, chunk = ((d.K + chunks - 1) / chunks + 3) / 4 * 4;
     const int blocks = (d.L + S::kWaveLabels - 1) / S::kWaveLabels, waves = kLdThreads / 64;
     const int streams = std::max(1, std::min((blocks + waves - 1) / waves, device_cu_count() / a.slices));
-    const size_t lds = lds_kernel_bytes<GL>(d.N);
+    const size_t lds = lds_kernel_bytes<GL>(d.N) + (a.sink.tau != nullptr ? kLdThresholdBytes : 0);
+    static_assert(2 * GL * LaneAcc<BF16>::kSamples * 4 <= kLdThresholdBytes, "thresholds of a slice");
     const dim3 grid((unsigned)(streams * a.slices)), block(kLdThreads);
     if (a.quads) {
         FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lds_kernel<GL, BF16, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1013,8 +1032,8 @@ int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const 
         FFI_HIP_TRY(hipGetLastError());
         FFI_TRY(forward_wide<BF16>(table, sample_idx, sample_w, bias ? sample_bias : nullptr, c.sample, TopkSink{}, ds, s));
     }
-    FFI_TRY(launch_topk_threshold(c.sample, (size_t)S, 1, S, tk.k, c, d.B, s));
-    FFI_TRY(forward_wide<BF16>(table, idx, w, bias, nullptr, TopkSink{c.tau, c.count, c.val, c.idx, kTopkCap}, d, s));
+    FFI_TRY(launch_topk_threshold(c.sample, (size_t)S, 1, S, TopkSampleLabels{step, 0}, tk.k, c, d.B, s));
+    FFI_TRY(forward_wide<BF16>(table, idx, w, bias, nullptr, TopkSink{c.tau, c.tie, c.count, c.val, c.idx, kTopkCap}, d, s));
     TopkRowSource src;
     src.x = x; src.tp = d.tp; src.bf16 = BF16; src.idx = idx; src.w = w; src.bias = bias; src.N = d.N; src.L = d.L; src.K = d.K;
     return launch_topk_select(c, d.B, tk, src, s);

@@ -4,8 +4,12 @@
 //
 // Long rows take a threshold: the k best of the maxima of disjoint groups of a sample of the labels are scores of k labels,
 // so the least of them is a bound that the k best scores of the row reach.  One pass collects the few scores at or above it
-// (about k L / S of L labels for a sample of S), and the k best of those are the answer.  Exact; a sample whose candidates
-// do not fit its list (thousands of labels tied at the top) is answered from its whole row.
+// (about k L / S of L labels for a sample of S), and the k best of those are the answer.  Exact.
+// Best and least are those of the order the answer is in, score and then label: of the labels whose scores equal the bound,
+// only those up to the bound's own label are collected, so a row of equal scores (a sample without features) is no longer a
+// list than any other.  (By score alone such a row was answered from the whole layer: one of 512 in bf16, 100,000 x 670,091 x 64,
+// took 70 ms in place of 2.7.)  What can still outgrow a list -- thousands of labels above all that the sample holds -- is
+// answered from the whole row by many workgroups together.
 #include "ffi_internal.h"
 #include "ffi_loss.h"
 
@@ -47,21 +51,38 @@ struct TopList {
     }
 };
 
-// The 64 lanes hold sorted lists; kTopMax rounds in which the best head (found with shuffles) is taken by lane `round` and
-// popped by its owner.  Afterwards lane s < 8 holds the s-th best in out_*.
+// The largest of the lanes' values (none of them NaN), and the smallest of their ids, in every lane: over sixteen lanes by DPP,
+// whose steps cost what an addition costs, then over the four rows.
+template <int CTRL> __device__ __forceinline__ int dpp_of(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false); }
+template <int CTRL> __device__ __forceinline__ float dpp_of(float v) { return __int_as_float(dpp_of<CTRL>(__float_as_int(v))); }
+__device__ __forceinline__ float wave_largest(float v) {
+    v = fmaxf(v, dpp_of<0xb1>(v));          // lane ^ 1
+    v = fmaxf(v, dpp_of<0x4e>(v));          // lane ^ 2
+    v = fmaxf(v, dpp_of<0x141>(v));         // 7 - lane within eight
+    v = fmaxf(v, dpp_of<0x140>(v));         // 15 - lane within sixteen
+    const int i = __float_as_int(v);
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))),
+                 fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));
+}
+__device__ __forceinline__ int wave_smallest(int v) {
+    v = min(v, dpp_of<0xb1>(v));
+    v = min(v, dpp_of<0x4e>(v));
+    v = min(v, dpp_of<0x141>(v));
+    v = min(v, dpp_of<0x140>(v));
+    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// The 64 lanes hold sorted lists; kTopMax rounds in which the best head is taken by lane `round` and popped by its owner.
+// Afterwards lane s < 8 holds the s-th best in out_*.  (A round is a chain of twenty-odd instructions; through shuffles of score
+// and label it took several times that, and the kernels below are little else: 10 -> 7 us for the thresholds of one sample.)
 __device__ __forceinline__ void wave_topk(TopList& l, int rounds, float& out_v, int& out_i) {
     const int lane = threadIdx.x & 63;
     out_v = -__builtin_inff();
     out_i = kNoId;
     for (int s = 0; s < rounds; ++s) {
-        float bv = l.v[0];
-        int bi = l.id[0];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off, 64);
-            const int oi = __shfl_xor(bi, off, 64);
-            if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-        }
+        const float bv = wave_largest(l.v[0]);
+        const int bi = wave_smallest(l.v[0] == bv ? l.id[0] : kNoId);
         if (lane == s) { out_v = bv; out_i = bi; }
         if (bi != kNoId && l.id[0] == bi && l.v[0] == bv) l.pop();
     }
@@ -114,34 +135,40 @@ __global__ __launch_bounds__(256) void topk_scan_kernel(const float* __restrict_
 }
 
 // The threshold of every sample and its empty candidate list: 1,024 groups of a sample of S scores (scores[b * row + i * step],
-// step > 1: straight from a score matrix), the k-th best of the groups' maxima.
-__global__ __launch_bounds__(1024) void topk_threshold_kernel(const float* __restrict__ scores, size_t row, int step, int S, int k,
-                                                              float* __restrict__ tau, int* __restrict__ count) {
+// step > 1: straight from a score matrix), the k-th best of the groups' best.  Fewer groups than k with a score: all scores reach it.
+__global__ __launch_bounds__(1024) void topk_threshold_kernel(const float* __restrict__ scores, size_t row, int step, int S, TopkSampleLabels labels,
+                                                              int k, int B, float* __restrict__ tau, int* __restrict__ tie, int* __restrict__ count) {
     const int b = blockIdx.x;
     TopList l;
     l.clear();
     float best = -__builtin_inff();
-    for (int i0 = threadIdx.x; i0 < S; i0 += 1024 * 4) {
-        float v[4];
+    int best_i = kNoId;
+    for (int i0 = threadIdx.x; i0 < S; i0 += 1024 * 8) {
+        float v[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = scores[(size_t)b * row + (size_t)min(i0 + 1024 * u, S - 1) * step];
+        for (int u = 0; u < 8; ++u) v[u] = scores[(size_t)b * row + (size_t)min(i0 + 1024 * u, S - 1) * step];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (i0 + 1024 * u < S) best = fmaxf(best, v[u]);      // (each score in one group only)
+        for (int u = 0; u < 8; ++u)
+            if (i0 + 1024 * u < S && (v[u] > best || (v[u] == best && best_i == kNoId))) { best = v[u]; best_i = i0 + 1024 * u; }      // (ids ascend; each score in one group only)
     }
     l.v[0] = best;
-    l.id[0] = (int)threadIdx.x < S ? (int)threadIdx.x : kNoId;
+    l.id[0] = best_i;
     float ov;
     int oi;
     block_topk<16>(l, k, ov, oi);
-    if ((int)threadIdx.x == k - 1) tau[b] = ov;
-    if (threadIdx.x == 0) count[(size_t)b * kTopkCountStep] = 0;
+    if ((int)threadIdx.x == k - 1) {
+        tau[b] = ov;
+        tie[b] = oi != kNoId ? (int)(((long long)oi * labels.num) >> labels.shift) : kNoId;
+    }
+    if (threadIdx.x < 2) count[(size_t)b * kTopkCountStep + threadIdx.x] = 0;
+    const int behind = B + (int)threadIdx.x;                                 // (a sample behind the batch's end, up to the next 64)
+    if (b == 0 && behind < (B + 63) / 64 * 64) { tau[behind] = __builtin_inff(); tie[behind] = kTopkListFull; }
 }
 
 // Every score at or above its row's threshold goes to the row's candidate list.  Such scores are a tiny share of the
 // row, so the scan is a plain stream: eight loads in flight per thread, one wave-wide test, the appends on the side.
 __global__ __launch_bounds__(256) void topk_filter_kernel(const float* __restrict__ scores, int L, int labels_per_split,
-                                                          const float* __restrict__ tau, int* __restrict__ count,
+                                                          const float* __restrict__ tau, int* tie, int* __restrict__ count,
                                                           float* __restrict__ cand_val, int* __restrict__ cand_idx, int cap) {
     constexpr int kPark = 1024;                       // hits a workgroup parks in LDS before it appends them to the row's list
     __shared__ int park_count;
@@ -153,6 +180,7 @@ __global__ __launch_bounds__(256) void topk_filter_kernel(const float* __restric
     const float* row = scores + (size_t)b * L;
     if (threadIdx.x == 0) park_count = 0;
     __syncthreads();
+    int last_tied = tie[b];                           // (on its way together with the scores)
     for (int j0 = begin + (int)threadIdx.x; j0 < end; j0 += 256 * 8) {
         float v8[8];
 #pragma unroll
@@ -164,13 +192,13 @@ __global__ __launch_bounds__(256) void topk_filter_kernel(const float* __restric
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int j = j0 + 256 * u;
-                if (j < end && v8[u] >= t) {
+                if (j < end && topk_reaches(v8[u], j, t, last_tied)) {
                     const int p = atomicAdd(&park_count, 1);          // an LDS counter: no round trip to memory
                     if (p < kPark) {
                         park_val[p] = v8[u];
                         park_idx[p] = j;
                     } else {
-                        const int slot = atomicAdd(&count[(size_t)b * kTopkCountStep], 1);
+                        const int slot = topk_slot(v8[u], j, t, last_tied, &tie[b], &count[(size_t)b * kTopkCountStep], cap);
                         if (slot < cap) {
                             cand_val[(size_t)b * cap + slot] = v8[u];
                             cand_idx[(size_t)b * cap + slot] = j;
@@ -198,19 +226,22 @@ template <typename T> __device__ __forceinline__ float as_float(T v);
 template <> __device__ __forceinline__ float as_float<float>(float v) { return v; }
 template <> __device__ __forceinline__ float as_float<unsigned short>(unsigned short v) { return __uint_as_float((unsigned)v << 16); }
 
-// The k best of a sample's candidates, or, where they did not fit the list, of its whole row: the stored scores, or scores
-// formed anew from the layer (k ascending, bias last); every thread keeps the best eight of its share.
+// The k best of a sample's candidates (workgroup b: sample b).  A sample whose candidates did not fit its list is answered from
+// its whole row -- the stored scores, or scores formed anew from the layer (k ascending, bias last) -- by the first `sharers`
+// workgroups: each keeps the best eight of its share in the place of the sample's candidates, the last to finish takes the best of
+// those.  (One workgroup per row: 28 ms of latency for 670,091 labels of fan-in 32.)
+constexpr int kTopkSharers = kTopkCap / kTopMax;        // lists of eight that fit there
+
 template <typename T>
-__global__ __launch_bounds__(256) void topk_select_kernel(const float* __restrict__ cand_val, const int* __restrict__ cand_idx,
-                                                          const int* __restrict__ count, int cap, int k, const TopkRowSource src, int B,
-                                                          float* __restrict__ values, int* __restrict__ indices) {
-    const int b = blockIdx.x;
+__global__ __launch_bounds__(256) void topk_select_kernel(float* cand_val, int* cand_idx, int* count, int cap, int k, const TopkRowSource src,
+                                                          int B, int sharers, float* __restrict__ values, int* __restrict__ indices) {
     TopList l;
-    l.clear();
-    const int n = count != nullptr ? count[(size_t)b * kTopkCountStep] : cap;
-    if (n <= cap) {
+    float ov;
+    int oi;
+    auto answer = [&](int b, int n) {                                 // from n listed entries
         const float* pv = cand_val + (size_t)b * cap;
         const int* pi = cand_idx + (size_t)b * cap;
+        l.clear();
         for (int c0 = threadIdx.x; c0 < n; c0 += 256 * 4) {           // four candidates per thread in flight
             float v4[4];
             int i4[4];
@@ -224,29 +255,61 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const float* __restric
             for (int u = 0; u < 4; ++u)
                 if (i4[u] >= 0) l.offer(v4[u], i4[u]);
         }
-    } else {
-        const T* x = static_cast<const T*>(src.x);
-        const T* w = static_cast<const T*>(src.w);
-        for (int j = threadIdx.x; j < src.L; j += 256) {
-            float v = 0.f;
-            if (src.scores != nullptr) {
-                v = src.scores[(size_t)b * src.L + j];
-            } else {
-                for (int c = 0; c < src.K; ++c) {
-                    const unsigned id = min((unsigned)src.idx[(size_t)j * src.K + c], (unsigned)src.N - 1u);
-                    v = fmaf(as_float(w[(size_t)j * src.K + c]), as_float(src.tp ? x[(size_t)id * B + b] : x[(size_t)b * src.N + id]), v);
-                }
-                if (src.bias != nullptr) v += src.bias[j];
-            }
-            l.offer(v, j);
+        block_topk<4>(l, k, ov, oi);
+        if ((int)threadIdx.x < k) {
+            values[(size_t)b * k + threadIdx.x] = ov;
+            indices[(size_t)b * k + threadIdx.x] = oi != kNoId ? oi : -1;
         }
+    };
+    if ((int)blockIdx.x < B) {
+        const int n = count != nullptr ? count[(size_t)blockIdx.x * kTopkCountStep] : cap;
+        if (n <= cap) answer((int)blockIdx.x, n);
     }
-    float ov;
-    int oi;
-    block_topk<4>(l, k, ov, oi);
-    if ((int)threadIdx.x < k) {
-        values[(size_t)b * k + threadIdx.x] = ov;
-        indices[(size_t)b * k + threadIdx.x] = oi != kNoId ? oi : -1;
+    if (count == nullptr || (int)blockIdx.x >= sharers) return;
+    // the samples whose lists overflowed (of 256 at a time)
+    __shared__ int over[256];
+    __shared__ int n_over, arrived;
+    const T* x = static_cast<const T*>(src.x);
+    const T* w = static_cast<const T*>(src.w);
+    for (int b0 = 0; b0 < B; b0 += 256) {
+        __syncthreads();
+        if (threadIdx.x == 0) n_over = 0;
+        __syncthreads();
+        const int mine = b0 + (int)threadIdx.x;
+        if (mine < B && count[(size_t)mine * kTopkCountStep] > cap) over[atomicAdd(&n_over, 1)] = mine;
+        __syncthreads();
+        const int todo = n_over;
+        for (int t = 0; t < todo; ++t) {
+            const int b = over[t];
+            l.clear();
+            for (int j = (int)(blockIdx.x * 256 + threadIdx.x); j < src.L; j += sharers * 256) {
+                float v = 0.f;
+                if (src.scores != nullptr) {
+                    v = src.scores[(size_t)b * src.L + j];
+                } else {
+                    for (int c = 0; c < src.K; ++c) {
+                        const unsigned id = min((unsigned)src.idx[(size_t)j * src.K + c], (unsigned)src.N - 1u);
+                        v = fmaf(as_float(w[(size_t)j * src.K + c]), as_float(src.tp ? x[(size_t)id * B + b] : x[(size_t)b * src.N + id]), v);
+                    }
+                    if (src.bias != nullptr) v += src.bias[j];
+                }
+                l.offer(v, j);
+            }
+            __syncthreads();                                          // (block_topk's own memory)
+            block_topk<4>(l, kTopMax, ov, oi);
+            if ((int)threadIdx.x < kTopMax) {
+                cand_val[(size_t)b * cap + blockIdx.x * kTopMax + threadIdx.x] = ov;
+                cand_idx[(size_t)b * cap + blockIdx.x * kTopMax + threadIdx.x] = oi != kNoId ? oi : -1;
+            }
+            __threadfence();
+            __syncthreads();
+            if (threadIdx.x == 0) arrived = atomicAdd(&count[(size_t)b * kTopkCountStep + 1], 1);
+            __syncthreads();
+            if (arrived == sharers - 1) {
+                __threadfence();
+                answer(b, sharers * kTopMax);
+            }
+        }
     }
 }
 
@@ -318,30 +381,37 @@ int topk_hits(const int32_t* top, int B, int top_stride, int k, const int64_t* l
 }
 
 // Thresholds, counters and candidates begin on cache lines of their own: counters that shared one with the thresholds, which
-// every workgroup reads, tripled the time of a sweep (43 -> 146 us at 12 x 3,000 x 300,000 x 32).
+// every workgroup reads, tripled the time of a sweep (43 -> 146 us at 12 x 3,000 x 300,000 x 32).  The forward kernels read the
+// thresholds a slice of up to 64 samples at a time: those of the samples behind the batch's end say that their lists are full.
 static size_t line_floats(size_t n) { return (n + 31) / 32 * 32; }
+static size_t padded_samples(int B) { return ((size_t)B + 63) / 64 * 64; }
 size_t topk_candidate_bytes(int B, int sample) {
-    return (line_floats((size_t)B * sample) + line_floats(B) + (size_t)B * kTopkCountStep + 2 * (size_t)B * kTopkCap) * 4;
+    return (line_floats((size_t)B * sample) + 2 * padded_samples(B) + (size_t)B * kTopkCountStep + 2 * (size_t)B * kTopkCap) * 4;
 }
 TopkCandidates topk_candidates_at(void* ws, int B, int sample) {
     TopkCandidates c;
     c.sample = static_cast<float*>(ws);
     c.tau = c.sample + line_floats((size_t)B * sample);
-    c.count = reinterpret_cast<int*>(c.tau + line_floats(B));
+    c.tie = reinterpret_cast<int*>(c.tau + padded_samples(B));
+    c.count = c.tie + padded_samples(B);
     c.val = reinterpret_cast<float*>(c.count + (size_t)B * kTopkCountStep);
     c.idx = reinterpret_cast<int*>(c.val + (size_t)B * kTopkCap);
     return c;
 }
 
-int launch_topk_threshold(const float* scores, size_t row, int step, int S, int k, const TopkCandidates& c, int B, hipStream_t s) {
-    hipLaunchKernelGGL(topk_threshold_kernel, dim3(B), dim3(1024), 0, s, scores, row, step, S, k, c.tau, c.count);
+int launch_topk_threshold(const float* scores, size_t row, int step, int S, TopkSampleLabels labels, int k, const TopkCandidates& c, int B,
+                          hipStream_t s) {
+    hipLaunchKernelGGL(topk_threshold_kernel, dim3(B), dim3(1024), 0, s, scores, row, step, S, labels, k, B, c.tau, c.tie, c.count);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 
 int launch_topk_select(const TopkCandidates& c, int B, const TopkArgs& tk, const TopkRowSource& src, hipStream_t s) {
-    if (src.bf16) hipLaunchKernelGGL(topk_select_kernel<unsigned short>, dim3(B), dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, tk.values, tk.indices);
-    else hipLaunchKernelGGL(topk_select_kernel<float>, dim3(B), dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, tk.values, tk.indices);
+    // (workgroups that find no overflowed list leave at once)
+    const int sharers = std::max(1, std::min({kTopkSharers, (src.L + 255) / 256, 4 * device_cu_count()}));
+    const dim3 grid((unsigned)std::max(B, sharers));
+    if (src.bf16) hipLaunchKernelGGL(topk_select_kernel<unsigned short>, grid, dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, sharers, tk.values, tk.indices);
+    else hipLaunchKernelGGL(topk_select_kernel<float>, grid, dim3(256), 0, s, c.val, c.idx, c.count, kTopkCap, tk.k, src, B, sharers, tk.values, tk.indices);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
@@ -363,15 +433,16 @@ int launch_topk_f32(const float* scores, int B, int L, int k, float* values, int
         float* pv = (float*)part;
         int* pi = (int*)(part + list_bytes);
         hipLaunchKernelGGL(topk_scan_kernel, dim3(splits, B), dim3(256), 0, s, scores, L, per, pv, pi, splits * 4);
-        hipLaunchKernelGGL(topk_select_kernel<float>, dim3(B), dim3(256), 0, s, pv, pi, (const int*)nullptr, entries, k, TopkRowSource{}, B, values, indices);
+        hipLaunchKernelGGL(topk_select_kernel<float>, dim3(B), dim3(256), 0, s, pv, pi, (int*)nullptr, entries, k, TopkRowSource{}, B, 0, values, indices);
         FFI_HIP_TRY(hipGetLastError());
         return FFI_OK;
     }
     void* ws = nullptr;
     FFI_TRY(workspace_get(s, kWsTopk, topk_candidate_bytes(B, 0), &ws));
     const TopkCandidates c = topk_candidates_at(ws, B, 0);
-    FFI_TRY(launch_topk_threshold(scores, (size_t)L, L / kTopkRowSample, kTopkRowSample, k, c, B, s));
-    hipLaunchKernelGGL(topk_filter_kernel, dim3(splits, B), dim3(256), 0, s, scores, L, per, c.tau, c.count, c.val, c.idx, kTopkCap);
+    const int step = L / kTopkRowSample;
+    FFI_TRY(launch_topk_threshold(scores, (size_t)L, step, kTopkRowSample, TopkSampleLabels{step, 0}, k, c, B, s));
+    hipLaunchKernelGGL(topk_filter_kernel, dim3(splits, B), dim3(256), 0, s, scores, L, per, c.tau, c.tie, c.count, c.val, c.idx, kTopkCap);
     FFI_HIP_TRY(hipGetLastError());
     TopkRowSource src;
     src.scores = scores; src.L = L;

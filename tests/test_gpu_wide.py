@@ -164,3 +164,37 @@ def test_topk_of_scores_that_are_not_finite(ffi, bf16, shape, n_inf):
     best = -np.sort(-rest, axis=1)[:, :k - n]
     assert np.abs(val[:, n:] - best).max(initial=0.0) <= 1e-5 * np.abs(rest[np.isfinite(rest)]).max()
     assert np.abs(np.take_along_axis(scores, idx[:, n:].astype(np.int64), 1) - val[:, n:]).max(initial=0.0) <= 1e-5 * np.abs(rest[np.isfinite(rest)]).max()
+
+
+# Scores that tie by the thousand -- small whole numbers, samples without features -- and layers whose every label outside the sample
+# that sets the threshold beats those in it, so that the lists overflow: the answer is that of the score matrix, ties to the
+# lower label.  (B, N, wide_phases): slices in LDS, gathered from L2, in phases; the 32-sample tile
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,phases", [(1, 500, 0), (7, 300, 0), (40, 200, 0), (70, 3000, 0), (70, 3000, 1)])
+@pytest.mark.parametrize("overflow", [False, True])
+def test_topk_of_tied_scores_and_full_lists(ffi, bf16, B, N, phases, overflow):
+    L, K, k = 81_920, 6, 8                                      # (samples of every 5th and 20th label)
+    rng = np.random.default_rng(B + N)
+    x = rng.integers(0, 4, (B, N)).astype(np.float32)
+    w = rng.integers(-2, 3, (L, K)).astype(np.float32)
+    lookup = rng.integers(0, N, (L, K)).astype(np.int32)
+    if overflow:
+        x[:, 0], lookup[:, 0], w[:, 0] = 1.0, 0, np.where(np.arange(L) % 5 == 0, 0.0, 100.0)
+    x[::3, overflow:] = 0.0
+    dx, dl, dw = dev(x), dev(lookup), dev(w)
+    print(f"case bf16={bf16} B={B} N={N} phases={phases} overflow={overflow}", flush=True)
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_phases", phases) == 0
+    try:
+        for _ in range(2):                                      # (the counters of the first call are cleared for the second)
+            if bf16:
+                val, idx = ffi.fan_in_sparse_topk_bf16(dx.bfloat16(), dl, dw.bfloat16(), k=k)
+            else:
+                val, idx = ffi.fan_in_sparse_topk(dx, dl, dw, k=k)
+    finally:
+        lib.ffi_set_option(b"wide_phases", 0)
+    scores = oracle.forward(x, lookup, w, transposed=False)     # (whole numbers: exact in any order)
+    ref_v, ref_i = oracle.topk(scores, k)
+    assert np.array_equal(idx.cpu().numpy(), ref_i) and np.array_equal(val.cpu().numpy(), ref_v)
+    val, idx = ffi.topk_scores(dev(scores), k)
+    assert np.array_equal(idx.cpu().numpy(), ref_i) and np.array_equal(val.cpu().numpy(), ref_v)
