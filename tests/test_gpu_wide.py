@@ -40,6 +40,12 @@ def test_forward_of_wide_inputs(ffi, phases):
                 assert rel_err(fwd(dx, dev(lookup), dev(w)).cpu().numpy(), ref) <= 1e-5, (B, N, L, K, tp)
             out = ffi.fan_in_sparse_matmul_bias(dev(x), dev(lookup), dev(w), dev(bias)).cpu().numpy()
             assert rel_err(out, ref + bias) <= 1e-5, (B, N, L, K)
+            # bf16 operands, whose sums are fp32 ones too
+            hx, hw = torch.from_numpy(x).bfloat16(), torch.from_numpy(w).bfloat16()
+            ref = oracle.forward(hx.float().numpy(), lookup, hw.float().numpy(), transposed=False)
+            for tp in (False, True):
+                out = ffi.fan_in_sparse_matmul_bf16((hx.t().contiguous() if tp else hx).cuda(), dev(lookup), hw.cuda(), transposed=tp)
+                assert rel_err(out.cpu().numpy(), ref) <= 1e-5, (B, N, L, K, tp, "bf16")
     finally:
         lib.ffi_set_option(b"wide_phases", 0)
 
@@ -198,3 +204,80 @@ def test_topk_of_tied_scores_and_full_lists(ffi, bf16, B, N, phases, overflow):
     assert np.array_equal(idx.cpu().numpy(), ref_i) and np.array_equal(val.cpu().numpy(), ref_v)
     val, idx = ffi.topk_scores(dev(scores), k)
     assert np.array_equal(idx.cpu().numpy(), ref_i) and np.array_equal(val.cpu().numpy(), ref_v)
+
+
+def _same_values(got, ref, tol, scale):
+    """NaN and infinities where the reference has them, the rest within tol x scale."""
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    special = np.isinf(ref)
+    assert np.array_equal(np.isinf(got), special) and np.array_equal(got[special], ref[special])
+    finite = np.isfinite(ref)
+    assert np.abs(got[finite].astype(np.float64) - ref[finite]).max(initial=0.0) <= tol * scale
+
+
+# (B, N, wide_phases), the small layers' path off: slices in LDS, the 32-sample tile, gathered from L2, in phases
+VALUE_SHAPES = [(3, 300, 0), (40, 700, 0), (5, 1300, 0), (70, 2000, 0), (160, 4096, -1), (40, 1300, 1), (70, 5000, 1)]
+
+
+# Infinities and NaN go where the sums of the layer's definition take them and nowhere else: padded samples, slots and connections
+# add none.  Both gradients too, through the walk over the columns.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,phases", VALUE_SHAPES)
+def test_infinities_and_nan_stay_where_they_belong(ffi, bf16, B, N, phases):
+    L, K = 1_003, 13
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B + N)
+    x[0, ::7], x[1, 3], x[B - 1, 5], x[B - 1, 11] = 0.0, np.inf, -np.inf, np.nan
+    w[7, 0], w[8, 2], w[L - 1, K - 1], w[L - 1, 0] = np.inf, np.nan, -np.inf, 0.0
+    g[0, 9], g[1, 10], g[B - 1, L - 1] = np.inf, np.nan, -np.inf
+    tx, tw = torch.from_numpy(x), torch.from_numpy(w)
+    if bf16:
+        tx, tw = tx.bfloat16(), tw.bfloat16()
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_phases", phases) == 0 and lib.ffi_set_option(b"small_path", -1) == 0
+    print(f"case bf16={bf16} B={B} N={N} phases={phases}", flush=True)
+    try:
+        with np.errstate(invalid="ignore"):
+            ref = oracle.forward(tx.float().numpy(), lookup, tw.float().numpy(), transposed=False)
+        out = (ffi.fan_in_sparse_matmul_bf16 if bf16 else ffi.fan_in_sparse_matmul)(tx.cuda(), dev(lookup), tw.cuda())
+        _same_values(out.cpu().numpy(), ref, 1e-5, np.abs(ref[np.isfinite(ref)]).max())
+        if not bf16:
+            ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+            for _ in range(2):
+                gx, gw = ffi.fan_in_sparse_matmul_grad(dev(x), dev(lookup), dev(w), dev(g))
+                _same_values(gx.cpu().numpy(), ref_gx, 1e-4, np.abs(ref_gx[np.isfinite(ref_gx)]).max())
+                _same_values(gw.cpu().numpy(), ref_gw, 1e-4, np.abs(ref_gw[np.isfinite(ref_gw)]).max())
+    finally:
+        lib.ffi_set_option(b"wide_phases", 0)
+        lib.ffi_set_option(b"small_path", 0)
+
+
+# Operands below the smallest normal number count for what they are, and so do sums that are subnormal themselves
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,phases", VALUE_SHAPES)
+def test_subnormal_operands_and_sums(ffi, bf16, B, N, phases):
+    L, K = 1_003, 12
+    rng = np.random.default_rng(B + N)
+    lookup = rng.integers(0, N, (L, K)).astype(np.int32)
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_phases", phases) == 0 and lib.ffi_set_option(b"small_path", -1) == 0
+    print(f"case bf16={bf16} B={B} N={N} phases={phases}", flush=True)
+    try:
+        for ex, ew, eg in ((-131, 110, 0), (110, -131, 0), (-70, -65, -65), (-131, 0, 0)):         # (bf16 holds multiples of 2^-133)
+            x = (rng.integers(-3, 4, (B, N)) * 2.0 ** ex).astype(np.float32)
+            w = (rng.integers(-3, 4, (L, K)) * 2.0 ** ew).astype(np.float32)
+            g = (rng.integers(-3, 4, (B, L)) * 2.0 ** eg).astype(np.float32)
+            tx, tw = torch.from_numpy(x), torch.from_numpy(w)
+            if bf16:
+                tx, tw = tx.bfloat16(), tw.bfloat16()
+                assert np.array_equal(tx.float().numpy(), x) and np.array_equal(tw.float().numpy(), w)
+            # (small whole numbers times a power of two: every sum is exact)
+            ref = oracle.forward(x, lookup, w, transposed=False)
+            out = (ffi.fan_in_sparse_matmul_bf16 if bf16 else ffi.fan_in_sparse_matmul)(tx.cuda(), dev(lookup), tw.cuda())
+            assert np.abs(ref).max() > 0 and np.array_equal(out.cpu().numpy(), ref), (ex, ew)
+            if not bf16:
+                ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+                gx, gw = ffi.fan_in_sparse_matmul_grad(dev(x), dev(lookup), dev(w), dev(g))
+                assert np.array_equal(gw.cpu().numpy(), ref_gw) and np.array_equal(gx.cpu().numpy(), ref_gx), (ex, ew)
+    finally:
+        lib.ffi_set_option(b"wide_phases", 0)
+        lib.ffi_set_option(b"small_path", 0)
