@@ -70,20 +70,21 @@ ffi_plan* find_cached_plan(const int32_t* lookup, const Dims& d, int dev) {
 
 // Builds a plan for a lookup that has none and adds it to the cache.  Caller holds g_cache_mutex.
 int create_cached_plan(const int32_t* lookup, const Dims& d, int dev, hipStream_t s, ffi_plan** out) {
+    ffi_plan* p = nullptr;
     if (g_cache.size() >= kMaxCachedPlans) {
-        // evict the least recently used plan of this device; its stream work must have drained
+        // the least recently used plan of this device makes room, and hands on its buffers (a program that goes from lookup to
+        // lookup would free and allocate a few of 100 MB for each); its stream work must have drained
         for (size_t i = 0; i < g_cache.size(); ++i) {
             if (g_cache[i]->device == dev) {
                 (void)hipDeviceSynchronize();
-                plan_free(g_cache[i]);
-                delete g_cache[i];
+                p = g_cache[i];
                 g_cache.erase(g_cache.begin() + i);
+                plan_reuse(p, d.L, d.K, d.N);
                 break;
             }
         }
     }
-    ffi_plan* p = nullptr;
-    FFI_TRY(plan_alloc(d.L, d.K, d.N, &p));
+    if (p == nullptr) FFI_TRY(plan_alloc(d.L, d.K, d.N, &p));
     p->batch_hint = d.B;
     int st = plan_build(p, lookup, s);
     if (st != FFI_OK) { plan_free(p); delete p; return st; }

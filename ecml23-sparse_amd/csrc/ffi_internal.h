@@ -380,6 +380,7 @@ inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 6
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
 int plan_block_labels(int N, int K, int L);
+size_t plan_expected_slots(int N, int K, int L);
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s);
 // Content fingerprint of `lookup` (and the count of ids outside [0,N)).  _begin enqueues the kernel
 // on `s` and returns; _end waits for that kernel only, not for what the caller enqueued on `s`
@@ -389,6 +390,8 @@ int plan_fingerprint_end(ffi_plan* p, unsigned long long* out, unsigned long lon
 int plan_fingerprint(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigned long long* out,
                      unsigned long long* bad_ids);
 int plan_scratch_alloc(ffi_plan* p);
+// Makes a plan that nothing uses any more one of another lookup, to be built: its buffers serve the build where they fit.
+void plan_reuse(ffi_plan* p, int L, int K, int N);
 // Enqueues a check of `lookup` against the plan's fingerprint on `s`: the verdict lands in p->d_guard[kGuardVerdict]
 // (device) for the kernels enqueued behind it, and in the pinned mirror for a later call of the host.
 constexpr int kGuardVerdict = 4;

@@ -8,12 +8,12 @@
 #include "ffi_lds_tile.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <functional>
 
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_scan.hpp>
-#include <rocprim/iterator/counting_iterator.hpp>
+#include <rocprim/types/double_buffer.hpp>
 
 namespace ffi {
 namespace {
@@ -743,17 +743,40 @@ inline size_t tile_fill_bitmap_lds(int threads, int tile_labels, int K, int* wor
 
 // ---- blocked global form ------------------------------------------------------------------------
 
-// col_ptr[n] = first position in the sorted key array whose key is >= n (n in [0,N]; N = number of keys).
-__global__ __launch_bounds__(kBlock) void col_ptr_kernel(const unsigned* __restrict__ sorted_keys,
-                                                          int total, int N, int32_t* __restrict__ col_ptr) {
-    const int n = blockIdx.x * kBlock + threadIdx.x;
-    if (n > N) return;
+// ptr[n] = first position in the sorted key array whose key is >= n (n in [0,nkeys]), and the octs that the kListsPerBlock lists
+// of a workgroup take together
+constexpr int kListsPerBlock = kBlock - 1;
+__global__ __launch_bounds__(kBlock) void list_ptr_kernel(const unsigned* __restrict__ sorted_keys, int total, int nkeys,
+                                                          int32_t* __restrict__ ptr, unsigned* __restrict__ block_octs) {
+    __shared__ int begin[kBlock];
+    const int n = min((int)(blockIdx.x * kListsPerBlock + threadIdx.x), nkeys);
     int lo = 0, hi = total;
     while (lo < hi) {
         const int mid = lo + ((hi - lo) >> 1);
         if (sorted_keys[mid] < (unsigned)n) lo = mid + 1; else hi = mid;
     }
-    col_ptr[n] = lo;
+    ptr[n] = lo;
+    begin[threadIdx.x] = lo;
+    __syncthreads();
+    // (behind the last list begin and end are the same)
+    const unsigned octs = threadIdx.x < kListsPerBlock ? (unsigned)(begin[threadIdx.x + 1] - lo + 7) / 8u : 0u;
+    unsigned long long sum = 0;
+    (void)block_sum_below<kBlock>(octs, &sum);
+    if (threadIdx.x == 0) block_octs[blockIdx.x] = (unsigned)sum;
+}
+
+// oct_ptr[n] = octs of the lists before list n, from the octs before the list's workgroup of list_ptr_kernel
+__global__ __launch_bounds__(kBlock) void oct_ptr_kernel(const int32_t* __restrict__ ptr, int nkeys, const unsigned* __restrict__ octs_before,
+                                                         unsigned* __restrict__ oct_ptr) {
+    const int n = blockIdx.x * kListsPerBlock + threadIdx.x;
+    const bool mine = threadIdx.x < kListsPerBlock && n < nkeys;
+    const unsigned octs = mine ? (unsigned)(ptr[n + 1] - ptr[n] + 7) / 8u : 0u;
+    unsigned long long sum = 0;
+    const unsigned at = octs_before[blockIdx.x] + (unsigned)block_sum_below<kBlock>(octs, &sum);
+    if (mine) {
+        oct_ptr[n] = at;
+        if (n == nkeys - 1) oct_ptr[nkeys] = at + octs;
+    }
 }
 
 int bits_for(unsigned max_value) {
@@ -807,6 +830,13 @@ bool dev_alloc(ffi_plan* p, T** ptr, size_t count) {
     void* raw = nullptr;
     if (hipMalloc(&raw, bytes) != hipSuccess) {
         (void)hipGetLastError();
+        raw = nullptr;
+        if (!p->spare.empty()) {                           // (what the last build left may be what is missing)
+            free_spares(p);
+            if (hipMalloc(&raw, bytes) != hipSuccess) { (void)hipGetLastError(); raw = nullptr; }
+        }
+    }
+    if (raw == nullptr) {
         *ptr = nullptr;
         return false;
     }
@@ -1006,93 +1036,112 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
 
 // key[p] = (label block of p) * N + column id of p
 __global__ __launch_bounds__(kBlock) void block_key_kernel(const int32_t* __restrict__ idx, int total, int K, int N,
-                                                           int block_labels, unsigned* __restrict__ key) {
+                                                           int block_labels, unsigned* __restrict__ key, int32_t* __restrict__ pos) {
     const int p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= total) return;
     const int j = p / K;
     key[p] = (unsigned)(j / block_labels) * (unsigned)N + (unsigned)idx[p];
+    pos[p] = p;
 }
 
-// octs[n] = octs of slots that list n takes; the last entry (a list of its own behind the lists) is 0
-__global__ __launch_bounds__(kBlock) void oct_count_kernel(const int32_t* __restrict__ ptr, int nkeys, unsigned* __restrict__ octs) {
-    const int n = blockIdx.x * kBlock + threadIdx.x;
-    if (n > nkeys) return;
-    octs[n] = n < nkeys ? (unsigned)(ptr[n + 1] - ptr[n] + 7) / 8u : 0u;
-}
-
-__global__ __launch_bounds__(kBlock) void slot_clear_kernel(int32_t* __restrict__ slot_pos, unsigned short* __restrict__ slot_lab, size_t slots) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= slots) return;
-    slot_pos[i] = -1;
-    slot_lab[i] = kNoLabel;
-}
-
+// The slots of every list; the list's last connection writes the padding behind it too.
 __global__ __launch_bounds__(kBlock) void slot_fill_kernel(const unsigned* __restrict__ sorted_keys, const int32_t* __restrict__ sorted_pos,
                                                            const int32_t* __restrict__ ptr, const unsigned* __restrict__ oct_ptr, int total,
                                                            int K, int N, int block_labels, int32_t* __restrict__ slot_pos,
                                                            unsigned short* __restrict__ slot_lab, unsigned* __restrict__ pos_slot) {
     const int e = blockIdx.x * kBlock + threadIdx.x;
     if (e >= total) return;
-    const unsigned key = sorted_keys[e];
-    const size_t slot = (size_t)oct_ptr[key] * 8 + (size_t)(e - ptr[key]);
+    const unsigned key = sorted_keys[e], next = sorted_keys[min(e + 1, total - 1)];
+    size_t slot = (size_t)oct_ptr[key] * 8 + (size_t)(e - ptr[key]);
     const int pos = sorted_pos[e];
     slot_pos[slot] = pos;
     pos_slot[pos] = (unsigned)slot;
     slot_lab[slot] = (unsigned short)(pos / K - (int)(key / (unsigned)N) * block_labels);
+    if (e + 1 == total || next != key)
+        while ((++slot & 7) != 0) { slot_pos[slot] = -1; slot_lab[slot] = kNoLabel; }
 }
 
+}  // namespace
+
+// Slots of the global form for column ids drawn uniformly: a list's length is a Poisson count, rounded up to whole octs.
+size_t plan_expected_slots(int N, int K, int L) {
+    const int labels = plan_block_labels(N, K, L);
+    const double lists = (double)((L + labels - 1) / labels) * N, mu = (double)L * K / lists;
+    double slots = mu + 3.5;
+    if (mu < 64.0) {
+        double p = std::exp(-mu);
+        slots = 0.0;
+        for (int n = 1; n < 256; ++n) { p *= mu / n; slots += p * (double)((n + 7) / 8 * 8); }
+    }
+    return (size_t)(slots * lists) + 8;
+}
+
+namespace {
+
+// The build's temporaries lie in arrays that it fills last and in the workspaces that the backward pass will ask for: nothing
+// is allocated and freed again.  The plan's own arrays are allocated for the slots that uniform ids would give while the sort
+// runs.  (Six buffers of the build's own, and the plan's only once the number of slots was known, held the host for 2 ms of the
+// 3.6 to 4.9 of a first pass at 50 x 32,768 x 670,000 x 32, whose kernels take 2.2.)
 int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     const int total = p->L * p->K;  // validated to fit int32 by the caller
     const int block_labels = plan_block_labels(p->N, p->K, p->L);
     const int nblocks = (p->L + block_labels - 1) / block_labels;
     const long long nkeys = (long long)nblocks * p->N;
-    if (nkeys >= (1ll << 31) - 1) return FFI_ERR_TOO_LARGE;
-    if (!dev_alloc(p, &p->oct_ptr, (size_t)nkeys + 1)) return FFI_ERR_OUT_OF_MEMORY;
-    unsigned *keys = nullptr, *sorted_keys = nullptr, *octs = nullptr;
-    int32_t *sorted_pos = nullptr, *ptr = nullptr;
-    void* temp = nullptr;
-    size_t temp_bytes = 0, scan_bytes = 0;
+    if (nkeys >= (1ll << 31) - kBlock) return FFI_ERR_TOO_LARGE;
     const int end_bit = bits_for((unsigned)(nkeys - 1));
-    rocprim::counting_iterator<int32_t> positions(0);
-    auto cleanup = [&]() {
-        for (void* q : {(void*)keys, (void*)sorted_keys, (void*)octs, (void*)sorted_pos, (void*)ptr, temp})
-            if (q) (void)hipFree(q);
+    const unsigned list_blocks = (unsigned)((nkeys + kListsPerBlock - 1) / kListsPerBlock);
+    size_t expected = plan_expected_slots(p->N, p->K, p->L), sort_bytes = 0;
+    expected = (std::max<size_t>((size_t)total, std::min<size_t>(expected + expected / 128, (1ull << 32) - 64)) + 7) / 8 * 8;
+    // (two buffers, not four: an allocation is 50 us and more)
+    auto alloc_slots = [&](size_t slots) {
+        if (!dev_alloc(p, &p->slot_pos, slots + (slots + 1) / 2)) return false;
+        p->slot_lab = reinterpret_cast<unsigned short*>(p->slot_pos + slots);
+        return true;
     };
+    if (!alloc_slots(expected) || !dev_alloc(p, &p->oct_ptr, (size_t)nkeys + 1 + (size_t)total)) return FFI_ERR_OUT_OF_MEMORY;
+    p->pos_slot = p->oct_ptr + nkeys + 1;
     // stable LSD radix sort of ((block, column), flat position): positions stay ascending inside a column
-    hipError_t e = rocprim::radix_sort_pairs(nullptr, temp_bytes, keys, sorted_keys, positions, sorted_pos, (unsigned)total, 0, end_bit, s);
-    if (e == hipSuccess) e = rocprim::exclusive_scan(nullptr, scan_bytes, octs, p->oct_ptr, 0u, (size_t)nkeys + 1, rocprim::plus<unsigned>(), s);
+    rocprim::double_buffer<unsigned> keys(reinterpret_cast<unsigned*>(p->slot_pos), nullptr);
+    rocprim::double_buffer<int32_t> positions(reinterpret_cast<int32_t*>(p->pos_slot), nullptr);
+    hipError_t e = rocprim::radix_sort_pairs(nullptr, sort_bytes, keys, positions, (unsigned)total, 0, end_bit, s);
     if (e != hipSuccess) return hip_fail(e);
-    temp_bytes = std::max<size_t>(std::max(temp_bytes, scan_bytes), 4);
-    if (hipMalloc(&keys, (size_t)total * sizeof(unsigned)) != hipSuccess ||
-        hipMalloc(&sorted_keys, (size_t)total * sizeof(unsigned)) != hipSuccess ||
-        hipMalloc(&sorted_pos, (size_t)total * sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&ptr, ((size_t)nkeys + 1) * sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&octs, ((size_t)nkeys + 1) * sizeof(unsigned)) != hipSuccess || hipMalloc(&temp, temp_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        cleanup();
-        return FFI_ERR_OUT_OF_MEMORY;
-    }
+    unsigned *key_ws = nullptr, *small_ws = nullptr;
+    int32_t* pos_ws = nullptr;
+    sort_bytes = (sort_bytes + 255) / 256 * 256;
+    FFI_TRY(workspace_get(s, kWsSlots, expected * sizeof(unsigned), (void**)&key_ws));
+    FFI_TRY(workspace_get(s, kWsWeightParts, expected * sizeof(int32_t), (void**)&pos_ws));
+    FFI_TRY(workspace_get(s, kWsPartials, sort_bytes + ((size_t)nkeys + 1 + 2 * (size_t)list_blocks + 1) * sizeof(unsigned), (void**)&small_ws));
+    int32_t* ptr = reinterpret_cast<int32_t*>(small_ws + sort_bytes / sizeof(unsigned));
+    unsigned *block_octs = reinterpret_cast<unsigned*>(ptr) + nkeys + 1, *octs_before = block_octs + list_blocks;
+    keys = rocprim::double_buffer<unsigned>(reinterpret_cast<unsigned*>(p->slot_pos), key_ws);
+    positions = rocprim::double_buffer<int32_t>(reinterpret_cast<int32_t*>(p->pos_slot), pos_ws);
     auto grid = [](size_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); };
-    hipLaunchKernelGGL(block_key_kernel, grid((size_t)total), dim3(kBlock), 0, s, lookup, total, p->K, p->N, block_labels, keys);
-    e = rocprim::radix_sort_pairs(temp, temp_bytes, keys, sorted_keys, positions, sorted_pos, (unsigned)total, 0, end_bit, s);
-    if (e != hipSuccess) { cleanup(); return hip_fail(e); }
-    hipLaunchKernelGGL(col_ptr_kernel, grid((size_t)nkeys + 1), dim3(kBlock), 0, s, sorted_keys, total, (int)nkeys, ptr);
-    hipLaunchKernelGGL(oct_count_kernel, grid((size_t)nkeys + 1), dim3(kBlock), 0, s, ptr, (int)nkeys, octs);
-    e = rocprim::exclusive_scan(temp, temp_bytes, octs, p->oct_ptr, 0u, (size_t)nkeys + 1, rocprim::plus<unsigned>(), s);
-    unsigned total_octs = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&total_octs, p->oct_ptr + nkeys, sizeof(unsigned), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) { cleanup(); return hip_fail(e); }
-    const size_t slots = (size_t)total_octs * 8;
-    if (slots >= (1ull << 32)) { cleanup(); return FFI_ERR_TOO_LARGE; }
-    if (!dev_alloc(p, &p->slot_pos, slots) || !dev_alloc(p, &p->slot_lab, slots) || !dev_alloc(p, &p->pos_slot, (size_t)total)) { cleanup(); return FFI_ERR_OUT_OF_MEMORY; }
-    hipLaunchKernelGGL(slot_clear_kernel, grid(slots), dim3(kBlock), 0, s, p->slot_pos, p->slot_lab, slots);
-    hipLaunchKernelGGL(slot_fill_kernel, grid((size_t)total), dim3(kBlock), 0, s, sorted_keys, sorted_pos, ptr, p->oct_ptr, total, p->K, p->N,
-                       block_labels, p->slot_pos, p->slot_lab, p->pos_slot);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    cleanup();
+    hipLaunchKernelGGL(block_key_kernel, grid((size_t)total), dim3(kBlock), 0, s, lookup, total, p->K, p->N, block_labels, keys.current(),
+                       positions.current());
+    FFI_HIP_TRY(hipGetLastError());
+    e = rocprim::radix_sort_pairs(small_ws, sort_bytes, keys, positions, (unsigned)total, 0, end_bit, s);
     if (e != hipSuccess) return hip_fail(e);
+    // (after an even number of passes the result lies in the plan's arrays, which are about to be filled)
+    if (keys.current() != key_ws) FFI_HIP_TRY(hipMemcpyAsync(key_ws, keys.current(), (size_t)total * sizeof(unsigned), hipMemcpyDeviceToDevice, s));
+    if (positions.current() != pos_ws) FFI_HIP_TRY(hipMemcpyAsync(pos_ws, positions.current(), (size_t)total * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+    unsigned long long* total_octs = nullptr;
+    FFI_HIP_TRY(hipHostGetDevicePointer((void**)&total_octs, p->h_scratch, 0));
+    hipLaunchKernelGGL(list_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, key_ws, total, (int)nkeys, ptr, block_octs);
+    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, block_octs, octs_before, (int)list_blocks, total_octs);
+    hipLaunchKernelGGL(oct_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, ptr, (int)nkeys, octs_before, p->oct_ptr);
+    FFI_HIP_TRY(hipGetLastError());
+    FFI_HIP_TRY(hipStreamSynchronize(s));
+    const size_t slots = (size_t)p->h_scratch[0] * 8;
+    if (slots >= (1ull << 32)) return FFI_ERR_TOO_LARGE;
+    if (slots > expected || expected > slots + slots / 4 + (1u << 18)) {
+        // ids that are not drawn uniformly
+        dev_release(p, p->slot_pos);
+        if (!alloc_slots(slots)) return FFI_ERR_OUT_OF_MEMORY;
+    }
+    hipLaunchKernelGGL(slot_fill_kernel, grid((size_t)total), dim3(kBlock), 0, s, key_ws, pos_ws, ptr, p->oct_ptr, total, p->K, p->N,
+                       block_labels, p->slot_pos, p->slot_lab, p->pos_slot);
+    FFI_HIP_TRY(hipGetLastError());
+    FFI_HIP_TRY(hipStreamSynchronize(s));
     p->block_labels = block_labels;
     p->nblocks = nblocks;
     p->slots = (long long)slots;
@@ -1243,6 +1292,14 @@ int plan_scratch_alloc(ffi_plan* p) {
     }
     std::memset(p->h_guard, 0, 8 * sizeof(unsigned long long));      // check number 0: nothing has finished yet
     return FFI_OK;
+}
+
+void plan_reuse(ffi_plan* p, int L, int K, int N) {
+    free_arrays(p, true);
+    p->L = L; p->K = K; p->N = N;
+    p->lookup = nullptr;
+    p->fingerprint = ~0ull;
+    std::memset(p->h_guard + 1, 0, 7 * sizeof(unsigned long long));      // (word 0: the number of a check, which only grows)
 }
 
 int plan_fingerprint_begin(ffi_plan* p, const int32_t* lookup, hipStream_t s) {

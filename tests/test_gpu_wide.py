@@ -281,3 +281,58 @@ def test_subnormal_operands_and_sums(ffi, bf16, B, N, phases):
     finally:
         lib.ffi_set_option(b"wide_phases", 0)
         lib.ffi_set_option(b"small_path", 0)
+
+
+# Plans of the global form: numbers of lists at the edges of the workgroups that count them (255 each), lists shorter than an oct,
+# of whole octs and longer, ids so uneven that the slots are far from what uniform ids would give; narrow layers too uneven for the
+# tiled form; sort keys of one, two and three digits
+@pytest.mark.parametrize("kind", ["uniform", "one column", "squared", "last column"])
+@pytest.mark.parametrize("N,L,K", [(1275, 40, 3), (1276, 2_000, 16), (1530, 9_000, 8), (1531, 30_000, 4), (70_000, 300, 2), (255, 5_000, 8), (256, 6_000, 9)])
+def test_plans_of_the_global_form(ffi, kind, N, L, K):
+    B = 7
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=N + L)
+    if kind == "one column":
+        lookup[:] = N // 2
+        lookup[::97] = 0
+    elif kind == "squared":
+        lookup = (lookup.astype(np.int64) ** 2 // N).astype(np.int32)
+    elif kind == "last column":
+        lookup[:, :] = N - 1
+    ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        dx, dl, dw, dg = dev(x), dev(lookup), dev(w), dev(g)
+        for _ in range(2):
+            gx, gw = ffi.fan_in_sparse_matmul_grad(dx, dl, dw, dg)
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4
+    finally:
+        lib.ffi_set_option(b"small_path", 0)
+
+
+def test_more_lookups_than_the_cache_holds(ffi):
+    # the plan that makes room hands its buffers on, to lookups of any shape and form; a lookup with an id out of range in between is
+    # refused and leaves the cache usable
+    shapes = [(9, 2000, 3_000, 12), (9, 300, 4_000, 16), (9, 1100, 3_000, 8), (9, 40_000, 900, 20), (9, 64, 50, 4), (9, 2000, 3_100, 12)]
+    cases = []
+    for n in range(14):
+        B, N, L, K = shapes[n % len(shapes)]
+        x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=n)
+        cases.append((oracle.backward(x, lookup, w, g, transposed=False), [dev(a) for a in (x, lookup, w, g)]))
+    lib = ffi._lib.lib()
+    ffi._lib.check(lib.ffi_cache_clear())
+    held = []
+    for turn in range(3):
+        for (ref_gx, ref_gw), (x, lookup, w, g) in cases:
+            for _ in range(2):
+                gx, gw = ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
+                assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4
+        held.append(lib.ffi_cache_bytes())
+        x, lookup, w, g = cases[turn][1]
+        bad = lookup.clone()
+        bad[1, 1] = x.shape[1]
+        with pytest.raises(ffi._lib.FfiError):
+            ffi.fan_in_sparse_matmul_grad(x, bad, w, g)
+    assert held[1] == held[2]                                    # (nothing piles up)
+    ffi._lib.check(lib.ffi_cache_clear())
+    assert lib.ffi_cache_bytes() == 0
