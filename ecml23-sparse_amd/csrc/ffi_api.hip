@@ -682,13 +682,19 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
     if (check_dims(batch, num_features, num_units, fan_in, transposed, &d) != FFI_OK) return 0;
     const size_t B = (size_t)d.B, N = (size_t)d.N, L = (size_t)d.L, K = (size_t)d.K;
     const bool narrow = tile_path_fits(d.N) && d.L < (1 << 25);
-    const size_t slice = 4 * (size_t)slice_lanes(d.B, 4), slice_pad = (B + slice - 1) / slice * slice;      // samples of the sliced copies
-    // the batch-major copy of the features (one slot, shared by the passes and by the permuted weights below)
-    size_t features_slot = 0;
-    if (narrow) features_slot = d.tp ? 0 : N * B * 4;
-    else features_slot = N * slice_pad * 4;
-    size_t total = 0, partial_slot = 0;
+    const bool forward = (passes & FFI_PASS_FORWARD) && !takes_small_forward(d), small_backward = takes_small_backward(d);
+    // a copy of the features (one slot, shared by the passes and by the permuted weights below): batch-major, or in slices
+    size_t total = 0, partial_slot = 0, features_slot = 0;
+    const bool copies = (forward && !few_samples(d)) || ((passes & FFI_PASS_BACKWARD) && !small_backward);
+    if (narrow) features_slot = copies && !d.tp ? N * B * 4 : 0;
+    else if (forward) {
+        size_t rows = 0;
+        forward_wide_workspaces(d, &features_slot, &rows);
+        total += rows;
+    }
     if (passes & FFI_PASS_BACKWARD) {
+        // small layers walk no plan: one is built for the check of the ids
+        if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;
         if ((one_window || two_windows) && d.K <= 1024 && d.L < (1 << 25)) {
             // tiled plan: the geometry of ffi_plan.hip, the slot rows of a slice estimated for column ids drawn uniformly
@@ -708,6 +714,7 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
                 const size_t slots = tiles * slices * rows * 64;
                 total += slots * 2 * 2 + (tiles * slices + 1) * 4 + L * 2;              // 4 bytes per slot (lab16 + pos16, or slot32), slice_off, rowpos
                 if (sorted) total += tiles * threads * 2;                               // the column of each thread in each tile
+                if (small_backward) continue;
                 if (!w_in_lds) features_slot = std::max(features_slot, slots * 4);     // weights in slot order
                 const size_t nbt = (B + 31) / 32;
                 const size_t per_cu = (size_t)tiled_workgroups_per_cu((int)threads, (int)TL, d.K, w_in_lds, (int)((B + 31) / 32));
@@ -719,14 +726,18 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
             if (tile_path_fits(d.N) && d.N < (1 << kArrIdBits)) total += arranged_words((long long)(L * ((K + 31) / 32))) * 2;   // idx16
         } else {
             const size_t labels = (size_t)plan_block_labels(d.N, d.K, d.L), nblocks = (L + labels - 1) / labels, lists = nblocks * N;
-            const double mu = (double)L * (double)K / (double)lists;                    // connections per list, Poisson-like
-            const size_t slots = (size_t)((double)lists * (mu + 3.5 * (1.0 - std::exp(-mu)) + std::max(0.0, 4.0 - mu) * (1.0 - std::exp(-mu))));
+            const size_t slots = plan_expected_slots(d.N, d.K, d.L);
             int gl, slices, m, streams, per_stream;
             walk_shape(d.N, d.B, d.L, (int)nblocks, &gl, &slices, &m, &streams, &per_stream);
-            total += slots * 6 + (lists + 1) * 4;                                       // slot_pos, slot_lab, oct_ptr
-            total += slots * 4 * (1 + (size_t)slices);                                  // weights and weight gradients in slot order
-            partial_slot = (L + N * (size_t)streams) * slice_pad * 4;                   // out_grad in slices, sums per stream
-            features_slot = std::max(features_slot, N * slice_pad * 4);
+            const size_t padded = (size_t)slices * gl * 4;                              // samples of the sliced copies
+            total += slots * 6 + (lists + 1) * 4 + L * K * 4;                           // slot_pos, slot_lab, oct_ptr, pos_slot
+            total += slots * 4 * 2;                                                     // weights and weight gradients in slot order
+            // out_grad in slices and the sums per stream; the lists' ends while the plan is built
+            partial_slot = std::max(partial_slot, lists * 4);
+            if (!small_backward) {
+                partial_slot = std::max(partial_slot, (L + N * (size_t)streams) * padded * 4);
+                features_slot = std::max(features_slot, N * padded * 4);
+            }
         }
     }
     return total + features_slot + partial_slot;

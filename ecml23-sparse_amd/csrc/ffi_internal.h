@@ -101,6 +101,8 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
 // any shape (the tile kernels cover narrow inputs only)
 int launch_forward_wide(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                         hipStream_t s);
+// device memory that pass keeps on its stream: the features in slices, and the ordered copy of the layer
+void forward_wide_workspaces(const Dims& d, size_t* features, size_t* rows);
 int launch_weight_grad_wide(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
                             hipStream_t s);
 
@@ -138,6 +140,7 @@ struct TopkArgs {
 // memory, becomes 1 where an id is out of range
 bool takes_small_forward(const Dims& d);
 bool takes_small_backward(const Dims& d);
+size_t small_backward_workspace(const Dims& d);
 int launch_forward_small(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s);
 int launch_backward_small(const float* x, const int32_t* idx, const float* w, const float* g, float* gx, float* gw, float* gb, const Dims& d,
                           hipStream_t s, unsigned long long* bad);

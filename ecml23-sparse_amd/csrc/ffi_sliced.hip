@@ -873,14 +873,16 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
     return FFI_OK;
 }
 
+// the ordered copy of the layer: [ids][weights], part by part
+template <bool BF16> size_t phased_rows_bytes(int L, int K) { return (size_t)L * ((K + 7) / 8) * 8 * (4 + sizeof(typename LaneAcc<BF16>::Element)); }
+
 template <bool BF16>
 int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
     using S = PhasedShape<BF16>;
-    const int octs = (d.K + 7) / 8, rows_per_block = 4 * (64 / (2 * octs)), value = BF16 ? 2 : 4;
+    const int octs = (d.K + 7) / 8, rows_per_block = 4 * (64 / (2 * octs));
     const int ranges = std::min(kMaxRanges, octs);
-    // [ids][weights], part by part
     unsigned* rows = nullptr;
-    FFI_TRY(workspace_get(s, kWsRows, (size_t)d.L * octs * 8 * (4 + value), (void**)&rows));
+    FFI_TRY(workspace_get(s, kWsRows, phased_rows_bytes<BF16>(d.L, d.K), (void**)&rows));
     void* row_w = rows + (size_t)d.L * octs * 8;
     hipLaunchKernelGGL((rows_by_range_kernel<BF16>), dim3((unsigned)((d.L + rows_per_block - 1) / rows_per_block)), dim3(256), 0, s, a.idx, a.w,
                        rows, row_w, d.L, d.K, (unsigned)((d.N + ranges - 1) / ranges), ranges);
@@ -981,6 +983,13 @@ int launch_forward_bf16(const unsigned short* x, const int32_t* idx, const unsig
     const void* table = nullptr;
     FFI_TRY(make_table<true>(x, d, s, &table));
     return forward_wide<true>(table, idx, w, nullptr, out, TopkSink{}, d, s);
+}
+
+void forward_wide_workspaces(const Dims& d, size_t* features, size_t* rows) {
+    const SlicedForm f = sliced_form<false>(d.B, d.N);
+    const size_t slice_bytes = (size_t)d.N * f.gl * 16;
+    *features = f.in_lds ? 0 : slice_bytes * f.slices;
+    *rows = !f.in_lds && takes_phases(slice_bytes, f.gl, f.slices, d.K, 4) ? phased_rows_bytes<false>(d.L, d.K) : 0;
 }
 
 // Narrow inputs, fp32: up to 16 samples half or more of a 32-sample tile would be computed for nothing (768 x 670,091 x 32, one to

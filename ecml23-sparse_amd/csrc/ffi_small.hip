@@ -217,19 +217,32 @@ int launch_forward_small(const float* x, const int32_t* idx, const float* w, con
     return FFI_OK;
 }
 
+namespace {
+
+// Shares of the connections with 2,048 adds each (2.5 us), or four to each sum that the share then has to exchange (25 G/s on
+// the whole GPU), as long as the workgroups stay within two per CU.
+int small_parts(const Dims& d, const SmallShape& sh) {
+    const long long share = (long long)std::max(2048, 4 * sh.window) * ((d.N + sh.window - 1) / sh.window), LK = (long long)d.L * d.K;
+    return (int)std::max(1ll, std::min((LK + share - 1) / share, 2 * device_cu_count() / std::max(1ll, sh.units)));
+}
+
+}  // namespace
+
+size_t small_backward_workspace(const Dims& d) {
+    const SmallShape sh = small_shape(d);
+    const int parts = small_parts(d, sh);
+    return parts > 1 ? (size_t)sh.units * parts * sh.window * sizeof(float) : 0;
+}
+
 int launch_backward_small(const float* x, const int32_t* idx, const float* w, const float* g, float* gx, float* gw, float* gb, const Dims& d,
                           hipStream_t s, unsigned long long* bad) {
     const SmallShape sh = small_shape(d);
-    const int window = sh.window, units = (int)sh.units, LK = d.L * d.K;
-    // Shares of the connections with 2,048 adds each (2.5 us), or four to each sum that the share then has to exchange (25 G/s on
-    // the whole GPU), as long as the workgroups stay within two per CU.
-    const long long share = (long long)std::max(2048, 4 * window) * ((d.N + window - 1) / window);
-    const int parts = (int)std::max(1ll, std::min((LK + share - 1) / share, (long long)(2 * device_cu_count() / std::max(1, units))));
+    const int window = sh.window, units = (int)sh.units, LK = d.L * d.K, parts = small_parts(d, sh);
     const int gx_groups = gx != nullptr ? units * parts : 0;
     unsigned* partial = nullptr;
     unsigned* tickets = nullptr;
     if (gx_groups && parts > 1) {
-        FFI_TRY(workspace_get(s, kWsPartials, (size_t)gx_groups * window * sizeof(float), (void**)&partial));
+        FFI_TRY(workspace_get(s, kWsPartials, small_backward_workspace(d), (void**)&partial));
         FFI_TRY(tickets_get(s, (void**)&tickets));
     }
     const int splits = std::min(sh.threads / 64, d.B > 64 ? 16 : d.B > 8 ? 4 : 1), total = LK + (gb != nullptr ? d.L : 0), per = sh.threads / splits;

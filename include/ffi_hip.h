@@ -220,7 +220,9 @@ size_t ffi_cache_bytes(void);
  * the per-stream workspaces.  The reference's op owns no memory (TensorFlow allocates every buffer,
  * tfsparse/cc/kernels/register.cpp:29,59-60); this lets a caller budget for what this library adds.  The plan's size
  * depends on the lookup's content: the figure assumes column ids drawn uniformly (as the reference draws them,
- * sparse/custom_layer.py:15,38) and is an estimate; ffi_cache_bytes() reports the actual amount afterwards.  Needs a
+ * sparse/custom_layer.py:15,38) and is an estimate; ffi_cache_bytes() reports the actual amount afterwards.  Other entry
+ * points keep workspaces of their own beside it: top-k calls 64 KiB of candidates per sample and the scores of up to 32,767
+ * sampled labels for each (wide inputs: those labels' rows too), the fused loss and optimizer calls a weight gradient.  Needs a
  * current device only for the number of compute units; returns 0 for shapes the entry points reject.
  */
 enum ffi_pass_flags { FFI_PASS_FORWARD = 1, FFI_PASS_BACKWARD = 2 };

@@ -808,7 +808,9 @@ def test_plan_layouts_serve_any_batch_size(ffi, shape):
 @pytest.mark.parametrize("shape", [(128, 768, 60_000, 32, True), (32, 768, 40_000, 32, True), (256, 512, 30_000, 64, True),
                                    (64, 300, 20_000, 12, False), (96, 2000, 5_000, 20, False), (40, 1100, 9_000, 16, True),
                                    (160, 128, 40_000, 16, True), (300, 200, 40_000, 16, False),     # (several input-gradient workgroups per CU)
-                                   (128, 768, 160_000, 32, True), (64, 1100, 200_000, 16, True)])   # (plans that sort a tile's columns by length; two column windows)
+                                   (128, 768, 160_000, 32, True), (64, 1100, 200_000, 16, True),    # (plans that sort a tile's columns by length; two column windows)
+                                   (96, 65_536, 40_000, 40, True), (20, 30_000, 200_000, 24, False), (3, 150_000, 20_000, 8, True),    # (forward in phases, several slices; short lists)
+                                   (17, 4000, 3000, 44, False), (8, 700, 9000, 24, False), (12, 600, 60_000, 8, False)])            # (small layers; few samples)
 def test_workspace_estimate_brackets_what_the_library_holds(ffi, shape):
     # ffi_workspace_bytes() is asked before anything is allocated; ffi_cache_bytes() says what forward + backward then
     # hold (plans + workspaces).  The estimate models the padding of the plan for uniformly drawn ids.
@@ -821,6 +823,9 @@ def test_workspace_estimate_brackets_what_the_library_holds(ffi, shape):
     x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=L)
     xin = np.ascontiguousarray(x.T) if tp else x
     hip_forward(ffi, xin, lookup, w, tp)
+    forward_only, held = lib.ffi_workspace_bytes(B, N, L, K, int(tp), 1), lib.ffi_cache_bytes()
+    print(f"case shape={shape} forward only: estimate={forward_only} held={held}", flush=True)
+    assert 0.8 * held <= forward_only <= 1.3 * held + (1 << 20)
     hip_backward(ffi, xin, lookup, w, g, tp)
     held = lib.ffi_cache_bytes()
     print(f"case shape={shape} estimate={estimate} held={held}", flush=True)
