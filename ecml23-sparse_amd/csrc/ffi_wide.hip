@@ -481,6 +481,9 @@ void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, 
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
                          bool tp, hipStream_t s) {
     if (!p->oct_ptr || !p->slot_pos || !p->slot_lab) return FFI_ERR_BAD_ARGUMENT;
+    // (before anything is enqueued: a refused call leaves its outputs alone)
+    const dim3 gx_grid((unsigned)((p->N + 31) / 32), (unsigned)(((long long)B + 31) / 32));
+    if (gx_grid.y > 65535u) return FFI_ERR_TOO_LARGE;
     const bool dot = gw != nullptr;
     int gl, slices, m;
     WalkArgs a{};
@@ -518,10 +521,8 @@ int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, cons
         hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((p->L + 63) / 64)), dim3(256), 0, s, g, bias_grad, B, p->L);
         FFI_HIP_TRY(hipGetLastError());
     }
-    const dim3 grid((unsigned)((p->N + 31) / 32), (unsigned)((B + 31) / 32));
-    if (grid.y > 65535u) return FFI_ERR_TOO_LARGE;
-    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
-    else hipLaunchKernelGGL(gather_gx_kernel<false>, grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
+    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
+    else hipLaunchKernelGGL(gather_gx_kernel<false>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }

@@ -336,3 +336,21 @@ def test_more_lookups_than_the_cache_holds(ffi):
     assert held[1] == held[2]                                    # (nothing piles up)
     ffi._lib.check(lib.ffi_cache_clear())
     assert lib.ffi_cache_bytes() == 0
+
+
+def test_a_batch_that_is_too_large_is_refused_before_anything_is_written(ffi):
+    B, N, L, K = 65_535 * 32 + 1, 1217, 4, 2
+    lib = ffi._lib.lib()
+    x, gx = torch.empty((N, B), device="cuda"), torch.empty((N, B), device="cuda")
+    gx[:, :8] = gx[:, -8:] = 7.0
+    lookup, w = torch.zeros((L, K), dtype=torch.int32, device="cuda"), torch.zeros((L, K), device="cuda")
+    g, gw = torch.zeros((B, L), device="cuda"), torch.full((L, K), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    status = lib.ffi_backward_f32(x.data_ptr(), lookup.data_ptr(), w.data_ptr(), g.data_ptr(), gx.data_ptr(), gw.data_ptr(), B, N, L, K, 1,
+                                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert status == -3
+    assert bool((gw == 7.0).all()) and bool((gx[:, :8] == 7.0).all()) and bool((gx[:, -8:] == 7.0).all())
+    del x, gx
+    torch.cuda.empty_cache()
+    ffi._lib.check(lib.ffi_cache_clear())
