@@ -287,9 +287,21 @@ __global__ __launch_bounds__(256) void topk_select_kernel(float* cand_val, int* 
                 if (src.scores != nullptr) {
                     v = src.scores[(size_t)b * src.L + j];
                 } else {
-                    for (int c = 0; c < src.K; ++c) {
-                        const unsigned id = min((unsigned)src.idx[(size_t)j * src.K + c], (unsigned)src.N - 1u);
-                        v = fmaf(as_float(w[(size_t)j * src.K + c]), as_float(src.tp ? x[(size_t)id * B + b] : x[(size_t)b * src.N + id]), v);
+                    const size_t row = (size_t)j * src.K;
+                    for (int c0 = 0; c0 < src.K; c0 += 8) {           // (eight ids, then eight operands in flight)
+                        unsigned id[8];
+                        float wv[8], xv[8];
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) {
+                            const size_t at = row + min(c0 + c, src.K - 1);
+                            id[c] = min((unsigned)src.idx[at], (unsigned)src.N - 1u);
+                            wv[c] = as_float(w[at]);
+                        }
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) xv[c] = as_float(src.tp ? x[(size_t)id[c] * B + b] : x[(size_t)b * src.N + id[c]]);
+#pragma unroll
+                        for (int c = 0; c < 8; ++c)
+                            if (c0 + c < src.K) v = fmaf(wv[c], xv[c], v);
                     }
                     if (src.bias != nullptr) v += src.bias[j];
                 }
