@@ -67,7 +67,7 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsScores = 8, kWsRows = 9, kWsWeightParts = 10, kWsHostWords = 11, kWsTickets = 12 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 // 128 bytes of pinned host memory of the stream, for results that the host waits for
 int host_words_get(hipStream_t s, void** out);
@@ -222,7 +222,6 @@ void nonzero_count_forget(int device);
 int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
                               float* bias_grad, unsigned char* active, const Dims& d, hipStream_t s);
 bool sparse_input_grad_fits(int N, int K);
-bool sparse_weight_grad_fits(int B, int N);   // x within 32-bit byte offsets
 bool sparse_weight_grad_fits(int B, int N);   // x within 32-bit byte offsets
 // g[b,j] = 0 wherever the mask bit of (b,j) is clear
 int launch_zero_unmasked(float* g, const unsigned* words, int B, int L, hipStream_t s);

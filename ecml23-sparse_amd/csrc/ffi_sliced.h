@@ -1,4 +1,4 @@
-// Sample-sliced copies of the gathered operand for inputs that do not fit in LDS: layout, and how work is dealt to the XCDs.
+// Sample-sliced copies of a gathered operand that does not fit in LDS: layout, and how work is dealt to the XCDs.
 //
 // A gather of a row costs what its cache lines cost where they are found.  Measured (rows of 128 bytes at random places,
 // eight lanes of 16 bytes per row): 31 TB/s out of an XCD's own 4-MB L2, 15 TB/s from a table of 8 MB per XCD, 10 from
@@ -36,7 +36,6 @@ inline unsigned xcd_grid(int units) { return (unsigned)((units + kXcds - 1) / kX
 
 // dst[slice][row][SL] = the samples of every row of a matrix given as [rows, B] (tp) or [B, rows]; zeros behind sample B.
 int launch_slices_f32(const float* src, float* dst, int rows, int B, int sl, bool tp, hipStream_t s);
-int launch_slices_bf16(const unsigned short* src, unsigned short* dst, int rows, int B, int sl, bool tp, hipStream_t s);
 
 }  // namespace ffi
 

@@ -1,5 +1,6 @@
-// Forward pass for inputs whose tile does not fit in LDS (more than 1,216 columns), fp32 and bf16: gathers from
-// sample-sliced tables that stay in an XCD's L2 (ffi_sliced.h).
+// Forward pass over slices of the samples, fp32 and bf16: gathers from tables that an XCD's L2 holds (ffi_sliced.h), in phases
+// where it does not hold them, or from the slice in LDS (narrow inputs in bf16 or with few samples); and the top-k of its scores
+// without the score matrix.
 #include "ffi_sliced.h"
 #include "ffi_lds_tile.h"
 
@@ -966,9 +967,6 @@ int forward_wide(const void* table, const int32_t* idx, const void* w, const flo
 }  // namespace
 
 int launch_slices_f32(const float* src, float* dst, int rows, int B, int sl, bool tp, hipStream_t s) {
-    return launch_slices(src, dst, rows, B, sl, tp, s);
-}
-int launch_slices_bf16(const unsigned short* src, unsigned short* dst, int rows, int B, int sl, bool tp, hipStream_t s) {
     return launch_slices(src, dst, rows, B, sl, tp, s);
 }
 

@@ -1,12 +1,7 @@
-// Wide-input kernels of the fixed-fan-in sparse layer for gfx950 (any shape; used when a
-// [N][32] tile of x does not fit in LDS).
-//
-// With tens of thousands of input columns neither x nor out_grad can live in LDS, so the gathered
-// operand comes through the cache hierarchy instead.  Everything is arranged so that one gather is
-// one contiguous row: features are used as xT[N][B] and out_grad (for the input gradient) as
-// gT[L][B], lanes run along the batch, and the column id / weight of the current connection are
-// wave-uniform scalars.  The kernels are bound by cache (L2 / last-level) bandwidth: every
-// connection moves B*4 bytes.
+// Backward pass for inputs whose tile does not fit in LDS (more than 1,216 columns), and for any other shape whose plan has the
+// global form: both gradients in one walk over the plan's lists, out_grad gathered from slices that an XCD's L2 holds a block of
+// labels of at a time (ffi_sliced.h); and the weight gradient alone, straight from the lookup, whose gathers of whole rows of the
+// batch-major features come through the cache hierarchy.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 #include "ffi_sliced.h"

@@ -24,7 +24,10 @@
  *     the staged features in LDS (reads past the end of LDS return zero; no device memory outside the call's
  *     buffers is touched).  ffi_check_lookup audits a matrix;
  *   - outputs are fully overwritten; work is enqueued on `stream` (a hipStream_t passed as void*,
- *     NULL = the default stream) and, with two documented exceptions, never synchronises the host;
+ *     NULL = the default stream) and the host does not wait for it, except where an entry says so: whatever builds a
+ *     plan (the first backward call of a lookup or after a rewiring, ffi_plan_create / ffi_plan_refresh), the calls that
+ *     count the non-zero loss gradients, ffi_topk_hits_f32 and ffi_check_lookup; and a call that needs a larger workspace
+ *     than its stream has kept;
  *   - every function returns FFI_OK (0) or a negative ffi_status instead of aborting, where the
  *     reference fail-fasts through gsl_Expects (forward.cu:19-28, backward.cu:27-40):
  *     null pointers, any dimension <= 0 or > INT32_MAX, num_units*fan_in > INT32_MAX.
@@ -105,7 +108,7 @@ int ffi_forward_noalloc_f32(const float* features, const int32_t* lookup, const 
  * pointer and shape, so in-place edits of lookup (rewiring, sparse/custom_layer.py:32-43) must be picked up:
  *   - edits made through this library (ffi_rewire_f32, ffi_arrange_connections_f32) mark the cached view outdated
  *     on the host, and the next backward call rebuilds it before it enqueues anything (that call synchronises
- *     `stream` and takes the time of a plan build, about 2 ms at 670,091 x 32 connections; results stay
+ *     `stream` and takes the time of a plan build, 0.75 ms at 768 columns and 670,091 x 32 connections; results stay
  *     bit-reproducible);
  *   - edits by foreign code are caught by a content fingerprint that a kernel re-checks on every call, on the
  *     device, without a host wait: every call enqueued before the host has seen the verdict -- the first call after
@@ -345,12 +348,12 @@ int ffi_forward_loss_f32(const float* features, const int32_t* lookup, const flo
  * Forward pass with a per-sample top-k in fp32 (1 <= k <= 8), same ordering rule as ffi_forward_topk_bf16 (scores
  * descending, equal scores by ascending label: tf.nn.top_k, sparse/metrics.py:19).  `bias` may be NULL.  The
  * [batch, num_units] score matrix is written only if `scores` is given.  How: a sample of the labels is scored
- * first and fixes, per sample, a threshold that k labels are known to reach; the forward kernel then appends
- * every score at or above its sample's threshold to a candidate list (a tiny share of all labels), and the k
- * best candidates are selected.  The result is exact.  A sample whose candidates overflow its list (8192 slots;
- * e.g. thousands of labels tied with the k-th score, as an all-zero feature row gives) is answered from a scan of its
- * whole row instead (on the device, without a host wait; slower for that sample only), so ties still resolve to the
- * lower labels as tf.nn.top_k resolves them.
+ * first and fixes, per sample, a score and label that k labels are known to reach in that order; the forward kernel
+ * then appends every label that reaches them to a candidate list (a tiny share of all labels, also where scores tie by
+ * the thousand, as an all-zero feature row gives), and the k best candidates are selected.  The result is exact.  A sample
+ * whose candidates overflow its list (8192 slots: thousands of labels better than all of the sample's, e.g. at every
+ * other label) is answered from a scan of its whole row instead (on the device, without a host wait).  Scores that are no
+ * number are never listed; where fewer than k others are left, the places behind them hold (-inf, -1).
  * ffi_forward_loss_topk_f32 is ffi_forward_loss_f32 with the same top-k of the scores as a by-product: what a
  * training step needs for the loss, the backward pass and the P@k metrics (sparse/metrics.py:31-71) without
  * the score matrix ever being stored.  No counterpart in the reference.
