@@ -749,7 +749,7 @@ constexpr int kListsPerBlock = kBlock - 1;
 __global__ __launch_bounds__(kBlock) void list_ptr_kernel(const unsigned* __restrict__ sorted_keys, int total, int nkeys,
                                                           int32_t* __restrict__ ptr, unsigned* __restrict__ block_octs) {
     __shared__ int begin[kBlock];
-    const int n = min((int)(blockIdx.x * kListsPerBlock + threadIdx.x), nkeys);
+    const int n = (int)min(blockIdx.x * (unsigned)kListsPerBlock + threadIdx.x, (unsigned)nkeys);
     int lo = 0, hi = total;
     while (lo < hi) {
         const int mid = lo + ((hi - lo) >> 1);
@@ -768,14 +768,14 @@ __global__ __launch_bounds__(kBlock) void list_ptr_kernel(const unsigned* __rest
 // oct_ptr[n] = octs of the lists before list n, from the octs before the list's workgroup of list_ptr_kernel
 __global__ __launch_bounds__(kBlock) void oct_ptr_kernel(const int32_t* __restrict__ ptr, int nkeys, const unsigned* __restrict__ octs_before,
                                                          unsigned* __restrict__ oct_ptr) {
-    const int n = blockIdx.x * kListsPerBlock + threadIdx.x;
-    const bool mine = threadIdx.x < kListsPerBlock && n < nkeys;
+    const unsigned n = blockIdx.x * (unsigned)kListsPerBlock + threadIdx.x;
+    const bool mine = threadIdx.x < kListsPerBlock && n < (unsigned)nkeys;
     const unsigned octs = mine ? (unsigned)(ptr[n + 1] - ptr[n] + 7) / 8u : 0u;
     unsigned long long sum = 0;
     const unsigned at = octs_before[blockIdx.x] + (unsigned)block_sum_below<kBlock>(octs, &sum);
     if (mine) {
         oct_ptr[n] = at;
-        if (n == nkeys - 1) oct_ptr[nkeys] = at + octs;
+        if (n == (unsigned)nkeys - 1u) oct_ptr[nkeys] = at + octs;
     }
 }
 
@@ -1087,19 +1087,21 @@ int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     const int block_labels = plan_block_labels(p->N, p->K, p->L);
     const int nblocks = (p->L + block_labels - 1) / block_labels;
     const long long nkeys = (long long)nblocks * p->N;
-    if (nkeys >= (1ll << 31) - kBlock) return FFI_ERR_TOO_LARGE;
+    if (nkeys >= (1ll << 31) - 1) return FFI_ERR_TOO_LARGE;
     const int end_bit = bits_for((unsigned)(nkeys - 1));
     const unsigned list_blocks = (unsigned)((nkeys + kListsPerBlock - 1) / kListsPerBlock);
     size_t expected = plan_expected_slots(p->N, p->K, p->L), sort_bytes = 0;
-    expected = (std::max<size_t>((size_t)total, std::min<size_t>(expected + expected / 128, (1ull << 32) - 64)) + 7) / 8 * 8;
-    // (two buffers, not four: an allocation is 50 us and more)
+    expected = (std::max<size_t>((size_t)total, std::min<size_t>(expected + expected / 128, (1ull << 32) - 64)) + 63) / 64 * 64;
+    // (two buffers, not four: an allocation is 50 us and more; each array on a line of its own)
     auto alloc_slots = [&](size_t slots) {
-        if (!dev_alloc(p, &p->slot_pos, slots + (slots + 1) / 2)) return false;
+        slots = (slots + 63) / 64 * 64;
+        if (!dev_alloc(p, &p->slot_pos, slots + slots / 2)) return false;
         p->slot_lab = reinterpret_cast<unsigned short*>(p->slot_pos + slots);
         return true;
     };
-    if (!alloc_slots(expected) || !dev_alloc(p, &p->oct_ptr, (size_t)nkeys + 1 + (size_t)total)) return FFI_ERR_OUT_OF_MEMORY;
-    p->pos_slot = p->oct_ptr + nkeys + 1;
+    const size_t lists_end = ((size_t)nkeys + 1 + 63) / 64 * 64;
+    if (!alloc_slots(expected) || !dev_alloc(p, &p->oct_ptr, lists_end + (size_t)total)) return FFI_ERR_OUT_OF_MEMORY;
+    p->pos_slot = p->oct_ptr + lists_end;
     // stable LSD radix sort of ((block, column), flat position): positions stay ascending inside a column
     rocprim::double_buffer<unsigned> keys(reinterpret_cast<unsigned*>(p->slot_pos), nullptr);
     rocprim::double_buffer<int32_t> positions(reinterpret_cast<int32_t*>(p->pos_slot), nullptr);
