@@ -938,7 +938,7 @@ int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds) 
 namespace {
 
 // Builds the tiled form.  Returns FFI_OK with p->tiled == false if the padded size would exceed
-// three times the connection count (heavily skewed column usage): the caller then builds the
+// three times the connection count, lanes without a column aside (heavily skewed column usage): the caller then builds the
 // global form instead.
 // (`after_row_assignment`, may be empty: called once the kernel that assigns the labels' LDS rows is enqueued -- it takes
 // nearly all of every CU's LDS for itself, and work for another stream enqueued behind it starts when it ends instead of
@@ -997,10 +997,15 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     if (e != hipSuccess) return hip_fail(e);
     const unsigned long long rows = p->h_scratch[2];
     const unsigned long long connections = (unsigned long long)p->L * p->K;
-    // too skewed (a window of the columns may have two slots per connection of the layer: how many of them fall into
-    // it is not counted), or beyond what the walking kernel's 32-bit buffer offsets reach (256 bytes per row)
+    // Too skewed (a window of the columns may have two slots per connection of the layer: how many of them fall into
+    // it is not counted), or beyond what the walking kernel's 32-bit buffer offsets reach (256 bytes per row).  Lanes
+    // that have no column do not count: they take slots, but no time that another form would save.  (With them counted,
+    // inputs of fewer than some 30 columns, of 40 where tiles are small, took the global form, whose walk has too few columns
+    // to fill the GPU.  Both gradients at 21 columns, tiled against global: 327 x 5,088 x 7 64 us against 391,
+    // 64 x 100,000 x 16 74 / 263, 128 x 670,091 x 32 1,115 / 2,614; at 12 columns, 8 x 200,000 x 12, 201 / 237.  At 6 and 3
+    // columns that last shape is the one that turns, 323 / 276 and 559 / 418; 327 x 5,088 x 7 there 80 / 1,023 and 99 / 2,020.)
     const unsigned long long allowed = p->col_n ? 2ull : 3ull;
-    if (rows * 64ull > allowed * connections + 64ull * nslices || rows >= (1ull << 24)) return FFI_OK;
+    if (rows * 64ull * (unsigned long long)cols > (allowed * connections + 64ull * nslices) * (unsigned long long)threads || rows >= (1ull << 24)) return FFI_OK;
     if (w_in_lds) {
         if (!dev_alloc(p, &p->slot32, (size_t)rows * 64)) return FFI_ERR_OUT_OF_MEMORY;
     } else if (!dev_alloc(p, &p->lab16, (size_t)rows * 64) || !dev_alloc(p, &p->pos16, (size_t)rows * 64)) {

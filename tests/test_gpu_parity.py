@@ -986,3 +986,31 @@ def test_drawn_shapes(ffi, shape):
     o_gx, o_gw = oracle.backward(xin, lookup, w, g, transposed=transposed)
     assert rel_err(gw, o_gw) <= GRAD_RTOL
     assert rel_err(gx, o_gx) <= GRAD_RTOL
+
+
+# A few columns: the tiled form for uniform ids, however few lanes of its workgroups have a column; the global form for a layer whose
+# connections meet in one of many
+@pytest.mark.parametrize("N", [1, 2, 12, 21, 33, 63, 65, 70, 129, 300])
+@pytest.mark.parametrize("B,L,K", [(33, 2_000, 5), (327, 5_088, 7), (8, 9_001, 32)])
+def test_plan_form_and_gradients_at_few_columns(ffi, N, B, L, K):
+    lib = ffi._lib.lib()
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=N + B)
+    for tiled in (True, False):
+        if not tiled:
+            if N < 300:
+                break
+            lookup[:] = 7
+        dl, dw, dg = dev(lookup), dev(w), dev(g)
+        plan, info = ctypes.c_void_p(), (ctypes.c_int64 * 8)()
+        ffi._lib.check(lib.ffi_plan_create(dl.data_ptr(), L, K, N, B, stream(), ctypes.byref(plan)))
+        ffi._lib.check(lib.ffi_plan_info(plan, info))
+        assert info[0] == int(tiled)
+        ffi._lib.check(lib.ffi_plan_destroy(plan))
+        assert lib.ffi_set_option(b"small_path", -1) == 0
+        try:
+            o_gx, o_gw = oracle.backward(x, lookup, w, g, transposed=False)
+            for _ in range(2):
+                gx, gw = ffi.fan_in_sparse_matmul_grad(dev(x), dl, dw, dg)
+                assert rel_err(gx.cpu().numpy(), o_gx) <= GRAD_RTOL and rel_err(gw.cpu().numpy(), o_gw) <= GRAD_RTOL
+        finally:
+            lib.ffi_set_option(b"small_path", 0)
