@@ -565,105 +565,149 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
 // octs with connections that name no column (the gather of one returns zero without touching memory).  Oct r of all rows --
 // part r -- is stored in one piece.  Octs of the ordered row and not the ranges themselves: the lists of the lane groups are
 // equally long, and the columns of a part still lie close together.
-// A lane holds four entries, a row a group of 2 Q neighbouring lanes: at most 256 connections.  Both sides go through the
-// wavefront's part of LDS, so that memory is read and written in whole lines.
+// Eight lanes have a row, each an eighth of it, one connection after the other: a counter per range in a byte of a register
+// says where the next connection of that range goes.  Both sides pass through the wavefront's part of LDS, so that memory is
+// read and written in whole lines.
+//
+// What bounds it: memory.  (With the places from ballots, range by range, 3.9 instructions of a wavefront per connection and
+// bound by them: 300 us for 670,091 x 72 in fp32, 210 for x 64 in bf16.)
 constexpr int kMaxRanges = 16;
 constexpr int kMaxRangedFanIn = 256;
+constexpr int kRbrRows = 8;                                       // rows per wavefront
+// connections per lane: odd, so that the lanes' words fall into different banks
+__host__ __device__ constexpr int ranged_share(int K) { return (K + 7) / 8 | 1; }
+inline size_t rows_by_range_lds(int K) { return (size_t)4 * kRbrRows * (8 * ranged_share(K) + (K + 7) / 8 * 8) * 2 * sizeof(unsigned); }
 
-template <bool BF16>
+template <bool BF16, bool MANY>
 __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __restrict__ idx, const void* __restrict__ w,
                                                             unsigned* __restrict__ idx_out, void* __restrict__ w_out,
-                                                            int L, int K, unsigned range_cols, int ranges) {
-    __shared__ __align__(16) unsigned mem[4][2][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned* sid = mem[wave][0];
-    unsigned* sw = mem[wave][1];
-    const int octs = (K + 7) / 8, gs = 2 * octs, rows = 64 / gs;         // lanes per row, rows per wavefront
-    const long long row0 = ((long long)blockIdx.x * 4 + wave) * rows;
-    const int nrows = (int)min((long long)rows, (long long)L - row0);    // (may be <= 0)
+                                                            int L, int K, unsigned magic, int ranges) {
+    extern __shared__ __align__(16) unsigned rbr_mem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int share = ranged_share(K), pitch = 8 * share, octs = (K + 7) / 8, out_pitch = octs * 8;
+    unsigned* const in_id = rbr_mem + wave * (kRbrRows * (pitch + out_pitch) * 2);
+    unsigned* const in_w = in_id + kRbrRows * pitch;
+    unsigned* const out_id = in_w + kRbrRows * pitch;
+    unsigned* const out_w = out_id + kRbrRows * out_pitch;
+    const long long row0 = ((long long)blockIdx.x * 4 + wave) * kRbrRows;
+    const int nrows = (int)min((long long)kRbrRows, (long long)L - row0);    // (may be <= 0)
     const int total = nrows * K;
-    for (int f = lane; f < total; f += 64) {
-        const size_t at = (size_t)row0 * K + f;
-        sid[f] = (unsigned)idx[at];
-        sw[f] = BF16 ? (unsigned)reinterpret_cast<const unsigned short*>(w)[at] : reinterpret_cast<const unsigned*>(w)[at];
-    }
-    __builtin_amdgcn_wave_barrier();
-    const int r = lane / gs, sub = lane - r * gs;
-    const bool in_row = r < nrows;
-    unsigned id[4], wv[4], range[4];
+    const unsigned per_row = (1u << 21) / (unsigned)K + 1u;                  // f / K = f * per_row >> 21 for f < 2,560 and K <= 256
+    constexpr int kTogether = 8;                                             // loads in flight
+    for (int f0 = lane; f0 < total; f0 += 64 * kTogether) {
+        unsigned id[kTogether], wv[kTogether];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int k = 4 * sub + e;
-        const bool on = in_row && k < K;
-        id[e] = on ? sid[r * K + k] : 0u;
-        wv[e] = on ? sw[r * K + k] : 0u;
-        range[e] = on ? min(id[e] / range_cols, (unsigned)ranges - 1u) : 0xffu;
-    }
-    const unsigned long long group = (gs == 64 ? ~0ull : (1ull << gs) - 1ull) << (r * gs);
-    const unsigned long long before = ((1ull << lane) - 1ull) & group;
-    int to[4] = {0, 0, 0, 0}, begin = 0;
-    for (unsigned q = 0; q < (unsigned)ranges; ++q) {
-        int mine = begin;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const unsigned long long m = __ballot(range[e] == q);
-            mine += __popcll(m & before);
-            begin += __popcll(m & group);
+        for (int i = 0; i < kTogether; ++i) {
+            const size_t at = (size_t)row0 * K + min(f0 + 64 * i, total - 1);
+            id[i] = (unsigned)idx[at];
+            wv[i] = BF16 ? (unsigned)reinterpret_cast<const unsigned short*>(w)[at] : reinterpret_cast<const unsigned*>(w)[at];
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (range[e] == q) to[e] = mine++;
-    }
-    __builtin_amdgcn_wave_barrier();
-    reinterpret_cast<uint4*>(sid)[lane] = make_uint4(~0u, ~0u, ~0u, ~0u);        // (rows * gs <= 64 quads)
-    reinterpret_cast<uint4*>(sw)[lane] = make_uint4(0u, 0u, 0u, 0u);
-    __builtin_amdgcn_wave_barrier();
-    if (in_row) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (range[e] != 0xffu) { sid[4 * r * gs + to[e]] = id[e]; sw[4 * r * gs + to[e]] = wv[e]; }
-    }
-    __builtin_amdgcn_wave_barrier();
-    for (int q = 0; q < octs; ++q) {
-        const size_t base = (size_t)q * 2 * L + (size_t)row0 * 2;        // (in quads)
-        for (int f = lane; f < nrows * 2; f += 64) {
-            const int from = (f >> 1) * gs + 2 * q + (f & 1);
-            reinterpret_cast<uint4*>(idx_out)[base + f] = reinterpret_cast<const uint4*>(sid)[from];
-            const uint4 v = reinterpret_cast<const uint4*>(sw)[from];
-            if (BF16) reinterpret_cast<uint2*>(w_out)[base + f] = make_uint2(v.x | v.y << 16, v.z | v.w << 16);
-            else reinterpret_cast<uint4*>(w_out)[base + f] = v;
+        for (int i = 0; i < kTogether; ++i) {
+            const int f = f0 + 64 * i, r = (int)((unsigned)f * per_row >> 21), to = r * pitch + (f - r * K);
+            if (f < total) { in_id[to] = id[i]; in_w[to] = wv[i]; }
         }
+    }
+    __builtin_amdgcn_wave_barrier();                                         // (the memory is the wavefront's own, and LDS serves it in order)
+    const int r = lane >> 3, sub = lane & 7;
+    const int first = sub * share, n = r < nrows ? min(share, K - first) : 0;
+    const unsigned* my_id = in_id + r * pitch + first;
+    const unsigned* my_w = in_w + r * pitch + first;
+    // any function of the id that never falls would do: this one is the column's range, give or take rounding
+    auto range_of = [&](unsigned id) { return min(__umulhi(id, magic), (unsigned)ranges - 1u); };
+    // a byte per range: the lane's connections, those of the lanes before it, all of the row's.  (A count of 256 runs over into
+    // bytes of ranges that are then empty.)
+    unsigned long long lo = 0, hi = 0;
+    for (int i = 0; i < n; ++i) {
+        const unsigned q = range_of(my_id[i]);
+        const unsigned long long one = 1ull << (8 * (q & 7));
+        if (MANY && q >= 8) hi += one;
+        else lo += one;
+    }
+    auto before = [&](unsigned long long mine, unsigned long long& row) {
+        unsigned long long sum = mine;
+#pragma unroll
+        for (int d = 1; d < 8; d *= 2) {
+            const unsigned long long other = __shfl_up(sum, d, 8);
+            if (sub >= d) sum += other;
+        }
+        row = __shfl(sum, 7, 8);
+        return sum - mine;
+    };
+    unsigned long long lo_row, hi_row = 0;
+    const unsigned long long lo_before = before(lo, lo_row), hi_before = MANY ? before(hi, hi_row) : 0;
+    constexpr unsigned long long kOnes = 0x0101010101010101ull;
+    const unsigned long long lo_upto = lo_row * kOnes;                       // byte q: the row's connections of ranges up to q
+    unsigned long long lo_next = (lo_upto << 8) + lo_before;
+    unsigned long long hi_next = MANY ? ((hi_row * kOnes) << 8) + (lo_upto >> 56) * kOnes + hi_before : 0;
+    for (int i = 0; i < n; ++i) {
+        const unsigned id = my_id[i], wv = my_w[i], q = range_of(id), shift = 8 * (q & 7);
+        const bool up = MANY && q >= 8;
+        const unsigned to = (unsigned)((up ? hi_next : lo_next) >> shift) & 255u;
+        if (up) hi_next += 1ull << shift;
+        else lo_next += 1ull << shift;
+        out_id[r * out_pitch + to] = id;
+        out_w[r * out_pitch + to] = wv;
+    }
+    if (K + sub < out_pitch) {
+        out_id[r * out_pitch + K + sub] = ~0u;
+        out_w[r * out_pitch + K + sub] = 0u;
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int f = lane; f < octs * 2 * kRbrRows; f += 64) {
+        const int q = f / (2 * kRbrRows), e = f % (2 * kRbrRows);            // oct; quad e & 1 of row e / 2
+        if (e >= 2 * nrows) continue;
+        const size_t to = (size_t)q * 2 * L + (size_t)row0 * 2 + e;          // (in quads)
+        const int from = (e >> 1) * out_pitch + q * 8 + (e & 1) * 4;
+        *(reinterpret_cast<uint4*>(idx_out) + to) = *reinterpret_cast<const uint4*>(out_id + from);
+        const uint4 v = *reinterpret_cast<const uint4*>(out_w + from);
+        if (BF16) reinterpret_cast<uint2*>(w_out)[to] = make_uint2(v.x | v.y << 16, v.z | v.w << 16);
+        else reinterpret_cast<uint4*>(w_out)[to] = v;
     }
 }
 
 // ---- forward in phases --------------------------------------------------------------------------------------------
-// For slices that do not fit an XCD's L2: a workgroup of 16 wavefronts takes 128 M labels -- their sums stay in registers -- and
-// goes through the parts of their rows (above: one oct of connections per label and part) in order, a barrier behind each.
-// All workgroups of an XCD begin at the same time and do the same work, so the gathers of a phase hit the few MB of the
-// slice that its part of the rows names.
+// For slices that do not fit an XCD's L2: a workgroup takes 88 M labels -- their sums stay in registers -- and goes through the
+// parts of their rows (above: one oct of connections per label and part) in order, a barrier behind each.  All workgroups of
+// an XCD begin at the same time and do the same work, so the gathers of a phase hit the few MB of the slice that its part of
+// the rows names.
 //
-// The gathers of a step (eight labels, an oct each) are issued before the sums of the step before them, so that a wavefront
-// always has eight in flight.  The lists of a part are written two parts, its ids and weights asked for three parts ahead of
-// their use at the latest: loads return in order, and a load from memory in front of the gathers would hold them up.
+// One wavefront brings the lists of all others, two parts ahead and past the registers; the others have nothing but gathers in
+// flight.  Loads return in order, and lists that each wavefront asked for itself held its gathers up for the time of the fabric
+// once a phase (with their lines marked for one use, which takes longer, the pass went from 2.1 to 2.9 ms).  The gathers of a
+// step (eight labels, an oct each) are issued before the sums of the step before them, so that a wavefront always has eight in
+// flight.  Twelve wavefronts and not sixteen: with 168 registers the sums of 704 labels fit a workgroup, and a slice is gone
+// through less often (misses of L2 77 -> 60 M lines in bf16).
 //
-// What bounds it: L2 delivery, as in fwd_sliced_kernel.
-constexpr int kPhThreads = 1024;
+// What bounds it: the L1's 64 bytes per clock, busy 88 % of the time.  670,091 labels, against sixteen wavefronts that bring
+// their own lists, 512 labels: 128 samples, 65,536 columns, fan-in 72 in fp32 1,215 -> 1,139 us (21.7 TB/s); 512 samples, 100,000
+// columns, fan-in 64 in bf16 2,112 -> 2,000 us.
+constexpr int kPhWaves = 11, kPhThreads = (kPhWaves + 1) * 64;    // wavefronts that walk, and one that brings their lists
 
-template <bool BF16> struct PhasedShape {
-    static constexpr int kM = 4;                                  // labels per lane group: 64 lanes bring the 32 labels' octs, a quad each
-    static constexpr int kWaveLabels = 8 * kM;
-    static constexpr int kLabels = kWaveLabels * (kPhThreads / 64);
-    static constexpr int kOctWords = 5;                           // 16-byte words per label in LDS: four, and one against bank conflicts
-    static constexpr size_t kListBytes = (size_t)2 * kLabels * kOctWords * 16;
+// `bytes` (a multiple of 1,024) from the resource's begin on into LDS, past the registers, by one wavefront
+__device__ __forceinline__ void bring_to_lds(buffer_rsrc from, unsigned char* to, int bytes, int lane) {
+#pragma unroll 4
+    for (int t = 0; t < bytes; t += 1024)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) unsigned char*)to + t, 16, lane * 16 + t, 0, 0, 0);
+}
+
+template <bool BF16, int M> struct PhasedShape {                  // M: labels per lane group
+    static constexpr int kWaveLabels = 8 * M;
+    static constexpr int kLabels = kWaveLabels * kPhWaves;
+    static constexpr int kIdBytes = kLabels * 32, kWeightBytes = (kLabels * (BF16 ? 16 : 32) + 1023) / 1024 * 1024;
+    static constexpr int kPartBytes = kIdBytes + kWeightBytes;    // a part of the rows: ids, then weights
+    static constexpr int kBuffers = 3;
+    static constexpr size_t kLdsBytes = (size_t)kBuffers * kPartBytes;
+    static_assert(kIdBytes % 1024 == 0, "whole loads of a wavefront");
 };
 
-template <bool BF16>
+template <bool BF16, int M>
 __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __restrict__ table, const unsigned* __restrict__ idx,
                                                                 const void* __restrict__ w, const float* __restrict__ bias,
                                                                 float* __restrict__ out, int B, int N, int L, int octs, int label_blocks,
                                                                 int units, const TopkSink sink) {
-    using S = PhasedShape<BF16>;
-    constexpr int GL = 8, kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer, M = S::kM;
+    using S = PhasedShape<BF16, M>;
+    constexpr int GL = 8, kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer;
     constexpr unsigned kRow = 128u;
     extern __shared__ __align__(16) unsigned char smem[];
     const int u = xcd_unit(blockIdx.x, units);
@@ -671,8 +715,33 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
     const int slice = u / label_blocks;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & (GL - 1), grp = lane / GL;
-    const int jw = (u % label_blocks) * S::kLabels + wave * S::kWaveLabels;             // first label of this wavefront
-    uint4* const lists = reinterpret_cast<uint4*>(smem) + wave * (2 * S::kWaveLabels * S::kOctWords);
+    const int j0 = (u % label_blocks) * S::kLabels;                                     // first label of the workgroup
+    // a barrier that leaves the gathers in flight alone
+    auto pace = [] { asm volatile("" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    if (wave == kPhWaves) {
+        // Part r of the workgroup's rows into its buffer, past the registers.  Behind the last label nothing is read (the
+        // buffers' ends are the resources').
+        const size_t left = (size_t)min(S::kLabels, L - j0);
+        auto bring = [&](int r) {
+            const size_t base = ((size_t)r * L + j0) * 8;
+            const buffer_rsrc ri = make_rsrc(idx + base, left * 32), rw = make_rsrc((const char*)w + base * (BF16 ? 2 : 4), left * (BF16 ? 16 : 32));
+            unsigned char* to = smem + (size_t)(r % S::kBuffers) * S::kPartBytes;
+            bring_to_lds(ri, to, S::kIdBytes, lane);
+            bring_to_lds(rw, to + S::kIdBytes, S::kWeightBytes, lane);
+        };
+        bring(0);
+        if (octs > 1) bring(1);
+        __builtin_amdgcn_s_waitcnt(0x0f70);                                             // vmcnt(0)
+        pace();
+        for (int r = 0; r < octs; ++r) {
+            if (r + 2 < octs) bring(r + 2);
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            pace();
+        }
+        __syncthreads();
+        return;
+    }
+    const int jw = j0 + wave * S::kWaveLabels;                                          // first label of this wavefront
     const size_t slice_bytes = (size_t)N * kRow;
     const buffer_rsrc rows = make_rsrc((const char*)table + (size_t)slice * slice_bytes, slice_bytes);
     const unsigned lane_off = (unsigned)sub * 16u;
@@ -681,82 +750,39 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
     for (int m = 0; m < M; ++m)
 #pragma unroll
         for (int i = 0; i < kPer; ++i) acc[m].a[i] = 0.f;
-
-    // lane f brings quad f & 1 of label f / 2 (of every 32 labels).  Labels behind the last read zeros: a gather of row 0 with
-    // weight zero.  The resource begins at the wavefront's first label and ends with the part (the scalar offset of a buffer
-    // load is not part of its bounds check in every form): a wavefront behind the last label has an empty one.
-    uint4 ids, ws;
-    const int jf = min(jw, L);
-    const size_t left = (size_t)(L - jf);
-    auto fetch = [&](int r) {
-        const size_t base = ((size_t)min(r, octs - 1) * L + jf) * 8;                     // (behind the last part: the last again)
-        const buffer_rsrc ri = make_rsrc(idx + base, left * 32), rw = make_rsrc((const char*)w + base * (BF16 ? 2 : 4), left * (BF16 ? 16 : 32));
-        ids = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ri, lane * 16u, 0, 0));
-        if (BF16) {
-            const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rw, lane * 8u, 0, 0));
-            ws.x = h.x; ws.y = h.y;
-        } else {
-            ws = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16u, 0, 0));
-        }
-    };
-    auto put = [&](int r) {
-        uint4* list = lists + (r & 1) * (S::kWaveLabels * S::kOctWords) + (lane >> 1) * S::kOctWords + (lane & 1) * 2;
-        if (BF16) {                                      // (the weights of two connections share a word)
-            list[0] = make_uint4(ids.x * kRow, ids.y * kRow, ids.z * kRow, ids.w * kRow);
-            reinterpret_cast<uint2*>(list)[2] = make_uint2(ws.x, ws.y);
-        } else {
-            list[0] = make_uint4(ids.x * kRow, ws.x, ids.y * kRow, ws.y);
-            list[1] = make_uint4(ids.z * kRow, ws.z, ids.w * kRow, ws.w);
-        }
-    };
     uint4 x[2][8];
     constexpr int kWt = BF16 ? 4 : 8;
     unsigned wt[2][kWt];
+    // (entries of no connection hold ~0: behind the slice's end, where a load returns zero without touching memory)
     auto gather = [&](int r, int m, uint4 (&xs)[8], unsigned (&wv)[kWt]) {
-        const uint4* list = lists + (r & 1) * (S::kWaveLabels * S::kOctWords) + (m * 8 + grp) * S::kOctWords;
-        unsigned at[8];
-        if (BF16) {
+        const unsigned char* part = smem + (size_t)(r % S::kBuffers) * S::kPartBytes;
+        const int label = wave * S::kWaveLabels + m * 8 + grp;
+        const uint4* ids = reinterpret_cast<const uint4*>(part + label * 32);
+        const uint4* ws = reinterpret_cast<const uint4*>(part + S::kIdBytes + label * (kWt * 4));
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint4 e = list[2 * h];
-                const uint2 f = reinterpret_cast<const uint2*>(list + 2 * h)[2];
-                at[4 * h] = e.x; at[4 * h + 1] = e.y; at[4 * h + 2] = e.z; at[4 * h + 3] = e.w;
-                wv[2 * h] = f.x; wv[2 * h + 1] = f.y;
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint4 e = list[v];
-                at[2 * v] = e.x; at[2 * v + 1] = e.z;
-                wv[(2 * v) % kWt] = e.y; wv[(2 * v + 1) % kWt] = e.w;
-            }
+        for (int v = 0; v < kWt / 4; ++v) {
+            const uint4 e = ws[v];
+            wv[4 * v] = e.x; wv[4 * v + 1] = e.y; wv[4 * v + 2] = e.z; wv[4 * v + 3] = e.w;
         }
+        const uint4 a = ids[0], b = ids[1];
+        const unsigned at[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
         for (int v = 0; v < 8; ++v)
-            xs[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, at[v] + lane_off, 0, 0));
+            xs[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, at[v] * kRow + lane_off, 0, 0));
     };
-    // (the lists are the wavefront's own, and LDS serves it in order)
-    fetch(0);
-    put(0);
-    fetch(1);
-    __builtin_amdgcn_wave_barrier();
+    pace();
     gather(0, 0, x[0], wt[0]);
     for (int r = 0; r < octs; ++r) {
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            if (m == 0) {
-                put(r + 1);
-                __builtin_amdgcn_wave_barrier();
-            }
             if (m + 1 < M) gather(r, m + 1, x[(m + 1) & 1], wt[(m + 1) & 1]);
-            else gather(r + 1, 0, x[(m + 1) & 1], wt[(m + 1) & 1]);
-            if (m == 0) fetch(r + 2);
+            else gather(min(r + 1, octs - 1), 0, x[(m + 1) & 1], wt[(m + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[m].add_pair(x[m & 1][2 * v], x[m & 1][2 * v + 1], &wt[m & 1][v * (kWt / 4)]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_s_barrier();                    // (for the pace: nothing is shared)
+        pace();
     }
     __syncthreads();
     const int b0 = slice * kSl;
@@ -778,11 +804,10 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
         return;
     }
     // a wavefront's labels are consecutive: rows of out leave in pieces of 8 M labels, through the wavefront's part of LDS
-    constexpr int kPitch = S::kWaveLabels + 1, kStep = 2 * S::kWaveLabels * S::kOctWords * 4 / kPitch;       // samples that fit there
-    float* tile = reinterpret_cast<float*>(lists);
+    constexpr int kPitch = S::kWaveLabels + 1, kTake = 16;                                     // samples at a time
+    float* tile = reinterpret_cast<float*>(smem) + wave * (kTake * kPitch);
     const int nb = min(kSl, B - b0);
-    static_assert(kStep >= 8, "a lane's samples at a time");
-    constexpr int kTake = kStep >= kSl ? kSl : kStep >= kSl / 2 ? kSl / 2 : kSl / 4;
+    static_assert((size_t)kPhWaves * kTake * kPitch * sizeof(float) <= S::kLdsBytes && kSl % kTake == 0, "the tiles lie in the lists' place");
     for (int s0 = 0; s0 < nb; s0 += kTake) {
         __builtin_amdgcn_wave_barrier();
         if (sub * kPer >= s0 && sub * kPer < s0 + kTake) {
@@ -792,11 +817,11 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
                 for (int i = 0; i < kPer; ++i) tile[(sub * kPer + i - s0) * kPitch + m * 8 + grp] = acc[m].a[i];
         }
         __builtin_amdgcn_wave_barrier();
-        constexpr int kRowsPerStep = 64 / S::kWaveLabels;
-        const int jl = lane % S::kWaveLabels, j = jw + jl;
-        const float bj = (bias != nullptr && j < L) ? bias[j] : 0.f;
-        for (int e = lane / S::kWaveLabels; e < kTake && s0 + e < nb; e += kRowsPerStep)
-            if (j < L) __builtin_nontemporal_store(bias != nullptr ? tile[e * kPitch + jl] + bj : tile[e * kPitch + jl], out + (size_t)(b0 + s0 + e) * L + j);
+        const int count = min(kTake, nb - s0) * S::kWaveLabels;
+        for (int f = lane; f < count; f += 64) {
+            const int e = f / S::kWaveLabels, jl = f - e * S::kWaveLabels, j = jw + jl;
+            if (j < L) __builtin_nontemporal_store(bias != nullptr ? tile[e * kPitch + jl] + bias[j] : tile[e * kPitch + jl], out + (size_t)(b0 + s0 + e) * L + j);
+        }
     }
 }
 
@@ -877,36 +902,66 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
 // the ordered copy of the layer: [ids][weights], part by part
 template <bool BF16> size_t phased_rows_bytes(int L, int K) { return (size_t)L * ((K + 7) / 8) * 8 * (4 + sizeof(typename LaneAcc<BF16>::Element)); }
 
-template <bool BF16>
-int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
-    using S = PhasedShape<BF16>;
-    const int octs = (d.K + 7) / 8, rows_per_block = 4 * (64 / (2 * octs));
-    const int ranges = std::min(kMaxRanges, octs);
-    unsigned* rows = nullptr;
-    FFI_TRY(workspace_get(s, kWsRows, phased_rows_bytes<BF16>(d.L, d.K), (void**)&rows));
-    void* row_w = rows + (size_t)d.L * octs * 8;
-    hipLaunchKernelGGL((rows_by_range_kernel<BF16>), dim3((unsigned)((d.L + rows_per_block - 1) / rows_per_block)), dim3(256), 0, s, a.idx, a.w,
-                       rows, row_w, d.L, d.K, (unsigned)((d.N + ranges - 1) / ranges), ranges);
-    FFI_HIP_TRY(hipGetLastError());
+template <bool BF16, int M>
+int launch_phased_walk(const FwdSliced& a, const unsigned* rows, const void* row_w, const Dims& d, hipStream_t s) {
+    using S = PhasedShape<BF16, M>;
     const int label_blocks = (d.L + S::kLabels - 1) / S::kLabels, units = label_blocks * a.slices;
-    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_phased_kernel<BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kListBytes));
-    hipLaunchKernelGGL((fwd_phased_kernel<BF16>), dim3(xcd_grid(units)), dim3(kPhThreads), S::kListBytes, s, a.table, rows, row_w, a.bias, a.out,
-                       d.B, d.N, d.L, octs, label_blocks, units, a.sink);
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_phased_kernel<BF16, M>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLdsBytes));
+    hipLaunchKernelGGL((fwd_phased_kernel<BF16, M>), dim3(xcd_grid(units)), dim3(kPhThreads), S::kLdsBytes, s, a.table, rows, row_w, a.bias, a.out,
+                       d.B, d.N, d.L, (d.K + 7) / 8, label_blocks, units, a.sink);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 
-// The phased kernel or the plain one, for slices of 128-byte rows.  Per label, in time of 1 TB/s; the rates are what the kernels
-// reach at 300,000 to 670,091 labels: plain 20 inside L2 and 5.8 over the share that misses it, in phases 18, ordering the rows
-// 3.2.  fp32, 128 samples, 65,536 columns, fan-in 72: 2.18 ms plain, 1.56 in phases; 32 samples, fan-in 32 there: 245 and 295 us;
-// bf16, 512 samples, 100,000 columns, fan-in 64: 4.1 and 2.6 ms.
-bool takes_phases(size_t slice_bytes, int gl, int slices, int K, int value_bytes) {
+int phased_labels(int L, int slices);
+
+template <bool BF16>
+int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
+    const int octs = (d.K + 7) / 8, ranges = std::min(kMaxRanges, octs);
+    unsigned* rows = nullptr;
+    FFI_TRY(workspace_get(s, kWsRows, phased_rows_bytes<BF16>(d.L, d.K), (void**)&rows));
+    void* row_w = rows + (size_t)d.L * octs * 8;
+    const size_t rbr_lds = rows_by_range_lds(d.K);
+    const auto rbr = ranges > 8 ? rows_by_range_kernel<BF16, true> : rows_by_range_kernel<BF16, false>;
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)rbr, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rbr_lds));
+    hipLaunchKernelGGL(rbr, dim3((unsigned)((d.L + 4 * kRbrRows - 1) / (4 * kRbrRows))), dim3(256), rbr_lds, s, a.idx, a.w, rows, row_w, d.L, d.K,
+                       (unsigned)(((unsigned long long)ranges << 32) / (unsigned long long)d.N), ranges);
+    FFI_HIP_TRY(hipGetLastError());
+    // (as many labels as the registers hold sums of: a slice is gone through as often as there are rounds; fewer where that
+    // leaves CUs idle)
+    return phased_labels(d.L, a.slices) == 8 ? launch_phased_walk<BF16, 8>(a, rows, row_w, d, s)
+                                                                          : launch_phased_walk<BF16, 4>(a, rows, row_w, d, s);
+}
+
+// Rounds of workgroups, one per CU and each with its XCD's share of the work, times the labels of a lane group.
+long long phased_cost(int L, int slices, int m) {
+    const long long units = ((long long)L + 8 * m * kPhWaves - 1) / (8 * m * kPhWaves) * slices;
+    const long long per_xcd = (units + kXcds - 1) / kXcds, cus = std::max(1, device_cu_count() / kXcds);
+    return (per_xcd + cus - 1) / cus * m;
+}
+// As many labels per lane group as the registers hold sums of -- a slice is gone through once a round -- or fewer where that
+// leaves CUs idle.
+int phased_labels(int L, int slices) { return phased_cost(L, slices, 8) <= phased_cost(L, slices, 4) ? 8 : 4; }
+
+// The phased kernel or the plain one, for slices of 128-byte rows.  In bytes of a gather per 1 TB/s; the rates are what the
+// kernels reach at 20,000 to 670,091 labels: plain 20 inside L2 and 5.8 over the share that misses it; in phases 21.5 for rounds
+// that fill the CUs, as far as L2 holds what the rows of a phase name -- a part of the slice and some two
+// spreads of a row's connection of that number --, ordering the rows 5, two launches.  us, plain and in phases: fp32, 128 samples,
+// 65,536 columns, 670,091 labels, fan-in 72: 2,180 and 1,300; 32 samples there 554 and 498, at fan-in 32 243 and 244; 128
+// samples, 8,000 labels, fan-in 64 38 and 56; bf16, 64 samples, 65,536 columns, 300,000 labels, fan-in 64 211 and 189; 131,072
+// columns, 500,000 labels, fan-in 16 150 and 171; 512 samples, 34,000 columns, 100,000 labels, fan-in 32 178 and 218.
+bool takes_phases(size_t slice_bytes, int gl, int slices, int L, int K, int value_bytes) {
     if (gl != 8 || K > kMaxRangedFanIn) return false;
     if (g_options.wide_phases != 0) return g_options.wide_phases > 0;
     if (K <= 8) return false;
-    const double gathered = 128.0 * slices * K, miss = std::max(0.0, 1.0 - (double)kXcdL2Bytes / (double)slice_bytes);
-    const double plain = gathered / (miss > 0.0 ? std::min(20.0, 5.8 / miss) : 20.0);
-    return gathered / 18.0 + 2.0 * K * (4 + value_bytes) / 3.2 < plain;
+    auto rate = [](double peak, double bytes) {
+        const double miss = std::max(0.0, 1.0 - (double)kXcdL2Bytes / bytes);
+        return miss > 0.0 ? std::min(peak, 5.8 / miss) : peak;
+    };
+    const double live = (double)slice_bytes * std::min(1.0, 8.0 / K + 0.9 / std::sqrt((double)K));
+    const double rounds = (double)phased_cost(L, slices, phased_labels(L, slices)) * 8 * kPhWaves * device_cu_count();     // labels
+    const double plain = 128.0 * slices * K * L / rate(20.0, (double)slice_bytes);
+    return 128.0 * K * rounds / rate(21.5, live) + 2.0 * K * (4 + value_bytes) * L / 5.0 + 8e6 < plain;
 }
 
 // How a forward pass over slices runs: lanes per row, number of slices, and whether a slice lies in LDS (then with as many
@@ -960,7 +1015,7 @@ int forward_wide(const void* table, const int32_t* idx, const void* w, const flo
             default: return launch_fwd_lds<8, BF16>(a, d, s);
         }
     }
-    if (takes_phases(slice_bytes, f.gl, f.slices, d.K, BF16 ? 2 : 4)) return launch_fwd_phased<BF16>(a, d, s);
+    if (takes_phases(slice_bytes, f.gl, f.slices, d.L, d.K, BF16 ? 2 : 4)) return launch_fwd_phased<BF16>(a, d, s);
     return launch_fwd_sliced_lanes<BF16>(f.gl, a, d, s);
 }
 
@@ -987,7 +1042,7 @@ void forward_wide_workspaces(const Dims& d, size_t* features, size_t* rows) {
     const SlicedForm f = sliced_form<false>(d.B, d.N);
     const size_t slice_bytes = (size_t)d.N * f.gl * 16;
     *features = f.in_lds ? 0 : slice_bytes * f.slices;
-    *rows = !f.in_lds && takes_phases(slice_bytes, f.gl, f.slices, d.K, 4) ? phased_rows_bytes<false>(d.L, d.K) : 0;
+    *rows = !f.in_lds && takes_phases(slice_bytes, f.gl, f.slices, d.L, d.K, 4) ? phased_rows_bytes<false>(d.L, d.K) : 0;
 }
 
 // Narrow inputs, fp32: up to 16 samples half or more of a 32-sample tile would be computed for nothing (768 x 670,091 x 32, one to

@@ -50,6 +50,38 @@ def test_forward_of_wide_inputs(ffi, phases):
         lib.ffi_set_option(b"wide_phases", 0)
 
 
+# The forward pass in phases: (B, L, K) with label blocks of 352 and (from 90,000 labels on) 704 and their edges, rows shorter
+# than an oct, of whole octs and with a remainder, up to the longest; ids spread, all of one range, all of the last column,
+# falling: a row's places come from counters of a byte each
+PHASED_SHAPES = [(32, 351, 9), (17, 353, 8), (40, 705, 64), (70, 352, 65), (33, 300, 255), (20, 101, 256), (18, 92_000, 9), (64, 91_000, 17)]
+
+
+@pytest.mark.parametrize("spread", ["uniform", "one_range", "last", "falling"])
+def test_forward_in_phases(ffi, spread):
+    N = 1301
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"wide_phases", 1) == 0
+    try:
+        for B, L, K in PHASED_SHAPES:
+            x, lookup, w, _ = reference_law_inputs(B, N, L, K, seed=B + L + K)
+            if spread == "one_range":
+                lookup = (lookup % 40 + 600).astype(np.int32)
+            elif spread == "last":
+                lookup[:] = N - 1
+            elif spread == "falling":
+                lookup = np.ascontiguousarray(-np.sort(-lookup, axis=1))
+            hx, hw = torch.from_numpy(x).bfloat16(), torch.from_numpy(w).bfloat16()
+            ref = oracle.forward(x, lookup, w, transposed=False)
+            ref16 = oracle.forward(hx.float().numpy(), lookup, hw.float().numpy(), transposed=False)
+            out = ffi.fan_in_sparse_matmul(dev(x), dev(lookup), dev(w)).cpu().numpy()
+            out16 = ffi.fan_in_sparse_matmul_bf16(hx.cuda(), dev(lookup), hw.cuda(), transposed=False).cpu().numpy()
+            # sums of K products in another order: K 2^-24 of the largest, 256 at most
+            assert rel_err(out, ref) <= 2e-5, (B, L, K)
+            assert rel_err(out16, ref16) <= 2e-5, (B, L, K)
+    finally:
+        lib.ffi_set_option(b"wide_phases", 0)
+
+
 # (B, N, L, K): lane groups of 1, 2, 4 and 8; lists that are empty, shorter and longer than a window; several label blocks,
 # streams and slices; one column
 BACKWARD_SHAPES = [(1, 1217, 900, 3), (4, 2000, 30_000, 9), (5, 1217, 129, 17), (8, 3000, 3000, 40), (9, 1300, 65, 33), (16, 2500, 5000, 64),
