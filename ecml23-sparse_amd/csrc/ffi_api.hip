@@ -130,10 +130,10 @@ void drop_cached_plan(ffi_plan* p) {
 // Input gradient through the plan cache, with `between(plan)` (the weight-gradient launch, or
 // nothing) enqueued ahead of it.  The host never waits in the steady state (the reference's op only
 // enqueues, tfsparse/cc/kernels/backward.cu:59-64): the lookup's content is checked against the cached
-// plan by a kernel that leaves its verdict on the device; the plan-driven kernels follow -- they read the
-// plan, never the lookup, so they are safe whatever the lookup holds now -- and behind them kernels that
-// recompute both gradients straight from the lookup if the verdict says the plan is outdated (a rewire),
-// and return at once otherwise.  The host looks at the verdict of an earlier call when that has arrived
+// plan by workgroups of the last plan-driven kernel, which leave their verdict on the device -- those kernels read the
+// plan, never the lookup, so they are safe whatever the lookup holds now -- and behind them comes what
+// recomputes both gradients straight from the lookup if the verdict says the plan is outdated (a rewire),
+// and returns at once otherwise.  The host looks at the verdict of an earlier call when that has arrived
 // (a poll, not a wait) and only then rebuilds the plan, which does synchronise.
 template <class Between>
 int input_grad_cached(const int32_t* lookup, const float* weights, const float* out_grad, float* feature_grad,
@@ -142,13 +142,12 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     ffi_plan* p = find_cached_plan(lookup, d, dev);
-    bool zeroed = false;
-    auto passes = [&](const unsigned long long* verdict) -> int {
+    auto passes = [&](const LookupCheck* check) -> int {
         // (the global form's walk has both operands of a connection at hand: one walk for both gradients)
         if (!p->tiled && wg.features != nullptr)
             return launch_backward_wide(p, wg.features, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d.B, d.tp, s);
         FFI_TRY(between(p));
-        return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, verdict, &zeroed);
+        return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, check);
     };
     // small layers read the lookup itself: of the plan they need that its build has found every id in range
     const bool small = takes_small_backward(d);
@@ -158,6 +157,7 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         if (wg.features == nullptr) FFI_TRY(between(p));       // (nothing, or a weight gradient formed without the plan)
         return launch_backward_small(wg.features, lookup, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d, s, bad);
     };
+    if (!small) FFI_TRY(backward_if_outdated_prepare(d, s));
     if (!p) {
         FFI_TRY(create_cached_plan(lookup, d, dev, s, &p));
         return small ? small_pass() : passes(nullptr);
@@ -179,10 +179,16 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         if (st != FFI_OK) { drop_cached_plan(p); return st; }
         return passes(nullptr);
     }
-    FFI_TRY(plan_guard_enqueue(p, lookup, s));
-    FFI_TRY(passes(p->d_guard + kGuardVerdict));
+    if (p->tiled) {
+        LookupCheck check;
+        FFI_TRY(plan_guard_begin(p, lookup, s, &check));
+        FFI_TRY(passes(&check));
+    } else {
+        FFI_TRY(plan_guard_enqueue(p, lookup, s));
+        FFI_TRY(passes(nullptr));
+    }
     return launch_backward_if_outdated(p->d_guard + kGuardVerdict, wg.features, lookup, weights, out_grad, feature_grad,
-                                       wg.weight_grad, wg.bias_grad, d, s, zeroed);
+                                       wg.weight_grad, wg.bias_grad, d, s);
 }
 
 }  // namespace
@@ -695,6 +701,8 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
     if (passes & FFI_PASS_BACKWARD) {
         // small layers walk no plan: one is built for the check of the ids
         if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
+        // what recomputes the gradients behind an outdated plan
+        else if (backward_if_outdated_workspace(d) > 0) partial_slot = backward_if_outdated_workspace(d), total += kTicketCount * sizeof(unsigned);
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;
         if ((one_window || two_windows) && d.K <= 1024 && d.L < (1 << 25)) {
             // tiled plan: the geometry of ffi_plan.hip, the slot rows of a slice estimated for column ids drawn uniformly

@@ -1,12 +1,10 @@
-// Plain kernels that recompute both gradients straight from the lookup matrix, without any preprocessed view of it.
+// Kernels that recompute both gradients straight from the lookup matrix, without any preprocessed view of it.
 // They are enqueued behind the plan-driven kernels of the stateless backward entry points and run only when the
-// device-side check of the lookup (ffi_plan.hip) found that the cached plan is outdated -- the one call after an
+// device-side check of the lookup (ffi_check.h) found that the cached plan is outdated -- the one call after an
 // in-place rewiring (sparse/custom_layer.py:32-43) -- and return at once otherwise.  Semantics:
-// tfsparse/cc/kernels/backward.cpp:8-36 (weight gradient) and :39-73 (input gradient); the input gradient scatters
-// with float atomics here, as the reference's GPU kernels do (backward.cu.h:119,139,161,182), so this one call is
-// not reproducible bit for bit.  Ids outside [0, num_features) are skipped.  Narrow inputs take the weight-gradient kernel
-// that reads the lookup itself and an input-gradient kernel that sorts each label tile's connections by column in LDS
-// (ffi_input_grad.hip; float atomics only where the workgroups add their sums to gx).
+// tfsparse/cc/kernels/backward.cpp:8-36 (weight gradient) and :39-73 (input gradient).  Ids outside [0, num_features) are
+// skipped.  Narrow inputs take one kernel for both gradients; others plain ones whose input gradient scatters with float
+// atomics, as the reference's GPU kernels do (backward.cu.h:119,139,161,182).
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 
@@ -52,24 +50,320 @@ __global__ __launch_bounds__(kFbBlock) void fallback_backward_kernel(const unsig
     }
 }
 
+// ---- narrow inputs: both gradients in one kernel -------------------------------------------------------------------
+// What is launched behind every backward pass and exits at once counts its launches: one of 256 workgroups, where a kernel per
+// gradient (and zeros by a third) took 3.8 us each.
+//
+// Weight gradient: the rows of one batch tile in LDS, a unit of (label, 32 connections) per thread, its sums in registers across
+// all batch tiles (ffi_weight_grad.hip).
+//
+// Input gradient: a workgroup takes a stream of label tiles for one batch tile and a window of the columns, a thread per column,
+// and sorts each tile's connections by column itself: counts per column (integer LDS atomics), an exclusive scan, then every
+// connection takes the next free place of its column's bucket.  Thread t then walks the bucket of column col_lo + t, gathering
+// rows of the tile's out_grad from LDS.  No slot balancing (rows lie in label order, so row parities are random and the reads
+// run at the 8-clock rate; a wavefront walks as long as its longest bucket), and the order inside a bucket is whatever the
+// atomics gave: sums are not reproducible bit for bit.  The workgroups that finish last add the streams' sums
+// up.  (670,091 labels x fan-in 32 over 768 columns, batch 128: float atomics into an LDS tile of gx -- ds_add_f32
+// retires a third of a lane per clock and CU here, integer atomics seven lanes -- took 14.3 ms.)
+// LDS: gs[tile_labels][32] | ws[tile_labels * K] | lst[tile_labels * K] | cursor[threads] | wave sums[16].
+constexpr int kRedoThreads = 1024;
+constexpr int kRedoChunk = 16;        // connections per unit of the weight gradient
+
+constexpr int kRedoTeam = 16;         // streams whose sums are added first
+__host__ __device__ constexpr int redo_teams(int streams) { return (streams + kRedoTeam - 1) / kRedoTeam; }
+
+struct RedoShape {
+    int nbt, windows, lower;              // batch tiles; windows of the columns, the first one's size
+    int tile_labels, tiles, tiles_per_stream, streams;
+    size_t lds;
+};
+struct RedoArgs {
+    const unsigned long long* verdict;
+    const float *x, *w, *g;
+    const int32_t* idx;
+    float *gx, *gw, *bias_grad;           // gx or gw may be null
+    float* partial;                       // [window][stream][batch tile][lower][32]
+    unsigned* tickets;                    // [window][batch tile][teams + 1], zero between launches
+    int B, N, L, K;
+    RedoShape s;
+};
+
+template <bool TP>
+__device__ __forceinline__ void redo_weight_grad(const RedoArgs& a, float* xs) {
+    const int lane = threadIdx.x & 63, K = a.K, nchunks = (K + kRedoChunk - 1) / kRedoChunk;
+    const long long units = (long long)a.L * nchunks;
+    for (long long u0 = (long long)blockIdx.x * kRedoThreads; u0 < units; u0 += (long long)gridDim.x * kRedoThreads) {
+        const bool mine = u0 + threadIdx.x < units;
+        const long long u = min(u0 + (long long)threadIdx.x, units - 1);
+        const int j = (int)(u / nchunks), k0 = (int)(u - (long long)j * nchunks) * kRedoChunk;
+        const int32_t* irow = a.idx + (size_t)j * K + k0;
+        // two 16-bit ids per register; row a.N - 1 in place of ids out of range, whose sums are not kept
+        unsigned ids[kRedoChunk / 2], out_of_range = 0;
+#pragma unroll
+        for (int k = 0; k < kRedoChunk; ++k) {
+            const unsigned id = k0 + k < K ? (unsigned)irow[k] : 0u, row = min(id, (unsigned)a.N - 1u);
+            ids[k / 2] = (k & 1) ? ids[k / 2] | row << 16 : row;
+            out_of_range |= (id >= (unsigned)a.N ? 1u : 0u) << k;
+        }
+        float res[kRedoChunk], gsum = 0.f;
+#pragma unroll
+        for (int k = 0; k < kRedoChunk; ++k) res[k] = 0.f;
+        for (int bt = 0; bt < a.s.nbt; ++bt) {
+            const int b0 = bt * kTileBatch;
+            __syncthreads();                                   // everyone is done with the previous tile
+            if (TP) {
+                stage_rows32<kRedoThreads>(xs, a.x, a.N, a.B, b0);
+            } else {
+                for (int e = threadIdx.x; e < a.N * kTileBatch; e += kRedoThreads) {
+                    const int b = e / a.N, n = e - b * a.N;
+                    xs[n * kTileBatch + b] = b0 + b < a.B ? a.x[(size_t)(b0 + b) * a.N + n] : 0.f;
+                }
+            }
+            __syncthreads();
+            unsigned skew = (unsigned)(size_t)(__attribute__((address_space(3))) float*)xs + (unsigned)(lane & 7) * 16u;
+            asm volatile("" : "+v"(skew));                     // keep the LDS addresses out of loop-invariant hoisting
+            float gb[32];
+            load_rows32(a.g, a.L, b0, a.B, (unsigned)j, gb);
+            if (a.bias_grad != nullptr) {
+#pragma unroll
+                for (int b = 0; b < 32; ++b) gsum += gb[b];
+            }
+            xor_permute_groups(gb, lane & 7);                  // match the skewed chunk order of the gathers
+#pragma unroll
+            for (int k = 0; k < kRedoChunk; ++k) {
+                // (four of the row's reads at a time: the registers hold no more)
+                const unsigned base = (((k & 1) ? ids[k / 2] >> 16 : ids[k / 2] & 0xffffu) << 7) + skew;
+                float sum = res[k];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 v[4] = {h ? row_chunk<4>(base) : row_chunk<0>(base), h ? row_chunk<5>(base) : row_chunk<1>(base),
+                                         h ? row_chunk<6>(base) : row_chunk<2>(base), h ? row_chunk<7>(base) : row_chunk<3>(base)};
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const float* gc = gb + 16 * h + 4 * c;
+                        sum = fmaf(v[c].w, gc[3], fmaf(v[c].z, gc[2], fmaf(v[c].y, gc[1], fmaf(v[c].x, gc[0], sum))));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                res[k] = sum;
+            }
+        }
+        if (mine) {
+            float* grow = a.gw + (size_t)j * K + k0;
+            if (a.bias_grad != nullptr && k0 == 0) a.bias_grad[j] = gsum;
+#pragma unroll
+            for (int k = 0; k < kRedoChunk; ++k)
+                if (k0 + k < K) grow[k] = (out_of_range >> k & 1u) ? 0.f : res[k];
+        }
+    }
+}
+
+template <bool TP>
+__device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, float* gs) {
+    const int K = a.K, L = a.L, tile_labels = a.s.tile_labels;
+    const int bt = item % a.s.nbt, stream = item / a.s.nbt % a.s.streams, window = item / (a.s.nbt * a.s.streams);
+    const int b0 = bt * kTileBatch, col_lo = window == 0 ? 0 : a.s.lower, ncols = window == 0 ? a.s.lower : a.N - a.s.lower;
+    float* ws = gs + (size_t)tile_labels * kTileBatch;
+    unsigned* lst = reinterpret_cast<unsigned*>(ws + (size_t)tile_labels * K);
+    int* cursor = reinterpret_cast<int*>(lst + (size_t)tile_labels * K);
+    int* wave_sum = cursor + kRedoThreads;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const unsigned skewbase = (unsigned)(size_t)(__attribute__((address_space(3))) float*)gs + (unsigned)(lane & 7) * 16u;
+    char* gs_bytes = reinterpret_cast<char*>(gs);
+    const int t_begin = stream * a.s.tiles_per_stream, t_end = min(t_begin + a.s.tiles_per_stream, a.s.tiles);
+    float acc[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+    for (int t = t_begin; t < t_end; ++t) {
+        const int j0 = t * tile_labels;
+        const int nl = min(tile_labels, L - j0);
+        const int total = nl * K;
+        const int32_t* src = a.idx + (size_t)j0 * K;
+        __syncthreads();                                   // the previous tile is no longer being read
+        cursor[threadIdx.x] = 0;
+        for (int jl = threadIdx.x; jl < nl; jl += kRedoThreads) {
+            float gb[32];
+            load_rows32(a.g, L, b0, a.B, (unsigned)(j0 + jl), gb);
+            const int r = jl & 7;
+            xor_permute_groups(gb, r);
+            char* rowp = gs_bytes + ((size_t)jl << 7);
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                *reinterpret_cast<float4*>(rowp + ((c ^ r) << 4)) = make_float4(gb[4 * c], gb[4 * c + 1], gb[4 * c + 2], gb[4 * c + 3]);
+        }
+        for (int q = threadIdx.x; q < total; q += kRedoThreads) ws[q] = a.w[(size_t)j0 * K + q];
+        __syncthreads();
+        for (int e = threadIdx.x; e < total; e += kRedoThreads) {
+            const unsigned c = (unsigned)(src[e] - col_lo);             // (ids outside [0, N) or outside the window: skipped)
+            if (c < (unsigned)ncols) atomicAdd(&cursor[c], 1);
+        }
+        __syncthreads();
+        // exclusive scan of the counts over the workgroup
+        const int mine = cursor[threadIdx.x];
+        int incl = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int v = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += v;
+        }
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        int before = 0;
+        for (int q = 0; q < wave; ++q) before += wave_sum[q];
+        const int begin = before + incl - mine;
+        cursor[threadIdx.x] = begin;
+        __syncthreads();
+        {
+            // (label of entry e without a division per entry: the thread's entries are kRedoThreads apart)
+            int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
+            const int dl = kRedoThreads / K, dk = kRedoThreads - dl * K;
+            for (int e = threadIdx.x; e < total; e += kRedoThreads) {
+                const unsigned c = (unsigned)(src[e] - col_lo);
+                if (c < (unsigned)ncols) lst[atomicAdd(&cursor[c], 1)] = ((unsigned)e << 10) | (unsigned)l;
+                l += dl; k += dk;
+                if (k >= K) { k -= K; ++l; }
+            }
+        }
+        __syncthreads();
+        const int len = cursor[threadIdx.x] - begin;
+        int longest = len;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off, 64));
+        for (int i = 0; i < longest; ++i) {
+            if (i < len) {
+                const unsigned entry = lst[begin + i];
+                const float wv = ws[entry >> 10];
+                float4 xv[8];
+                read_row(((entry & 1023u) << 7) + skewbase, xv);
+                row_fmas(xv, wv, acc);
+            }
+        }
+    }
+    xor_permute_groups(acc, lane & 7);
+    // The sums of kRedoTeam consecutive streams are added by the workgroup of theirs that finishes last, the teams' sums by the
+    // last of those.  (All streams' by one workgroup: 1.4 ms for 256.)
+    auto sums_of = [&](int st) { return a.partial + (((size_t)window * a.s.streams + st) * a.s.nbt + bt) * ((size_t)a.s.lower * kTileBatch); };
+    float* out = sums_of(stream) + threadIdx.x * kTileBatch;
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+        if ((int)threadIdx.x < ncols) *reinterpret_cast<float4*>(out + 4 * c) = make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]);
+    const int teams = redo_teams(a.s.streams), team = stream / kRedoTeam, lead = team * kRedoTeam;
+    unsigned* const tickets = a.tickets + (size_t)(window * a.s.nbt + bt) * (teams + 1);
+    auto last_of = [&](unsigned* ticket, int count) {
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) wave_sum[0] = atomicAdd(ticket, 1u) == (unsigned)count - 1u;
+        __syncthreads();
+        const bool last = wave_sum[0] != 0;
+        if (last) {
+            __threadfence();
+            if (threadIdx.x == 0) *ticket = 0u;
+        }
+        return last;
+    };
+    auto sum = [&](int q, int count, int step) {               // of quad q over `count` streams from `lead` or the first on
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        const int from = step == 1 ? lead : 0;
+#pragma unroll 8
+        for (int i = 0; i < count; ++i) {
+            const float4 p = reinterpret_cast<const float4*>(sums_of(from + i * step))[q];
+            v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+        }
+        return v;
+    };
+    const int quads = ncols * (kTileBatch / 4), in_team = min(kRedoTeam, a.s.streams - lead);
+    if (!last_of(tickets + team, in_team)) return;
+    for (int q = threadIdx.x; q < quads; q += kRedoThreads) reinterpret_cast<float4*>(sums_of(lead))[q] = sum(q, in_team, 1);
+    if (!last_of(tickets + teams, teams)) return;
+    for (int q = threadIdx.x; q < quads; q += kRedoThreads) {
+        const float4 v = sum(q, teams, kRedoTeam);
+        const int n = q / (kTileBatch / 4), b = b0 + q % (kTileBatch / 4) * 4;
+        const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (b + i < a.B) a.gx[TP ? (size_t)(col_lo + n) * a.B + b + i : (size_t)(b + i) * a.N + col_lo + n] = e[i];
+    }
+}
+
+template <bool TP>
+__global__ __launch_bounds__(kRedoThreads) void redo_backward_kernel(const RedoArgs a) {
+    if (*a.verdict != 0) return;
+    extern __shared__ __align__(16) float redo_mem[];
+    if (a.gw != nullptr) redo_weight_grad<TP>(a, redo_mem);
+    if (a.gx == nullptr) return;
+    const int items = a.s.nbt * a.s.streams * a.s.windows;
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        __syncthreads();
+        redo_input_grad<TP>(a, item, redo_mem);
+    }
+}
+
+size_t redo_lds_bytes(int tile_labels, int K) {
+    return (size_t)tile_labels * (kTileBatch * sizeof(float) + 8u * (size_t)K) + (size_t)kRedoThreads * 4u + 64u;
+}
+
+// Whether the kernel above takes the shape -- inputs that fit the LDS tile, fan-ins whose tile of one label fits beside it -- and how.
+bool redo_shape(const Dims& d, RedoShape* s) {
+    s->nbt = (d.B + kTileBatch - 1) / kTileBatch;
+    s->windows = d.N > kRedoThreads ? 2 : 1;
+    s->lower = s->windows == 1 ? d.N : ((d.N + 1) / 2 + 63) / 64 * 64;
+    if (!tile_path_fits(d.N) || d.N > 2 * kRedoThreads || d.L >= (1 << 25) || redo_lds_bytes(1, d.K) > kPlanLdsBudget)
+        return false;
+    // as many labels per tile as the LDS holds (entries keep the label in 10 bits), then evened out so that every
+    // workgroup of a batch tile gets the same number of tiles
+    const size_t per_label = kTileBatch * sizeof(float) + 8u * (size_t)d.K;
+    int tl = (int)std::min<size_t>(1023, (kPlanLdsBudget - redo_lds_bytes(0, d.K)) / per_label);
+    const int streams0 = std::max(1, device_cu_count() / std::max(1, s->nbt));
+    const int tiles0 = (d.L + tl - 1) / tl;
+    s->tiles_per_stream = (tiles0 + streams0 - 1) / streams0;
+    if (tiles0 > streams0) tl = std::min(tl, (int)(((long long)d.L + (long long)s->tiles_per_stream * streams0 - 1) / ((long long)s->tiles_per_stream * streams0)));
+    s->tile_labels = tl;
+    s->tiles = (d.L + tl - 1) / tl;
+    s->streams = (s->tiles + s->tiles_per_stream - 1) / s->tiles_per_stream;
+    s->lds = std::max(redo_lds_bytes(tl, d.K), tile_lds_bytes(d.N));
+    return (long long)s->nbt * s->windows * (redo_teams(s->streams) + 1) <= kTicketCount;
+}
+
 }  // namespace
+
+size_t backward_if_outdated_workspace(const Dims& d) {
+    RedoShape s;
+    return redo_shape(d, &s) ? (size_t)s.windows * s.streams * s.nbt * s.lower * kTileBatch * sizeof(float) : 0;
+}
+
+int backward_if_outdated_prepare(const Dims& d, hipStream_t s) {
+    void* ws = nullptr;
+    const size_t bytes = backward_if_outdated_workspace(d);
+    if (bytes == 0) return FFI_OK;
+    FFI_TRY(workspace_get(s, kWsPartials, bytes, &ws));
+    return tickets_get(s, &ws);
+}
 
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,
                                 const float* weights, const float* out_grad, float* feature_grad, float* weight_grad,
-                                float* bias_grad, const Dims& d, hipStream_t s, bool feature_grad_is_zeroed) {
+                                float* bias_grad, const Dims& d, hipStream_t s) {
     const int cus = device_cu_count();
-    if (feature_grad != nullptr && !feature_grad_is_zeroed) {
-        hipLaunchKernelGGL(fallback_zero_kernel, dim3(cus), dim3(kFbBlock), 0, s, verdict, feature_grad, (size_t)d.B * d.N);
-        FFI_HIP_TRY(hipGetLastError());
-    }
     float* gw = features != nullptr ? weight_grad : nullptr;
     float* gb = features != nullptr ? bias_grad : nullptr;
-    if (tile_path_fits(d.N) && d.L < (1 << 25) && input_grad_unplanned_fits(d.N, d.K)) {
-        // narrow inputs: the weight gradient by the kernel that needs no plan (it returns at once unless the verdict says
-        // "outdated"), the input gradient by the kernel that sorts each label tile's connections by column in LDS
-        if (gw != nullptr) FFI_TRY(launch_weight_grad(features, lookup, out_grad, gw, gb, d, s, nullptr, verdict));
-        if (feature_grad != nullptr) FFI_TRY(launch_input_grad_unplanned(verdict, lookup, weights, out_grad, feature_grad, d, s));
+    RedoArgs a{};
+    if (redo_shape(d, &a.s)) {
+        a.verdict = verdict;
+        a.x = features; a.w = weights; a.g = out_grad; a.idx = lookup;
+        a.gx = feature_grad; a.gw = gw; a.bias_grad = gb;
+        a.B = d.B; a.N = d.N; a.L = d.L; a.K = d.K;
+        FFI_TRY(workspace_get(s, kWsPartials, backward_if_outdated_workspace(d), (void**)&a.partial));
+        FFI_TRY(tickets_get(s, (void**)&a.tickets));
+        const auto kernel = d.tp ? redo_backward_kernel<true> : redo_backward_kernel<false>;
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)a.s.lds));
+        const int items = std::min(a.s.nbt * a.s.streams * a.s.windows, 4 * cus);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)std::max(cus, items)), dim3(kRedoThreads), a.s.lds, s, a);
+        FFI_HIP_TRY(hipGetLastError());
         return FFI_OK;
+    }
+    if (feature_grad != nullptr) {
+        hipLaunchKernelGGL(fallback_zero_kernel, dim3(cus), dim3(kFbBlock), 0, s, verdict, feature_grad, (size_t)d.B * d.N);
+        FFI_HIP_TRY(hipGetLastError());
     }
     if (d.tp)
         hipLaunchKernelGGL(fallback_backward_kernel<true>, dim3(cus * 2), dim3(kFbBlock), 0, s, verdict, features, lookup, weights,

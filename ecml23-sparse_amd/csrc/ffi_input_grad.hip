@@ -9,6 +9,7 @@
 // across all the tiles of the workgroup's label stream.  Streams are then summed in a fixed order.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
+#include "ffi_check.h"
 
 #include <algorithm>
 
@@ -83,40 +84,6 @@ __global__ __launch_bounds__(1024) void igrad_permute_weights_kernel(
             if (resume == 0xffffffffu && __any(any_later)) resume = i;
         }
         lo = (resume == 0xffffffffu) ? rows : resume;
-    }
-}
-
-// The eight 16-byte reads of one row (chunk order skewed by the lane id) ...
-// `skewbase` = LDS address of the tile + (lane & 7) * 16; the tile is 128-byte aligned, so the chunk
-// bits can be flipped with XOR after the row offset has been added (one add + seven XORs per row).
-typedef float lds_v4f __attribute__((ext_vector_type(4)));
-typedef const lds_v4f __attribute__((address_space(3)))* lds_v4f_ptr;
-template <int C>
-__device__ __forceinline__ float4 igrad_read_chunk(unsigned base) {
-    const lds_v4f t = *(lds_v4f_ptr)(size_t)(skew_addr<C>(base));
-    return make_float4(t.x, t.y, t.z, t.w);
-}
-__device__ __forceinline__ void igrad_reads_at(unsigned base, float4 (&v)[8]) {
-    v[0] = igrad_read_chunk<0>(base); v[1] = igrad_read_chunk<1>(base);
-    v[2] = igrad_read_chunk<2>(base); v[3] = igrad_read_chunk<3>(base);
-    v[4] = igrad_read_chunk<4>(base); v[5] = igrad_read_chunk<5>(base);
-    v[6] = igrad_read_chunk<6>(base); v[7] = igrad_read_chunk<7>(base);
-}
-__device__ __forceinline__ void igrad_reads(unsigned e, unsigned skewbase, float4 (&v)[8]) {
-    const unsigned base = (e << 7) + skewbase;
-    v[0] = igrad_read_chunk<0>(base); v[1] = igrad_read_chunk<1>(base);
-    v[2] = igrad_read_chunk<2>(base); v[3] = igrad_read_chunk<3>(base);
-    v[4] = igrad_read_chunk<4>(base); v[5] = igrad_read_chunk<5>(base);
-    v[6] = igrad_read_chunk<6>(base); v[7] = igrad_read_chunk<7>(base);
-}
-// ... and the 32 multiply-adds that consume them.
-__device__ __forceinline__ void igrad_fmas(const float4 (&v)[8], float wv, float (&acc)[32]) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        acc[4 * c + 0] = fmaf(wv, v[c].x, acc[4 * c + 0]);
-        acc[4 * c + 1] = fmaf(wv, v[c].y, acc[4 * c + 1]);
-        acc[4 * c + 2] = fmaf(wv, v[c].z, acc[4 * c + 2]);
-        acc[4 * c + 3] = fmaf(wv, v[c].w, acc[4 * c + 3]);
     }
 }
 
@@ -334,11 +301,11 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
                     // (the tile starts at LDS address 0 -- the kernel has no other LDS -- so the row's byte offset and the
                     // lane's skew, which share no bit, combine with an OR: one instruction with the mask)
                     const float wv = *(const float __attribute__((address_space(3)))*)(size_t)(wsbase + (e4[q] >> 17) * 4u);
-                    igrad_reads_at((e4[q] & 0x1ff80u) | skewbase, xv);
-                    igrad_fmas(xv, wv, acc);
+                    read_row((e4[q] & 0x1ff80u) | skewbase, xv);
+                    row_fmas(xv, wv, acc);
                 } else {
-                    igrad_reads(in ? e4[q] : (unsigned)zero_row, skewbase, xv);
-                    igrad_fmas(xv, in ? w4[q] : 0.f, acc);
+                    read_row(((in ? e4[q] : (unsigned)zero_row) << 7) + skewbase, xv);
+                    row_fmas(xv, in ? w4[q] : 0.f, acc);
                 }
             }
 #pragma unroll
@@ -359,81 +326,55 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
         *reinterpret_cast<float4*>(out + 4 * c) = make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]);
 }
 
-// gx = sum over streams, ascending: a fixed order, so results are reproducible.
+// gx = sum over the streams in a fixed order, so results are reproducible: `groups` threads per sum add consecutive streams in
+// ascending order, eight loads in flight each, then the groups' sums are added in ascending order.  A workgroup has `width`
+// samples of `cols` columns.
+// The first check.blocks workgroups check the lookup's content against the plan instead (ffi_check.h).
+//
+// Bound by the chain of loads, a round trip to the Infinity Cache each, and by the ids that the check reads: 768 columns x 32
+// samples x 256 streams by one thread per sum 10.5 us, by eight 6.4.  As kernels one behind the other the check took 9.9 us of
+// that layer's backward pass (131,072 labels x 32) beside 6.7 for the sums, together they take 10.9.
+constexpr int kReduceThreads = kCheckThreads;
 template <bool TP>
-__global__ __launch_bounds__(256) void igrad_reduce_kernel(const float* __restrict__ partial, float* __restrict__ gx,
-                                                           int B, int N, int streams, int nthreads, int bpad,
-                                                           const unsigned long long* __restrict__ verdict, int col_lo) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    const int n = blockIdx.y;                          // column inside the plan's window; gx column n + col_lo
-    if (b >= B) return;
-    gx += TP ? (size_t)col_lo * B : (size_t)col_lo;
-    // the plan is known to be outdated: zeros, for the kernel that recomputes the gradient from the lookup to add to
-    if (verdict != nullptr && *verdict == 0) {
-        if (TP) gx[(size_t)n * B + b] = 0.f; else gx[(size_t)b * N + n] = 0.f;
-        return;
-    }
-    float v = 0.f;
-    const size_t step = (size_t)nthreads * bpad;
-    const float* p = partial + (size_t)n * bpad + b;
-    int r = 0;
-    for (; r + 8 <= streams; r += 8) {                 // eight loads in flight, added in ascending order
-        float t[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) t[q] = p[(size_t)(r + q) * step];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v += t[q];
-    }
-    for (; r < streams; ++r) v += p[(size_t)r * step];
-    if (TP) gx[(size_t)n * B + b] = v; else gx[(size_t)b * N + n] = v;
-}
-
-// The same where the streams are many and the samples few: every group of `width` threads adds consecutive streams in ascending
-// order, then the groups' sums are added in ascending order.  Bound by the chain of loads (eight in flight, a round trip to the
-// Infinity Cache each): 768 columns x 32 samples x 256 streams by one thread per sum 10.5 us, by eight 6.4.
-constexpr int kReduceThreads = 1024;
-template <bool TP>
-__global__ __launch_bounds__(kReduceThreads) void igrad_reduce_split_kernel(const float* __restrict__ partial, float* __restrict__ gx,
+__global__ __launch_bounds__(kReduceThreads) void igrad_reduce_kernel(const float* __restrict__ partial, float* __restrict__ gx,
                                                                       int B, int N, int streams, int nthreads, int bpad,
-                                                                      const unsigned long long* __restrict__ verdict, int col_lo, int width) {
-    __shared__ float sums[kReduceThreads];
-    const int group = threadIdx.x / width, groups = blockDim.x / width;
-    const int b = blockIdx.x * width + (threadIdx.x - group * width);
-    const int n = blockIdx.y;                          // column inside the plan's window; gx column n + col_lo
-    gx += TP ? (size_t)col_lo * B : (size_t)col_lo;
-    float* const dst = gx + (TP ? (size_t)n * B + b : (size_t)b * N + n);
-    const bool mine = group == 0 && b < B;
-    // the plan is known to be outdated: zeros, for the kernel that recomputes the gradient from the lookup to add to
-    if (verdict != nullptr && *verdict == 0) {
-        if (mine) *dst = 0.f;
+                                                                      int col_lo, int ncols, int width, int groups, int cols, int col_blocks,
+                                                                      const LookupCheck check) {
+    __shared__ union { float sums[kReduceThreads]; CheckShared check; } shared;
+    if ((int)blockIdx.x < check.blocks) {
+        check_block(check, blockIdx.x, shared.check);
         return;
     }
+    const int block = blockIdx.x - check.blocks;
+    const int per_col = width * groups, c = threadIdx.x / per_col, t = threadIdx.x - c * per_col, group = t / width;
+    const int n = block % col_blocks * cols + c;       // column inside the plan's window; gx column n + col_lo
+    const int b = block / col_blocks * width + (t - group * width);
+    const bool on = c < cols && n < ncols && b < B;
     const int per = (streams + groups - 1) / groups, end = min((group + 1) * per, streams);
     float v = 0.f;
-    if (b < B) {
+    if (on) {
         const size_t step = (size_t)nthreads * bpad;
         const float* p = partial + (size_t)n * bpad + b;
         int r = group * per;
-        for (; r + 8 <= end; r += 8) {                 // eight loads in flight, added in ascending order
-            float t[8];
+        for (; r + 8 <= end; r += 8) {
+            float q[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) t[q] = p[(size_t)(r + q) * step];
+            for (int i = 0; i < 8; ++i) q[i] = p[(size_t)(r + i) * step];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) v += t[q];
+            for (int i = 0; i < 8; ++i) v += q[i];
         }
         for (; r < end; ++r) v += p[(size_t)r * step];
     }
     if (groups > 1) {
-        sums[threadIdx.x] = v;
+        shared.sums[threadIdx.x] = v;
         __syncthreads();
-        if (mine)
-            for (int i = 1; i < groups; ++i) v += sums[threadIdx.x + i * width];
+        if (on && group == 0)
+            for (int i = 1; i < groups; ++i) v += shared.sums[threadIdx.x + i * width];
     }
-    if (mine) *dst = v;
+    if (on && group == 0) gx[TP ? (size_t)(col_lo + n) * B + b : (size_t)b * N + col_lo + n] = v;
 }
 
-int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp, hipStream_t s,
-                 const unsigned long long* verdict) {
+int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp, hipStream_t s, const LookupCheck* check) {
     const int nbt = (B + kTileBatch - 1) / kTileBatch;
     const int cus = device_cu_count();
     const int per_cu = tiled_workgroups_per_cu(p->threads, p->tile_labels, p->K, p->w_in_lds, nbt);
@@ -487,192 +428,33 @@ int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, i
     }
 #undef FFI_LAUNCH_TILE
     // (64 streams of 128 samples: 6.2 us by one thread per sum, 6.9 by two)
-    const bool split = streams >= 128 && B <= 128;
-    const int width = B <= 32 ? 32 : B <= 64 ? 64 : 128, groups = std::min(8, streams / 32);
-    const dim3 rgrid(split ? 1 : (B + 255) / 256, p->col_n ? p->col_n : p->N);
-    if (split && tp)
-        hipLaunchKernelGGL(igrad_reduce_split_kernel<true>, rgrid, dim3(width * groups), 0, s, partial, gx, B, p->N, streams, p->threads, bpad, verdict, p->col_lo, width);
-    else if (split)
-        hipLaunchKernelGGL(igrad_reduce_split_kernel<false>, rgrid, dim3(width * groups), 0, s, partial, gx, B, p->N, streams, p->threads, bpad, verdict, p->col_lo, width);
-    else if (tp)
-        hipLaunchKernelGGL(igrad_reduce_kernel<true>, rgrid, dim3(256), 0, s, partial, gx, B, p->N, streams, p->threads, bpad, verdict, p->col_lo);
-    else
-        hipLaunchKernelGGL(igrad_reduce_kernel<false>, rgrid, dim3(256), 0, s, partial, gx, B, p->N, streams, p->threads, bpad, verdict, p->col_lo);
+    const int width = B <= 32 ? 32 : B <= 64 ? 64 : B <= 128 ? 128 : 256, groups = streams >= 128 && B <= 128 ? std::min(8, streams / 32) : 1;
+    const int ncols = p->col_n ? p->col_n : p->N, btiles = (B + width - 1) / width;
+    // (a workgroup per CU where a workgroup's threads allow; 768 columns x 128 samples by 96 full workgroups 9.4 us, by 256 7.5)
+    const int cols = std::min(kReduceThreads / (width * groups), std::max(1, (ncols * btiles + cus - 1) / cus)), col_blocks = (ncols + cols - 1) / cols;
+    const LookupCheck with = check != nullptr ? *check : LookupCheck{};
+    const dim3 rgrid((unsigned)(col_blocks * btiles + with.blocks));
+    const auto reduce = tp ? igrad_reduce_kernel<true> : igrad_reduce_kernel<false>;
+    hipLaunchKernelGGL(reduce, rgrid, dim3(kReduceThreads), 0, s, partial, gx, B, p->N, streams, p->threads, bpad, p->col_lo, ncols, width, groups,
+                       cols, col_blocks, with);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 
-// ---- without a plan --------------------------------------------------------------------------------
-// The input gradient straight from the lookup, for the one call after the lookup was edited behind the library's back:
-// the kernel runs only if *verdict == 0 ("the cached plan is outdated") and returns at once otherwise.  A workgroup takes a
-// stream of label tiles for one batch tile, as igrad_tile_kernel does, and sorts each tile's connections by column itself:
-// counts per column (integer LDS atomics), an exclusive scan, then every connection takes the next free place of its
-// column's bucket.  Thread t then walks the bucket of column col_lo + t, gathering rows of the tile's out_grad from LDS.
-// No slot balancing (rows lie in label order, so row parities are random and the reads run at the 8-clock rate; a
-// wavefront walks as long as its longest bucket), and the order inside a bucket is whatever the atomics gave: sums are
-// not reproducible bit for bit.  Measured at 670,091 labels x fan-in 32 over 768 columns, batch 128, against float
-// atomics into an LDS tile of gx (ds_add_f32 retires a third of a lane per clock and CU here, integer atomics seven
-// lanes): 14.3 ms before.  gx must be zero; the workgroups add their sums with one global atomic per (column, sample).
-// LDS: gs[tile_labels][32] | ws[tile_labels * K] | lst[tile_labels * K] | cursor[threads] | wave sums[16].
-template <bool TP>
-__global__ __launch_bounds__(1024) void igrad_unplanned_kernel(const unsigned long long* __restrict__ verdict,
-                                                               const int32_t* __restrict__ idx, const float* __restrict__ w,
-                                                               const float* __restrict__ g, float* __restrict__ gx, int B, int N,
-                                                               int L, int K, int tile_labels, int tiles, int tiles_per_stream,
-                                                               int nbt, int col_lo, int ncols) {
-    if (*verdict != 0) return;
-    extern __shared__ __align__(16) float gs[];
-    const int nthreads = blockDim.x;
-    float* ws = gs + (size_t)tile_labels * kTileBatch;
-    unsigned* lst = reinterpret_cast<unsigned*>(ws + (size_t)tile_labels * K);
-    int* cursor = reinterpret_cast<int*>(lst + (size_t)tile_labels * K);
-    int* wave_sum = cursor + nthreads;
-    const int bt = blockIdx.x % nbt, stream = blockIdx.x / nbt;
-    const int b0 = bt * kTileBatch;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const unsigned skewbase = (unsigned)(size_t)(__attribute__((address_space(3))) float*)gs + (unsigned)(lane & 7) * 16u;
-    char* gs_bytes = reinterpret_cast<char*>(gs);
-    const int t_begin = stream * tiles_per_stream, t_end = min(t_begin + tiles_per_stream, tiles);
-    float acc[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] = 0.f;
-    for (int t = t_begin; t < t_end; ++t) {
-        const int j0 = t * tile_labels;
-        const int nl = min(tile_labels, L - j0);
-        const int total = nl * K;
-        const int32_t* src = idx + (size_t)j0 * K;
-        __syncthreads();                                   // the previous tile is no longer being read
-        cursor[threadIdx.x] = 0;
-        for (int jl = threadIdx.x; jl < nl; jl += nthreads) {
-            float gb[32];
-            load_rows32(g, L, b0, B, (unsigned)(j0 + jl), gb);
-            const int r = jl & 7;
-            xor_permute_groups(gb, r);
-            char* rowp = gs_bytes + ((size_t)jl << 7);
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                *reinterpret_cast<float4*>(rowp + ((c ^ r) << 4)) = make_float4(gb[4 * c], gb[4 * c + 1], gb[4 * c + 2], gb[4 * c + 3]);
-        }
-        for (int q = threadIdx.x; q < total; q += nthreads) ws[q] = w[(size_t)j0 * K + q];
-        __syncthreads();
-        for (int e = threadIdx.x; e < total; e += nthreads) {
-            const unsigned c = (unsigned)(src[e] - col_lo);             // (ids outside [0, N) or outside the window: skipped)
-            if (c < (unsigned)ncols) atomicAdd(&cursor[c], 1);
-        }
-        __syncthreads();
-        // exclusive scan of the counts over the workgroup
-        const int mine = cursor[threadIdx.x];
-        int incl = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int v = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += v;
-        }
-        if (lane == 63) wave_sum[wave] = incl;
-        __syncthreads();
-        int before = 0;
-        for (int q = 0; q < wave; ++q) before += wave_sum[q];
-        const int begin = before + incl - mine;
-        cursor[threadIdx.x] = begin;
-        __syncthreads();
-        {
-            // (label of entry e without a division per entry: the thread's entries are nthreads apart)
-            int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
-            const int dl = nthreads / K, dk = nthreads - dl * K;
-            for (int e = threadIdx.x; e < total; e += nthreads) {
-                const unsigned c = (unsigned)(src[e] - col_lo);
-                if (c < (unsigned)ncols) lst[atomicAdd(&cursor[c], 1)] = ((unsigned)e << 10) | (unsigned)l;
-                l += dl; k += dk;
-                if (k >= K) { k -= K; ++l; }
-            }
-        }
-        __syncthreads();
-        const int len = cursor[threadIdx.x] - begin;
-        int longest = len;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off, 64));
-        for (int i = 0; i < longest; ++i) {
-            if (i < len) {
-                const unsigned entry = lst[begin + i];
-                const float wv = ws[entry >> 10];
-                float4 xv[8];
-                igrad_reads(entry & 1023u, skewbase, xv);
-                igrad_fmas(xv, wv, acc);
-            }
-        }
-    }
-    xor_permute_groups(acc, lane & 7);
-    if ((int)threadIdx.x < ncols) {
-        const int n = col_lo + (int)threadIdx.x;
-#pragma unroll
-        for (int c = 0; c < 32; ++c)
-            if (b0 + c < B) atomicAdd(&gx[TP ? (size_t)n * B + (b0 + c) : (size_t)(b0 + c) * N + n], acc[c]);
-    }
-}
-
 }  // namespace
 
-// LDS of igrad_unplanned_kernel for tiles of `tile_labels` labels
-static size_t unplanned_lds_bytes(int tile_labels, int K, int threads) {
-    return (size_t)tile_labels * (kTileBatch * sizeof(float) + 8u * (size_t)K) + (size_t)threads * 4u + 64u;
-}
-
-bool input_grad_unplanned_fits(int N, int K) {
-    const int threads = std::min(1024, (N + 63) / 64 * 64);
-    return tile_path_fits(N) && N <= 2048 && unplanned_lds_bytes(1, K, threads) <= (size_t)kPlanLdsBudget;
-}
-
-int launch_input_grad_unplanned(const unsigned long long* verdict, const int32_t* idx, const float* w, const float* g, float* gx,
-                                const Dims& d, hipStream_t s) {
-    if (!input_grad_unplanned_fits(d.N, d.K)) return FFI_ERR_BAD_ARGUMENT;
-    const int nbt = (d.B + kTileBatch - 1) / kTileBatch;
-    const int cus = device_cu_count();
-    // inputs of more than 1,024 columns: one launch per half of the columns (a thread per column)
-    const int windows = d.N > 1024 ? 2 : 1;
-    const int lower = windows == 1 ? d.N : ((d.N + 1) / 2 + 63) / 64 * 64;
-    for (int win = 0; win < windows; ++win) {
-        const int col_lo = win == 0 ? 0 : lower, ncols = win == 0 ? lower : d.N - lower;
-        const int threads = (ncols + 63) / 64 * 64;
-        // as many labels per tile as the LDS holds (entries keep the label in 10 bits), then evened out so that every
-        // workgroup of a batch tile gets the same number of tiles
-        const size_t per_label = kTileBatch * sizeof(float) + 8u * (size_t)d.K;
-        int tl = (int)std::min<size_t>(1023, ((size_t)kPlanLdsBudget - (size_t)threads * 4u - 64u) / per_label);
-        const int streams0 = std::max(1, cus / std::max(1, nbt));
-        const int tiles0 = (d.L + tl - 1) / tl;
-        const int tps = (tiles0 + streams0 - 1) / streams0;
-        if (tiles0 > streams0) tl = std::min(tl, (int)(((long long)d.L + (long long)tps * streams0 - 1) / ((long long)tps * streams0)));
-        const int tiles = (d.L + tl - 1) / tl;
-        const int streams = (tiles + tps - 1) / tps;
-        const size_t lds = unplanned_lds_bytes(tl, d.K, threads);
-        const dim3 grid((unsigned)(streams * nbt)), block((unsigned)threads);
-        if (d.tp) {
-            FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_unplanned_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(igrad_unplanned_kernel<true>, grid, block, lds, s, verdict, idx, w, g, gx, d.B, d.N, d.L, d.K, tl, tiles, tps, nbt,
-                               col_lo, ncols);
-        } else {
-            FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_unplanned_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(igrad_unplanned_kernel<false>, grid, block, lds, s, verdict, idx, w, g, gx, d.B, d.N, d.L, d.K, tl, tiles, tps, nbt,
-                               col_lo, ncols);
-        }
-        FFI_HIP_TRY(hipGetLastError());
-    }
-    return FFI_OK;
-}
-
 int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp,
-                      hipStream_t s, const unsigned long long* verdict, bool* zeroed_if_outdated) {
-    if (zeroed_if_outdated) *zeroed_if_outdated = false;
+                      hipStream_t s, const LookupCheck* check) {
     // (a plan whose last build failed holds no arrays)
     if (p->lookup == nullptr) return FFI_ERR_BAD_ARGUMENT;
     if (p->tiled) {
         if (!p->slice_off || !p->rowpos || (p->w_in_lds ? !p->slot32 : (!p->lab16 || !p->pos16))) return FFI_ERR_BAD_ARGUMENT;
-        if (zeroed_if_outdated) *zeroed_if_outdated = verdict != nullptr;
-        FFI_TRY(launch_tiled(p, w, g, gx, B, tp, s, verdict));
+        FFI_TRY(launch_tiled(p, w, g, gx, B, tp, s, p->upper != nullptr ? nullptr : check));
         // inputs wider than one workgroup has threads: the second half of the columns has a tiled form of its own
         if (p->upper != nullptr) {
             const ffi_plan* u = p->upper;
             if (!u->tiled || !u->slice_off || !u->rowpos || (u->w_in_lds ? !u->slot32 : (!u->lab16 || !u->pos16))) return FFI_ERR_BAD_ARGUMENT;
-            return launch_tiled(u, w, g, gx, B, tp, s, verdict);
+            return launch_tiled(u, w, g, gx, B, tp, s, check);
         }
         return FFI_OK;
     }

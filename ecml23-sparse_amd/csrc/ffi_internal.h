@@ -95,9 +95,8 @@ int launch_transpose(const float* src, float* dst, int rows, int cols, hipStream
 int launch_forward(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                    hipStream_t s);
 // `plan` (may be null): a plan of the same lookup whose arranged copy of the column ids the kernel may use
-// `only_if_outdated` (may be null; without a plan only): device word of a lookup check -- the kernel returns at once unless it is 0
 int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
-                       hipStream_t s, const ffi_plan* plan = nullptr, const unsigned long long* only_if_outdated = nullptr);
+                       hipStream_t s, const ffi_plan* plan = nullptr);
 // any shape (the tile kernels cover narrow inputs only)
 int launch_forward_wide(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                         hipStream_t s);
@@ -397,26 +396,35 @@ void plan_reuse(ffi_plan* p, int L, int K, int N);
 // Enqueues a check of `lookup` against the plan's fingerprint on `s`: the verdict lands in p->d_guard[kGuardVerdict]
 // (device) for the kernels enqueued behind it, and in the pinned mirror for a later call of the host.
 constexpr int kGuardVerdict = 4;
+constexpr int kCheckThreads = 1024;
+constexpr int kCheckBlocks = 256;                  // workgroups of a check (at most)
+constexpr int kCheckWords = 8 + 2 * kCheckBlocks;
+struct LookupCheck {                               // (ffi_check.h)
+    const int32_t* idx;
+    size_t total;
+    unsigned num_features;
+    int blocks;
+    unsigned long long *guard, *host_mirror, seq;
+};
 int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s);
+// The same without the launch: for a kernel on `s` that has check.blocks workgroups of kCheckThreads threads run it.
+int plan_guard_begin(ffi_plan* p, const int32_t* lookup, hipStream_t s, LookupCheck* check);
 // What the last finished check found, if the host has not seen it yet: *seen = false when no check has finished
 // since the last poll.  Never waits.
 int plan_guard_poll(ffi_plan* p, bool* seen, bool* current, unsigned long long* bad_ids);
-// Both gradients recomputed straight from `lookup` by plain kernels that run only if *verdict == 0 (and return at
+// Both gradients recomputed straight from `lookup` by kernels that run only if *verdict == 0 (and return at
 // once otherwise): enqueued behind plan-driven kernels, they overwrite what an outdated plan produced.  features /
-// weight_grad / bias_grad may be null (no weight gradient wanted), feature_grad may be null.
+// weight_grad / bias_grad may be null (no weight gradient wanted), feature_grad may be null.  What they need on the stream is
+// allocated by backward_if_outdated_prepare, ahead of the first kernel of the call.
+size_t backward_if_outdated_workspace(const Dims& d);
+int backward_if_outdated_prepare(const Dims& d, hipStream_t s);
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,
                                 const float* weights, const float* out_grad, float* feature_grad, float* weight_grad,
-                                float* bias_grad, const Dims& d, hipStream_t s, bool feature_grad_is_zeroed);
+                                float* bias_grad, const Dims& d, hipStream_t s);
 void plan_free(ffi_plan* p);
-// `verdict` (may be null): device word of a lookup check enqueued ahead; where the kernels can, they leave zeros in gx
-// when it says the plan is outdated (*zeroed_if_outdated tells whether they could)
+// `check` (may be null; tiled form only): run by the last kernel, beside its own work
 int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp,
-                      hipStream_t s, const unsigned long long* verdict = nullptr, bool* zeroed_if_outdated = nullptr);
-// The input gradient straight from the lookup (no plan), added into a zeroed gx by a kernel that runs only if *verdict == 0;
-// for inputs that fit the LDS tile and fan-ins whose tile of one label fits beside it (input_grad_unplanned_fits).
-bool input_grad_unplanned_fits(int N, int K);
-int launch_input_grad_unplanned(const unsigned long long* verdict, const int32_t* idx, const float* w, const float* g, float* gx,
-                                const Dims& d, hipStream_t s);
+                      hipStream_t s, const LookupCheck* check = nullptr);
 // Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.
 void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, int* streams, int* blocks_per_stream);
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,

@@ -132,6 +132,45 @@ __device__ __forceinline__ unsigned xor_permute_bits(unsigned m, int r) {
 template <int C>
 __device__ __forceinline__ unsigned skew_addr(unsigned base) { return C == 0 ? base : (base ^ (unsigned)(C * 16)); }
 
+// The eight 16-byte reads of one row, all issued before the first use ...
+// `base` = LDS address of the row + (lane & 7) * 16 (rows are 128-byte aligned, so the chunk bits can
+// be flipped with XOR).
+typedef float lds_v4f __attribute__((ext_vector_type(4)));
+typedef const lds_v4f __attribute__((address_space(3)))* lds_v4f_ptr;
+template <int C>
+__device__ __forceinline__ float4 row_chunk(unsigned base) {
+    const lds_v4f t = *(lds_v4f_ptr)(size_t)(skew_addr<C>(base));
+    return make_float4(t.x, t.y, t.z, t.w);
+}
+__device__ __forceinline__ void read_row(unsigned base, float4 (&v)[8]) {
+    v[0] = row_chunk<0>(base); v[1] = row_chunk<1>(base);
+    v[2] = row_chunk<2>(base); v[3] = row_chunk<3>(base);
+    v[4] = row_chunk<4>(base); v[5] = row_chunk<5>(base);
+    v[6] = row_chunk<6>(base); v[7] = row_chunk<7>(base);
+}
+// ... and their dot product with the (equally skewed) out_grad values.
+__device__ __forceinline__ float row_dot(const float4 (&v)[8], const float (&gb)[32], float acc) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        acc = fmaf(v[c].x, gb[4 * c + 0], acc);
+        acc = fmaf(v[c].y, gb[4 * c + 1], acc);
+        acc = fmaf(v[c].z, gb[4 * c + 2], acc);
+        acc = fmaf(v[c].w, gb[4 * c + 3], acc);
+    }
+    return acc;
+}
+
+// ... or the 32 multiply-adds of the row by one weight.
+__device__ __forceinline__ void row_fmas(const float4 (&v)[8], float wv, float (&acc)[32]) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        acc[4 * c + 0] = fmaf(wv, v[c].x, acc[4 * c + 0]);
+        acc[4 * c + 1] = fmaf(wv, v[c].y, acc[4 * c + 1]);
+        acc[4 * c + 2] = fmaf(wv, v[c].z, acc[4 * c + 2]);
+        acc[4 * c + 3] = fmaf(wv, v[c].w, acc[4 * c + 3]);
+    }
+}
+
 #endif  // __HIPCC__
 
 }  // namespace ffi

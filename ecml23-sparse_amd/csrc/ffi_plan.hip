@@ -4,6 +4,7 @@
 // lookup[j,k] == n.  The plan lists those connections column by column so that they can be walked
 // sequentially, without atomics, in an order that never changes from run to run.
 #include "ffi_internal.h"
+#include "ffi_check.h"
 #include "ffi_scan.h"
 #include "ffi_lds_tile.h"
 
@@ -21,13 +22,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kFingerprintBlocks = 1024;                 // workgroups of the fingerprint kernel (at most)
 constexpr int kScratchWords = 8 + 2 * kFingerprintBlocks;  // plan scratch: 8 words for the build, then fingerprint partial sums
-
-__device__ __forceinline__ unsigned mix32(unsigned v) {
-    v ^= v >> 16; v *= 0x7feb352du;
-    v ^= v >> 15; v *= 0x846ca68bu;
-    v ^= v >> 16;
-    return v;
-}
 
 // Order-independent 64-bit content fingerprint: sum over positions p of mix(id_p + p * odd), plus
 // the number of ids outside [0,N).  Every workgroup writes its own pair of partial sums (no atomics:
@@ -76,97 +70,9 @@ __global__ __launch_bounds__(kBlock) void fingerprint_kernel(const int32_t* __re
     }
 }
 
-// The same fingerprint, checked on the device.  Workgroups leave their pairs of sums in guard[8 + 2 * block ..]
-// (plain stores) and take a ticket from guard[2], the only atomic: a few hundred adds to one address, not
-// thousands (those serialise and were measured to triple the kernel's time).  The workgroup that draws the last
-// ticket adds the pairs up (integer adds: the total does not depend on the order), compares with guard[3], leaves
-// the verdict in guard[4] (1 = content unchanged and every id in range), the sums in guard[5] / guard[6], and
-// clears the ticket counter for the next check.
-constexpr int kGuardBlock = 1024;
-constexpr int kGuardBlocks = 256;                         // workgroups of the guard kernel (at most)
-constexpr int kGuardWords = 8 + 2 * kGuardBlocks;
-__global__ __launch_bounds__(kGuardBlock) void fingerprint_guard_kernel(const int32_t* __restrict__ idx, size_t total, unsigned N,
-                                                                         unsigned long long* __restrict__ guard,
-                                                                         unsigned long long* __restrict__ host_mirror,
-                                                                         unsigned long long seq) {
-    unsigned long long h = 0;
-    unsigned bad = 0;
-    const size_t stride = (size_t)gridDim.x * kGuardBlock;
-    const size_t tid = (size_t)blockIdx.x * kGuardBlock + threadIdx.x;
-    const bool vec = ((uintptr_t)idx & 15) == 0;
-    const size_t nvec = vec ? total / 4 : 0;
-    const int4* idx4 = reinterpret_cast<const int4*>(idx);
-#pragma unroll 4
-    for (size_t q = tid; q < nvec; q += stride) {
-        const int4 v = idx4[q];
-        const unsigned p = (unsigned)(q * 4);
-        h += mix32((unsigned)v.x + p * 0x9e3779b1u);
-        h += mix32((unsigned)v.y + (p + 1) * 0x9e3779b1u);
-        h += mix32((unsigned)v.z + (p + 2) * 0x9e3779b1u);
-        h += mix32((unsigned)v.w + (p + 3) * 0x9e3779b1u);
-        bad += ((unsigned)v.x >= N) + ((unsigned)v.y >= N) + ((unsigned)v.z >= N) + ((unsigned)v.w >= N);
-    }
-    for (size_t p = nvec * 4 + tid; p < total; p += stride) {
-        const unsigned id = (unsigned)idx[p];
-        h += mix32(id + (unsigned)p * 0x9e3779b1u);
-        bad += id >= N;
-    }
-    unsigned long long b64 = bad;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        h += __shfl_down(h, off);
-        b64 += __shfl_down(b64, off);
-    }
-    __shared__ unsigned long long part[2][kGuardBlock / 64];
-    __shared__ bool last;
-    if ((threadIdx.x & 63) == 0) { part[0][threadIdx.x >> 6] = h; part[1][threadIdx.x >> 6] = b64; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long hs = 0, bs = 0;
-#pragma unroll
-        for (int i = 0; i < kGuardBlock / 64; ++i) { hs += part[0][i]; bs += part[1][i]; }
-        // Published with atomic exchanges whose results are waited for, then the ticket: a read-modify-write at
-        // device scope is carried out where all XCDs see it, and its returned value says that it has been.  (A
-        // fence here would first write back every dirty line of this XCD's L2 -- the scores the forward kernel has
-        // just stored among them -- which was measured to cost a third of the kernel's time.)
-        const unsigned long long o1 = __hip_atomic_exchange(&guard[8 + 2 * blockIdx.x], hs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long o2 = __hip_atomic_exchange(&guard[9 + 2 * blockIdx.x], bs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned long long one = 1ull;
-        asm volatile("" : "+v"(one) : "v"(o1), "v"(o2));       // the ticket is not drawn before both exchanges have returned
-        last = __hip_atomic_fetch_add(&guard[2], one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned long long)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    // the last workgroup adds the pairs of all workgroups: one load per thread, all in flight together (a loop of
-    // dependent loads per lane costs a memory round trip per step)
-    static_assert(kGuardBlocks <= kGuardBlock, "one thread per pair");
-    unsigned long long hs = 0, bs = 0;
-    if (threadIdx.x < gridDim.x) {
-        hs = __hip_atomic_fetch_add(&guard[8 + 2 * threadIdx.x], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bs = __hip_atomic_fetch_add(&guard[9 + 2 * threadIdx.x], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        hs += __shfl_down(hs, off);
-        bs += __shfl_down(bs, off);
-    }
-    __syncthreads();                                       // (thread 0 has read part[] above)
-    if ((threadIdx.x & 63) == 0) { part[0][threadIdx.x >> 6] = hs; part[1][threadIdx.x >> 6] = bs; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        hs = 0; bs = 0;
-#pragma unroll
-        for (int i = 0; i < kGuardBlock / 64; ++i) { hs += part[0][i]; bs += part[1][i]; }
-        const unsigned long long verdict = (hs == guard[3] && bs == 0) ? 1ull : 0ull;
-        guard[5] = hs;
-        guard[6] = bs;
-        guard[4] = verdict;
-        guard[2] = 0;
-        // For the host, one word in pinned host memory: (number of this check << 2) | (verdict << 1) | (bad ids seen).
-        // The host polls that word; neither a copy command nor an event is enqueued behind the kernel (an event
-        // record between two kernels was measured to open a 6-us gap in front of the second).
-        __hip_atomic_store(host_mirror, (seq << 2) | (verdict << 1) | (bs != 0 ? 1ull : 0ull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+__global__ __launch_bounds__(kCheckThreads) void fingerprint_guard_kernel(const LookupCheck check) {
+    __shared__ CheckShared shared;
+    check_block(check, blockIdx.x, shared);
 }
 
 // ---- tiled form ---------------------------------------------------------------------------------
@@ -1300,9 +1206,9 @@ int plan_scratch_alloc(ffi_plan* p) {
                     hipHostMalloc(&p->h_scratch, kScratchWords * sizeof(unsigned long long)) == hipSuccess &&
                     hipEventCreateWithFlags(&p->fp_done, hipEventDisableTiming) == hipSuccess &&
                     hipMemset(p->d_scratch, 0, kScratchWords * sizeof(unsigned long long)) == hipSuccess &&
-                    hipMalloc(&p->d_guard, kGuardWords * sizeof(unsigned long long)) == hipSuccess &&
+                    hipMalloc(&p->d_guard, kCheckWords * sizeof(unsigned long long)) == hipSuccess &&
                     hipHostMalloc(&p->h_guard, 8 * sizeof(unsigned long long)) == hipSuccess &&
-                    hipMemset(p->d_guard, 0, kGuardWords * sizeof(unsigned long long)) == hipSuccess;
+                    hipMemset(p->d_guard, 0, kCheckWords * sizeof(unsigned long long)) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
         return FFI_ERR_OUT_OF_MEMORY;
@@ -1473,7 +1379,7 @@ int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigne
 }
 }  // namespace
 
-int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
+int plan_guard_begin(ffi_plan* p, const int32_t* lookup, hipStream_t s, LookupCheck* check) {
     // A check of this plan that may still be running on another stream shares the accumulators: the two must not
     // overlap.  The other stream's handle may be gone by now (its owner may have destroyed it), so it is not touched:
     // the host waits for the device.  Only a lookup used from two streams in turn pays this, once per switch.
@@ -1485,14 +1391,20 @@ int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
         if (seen && !current) p->guard_stale = true;
     }
     const size_t total = (size_t)p->L * p->K;
-    const unsigned blocks = (unsigned)std::min<size_t>((total / 4 + kGuardBlock - 1) / kGuardBlock + 1, kGuardBlocks);
     unsigned long long* mirror = nullptr;
     FFI_HIP_TRY(hipHostGetDevicePointer((void**)&mirror, p->h_guard, 0));
-    hipLaunchKernelGGL(fingerprint_guard_kernel, dim3(blocks), dim3(kGuardBlock), 0, s, lookup, total, (unsigned)p->N, p->d_guard, mirror,
-                       p->guard_seq + 1);
-    FFI_HIP_TRY(hipGetLastError());
+    *check = LookupCheck{lookup, total, (unsigned)p->N, (int)std::min<size_t>((total / 4 + kCheckThreads - 1) / kCheckThreads + 1, kCheckBlocks),
+                         p->d_guard, mirror, p->guard_seq + 1};
     p->guard_seq += 1;
     p->guard_stream = s;
+    return FFI_OK;
+}
+
+int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
+    LookupCheck check;
+    FFI_TRY(plan_guard_begin(p, lookup, s, &check));
+    hipLaunchKernelGGL(fingerprint_guard_kernel, dim3((unsigned)check.blocks), dim3(kCheckThreads), 0, s, check);
+    FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 

@@ -29,34 +29,6 @@ constexpr int kWgChunk = 32;        // connections per unit
 constexpr int kResThreads = 512;
 constexpr int kResUnits = 4;        // units per thread
 
-// The eight 16-byte reads of one row, all issued before the first use ...
-// `base` = LDS address of the row + (lane & 7) * 16 (rows are 128-byte aligned, so the chunk bits can
-// be flipped with XOR).
-typedef float lds_v4f __attribute__((ext_vector_type(4)));
-typedef const lds_v4f __attribute__((address_space(3)))* lds_v4f_ptr;
-template <int C>
-__device__ __forceinline__ float4 wgrad_read_chunk(unsigned base) {
-    const lds_v4f t = *(lds_v4f_ptr)(size_t)(skew_addr<C>(base));
-    return make_float4(t.x, t.y, t.z, t.w);
-}
-__device__ __forceinline__ void wgrad_reads(unsigned base, float4 (&v)[8]) {
-    v[0] = wgrad_read_chunk<0>(base); v[1] = wgrad_read_chunk<1>(base);
-    v[2] = wgrad_read_chunk<2>(base); v[3] = wgrad_read_chunk<3>(base);
-    v[4] = wgrad_read_chunk<4>(base); v[5] = wgrad_read_chunk<5>(base);
-    v[6] = wgrad_read_chunk<6>(base); v[7] = wgrad_read_chunk<7>(base);
-}
-// ... and their dot product with the (equally skewed) out_grad values.
-__device__ __forceinline__ float wgrad_dot(const float4 (&v)[8], const float (&gb)[32], float acc) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        acc = fmaf(v[c].x, gb[4 * c + 0], acc);
-        acc = fmaf(v[c].y, gb[4 * c + 1], acc);
-        acc = fmaf(v[c].z, gb[4 * c + 2], acc);
-        acc = fmaf(v[c].w, gb[4 * c + 3], acc);
-    }
-    return acc;
-}
-
 template <bool VEC4>
 __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float* __restrict__ xT,
                                                                      const int32_t* __restrict__ idx,
@@ -64,8 +36,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
                                                                      float* __restrict__ gw,
                                                                      float* __restrict__ bias_grad, int B, int N,
                                                                      int L, int K, int nchunks, int n1, int upb1,
-                                                                     int upb2, const unsigned long long* __restrict__ only_if_outdated) {
-    if (only_if_outdated != nullptr && *only_if_outdated != 0) return;     // (enqueued as a fallback: the plan was current)
+                                                                     int upb2) {
     extern __shared__ __align__(16) float xs[];
     const int lane = threadIdx.x & 63;
     const int blk = blockIdx.x;
@@ -130,9 +101,9 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
                 for (int k = 0; k < kWgChunk; ++k) {
                     const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
                     float4 xv[8];
-                    wgrad_reads((id << 7) + skew, xv);
+                    read_row((id << 7) + skew, xv);
                     __builtin_amdgcn_sched_barrier(0);
-                    res[q][k] = wgrad_dot(xv, gb, res[q][k]);
+                    res[q][k] = row_dot(xv, gb, res[q][k]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -240,9 +211,9 @@ __global__ __launch_bounds__(kResThreads) void wgrad_arranged_kernel(const float
                     for (int k = 0; k < kWgChunk; ++k) {
                         const unsigned e = (k & 1) ? (idp[k >> 1] >> 16) : idp[k >> 1];
                         float4 xv[8];
-                        wgrad_reads(((e & kArrIdMask) << 7) + skew, xv);
+                        read_row(((e & kArrIdMask) << 7) + skew, xv);
                         __builtin_amdgcn_sched_barrier(0);
-                        res[qq * NCH + c][k] = wgrad_dot(xv, gb, res[qq * NCH + c][k]);
+                        res[qq * NCH + c][k] = row_dot(xv, gb, res[qq * NCH + c][k]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -491,9 +462,9 @@ __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* 
                         if constexpr (k % kStep == kAt && k / kStep < kQuarters)
                             fetch_ids_quarter(c + 1 < NCH ? item[qq] : itn, c + 1 < NCH ? c + 1 : 0, k / kStep, idn);
                         float4 xv[8];
-                        wgrad_reads(((e & kArrIdMask) << 7) + skew, xv);
+                        read_row(((e & kArrIdMask) << 7) + skew, xv);
                         __builtin_amdgcn_sched_barrier(0);
-                        res[qq * NCH + c][k] = wgrad_dot(xv, gb, res[qq * NCH + c][k]);
+                        res[qq * NCH + c][k] = row_dot(xv, gb, res[qq * NCH + c][k]);
                         __builtin_amdgcn_sched_barrier(0);
                     });
                     asm volatile("" ::: "memory");
@@ -602,8 +573,8 @@ bool three_units_cheaper(long long units, int N, int cus) {
 }
 
 int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
-                       hipStream_t s, const ffi_plan* plan, const unsigned long long* only_if_outdated) {
-    if (only_if_outdated == nullptr && takes_small_backward(d)) return launch_backward_small(x, idx, nullptr, g, nullptr, gw, bias_grad, d, s, nullptr);
+                       hipStream_t s, const ffi_plan* plan) {
+    if (takes_small_backward(d)) return launch_backward_small(x, idx, nullptr, g, nullptr, gw, bias_grad, d, s, nullptr);
     // (32 rows of out_grad must be reachable through 32-bit byte offsets)
     if (tile_path_fits(d.N) && d.L < (1 << 25)) {
         const float* xT = x;
@@ -696,10 +667,10 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
         const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx) % 16 == 0);
         if (vec4) {
             FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<true>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, only_if_outdated);
+            hipLaunchKernelGGL(wgrad_resident_kernel<true>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2);
         } else {
             FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<false>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, only_if_outdated);
+            hipLaunchKernelGGL(wgrad_resident_kernel<false>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2);
         }
         FFI_HIP_TRY(hipGetLastError());
         return FFI_OK;

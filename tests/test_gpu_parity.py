@@ -564,6 +564,31 @@ def test_in_place_rewiring_is_picked_up(ffi, shape):
     assert np.array_equal(rebuilt, run())               # plan-driven again: bit-identical from call to call
 
 
+# What recomputes both gradients behind an outdated plan: one and several teams of label streams (16 each) and a team of one,
+# two windows of columns, a batch tile of one sample, fan-ins off the 16 connections of a unit, fewer units than threads and
+# several rounds of them
+@pytest.mark.parametrize("shape", [(33, 1200, 9001, 17), (7, 40, 30_000, 300), (1, 1216, 20_011, 33), (130, 64, 17_000, 15), (64, 768, 140_000, 32)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_both_gradients_behind_an_outdated_plan(ffi, shape, transposed):
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B + K)
+    xin = np.ascontiguousarray(x.T) if transposed else x
+    dx, dl, dw, dg = dev(xin), dev(lookup), dev(w), dev(g)
+    bwd = ffi.fan_in_sparse_matmul_grad_tp if transposed else ffi.fan_in_sparse_matmul_grad
+    bwd(dx, dl, dw, dg)
+    rng = np.random.default_rng(8)
+    outs = []
+    for _ in range(2):                                  # two edits, both served before the host has seen a verdict
+        lookup = lookup.copy()
+        lookup[rng.integers(0, L, 400), rng.integers(0, K, 400)] = rng.integers(0, N, 400)
+        dl.copy_(dev(lookup))
+        outs.append((lookup, *bwd(dx, dl, dw, dg)))
+    for edited, gx, gw in outs:
+        ref_gx, ref_gw = oracle.backward(xin, edited, w, g, transposed=transposed)
+        assert rel_err(gx.cpu().numpy(), ref_gx) <= GRAD_RTOL
+        assert rel_err(gw.cpu().numpy(), ref_gw) <= GRAD_RTOL
+
+
 def _label_sample_errors(lookup, w, g, x, gx, gw, B, N, K, labels):
     """weight gradient of a label sample and the full input gradient against the oracle ([N,B] features)"""
     o_gw = oracle.weight_grad(x, lookup[labels], w[labels], np.ascontiguousarray(g[:, labels]), transposed=True)
