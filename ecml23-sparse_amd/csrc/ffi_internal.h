@@ -193,6 +193,10 @@ struct TopkRowSource {
     int N = 0, L = 0, K = 0;
     bool tp = false, bf16 = false;
 };
+// few samples with their features in LDS: scores and the k best of them in one launch
+bool takes_topk_direct(const Dims& d);
+int launch_topk_direct(const void* x, const int32_t* idx, const void* w, const float* bias, bool bf16, const TopkArgs& tk, const Dims& d,
+                       hipStream_t s);
 // the k best candidates of every sample; a sample whose count exceeds the cap is answered from its whole row (src)
 int launch_topk_select(const TopkCandidates& c, int B, const TopkArgs& tk, const TopkRowSource& src, hipStream_t s);
 

@@ -1105,6 +1105,7 @@ int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const 
 
 int launch_forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, bool bf16, const TopkArgs& tk, const Dims& d,
                                hipStream_t s) {
+    if (takes_topk_direct(d)) return launch_topk_direct(x, idx, w, bias, bf16, tk, d, s);
     return bf16 ? forward_topk_sliced<true>(x, idx, w, bias, tk, d, s) : forward_topk_sliced<false>(x, idx, w, bias, tk, d, s);
 }
 

@@ -14,6 +14,7 @@
 #include "ffi_loss.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ffi {
 namespace {
@@ -325,6 +326,260 @@ __global__ __launch_bounds__(256) void topk_select_kernel(float* cand_val, int* 
     }
 }
 
+// ---- few samples: scores and answer in one pass --------------------------------------------------------------------
+// For up to four samples whose features fit in LDS (all of them, BP floats a column).  A group of `lanes` neighbouring lanes has a
+// label, a lane four connections of it: 16 bytes of ids and of weights in whole lines, the features of a connection by one read of
+// LDS, the products summed over the group by DPP.  Every lane keeps the best eight of the labels that fall to it, a workgroup the best
+// of its lanes'; the workgroup that ends last takes the best of those.
+//
+// What bounds it: the stream of ids and weights.  One sample, 768 columns, 670,091 labels, fan-in 32: 36.9 us, 4.7 TB/s;
+// a sample of the labels, a threshold, all scores and a selection took four launches and 67 us; four samples, k = 8, 60 against 71.
+// (From eight samples on the sums over the lanes cost more than the launches.)
+constexpr int kDirectThreads = 1024;
+constexpr int direct_rounds(int bp) { return bp == 1 ? 4 : 2; }      // rounds of labels whose loads are in flight together
+constexpr size_t kDirectLds = 144 * 1024;       // for the features
+constexpr int kDirectHeld = 4;                  // labels per lane, at most
+
+// The labels that fell to a lane.
+struct FewLabels {
+    float v[kDirectHeld];
+    int id[kDirectHeld];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int s = 0; s < kDirectHeld; ++s) { v[s] = -__builtin_inff(); id[s] = kNoId; }
+    }
+};
+
+// The k best of a workgroup's labels, in m.out_v and m.out_id (-inf and kNoId behind the last), for every thread to read.  The k-th best of the wavefronts' best bounds the answer from below; the few labels that reach it are listed, and
+// each counts those that are better.  (By rounds that take the best of all that is left, 10 us a sample and workgroup; where
+// more labels than the list holds reach the bound, that is what happens.)  k <= 16 wavefronts.
+constexpr int kFewCap = 512;
+struct FewShared {
+    float best_v[kDirectThreads / 64], v[kFewCap], out_v[kTopMax];
+    int best_id[kDirectThreads / 64], id[kFewCap], out_id[kTopMax];
+    int count;
+};
+__device__ __forceinline__ void few_topk(const FewLabels& l, int k, FewShared& m) {
+    constexpr int kWaves = kDirectThreads / 64;
+    static_assert(kTopMax <= kWaves, "a bound from the wavefronts' best");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float bv = l.v[0];
+    int bi = l.id[0];
+#pragma unroll
+    for (int s = 1; s < kDirectHeld; ++s)
+        if (better(l.v[s], l.id[s], bv, bi)) { bv = l.v[s]; bi = l.id[s]; }
+    const float wv = wave_largest(bv);
+    const int wi = wave_smallest(bv == wv ? bi : kNoId);
+    if (lane == 0) { m.best_v[wave] = wv; m.best_id[wave] = wi; }
+    if (threadIdx.x == 0) m.count = 0;
+    if (threadIdx.x < kTopMax) { m.out_v[threadIdx.x] = -__builtin_inff(); m.out_id[threadIdx.x] = kNoId; }
+    __syncthreads();
+    // (equal entries -- wavefronts without a label -- in the order of the wavefronts)
+    const float mv = m.best_v[lane % kWaves];
+    const int mi = m.best_id[lane % kWaves];
+    int rank = 0;
+#pragma unroll
+    for (int s = 0; s < kWaves; ++s) {
+        const float ov = m.best_v[s];
+        const int oi = m.best_id[s];
+        rank += better(ov, oi, mv, mi) || (ov == mv && oi == mi && s < lane % kWaves);
+    }
+    const int at = __ffsll((unsigned long long)__ballot(rank == k - 1)) - 1;
+    const float tv = m.best_v[at];
+    const int ti = m.best_id[at];
+#pragma unroll
+    for (int s = 0; s < kDirectHeld; ++s) {
+        if (l.id[s] != kNoId && !better(tv, ti, l.v[s], l.id[s])) {
+            const int to = atomicAdd(&m.count, 1);
+            if (to < kFewCap) { m.v[to] = l.v[s]; m.id[to] = l.id[s]; }
+        }
+    }
+    __syncthreads();
+    const int n = m.count;
+    if (n <= kFewCap) {
+        if ((int)threadIdx.x < n) {
+            const float v = m.v[threadIdx.x];
+            const int id = m.id[threadIdx.x];
+            int r = 0;
+            for (int s = 0; s < n; ++s) r += better(m.v[s], m.id[s], v, id);
+            if (r < k) { m.out_v[r] = v; m.out_id[r] = id; }
+        }
+    } else {
+        TopList all;
+        all.clear();
+#pragma unroll
+        for (int s = 0; s < kDirectHeld; ++s)
+            if (l.id[s] != kNoId) all.offer(l.v[s], l.id[s]);
+        float ov;
+        int oi;
+        block_topk<kWaves>(all, k, ov, oi);
+        if ((int)threadIdx.x < k) { m.out_v[threadIdx.x] = ov; m.out_id[threadIdx.x] = oi; }
+    }
+    __syncthreads();
+}
+
+// the four connections of a label that begin at k0, at any alignment of their type
+template <typename T> struct Four { T v[4]; };
+
+template <bool BF16, int BP>
+__global__ __launch_bounds__(kDirectThreads) void topk_direct_kernel(const void* __restrict__ features, const int32_t* __restrict__ idx,
+                                                                     const void* __restrict__ weights, const float* __restrict__ bias, int B, int N,
+                                                                     int L, int K, int tp, int lanes, int passes, int k, unsigned long long* part,
+                                                                     unsigned* ticket, float* __restrict__ values,
+                                                                     int32_t* __restrict__ indices) {
+    using T = std::conditional_t<BF16, unsigned short, float>;
+    const T* const x = static_cast<const T*>(features);
+    const T* const w = static_cast<const T*>(weights);
+    constexpr int kDirectRounds = direct_rounds(BP);
+    extern __shared__ __align__(16) float direct_xs[];            // [N][BP]
+    for (int e = threadIdx.x; e < N * B; e += kDirectThreads) {
+        const int n = tp ? e / B : e % N, b = tp ? e % B : e / N;
+        direct_xs[n * BP + b] = as_float(x[e]);
+    }
+    if (B < BP)
+        for (int e = threadIdx.x; e < N * (BP - B); e += kDirectThreads) direct_xs[e / (BP - B) * BP + B + e % (BP - B)] = 0.f;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, sub = lane & (lanes - 1), per_round = 64 / lanes;
+    const int wave = blockIdx.x * (kDirectThreads / 64) + (threadIdx.x >> 6), waves = gridDim.x * (kDirectThreads / 64);
+    const int step = waves * per_round * kDirectRounds;
+    FewLabels list[BP];
+#pragma unroll
+    for (int b = 0; b < BP; ++b) list[b].clear();
+    auto label_of = [&](int j0, int u) { return j0 + u * per_round + lane / lanes; };
+    Four<int> id[kDirectRounds];
+    Four<T> wt[kDirectRounds];
+    auto fetch = [&](int j0, int pass) {
+        const int k0 = min((pass * lanes + sub) * 4, K - 4);      // (the last quad of a row ends with it)
+#pragma unroll
+        for (int u = 0; u < kDirectRounds; ++u) {
+            const size_t at = (size_t)min(label_of(j0, u), L - 1) * K + k0;
+            id[u] = *reinterpret_cast<const Four<int>*>(idx + at);
+            wt[u] = *reinterpret_cast<const Four<T>*>(w + at);
+        }
+    };
+    int j0 = wave * per_round * kDirectRounds, held = 0, place = 0, mine = kNoId;
+    float score[BP];
+    // (NaN is no score: it takes no place)
+    auto keep = [&]() {
+        const float bj = bias != nullptr && mine != kNoId ? bias[mine] : 0.f;
+#pragma unroll
+        for (int b = 0; b < BP; ++b) {
+            const float v = bias != nullptr ? score[b] + bj : score[b];
+            const bool on = mine != kNoId && v == v;
+#pragma unroll
+            for (int t = 0; t < kDirectHeld; ++t)
+                if (place == t) { list[b].v[t] = on ? v : -__builtin_inff(); list[b].id[t] = on ? mine : kNoId; }
+        }
+        ++place;
+        held = 0;
+        mine = kNoId;
+    };
+    if (j0 < L) fetch(j0, 0);
+    for (; j0 < L; j0 += step) {
+        float acc[kDirectRounds][BP];
+#pragma unroll
+        for (int u = 0; u < kDirectRounds; ++u)
+#pragma unroll
+            for (int b = 0; b < BP; ++b) acc[u][b] = 0.f;
+        for (int pass = 0; pass < passes; ++pass) {
+            const int first = (pass * lanes + sub) * 4;
+            Four<int> at[kDirectRounds];
+            Four<T> wv[kDirectRounds];
+#pragma unroll
+            for (int u = 0; u < kDirectRounds; ++u) { at[u] = id[u]; wv[u] = wt[u]; }
+            if (pass + 1 < passes) fetch(j0, pass + 1);
+            else fetch(min(j0 + step, L - 1), 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool on = min(first, K - 4) + e >= first;   // (what a pulled-back quad shares with the one before it, and quads behind the row)
+#pragma unroll
+                for (int u = 0; u < kDirectRounds; ++u) {
+                    const float* row = direct_xs + (size_t)(unsigned)at[u].v[e] * BP;
+                    const float we = on ? as_float(wv[u].v[e]) : 0.f;
+                    float xv[BP];
+                    if constexpr (BP == 4) { const float4 t = *reinterpret_cast<const float4*>(row); xv[0] = t.x; xv[1] = t.y; xv[2] = t.z; xv[3] = t.w; }
+                    else if constexpr (BP == 2) { const float2 t = *reinterpret_cast<const float2*>(row); xv[0] = t.x; xv[1] = t.y; }
+                    else xv[0] = row[0];
+#pragma unroll
+                    for (int b = 0; b < BP; ++b) acc[u][b] = fmaf(we, on ? xv[b] : 0.f, acc[u][b]);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kDirectRounds; ++u) {
+            const int j = label_of(j0, u);
+#pragma unroll
+            for (int b = 0; b < BP; ++b) {
+                float v = acc[u][b];
+                if (lanes > 1) v += dpp_of<0xb1>(v);
+                if (lanes > 2) v += dpp_of<0x4e>(v);
+                if (lanes > 4) v += dpp_of<0x141>(v);
+                if (lanes > 8) v += dpp_of<0x140>(v);
+                if (lanes > 16) v += __shfl_xor(v, 16);
+                if (lanes > 32) v += __shfl_xor(v, 32);
+                if (held == sub) score[b] = v;
+            }
+            if (held == sub && j < L) mine = j;
+            if (++held == lanes) keep();                          // every lane of the group has a label
+        }
+    }
+    if (held > 0) keep();
+    // A workgroup's answers are published by exchanges whose results are waited for, then its ticket is drawn: read-modify-writes at
+    // device scope, carried out where all XCDs see them.  (A fence by all wavefronts: 94 us for the kernel, not 44.)
+    __shared__ FewShared shared;
+    unsigned long long seen = 0;
+#pragma unroll
+    for (int b = 0; b < BP; ++b) {
+        if (b >= B) break;
+        few_topk(list[b], k, shared);
+        if ((int)threadIdx.x < k)
+            seen += __hip_atomic_exchange(&part[((size_t)b * gridDim.x + blockIdx.x) * kTopMax + threadIdx.x],
+                                          (unsigned long long)(unsigned)shared.out_id[threadIdx.x] << 32 | __float_as_uint(shared.out_v[threadIdx.x]),
+                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __shared__ bool last;
+    if (threadIdx.x < 64) {
+        unsigned one = 1u;
+        asm volatile("" : "+v"(one) : "v"(seen));             // (of all the wavefront's lanes: they wait together)
+        if (threadIdx.x == 0) last = __hip_atomic_fetch_add(ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    const int entries = (int)gridDim.x * k;
+    for (int b = 0; b < B; ++b) {
+        FewLabels l;
+        l.clear();
+        TopList more;
+        more.clear();
+        for (int e = threadIdx.x, t = 0; e < entries; e += kDirectThreads, ++t) {
+            const unsigned long long p = __hip_atomic_fetch_add(&part[((size_t)b * gridDim.x + e / k) * kTopMax + e % k], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const float v = __uint_as_float((unsigned)p);
+            const int id = (int)(p >> 32);
+            if (entries > kDirectHeld * kDirectThreads) {
+                if (id != kNoId) more.offer(v, id);
+            } else {
+#pragma unroll
+                for (int q = 0; q < kDirectHeld; ++q)
+                    if (t == q) { l.v[q] = v; l.id[q] = id; }
+            }
+        }
+        if (entries > kDirectHeld * kDirectThreads) {
+            float ov;
+            int oi;
+            block_topk<kDirectThreads / 64>(more, k, ov, oi);
+            if (threadIdx.x < kTopMax) { shared.out_v[threadIdx.x] = ov; shared.out_id[threadIdx.x] = oi; }
+        } else {
+            few_topk(l, k, shared);
+        }
+        if ((int)threadIdx.x < k) {
+            values[(size_t)b * k + threadIdx.x] = shared.out_v[threadIdx.x];
+            indices[(size_t)b * k + threadIdx.x] = shared.out_id[threadIdx.x] != kNoId ? shared.out_id[threadIdx.x] : -1;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *ticket = 0u;
+}
+
 constexpr int kTopkRowSample = 4096;
 
 // Label values at the k best labels of every sample, summed per rank: host[r] over all samples, and the loss of the step beside
@@ -409,6 +664,40 @@ TopkCandidates topk_candidates_at(void* ws, int B, int sample) {
     c.val = reinterpret_cast<float*>(c.count + (size_t)B * kTopkCountStep);
     c.idx = reinterpret_cast<int*>(c.val + (size_t)B * kTopkCap);
     return c;
+}
+
+int direct_width(int B) { return B <= 1 ? 1 : B <= 2 ? 2 : 4; }
+bool takes_topk_direct(const Dims& d) {
+    return d.B <= 4 && d.K >= 4 && (size_t)d.N * direct_width(d.B) * sizeof(float) <= kDirectLds;
+}
+
+int launch_topk_direct(const void* x, const int32_t* idx, const void* w, const float* bias, bool bf16, const TopkArgs& tk, const Dims& d,
+                       hipStream_t s) {
+    const int quads = (d.K + 3) / 4;
+    int lanes = 1;
+    while (lanes < 64 && lanes < quads) lanes *= 2;
+    const int per_round = 64 / lanes, passes = (quads + lanes - 1) / lanes;
+    const long long per_block = (long long)(kDirectThreads / 64) * per_round * direct_rounds(direct_width(d.B));     // labels per step
+    const long long steps = std::max(1, kDirectHeld * lanes / direct_rounds(direct_width(d.B)));                      // of a workgroup, at most
+    const long long fill = std::min<long long>(device_cu_count(), (d.L + per_block - 1) / per_block);
+    const int blocks = (int)std::max(fill, (d.L + per_block * steps - 1) / (per_block * steps));
+    const size_t entries = (size_t)d.B * blocks * kTopMax, lds = (size_t)d.N * direct_width(d.B) * sizeof(float);
+    unsigned long long* part = nullptr;
+    unsigned* ticket = nullptr;
+    FFI_TRY(workspace_get(s, kWsTopk, entries * sizeof(*part), (void**)&part));
+    FFI_TRY(tickets_get(s, (void**)&ticket));
+    auto go = [&](auto kernel) -> int {
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kDirectThreads), lds, s, x, idx, w, bias, d.B, d.N, d.L, d.K, d.tp ? 1 : 0, lanes,
+                           passes, tk.k, part, ticket, tk.values, tk.indices);
+        FFI_HIP_TRY(hipGetLastError());
+        return FFI_OK;
+    };
+    switch (direct_width(d.B)) {
+        case 1: return bf16 ? go(topk_direct_kernel<true, 1>) : go(topk_direct_kernel<false, 1>);
+        case 2: return bf16 ? go(topk_direct_kernel<true, 2>) : go(topk_direct_kernel<false, 2>);
+        default: return bf16 ? go(topk_direct_kernel<true, 4>) : go(topk_direct_kernel<false, 4>);
+    }
 }
 
 int launch_topk_threshold(const float* scores, size_t row, int step, int S, TopkSampleLabels labels, int k, const TopkCandidates& c, int B,

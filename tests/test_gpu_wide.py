@@ -133,6 +133,54 @@ def test_forward_from_slices_in_lds(ffi, bf16, transposed):
         assert rel_err(out.cpu().numpy(), ref) <= 1e-5, (B, N, L, K)
 
 
+# Up to four samples, scores and answer in one launch: fan-ins of one quad, off the quads and of several passes over a row; fewer
+# labels than asked for, a label per lane and four, more workgroups than CUs; features that just fit
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,L,K,k", [(1, 12, 3, 4, 5), (2, 768, 70_001, 31, 8), (3, 500, 9_000, 64, 3), (4, 9_216, 40_000, 5, 5), (1, 36_864, 5_000, 257, 8),
+                                       (1, 30, 3_000_000, 4, 8), (4, 100, 1_100_003, 9, 1)])
+def test_topk_of_few_samples(ffi, bf16, B, N, L, K, k):
+    rng = np.random.default_rng(L + K)
+    x, w = rng.standard_normal((B, N)).astype(np.float32), rng.standard_normal((L, K)).astype(np.float32)
+    lookup, bias = rng.integers(0, N, (L, K)).astype(np.int32), rng.standard_normal(L).astype(np.float32)
+    tx, tw = torch.from_numpy(x), torch.from_numpy(w)
+    if bf16:
+        tx, tw = tx.bfloat16(), tw.bfloat16()
+        bias[:] = 0
+    ref = oracle.forward(tx.float().numpy(), lookup, tw.float().numpy(), transposed=False) + bias
+    want = np.argsort(-ref, axis=1, kind="stable")[:, :k]
+    values = np.full((B, k), -np.inf, np.float32)
+    values[:, :min(k, L)] = np.take_along_axis(ref, want, 1)
+    if bf16:
+        v, i = ffi.fan_in_sparse_topk_bf16(tx.cuda(), dev(lookup), tw.cuda(), k=k)
+    else:
+        v, i = ffi.fan_in_sparse_topk(tx.cuda(), dev(lookup), tw.cuda(), bias=dev(bias), k=k)
+    v, i = v.cpu().numpy(), i.cpu().numpy()
+    bound = 2e-5 * np.abs(ref).max()                    # sums of K products in another order; labels closer than that may change places
+    assert (i[:, min(k, L):] == -1).all() and (v[:, min(k, L):] == -np.inf).all()
+    assert np.abs(v[:, :min(k, L)] - values[:, :min(k, L)]).max() <= bound
+    assert np.abs(np.take_along_axis(ref, i[:, :min(k, L)].astype(np.int64), 1) - values[:, :min(k, L)]).max() <= bound
+    assert all(len(set(row[:min(k, L)])) == min(k, L) for row in i)
+
+
+def test_topk_of_few_samples_ties_and_specials(ffi):
+    N, L, K = 20, 100_000, 4
+    lookup = (np.arange(L * K, dtype=np.int64) * 7 % N).astype(np.int32).reshape(L, K)
+    w = torch.ones((L, K), device="cuda")
+    zeros = torch.zeros((2, N), device="cuda")
+    # equal scores go to the lower labels; many labels of few wavefronts above all others (more than the list of candidates holds)
+    v, i = ffi.fan_in_sparse_topk(zeros, dev(lookup), w, bias=torch.zeros(L, device="cuda"), k=8)
+    assert (i.cpu().numpy() == np.arange(8)).all() and (v == 0).all()
+    high = torch.from_numpy((np.arange(L) % 4096 < 1500).astype(np.float32)).cuda()
+    high[70_000] = 2.0
+    v, i = ffi.fan_in_sparse_topk(zeros, dev(lookup), w, bias=high, k=8)
+    assert (i.cpu().numpy() == np.array([70_000, 0, 1, 2, 3, 4, 5, 6])).all() and v[0, 0] == 2 and (v[:, 1:] == 1).all()
+    special = torch.full((L,), -float("inf"), device="cuda")
+    special[5], special[99_999], special[17] = float("nan"), float("inf"), 3.0
+    v, i = ffi.fan_in_sparse_topk(zeros, dev(lookup), w, bias=special, k=4)
+    assert (i.cpu().numpy() == np.array([99_999, 17, 0, 1])).all()
+    assert (v.cpu().numpy() == np.array([np.inf, 3, -np.inf, -np.inf], np.float32)).all()
+
+
 # Top-k without the scores: every label in the sample that sets the threshold and a part of them; ties across the whole layer,
 # more than a candidate list holds
 @pytest.mark.parametrize("bf16", [False, True])
