@@ -363,33 +363,50 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
 
 // ---- forward, slice in LDS ----------------------------------------------------------------------------------------
 // For slices that fit in LDS beside the lists: narrow inputs with few samples or in bf16.  The workgroup brings its slice, then
-// its wavefronts take blocks of consecutive labels (every row_step-th row of the layer) -- one round of lane groups after the other, as in fwd_sliced_kernel,
-// the rows read from LDS -- and write their rows of out in pieces of that many labels.
+// its wavefronts take rounds of consecutive labels (every row_step-th row of the layer), a lane group per label, the rows of the
+// slice read from LDS.
 //
 // What bounds it: for one to four samples the stream of ids and weights from memory; from there on LDS delivery (a row of
-// 16 GL bytes and half a list entry of 16 per connection and lane group).
+// 16 GL bytes per connection and lane group, and the lists) and the instructions around it.
+//   Scores leave from the registers: the lanes' low bits change places with the rounds (exchange_bit), which makes pieces of 32
+// labels without the tile in LDS that took them through it twice more; pieces of 32 bytes cost 140 us at 128 x 768 x 300,000 x 32
+// in bf16, the tile 112, these 89.  What a lane fetches is the same place of every chunk, so its divisions are done once.
+//   A wavefront takes 32 labels at a time, the last ones in even shares; with fewer labels than that for all, the workgroups are
+// as many as give each wavefront one round (64 x 768 x 8,192 x 32 in bf16: 28.7 us with 32 labels each, 18.0 so).
+//   The slice comes in with four columns of a lane's four samples per step, lanes side by side holding a row of the slice: with
+// a column per lane, 32 lanes wrote to one pair of banks (the same shape: 18.0 -> 14.4 us, a first list already in flight).
+//   At 100 x 500 x 131,073 x 24 in bf16, all of it together: 45.6 -> 36.4 us.
 typedef unsigned lds_v4u __attribute__((ext_vector_type(4)));
 constexpr int kLdThreads = 1024;
 constexpr size_t kLdThresholdBytes = 512;       // (behind the rest: thresholds of up to 64 samples, which would take 16 registers through the label loop)
 constexpr size_t kLdBudget = 160 * 1024 - kLdThresholdBytes;
 
-template <int GL> struct LdsShape {
+template <int GL, bool BF16> struct LdsShape {
     static constexpr int kGroups = 64 / GL;
-    static constexpr int kRounds = GL / 2;
-    static constexpr int kWaveLabels = kGroups * kRounds;                 // 32
+    static constexpr int kRounds = GL / 2;                                // whose scores leave together: of 32 labels
     static constexpr int kChunk = GL == 8 ? 32 : 16;
     static constexpr int kQuads = (kGroups * kChunk + 255) / 256;
-    static constexpr int kStride = kChunk + 2;
-    static constexpr int kWaveBytes = kGroups * kStride * 8;              // (also holds 8 samples of a wavefront's labels)
+    // a label's list, in words: (row offset, weight) pairs; in bf16 the offsets, and in an array of their own the weights as they are,
+    // two to a word
+    static constexpr int kPitch = BF16 ? kChunk + 4 : 2 * kChunk + 4, kWeightPitch = BF16 ? kChunk / 2 + 2 : 0;
+    static constexpr int kWaveBytes = kGroups * (kPitch + kWeightPitch) * 4;
 };
-template <int GL> inline size_t lds_kernel_bytes(int N) { return (size_t)(N + 1) * GL * 16 + (size_t)(kLdThreads / 64) * LdsShape<GL>::kWaveBytes; }
+template <int GL, bool BF16> inline size_t lds_kernel_bytes(int N) { return (size_t)(N + 1) * GL * 16 + (size_t)(kLdThreads / 64) * LdsShape<GL, BF16>::kWaveBytes; }
+
+// Lanes whose bit is clear and set (DPP step CTRL pairs them): the pair's a to the former in place of (a, b), its b to the latter.
+template <int CTRL> __device__ __forceinline__ void exchange_bit(bool bit, float& a, float& b) {
+    const int send = __float_as_int(bit ? a : b);
+    const float other = __int_as_float(__builtin_amdgcn_update_dpp(send, send, CTRL, 0xf, 0xf, false));
+    a = bit ? other : a;
+    b = bit ? b : other;
+}
 
 template <int GL, bool BF16, bool QUADS>
 __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restrict__ features, const int32_t* __restrict__ idx,
                                                              const void* __restrict__ w, const float* __restrict__ bias,
                                                              float* __restrict__ out, int B, int N, int L, int K, int tp, int row_step,
                                                              int slices, int streams, int chunk, const TopkSink sink) {
-    using S = LdsShape<GL>;
+    using S = LdsShape<GL, BF16>;
     constexpr int kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer, kWaves = kLdThreads / 64;
     constexpr unsigned kRow = GL * 16u;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -397,61 +414,85 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
     const int slice = u % slices, stream = u / slices;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & (GL - 1), grp = lane / GL;
-    {
-        // four samples of a column per thread and step: from a row of [N,B], or from four rows of [B,N]
+    auto stage = [&]() {
+        // four samples of a column from a row of [N,B], or of four columns from four rows of [B,N]; lanes side by side hold a
+        // column's samples, and write its row of the slice together
         using T = typename LaneAcc<BF16>::Element;
         const T* x = static_cast<const T*>(features);
         Quad<T>* dst = reinterpret_cast<Quad<T>*>(smem);
         constexpr int kQ = kSl / 4;
-#pragma unroll 4
-        for (int e = threadIdx.x; e < N * kQ; e += kLdThreads) {
-            const int n = tp ? e / kQ : e % N, c = tp ? e % kQ : e / N;
+        const int width = tp ? B : N;                                     // of a row of the features
+        auto read4 = [&](int row, int at) {
+            const T* from = x + (size_t)row * width;
             Quad<T> q;
+            if (at + 4 <= width) {
+                q = *reinterpret_cast<const Quad<T>*>(from + at);         // (at any alignment)
+            } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int b = slice * kSl + 4 * c + i;
-                const size_t at = tp ? (size_t)n * B + min(b, B - 1) : (size_t)min(b, B - 1) * N + n;
-                q.v[i] = b < B ? x[at] : (T)0;
+                for (int i = 0; i < 4; ++i) q.v[i] = from[min(at + i, width - 1)];
             }
-            dst[n * kQ + c] = q;
+            return q;
+        };
+        if (tp) {
+#pragma unroll 4
+            for (int e = threadIdx.x; e < N * kQ; e += kLdThreads) {
+                const int n = e / kQ, c = e % kQ, b = slice * kSl + 4 * c;
+                Quad<T> q = read4(n, b);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q.v[i] = b + i < B ? q.v[i] : (T)0;
+                dst[n * kQ + c] = q;
+            }
+        } else {
+#pragma unroll 2
+            for (int e = threadIdx.x; e < (N + 3) / 4 * kQ; e += kLdThreads) {
+                const int n = e / kQ * 4, c = e % kQ, b = slice * kSl + 4 * c;
+                Quad<T> rows[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rows[i] = read4(min(b + i, B - 1), n);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    Quad<T> q;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) q.v[i] = b + i < B ? rows[i].v[v] : (T)0;
+                    if (n + v < N) dst[(n + v) * kQ + c] = q;
+                }
+            }
         }
         if (threadIdx.x < GL) reinterpret_cast<uint4*>(smem)[N * GL + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);    // what entries behind a list's end name
-    }
+    };
     float* const slice_tau = reinterpret_cast<float*>(smem + (size_t)(N + 1) * kRow + (size_t)kWaves * S::kWaveBytes);
     int* const slice_tie = reinterpret_cast<int*>(slice_tau + kSl);
-    if (sink.tau != nullptr && threadIdx.x < kSl) {
-        slice_tau[threadIdx.x] = sink.tau[slice * kSl + threadIdx.x];
-        slice_tie[threadIdx.x] = sink.tie[slice * kSl + threadIdx.x];
-    }
-    __syncthreads();
     unsigned char* const mine = smem + (size_t)(N + 1) * kRow + (size_t)wave * S::kWaveBytes;
-    uint2* list = reinterpret_cast<uint2*>(mine);
+    unsigned* const list = reinterpret_cast<unsigned*>(mine);
+    unsigned* const list_w = list + S::kGroups * S::kPitch;               // (bf16)
     // (raw LDS addresses: what a column id beyond the slice names is outside the LDS and reads as zero, or some of the LDS)
     const unsigned rows = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem + (unsigned)sub * 16u;
     const unsigned no_row = (unsigned)N * kRow;
     const unsigned* w32 = reinterpret_cast<const unsigned*>(w);
     const unsigned short* w16 = reinterpret_cast<const unsigned short*>(w);
-    const int blocks = (L + S::kWaveLabels - 1) / S::kWaveLabels, step = streams * kWaves;
     const int b0 = slice * kSl, nb = min(kSl, B - b0);
     const int mine0 = b0 + sub * kPer;                                    // first sample of this lane
 
+    // Lane and quad v (or, without QUADS, element 4 v + e) number the connections of a chunk of kGroups labels through: label f / n,
+    // connection f % n, the same for every chunk.  What lies behind the row, or the last label, is read in place of something else.
     uint4 ids[S::kQuads], ws[S::kQuads];
     auto place = [&](unsigned f, int n, int& l, int& k) {
         l = (int)((f * (65536u / (unsigned)n + 1u)) >> 16);               // f / n for f < 1,024 and n <= 32
         k = (int)f - l * n;
     };
-    auto fetch = [&](int blk, int q, int k0) {
-        const int kc = min(chunk, K - k0), j = blk * S::kWaveLabels + q * S::kGroups;
+    const unsigned row_pitch = (unsigned)row_step * (unsigned)K;          // (labels * row_step * K < 2^31)
+    auto fetch = [&](int q, int k0) {
+        const int kc = min(chunk, K - k0), j = q * S::kGroups;
 #pragma unroll
         for (int v = 0; v < S::kQuads; ++v) {
             int l, k;
             if (QUADS) {
-                place((unsigned)(64 * v + lane), kc / 4, l, k);
-                const size_t at = (size_t)min(j + min(l, S::kGroups - 1), L - 1) * row_step * K + k0 + 4 * k;
+                place((unsigned)(64 * v + lane), chunk / 4, l, k);
+                const unsigned at = (unsigned)min(j + min(l, S::kGroups - 1), L - 1) * row_pitch + (unsigned)(k0 + (4 * k < kc ? 4 * k : 0));
                 ids[v] = *reinterpret_cast<const uint4*>(idx + at);
                 if (BF16) {
                     const uint2 h = *reinterpret_cast<const uint2*>(w16 + at);
-                    ws[v] = make_uint4(h.x << 16, h.x & 0xffff0000u, h.y << 16, h.y & 0xffff0000u);
+                    ws[v].x = h.x; ws[v].y = h.y;
                 } else {
                     ws[v] = *reinterpret_cast<const uint4*>(w32 + at);
                 }
@@ -460,10 +501,10 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
                 unsigned* w4 = &ws[v].x;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    place((unsigned)(64 * (4 * v + e) + lane), kc, l, k);
-                    const size_t at = (size_t)min(j + min(l, S::kGroups - 1), L - 1) * row_step * K + k0 + k;
+                    place((unsigned)(64 * (4 * v + e) + lane), chunk, l, k);
+                    const unsigned at = (unsigned)min(j + min(l, S::kGroups - 1), L - 1) * row_pitch + (unsigned)(k0 + (k < kc ? k : 0));
                     id4[e] = (unsigned)idx[at];
-                    w4[e] = BF16 ? (unsigned)w16[at] << 16 : w32[at];
+                    w4[e] = BF16 ? (unsigned)w16[at] : w32[at];
                 }
             }
         }
@@ -474,89 +515,132 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
         for (int v = 0; v < S::kQuads; ++v) {
             int l, k;
             if (QUADS) {
-                place((unsigned)(64 * v + lane), kc / 4, l, k);
-                if (l < S::kGroups) {
-                    uint4* p = reinterpret_cast<uint4*>(list + l * S::kStride + 4 * k);
-                    p[0] = make_uint4(ids[v].x * kRow, ws[v].x, ids[v].y * kRow, ws[v].y);
-                    p[1] = make_uint4(ids[v].z * kRow, ws[v].z, ids[v].w * kRow, ws[v].w);
+                place((unsigned)(64 * v + lane), chunk / 4, l, k);
+                if (l < S::kGroups && 4 * k < kc) {
+                    if (BF16) {
+                        *reinterpret_cast<uint4*>(list + l * S::kPitch + 4 * k) = make_uint4(ids[v].x * kRow, ids[v].y * kRow, ids[v].z * kRow, ids[v].w * kRow);
+                        *reinterpret_cast<uint2*>(list_w + l * S::kWeightPitch + 2 * k) = make_uint2(ws[v].x, ws[v].y);
+                    } else {
+                        uint4* p = reinterpret_cast<uint4*>(list + l * S::kPitch + 8 * k);
+                        p[0] = make_uint4(ids[v].x * kRow, ws[v].x, ids[v].y * kRow, ws[v].y);
+                        p[1] = make_uint4(ids[v].z * kRow, ws[v].z, ids[v].w * kRow, ws[v].w);
+                    }
                 }
             } else {
                 const unsigned id4[4] = {ids[v].x, ids[v].y, ids[v].z, ids[v].w}, w4[4] = {ws[v].x, ws[v].y, ws[v].z, ws[v].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    place((unsigned)(64 * (4 * v + e) + lane), kc, l, k);
-                    if (l < S::kGroups) list[l * S::kStride + k] = make_uint2(id4[e] * kRow, w4[e]);
+                    place((unsigned)(64 * (4 * v + e) + lane), chunk, l, k);
+                    if (l >= S::kGroups) continue;
+                    const unsigned row = k < kc ? id4[e] * kRow : no_row, wv = k < kc ? w4[e] : 0u;       // (the walk takes four at a time)
+                    if (BF16) {
+                        list[l * S::kPitch + k] = row;
+                        reinterpret_cast<unsigned short*>(list_w + l * S::kWeightPitch)[k] = (unsigned short)wv;
+                    } else {
+                        *reinterpret_cast<uint2*>(list + l * S::kPitch + 2 * k) = make_uint2(row, wv);
+                    }
                 }
             }
         }
-        if ((kc & 3) != 0 && lane < S::kGroups)                           // the walk takes four at a time
-            for (int k = kc; k < (kc + 3) / 4 * 4; ++k) list[lane * S::kStride + k] = make_uint2(no_row, 0u);
     };
-    const uint4* mylist = reinterpret_cast<const uint4*>(list + grp * S::kStride);
-    int blk = stream * kWaves + wave;
-    if (blk >= blocks) return;
-    fetch(blk, 0, 0);
-    for (; blk < blocks; blk += step) {
+    const unsigned* const mylist = list + grp * S::kPitch;
+    const unsigned* const my_w = list_w + grp * S::kWeightPitch;
+    // Rounds of kGroups consecutive labels.  The wavefronts take kRounds at a time, side by side, as long as all have some to take, then
+    // an even share of what is left.
+    const int rounds = (L + S::kGroups - 1) / S::kGroups, all = streams * kWaves, me = stream * kWaves + wave;
+    const int full = rounds / (all * S::kRounds), tail = rounds - full * all * S::kRounds, share = (tail + all - 1) / all;
+    auto begin_of = [&](int t) { return t < full ? (t * all + me) * S::kRounds : min(full * all * S::kRounds + me * share, rounds); };
+    fetch(begin_of(0), 0);                                                // (in flight beside the slice)
+    stage();
+    if (sink.tau != nullptr && threadIdx.x < kSl) {
+        slice_tau[threadIdx.x] = sink.tau[slice * kSl + threadIdx.x];
+        slice_tie[threadIdx.x] = sink.tie[slice * kSl + threadIdx.x];
+    }
+    __syncthreads();
+    if (full == 0 && begin_of(0) >= rounds) return;
+    const int lane_row = (sub & ~(S::kRounds - 1)) * kPer;                // first of the rows of out that this lane stores
+    for (int t = 0; t <= full; ++t) {
+        const int q = begin_of(t), q_end = t < full ? q + S::kRounds : min(q + share, rounds), after = min(begin_of(min(t + 1, full)), rounds - 1);
         LaneAcc<BF16> acc[S::kRounds];
-        const int jb = blk * S::kWaveLabels;
 #pragma unroll
-        for (int q = 0; q < S::kRounds; ++q) {
+        for (int r = 0; r < S::kRounds; ++r) {
 #pragma unroll
-            for (int i = 0; i < kPer; ++i) acc[q].a[i] = 0.f;
+            for (int i = 0; i < kPer; ++i) acc[r].a[i] = 0.f;
+            if (q + r >= q_end) continue;                                 // (wave-uniform)
             for (int k0 = 0; k0 < K; k0 += chunk) {
                 __builtin_amdgcn_wave_barrier();                          // (the list is the wavefront's own, and LDS serves it in order)
                 put(k0);
-                if (k0 + chunk < K) fetch(blk, q, k0 + chunk);
-                else if (q + 1 < S::kRounds) fetch(blk, q + 1, 0);
-                else fetch(min(blk + step, blocks - 1), 0, 0);
+                if (k0 + chunk < K) fetch(q + r, k0 + chunk);
+                else fetch(q + r + 1 < q_end ? q + r + 1 : after, 0);
                 __builtin_amdgcn_wave_barrier();
                 const int n = min(chunk, K - k0);
 #pragma unroll 2
                 for (int i = 0; i < n; i += 4) {
-                    uint4 e[2], x[4];
+                    uint4 x[4];
+                    unsigned at[4], wv[4];
+                    if (BF16) {
+                        const uint4 e = *reinterpret_cast<const uint4*>(mylist + i);
+                        const uint2 f = *reinterpret_cast<const uint2*>(my_w + i / 2);
+                        at[0] = e.x; at[1] = e.y; at[2] = e.z; at[3] = e.w;
+                        wv[0] = f.x; wv[1] = f.y;
+                    } else {
 #pragma unroll
-                    for (int v = 0; v < 2; ++v) e[v] = mylist[i / 2 + v];
+                        for (int v = 0; v < 2; ++v) {
+                            const uint4 e = *reinterpret_cast<const uint4*>(mylist + 2 * i + 4 * v);
+                            at[2 * v] = e.x; at[2 * v + 1] = e.z;
+                            wv[2 * v] = e.y; wv[2 * v + 1] = e.w;
+                        }
+                    }
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) x[v] = __builtin_bit_cast(uint4, *(const lds_v4u __attribute__((address_space(3)))*)(size_t)(rows + ((v & 1) ? e[v / 2].z : e[v / 2].x)));
+                    for (int v = 0; v < 4; ++v) x[v] = __builtin_bit_cast(uint4, *(const lds_v4u __attribute__((address_space(3)))*)(size_t)(rows + at[v]));
 #pragma unroll
-                    for (int v = 0; v < 2; ++v) acc[q].add2(x[2 * v], x[2 * v + 1], e[v].y, e[v].w);
+                    for (int v = 0; v < 2; ++v) acc[r].add_pair(x[2 * v], x[2 * v + 1], wv + v * (BF16 ? 1 : 2));
                 }
             }
-        }
-        if (sink.tau != nullptr) {
-            float tau[kPer];
+            const int j = (q + r) * S::kGroups + grp;
+            if (bias != nullptr) {
+                const float bj = bias[(size_t)min(j, L - 1) * row_step];
 #pragma unroll
-            for (int i = 0; i < kPer; ++i) tau[i] = slice_tau[sub * kPer + i];
-#pragma unroll
-            for (int q = 0; q < S::kRounds; ++q) {
-                const int j = jb + q * S::kGroups + grp;
-                if (bias != nullptr) {
-                    const float bj = bias[(size_t)min(j, L - 1) * row_step];
-#pragma unroll
-                    for (int i = 0; i < kPer; ++i) acc[q].a[i] += bj;
-                }
-                topk_append(sink, acc[q].a, tau, slice_tie + sub * kPer, mine0, B - mine0, j, j < L);
+                for (int i = 0; i < kPer; ++i) acc[r].a[i] += bj;
             }
-            continue;
-        }
-        float* tile = reinterpret_cast<float*>(mine);                     // eight samples (or what a lane holds of four) x the labels
-        constexpr int kPitch = S::kWaveLabels + 1, kTake = kSl < 8 ? kSl : 8, kRowsPerStep = 64 / S::kWaveLabels;
-        static_assert(kTake * kPitch * 4 <= S::kWaveBytes, "the tile lies in the list's place");
-        const int jl = lane % S::kWaveLabels, j = jb + jl;
-        const float bj = (bias != nullptr && j < L) ? bias[(size_t)j * row_step] : 0.f;
-        for (int s0 = 0; s0 < nb; s0 += kTake) {
-            __builtin_amdgcn_wave_barrier();
-            if (sub * kPer >= s0 && sub * kPer < s0 + kTake) {
+            if (sink.tau != nullptr) {
+                float tau[kPer];
 #pragma unroll
-                for (int q = 0; q < S::kRounds; ++q)
-#pragma unroll
-                    for (int i = 0; i < kPer; ++i) tile[(sub * kPer + i - s0) * kPitch + q * S::kGroups + grp] = acc[q].a[i];
+                for (int i = 0; i < kPer; ++i) tau[i] = slice_tau[sub * kPer + i];
+                topk_append(sink, acc[r].a, tau, slice_tie + sub * kPer, mine0, B - mine0, j, j < L);
             }
-            __builtin_amdgcn_wave_barrier();
-            for (int e = lane / S::kWaveLabels; e < kTake && s0 + e < nb; e += kRowsPerStep)
-                if (j < L) out[(size_t)(b0 + s0 + e) * L + j] = bias != nullptr ? tile[e * kPitch + jl] + bj : tile[e * kPitch + jl];
         }
-        __builtin_amdgcn_wave_barrier();
+        if (sink.tau != nullptr) continue;
+        // Rows of out leave in pieces of 32 labels: the lanes' low bits, which number samples, change places with the rounds.
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if constexpr (S::kRounds >= 2) {
+#pragma unroll
+                for (int r = 0; r < S::kRounds; r += 2) exchange_bit<0xb1>((sub & 1) != 0, acc[r].a[i], acc[r + 1].a[i]);
+            }
+            if constexpr (S::kRounds == 4) {
+#pragma unroll
+                for (int r = 0; r < 2; ++r) exchange_bit<0x4e>((sub & 2) != 0, acc[r].a[i], acc[r + 2].a[i]);
+            }
+        }
+        const int j = (q + (sub & (S::kRounds - 1))) * S::kGroups + grp;
+        const bool have = j < min(L, q_end * S::kGroups);
+        float* to = out + (size_t)(b0 + lane_row) * L + min(j, L - 1);
+        if (nb == kSl) {
+            if (have) {
+#pragma unroll
+                for (int r = 0; r < S::kRounds; ++r)
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) to[(size_t)(r * kPer + i) * L] = acc[r].a[i];
+            }
+        } else {
+            const int mine_nb = have ? nb : 0;
+#pragma unroll
+            for (int r = 0; r < S::kRounds; ++r)
+#pragma unroll
+                for (int i = 0; i < kPer; ++i)
+                    if (lane_row + r * kPer + i < mine_nb) to[(size_t)(r * kPer + i) * L] = acc[r].a[i];
+        }
     }
 }
 
@@ -879,11 +963,11 @@ int launch_fwd_sliced_lanes(int gl, const FwdSliced& a, const Dims& d, hipStream
 
 template <int GL, bool BF16>
 int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
-    using S = LdsShape<GL>;
+    using S = LdsShape<GL, BF16>;
     const int chunks = (d.K + S::kChunk - 1) / S::kChunk, chunk = ((d.K + chunks - 1) / chunks + 3) / 4 * 4;
-    const int blocks = (d.L + S::kWaveLabels - 1) / S::kWaveLabels, waves = kLdThreads / 64;
-    const int streams = std::max(1, std::min((blocks + waves - 1) / waves, device_cu_count() / a.slices));
-    const size_t lds = lds_kernel_bytes<GL>(d.N) + (a.sink.tau != nullptr ? kLdThresholdBytes : 0);
+    const int waves = kLdThreads / 64, rounds = (d.L + S::kGroups - 1) / S::kGroups;
+    const int streams = std::max(1, std::min((rounds + waves - 1) / waves, device_cu_count() / a.slices));
+    const size_t lds = lds_kernel_bytes<GL, BF16>(d.N) + (a.sink.tau != nullptr ? kLdThresholdBytes : 0);
     static_assert(2 * GL * LaneAcc<BF16>::kSamples * 4 <= kLdThresholdBytes, "thresholds of a slice");
     const dim3 grid((unsigned)(streams * a.slices)), block(kLdThreads);
     if (a.quads) {
@@ -977,7 +1061,7 @@ SlicedForm sliced_form(int B, int N) {
     f.gl = slice_lanes(B, kPer);
     // (two lanes per row at least: with one the lists of a wavefront are as long as its ids are short of a line; one sample,
     // 670,091 labels: 98 us against 51)
-    auto fits = [&](int gl) { return (gl == 8 ? lds_kernel_bytes<8>(N) : gl == 4 ? lds_kernel_bytes<4>(N) : lds_kernel_bytes<2>(N)) <= kLdBudget; };
+    auto fits = [&](int gl) { return (gl == 8 ? lds_kernel_bytes<8, BF16>(N) : gl == 4 ? lds_kernel_bytes<4, BF16>(N) : lds_kernel_bytes<2, BF16>(N)) <= kLdBudget; };
     f.in_lds = fits(std::max(f.gl, 2));
     if (f.in_lds) f.gl = std::max(f.gl, 2);
     else if (f.gl == 8 && fits(4)) { f.gl = 4; f.in_lds = true; }

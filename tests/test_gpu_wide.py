@@ -133,6 +133,34 @@ def test_forward_from_slices_in_lds(ffi, bf16, transposed):
         assert rel_err(out.cpu().numpy(), ref) <= 1e-5, (B, N, L, K)
 
 
+# Slices in LDS, what the wavefronts share out: full turns of 32 labels and a last one of one round, a single label or none left for
+# most of them, fewer rounds than wavefronts; slices with samples missing; features whose rows start at every alignment
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,N,L,K", [(61, 33, 131_073, 4), (64, 32, 2_049, 24), (250, 31, 33_000, 9), (13, 30, 140_001, 5), (7, 29, 270_000, 3), (3, 2, 7, 2)])
+def test_forward_from_slices_in_lds_shares(ffi, bf16, B, N, L, K):
+    rng = np.random.default_rng(L + K)
+    lookup = rng.integers(0, N, (L, K)).astype(np.int32)
+    tx = torch.from_numpy(rng.standard_normal(B * N + 1).astype(np.float32))
+    tw = torch.from_numpy(rng.standard_normal((L, K)).astype(np.float32))
+    if bf16:
+        tx, tw = tx.bfloat16(), tw.bfloat16()
+    for transposed in (False, True):
+        x = tx[1:].view(N, B) if transposed else tx[1:].view(B, N)
+        xn = (x.t() if transposed else x).float().numpy().astype(np.float64)
+        ref, size = np.zeros((B, L)), np.zeros((B, L))
+        for k in range(K):
+            term = xn[:, lookup[:, k]] * tw[:, k].float().numpy().astype(np.float64)
+            ref += term
+            size += np.abs(term)
+        xd = tx.cuda()[1:].view(x.shape)
+        if bf16:
+            out = ffi.fan_in_sparse_matmul_bf16(xd, dev(lookup), tw.cuda(), transposed=transposed)
+        else:
+            out = (ffi.fan_in_sparse_matmul_tp if transposed else ffi.fan_in_sparse_matmul)(xd, dev(lookup), tw.cuda())
+        # K fused products and at most two more sums of partial ones, each rounded once: (K + 2) 2^-24 of the sum of magnitudes
+        assert (np.abs(out.cpu().numpy() - ref) <= (K + 2) * 2.0 ** -24 * size + 1e-30).all()
+
+
 # Up to four samples, scores and answer in one launch: fan-ins of one quad, off the quads and of several passes over a row; fewer
 # labels than asked for, a label per lane and four, more workgroups than CUs; features that just fit
 @pytest.mark.parametrize("bf16", [False, True])
