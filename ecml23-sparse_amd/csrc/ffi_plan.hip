@@ -90,13 +90,17 @@ __device__ __forceinline__ unsigned column_slots(unsigned thread, unsigned even,
     return max(first ? 2u * first - 1u : 0u, 2u * second);
 }
 
-// The sum of v over the 64 lanes, in a scalar register.
-__device__ __forceinline__ int wave_total(int v) {
+// The sum of v over each LANES consecutive lanes (32 or 64), in all of them.
+template <int LANES> __device__ __forceinline__ int lanes_total(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);         // lane ^ 1
     v += __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);         // lane ^ 2
     v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);        // 7 - lane within eight
     v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);        // 15 - lane within sixteen
-    return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) + (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
+    const auto rows = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = (int)(rows[0] + rows[1]);
+    if (LANES == 32) return v;
+    const auto halves = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (int)(halves[0] + halves[1]);
 }
 
 // Which LDS row of the walking kernel's tile each label is staged into (rowpos[j], inside the label's tile).
@@ -106,10 +110,12 @@ __device__ __forceinline__ int wave_total(int v) {
 // and each goes to the half that the columns it feeds have used less so far (weighted sum over its connections
 // of even-count minus odd-count of the column), which keeps the columns that matter close to an even split.
 // Rows of a half are handed out in ascending order, at most `cap` per half.  One workgroup per tile; the tile's
-// column ids are staged in LDS, one wavefront then decides label after label (lane <-> connection).
+// column ids are staged in LDS, one wavefront then decides label after label (lane <-> connection), or two at a time where 32 lanes
+// hold a fan-in; beyond a fan-in of 64 a lane has several connections.
 // (`col_lo`: the plan covers the columns [col_lo, col_lo + ncols) only; connections into other columns are left out)
 // (`all_columns_count`: plans that hand the columns to threads by length -- there every column is about as long as the
 // longest of its slice, so every column's balance weighs the same)
+template <int LANES, bool MORE>              // (MORE: fan-ins above LANES = 64)
 __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restrict__ idx, int L, int K, int tile_labels, int cap,
                                                          int ncols, unsigned short* __restrict__ rowpos, int col_lo,
                                                          int all_columns_count) {
@@ -162,72 +168,98 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     __syncthreads();
     if (threadIdx.x >= 64) return;
     const int lane = threadIdx.x;
+    constexpr int kAbreast = 64 / LANES;                                         // labels decided together
+    const int groups = (nl + kAbreast - 1) / kAbreast, k_mine = lane & (LANES - 1), abreast = lane / LANES;
     unsigned char* half = reinterpret_cast<unsigned char*>(wt + ncols + 2);      // [tile_labels] the half each label goes to
-    // column of connection k of label jl
-    auto id_of = [&](int jl, int k) {
-        const int q = (k * 43691) >> 17;                                         // k / 3 for k < 2^15
-        return (int)((ids3[jl * W + q] >> (10 * (k - 3 * q))) & 1023u);
-    };
     int placed[2] = {0, 0};
-    // What bounds the kernel is the chain from one label's adds to the next label's decision: an LDS round trip and the sum
-    // over the lanes, by DPP (through the LDS crossbar, six round trips more: 615 us at 670,091 labels x fan-in 32; 317 so).
-    // With at most 64 connections a lane has one: its column is asked for two labels ahead, the column's weight one.
-    const bool one_each = K <= 64;
-    const unsigned* const my_ids = ids3 + (lane < K ? lane / 3 : 0);
-    const int my_shift = 10 * (lane % 3);
-    auto word_of = [&](int jl) { return my_ids[min(jl, nl - 1) * W]; };
-    int col1 = 0, w0 = 0;
+    // What bounds the kernel is the chain from one step's adds to the next step's decision: an LDS round trip, the sum over the
+    // lanes by DPP and lane swaps, a comparison in every lane; what it does to the counts of placed labels is beside the chain.  Of
+    // two labels decided together the second does not see what the first just did: 670,091 labels x fan-in 32 over 768 columns
+    // 322 -> 181 us, 200,000 x 8 over 300 143 -> 81, with slot rows per connection 1.1522 -> 1.1523, 2.0510 -> 2.0514.  (Four
+    // together: 0.1 to 0.4 % more slot rows, which every walk pays for.  Two of a fan-in of 64, two connections a lane: 528 -> 455
+    // us at 501,070 labels, for 0.16 % more.)
+    // A lane's column is asked for two steps ahead, the column's weight one.
+    auto place_of = [&](int k) { return make_int2(k / 3, 10 * (k % 3)); };
+    const int2 place = place_of(min(k_mine, K - 1));
+    auto label_of = [&](int g) { return g * kAbreast + abreast; };
+    auto word_of = [&](int g) { return ids3[min(label_of(g), nl - 1) * W + place.x]; };
+    const bool on = k_mine < K;
+    int col1 = 0, w1 = 0;                                                        // the next label's
     unsigned word2 = 0;
-    auto column = [&](unsigned word) { return (int)((word >> my_shift) & 1023u); };
-    auto begin = [&]() {
-        col1 = column(word_of(0));
-        word2 = word_of(1);
-        w0 = lane < K ? (int)wt[col1] : 0;
+    auto advance = [&](int g) {                                                  // to label_of(g), whose word is here
+        col1 = (int)((word2 >> place.y) & 1023u);
+        if (kAbreast > 1 && label_of(g) >= nl) col1 = ncols;                     // (behind the last label: weight 0)
+        word2 = word_of(g + 1);
+        const int w = (int)wt[col1];
+        w1 = on ? w : 0;
     };
-    // the balance that label jl asks for, after `back` (0: nothing) is added to its columns; then `decide` says what is added
-    auto step = [&](int jl, int back, auto decide) {
-        if (one_each) {
-            const int c = col1, w = w0;
-            if (back != 0 && lane < K) atomicAdd(&imb[c], back);
-            const int v = imb[c];
-            col1 = column(word2);
-            word2 = word_of(jl + 2);
-            w0 = lane < K ? (int)wt[col1] : 0;
-            const int delta = decide(wave_total(w * v));
-            if (lane < K) atomicAdd(&imb[c], delta);                                // (a column may occur twice in a label)
-        } else {
-            if (back != 0)
-                for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], back);
-            int sum = 0;
-            for (int k = lane; k < K; k += 64) { const int c = id_of(jl, k); sum += wt[c] * imb[c]; }
-            const int delta = decide(wave_total(sum));
-            for (int k = lane; k < K; k += 64) atomicAdd(&imb[id_of(jl, k)], delta);
+    // connections behind the first of a lane (fan-ins above 64)
+    auto rest = [&](int g, auto visit) {
+        if (!MORE) return;
+        for (int k = lane + 64; k < K; k += 64) {
+            const int2 at = place_of(k);
+            visit((int)((ids3[label_of(g) * W + at.x] >> at.y) & 1023u));
         }
     };
-    begin();
-    for (int jl = 0; jl < nl; ++jl) {
-        step(jl, 0, [&](int sum) {
-            int color = sum > 0 ? 1 : (sum < 0 ? 0 : (placed[1] < placed[0] ? 1 : 0));
-            if (placed[color] >= cap) color ^= 1;
-            if (lane == 0) half[jl] = (unsigned char)color;
-            ++placed[color];
-            return color ? -1 : 1;
-        });
+    // the balance that a lane's label asks for, after `back` (0: nothing) is added to its columns; then `decide` says which half
+    auto step = [&](int g, int back, auto decide) {
+        const int c = col1, w = w1;
+        if (back != 0) {
+            if (__builtin_expect(on, 1)) atomicAdd(&imb[c], back);
+            rest(g, [&](int q) { atomicAdd(&imb[q], back); });
+        }
+        int sum = __mul24(w, imb[c]);
+        advance(g + 1);
+        rest(g, [&](int q) { sum += wt[q] * imb[q]; });
+        const int color = decide(lanes_total<LANES>(sum)), delta = color ? -1 : 1;
+        if (__builtin_expect(on, 1)) atomicAdd(&imb[c], delta);                                          // (a column may occur twice in a label)
+        rest(g, [&](int q) { atomicAdd(&imb[q], delta); });
+        if (__builtin_expect(k_mine == 0 && label_of(g) < nl, 1)) half[label_of(g)] = (unsigned char)color;
+    };
+    // where the labels of a step go once the halves may be full: `color` as far as there is room, else `other`
+    auto settle = [&](int g, int color, int other, bool again) {
+        const unsigned long long first = kAbreast == 1 ? 1ull : 1ull | 1ull << LANES;            // a label's first lane
+        const unsigned long long there = first & (g * kAbreast + kAbreast > nl ? 1ull : ~0ull);
+        unsigned long long to = __ballot(color != 0) & there;
+        const unsigned long long was = __ballot(other != 0) & there;
+        if (again) {
+            placed[1] -= __popcll(was);
+            placed[0] -= __popcll(there & ~was);
+        }
+        if (__builtin_expect(max(placed[0], placed[1]) + kAbreast > cap, 0)) {                          // (uniform)
+            int room[2] = {cap - placed[0], cap - placed[1]};
+            // (labels that stay keep their places: theirs first)
+#pragma unroll
+            for (int pass = 0; pass < 2; ++pass)
+#pragma unroll
+                for (int h = 0; h < kAbreast; ++h) {
+                    const unsigned long long bit = 1ull << (h * LANES);
+                    if (!(there & bit) || (again && ((to ^ was) & bit)) != (pass == 1)) continue;
+                    if (room[(to & bit) ? 1 : 0] <= 0) to ^= bit;
+                    --room[(to & bit) ? 1 : 0];
+                }
+            color = (int)(to >> (abreast * LANES) & 1ull);
+        }
+        placed[1] += __popcll(to);
+        placed[0] += __popcll(there & ~to);
+        return color;
+    };
+    word2 = word_of(0);
+    advance(0);
+    for (int g = 0; g < groups; ++g) {
+        const int even = placed[1] < placed[0] ? 1 : 0;
+        step(g, 0, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : even ^ abreast), 0, false); });
     }
     // Second sweep: every label is taken out and put back into the half its columns now ask for -- the first sweep placed
     // the early labels knowing nothing of the later ones.  (Measured on uniformly drawn ids, 586-label tiles of fan-in 32
     // over 768 columns: slot rows 1.528 -> 1.514 per connection, where columns of unconstrained order would need 1.490.)
-    begin();
-    int next_old = half[0];                               // (written by lane 0 above; LDS accesses of a wavefront are in order)
-    for (int jl = 0; jl < nl; ++jl) {
-        const int old = __builtin_amdgcn_readfirstlane(next_old);
-        next_old = half[min(jl + 1, nl - 1)];
-        step(jl, old ? 1 : -1, [&](int sum) {
-            int color = sum > 0 ? 1 : (sum < 0 ? 0 : old);
-            if (color != old && placed[color] >= cap) color = old;
-            if (color != old) { --placed[old]; ++placed[color]; if (lane == 0) half[jl] = (unsigned char)color; }
-            return color ? -1 : 1;
-        });
+    word2 = word_of(0);
+    advance(0);
+    int next_old = half[min(label_of(0), nl - 1)];       // (written by this wavefront above, whose LDS accesses are in order)
+    for (int g = 0; g < groups; ++g) {
+        const int old = next_old;
+        next_old = half[min(label_of(g + 1), nl - 1)];
+        step(g, old ? 1 : -1, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : old), old, true); });
     }
     // rows of a half are handed out in ascending label order
     int next[2] = {0, 0};
@@ -877,9 +909,10 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     if (!dev_alloc(p, &p->rowpos, (size_t)p->L)) return FFI_ERR_OUT_OF_MEMORY;
     {
         const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + ((size_t)threads + 2) * sizeof(unsigned short) + (size_t)TL;
-        hipError_t ea = hipFuncSetAttribute((const void*)tile_color_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const auto color = p->K <= 32 ? tile_color_kernel<32, false> : p->K <= 64 ? tile_color_kernel<64, false> : tile_color_kernel<64, true>;
+        hipError_t ea = hipFuncSetAttribute((const void*)color, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (ea != hipSuccess) return hip_fail(ea);
-        hipLaunchKernelGGL(tile_color_kernel, dim3(tiles), dim3(256), lds, s, lookup, p->L, p->K, TL, cap, threads, p->rowpos, p->col_lo,
+        hipLaunchKernelGGL(color, dim3(tiles), dim3(256), lds, s, lookup, p->L, p->K, TL, cap, threads, p->rowpos, p->col_lo,
                            sorted_columns ? 1 : 0);
     }
     if (after_row_assignment) {

@@ -288,6 +288,18 @@ def test_plans_that_sort_a_tiles_columns_by_length(ffi, shape, ids):
         assert results[1][3] <= results[-1][3]
 
 
+@pytest.mark.parametrize("fan_in", [1, 31, 32, 33, 64, 65])
+@pytest.mark.parametrize("labels", [1, 2, 3, 64, 65, 1003])
+def test_rows_of_a_tiles_labels_at_the_fan_ins_where_lanes_are_shared(ffi, fan_in, labels):
+    # a label's connections in half a wavefront, in all of it and in more than one pass; an odd last label; neighbours with the same
+    # columns, which are decided together
+    x, lookup, w, g = reference_law_inputs(20, 100, labels, fan_in, seed=labels + fan_in)
+    lookup[1::2] = lookup[0::2][: len(lookup[1::2])]
+    got_gx, got_gw = hip_backward(ffi, x, lookup, w, g, False)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    assert rel_err(got_gx, o_gx) <= GRAD_RTOL and rel_err(got_gw, o_gw) <= GRAD_RTOL
+
+
 @pytest.mark.parametrize("shape", [(300, 700, 5000, 32), (33, 96, 9, 5), (128, 512, 4100, 100), (40, 1216, 2500, 36), (64, 1100, 3000, 12),
                                    (48, 1300, 2000, 20),
                                    (96, 512, 20000, 64),     # two chunks per label, both held by one thread
