@@ -70,6 +70,11 @@ __global__ __launch_bounds__(kBlock) void fingerprint_kernel(const int32_t* __re
     }
 }
 
+__global__ __launch_bounds__(64) void guard_init_kernel(unsigned long long* __restrict__ guard, unsigned long long fingerprint) {
+    const int i = threadIdx.x;
+    if (i < 8) guard[i] = i == 3 || i == 5 ? fingerprint : i == 4 ? 1ull : 0ull;
+}
+
 __global__ __launch_bounds__(kCheckThreads) void fingerprint_guard_kernel(const LookupCheck check) {
     __shared__ CheckShared shared;
     check_block(check, blockIdx.x, shared);
@@ -124,7 +129,7 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     int* imb = color_lds;                                                        // [ncols + 1] even minus odd labels per column
     // The tile's column ids, three 10-bit ids per word, a label's ids in W = ceil(K / 3) words of its own, and the weights as
     // 16-bit numbers: with 16-bit ids and 32-bit weights a tile of 582 labels x fan-in 32 took 44 KB of LDS, three workgroups per
-    // CU and two rounds for 1,152 tiles; now 31 KB, five workgroups per CU, all tiles at once (the work of a tile is one
+    // CU and two rounds for 1,152 tiles; now 30 KB, five workgroups per CU, all tiles at once (the work of a tile is one
     // wavefront's sequential loop).
     const int W = (K + 2) / 3;
     unsigned* ids3 = reinterpret_cast<unsigned*>(color_lds + ncols + 1);         // [tile_labels * W]
@@ -170,7 +175,8 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     const int lane = threadIdx.x;
     constexpr int kAbreast = 64 / LANES;                                         // labels decided together
     const int groups = (nl + kAbreast - 1) / kAbreast, k_mine = lane & (LANES - 1), abreast = lane / LANES;
-    unsigned char* half = reinterpret_cast<unsigned char*>(wt + ncols + 2);      // [tile_labels] the half each label goes to
+    // the half a label goes to: bit 30 of its first word
+    auto half_of = [&](int jl) { return (int)(ids3[jl * W] >> 30 & 1u); };
     int placed[2] = {0, 0};
     // What bounds the kernel is the chain from one step's adds to the next step's decision: an LDS round trip, the sum over the
     // lanes by DPP and lane swaps, a comparison in every lane; what it does to the counts of placed labels is beside the chain.  Of
@@ -202,7 +208,7 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         }
     };
     // the balance that a lane's label asks for, after `back` (0: nothing) is added to its columns; then `decide` says which half
-    auto step = [&](int g, int back, auto decide) {
+    auto step = [&](int g, int had, int back, auto decide) {
         const int c = col1, w = w1;
         if (back != 0) {
             if (__builtin_expect(on, 1)) atomicAdd(&imb[c], back);
@@ -214,7 +220,7 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         const int color = decide(lanes_total<LANES>(sum)), delta = color ? -1 : 1;
         if (__builtin_expect(on, 1)) atomicAdd(&imb[c], delta);                                          // (a column may occur twice in a label)
         rest(g, [&](int q) { atomicAdd(&imb[q], delta); });
-        if (__builtin_expect(k_mine == 0 && label_of(g) < nl, 1)) half[label_of(g)] = (unsigned char)color;
+        if (k_mine == 0 && label_of(g) < nl && color != had) atomicXor(&ids3[label_of(g) * W], 1u << 30);
     };
     // where the labels of a step go once the halves may be full: `color` as far as there is room, else `other`
     auto settle = [&](int g, int color, int other, bool again) {
@@ -248,23 +254,23 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     advance(0);
     for (int g = 0; g < groups; ++g) {
         const int even = placed[1] < placed[0] ? 1 : 0;
-        step(g, 0, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : even ^ abreast), 0, false); });
+        step(g, 0, 0, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : even ^ abreast), 0, false); });
     }
     // Second sweep: every label is taken out and put back into the half its columns now ask for -- the first sweep placed
     // the early labels knowing nothing of the later ones.  (Measured on uniformly drawn ids, 586-label tiles of fan-in 32
     // over 768 columns: slot rows 1.528 -> 1.514 per connection, where columns of unconstrained order would need 1.490.)
     word2 = word_of(0);
     advance(0);
-    int next_old = half[min(label_of(0), nl - 1)];       // (written by this wavefront above, whose LDS accesses are in order)
+    int next_old = half_of(min(label_of(0), nl - 1));       // (written by this wavefront above, whose LDS accesses are in order)
     for (int g = 0; g < groups; ++g) {
         const int old = next_old;
-        next_old = half[min(label_of(g + 1), nl - 1)];
-        step(g, old ? 1 : -1, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : old), old, true); });
+        next_old = half_of(min(label_of(g + 1), nl - 1));
+        step(g, old, old ? 1 : -1, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : old), old, true); });
     }
     // rows of a half are handed out in ascending label order
     int next[2] = {0, 0};
     for (int l0 = 0; l0 < nl; l0 += 64) {
-        const bool on = l0 + lane < nl, odd = on && half[min(l0 + lane, nl - 1)] != 0;
+        const bool on = l0 + lane < nl, odd = on && half_of(min(l0 + lane, nl - 1)) != 0;
         const unsigned long long odds = __ballot(odd), evens = __ballot(on && !odd), before = (1ull << lane) - 1ull;
         if (on) rowpos[j0 + l0 + lane] = (unsigned short)(2 * (next[odd] + __popcll((odd ? odds : evens) & before)) + (odd ? 1 : 0));
         next[0] += __popcll(evens);
@@ -303,9 +309,11 @@ __device__ __forceinline__ void count_halves(const int32_t* __restrict__ src, co
 // blocks dealt to the wavefronts so that the wavefronts of a SIMD (wave, wave + 4, wave + 8, ...) have about the same
 // rows in total: longest block first, each to the SIMD with the least so far that still has a wavefront free.
 // One workgroup per tile, one thread per column (columns up to the workgroup size exist for this purpose: the ones
-// beyond the input's width have no connections).  Bound by the comparison of every column with every other (two instructions
-// each) and the dealing, which four lanes do for the four SIMDs: 670,091 labels over 768 columns 157 -> 83 us.  Also stores the slot rows of each slice, as tile_count_kernel does
+// beyond the input's width have no connections).  Sorted by counting; the dealing is done by four lanes for the four SIMDs.  Bound by
+// the counting of the connections: 670,091 labels over 768 columns 157 us, 85 with four lanes dealing, 58 with no comparison of
+// every column with every other.  Also stores the slot rows of each slice, as tile_count_kernel does
 // for plans without the permutation.  LDS: counts [2][threads], keys [threads].
+constexpr int kPermLengths = 512;            // sorted by counting up to here
 __global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
                                  int tile_labels, int col_lo, unsigned short* __restrict__ colperm, unsigned* __restrict__ slice_len) {
     extern __shared__ __align__(16) unsigned perm_lds[];
@@ -314,31 +322,65 @@ __global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned
     unsigned* key = cnt + 2 * nthreads;        // [threads]
     __shared__ unsigned short wave_of_block[16];
     __shared__ unsigned slice_rows[16];
+    __shared__ __align__(16) unsigned char of_wave[16][kPermLengths];     // columns of each length in a wavefront
+    __shared__ unsigned longer[kPermLengths];                             // columns of greater length
     if (threadIdx.x < 16) slice_rows[threadIdx.x] = 0u;
+    for (int i = threadIdx.x; i < nslices * kPermLengths / 16; i += nthreads) reinterpret_cast<uint4*>(of_wave)[i] = make_uint4(0u, 0u, 0u, 0u);
     cnt[threadIdx.x] = 0;
     cnt[nthreads + threadIdx.x] = 0;
     __syncthreads();
     const int j0 = t * tile_labels;
     count_halves(idx + (size_t)j0 * K, rowpos + j0, min(tile_labels, L - j0) * K, K, col_lo, cnt);
     __syncthreads();
-    // (the slots a column needs depend by one on the lane it gets; the larger of the two)
-    // (with the column below it, so that no two keys are equal: columns of equal length stay in index order)
-    const unsigned mine = 2u * max(cnt[threadIdx.x], cnt[nthreads + threadIdx.x]) * 1024u + (1023u - threadIdx.x);
-    key[threadIdx.x] = mine;
-    __syncthreads();
-    // place among the columns in descending order of the key
+    // (the slots a column needs depend by one on the lane it gets; the larger of the two; columns of equal length stay in index order)
+    const unsigned length = max(cnt[threadIdx.x], cnt[nthreads + threadIdx.x]);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // place among the columns in descending order of the length: the longer ones, the equal ones of the wavefronts before, the equal
+    // ones of the lanes before
     unsigned place = 0;
-#pragma unroll 4
-    for (int c0 = 0; c0 < nthreads; c0 += 4) {
-        const uint4 k4 = *reinterpret_cast<const uint4*>(key + c0);       // (the same address in every lane: one broadcast read)
-        place += k4.x > mine ? 1u : 0u;
-        place += k4.y > mine ? 1u : 0u;
-        place += k4.z > mine ? 1u : 0u;
-        place += k4.w > mine ? 1u : 0u;
+    if (!__syncthreads_or(length >= (unsigned)kPermLengths)) {
+        unsigned long long equal = ~0ull;
+#pragma unroll
+        for (int bit = 1; bit < kPermLengths; bit <<= 1) {
+            const unsigned long long set = __ballot((length & bit) != 0u);
+            equal &= (length & bit) != 0u ? set : ~set;
+        }
+        const unsigned below = (unsigned)__popcll(equal & ((1ull << lane) - 1ull));
+        if (below == 0u) of_wave[wave][length] = (unsigned char)__popcll(equal);      // (at most 64)
+        __syncthreads();
+        for (int n = threadIdx.x; n < kPermLengths; n += nthreads) {
+            unsigned all = 0;
+            for (int v = 0; v < nslices; ++v) all += of_wave[v][n];
+            longer[n] = all;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            constexpr int kPer = kPermLengths / 64;
+            unsigned n[kPer], sum = 0;
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) { n[i] = longer[lane * kPer + i]; sum += n[i]; }
+            unsigned from = sum;                                          // columns of this lane's lengths and of longer ones
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned above = __shfl_down(from, off, 64);
+                if (lane + off < 64) from += above;
+            }
+            from -= sum;
+#pragma unroll
+            for (int i = kPer - 1; i >= 0; --i) { longer[lane * kPer + i] = from; from += n[i]; }
+        }
+        __syncthreads();
+        place = longer[length] + below;
+        for (int v = 0; v < wave; ++v) place += of_wave[v][length];
+    } else {
+        // (lengths that few tiles have: every column compared with every other)
+        key[threadIdx.x] = length;
+        __syncthreads();
+        for (int c = 0; c < nthreads; ++c) place += key[c] > length || (key[c] == length && c < (int)threadIdx.x) ? 1u : 0u;
+        __syncthreads();
     }
-    __syncthreads();
     // key[] now by place: the first of each block of 64 is the block's longest column
-    key[place] = mine / 1024u;
+    key[place] = 2u * length;
     __syncthreads();
     if (threadIdx.x < 64) {
         // (four lanes are the SIMDs: their sums so far, wavefronts handed out)
@@ -385,298 +427,224 @@ __global__ void tile_count_kernel(const int32_t* __restrict__ idx, const unsigne
     if ((threadIdx.x & 63) == 0) slice_len[(size_t)t * (nthreads >> 6) + (threadIdx.x >> 6)] = c;
 }
 
-// Exclusive prefix sum of n values into off[0..n] by one workgroup (n is a few thousand; 25 us with the
-// threads' sums added up by one of them, 15 so).
+// Exclusive prefix sum of n values into off[0..n] by one workgroup, and with `group` the largest sum of `group` consecutive ones
+// from a multiple of it on, both to the host's memory (n is a few thousand; 25 us with the threads' sums added up by one of them,
+// 15 with a thread's values asked for one by one, 13 so, 3 of them the largest sum).
 __global__ __launch_bounds__(1024) void slice_scan_kernel(const unsigned* __restrict__ len, unsigned* __restrict__ off,
-                                                           int n, unsigned long long* __restrict__ total_out) {
+                                                           int n, int group, unsigned long long* __restrict__ total_out) {
+    constexpr int kAtOnce = 16;
     const int per = (n + 1023) / 1024;
     const int b = min((int)threadIdx.x * per, n), e = min(b + per, n);
     unsigned long long sum = 0, total = 0;
-    for (int i = b; i < e; ++i) sum += len[i];
+    unsigned v[kAtOnce];                                                  // (the last ones asked for stay)
+    auto ask = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) v[i] = i0 + i < e ? len[i0 + i] : 0u;
+    };
+    for (int i0 = b; i0 < e; i0 += kAtOnce) {
+        ask(i0);
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) sum += v[i];
+    }
     unsigned long long run = block_sum_below<1024>(sum, &total);
-    for (int i = b; i < e; ++i) { off[i] = (unsigned)run; run += len[i]; }
+    for (int i0 = b; i0 < e; i0 += kAtOnce) {
+        if (per > kAtOnce) ask(i0);
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            if (i0 + i < e) off[i0 + i] = (unsigned)run;
+            run += v[i];
+        }
+    }
     if (threadIdx.x == 1023) {
         off[n] = (unsigned)total;
         *total_out = total;
     }
+    if (group <= 0) return;
+    __shared__ unsigned longest;
+    if (threadIdx.x == 0) longest = 0u;
+    __syncthreads();                                                      // (off[] as well)
+    unsigned most = 0u;
+    for (int t = threadIdx.x; t < n / group; t += 1024) most = max(most, off[(t + 1) * group] - off[t * group]);
+    atomicMax(&longest, most);
+    __syncthreads();
+    if (threadIdx.x == 0) total_out[1] = longest;
 }
 
-// One workgroup per label tile, one thread per column n.  The tile's column ids pass through LDS
-// in chunks; every thread scans them in flat-position order and places the ones equal to its
-// column (see column_slots for the order), so the result is deterministic without any sort.
+// Slots of a tile, one workgroup per tile; its wavefronts take consecutive stretches of the tile's connections.
 // Per slot: lab16 = LDS row of the label (rowpos), pos16 = position inside the tile's rows of lookup; the
 // slots a column leaves empty up to the slice's length become padding: pos16 = pad_pos (kPadPos; in plans whose walking
 // kernel keeps the tile's weights in LDS, tile_labels * K: the position of a zero word behind them), lab16 =
 // zero_row + parity (all-zero rows).
-constexpr int kFillChunk = 8192;
 // With `slot32` (plans whose walking kernel keeps the tile's weights in LDS) the two go into one word per slot,
 // (position << 17) | (LDS row << 7): one load per slot, the row's byte offset already in place.
-__global__ void tile_fill_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
-                                 int tile_labels, int zero_row, const unsigned* __restrict__ slice_off,
-                                 unsigned short* __restrict__ lab16, unsigned short* __restrict__ pos16, unsigned pad_pos,
-                                 unsigned* __restrict__ slot32, int col_lo, const unsigned short* __restrict__ colperm) {
-    __shared__ __align__(16) int keys[kFillChunk];
-    __shared__ unsigned short rows_of[kPlanTileLabels];     // LDS row of each label of the tile
-    const int t = blockIdx.x, nthreads = blockDim.x;
-    const int j0 = t * tile_labels;
-    const int nl = min(tile_labels, L - j0);
-    const int* src = idx + (size_t)j0 * K;
-    const int total = nl * K;
-    const int mine = (colperm != nullptr ? (int)colperm[(size_t)blockIdx.x * blockDim.x + threadIdx.x] : (int)threadIdx.x) + col_lo;
-    const size_t sl = (size_t)t * (nthreads >> 6) + (threadIdx.x >> 6);
-    const size_t row0 = slice_off[sl];
-    const unsigned rows = slice_off[sl + 1] - slice_off[sl];
-    const size_t at = row0 * 64 + (threadIdx.x & 63);
-    auto put = [&](size_t r, unsigned lab, unsigned pos) {
-        if (slot32 != nullptr) slot32[at + r * 64] = (pos << 17) | (lab << 7);
-        else { lab16[at + r * 64] = (unsigned short)lab; pos16[at + r * 64] = (unsigned short)pos; }
-    };
-    const unsigned first = parity_first(threadIdx.x);
-    for (int i = threadIdx.x; i < nl; i += nthreads) rows_of[i] = rowpos[j0 + i];
-    // padding everywhere first; the thread's own slots are then overwritten (same thread: ordered)
-    for (unsigned r = 0; r < rows; ++r) {
-        put(r, (unsigned)zero_row + ((r & 1u) ^ first), pad_pos);
-    }
-    unsigned seen[2] = {0u, 0u};  // labels of each parity placed so far
-    int label = 0, kk = 0;        // label and connection slot of the entry under the cursor
-    for (int c0 = 0; c0 < total; c0 += kFillChunk) {
-        const int n = min(kFillChunk, total - c0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < n; e += nthreads) keys[e] = src[c0 + e];
-        __syncthreads();
-        for (int e = 0; e < n; ++e) {
-            if (keys[e] == mine) {
-                const unsigned row = rows_of[label];
-                const unsigned par = row & 1u;
-                const unsigned t2 = par ? seen[1]++ : seen[0]++;
-                const unsigned slot = 2u * t2 + (par ^ first);
-                put(slot, row, (unsigned)(c0 + e));
-            }
-            if (++kk == K) { kk = 0; ++label; }
-        }
-    }
-}
-
-// The same placement without the all-pairs scan, for tiles whose column ids, a bitmap [column][label of the tile]
-// and its prefix counts fit in LDS together (every tile of a narrow layer at the fan-ins the weights-in-LDS form
-// takes).  Every connection sets the bit of (its column, its label) -- integer OR, order-independent; every column's
-// thread then counts, word by word of its bitmap row, the labels in even and in odd LDS rows before that word; and
-// every connection finds its own slot from those counts and the bits below its own (its rank among the column's
-// connections of the same bank half in ascending flat position: the order tile_fill_kernel produces), so the slots
-// are written by threads <-> connections, not by a column's thread scanning for them.  Padding goes to the slots no
-// connection takes (a column's thread knows them from its two totals).  A label that lists one column twice sets one
-// bit for two connections -- sources drawn with replacement do so all the time, two labels in five at fan-in 32 over 768
-// columns.  The connections that find their bit set are kept in chains, one per column, and a connection's rank then counts
-// the chain's entries in front of it too.  A chain is 0.5 entries on average there; beyond dup_cap entries in a tile (four per
-// column, or what LDS is left) the columns' threads place the tile (see below).
-// Measured at 670,091 labels x fan-in 32 over 768 columns: 6.2 ms by the scan of all pairs, 0.83 ms by the columns' threads
-// (0.19 without labels that list a column twice), 0.21 by chains (0.26 where every connection looked through its label's row
-// for the equal ids in front of it); 501,070 labels x fan-in 64 over 512 columns: 0.66 by chains (0.97).
-__global__ void tile_fill_bitmap_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
-                                        int tile_labels, int zero_row, const unsigned* __restrict__ slice_off,
-                                        unsigned short* __restrict__ lab16, unsigned short* __restrict__ pos16, unsigned pad_pos,
-                                        unsigned* __restrict__ slot32, int words, int col_lo,
-                                        const unsigned short* __restrict__ colperm, unsigned dup_cap) {
+// Every wavefront counts its connections per column and bank half; sums over the wavefronts turn the counts into the slots that
+// each wavefront's first connection of a column and half goes to (see column_slots), counted from the tile's first; then the wavefronts
+// walk their stretches again, 64 connections at a time, and each takes the slot it finds and leaves the next one there.  Slots are
+// in the order of flat positions: of several connections of one column and half among 64, which find what one of the others has
+// already moved on, the lanes' order decides, not the LDS's.
+// STAGED: the tile's positions gather in LDS and leave in whole rows; the next form, for tiles that do not fit there or whose
+// slots 16 bits do not number, counts ranks and writes slots where they belong.
+// Bound by the LDS's atomics and the latency of the walk.  Written where they belong one by one, slots are bound by the L2's write
+// requests instead.  670,091 labels x fan-in 32 over 768 columns 216 -> 129 us, against bitmaps of labels per column with chains for
+// labels that list a column twice, slots written one by one; 501,070 x 64 over 512 772 -> 171; tiles that had no room for the bitmaps,
+// or more such labels than the chains held, were scanned: 200,000 x 40 over 1,000 4,392 -> 76, 300,000 x 16 over 768 2,254 -> 288 (all
+// of the build).
+constexpr int kFillThreads = 1024;
+constexpr unsigned kFillRows = 1021;         // (a slot of its last row and 128 more are below 2^16)
+template <bool STAGED>
+__global__ __launch_bounds__(kFillThreads) void tile_fill_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
+                                                                 int tile_labels, int zero_row, const unsigned* __restrict__ slice_off,
+                                                                 unsigned short* __restrict__ lab16, unsigned short* __restrict__ pos16, unsigned pad_pos,
+                                                                 unsigned* __restrict__ slot32, int col_lo, const unsigned short* __restrict__ colperm,
+                                                                 int ncols, unsigned stage_rows) {
     extern __shared__ __align__(16) unsigned fill_lds[];
-    const int t = blockIdx.x, nthreads = blockDim.x;
-    unsigned* bm = fill_lds;                                                   // [nthreads][words] (words odd: no bank conflicts)
-    unsigned* pm = bm + (size_t)nthreads * words;                              // [words] labels staged in odd LDS rows
-    unsigned* heads = pm + words;                                              // [nthreads] first entry of the column's chain
-    unsigned* chain = heads + nthreads;                                        // [dup_cap] connection | half of its label's row << 16 | next entry << 17
-    unsigned short* pre = reinterpret_cast<unsigned short*>(chain + dup_cap);  // [nthreads][words][2] labels before word w, even / odd rows
-    unsigned short* rows_of = pre + (size_t)nthreads * words * 2;              // [tile_labels]
-    unsigned short* ids = rows_of + ((tile_labels + 1) & ~1);                  // [tile_labels * K]
-    unsigned short* thread_of = ids + (((size_t)tile_labels * K + 1) & ~(size_t)1);   // [nthreads] the thread that walks each column
-    __shared__ unsigned duplicates;
-    __shared__ unsigned deep;
-    constexpr unsigned kNoEntry = 0x7fffu, kColumn = 0x3ffu, kMaxRank = 61u;
-    // (bitmap and prefix counts are kept per column; slices, lanes and slot parities belong to threads)
-    const unsigned mycol = colperm != nullptr ? colperm[(size_t)blockIdx.x * blockDim.x + threadIdx.x] : threadIdx.x;
-    thread_of[mycol] = (unsigned short)threadIdx.x;
-    const int j0 = t * tile_labels;
-    const int nl = min(tile_labels, L - j0);
-    const int* src = idx + (size_t)j0 * K;
+    constexpr int kInflight = 8;
+    constexpr unsigned kNone = 0xffffu;                                   // (no position: a tile has fewer than 2^16 - 1 connections)
+    const int t = blockIdx.x, nthreads = blockDim.x, nwaves = nthreads >> 6, nslices = ncols >> 6;
+    const unsigned* const offs = slice_off + (size_t)t * nslices;         // [nslices + 1]
+    const unsigned tile_row0 = offs[0], tile_rows = offs[nslices] - tile_row0;
+    const bool staged = tile_rows <= stage_rows;                          // (stage_rows <= kFillRows)
+    if (staged != STAGED) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned short* const stage = reinterpret_cast<unsigned short*>(fill_lds);        // [stage_rows][64] positions
+    unsigned* const base_of = fill_lds;                                   // (not staged: [ncols] a column's first slot << 1 | half that even slots hold)
+    unsigned* const counts = fill_lds + (STAGED ? (size_t)stage_rows * 32 : (size_t)ncols);     // [wave][ncols] for labels in even rows | in odd rows << 16
+    unsigned short* const row_of = reinterpret_cast<unsigned short*>(counts + (size_t)nwaves * ncols);          // [tile_labels]
+    unsigned* const mine = counts + (size_t)wave * ncols;
+    const int j0 = t * tile_labels, nl = min(tile_labels, L - j0);
     const int total = nl * K;
-    const int nslices = nthreads >> 6;
-    if (threadIdx.x == 0) { duplicates = 0u; deep = 0u; }
-    heads[threadIdx.x] = kNoEntry;
-    for (int i = threadIdx.x; i < nthreads * words; i += nthreads) bm[i] = 0u;
-    for (int i = threadIdx.x; i < words; i += nthreads) pm[i] = 0u;
-    for (int i = threadIdx.x; i < nl; i += nthreads) rows_of[i] = rowpos[j0 + i];
-    for (int e = threadIdx.x; e < total; e += nthreads) {
-        const unsigned c = (unsigned)(src[e] - col_lo);                       // (columns outside the plan's window: never matched)
-        ids[e] = c < (unsigned)nthreads ? (unsigned short)c : (unsigned short)0xffffu;
-    }
+    const int* src = idx + (size_t)j0 * K;
+    for (int i = threadIdx.x; i < nwaves * ncols; i += nthreads) counts[i] = 0u;
+    for (int i = threadIdx.x; i < nl; i += nthreads) row_of[i] = rowpos[j0 + i];
+    if (STAGED)
+        for (unsigned i = threadIdx.x; i < tile_rows * 8u; i += nthreads) reinterpret_cast<uint4*>(stage)[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
     __syncthreads();
-    for (int i = threadIdx.x; i < nl; i += nthreads)
-        if (rows_of[i] & 1u) atomicOr(&pm[i >> 5], 1u << (i & 31));
-    {
-        // (label of entry e without a division per entry: the thread's entries are nthreads apart)
-        int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
-        const int dl = nthreads / K, dk = nthreads - dl * K;
-        for (int e = threadIdx.x; e < total; e += nthreads) {
-            const unsigned c = ids[e];
-            if (c < (unsigned)nthreads) {
-                const unsigned bit = 1u << (l & 31);
-                if (atomicOr(&bm[(size_t)c * words + (l >> 5)], bit) & bit) {
-                    const unsigned at = atomicAdd(&duplicates, 1u);
-                    if (at < dup_cap) chain[at] = (unsigned)e | (rows_of[l] & 1u) << 16 | atomicExch(&heads[c], at) << 17;
-                }
+    // this wavefront's connections, kInflight x 64 at a time: visit(column or ~0, LDS row of the label, position)
+    const float per_label = 1.f / (float)K;
+    auto label_at = [&](unsigned e) { return (unsigned)(((float)e + 0.5f) * per_label); };         // e / K for e < 2^16
+    const int stretch = ((total + nwaves - 1) / nwaves + 63) & ~63, e_begin = min(wave * stretch, total), e_end = min(e_begin + stretch, total);
+    auto walk = [&](auto visit) {
+        unsigned next[kInflight];
+        auto fetch = [&](int e0) {
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i) {
+                const int e = e0 + 64 * i + lane;
+                next[i] = e < e_end ? (unsigned)(src[e] - col_lo) : ~0u;  // (columns outside the plan's window: no thread's)
             }
-            l += dl; k += dk;
-            if (k >= K) { k -= K; ++l; }
-        }
-    }
-    __syncthreads();
-    // The rank of a chained connection among the equal ones of its label: one of them is not in the chain (which one, the order
-    // of the atomics decides), so the label's row is looked through.  It is kept, plus one, above the ten bits of its column.
-    // The one that is not chained finds all that are in front of it in the chain.
-    const bool chained = duplicates <= dup_cap;
-    if (chained) {
-        for (unsigned i = threadIdx.x; i < duplicates; i += nthreads) {
-            const unsigned e = chain[i] & 0xffffu, l = e / (unsigned)K, c = ids[e];
-            const unsigned short* row_ids = ids + l * K;
-            unsigned before = 0;
-#pragma unroll 8
-            for (unsigned q = 0; q < e - l * K; ++q) before += (row_ids[q] & kColumn) == c ? 1u : 0u;
-            if (before > kMaxRank) deep = 1u;
-            else ids[e] = (unsigned short)(c | (before + 1u) << 10);
-        }
-    }
-    __syncthreads();
-    if (deep) {
-        for (int e = threadIdx.x; e < total; e += nthreads)
-            if (ids[e] != 0xffffu) ids[e] &= kColumn;
-        __syncthreads();
-    }
-    if (!chained || deep) {
-        // (uniform) more such connections than the chains hold: the column's thread walks its bitmap row in ascending label order and scans each
-        // label found for the matching connections, which yields every connection, in ascending flat position
-        const unsigned mine = mycol;
-        const size_t sl = (size_t)t * nslices + (threadIdx.x >> 6);
-        const size_t row0 = slice_off[sl];
-        const unsigned rows = slice_off[sl + 1] - slice_off[sl];
-        const size_t at = row0 * 64 + (threadIdx.x & 63);
-        auto put = [&](size_t r, unsigned lab, unsigned pos) {
-            if (slot32 != nullptr) slot32[at + r * 64] = (pos << 17) | (lab << 7);
-            else { lab16[at + r * 64] = (unsigned short)lab; pos16[at + r * 64] = (unsigned short)pos; }
         };
-        const unsigned first = parity_first(threadIdx.x);
-        // padding everywhere first; the thread's own slots are then overwritten (same thread: ordered)
-        for (unsigned r = 0; r < rows; ++r) put(r, (unsigned)zero_row + ((r & 1u) ^ first), pad_pos);
-        unsigned seen[2] = {0u, 0u};
-        const unsigned* my = bm + (size_t)mine * words;
-        for (int wd = 0; wd < words; ++wd) {
-            unsigned bits = my[wd];
-            while (bits) {
-                const unsigned b = (unsigned)__builtin_ctz(bits);
-                bits &= bits - 1u;
-                const unsigned l = 32u * (unsigned)wd + b;
-                const unsigned row = rows_of[l];
-                const unsigned par = row & 1u;
-                const unsigned short* lrow = ids + (size_t)l * K;
-                auto found = [&](int k) {
-                    const unsigned t2 = par ? seen[1]++ : seen[0]++;
-                    put(2u * t2 + (par ^ first), row, l * (unsigned)K + (unsigned)k);
-                };
-                if ((K & 7) == 0 && ((size_t)lrow & 3) == 0) {
-                    // eight ids per step, as four words whose halves are compared with the column at once: a half is
-                    // equal where (x ^ pattern) has a zero half (the classic "has a zero byte" test, for 16-bit lanes)
-                    const unsigned* lrow2 = reinterpret_cast<const unsigned*>(lrow);
-                    const unsigned pattern = mine * 0x00010001u;
-                    for (int k = 0; k < K; k += 8) {
-                        unsigned x[4];
+        fetch(e_begin);
+        for (int e0 = e_begin; e0 < e_end; e0 += 64 * kInflight) {
+            unsigned c[kInflight], row[kInflight];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) x[i] = lrow2[(k >> 1) + i] ^ pattern;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            if (((x[i] - 0x00010001u) & ~x[i] & 0x80008000u) != 0u) {
-                                if ((x[i] & 0xffffu) == 0u) found(k + 2 * i);
-                                if ((x[i] >> 16) == 0u) found(k + 2 * i + 1);
-                            }
-                        }
-                    }
-                } else {
-                    for (int k = 0; k < K; ++k)
-                        if (lrow[k] == mine) found(k);
-                }
+            for (int i = 0; i < kInflight; ++i) {
+                c[i] = next[i];
+                row[i] = row_of[label_at((unsigned)min(e0 + 64 * i + lane, e_end - 1))];
             }
+            fetch(e0 + 64 * kInflight);
+            visit(c, row, (unsigned)(e0 + lane));
         }
-        return;
-    }
-    // per column: labels in even / odd rows before each word; then the column's padding slots
-    {
-        const unsigned mine = mycol;
-        const unsigned* my = bm + (size_t)mine * words;
-        unsigned short* mp = pre + (size_t)mine * words * 2;
-        unsigned ev = 0, od = 0;
-        for (int wd = 0; wd < words; ++wd) {
-            mp[2 * wd] = (unsigned short)ev; mp[2 * wd + 1] = (unsigned short)od;
-            const unsigned b = my[wd], o = pm[wd];
-            ev += __builtin_popcount(b & ~o); od += __builtin_popcount(b & o);
+    };
+    walk([&](const unsigned* c, const unsigned* row, unsigned) {
+#pragma unroll
+        for (int i = 0; i < kInflight; ++i)
+            if (c[i] < (unsigned)ncols) atomicAdd(&mine[c[i]], (row[i] & 1u) ? 0x10000u : 1u);
+    });
+    __syncthreads();
+    const size_t tile_slot0 = (size_t)tile_row0 * 64;
+    auto put = [&](size_t slot, unsigned lab, unsigned pos) {
+        const size_t at = tile_slot0 + slot;
+        if (slot32 != nullptr) slot32[at] = (pos << 17) | (lab << 7);
+        else { lab16[at] = (unsigned short)lab; pos16[at] = (unsigned short)pos; }
+    };
+    for (int walker = threadIdx.x; walker < ncols; walker += nthreads) {
+        // (counts are kept per column; slices, lanes and slot parities belong to the threads that walk the plan)
+        const unsigned col = colperm != nullptr ? colperm[(size_t)t * ncols + walker] : walker;
+        const int sl = wave + (walker - (int)threadIdx.x) / 64;
+        const unsigned first = parity_first(walker), base = (offs[sl] - tile_row0) * 64u + (unsigned)lane;
+        unsigned run = STAGED ? (base + first * 64u) | (base + (first ^ 1u) * 64u) << 16 : 0u;
+        for (int v = 0; v < nwaves; ++v) {
+            const unsigned n = counts[(size_t)v * ncols + col];
+            counts[(size_t)v * ncols + col] = run;
+            run += STAGED ? n * 128u : n;                                 // (the next slot of a half is two rows on; both halves stay below 2^16)
         }
-        const size_t sl = (size_t)t * nslices + (threadIdx.x >> 6);
-        const size_t row0 = slice_off[sl];
-        const unsigned rows = slice_off[sl + 1] - slice_off[sl];
-        const size_t at = row0 * 64 + (threadIdx.x & 63);
-        const unsigned first = parity_first(threadIdx.x);
-        for (unsigned h = heads[mine]; h != kNoEntry;) {
-            const unsigned entry = chain[h];
-            if (entry & 0x10000u) ++od;
-            else ++ev;
-            h = entry >> 17;
-        }
-        const unsigned cnt[2] = {ev, od};
-        for (unsigned r = 0; r < rows; ++r) {
-            const unsigned par = (r & 1u) ^ first;          // bank half this slot belongs to
-            if ((r >> 1) >= cnt[par]) {
-                const unsigned lab = (unsigned)zero_row + par;
-                if (slot32 != nullptr) slot32[at + (size_t)r * 64] = (pad_pos << 17) | (lab << 7);
-                else { lab16[at + (size_t)r * 64] = (unsigned short)lab; pos16[at + (size_t)r * 64] = (unsigned short)pad_pos; }
+        if (!STAGED) {
+            base_of[col] = base << 1 | first;                             // (rows < 2^24)
+            const unsigned cnt[2] = {run & 0xffffu, run >> 16}, rows = offs[sl + 1] - offs[sl];
+            for (unsigned r = 0; r < rows; ++r) {
+                const unsigned par = (r & 1u) ^ first;                    // bank half this slot belongs to
+                if ((r >> 1) >= cnt[par]) put((size_t)base + (size_t)r * 64, (unsigned)zero_row + par, pad_pos);
             }
         }
     }
     __syncthreads();
-    // per connection: its slot
-    {
-        int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
-        const int dl = nthreads / K, dk = nthreads - dl * K;
-        for (int e = threadIdx.x; e < total; e += nthreads) {
-            const unsigned id = ids[e], c = id & kColumn;
-            if (id != 0xffffu) {
-                const unsigned row = rows_of[l];
-                const unsigned par = row & 1u;
-                const int wd = l >> 5;
-                const unsigned o = pm[wd];
-                const unsigned same = bm[(size_t)c * words + wd] & (par ? o : ~o) & ((1u << (l & 31)) - 1u);
-                unsigned rank = pre[((size_t)c * words + wd) * 2 + par] + __builtin_popcount(same);
-                const unsigned in_label = id >> 10, front = in_label ? (unsigned)(e - k) : (unsigned)e;
-                for (unsigned h = heads[c]; h != kNoEntry;) {
-                    const unsigned entry = chain[h];
-                    rank += ((entry & 0xffffu) < front && (entry >> 16 & 1u) == par) ? 1u : 0u;
-                    h = entry >> 17;
-                }
-                rank += in_label ? in_label - 1u : 0u;
-                const unsigned thr = thread_of[c];
-                const unsigned slot = 2u * rank + (par ^ parity_first(thr));
-                const size_t at = (size_t)slice_off[(size_t)t * nslices + (thr >> 6)] * 64 + (thr & 63u) + (size_t)slot * 64;
-                if (slot32 != nullptr) slot32[at] = ((unsigned)e << 17) | (row << 7);
-                else { lab16[at] = (unsigned short)row; pos16[at] = (unsigned short)e; }
+    walk([&](const unsigned* c, const unsigned* row, unsigned e) {
+        constexpr unsigned kStep = STAGED ? 128u : 1u;
+        unsigned before[kInflight], found[kInflight];
+#pragma unroll
+        for (int i = 0; i < kInflight; ++i) {
+            before[i] = found[i] = 0u;
+            if (c[i] < (unsigned)ncols) {
+                before[i] = mine[c[i]];
+                found[i] = atomicAdd(&mine[c[i]], (row[i] & 1u) ? kStep << 16 : kStep);
             }
-            l += dl; k += dk;
-            if (k >= K) { k -= K; ++l; }
+        }
+#pragma unroll
+        for (int i = 0; i < kInflight; ++i) {
+            const bool on = c[i] < (unsigned)ncols;
+            const unsigned par = row[i] & 1u, shift = par * 16u, key = on ? c[i] * 2u + par : ~0u;
+            unsigned at = before[i] >> shift & 0xffffu;
+            for (unsigned long long left = __ballot(on && (found[i] >> shift & 0xffffu) != at); left != 0ull;) {
+                const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)key, __builtin_ctzll(left));
+                const unsigned long long same = __ballot(key == k);
+                if (key == k) at += kStep * (unsigned)__popcll(same & ((1ull << lane) - 1ull));
+                left &= ~same;
+            }
+            if (on) {
+                if (STAGED) {
+                    stage[at] = (unsigned short)(e + 64u * i);
+                } else {
+                    const unsigned base = base_of[c[i]];
+                    put((size_t)(base >> 1) + (size_t)(2u * at + (par ^ (base & 1u))) * 64, row[i], e + 64u * i);
+                }
+            }
+        }
+    });
+    if (!STAGED) return;
+    __syncthreads();
+    // eight slots of a row per lane; two wavefronts take the rows of a slice
+    for (int u = wave; u < 2 * nslices; u += nwaves) {
+        const int sl = u >> 1;
+        const unsigned begin = offs[sl] - tile_row0, len = offs[sl + 1] - offs[sl], lane8 = (unsigned)lane & 7u;
+        const unsigned first = parity_first(8u * lane8);
+        for (unsigned r = (unsigned)(u & 1) * 8u + ((unsigned)lane >> 3); r < len; r += 16u) {
+            const uint4 q = reinterpret_cast<const uint4*>(stage)[(begin + r) * 8u + lane8];
+            const unsigned w[4] = {q.x, q.y, q.z, q.w};
+            unsigned lab[8], pos[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const unsigned at = w[i / 2] >> (16 * (i & 1)) & 0xffffu;
+                const bool pad = at == kNone;
+                lab[i] = row_of[pad ? 0u : label_at(at)];
+                lab[i] = pad ? (unsigned)zero_row + ((r & 1u) ^ first) : lab[i];
+                pos[i] = pad ? pad_pos : at;
+            }
+            const size_t to = tile_slot0 + (size_t)(begin + r) * 64 + 8u * lane8;
+            if (slot32 != nullptr) {
+                uint4* out = reinterpret_cast<uint4*>(slot32 + to);
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    out[h] = make_uint4(pos[4 * h] << 17 | lab[4 * h] << 7, pos[4 * h + 1] << 17 | lab[4 * h + 1] << 7,
+                                        pos[4 * h + 2] << 17 | lab[4 * h + 2] << 7, pos[4 * h + 3] << 17 | lab[4 * h + 3] << 7);
+            } else {
+                *reinterpret_cast<uint4*>(lab16 + to) = make_uint4(lab[0] | lab[1] << 16, lab[2] | lab[3] << 16, lab[4] | lab[5] << 16, lab[6] | lab[7] << 16);
+                *reinterpret_cast<uint4*>(pos16 + to) = make_uint4(pos[0] | pos[1] << 16, pos[2] | pos[3] << 16, pos[4] | pos[5] << 16, pos[6] | pos[7] << 16);
+            }
         }
     }
 }
-
-// LDS the bitmap form needs without its chains' entries, and may have
-constexpr size_t kFillLdsLimit = 160 * 1024 - 64;
-inline size_t tile_fill_bitmap_lds(int threads, int tile_labels, int K, int* words_out) {
-    const int words = ((tile_labels + 31) / 32) | 1;
-    *words_out = words;
-    return (size_t)threads * words * sizeof(unsigned) + (size_t)words * sizeof(unsigned) +
-           (size_t)threads * words * 2 * sizeof(unsigned short) + (size_t)threads * sizeof(unsigned) + (size_t)((tile_labels + 1) & ~1) * sizeof(unsigned short) +
-           (((size_t)tile_labels * K + 1) & ~(size_t)1) * sizeof(unsigned short) + (size_t)threads * sizeof(unsigned short);
+// LDS of a workgroup, without its stage; the form that has none has the columns' slots in its place
+inline size_t tile_fill_lds(int threads, int ncols, int tile_labels) {
+    return (size_t)(threads / 64) * ncols * sizeof(unsigned) + (size_t)((tile_labels + 1) & ~1) * sizeof(unsigned short);
 }
 
 // ---- blocked global form ------------------------------------------------------------------------
@@ -841,17 +809,10 @@ int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds) 
         const size_t budget = (threads <= 256 && nbt_hint >= 2) ? kPlanLdsBudget / (size_t)(768 / threads) : kPlanLdsBudget;
         while (tw >= 64 && tiled_lds_bytes(tw, K, true) > budget) tw -= 2;
         while (tw >= 64 && (long long)tw * K >= 32768) tw -= 2;
-        // a tile the bitmap fill has the LDS for (its bitmaps grow by whole words of 32 labels) builds five times faster
-        // than one it has not; take the next smaller such tile where that costs at most a twentieth of the tile
-        int words = 0;
-        if (tw >= 64 && tile_fill_bitmap_lds(threads, tw, K, &words) > kFillLdsLimit) {
-            const int fits = tw & ~31;
-            if (fits >= 64 && fits * 20 >= tw * 19 && tile_fill_bitmap_lds(threads, fits, K, &words) <= kFillLdsLimit) tw = fits;
-        }
         // Tiles per workgroup come in whole numbers: the walking kernel runs cus / batch tiles label streams of
         // ceil(tiles / streams) tiles each, and the largest tile can leave the last stream nearly empty, or whole CUs
         // without a stream (670,091 labels in 608-label tiles: 62 streams of 18 tiles on 64 CUs' worth of workgroups).
-        // The tile shrinks to what fills every stream with that same number of tiles (582 labels there: 64 x 18); a
+        // The tile shrinks to what fills every stream with that same number of tiles (582 labels in that example: 64 x 18); a
         // smaller tile pads a little more per connection, which costs less than the idle streams.  (Workgroups that share
         // a CU are left alone: there the streams outnumber the CUs.)
         if (tw >= 64 && (threads > 256 || nbt_hint < 2)) {
@@ -908,7 +869,7 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     const int cap = tiled_rows_per_half(TL);
     if (!dev_alloc(p, &p->rowpos, (size_t)p->L)) return FFI_ERR_OUT_OF_MEMORY;
     {
-        const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + ((size_t)threads + 2) * sizeof(unsigned short) + (size_t)TL;
+        const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + ((size_t)threads + 2) * sizeof(unsigned short);
         const auto color = p->K <= 32 ? tile_color_kernel<32, false> : p->K <= 64 ? tile_color_kernel<64, false> : tile_color_kernel<64, true>;
         hipError_t ea = hipFuncSetAttribute((const void*)color, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (ea != hipSuccess) return hip_fail(ea);
@@ -927,14 +888,15 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
         hipLaunchKernelGGL(tile_count_kernel, dim3(tiles), dim3(threads), 2 * threads * sizeof(unsigned), s, lookup, p->rowpos, p->L,
                            p->K, TL, slice_len, p->col_lo);
     }
+    unsigned long long* found = nullptr;                   // (slot rows, and those of the longest tile: written where the host reads them)
+    FFI_HIP_TRY(hipHostGetDevicePointer((void**)&found, p->h_scratch + 2, 0));
     hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, slice_len, p->slice_off, (int)nslices,
-                       p->d_scratch + 2);
+                       slices, found);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(p->h_scratch + 2, p->d_scratch + 2, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     dev_release(p, slice_len);
     if (e != hipSuccess) return hip_fail(e);
-    const unsigned long long rows = p->h_scratch[2];
+    const unsigned long long rows = p->h_scratch[2], longest_tile = p->h_scratch[3];
     const unsigned long long connections = (unsigned long long)p->L * p->K;
     // Too skewed (a window of the columns may have two slots per connection of the layer: how many of them fall into
     // it is not counted), or beyond what the walking kernel's 32-bit buffer offsets reach (256 bytes per row).  Lanes
@@ -951,19 +913,22 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
         return FFI_ERR_OUT_OF_MEMORY;
     }
     {
-        int words = 0;
-        size_t fill_lds = tile_fill_bitmap_lds(threads, TL, p->K, &words);
         const unsigned pad_pos = w_in_lds ? (unsigned)TL * (unsigned)p->K : kPadPos;
-        if (fill_lds <= kFillLdsLimit) {
-            const unsigned dup_cap = (unsigned)std::min<size_t>((size_t)threads * 4, (kFillLdsLimit - fill_lds) / sizeof(unsigned));
-            fill_lds += dup_cap * sizeof(unsigned);
-            hipError_t ea = hipFuncSetAttribute((const void*)tile_fill_bitmap_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds);
+        // a wavefront for each eight rounds of 64 connections, fewer where a tile's slots fit beside their counts only then;
+        // what does not fit even so is left to the other form
+        const size_t most = 160 * 1024, whole = std::min<size_t>((size_t)longest_tile, kFillRows);
+        int fill_threads = std::min(kFillThreads, std::max(1, TL * p->K / 512) * 64);
+        for (int fewer = fill_threads; fewer >= 512; fewer -= 64)
+            if (tile_fill_lds(fewer, threads, TL) + whole * 128 <= most) { fill_threads = fewer; break; }
+        const size_t counts = tile_fill_lds(fill_threads, threads, TL), stage_rows = std::min((most - counts) / 128, whole);
+        for (const bool staged : {true, false}) {
+            if (!staged && longest_tile <= stage_rows) break;
+            const auto fill = staged ? tile_fill_kernel<true> : tile_fill_kernel<false>;
+            const size_t lds = counts + (staged ? stage_rows * 128 : threads * sizeof(unsigned));
+            hipError_t ea = hipFuncSetAttribute((const void*)fill, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (ea != hipSuccess) return hip_fail(ea);
-            hipLaunchKernelGGL(tile_fill_bitmap_kernel, dim3(tiles), dim3(threads), fill_lds, s, lookup, p->rowpos, p->L, p->K, TL, 2 * cap,
-                               p->slice_off, p->lab16, p->pos16, pad_pos, p->slot32, words, p->col_lo, p->colperm, dup_cap);
-        } else {
-            hipLaunchKernelGGL(tile_fill_kernel, dim3(tiles), dim3(threads), 0, s, lookup, p->rowpos, p->L, p->K, TL, 2 * cap, p->slice_off,
-                               p->lab16, p->pos16, pad_pos, p->slot32, p->col_lo, p->colperm);
+            hipLaunchKernelGGL(fill, dim3(tiles), dim3(fill_threads), lds, s, lookup, p->rowpos, p->L, p->K, TL, 2 * cap, p->slice_off,
+                               p->lab16, p->pos16, pad_pos, p->slot32, p->col_lo, p->colperm, threads, (unsigned)stage_rows);
         }
     }
     e = hipGetLastError();
@@ -1082,7 +1047,7 @@ int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     unsigned long long* total_octs = nullptr;
     FFI_HIP_TRY(hipHostGetDevicePointer((void**)&total_octs, p->h_scratch, 0));
     hipLaunchKernelGGL(list_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, key_ws, total, (int)nkeys, ptr, block_octs);
-    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, block_octs, octs_before, (int)list_blocks, total_octs);
+    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, block_octs, octs_before, (int)list_blocks, 0, total_octs);
     hipLaunchKernelGGL(oct_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, ptr, (int)nkeys, octs_before, p->oct_ptr);
     FFI_HIP_TRY(hipGetLastError());
     FFI_HIP_TRY(hipStreamSynchronize(s));
@@ -1306,9 +1271,6 @@ int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     }
     p->lookup = lookup;
     p->fingerprint = fp;
-    // what the device-side check compares with; the build has synchronised, no check of this plan is in flight
-    const unsigned long long guard_init[8] = {0, 0, 0, fp, 1, fp, 0, 0};
-    FFI_HIP_TRY(hipMemcpy(p->d_guard, guard_init, sizeof(guard_init), hipMemcpyHostToDevice));
     // checks enqueued before this build (all finished: the build synchronises) are of no interest any more
     p->guard_seen = p->guard_seq;
     p->guard_stale = false;
@@ -1324,6 +1286,9 @@ int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigne
     // a rebuild replaces the arrays: whatever still reads the old ones must have drained
     if (!p->owned.empty()) FFI_HIP_TRY(hipDeviceSynchronize());
     free_arrays(p, true);                      // (their buffers serve the new arrays where they fit)
+    // what the device-side check compares with: no check of this plan is in flight, and the build waits for the stream
+    hipLaunchKernelGGL(guard_init_kernel, dim3(1), dim3(64), 0, s, p->d_guard, fp);
+    FFI_HIP_TRY(hipGetLastError());
     // The arranged ids of the weight gradient depend on the lookup alone: their kernel runs on a helper stream beside
     // the kernels of the tiled form (of which the longest runs one wavefront per tile and leaves the memory system idle).
     // (ids < 2^11 and an [N][32] fp32 tile in LDS: the shapes the narrow weight-gradient kernel takes)

@@ -300,6 +300,37 @@ def test_rows_of_a_tiles_labels_at_the_fan_ins_where_lanes_are_shared(ffi, fan_i
     assert rel_err(got_gx, o_gx) <= GRAD_RTOL and rel_err(got_gw, o_gw) <= GRAD_RTOL
 
 
+@pytest.mark.parametrize("shape", [(9, 1000, 1100, 60),       # a tile whose slots are written one by one, beside a short one that is staged
+                                   (9, 1000, 1100, 40),       # staged, with fewer wavefronts
+                                   (40, 768, 1300, 32), (8, 320, 700, 3),
+                                   (5, 3, 200, 9),            # every connection of a label has company in its column
+                                   (6, 700, 500, 257)])
+@pytest.mark.parametrize("ids", ["uniform", "one_column", "rising"])
+def test_slots_of_a_tile_in_flat_order(ffi, shape, ids):
+    # connections of one column among the 64 that a wavefront places at a time; columns longer than the counting sort takes; rebuilt
+    # twice: the same plan, thus the same bits
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=N + K)
+    if ids == "one_column":
+        lookup[:, : (K + 2) // 3] = N // 2
+    elif ids == "rising":
+        lookup = ((np.arange(L)[:, None] * K + np.arange(K)[None, :]) // 5 % N).astype(np.int32)
+    lib = ffi._lib.lib()
+    dl, dw, dg = dev(lookup), dev(w), dev(g)
+    runs = []
+    plan = ctypes.c_void_p()
+    ffi._lib.check(lib.ffi_plan_create(dl.data_ptr(), L, K, N, B, stream(), ctypes.byref(plan)))
+    for _ in range(3):
+        gx = torch.full((B, N), float("nan"), device="cuda")
+        ffi._lib.check(lib.ffi_input_grad_planned_f32(plan, dw.data_ptr(), dg.data_ptr(), gx.data_ptr(), B, 0, stream()))
+        torch.cuda.synchronize()
+        runs.append(gx.cpu().numpy())
+        ffi._lib.check(lib.ffi_plan_refresh(plan, dl.data_ptr(), stream()))
+    ffi._lib.check(lib.ffi_plan_destroy(plan))
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+    assert rel_err(runs[0], oracle.input_grad(x, lookup, w, g)) <= GRAD_RTOL
+
+
 @pytest.mark.parametrize("shape", [(300, 700, 5000, 32), (33, 96, 9, 5), (128, 512, 4100, 100), (40, 1216, 2500, 36), (64, 1100, 3000, 12),
                                    (48, 1300, 2000, 20),
                                    (96, 512, 20000, 64),     # two chunks per label, both held by one thread
