@@ -839,7 +839,8 @@ namespace {
 // Builds the tiled form.  Returns FFI_OK with p->tiled == false if the padded size would exceed
 // three times the connection count, lanes without a column aside (heavily skewed column usage): the caller then builds the
 // global form instead.
-// (`after_row_assignment`, may be empty: called once the kernel that assigns the labels' LDS rows is enqueued -- it takes
+// (`after_row_assignment`, may be empty: called once the kernel that assigns the labels' LDS rows is enqueued, and before any that relies
+// on the ids' range -- it takes
 // nearly all of every CU's LDS for itself, and work for another stream enqueued behind it starts when it ends instead of
 // halving the number of its workgroups that fit)
 int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::function<int()>& after_row_assignment = {}) {
@@ -1280,15 +1281,28 @@ int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
 
 namespace {
 int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigned long long* fp_out) {
-    unsigned long long fp = 0, bad = 0;
-    FFI_TRY(plan_fingerprint(p, lookup, s, &fp, &bad));
-    if (bad != 0) return FFI_ERR_BAD_LOOKUP;   // also keeps the build kernels' LDS counters in range
     // a rebuild replaces the arrays: whatever still reads the old ones must have drained
     if (!p->owned.empty()) FFI_HIP_TRY(hipDeviceSynchronize());
     free_arrays(p, true);                      // (their buffers serve the new arrays where they fit)
-    // what the device-side check compares with: no check of this plan is in flight, and the build waits for the stream
-    hipLaunchKernelGGL(guard_init_kernel, dim3(1), dim3(64), 0, s, p->d_guard, fp);
-    FFI_HIP_TRY(hipGetLastError());
+    // The ids are checked, and the words that later checks compare with are set, beside the kernel that assigns the labels' rows, which
+    // takes any ids: the others' LDS counters want them in range.  (A rewiring and the pass behind it at 128 x 768 x 670,091
+    // x 32: 1,280 us with the host waiting before that kernel, 1,252 so.)
+    FFI_TRY(plan_fingerprint_begin(p, lookup, s));
+    bool checked = false;
+    auto check_ids = [&]() -> int {
+        if (checked) return FFI_OK;
+        checked = true;
+        unsigned long long bad = 0;
+        FFI_TRY(plan_fingerprint_end(p, fp_out, &bad));
+        if (bad != 0) {
+            FFI_HIP_TRY(hipStreamSynchronize(s));
+            return FFI_ERR_BAD_LOOKUP;
+        }
+        // no check of this plan is in flight, and the build waits for the stream
+        hipLaunchKernelGGL(guard_init_kernel, dim3(1), dim3(64), 0, s, p->d_guard, *fp_out);
+        FFI_HIP_TRY(hipGetLastError());
+        return FFI_OK;
+    };
     // The arranged ids of the weight gradient depend on the lookup alone: their kernel runs on a helper stream beside
     // the kernels of the tiled form (of which the longest runs one wavefront per tile and leaves the memory system idle).
     // (ids < 2^11 and an [N][32] fp32 tile in LDS: the shapes the narrow weight-gradient kernel takes)
@@ -1306,10 +1320,11 @@ int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigne
     // (enqueued from inside the tiled build, behind the row-assignment kernel, where there is a tiled build)
     bool arranged_enqueued = !arranged;
     auto enqueue_arranged = [&]() -> int {
+        FFI_TRY(check_ids());
         if (arranged_enqueued) return FFI_OK;
         arranged_enqueued = true;
         hipStream_t hs = p->helper_stream ? p->helper_stream : s;
-        // (the fingerprint above has synchronised `s`: the lookup is final, the helper needs no further ordering)
+        // (the host has waited for the fingerprint: the lookup is final, the helper needs no further ordering)
         if (hs != s) helper_busy = true;
         return build_arranged(p, lookup, hs);
     };
@@ -1372,7 +1387,6 @@ int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigne
         if (st != FFI_OK) { free_arrays(p); return st; }
     }
     free_spares(p);                            // what this build did not reuse
-    *fp_out = fp;
     return FFI_OK;
 }
 }  // namespace
