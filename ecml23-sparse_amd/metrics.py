@@ -16,7 +16,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .fixed_fan_in_ops import _check_bias, _check_inputs, _stream_handle, backward_sparse, topk_scores
+from .fixed_fan_in_ops import _check_bias, _check_inputs, _on, _stream_handle, backward_sparse, topk_scores
 
 LOSS_HINGE, LOSS_SQUARED_HINGE, LOSS_BCE = 1, 2, 3
 SKIP_ZERO_STORES = 0x100      # flag on the loss kind of forward_loss: zero gradients are not stored
@@ -56,7 +56,7 @@ def sparse_loss_grad(scores, y_true, kind, grad_scale=None, in_place=False, want
     batch, num_units = scores.shape
     indices, values = _labels(y_true, scores.device)
     scale = 1.0 / (batch * num_units) if grad_scale is None else float(grad_scale)
-    with torch.cuda.device(scores.device):
+    with _on(scores.device):
         out_grad = scores if in_place else torch.empty_like(scores)
         loss_sum = torch.empty((1,), dtype=torch.float32, device=scores.device)
         masks = torch.empty(((batch + 31) // 32, num_units), dtype=torch.int32, device=scores.device) if want_masks else None
@@ -85,7 +85,7 @@ def forward_loss(features, lookup, weights, bias, y_true, kind, grad_scale=None,
         raise ValueError("skip_zero_stores needs want_masks: the masks say which entries of out_grad were written")
     indices, values = _labels(y_true, features.device)
     scale = 1.0 / (batch * num_units) if grad_scale is None else float(grad_scale)
-    with torch.cuda.device(features.device):
+    with _on(features.device):
         out_grad = torch.empty((batch, num_units), dtype=torch.float32, device=features.device)
         scores = torch.empty_like(out_grad) if want_scores else None
         loss_sum = torch.empty((1,), dtype=torch.float32, device=features.device)
@@ -259,7 +259,7 @@ def topk_hits(top_labels, k, y_true, also_read=None):
     wait for the stream."""
     indices, values = _labels(y_true, top_labels.device)
     result = (ctypes.c_double * (k + 1))()
-    with torch.cuda.device(top_labels.device):
+    with _on(top_labels.device):
         _lib.check(_lib.lib().ffi_topk_hits_f32(
             top_labels.data_ptr(), top_labels.shape[0], top_labels.stride(0), k, indices.data_ptr() if indices.numel() else None,
             values.data_ptr() if values is not None and values.numel() else None, indices.shape[0],
@@ -322,7 +322,7 @@ def threshold_counts(scores, y_true, threshold):
     scores = scores.contiguous()
     batch, num_units = scores.shape
     indices, values = _labels(y_true, scores.device)
-    with torch.cuda.device(scores.device):
+    with _on(scores.device):
         counts = torch.empty((3,), dtype=torch.float64, device=scores.device)
         _lib.check(_lib.lib().ffi_threshold_metrics_f32(
             scores.data_ptr(), indices.data_ptr() if indices.numel() else None,

@@ -10,7 +10,7 @@ import torch
 
 from . import _lib
 from . import metrics as metrics_mod
-from .fixed_fan_in_ops import _stream_handle, topk_scores
+from .fixed_fan_in_ops import _on, _stream_handle, topk_scores
 
 
 def adam_step(variable, m, v, gradient, learning_rate, beta_1, beta_2, epsilon, step):
@@ -20,7 +20,7 @@ def adam_step(variable, m, v, gradient, learning_rate, beta_1, beta_2, epsilon, 
             raise TypeError(f"{name} must be a contiguous float32 device tensor")
         if t.numel() != variable.numel():
             raise ValueError(f"{name} has {t.numel()} elements, variable has {variable.numel()}")
-    with torch.cuda.device(variable.device):
+    with _on(variable.device):
         _lib.check(_lib.lib().ffi_adam_step_f32(variable.data_ptr(), m.data_ptr(), v.data_ptr(), gradient.data_ptr(),
                                                 variable.numel(), float(learning_rate), float(beta_1), float(beta_2),
                                                 float(epsilon), int(step), _stream_handle(variable.device)))
@@ -189,7 +189,7 @@ def backward_sparse_adam(features, lookup, weights, out_grad, nz_words, weight_m
             if t is None or t.dtype != torch.float32 or t.numel() != num_units or not t.is_contiguous() or t.device != weights.device:
                 raise TypeError(f"{name} must be a contiguous float32 tensor of {num_units} elements on the weights' device")
     taken = ctypes.c_int(-1)
-    with torch.cuda.device(features.device):
+    with _on(features.device):
         feature_grad = torch.empty_like(features) if need_feature_grad else None
         _lib.check(_lib.lib().ffi_backward_sparse_adam_f32(
             features.data_ptr(), lookup.data_ptr(), weights.data_ptr(), out_grad.data_ptr(),

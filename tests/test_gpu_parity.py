@@ -1082,3 +1082,24 @@ def test_plan_form_and_gradients_at_few_columns(ffi, N, B, L, K):
                 assert rel_err(gx.cpu().numpy(), o_gx) <= GRAD_RTOL and rel_err(gw.cpu().numpy(), o_gw) <= GRAD_RTOL
         finally:
             lib.ffi_set_option(b"small_path", 0)
+
+
+def test_calls_find_the_current_stream(ffi):
+    # the handle that calls pass on is the one torch would name, inside a stream's context, behind it and on another thread
+    import threading
+    ops, device = ffi.fixed_fan_in_ops, torch.empty(1, device="cuda").device
+    side = torch.cuda.Stream()
+    seen = []
+
+    def look():
+        seen.append((ops._stream_handle(device), torch.cuda.current_stream(device).cuda_stream))
+        with torch.cuda.stream(side):
+            seen.append((ops._stream_handle(device), side.cuda_stream))
+        with ops._on(device):
+            seen.append((ops._stream_handle(device), torch.cuda.current_stream().cuda_stream))
+
+    look()
+    thread = threading.Thread(target=look)
+    thread.start()
+    thread.join()
+    assert len(seen) == 6 and all(a == b for a, b in seen)
