@@ -437,7 +437,7 @@ int ffi_backward_sparse_f32(const float* features, const int32_t* lookup, const 
     if (!sparse && grad_is_partial) FFI_TRY(launch_zero_unmasked(out_grad, words, d.B, d.L, s));
     auto wgrad = [&](const ffi_plan* plan) {
         if (!weight_grad) return (int)FFI_OK;
-        if (sparse) return launch_weight_grad_sparse(features, lookup, out_grad, words, weight_grad, bias_grad, nullptr, d, s);
+        if (sparse) return launch_weight_grad_sparse(features, lookup, out_grad, words, weight_grad, bias_grad, d, s);
         return launch_weight_grad(features, lookup, out_grad, weight_grad, bias_grad, d, s, plan);
     };
     if (!feature_grad) return wgrad(nullptr);
@@ -476,24 +476,28 @@ int ffi_backward_sparse_adam_f32(const float* features, const int32_t* lookup, f
     Dims d;
     FFI_TRY(check_dims(batch, num_features, num_units, fan_in, transposed, &d));
     hipStream_t s = (hipStream_t)stream;
-    const unsigned* words = nullptr;
+    const unsigned* words = nz_words;
     unsigned long long set_bits = 0;
-    FFI_TRY(nonzero_count(out_grad, nz_words, d.B, d.L, s, (flags & FFI_SPARSE_DECIDE_FROM_PREVIOUS) != 0, &words, &set_bits));
+    const bool lagged = (flags & FFI_SPARSE_DECIDE_FROM_PREVIOUS) != 0;
     const double limit = (double)(max_density > 0.f ? max_density : kSparseDefaultMaxDensity) * (double)d.B * (double)d.L;
-    const bool sparse = (double)set_bits <= limit && sparse_weight_grad_fits(d.B, d.N);
+    auto takes_sparse = [&]() { return (double)set_bits <= limit && sparse_weight_grad_fits(d.B, d.N); };
+    // (the sparse kernels count the bits themselves, for the next call; a call that has no count yet waits for one)
+    bool sparse = lagged && nz_words != nullptr && nonzero_previous(d.B, d.L, s, &set_bits) && takes_sparse();
+    if (!sparse) {
+        FFI_TRY(nonzero_count(out_grad, nz_words, d.B, d.L, s, lagged, &words, &set_bits));
+        sparse = takes_sparse();
+    }
     if (sparse_path_taken) *sparse_path_taken = sparse ? 1 : 0;
-    // the gradients live in a workspace: [L*K] weight gradient (16-byte aligned end), [L] bias gradient, [L] row flags
+    // the gradients live in a workspace: [L*K] weight gradient (16-byte aligned end), [L] bias gradient
     const size_t wcount = (size_t)d.L * d.K;
     const size_t bias_at = (wcount + 3) / 4 * 4;
     float* grads = nullptr;
-    FFI_TRY(workspace_get(s, kWsGradients, (bias_at + (size_t)d.L) * sizeof(float) + (size_t)d.L, (void**)&grads));
+    FFI_TRY(workspace_get(s, kWsGradients, (bias_at + (size_t)d.L) * sizeof(float), (void**)&grads));
     float* gw = grads;
     float* gb = bias ? grads + bias_at : nullptr;
-    unsigned char* active = reinterpret_cast<unsigned char*>(grads + bias_at + d.L);
     if (sparse) {
-        // the weight gradient of labels without a non-zero out_grad entry is neither written nor read: the Adam
-        // pass takes a zero for them
-        FFI_TRY(launch_weight_grad_sparse(features, lookup, out_grad, words, gw, gb, active, d, s));
+        // the weight gradient of labels without a non-zero out_grad entry is neither written nor read
+        if (bias && (((uintptr_t)bias | (uintptr_t)bias_m | (uintptr_t)bias_v) % 16) != 0) return FFI_ERR_BAD_ARGUMENT;
         if (feature_grad) {
             if (sparse_input_grad_fits(d.N, d.K)) {
                 FFI_TRY(launch_input_grad_sparse(lookup, weights, out_grad, words, feature_grad, d, s));
@@ -501,10 +505,8 @@ int ffi_backward_sparse_adam_f32(const float* features, const int32_t* lookup, f
                 FFI_TRY(input_grad_cached(lookup, weights, out_grad, feature_grad, d, s, [](const ffi_plan*) { return (int)FFI_OK; }));
             }
         }
-        FFI_TRY(launch_adam_step_rows(weights, weight_m, weight_v, gw, active, d.L, d.K, learning_rate, beta_1, beta_2, epsilon,
-                                      (long long)step, s));
-        if (bias) FFI_TRY(launch_adam_step(bias, bias_m, bias_v, gb, (size_t)d.L, learning_rate, beta_1, beta_2, epsilon, (long long)step, s));
-        return FFI_OK;
+        const AdamVariables v{weights, weight_m, weight_v, bias, bias_m, bias_v};
+        return launch_weight_grad_adam_sparse(features, lookup, out_grad, words, gw, gb, v, learning_rate, beta_1, beta_2, epsilon, (long long)step, d, s);
     }
     // dense kernels: gradients into a workspace, then the Adam pass
     if (grad_is_partial) FFI_TRY(launch_zero_unmasked(out_grad, words, d.B, d.L, s));

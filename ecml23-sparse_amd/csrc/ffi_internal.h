@@ -220,10 +220,19 @@ int nonzero_count(const float* g, const unsigned* given_words, int B, int L, hip
                   const unsigned** words_out, unsigned long long* count_out);
 // drops the counts remembered for a device (the next lagged call waits again)
 void nonzero_count_forget(int device);
-// active == null: every row of gw is written (zeros for labels without a set bit).  active != null ([L] bytes):
-// only the rows of labels with a set bit are written and active[j] tells which
+// the count that an earlier call of the shape on this stream has left, if one has
+bool nonzero_previous(int B, int L, hipStream_t s, unsigned long long* count_out);
+// every row of gw is written (zeros for labels without a set bit)
 int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
-                              float* bias_grad, unsigned char* active, const Dims& d, hipStream_t s);
+                              float* bias_grad, const Dims& d, hipStream_t s);
+// the same gradients, of which the rows without a set bit are not written, and the Adam step on the variables; leaves the number of
+// set bits for nonzero_previous.  gw and bias_grad 16-byte aligned; the variables at any alignment; bias and its moments may be null.
+struct AdamVariables {
+    float *weights, *weight_m, *weight_v, *bias, *bias_m, *bias_v;
+};
+int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad,
+                                   const AdamVariables& v, float lr, float beta_1, float beta_2, float eps, long long step, const Dims& d,
+                                   hipStream_t s);
 bool sparse_input_grad_fits(int N, int K);
 bool sparse_weight_grad_fits(int B, int N);   // x within 32-bit byte offsets
 // g[b,j] = 0 wherever the mask bit of (b,j) is clear
@@ -235,9 +244,6 @@ int launch_input_grad_sparse(const int32_t* idx, const float* w, const float* g,
 // one Adam step (Keras' update rule) on `count` float32 variables; arrays 16-byte aligned; step is 1-based
 int launch_adam_step(float* var, float* m, float* v, const float* g, size_t count, float lr, float beta_1, float beta_2,
                      float eps, long long step, hipStream_t s);
-// the same for a [rows, row_len] variable whose gradient rows are valid only where active[row] != 0 (zero elsewhere)
-int launch_adam_step_rows(float* var, float* m, float* v, const float* g, const unsigned char* active, int rows, int row_len,
-                          float lr, float beta_1, float beta_2, float eps, long long step, hipStream_t s);
 
 // ---- rewiring (ffi_rewire.hip) -------------------------------------------------------------------
 // *threshold (device) = the k-th smallest |w| (k counted from 1; k == 0 gives 0)

@@ -9,6 +9,7 @@
 //   nz_scan_kernel          words from out_grad
 //   nz_count_kernel, nz_count_finish_kernel   the number of set bits (two steps, no atomics)
 //   nz_transpose_kernel     bits from words
+//   wgrad_adam_kernel       wgrad_sparse_kernel and the Adam step on all rows, those without a set bit included
 //   wgrad_sparse_kernel     a wavefront lists the labels of its block that have a set bit, then lane <-> listed
 //                           label: every lane walks the set bits of its own label and keeps 32 sums (one chunk of
 //                           connections) in registers; labels with many set bits are done by the whole wavefront
@@ -18,6 +19,7 @@
 //                           connections into per-wavefront accumulators gx[n] in LDS (LDS float adds issued in a
 //                           fixed order)
 //   igrad_sparse_reduce_kernel  sums the segments in ascending order into feature_grad
+#include "ffi_adam.h"
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 
@@ -155,26 +157,42 @@ constexpr int kHeavyBits = 12;     // labels with more set bits than this are le
 
 // x is addressed as x[b * xsb + n * xsn] (either layout; byte strides), through a buffer resource with 32-bit
 // offsets: batch * num_features * 4 < 2^32, checked by the launcher.
-// ZERO_FILL == true: rows of labels without a set bit are written as zeros.
-// ZERO_FILL == false: those rows are left alone and active[j] (one byte per label) says which rows were written:
-// for a consumer that does not want to read 4 * K bytes of zeros per idle label.
+// ZERO_FILL == true: rows of labels without a set bit (and their bias gradients) are written as zeros.
+// ZERO_FILL == false: they are left alone.
+// `done(labels listed, how many, first label of the block)` comes behind each block of kWsBlock labels.  Returns the set bits that
+// the lane's labels had.
 constexpr int kWsLabelsPerLane = 4;
 constexpr int kWsBlock = 64 * kWsLabelsPerLane;      // labels a wavefront looks at in one go
 
-template <bool VEC4, bool ZERO_FILL>
-__global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const float* __restrict__ x, unsigned xsb, unsigned xsn,
-                                                              const int32_t* __restrict__ idx, const float* __restrict__ g,
-                                                              const unsigned* __restrict__ words, float* __restrict__ gw,
-                                                              float* __restrict__ bias_grad,
-                                                              unsigned char* __restrict__ active, int B, int N, int L,
-                                                              int K, int nbt) {
+struct SparseRows {
+    const float* x;
+    unsigned xsb, xsn;
+    const int32_t* idx;
+    const float* g;
+    const unsigned* words;
+    float* gw;
+    float* bias_grad;
+    int B, N, L, K, nbt;
+};
+
+template <bool VEC4, bool ZERO_FILL, class Done>
+__device__ __forceinline__ unsigned sparse_rows(const SparseRows& r, int block, int nblocks, Done done) {
+    const float* __restrict__ x = r.x;
+    const int32_t* __restrict__ idx = r.idx;
+    const float* __restrict__ g = r.g;
+    const unsigned* __restrict__ words = r.words;
+    float* gw = r.gw;
+    float* bias_grad = r.bias_grad;
+    const unsigned xsb = r.xsb, xsn = r.xsn;
+    const int B = r.B, N = r.N, L = r.L, K = r.K, nbt = r.nbt;
     // per wavefront: the labels of its block that have a set bit, as (set bits << 8) | offset in the block.  Most labels
     // have none when the gradient is sparse; the lanes then work on the compacted list, not on 64 neighbouring labels of
     // which a few are busy.
     __shared__ unsigned active_list[4][kWsBlock];
+    unsigned set_bits = 0;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wave = blockIdx.x * 4 + wv;
-    const int nwaves = gridDim.x * 4;
+    const int wave = block * 4 + wv;
+    const int nwaves = nblocks * 4;
     const int nblk = (L + kWsBlock - 1) / kWsBlock;
     const unsigned tail = (B & 31) ? (1u << (B & 31)) - 1u : 0xffffffffu;   // bits past the batch are ignored
     const buffer_rsrc xr = make_rsrc(x, (size_t)B * (size_t)N * sizeof(float));
@@ -216,10 +234,9 @@ __global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const float* __res
                     for (int e = lane; e < rows * K; e += 64)
                         if ((zero_rows >> (e / K)) & 1ull) blockrows[e] = 0.f;
                 }
-            } else if (mine) {
-                active[base + lane] = cnt != 0;
+                if (bias_grad != nullptr && mine && cnt == 0) bias_grad[base + lane] = 0.f;
             }
-            if (bias_grad != nullptr && mine && cnt == 0) bias_grad[base + lane] = 0.f;
+            if (mine) set_bits += (unsigned)cnt;
             const bool busy = mine && cnt > 0;
             const unsigned long long bal = __ballot(busy);
             if (busy) mylist[total + __popcll(bal & ((1ull << lane) - 1ull))] = ((unsigned)cnt << 8) | (unsigned)(q * 64 + lane);
@@ -352,6 +369,129 @@ __global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const float* __res
             if (bias_grad != nullptr && lane == 0) bias_grad[jh] = hsum;
         }
         }
+        done(mylist, total, block_base);
+    }
+    return set_bits;
+}
+
+template <bool VEC4>
+__global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const SparseRows rows) {
+    sparse_rows<VEC4, true>(rows, blockIdx.x, gridDim.x, [](const unsigned*, int, int) {});
+}
+
+// The same gradients and the Adam step on weights and bias in one launch: labels without a set bit take the step of a zero gradient,
+// which nothing but the moments and variables is read for, labels with one take theirs from the rows that their own wavefront has
+// just formed.  The former are bound by memory and the latter by the latency of their gathers: the latter's workgroups come first, the
+// others take the room that they leave.  (Alternating, 174 us for the step below: under the others' loads every gather waits longer.)
+// They also count the set bits, which the next call decides from (host_count; totals: a sum and a count of workgroups, zero between
+// launches).
+// (32 x 768 x 670,091 x 32, 0.2 % of the gradients not zero, late in training: two launches that count 9.6 us, the gradient 22, the
+// step on the weights 72 and on the bias 5.8; 98 so.  The whole step with its forward pass 183 -> 170.)
+struct AdamRows {
+    float *var, *m, *v, *bias, *bias_m, *bias_v;
+    AdamCoefficients a;
+    unsigned long long* totals;
+    unsigned long long* host_count;
+    int gradient_blocks;
+};
+
+template <bool VEC4>
+__global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, const AdamRows o) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if ((int)blockIdx.x < o.gradient_blocks) {
+        const unsigned bits = sparse_rows<VEC4, false>(r, blockIdx.x, o.gradient_blocks, [&](const unsigned* list, int total, int base) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");        // (rows and list are the wavefront's own)
+            __builtin_amdgcn_wave_barrier();
+            const int len = VEC4 ? r.K / 4 : r.K;
+            for (int e = lane; e < total * len; e += 64) {
+                const int i = e / len;
+                const size_t at = (size_t)(base + (int)(list[i] & 255u)) * len + (size_t)(e - i * len);
+                if (VEC4) {
+                    float4 w4 = reinterpret_cast<float4*>(o.var)[at], m4 = reinterpret_cast<float4*>(o.m)[at], v4 = reinterpret_cast<float4*>(o.v)[at];
+                    adam_four(w4, m4, v4, reinterpret_cast<const float4*>(r.gw)[at], o.a);
+                    reinterpret_cast<float4*>(o.var)[at] = w4;
+                    reinterpret_cast<float4*>(o.m)[at] = m4;
+                    reinterpret_cast<float4*>(o.v)[at] = v4;
+                } else {
+                    adam_one(o.var[at], o.m[at], o.v[at], r.gw[at], o.a);
+                }
+            }
+            if (o.bias != nullptr)
+                for (int i = lane; i < total; i += 64) {
+                    const int j = base + (int)(list[i] & 255u);
+                    adam_one(o.bias[j], o.bias_m[j], o.bias_v[j], r.bias_grad[j], o.a);
+                }
+            __builtin_amdgcn_wave_barrier();
+        });
+        unsigned long long n = bits;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+        __shared__ unsigned long long of_wave[4];
+        if (lane == 0) of_wave[wv] = n;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            n = (of_wave[0] + of_wave[1]) + (of_wave[2] + of_wave[3]);
+            // the ticket is drawn once the sum is known to have this workgroup's bits
+            const unsigned long long before = __hip_atomic_fetch_add(o.totals, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long one = before == ~0ull ? 0ull : 1ull;
+            if (__hip_atomic_fetch_add(o.totals + 1, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned long long)o.gradient_blocks - 1ull) {
+                *o.host_count = __hip_atomic_exchange(o.totals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // pinned host memory
+                __hip_atomic_store(o.totals + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        return;
+    }
+    // 64 labels per wavefront and step
+    const int stepper = (int)blockIdx.x - o.gradient_blocks, steppers = gridDim.x - o.gradient_blocks;
+    const unsigned tail = (r.B & 31) ? (1u << (r.B & 31)) - 1u : 0xffffffffu;
+    for (int base = (stepper * 4 + wv) * 64; base < r.L; base += steppers * 256) {
+        const int rows = min(64, r.L - base);
+        bool idle_row = false;
+        unsigned long long idle = 0ull;
+        auto look = [&]() {
+            unsigned set = 0u;
+            for (int t = 0; t < r.nbt; ++t) {
+                const unsigned m = r.words[(size_t)t * r.L + min(base + lane, r.L - 1)];
+                set |= t == r.nbt - 1 ? m & tail : m;
+            }
+            idle_row = lane < rows && set == 0u;
+            idle = __ballot(idle_row);
+        };
+        if (VEC4) {
+            const int len = r.K / 4, loads = rows * len;
+            const float inv_len = 1.f / (float)len;
+            float4* var = reinterpret_cast<float4*>(o.var) + (size_t)base * len;
+            float4* m = reinterpret_cast<float4*>(o.m) + (size_t)base * len;
+            float4* v = reinterpret_cast<float4*>(o.v) + (size_t)base * len;
+            // (all rows are read, so that nothing waits for the masks; what another wavefront makes of the ones with a set bit is not used)
+            constexpr int kAtOnce = 2;
+            for (int e0 = lane; e0 < loads; e0 += 64 * kAtOnce) {
+                float4 w4[kAtOnce], m4[kAtOnce], v4[kAtOnce];
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    const int e = min(e0 + 64 * u, loads - 1);
+                    w4[u] = var[e]; m4[u] = m[e]; v4[u] = v[e];
+                }
+                if (e0 == lane) look();
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    const int e = e0 + 64 * u;
+                    int row = (int)((float)e * inv_len);                  // e / len, once it is set right
+                    row += e >= (row + 1) * len ? 1 : e < row * len ? -1 : 0;
+                    if (e >= loads || !(idle >> row & 1ull)) continue;
+                    adam_four(w4[u], m4[u], v4[u], make_float4(0.f, 0.f, 0.f, 0.f), o.a);
+                    var[e] = w4[u];
+                    m[e] = m4[u];
+                    v[e] = v4[u];
+                }
+            }
+        } else {
+            look();
+            const size_t from = (size_t)base * r.K;
+            for (int e = lane; e < rows * r.K; e += 64)
+                if (idle >> (e / r.K) & 1ull) adam_one(o.var[from + e], o.m[from + e], o.v[from + e], 0.f, o.a);
+        }
+        if (o.bias != nullptr && idle_row) adam_one(o.bias[base + lane], o.bias_m[base + lane], o.bias_v[base + lane], 0.f, o.a);
     }
 }
 
@@ -486,13 +626,37 @@ __global__ __launch_bounds__(256) void igrad_sparse_reduce_kernel(const float* _
 struct CountSlot {
     int device;
     hipStream_t stream;
-    unsigned long long* host;    // hipHostMalloc'ed, written by nz_count_finish_kernel
+    unsigned long long* host;    // hipHostMalloc'ed, written by nz_count_finish_kernel or wgrad_adam_kernel
     int B, L;                    // shape of the last call (0: none yet)
 };
 std::mutex g_count_mutex;
 std::vector<CountSlot> g_count_slots;
 
+// (under the lock; the slot stays where it is as long as that is held)
+int count_slot(int dev, hipStream_t s, CountSlot** out) {
+    for (CountSlot& c : g_count_slots)
+        if (c.device == dev && c.stream == s) { *out = &c; return FFI_OK; }
+    CountSlot c{dev, s, nullptr, 0, 0};
+    if (hipHostMalloc((void**)&c.host, 64) != hipSuccess) { (void)hipGetLastError(); return FFI_ERR_OUT_OF_MEMORY; }
+    *c.host = 0;
+    g_count_slots.push_back(c);
+    *out = &g_count_slots.back();
+    return FFI_OK;
+}
+
 }  // namespace
+
+bool nonzero_previous(int B, int L, hipStream_t s, unsigned long long* count_out) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(g_count_mutex);
+    for (const CountSlot& c : g_count_slots) {
+        if (c.device != dev || c.stream != s || c.B != B || c.L != L) continue;
+        *count_out = *reinterpret_cast<volatile unsigned long long*>(c.host);
+        return true;
+    }
+    return false;
+}
 
 int launch_nonzero_scan(const float* g, unsigned* words, int B, int L, hipStream_t s) {
     const int nbt = (B + 31) / 32;
@@ -528,15 +692,7 @@ int nonzero_count(const float* g, const unsigned* given_words, int B, int L, hip
     *words_out = words;
     std::lock_guard<std::mutex> lock(g_count_mutex);
     CountSlot* slot = nullptr;
-    for (CountSlot& c : g_count_slots)
-        if (c.device == dev && c.stream == s) slot = &c;
-    if (!slot) {
-        CountSlot c{dev, s, nullptr, 0, 0};
-        if (hipHostMalloc((void**)&c.host, 64) != hipSuccess) { (void)hipGetLastError(); return FFI_ERR_OUT_OF_MEMORY; }
-        *c.host = 0;
-        g_count_slots.push_back(c);
-        slot = &g_count_slots.back();
-    }
+    FFI_TRY(count_slot(dev, s, &slot));
     // the count of an earlier call of the same shape on this stream, read before this call's kernels can overwrite it
     const bool use_previous = lagged && slot->B == B && slot->L == L;
     const unsigned long long previous = *reinterpret_cast<volatile unsigned long long*>(slot->host);
@@ -560,20 +716,40 @@ void nonzero_count_forget(int device) {
         if (c.device == device) { c.B = 0; c.L = 0; }
 }
 
-int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
-                              float* bias_grad, unsigned char* active, const Dims& d, hipStream_t s) {
-    const int nbt = (d.B + 31) / 32;
-    const int nblk = (d.L + kWsBlock - 1) / kWsBlock;
-    const int blocks = std::max(1, std::min((nblk + 3) / 4, device_cu_count() * 8));
+namespace {
+SparseRows sparse_rows_of(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad, const Dims& d) {
     // byte strides of x along the batch and along the features
-    const unsigned xsb = (d.tp ? 1u : (unsigned)d.N) * 4u, xsn = (d.tp ? (unsigned)d.B : 1u) * 4u;
+    return SparseRows{x, (d.tp ? 1u : (unsigned)d.N) * 4u, (d.tp ? (unsigned)d.B : 1u) * 4u, idx, g, words, gw, bias_grad, d.B, d.N, d.L, d.K, (d.B + 31) / 32};
+}
+int sparse_rows_blocks(const Dims& d) { return std::max(1, std::min(((d.L + kWsBlock - 1) / kWsBlock + 3) / 4, device_cu_count() * 8)); }
+}  // namespace
+
+int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
+                              float* bias_grad, const Dims& d, hipStream_t s) {
     const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx) % 16 == 0);
-#define FFI_LAUNCH_WS(V, Z)                                                                                                  \
-    hipLaunchKernelGGL((wgrad_sparse_kernel<V, Z>), dim3(blocks), dim3(256), 0, s, x, xsb, xsn, idx, g, words, gw, bias_grad, active, \
-                       d.B, d.N, d.L, d.K, nbt)
-    if (active == nullptr) { if (vec4) FFI_LAUNCH_WS(true, true); else FFI_LAUNCH_WS(false, true); }
-    else                   { if (vec4) FFI_LAUNCH_WS(true, false); else FFI_LAUNCH_WS(false, false); }
-#undef FFI_LAUNCH_WS
+    hipLaunchKernelGGL((vec4 ? wgrad_sparse_kernel<true> : wgrad_sparse_kernel<false>), dim3(sparse_rows_blocks(d)), dim3(256), 0, s,
+                       sparse_rows_of(x, idx, g, words, gw, bias_grad, d));
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
+int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad,
+                                   const AdamVariables& v, float lr, float beta_1, float beta_2, float eps, long long step, const Dims& d,
+                                   hipStream_t s) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
+    unsigned* tickets = nullptr;
+    FFI_TRY(tickets_get(s, (void**)&tickets));
+    std::lock_guard<std::mutex> lock(g_count_mutex);
+    CountSlot* slot = nullptr;
+    FFI_TRY(count_slot(dev, s, &slot));
+    const int gradient_blocks = sparse_rows_blocks(d), steps = (d.L + 255) / 256;
+    const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx | (uintptr_t)v.weights | (uintptr_t)v.weight_m | (uintptr_t)v.weight_v) % 16 == 0);
+    const AdamRows o{v.weights, v.weight_m, v.weight_v, v.bias, v.bias_m, v.bias_v, adam_coefficients(lr, beta_1, beta_2, eps, step),
+                     reinterpret_cast<unsigned long long*>(tickets), slot->host, gradient_blocks};
+    const int steppers = std::min(steps, device_cu_count() * 16);
+    hipLaunchKernelGGL((vec4 ? wgrad_adam_kernel<true> : wgrad_adam_kernel<false>), dim3(gradient_blocks + steppers), dim3(256), 0, s,
+                       sparse_rows_of(x, idx, g, words, gw, bias_grad, d), o);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }

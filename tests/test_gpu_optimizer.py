@@ -120,6 +120,50 @@ def test_backward_with_adam_epilogue_matches_backward_then_adam(ffi, shape, forc
         assert rel_err(a, b) <= 1e-5
 
 
+@pytest.mark.parametrize("share", [0.0, 0.02, 1.0])
+@pytest.mark.parametrize("shape", [(5, 30, 1, 4), (33, 40, 63, 7), (70, 64, 257, 32), (32, 50, 1300, 40), (3, 9, 5000, 1), (40, 300, 300, 260)])
+def test_step_on_rows_with_and_without_gradient(ffi, shape, share):
+    # rows of both kinds side by side, none of one kind, labels that the whole wavefront takes (share 1: every sample's bit), mask bits
+    # behind the batch, and the count that the next call decides from
+    B, N, L, K = shape
+    rng = np.random.default_rng(sum(shape) + int(100 * share))
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    x, lookup = rng.standard_normal((B, N)).astype(np.float32), rng.integers(0, N, (L, K)).astype(np.int32)
+    g = rng.standard_normal((B, L)).astype(np.float32)
+    g[rng.random((B, L)) >= share] = 0.0
+    words = np.full(((B + 31) // 32, L), 0, dtype=np.uint32)
+    for b in range(B):
+        words[b // 32] |= (g[b] != 0).astype(np.uint32) << np.uint32(b % 32)
+    if B % 32:
+        words[-1] |= np.uint32(0x80000000)
+    w0, b0 = rng.standard_normal((L, K)).astype(np.float32), rng.standard_normal(L).astype(np.float32)
+    start = [w0, 0.1 * rng.standard_normal((L, K)).astype(np.float32), rng.random((L, K)).astype(np.float32),
+             b0, 0.1 * rng.standard_normal(L).astype(np.float32), rng.random(L).astype(np.float32)]
+    w, mw, vw, bias, mb, vb = [dev(a) for a in start]
+    _, sparse = ffi.optimizer.backward_sparse_adam(dev(x), dev(lookup), w, dev(g), dev(words.view(np.int32)), mw, vw, bias, mb, vb,
+                                                   0.01, 0.9, 0.999, 1e-7, 3, max_density=4.0, need_feature_grad=False)
+    assert sparse
+    gw = np.zeros((L, K))
+    for k in range(K):
+        gw[:, k] = (g.astype(np.float64) * x.astype(np.float64)[:, lookup[:, k]]).sum(axis=0)
+    alpha = 0.01 * np.sqrt(1.0 - 0.999 ** 3) / (1.0 - 0.9 ** 3)
+    for got, (var, m, v), grad in (((w, mw, vw), start[:3], gw), ((bias, mb, vb), start[3:], g.astype(np.float64).sum(axis=0))):
+        m1 = m + (grad - m) * 0.1
+        v1 = v + (grad * grad - v) * 0.001
+        for a, ref in zip(got, (var - m1 * alpha / (np.sqrt(v1) + 1e-7), m1, v1)):
+            assert rel_err(a.cpu().numpy(), ref.astype(np.float32)) <= 1e-5
+    # the density that the call has found decides for the next one of the shape
+    found = sum(int(np.unpackbits(words[t].view(np.uint8)).sum()) for t in range(words.shape[0])) - (L if B % 32 else 0)
+    for limit, expected in (((found + 0.5) / (B * L), True), ((found - 0.5) / (B * L), False)):
+        if limit <= 0.0:
+            continue
+        _, sparse = ffi.optimizer.backward_sparse_adam(dev(x), dev(lookup), w, dev(g), dev(words.view(np.int32)), mw, vw, bias, mb, vb,
+                                                       0.01, 0.9, 0.999, 1e-7, 4, max_density=limit, need_feature_grad=False,
+                                                       decide_from_previous=True)
+        torch.cuda.synchronize()
+        assert sparse == expected
+
+
 def test_fused_train_step_follows_the_unfused_loop(ffi):
     # layer.fused_train_step + optimizer.step() against forward_loss / backward / optimizer.step(), three steps
     B, N, L = 64, 128, 2000
