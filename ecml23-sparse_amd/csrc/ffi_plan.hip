@@ -123,7 +123,7 @@ template <int LANES> __device__ __forceinline__ int lanes_total(int v) {
 template <int LANES, bool MORE>              // (MORE: fan-ins above LANES = 64)
 __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restrict__ idx, int L, int K, int tile_labels, int cap,
                                                          int ncols, unsigned short* __restrict__ rowpos, int col_lo,
-                                                         int all_columns_count) {
+                                                         int all_columns_count, unsigned* __restrict__ counts) {
     extern __shared__ int color_lds[];
     // (entry `ncols` of both: where connections into columns outside the window go -- weight 0, so they never count)
     int* imb = color_lds;                                                        // [ncols + 1] even minus odd labels per column
@@ -171,12 +171,12 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         wt[c] = (unsigned short)(all_columns_count ? (len > 0 ? 256 : 0) : (int)(256.f * r));
     }
     __syncthreads();
-    if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x;
-    constexpr int kAbreast = 64 / LANES;                                         // labels decided together
-    const int groups = (nl + kAbreast - 1) / kAbreast, k_mine = lane & (LANES - 1), abreast = lane / LANES;
     // the half a label goes to: bit 30 of its first word
     auto half_of = [&](int jl) { return (int)(ids3[jl * W] >> 30 & 1u); };
+    const int lane = threadIdx.x & 63;
+    auto decide_all = [&]() {
+    constexpr int kAbreast = 64 / LANES;                                         // labels decided together
+    const int groups = (nl + kAbreast - 1) / kAbreast, k_mine = lane & (LANES - 1), abreast = lane / LANES;
     int placed[2] = {0, 0};
     // What bounds the kernel is the chain from one step's adds to the next step's decision: an LDS round trip, the sum over the
     // lanes by DPP and lane swaps, a comparison in every lane; what it does to the counts of placed labels is beside the chain.  Of
@@ -276,30 +276,22 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         next[0] += __popcll(evens);
         next[1] += __popcll(odds);
     }
-}
-
-// Adds a tile's connections to cnt[half of the label's row][column].  Eight ids and the rows of their labels are on their way
-// at a time; labels by stepping, not division.
-__device__ __forceinline__ void count_halves(const int32_t* __restrict__ src, const unsigned short* __restrict__ row_of, int total, int K,
-                                             int col_lo, unsigned* cnt) {
-    constexpr int kInflight = 8;
-    const int nthreads = blockDim.x, dl = nthreads / K, dk = nthreads - dl * K;
-    int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
-    for (int e0 = threadIdx.x; e0 < total; e0 += nthreads * kInflight) {
-        unsigned c[kInflight], row[kInflight];
+    };
+    if (threadIdx.x < 64) decide_all();
+    __syncthreads();
+    // what became of the columns: labels in even rows | in odd rows << 16, for the kernels that lay the slots out
+    for (int c = threadIdx.x; c <= ncols; c += 256) imb[c] = 0;
+    __syncthreads();
+    for (int wi = threadIdx.x; wi < nl * W; wi += 256) {
+        const int jl = wi / W, k0 = 3 * (wi - jl * W);
+        const unsigned word = ids3[wi];
+        const int one = half_of(jl) ? 0x10000 : 1;
 #pragma unroll
-        for (int i = 0; i < kInflight; ++i) {
-            const bool on = e0 + i * nthreads < total;
-            c[i] = on ? (unsigned)(src[e0 + i * nthreads] - col_lo) : ~0u;
-            row[i] = on ? row_of[l] : 0u;
-            l += dl;
-            k += dk;
-            if (k >= K) { k -= K; ++l; }
-        }
-#pragma unroll
-        for (int i = 0; i < kInflight; ++i)
-            if (c[i] < (unsigned)nthreads) atomicAdd(&cnt[(row[i] & 1u) * nthreads + c[i]], 1u);
+        for (int i = 0; i < 3; ++i)
+            if (k0 + i < K) atomicAdd(&imb[(word >> (10 * i)) & 1023u], one);
     }
+    __syncthreads();
+    for (int c = threadIdx.x; c < ncols; c += 256) counts[(size_t)t * ncols + c] = (unsigned)imb[c];
 }
 
 // Which column each thread of the walking kernel takes in each tile (plans with `colperm`).  A wavefront walks as many
@@ -309,31 +301,23 @@ __device__ __forceinline__ void count_halves(const int32_t* __restrict__ src, co
 // blocks dealt to the wavefronts so that the wavefronts of a SIMD (wave, wave + 4, wave + 8, ...) have about the same
 // rows in total: longest block first, each to the SIMD with the least so far that still has a wavefront free.
 // One workgroup per tile, one thread per column (columns up to the workgroup size exist for this purpose: the ones
-// beyond the input's width have no connections).  Sorted by counting; the dealing is done by four lanes for the four SIMDs.  Bound by
-// the counting of the connections: 670,091 labels over 768 columns 157 us, 85 with four lanes dealing, 58 with no comparison of
-// every column with every other.  Also stores the slot rows of each slice, as tile_count_kernel does
-// for plans without the permutation.  LDS: counts [2][threads], keys [threads].
+// beyond the input's width have no connections).  Sorted by counting; the dealing is done by four lanes for the four SIMDs;
+// the columns' lengths come from tile_color_kernel, whose ids lie in LDS.  (670,091 labels over 768 columns 157 us, 85 with four lanes
+// dealing, 58 with no comparison of every column with every other, 16 with no reading of the ids -- which there costs 12.)
+// Also stores the slot rows of each slice, as tile_count_kernel does for plans without the permutation.  LDS: keys [threads].
 constexpr int kPermLengths = 512;            // sorted by counting up to here
-__global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
-                                 int tile_labels, int col_lo, unsigned short* __restrict__ colperm, unsigned* __restrict__ slice_len) {
-    extern __shared__ __align__(16) unsigned perm_lds[];
-    unsigned* cnt = perm_lds;                  // [2][threads]: labels in even rows, labels in odd rows
+__global__ void tile_perm_kernel(const unsigned* __restrict__ counts, unsigned short* __restrict__ colperm, unsigned* __restrict__ slice_len) {
+    extern __shared__ __align__(16) unsigned key[];                       // [threads]
     const int t = blockIdx.x, nthreads = blockDim.x, nslices = nthreads >> 6;
-    unsigned* key = cnt + 2 * nthreads;        // [threads]
+    const unsigned halves = counts[(size_t)t * nthreads + threadIdx.x], even = halves & 0xffffu, odd = halves >> 16;
     __shared__ unsigned short wave_of_block[16];
     __shared__ unsigned slice_rows[16];
     __shared__ __align__(16) unsigned char of_wave[16][kPermLengths];     // columns of each length in a wavefront
     __shared__ unsigned longer[kPermLengths];                             // columns of greater length
     if (threadIdx.x < 16) slice_rows[threadIdx.x] = 0u;
     for (int i = threadIdx.x; i < nslices * kPermLengths / 16; i += nthreads) reinterpret_cast<uint4*>(of_wave)[i] = make_uint4(0u, 0u, 0u, 0u);
-    cnt[threadIdx.x] = 0;
-    cnt[nthreads + threadIdx.x] = 0;
-    __syncthreads();
-    const int j0 = t * tile_labels;
-    count_halves(idx + (size_t)j0 * K, rowpos + j0, min(tile_labels, L - j0) * K, K, col_lo, cnt);
-    __syncthreads();
     // (the slots a column needs depend by one on the lane it gets; the larger of the two; columns of equal length stay in index order)
-    const unsigned length = max(cnt[threadIdx.x], cnt[nthreads + threadIdx.x]);
+    const unsigned length = max(even, odd);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // place among the columns in descending order of the length: the longer ones, the equal ones of the wavefronts before, the equal
     // ones of the lanes before
@@ -402,26 +386,17 @@ __global__ void tile_perm_kernel(const int32_t* __restrict__ idx, const unsigned
     const unsigned thread = wave_of_block[place >> 6] * 64u + (place & 63u);
     colperm[(size_t)t * nthreads + thread] = (unsigned short)threadIdx.x;
     // the slot rows of each slice: those of its longest column, now that every column knows its lane
-    atomicMax(&slice_rows[thread >> 6], column_slots(thread, cnt[threadIdx.x], cnt[nthreads + threadIdx.x]));
+    atomicMax(&slice_rows[thread >> 6], column_slots(thread, even, odd));
     __syncthreads();
     if ((int)threadIdx.x < nslices) slice_len[(size_t)t * nslices + threadIdx.x] = slice_rows[threadIdx.x];
 }
 
-// One workgroup per label tile, one thread per column.  Counts the tile's connections per column
-// and bank half of the label's row (integer LDS atomics: order-independent), stores the slot count of the
-// longest column of each slice.
-__global__ void tile_count_kernel(const int32_t* __restrict__ idx, const unsigned short* __restrict__ rowpos, int L, int K,
-                                  int tile_labels, unsigned* __restrict__ slice_len, int col_lo) {
-    extern __shared__ unsigned cnt[];          // [2][threads]: labels in even rows, labels in odd rows
+// The slot rows of each slice, those of its longest column, where thread t takes column t.  One workgroup per label tile, one
+// thread per column.
+__global__ void tile_count_kernel(const unsigned* __restrict__ counts, unsigned* __restrict__ slice_len) {
     const int t = blockIdx.x, nthreads = blockDim.x;
-    cnt[threadIdx.x] = 0;
-    cnt[nthreads + threadIdx.x] = 0;
-    __syncthreads();
-    const int j0 = t * tile_labels;
-    count_halves(idx + (size_t)j0 * K, rowpos + j0, min(tile_labels, L - j0) * K, K, col_lo, cnt);
-    __syncthreads();
-    const unsigned even = cnt[threadIdx.x], odd = cnt[nthreads + threadIdx.x];
-    unsigned c = column_slots(threadIdx.x, even, odd);
+    const unsigned halves = counts[(size_t)t * nthreads + threadIdx.x];
+    unsigned c = column_slots(threadIdx.x, halves & 0xffffu, halves >> 16);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) c = max(c, (unsigned)__shfl_xor((int)c, off));
     if ((threadIdx.x & 63) == 0) slice_len[(size_t)t * (nthreads >> 6) + (threadIdx.x >> 6)] = c;
@@ -486,7 +461,8 @@ __global__ __launch_bounds__(1024) void slice_scan_kernel(const unsigned* __rest
 // slots 16 bits do not number, counts ranks and writes slots where they belong.
 // Bound by the LDS's atomics and the latency of the walk.  Written where they belong one by one, slots are bound by the L2's write
 // requests instead.  670,091 labels x fan-in 32 over 768 columns 216 -> 129 us, against bitmaps of labels per column with chains for
-// labels that list a column twice, slots written one by one; 501,070 x 64 over 512 772 -> 171; tiles that had no room for the bitmaps,
+// labels that list a column twice, slots written one by one; 501,070 x 64 over 512 772 -> 171; with two workgroups on a CU, where
+// both fit, the former 112; tiles that had no room for the bitmaps,
 // or more such labels than the chains held, were scanned: 200,000 x 40 over 1,000 4,392 -> 76, 300,000 x 16 over 768 2,254 -> 288 (all
 // of the build).
 constexpr int kFillThreads = 1024;
@@ -864,8 +840,8 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     // 32: 35.4 -> 36.5 us): there the order of the columns stays.
     const bool sorted_columns = plan_sorts_columns(threads, TL, p->K, w_in_lds, tiles, p->batch_hint);
     p->colperm = nullptr;
-    unsigned* slice_len = nullptr;
-    if (!dev_alloc(p, &p->slice_off, nslices + 1) || !dev_alloc(p, &slice_len, nslices)) return FFI_ERR_OUT_OF_MEMORY;
+    unsigned *slice_len = nullptr, *counts = nullptr;
+    if (!dev_alloc(p, &p->slice_off, nslices + 1) || !dev_alloc(p, &slice_len, nslices) || !dev_alloc(p, &counts, (size_t)tiles * threads)) return FFI_ERR_OUT_OF_MEMORY;
     // rows per bank half: half the tile plus some room for the balancing, within the LDS the walking kernel can have
     const int cap = tiled_rows_per_half(TL);
     if (!dev_alloc(p, &p->rowpos, (size_t)p->L)) return FFI_ERR_OUT_OF_MEMORY;
@@ -875,7 +851,7 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
         hipError_t ea = hipFuncSetAttribute((const void*)color, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (ea != hipSuccess) return hip_fail(ea);
         hipLaunchKernelGGL(color, dim3(tiles), dim3(256), lds, s, lookup, p->L, p->K, TL, cap, threads, p->rowpos, p->col_lo,
-                           sorted_columns ? 1 : 0);
+                           sorted_columns ? 1 : 0, counts);
     }
     if (after_row_assignment) {
         const int st = after_row_assignment();
@@ -883,11 +859,9 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     }
     if (sorted_columns) {
         if (!dev_alloc(p, &p->colperm, (size_t)tiles * threads)) return FFI_ERR_OUT_OF_MEMORY;
-        hipLaunchKernelGGL(tile_perm_kernel, dim3(tiles), dim3(threads), 3 * threads * sizeof(unsigned), s, lookup, p->rowpos, p->L, p->K, TL,
-                           p->col_lo, p->colperm, slice_len);
+        hipLaunchKernelGGL(tile_perm_kernel, dim3(tiles), dim3(threads), threads * sizeof(unsigned), s, counts, p->colperm, slice_len);
     } else {
-        hipLaunchKernelGGL(tile_count_kernel, dim3(tiles), dim3(threads), 2 * threads * sizeof(unsigned), s, lookup, p->rowpos, p->L,
-                           p->K, TL, slice_len, p->col_lo);
+        hipLaunchKernelGGL(tile_count_kernel, dim3(tiles), dim3(threads), 0, s, counts, slice_len);
     }
     unsigned long long* found = nullptr;                   // (slot rows, and those of the longest tile: written where the host reads them)
     FFI_HIP_TRY(hipHostGetDevicePointer((void**)&found, p->h_scratch + 2, 0));
@@ -896,6 +870,7 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     dev_release(p, slice_len);
+    dev_release(p, counts);
     if (e != hipSuccess) return hip_fail(e);
     const unsigned long long rows = p->h_scratch[2], longest_tile = p->h_scratch[3];
     const unsigned long long connections = (unsigned long long)p->L * p->K;
@@ -915,13 +890,16 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     }
     {
         const unsigned pad_pos = w_in_lds ? (unsigned)TL * (unsigned)p->K : kPadPos;
-        // a wavefront for each eight rounds of 64 connections, fewer where a tile's slots fit beside their counts only then;
-        // what does not fit even so is left to the other form
-        const size_t most = 160 * 1024, whole = std::min<size_t>((size_t)longest_tile, kFillRows);
+        // a wavefront for each eight rounds of 64 connections, fewer where two workgroups fit a CU, or one does, only then; what does not
+        // fit even so is left to the other form
+        const size_t cu = 160 * 1024, whole = std::min<size_t>((size_t)longest_tile, kFillRows);
         int fill_threads = std::min(kFillThreads, std::max(1, TL * p->K / 512) * 64);
-        for (int fewer = fill_threads; fewer >= 512; fewer -= 64)
-            if (tile_fill_lds(fewer, threads, TL) + whole * 128 <= most) { fill_threads = fewer; break; }
-        const size_t counts = tile_fill_lds(fill_threads, threads, TL), stage_rows = std::min((most - counts) / 128, whole);
+        for (const size_t most : {cu / 2, cu}) {
+            int fewer = fill_threads;
+            while (fewer >= 512 && tile_fill_lds(fewer, threads, TL) + whole * 128 > most) fewer -= 64;
+            if (fewer >= std::min(fill_threads, 512)) { fill_threads = fewer; break; }
+        }
+        const size_t counts = tile_fill_lds(fill_threads, threads, TL), stage_rows = std::min((cu - counts) / 128, whole);
         for (const bool staged : {true, false}) {
             if (!staged && longest_tile <= stage_rows) break;
             const auto fill = staged ? tile_fill_kernel<true> : tile_fill_kernel<false>;
