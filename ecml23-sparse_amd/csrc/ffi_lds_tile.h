@@ -26,36 +26,40 @@ __device__ __forceinline__ int xcd_contiguous_block(int block, int nblocks) {
 // xs[r][c] = src[r*ld + c0 + c] for c < 32 (zero beyond column `ld`), r < rows.  src rows are read
 // in 128-byte pieces, LDS writes are conflict-free.  All of a thread's loads are issued before its
 // first LDS write, so the staging costs one memory round trip, not one per row.
+// thread -> (row, 16-byte chunk): 8 threads per row, whose rows start at any float (the memory system serves them; element by
+// element, one in flight, a tile of 768 rows took some 12 us instead of 2: all passes at 127 x 768 x 131,072 x 32 208 us, at 127 x 767 x
+// 131,072 x 4 130, at 163 x 797 x 10,774 x 4 114; 165, 87 and 82 so).
+typedef float f32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 template <int THREADS, int INFLIGHT = 4>
 __device__ __forceinline__ void stage_rows32(float* __restrict__ xs, const float* __restrict__ src, int rows,
                                              int ld, int c0) {
-    const bool vec = (ld % 4 == 0) && (c0 + kTileBatch <= ld) && (((uintptr_t)src & 15) == 0);
-    if (vec) {
-        // thread -> (row, 16-byte chunk): 8 threads per row
-        constexpr int kRowsPerIter = THREADS / 8;
-        constexpr int kInFlight = INFLIGHT;
-        const int q = threadIdx.x & 7;
-        const float* p = src + c0 + 4 * q;
-        for (int r0 = threadIdx.x >> 3; r0 < rows; r0 += kRowsPerIter * kInFlight) {
-            float4 v[kInFlight];
+    constexpr int kRowsPerIter = THREADS / 8;
+    constexpr int kInFlight = INFLIGHT;
+    const int q = threadIdx.x & 7;
+    const int there = ld - (c0 + 4 * q);                                  // elements of the chunk, if fewer than four
+    const float* p = src + c0 + 4 * q;
+    for (int r0 = threadIdx.x >> 3; r0 < rows; r0 += kRowsPerIter * kInFlight) {
+        float4 v[kInFlight];
 #pragma unroll
-            for (int i = 0; i < kInFlight; ++i) {
-                const int r = r0 + i * kRowsPerIter;
-                v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (r < rows) v[i] = *reinterpret_cast<const float4*>(p + (size_t)r * ld);
-            }
-#pragma unroll
-            for (int i = 0; i < kInFlight; ++i) {
-                const int r = r0 + i * kRowsPerIter;
-                if (r < rows) *reinterpret_cast<float4*>(xs + r * kTileBatch + 4 * q) = v[i];
+        for (int i = 0; i < kInFlight; ++i) {
+            const int r = r0 + i * kRowsPerIter;
+            v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (r >= rows) continue;
+            const float* from = p + (size_t)r * ld;
+            if (there >= 4) {
+                const f32x4_unaligned u = *reinterpret_cast<const f32x4_unaligned*>(from);
+                v[i] = make_float4(u.x, u.y, u.z, u.w);
+            } else {
+                if (there > 0) v[i].x = from[0];
+                if (there > 1) v[i].y = from[1];
+                if (there > 2) v[i].z = from[2];
             }
         }
-    } else {
-        const int c = threadIdx.x & 31;
-        const bool in = c0 + c < ld;
-        const float* p = src + c0 + c;
-        for (int r = threadIdx.x >> 5; r < rows; r += THREADS / 32)
-            xs[r * kTileBatch + c] = in ? p[(size_t)r * ld] : 0.f;
+#pragma unroll
+        for (int i = 0; i < kInFlight; ++i) {
+            const int r = r0 + i * kRowsPerIter;
+            if (r < rows) *reinterpret_cast<float4*>(xs + r * kTileBatch + 4 * q) = v[i];
+        }
     }
 }
 

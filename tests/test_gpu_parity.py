@@ -1084,6 +1084,21 @@ def test_plan_form_and_gradients_at_few_columns(ffi, N, B, L, K):
             lib.ffi_set_option(b"small_path", 0)
 
 
+@pytest.mark.parametrize("batch", [1, 30, 31, 33, 34, 35, 64, 127])
+@pytest.mark.parametrize("features,labels,fan_in", [(100, 300, 32), (767, 4100, 9), (1000, 700, 40)])
+def test_rows_of_features_that_start_at_any_float(ffi, batch, features, labels, fan_in):
+    # tiles of 32 samples whose rows start and end anywhere, the last one short, from an array that itself starts one float late
+    x, lookup, w, g = reference_law_inputs(batch, features, labels, fan_in, seed=batch + fan_in)
+    ref = oracle.forward(x, lookup, w, transposed=False)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    late = torch.empty(batch * features + 1, device="cuda")[1:].view(features, batch)
+    late.copy_(torch.from_numpy(x).t())
+    out = ffi.fan_in_sparse_matmul_tp(late, dev(lookup), dev(w))
+    gx, gw = ffi.fan_in_sparse_matmul_grad_tp(late, dev(lookup), dev(w), dev(g))
+    assert rel_err(out.cpu().numpy(), ref) <= 1e-5
+    assert rel_err(gx.t().cpu().numpy(), o_gx) <= GRAD_RTOL and rel_err(gw.cpu().numpy(), o_gw) <= GRAD_RTOL
+
+
 def test_calls_find_the_current_stream(ffi):
     # the handle that calls pass on is the one torch would name, inside a stream's context, behind it and on another thread
     import threading
