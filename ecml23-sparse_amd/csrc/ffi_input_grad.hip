@@ -40,30 +40,25 @@ __global__ __launch_bounds__(1024) void igrad_permute_weights_kernel(
     const int nl = min(tile_labels, L - t * tile_labels);
     const unsigned npos = (unsigned)nl * (unsigned)K;
     const float* wt = w + (size_t)t * tile_labels * K;
-    const bool vec = ((((uintptr_t)wt) & 15) == 0);
     const unsigned short* ep = pos16 + (size_t)row0 * 64 + lane;
     float* op = wp + (size_t)row0 * 64 + lane;
     unsigned lo = 0;                 // wave-uniform: rows below lo hold nothing of this or a later piece
     for (unsigned c0 = 0; c0 < npos; c0 += (unsigned)chunk) {
         const unsigned n = min((unsigned)chunk, npos - c0);
         __syncthreads();
-        if (vec) {
-            // all of a thread's loads go out before its first LDS write: one round trip per piece
-            const unsigned nv = n / 4;
-            const float4* src4 = reinterpret_cast<const float4*>(wt + c0);
-            float4* dst4 = reinterpret_cast<float4*>(ws);
-            for (unsigned q0 = threadIdx.x; q0 < nv; q0 += nthreads * 8) {
-                float4 v[8];
+        // all of a thread's loads go out before its first LDS write: one round trip per piece (of rows at any alignment)
+        const unsigned nv = n / 4;
+        const f32x4_unaligned* src4 = reinterpret_cast<const f32x4_unaligned*>(wt + c0);
+        float4* dst4 = reinterpret_cast<float4*>(ws);
+        for (unsigned q0 = threadIdx.x; q0 < nv; q0 += nthreads * 8) {
+            f32x4_unaligned v[8];
 #pragma unroll
-                for (int r = 0; r < 8; ++r) v[r] = src4[min(q0 + r * nthreads, nv - 1)];
+            for (int r = 0; r < 8; ++r) v[r] = src4[min(q0 + r * nthreads, nv - 1)];
 #pragma unroll
-                for (int r = 0; r < 8; ++r)
-                    if (q0 + r * nthreads < nv) dst4[q0 + r * nthreads] = v[r];
-            }
-            for (unsigned r = nv * 4 + threadIdx.x; r < n; r += nthreads) ws[r] = wt[c0 + r];
-        } else {
-            for (unsigned q = threadIdx.x; q < n; q += nthreads) ws[q] = wt[c0 + q];
+            for (int r = 0; r < 8; ++r)
+                if (q0 + r * nthreads < nv) dst4[q0 + r * nthreads] = make_float4(v[r].x, v[r].y, v[r].z, v[r].w);
         }
+        for (unsigned r = nv * 4 + threadIdx.x; r < n; r += nthreads) ws[r] = wt[c0 + r];
         __syncthreads();
         const unsigned hi = c0 + n;
         unsigned resume = 0xffffffffu;
@@ -389,7 +384,10 @@ int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, i
     FFI_TRY(workspace_get(s, kWsPartials, (size_t)streams * p->threads * bpad * sizeof(float), (void**)&partial));
     // large pieces (a whole tile of 1024 labels x 32 connections in one) as soon as the small one does not hold the
     // tile: every piece costs a walk over the tile's slots
-    const int chunk = ((long long)p->tile_labels * p->K <= kPermChunk) ? kPermChunk : kPermChunkBig;
+    // (and no larger than the tile, so that as many workgroups share a CU as the threads allow: plans of few columns have small ones;
+    // 369,076 labels x fan-in 61 over 24 columns, a wavefront each: 462 us with 64 KB per tile, 150 so)
+    const long long tile_weights = ((long long)p->tile_labels * p->K + 3) / 4 * 4;
+    const int chunk = (int)std::min<long long>(tile_weights, tile_weights <= kPermChunk ? kPermChunk : kPermChunkBig);
     if (!p->w_in_lds) {
         FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_permute_weights_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, chunk * 4));
         hipLaunchKernelGGL(igrad_permute_weights_kernel, dim3(p->tiles), dim3(p->threads), chunk * sizeof(float), s, p->pos16,
