@@ -390,6 +390,7 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
+constexpr int kWalkColumns = 128;          // columns of a workgroup that walks the global form, eight lanes each
 int plan_block_labels(int N, int K, int L);
 size_t plan_expected_slots(int N, int K, int L);
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s);

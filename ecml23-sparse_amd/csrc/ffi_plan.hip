@@ -741,10 +741,15 @@ void dev_release(ffi_plan* p, void* ptr) {
 
 // Labels per block of the global form: the block's rows of one slice of out_grad (128 bytes each) take five eighths of an
 // XCD's L2 -- shared by as many blocks as the workgroups of that many columns leave room for at a time -- unless the
-// lists of a block's columns would then hold fewer than eight connections.
+// lists of a block's columns would then hold fewer than eight connections.  Few columns (kWalkColumns to a workgroup of the walk) and
+// few labels get as many blocks as the CUs have workgroups for in one go, as far as the lists stay that long.  All passes at 126 x 1,242
+// x 15,823 x 95: 449 us with three blocks, 160 with 25; 128 x 2,000 x 13,330 x 32 197 and 97, 128 x 2,500 x 131,072 x 32 351 and 328.
+// (One block more, so that some CUs have two workgroups: 418 us at 128 x 1,300 x 131,072 x 32, where the former blocks took 345 and these 331.)
 int plan_block_labels(int N, int K, int L) {
     const double resident = 20480.0 * std::min(1.0, (double)N / 4096.0), filled = 8.0 * (double)N / (double)K;
-    const int labels = (int)std::min(65535.0, std::max(1024.0, std::max(resident, filled)));
+    const int chunks = (N + kWalkColumns - 1) / kWalkColumns, wanted = std::max(1, device_cu_count() / chunks);
+    const double busy = std::max(128.0, std::ceil((double)L / wanted));
+    const int labels = (int)std::min(65535.0, std::max(std::min(busy, 1024.0), std::max(std::min(resident, busy), filled)));
     return std::min(labels, L);
 }
 

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kWideThreads) void wgrad_wide_kernel(const float* _
 //
 // What bounds it: L2 delivery of the gathered rows (31 TB/s at most) and, with DOT, the instructions beside it (per oct and
 // lane 64 multiply-adds, 21 for the sums over the lanes, 8 gathers).
-constexpr int kWalkThreads = 1024;
+constexpr int kWalkThreads = kWalkColumns * 8;
 constexpr int kWalkMaxM = 4;
 // octs per window of a lane group, quads of it that a lane brings, and the window's place in LDS (16-byte words, one more
 // than it holds: the groups read from different banks)

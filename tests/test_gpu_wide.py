@@ -161,6 +161,21 @@ def test_forward_from_slices_in_lds_shares(ffi, bf16, B, N, L, K):
         assert (np.abs(out.cpu().numpy() - ref) <= (K + 2) * 2.0 ** -24 * size + 1e-30).all()
 
 
+# Wide inputs with few columns and few labels: more blocks than labels fill, lists of few connections, a last block of one label;
+# many blocks whose sums are added
+@pytest.mark.parametrize("B,N,L,K", [(5, 1_217, 130, 3), (33, 1_242, 3_201, 95), (64, 5_000, 129, 40), (17, 2_000, 13_331, 8), (3, 20_000, 700, 16)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_backward_over_many_label_blocks(ffi, B, N, L, K, transposed):
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=N + L)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    xd = dev(np.ascontiguousarray(x.T) if transposed else x)
+    call = ffi.fan_in_sparse_matmul_grad_tp if transposed else ffi.fan_in_sparse_matmul_grad
+    for _ in range(2):
+        gx, gw = call(xd, dev(lookup), dev(w), dev(g))
+        gx = gx.t() if transposed else gx
+        assert rel_err(gx.cpu().numpy(), o_gx) <= 2e-5 and rel_err(gw.cpu().numpy(), o_gw) <= 2e-5
+
+
 # Up to four samples, scores and answer in one launch: fan-ins of one quad, off the quads and of several passes over a row; fewer
 # labels than asked for, a label per lane and four, more workgroups than CUs; features that just fit
 @pytest.mark.parametrize("bf16", [False, True])
