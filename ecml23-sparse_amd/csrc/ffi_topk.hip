@@ -332,8 +332,8 @@ __global__ __launch_bounds__(256) void topk_select_kernel(float* cand_val, int* 
 // LDS, the products summed over the group by DPP.  Every lane keeps the best eight of the labels that fall to it, a workgroup the best
 // of its lanes'; the workgroup that ends last takes the best of those.
 //
-// What bounds it: the stream of ids and weights.  One sample, 768 columns, 670,091 labels, fan-in 32: 36.9 us, 4.7 TB/s;
-// a sample of the labels, a threshold, all scores and a selection took four launches and 67 us; four samples, k = 8, 60 against 71.
+// What bounds it: the stream of ids and weights.  One sample, 768 columns, 670,091 labels, fan-in 32: 35.6 us, 4.9 TB/s;
+// a sample of the labels, a threshold, all scores and a selection took four launches and 67 us; four samples 56 against 59.
 // (From eight samples on the sums over the lanes cost more than the launches.)
 constexpr int kDirectThreads = 1024;
 constexpr int direct_rounds(int bp) { return bp == 1 ? 4 : 2; }      // rounds of labels whose loads are in flight together
@@ -401,6 +401,7 @@ __device__ __forceinline__ void few_topk(const FewLabels& l, int k, FewShared& m
             const float v = m.v[threadIdx.x];
             const int id = m.id[threadIdx.x];
             int r = 0;
+#pragma unroll 8
             for (int s = 0; s < n; ++s) r += better(m.v[s], m.id[s], v, id);
             if (r < k) { m.out_v[r] = v; m.out_id[r] = id; }
         }
@@ -440,12 +441,14 @@ __global__ __launch_bounds__(kDirectThreads) void topk_direct_kernel(const void*
         for (int e = threadIdx.x; e < N * (BP - B); e += kDirectThreads) direct_xs[e / (BP - B) * BP + B + e % (BP - B)] = 0.f;
     __syncthreads();
     const int lane = threadIdx.x & 63, sub = lane & (lanes - 1), per_round = 64 / lanes;
-    const int wave = blockIdx.x * (kDirectThreads / 64) + (threadIdx.x >> 6), waves = gridDim.x * (kDirectThreads / 64);
-    const int step = waves * per_round * kDirectRounds;
+    const int step = gridDim.x * (kDirectThreads / 64) * per_round * kDirectRounds;
     FewLabels list[BP];
 #pragma unroll
     for (int b = 0; b < BP; ++b) list[b].clear();
-    auto label_of = [&](int j0, int u) { return j0 + u * per_round + lane / lanes; };
+    // (a round's labels from all wavefronts of the workgroup side by side: one whose few labels fell to few wavefronts had no bound from
+    // the others, 52 us at 1 x 500 x 150,000 x 8 where 12 are enough)
+    constexpr int kWaves = kDirectThreads / 64;
+    auto label_of = [&](int j0, int u) { return j0 + u * kWaves * per_round + lane / lanes; };
     Four<int> id[kDirectRounds];
     Four<T> wt[kDirectRounds];
     auto fetch = [&](int j0, int pass) {
@@ -457,7 +460,7 @@ __global__ __launch_bounds__(kDirectThreads) void topk_direct_kernel(const void*
             wt[u] = *reinterpret_cast<const Four<T>*>(w + at);
         }
     };
-    int j0 = wave * per_round * kDirectRounds, held = 0, place = 0, mine = kNoId;
+    int j0 = (blockIdx.x * kWaves * kDirectRounds + (threadIdx.x >> 6)) * per_round, held = 0, place = 0, mine = kNoId;
     float score[BP];
     // (NaN is no score: it takes no place)
     auto keep = [&]() {
@@ -545,31 +548,44 @@ __global__ __launch_bounds__(kDirectThreads) void topk_direct_kernel(const void*
     }
     __syncthreads();
     if (!last) return;
-    const int entries = (int)gridDim.x * k;
-    for (int b = 0; b < B; ++b) {
-        FewLabels l;
-        l.clear();
-        TopList more;
-        more.clear();
-        for (int e = threadIdx.x, t = 0; e < entries; e += kDirectThreads, ++t) {
-            const unsigned long long p = __hip_atomic_fetch_add(&part[((size_t)b * gridDim.x + e / k) * kTopMax + e % k], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const float v = __uint_as_float((unsigned)p);
-            const int id = (int)(p >> 32);
-            if (entries > kDirectHeld * kDirectThreads) {
-                if (id != kNoId) more.offer(v, id);
-            } else {
+    // The workgroups' best before their second best, and each in all wavefronts, whose best bound the answer: with a workgroup's entries
+    // in neighbouring lanes of few wavefronts the bound was none, 94 us at 4 x 500 x 10,000 x 32.  All samples' entries are on their way
+    // together.
+    const int entries = (int)gridDim.x * k, first = (threadIdx.x & 63) * (kDirectThreads / 64) + (threadIdx.x >> 6);
+    const bool few = entries <= kDirectHeld * kDirectThreads;
+    auto entry = [&](int b, int e) {
+        return __hip_atomic_load(&part[((size_t)b * gridDim.x + e % (int)gridDim.x) * kTopMax + e / (int)gridDim.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
 #pragma unroll
-                for (int q = 0; q < kDirectHeld; ++q)
-                    if (t == q) { l.v[q] = v; l.id[q] = id; }
+    for (int b = 0; b < BP; ++b) {
+        list[b].clear();
+        if (b >= B || !few) continue;
+#pragma unroll
+        for (int t = 0; t < kDirectHeld; ++t) {
+            const int e = first + t * kDirectThreads;
+            if (e < entries) {
+                const unsigned long long p = entry(b, e);
+                list[b].v[t] = __uint_as_float((unsigned)p);
+                list[b].id[t] = (int)(p >> 32);
             }
         }
-        if (entries > kDirectHeld * kDirectThreads) {
+    }
+#pragma unroll
+    for (int b = 0; b < BP; ++b) {
+        if (b >= B) break;
+        if (few) {
+            few_topk(list[b], k, shared);
+        } else {
+            TopList more;
+            more.clear();
+            for (int e = threadIdx.x; e < entries; e += kDirectThreads) {
+                const unsigned long long p = entry(b, e);
+                if ((int)(p >> 32) != kNoId) more.offer(__uint_as_float((unsigned)p), (int)(p >> 32));
+            }
             float ov;
             int oi;
             block_topk<kDirectThreads / 64>(more, k, ov, oi);
             if (threadIdx.x < kTopMax) { shared.out_v[threadIdx.x] = ov; shared.out_id[threadIdx.x] = oi; }
-        } else {
-            few_topk(l, k, shared);
         }
         if ((int)threadIdx.x < k) {
             values[(size_t)b * k + threadIdx.x] = shared.out_v[threadIdx.x];
@@ -667,7 +683,11 @@ TopkCandidates topk_candidates_at(void* ws, int B, int sample) {
 }
 
 int direct_width(int B) { return B <= 1 ? 1 : B <= 2 ? 2 : 4; }
+// A workgroup's k best take some 5 us a sample, which four samples have to save by the three launches and the second reading that there
+// are no more: fan-ins and labels (thousands) 8 x 400 33 us against 27, 32 x 400 47 and 46, 32 x 670 56 and 59, 100 x 300 73 and 111;
+// three samples 27 and 27, 40 and 45, 50 and 58, 66 and 110; one 13 and 26, 26 and 45, 35 and 58, 47 and 110.
 bool takes_topk_direct(const Dims& d) {
+    if (d.B == 4 && (long long)d.L * d.K < (16ll << 20)) return false;
     return d.B <= 4 && d.K >= 4 && (size_t)d.N * direct_width(d.B) * sizeof(float) <= kDirectLds;
 }
 
