@@ -161,7 +161,7 @@ constexpr int kHeavyBits = 12;     // labels with more set bits than this are le
 // ZERO_FILL == false: they are left alone.
 // `done(labels listed, how many, first label of the block)` comes behind each block of kWsBlock labels.  Returns the set bits that
 // the lane's labels had.
-constexpr int kWsLabelsPerLane = 4;
+constexpr int kWsLabelsPerLane = 4;                  // at most
 constexpr int kWsBlock = 64 * kWsLabelsPerLane;      // labels a wavefront looks at in one go
 
 struct SparseRows {
@@ -173,6 +173,7 @@ struct SparseRows {
     float* gw;
     float* bias_grad;
     int B, N, L, K, nbt;
+    int per_lane;                  // labels of a lane: 1, 2 or kWsLabelsPerLane
 };
 
 template <bool VEC4, bool ZERO_FILL, class Done>
@@ -193,18 +194,19 @@ __device__ __forceinline__ unsigned sparse_rows(const SparseRows& r, int block, 
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int wave = block * 4 + wv;
     const int nwaves = nblocks * 4;
-    const int nblk = (L + kWsBlock - 1) / kWsBlock;
+    const int block_labels = 64 * r.per_lane, nblk = (L + block_labels - 1) / block_labels;
     const unsigned tail = (B & 31) ? (1u << (B & 31)) - 1u : 0xffffffffu;   // bits past the batch are ignored
     const buffer_rsrc xr = make_rsrc(x, (size_t)B * (size_t)N * sizeof(float));
     unsigned* mylist = active_list[wv];
     for (int blk = wave; blk < nblk; blk += nwaves) {
-        const int block_base = blk * kWsBlock;
+        const int block_base = blk * block_labels;
         int cnts[kWsLabelsPerLane];
 #pragma unroll
         for (int q = 0; q < kWsLabelsPerLane; ++q) cnts[q] = 0;
         for (int t = 0; t < nbt; ++t) {
 #pragma unroll
             for (int q = 0; q < kWsLabelsPerLane; ++q) {
+                if (q >= r.per_lane) break;                             // (uniform)
                 unsigned m = words[(size_t)t * L + min(block_base + q * 64 + lane, L - 1)];
                 if (t == nbt - 1) m &= tail;
                 cnts[q] += __popc(m);
@@ -214,7 +216,7 @@ __device__ __forceinline__ unsigned sparse_rows(const SparseRows& r, int block, 
 #pragma unroll
         for (int q = 0; q < kWsLabelsPerLane; ++q) {
             const int base = block_base + q * 64;
-            if (base >= L) break;                                   // wave-uniform
+            if (base >= L || q >= r.per_lane) break;                // wave-uniform
             const int rows = min(64, L - base);
             const bool mine = lane < rows;
             const int cnt = cnts[q];
@@ -387,6 +389,12 @@ __global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const SparseRows r
 // launches).
 // (32 x 768 x 670,091 x 32, 0.2 % of the gradients not zero, late in training: two launches that count 9.6 us, the gradient 22, the
 // step on the weights 72 and on the bias 5.8; 98 so.  The whole step with its forward pass 183 -> 170.)
+__device__ __forceinline__ f32x4_unaligned& four_at(float* p) { return *reinterpret_cast<f32x4_unaligned*>(p); }
+__device__ __forceinline__ void adam_element(f32x4_unaligned& w, f32x4_unaligned& m, f32x4_unaligned& v, int q, float g, const AdamCoefficients& a) {
+    float wq = w[q], mq = m[q], vq = v[q];
+    adam_one(wq, mq, vq, g, a);
+    w[q] = wq; m[q] = mq; v[q] = vq;
+}
 struct AdamRows {
     float *var, *m, *v, *bias, *bias_m, *bias_v;
     AdamCoefficients a;
@@ -402,18 +410,20 @@ __global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, 
         const unsigned bits = sparse_rows<VEC4, false>(r, blockIdx.x, o.gradient_blocks, [&](const unsigned* list, int total, int base) {
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");        // (rows and list are the wavefront's own)
             __builtin_amdgcn_wave_barrier();
-            const int len = VEC4 ? r.K / 4 : r.K;
+            const int len = (r.K + 3) / 4;
             for (int e = lane; e < total * len; e += 64) {
-                const int i = e / len;
-                const size_t at = (size_t)(base + (int)(list[i] & 255u)) * len + (size_t)(e - i * len);
-                if (VEC4) {
-                    float4 w4 = reinterpret_cast<float4*>(o.var)[at], m4 = reinterpret_cast<float4*>(o.m)[at], v4 = reinterpret_cast<float4*>(o.v)[at];
-                    adam_four(w4, m4, v4, reinterpret_cast<const float4*>(r.gw)[at], o.a);
-                    reinterpret_cast<float4*>(o.var)[at] = w4;
-                    reinterpret_cast<float4*>(o.m)[at] = m4;
-                    reinterpret_cast<float4*>(o.v)[at] = v4;
+                const int i = e / len, k = 4 * (e - i * len), n = min(4, r.K - k);
+                const size_t at = (size_t)(base + (int)(list[i] & 255u)) * r.K + (size_t)k;
+                if (n == 4) {
+                    f32x4_unaligned w4 = four_at(o.var + at), m4 = four_at(o.m + at), v4 = four_at(o.v + at);
+                    const f32x4_unaligned g4 = four_at(r.gw + at);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) adam_element(w4, m4, v4, q, g4[q], o.a);
+                    four_at(o.var + at) = w4;
+                    four_at(o.m + at) = m4;
+                    four_at(o.v + at) = v4;
                 } else {
-                    adam_one(o.var[at], o.m[at], o.v[at], r.gw[at], o.a);
+                    for (int q = 0; q < n; ++q) adam_one(o.var[at + q], o.m[at + q], o.v[at + q], r.gw[at + q], o.a);
                 }
             }
             if (o.bias != nullptr)
@@ -457,39 +467,59 @@ __global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, 
             idle_row = lane < rows && set == 0u;
             idle = __ballot(idle_row);
         };
-        if (VEC4) {
-            const int len = r.K / 4, loads = rows * len;
-            const float inv_len = 1.f / (float)len;
-            float4* var = reinterpret_cast<float4*>(o.var) + (size_t)base * len;
-            float4* m = reinterpret_cast<float4*>(o.m) + (size_t)base * len;
-            float4* v = reinterpret_cast<float4*>(o.v) + (size_t)base * len;
-            // (all rows are read, so that nothing waits for the masks; what another wavefront makes of the ones with a set bit is not used)
-            constexpr int kAtOnce = 2;
-            for (int e0 = lane; e0 < loads; e0 += 64 * kAtOnce) {
-                float4 w4[kAtOnce], m4[kAtOnce], v4[kAtOnce];
+        // sixteen bytes of the rows at a time, where they end and begin does not matter; all rows are read, so that nothing waits for the
+        // masks (what another wavefront makes of the ones with a set bit is not used)
+        const int floats = rows * r.K, quads = floats / 4;
+        const float inv_len = 1.f / (float)r.K;
+        float* const var = o.var + (size_t)base * r.K;
+        float* const m = o.m + (size_t)base * r.K;
+        float* const v = o.v + (size_t)base * r.K;
+        auto row_of = [&](int e) {                                        // e / K, once it is set right
+            int row = (int)((float)e * inv_len);
+            row += e >= (row + 1) * r.K ? 1 : e < row * r.K ? -1 : 0;
+            return row;
+        };
+        constexpr int kAtOnce = 2;
+        bool looked = false;
+        for (int from = 0; from < quads; from += 64 * kAtOnce) {           // (all lanes: look() asks them all)
+            const int e0 = from + lane;
+            f32x4_unaligned w4[kAtOnce], m4[kAtOnce], v4[kAtOnce];
 #pragma unroll
-                for (int u = 0; u < kAtOnce; ++u) {
-                    const int e = min(e0 + 64 * u, loads - 1);
-                    w4[u] = var[e]; m4[u] = m[e]; v4[u] = v[e];
+            for (int u = 0; u < kAtOnce; ++u) {
+                const int e = 4 * min(e0 + 64 * u, quads - 1);
+                w4[u] = four_at(var + e); m4[u] = four_at(m + e); v4[u] = four_at(v + e);
+            }
+            if (!looked) { look(); looked = true; }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                const int e = 4 * (e0 + 64 * u);
+                if (e0 + 64 * u >= quads) continue;
+                const int row = row_of(e), end = (row + 1) * r.K;
+                bool on[4];
+                on[0] = (idle >> row & 1ull) != 0ull;
+                if (VEC4 || e + 4 <= end) {
+                    on[1] = on[2] = on[3] = on[0];
+                } else {
+#pragma unroll
+                    for (int q = 1; q < 4; ++q) on[q] = (idle >> row_of(e + q) & 1ull) != 0ull;
                 }
-                if (e0 == lane) look();
 #pragma unroll
-                for (int u = 0; u < kAtOnce; ++u) {
-                    const int e = e0 + 64 * u;
-                    int row = (int)((float)e * inv_len);                  // e / len, once it is set right
-                    row += e >= (row + 1) * len ? 1 : e < row * len ? -1 : 0;
-                    if (e >= loads || !(idle >> row & 1ull)) continue;
-                    adam_four(w4[u], m4[u], v4[u], make_float4(0.f, 0.f, 0.f, 0.f), o.a);
-                    var[e] = w4[u];
-                    m[e] = m4[u];
-                    v[e] = v4[u];
+                for (int q = 0; q < 4; ++q) adam_element(w4[u], m4[u], v4[u], q, 0.f, o.a);
+                if (on[0] && on[1] && on[2] && on[3]) {
+                    four_at(var + e) = w4[u];
+                    four_at(m + e) = m4[u];
+                    four_at(v + e) = v4[u];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (on[q]) { var[e + q] = w4[u][q]; m[e + q] = m4[u][q]; v[e + q] = v4[u][q]; }
                 }
             }
-        } else {
-            look();
-            const size_t from = (size_t)base * r.K;
-            for (int e = lane; e < rows * r.K; e += 64)
-                if (idle >> (e / r.K) & 1ull) adam_one(o.var[from + e], o.m[from + e], o.v[from + e], 0.f, o.a);
+        }
+        if (!looked) look();
+        if (!VEC4 && lane < (floats & 3)) {
+            const int e = 4 * quads + lane;
+            if (idle >> row_of(e) & 1ull) adam_one(var[e], m[e], v[e], 0.f, o.a);
         }
         if (o.bias != nullptr && idle_row) adam_one(o.bias[base + lane], o.bias_m[base + lane], o.bias_v[base + lane], 0.f, o.a);
     }
@@ -717,11 +747,22 @@ void nonzero_count_forget(int device) {
 }
 
 namespace {
+// Labels of a lane: as many as leave two workgroups for each CU.  (Batch 166 x 43 x 18,691 x 55, a step of which 28 % of the labels have
+// a gradient: PLOLD us with four each, PLNEW with one.)
+int sparse_per_lane(const Dims& d) {
+    int per = kWsLabelsPerLane;
+    while (per > 1 && (d.L + 256 * per - 1) / (256 * per) < 2 * device_cu_count()) per /= 2;
+    return per;
+}
 SparseRows sparse_rows_of(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad, const Dims& d) {
     // byte strides of x along the batch and along the features
-    return SparseRows{x, (d.tp ? 1u : (unsigned)d.N) * 4u, (d.tp ? (unsigned)d.B : 1u) * 4u, idx, g, words, gw, bias_grad, d.B, d.N, d.L, d.K, (d.B + 31) / 32};
+    return SparseRows{x, (d.tp ? 1u : (unsigned)d.N) * 4u, (d.tp ? (unsigned)d.B : 1u) * 4u, idx, g, words, gw, bias_grad, d.B, d.N, d.L, d.K, (d.B + 31) / 32,
+                      sparse_per_lane(d)};
 }
-int sparse_rows_blocks(const Dims& d) { return std::max(1, std::min(((d.L + kWsBlock - 1) / kWsBlock + 3) / 4, device_cu_count() * 8)); }
+int sparse_rows_blocks(const Dims& d) {
+    const int labels = 256 * sparse_per_lane(d);
+    return std::max(1, std::min((d.L + labels - 1) / labels, device_cu_count() * 8));
+}
 }  // namespace
 
 int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
