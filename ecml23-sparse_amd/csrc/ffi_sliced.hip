@@ -481,6 +481,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
         k = (int)f - l * n;
     };
     const unsigned row_pitch = (unsigned)row_step * (unsigned)K;          // (labels * row_step * K < 2^31)
+    const int per = min(chunk, K);                                        // connections of a chunk (a multiple of four where there are several)
     auto fetch = [&](int q, int k0) {
         const int kc = min(chunk, K - k0), j = q * S::kGroups;
 #pragma unroll
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
                 unsigned* w4 = &ws[v].x;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    place((unsigned)(64 * (4 * v + e) + lane), chunk, l, k);
+                    place((unsigned)(64 * (4 * v + e) + lane), per, l, k);
                     const unsigned at = (unsigned)min(j + min(l, S::kGroups - 1), L - 1) * row_pitch + (unsigned)(k0 + (k < kc ? k : 0));
                     id4[e] = (unsigned)idx[at];
                     w4[e] = BF16 ? (unsigned)w16[at] : w32[at];
@@ -530,7 +531,7 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
                 const unsigned id4[4] = {ids[v].x, ids[v].y, ids[v].z, ids[v].w}, w4[4] = {ws[v].x, ws[v].y, ws[v].z, ws[v].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    place((unsigned)(64 * (4 * v + e) + lane), chunk, l, k);
+                    place((unsigned)(64 * (4 * v + e) + lane), per, l, k);
                     if (l >= S::kGroups) continue;
                     const unsigned row = k < kc ? id4[e] * kRow : no_row, wv = k < kc ? w4[e] : 0u;       // (the walk takes four at a time)
                     if (BF16) {
@@ -543,6 +544,16 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
             }
         }
     };
+    if (!QUADS)                                                           // (the walk takes four at a time: what no chunk of a short fan-in writes)
+        for (int k = per; k < (per + 3) / 4 * 4; ++k)
+            for (int l = lane; l < S::kGroups; l += 64) {
+                if (BF16) {
+                    list[l * S::kPitch + k] = no_row;
+                    reinterpret_cast<unsigned short*>(list_w + l * S::kWeightPitch)[k] = 0;
+                } else {
+                    *reinterpret_cast<uint2*>(list + l * S::kPitch + 2 * k) = make_uint2(no_row, 0u);
+                }
+            }
     const unsigned* const mylist = list + grp * S::kPitch;
     const unsigned* const my_w = list_w + grp * S::kWeightPitch;
     // Rounds of kGroups consecutive labels.  The wavefronts take kRounds at a time, side by side, as long as all have some to take, then
