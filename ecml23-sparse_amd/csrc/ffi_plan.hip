@@ -742,13 +742,13 @@ void dev_release(ffi_plan* p, void* ptr) {
 // Labels per block of the global form: the block's rows of one slice of out_grad (128 bytes each) take five eighths of an
 // XCD's L2 -- shared by as many blocks as the workgroups of that many columns leave room for at a time -- unless the
 // lists of a block's columns would then hold fewer than eight connections.  Few columns (kWalkColumns to a workgroup of the walk) and
-// few labels get as many blocks as the CUs have workgroups for in one go, as far as the lists stay that long.  All passes at 126 x 1,242
+// few labels get as many blocks as the CUs have workgroups for in one go, as far as the lists keep twelve.  All passes at 126 x 1,242
 // x 15,823 x 95: 449 us with three blocks, 160 with 25; 128 x 2,000 x 13,330 x 32 197 and 97, 128 x 2,500 x 131,072 x 32 351 and 328.
 // (One block more, so that some CUs have two workgroups: 418 us at 128 x 1,300 x 131,072 x 32, where the former blocks took 345 and these 331.)
 int plan_block_labels(int N, int K, int L) {
     const double resident = 20480.0 * std::min(1.0, (double)N / 4096.0), filled = 8.0 * (double)N / (double)K;
     const int chunks = (N + kWalkColumns - 1) / kWalkColumns, wanted = std::max(1, device_cu_count() / chunks);
-    const double busy = std::max(128.0, std::ceil((double)L / wanted));
+    const double busy = std::max(std::max(128.0, 12.0 * N / K), std::ceil((double)L / wanted));
     const int labels = (int)std::min(65535.0, std::max(std::min(busy, 1024.0), std::max(std::min(resident, busy), filled)));
     return std::min(labels, L);
 }
@@ -1264,13 +1264,17 @@ int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
 
 namespace {
 int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigned long long* fp_out) {
+    // (what the host waits for first comes behind the work that is under way; the kernel below comes right behind it where there is one:
+    // 1,221 us for a rewiring at 128 x 768 x 670,091 x 32, 1,235 the other way round)
+    const bool wide = !tile_path_fits(p->N);
+    if (wide) FFI_TRY(plan_fingerprint_begin(p, lookup, s));
     // a rebuild replaces the arrays: whatever still reads the old ones must have drained
     if (!p->owned.empty()) FFI_HIP_TRY(hipDeviceSynchronize());
     free_arrays(p, true);                      // (their buffers serve the new arrays where they fit)
     // The ids are checked, and the words that later checks compare with are set, beside the kernel that assigns the labels' rows, which
     // takes any ids: the others' LDS counters want them in range.  (A rewiring and the pass behind it at 128 x 768 x 670,091
     // x 32: 1,280 us with the host waiting before that kernel, 1,252 so.)
-    FFI_TRY(plan_fingerprint_begin(p, lookup, s));
+    if (!wide) FFI_TRY(plan_fingerprint_begin(p, lookup, s));
     bool checked = false;
     auto check_ids = [&]() -> int {
         if (checked) return FFI_OK;

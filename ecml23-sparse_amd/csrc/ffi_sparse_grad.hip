@@ -748,7 +748,7 @@ void nonzero_count_forget(int device) {
 
 namespace {
 // Labels of a lane: as many as leave two workgroups for each CU.  (Batch 166 x 43 x 18,691 x 55, a step of which 28 % of the labels have
-// a gradient: PLOLD us with four each, PLNEW with one.)
+// a gradient: the whole step 128 us with four each, 95 with one.)
 int sparse_per_lane(const Dims& d) {
     int per = kWsLabelsPerLane;
     while (per > 1 && (d.L + 256 * per - 1) / (256 * per) < 2 * device_cu_count()) per /= 2;
