@@ -196,16 +196,22 @@ SmallShape small_shape(const Dims& d) {
 // Where the launches for small layers beat the paths made for large ones.  Forward: at 4 M products 14 us against 14 to 37, at 8 M
 // up to 21.  Backward, whose work is a visit of every connection per sample and window: at 4 M visits 31 to 39 us against 42 to
 // 320, at 8 M 48 to 75 against 44 to 205; 4 M sums of gx take 55 to 60 us against 92.
+// Layers of few labels give the larger paths few workgroups, each with all batch tiles one after the other.  Up to 1,024 labels,
+// backward: 128 x 1,000 x 1,000 x 64 61 us against 117, 256 x 300 x 1,024 x 40 73 against 85, 365 x 53 x 1,000 x 32 85 against 91 (12 M
+// visits; at 15 to 25 M 106 to 176 against 106 to 147); up to 512 and fan-ins up to 128: 365 x 53 x 549 x 45 67 against 119, 512 x 1,000
+// x 500 x 128 216 against 372 (fan-in 200 94 against 75).  Forward up to 512 labels and from fan-in 64 on: 128 x 300 x 256 x 200 15
+// against 119, 365 x 100 x 500 x 64 19 against 41, 128 x 768 x 500 x 128 18 against 30 (16 M products: 33 against 31).
 bool takes_small_forward(const Dims& d) {
     const long long sums = (long long)d.B * d.L * d.K;
     if (d.B > 65535 * kSmSamples) return false;            // (groups of samples are the grid's second dimension)
     if (g_options.small_path != 0) return g_options.small_path > 0 && sums < (1ll << 30);
-    return sums <= (4ll << 20);
+    return sums <= (4ll << 20) || (d.L <= 512 && d.K >= 64 && sums <= 12'000'000);
 }
 bool takes_small_backward(const Dims& d) {
     const long long visits = small_shape(d).units * d.L * d.K, cells = (long long)d.B * d.N;
     if (g_options.small_path != 0) return g_options.small_path > 0 && visits < (1ll << 30) && cells < (1ll << 30);
-    return visits <= (4ll << 20) && cells <= (4ll << 20);
+    const bool few_labels = (d.L <= 1024 && visits <= 12'000'000) || (d.L <= 512 && d.K <= 128 && visits <= (32ll << 20));
+    return (visits <= (4ll << 20) || (few_labels && d.N <= 1216)) && cells <= (4ll << 20);
 }
 
 int launch_forward_small(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s) {

@@ -1084,6 +1084,23 @@ def test_plan_form_and_gradients_at_few_columns(ffi, N, B, L, K):
             lib.ffi_set_option(b"small_path", 0)
 
 
+@pytest.mark.parametrize("shape", [(365, 53, 512, 65), (365, 53, 513, 20), (128, 300, 256, 200), (90, 1000, 1024, 65), (90, 1216, 1025, 65),
+                                   (500, 200, 512, 128), (500, 200, 500, 129), (300, 1217, 512, 64)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_layers_of_few_labels(ffi, shape, transposed):
+    # both sides of the lines up to which the launches for small layers take them
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=sum(shape))
+    ref = oracle.forward(x, lookup, w, transposed=False)
+    o_gx, o_gw = oracle.backward(x, lookup, w, g)
+    xd = dev(np.ascontiguousarray(x.T) if transposed else x)
+    out = (ffi.fan_in_sparse_matmul_tp if transposed else ffi.fan_in_sparse_matmul)(xd, dev(lookup), dev(w))
+    gx, gw = (ffi.fan_in_sparse_matmul_grad_tp if transposed else ffi.fan_in_sparse_matmul_grad)(xd, dev(lookup), dev(w), dev(g))
+    gx = gx.t() if transposed else gx
+    assert rel_err(out.cpu().numpy(), ref) <= 2e-5
+    assert rel_err(gx.cpu().numpy(), o_gx) <= GRAD_RTOL and rel_err(gw.cpu().numpy(), o_gw) <= GRAD_RTOL
+
+
 @pytest.mark.parametrize("batch", [1, 30, 31, 33, 34, 35, 64, 127])
 @pytest.mark.parametrize("features,labels,fan_in", [(100, 300, 32), (767, 4100, 9), (1000, 700, 40)])
 def test_rows_of_features_that_start_at_any_float(ffi, batch, features, labels, fan_in):
