@@ -479,7 +479,7 @@ __global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, 
             row += e >= (row + 1) * r.K ? 1 : e < row * r.K ? -1 : 0;
             return row;
         };
-        constexpr int kAtOnce = 2;
+        constexpr int kAtOnce = 4;
         bool looked = false;
         for (int from = 0; from < quads; from += 64 * kAtOnce) {           // (all lanes: look() asks them all)
             const int e0 = from + lane;
@@ -747,11 +747,11 @@ void nonzero_count_forget(int device) {
 }
 
 namespace {
-// Labels of a lane: as many as leave two workgroups for each CU.  (Batch 166 x 43 x 18,691 x 55, a step of which 28 % of the labels have
-// a gradient: the whole step 128 us with four each, 95 with one.)
+// Labels of a lane: as many as leave a workgroup for every second CU.  (Batch 166 x 43 x 18,691 x 55, a step of which 28 % of the labels
+// have a gradient: the whole step 128 us with four each, 97 with one; 41 x 4,096 x 245,894 x 5: 116 with four, 122 with two, 131 with one.)
 int sparse_per_lane(const Dims& d) {
     int per = kWsLabelsPerLane;
-    while (per > 1 && (d.L + 256 * per - 1) / (256 * per) < 2 * device_cu_count()) per /= 2;
+    while (per > 1 && (d.L + 256 * per - 1) / (256 * per) < device_cu_count() / 2) per /= 2;
     return per;
 }
 SparseRows sparse_rows_of(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad, const Dims& d) {
