@@ -388,7 +388,10 @@ __global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const SparseRows r
 // They also count the set bits, which the next call decides from (host_count; totals: a sum and a count of workgroups, zero between
 // launches).
 // (32 x 768 x 670,091 x 32, 0.2 % of the gradients not zero, late in training: two launches that count 9.6 us, the gradient 22, the
-// step on the weights 72 and on the bias 5.8; 98 so.  The whole step with its forward pass 183 -> 170.)
+// step on the weights 72 and on the bias 5.8; 93 so.  The whole step with its forward pass 183 -> 170.)
+//   A wavefront that steps looks at the masks of its labels first and leaves out the rows with a gradient, by accesses that the end of
+// a buffer keeps from memory: no branch parts the loads.  (All rows read beside the masks, 168 us for the whole step above, and this
+// 168; loads under branches 172.  What rows of other lengths share sixteen bytes of is read element by element, three a lane at most.)
 __device__ __forceinline__ f32x4_unaligned& four_at(float* p) { return *reinterpret_cast<f32x4_unaligned*>(p); }
 __device__ __forceinline__ void adam_element(f32x4_unaligned& w, f32x4_unaligned& m, f32x4_unaligned& v, int q, float g, const AdamCoefficients& a) {
     float wq = w[q], mq = m[q], vq = v[q];
@@ -402,6 +405,8 @@ struct AdamRows {
     unsigned long long* host_count;
     int gradient_blocks;
 };
+
+typedef unsigned four_words __attribute__((ext_vector_type(4)));
 
 template <bool VEC4>
 __global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, const AdamRows o) {
@@ -451,75 +456,80 @@ __global__ __launch_bounds__(256, 4) void wgrad_adam_kernel(const SparseRows r, 
         }
         return;
     }
-    // 64 labels per wavefront and step
+    // 64 labels per wavefront and step, sixteen bytes of their rows at a time, where those end and begin does not matter.  Rows with a set bit
+    // belong to another wavefront, which may be writing them: nothing of them is read (buffer accesses beyond the end do not touch memory).
     const int stepper = (int)blockIdx.x - o.gradient_blocks, steppers = gridDim.x - o.gradient_blocks;
     const unsigned tail = (r.B & 31) ? (1u << (r.B & 31)) - 1u : 0xffffffffu;
-    for (int base = (stepper * 4 + wv) * 64; base < r.L; base += steppers * 256) {
-        const int rows = min(64, r.L - base);
-        bool idle_row = false;
-        unsigned long long idle = 0ull;
-        auto look = [&]() {
-            unsigned set = 0u;
-            for (int t = 0; t < r.nbt; ++t) {
-                const unsigned m = r.words[(size_t)t * r.L + min(base + lane, r.L - 1)];
-                set |= t == r.nbt - 1 ? m & tail : m;
-            }
-            idle_row = lane < rows && set == 0u;
-            idle = __ballot(idle_row);
-        };
-        // sixteen bytes of the rows at a time, where they end and begin does not matter; all rows are read, so that nothing waits for the
-        // masks (what another wavefront makes of the ones with a set bit is not used)
-        const int floats = rows * r.K, quads = floats / 4;
-        const float inv_len = 1.f / (float)r.K;
-        float* const var = o.var + (size_t)base * r.K;
-        float* const m = o.m + (size_t)base * r.K;
-        float* const v = o.v + (size_t)base * r.K;
+    const float inv_len = 1.f / (float)r.K;
+    constexpr unsigned kNowhere = 0x80000000u;
+    for (long long first = (stepper * 4 + wv) * 64ll; first < r.L; first += steppers * 256ll) {
+        const int base = (int)first, rows = min(64, r.L - base);
+        unsigned set = 0u;
+        for (int t = 0; t < r.nbt; ++t) {
+            const unsigned m = r.words[(size_t)t * r.L + base + min(lane, rows - 1)];
+            set |= t == r.nbt - 1 ? m & tail : m;
+        }
+        const bool idle_row = lane < rows && set == 0u;
+        const unsigned long long idle = __ballot(idle_row);
+        const int all_quads = !VEC4 && r.K < 4 ? 0 : rows * r.K / 4;        // (rows of three and fewer go element by element)
+        const size_t at = (size_t)base * r.K;
         auto row_of = [&](int e) {                                        // e / K, once it is set right
-            int row = (int)((float)e * inv_len);
-            row += e >= (row + 1) * r.K ? 1 : e < row * r.K ? -1 : 0;
-            return row;
+            const int row = min((int)((float)e * inv_len), rows - 1);
+            return row + (e >= (row + 1) * r.K ? 1 : e < row * r.K ? -1 : 0);
         };
-        constexpr int kAtOnce = 4;
-        bool looked = false;
-        for (int from = 0; from < quads; from += 64 * kAtOnce) {           // (all lanes: look() asks them all)
-            const int e0 = from + lane;
-            f32x4_unaligned w4[kAtOnce], m4[kAtOnce], v4[kAtOnce];
-#pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) {
-                const int e = 4 * min(e0 + 64 * u, quads - 1);
-                w4[u] = four_at(var + e); m4[u] = four_at(m + e); v4[u] = four_at(v + e);
-            }
-            if (!looked) { look(); looked = true; }
-#pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) {
-                const int e = 4 * (e0 + 64 * u);
-                if (e0 + 64 * u >= quads) continue;
-                const int row = row_of(e), end = (row + 1) * r.K;
-                bool on[4];
-                on[0] = (idle >> row & 1ull) != 0ull;
-                if (VEC4 || e + 4 <= end) {
-                    on[1] = on[2] = on[3] = on[0];
-                } else {
-#pragma unroll
-                    for (int q = 1; q < 4; ++q) on[q] = (idle >> row_of(e + q) & 1ull) != 0ull;
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) adam_element(w4[u], m4[u], v4[u], q, 0.f, o.a);
-                if (on[0] && on[1] && on[2] && on[3]) {
-                    four_at(var + e) = w4[u];
-                    four_at(m + e) = m4[u];
-                    four_at(v + e) = v4[u];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (on[q]) { var[e + q] = w4[u][q]; m[e + q] = m4[u][q]; v[e + q] = v4[u][q]; }
-                }
+        auto load = [&](buffer_rsrc from, unsigned off) { return __builtin_bit_cast(f32x4_unaligned, __builtin_amdgcn_raw_buffer_load_b128(from, off, 0, 0)); };
+        auto store = [&](buffer_rsrc to, unsigned off, f32x4_unaligned q) { __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(four_words, q), to, off, 0, 0); };
+        // The lane's row ends in a quad that holds the first elements of the next one: where one of the two has a set bit, or the next
+        // is not there, the other's elements go one by one.  All elements of rows of three and fewer do.
+        int edge = 0;
+        size_t edge_at = at + (size_t)lane * r.K;
+        if (!VEC4 && lane < rows) {
+            const bool next = lane < 63 && (idle >> (lane + 1) & 1ull) != 0ull;
+            const int mine = (lane + 1) * r.K & 3;
+            if (r.K < 4) {
+                edge = idle_row ? r.K : 0;
+            } else if (mine != 0 && idle_row != next) {
+                edge = idle_row ? mine : 4 - mine;
+                edge_at += (size_t)(idle_row ? r.K - mine : r.K);
             }
         }
-        if (!looked) look();
-        if (!VEC4 && lane < (floats & 3)) {
-            const int e = 4 * quads + lane;
-            if (idle >> row_of(e) & 1ull) adam_one(var[e], m[e], v[e], 0.f, o.a);
+        float ew[3], em[3], ev[3];
+        if (!VEC4) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (i < edge) { ew[i] = o.var[edge_at + i]; em[i] = o.m[edge_at + i]; ev[i] = o.v[edge_at + i]; }
+        }
+        constexpr int kAtOnce = 4;
+        for (int from = 0; from < all_quads; from += 64 * kAtOnce) {
+            const int quads = min(all_quads - from, 64 * kAtOnce);
+            const size_t here = at + 4 * (size_t)from;
+            const buffer_rsrc wr = make_rsrc(o.var + here, quads * 16u), mr = make_rsrc(o.m + here, quads * 16u), vr = make_rsrc(o.v + here, quads * 16u);
+            f32x4_unaligned w4[kAtOnce], m4[kAtOnce], v4[kAtOnce];
+            unsigned off[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                if (64 * u >= quads) break;                               // (uniform)
+                const int q = lane + 64 * u, e = 4 * (from + min(q, quads - 1)), row = row_of(e);
+                bool on = (idle >> row & 1ull) != 0ull;
+                if (!VEC4 && e + 4 > (row + 1) * r.K) on = on && (idle >> (row + 1) & 1ull) != 0ull;
+                off[u] = on && q < quads ? 16u * (unsigned)q : kNowhere;
+                w4[u] = load(wr, off[u]); m4[u] = load(mr, off[u]); v4[u] = load(vr, off[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                if (64 * u >= quads) break;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) adam_element(w4[u], m4[u], v4[u], q, 0.f, o.a);
+                store(wr, off[u], w4[u]); store(mr, off[u], m4[u]); store(vr, off[u], v4[u]);
+            }
+        }
+        if (!VEC4) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (i < edge) {
+                    adam_one(ew[i], em[i], ev[i], 0.f, o.a);
+                    o.var[edge_at + i] = ew[i]; o.m[edge_at + i] = em[i]; o.v[edge_at + i] = ev[i];
+                }
         }
         if (o.bias != nullptr && idle_row) adam_one(o.bias[base + lane], o.bias_m[base + lane], o.bias_v[base + lane], 0.f, o.a);
     }
@@ -784,7 +794,7 @@ int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const flo
     std::lock_guard<std::mutex> lock(g_count_mutex);
     CountSlot* slot = nullptr;
     FFI_TRY(count_slot(dev, s, &slot));
-    const int gradient_blocks = sparse_rows_blocks(d), steps = (d.L + 255) / 256;
+    const int gradient_blocks = sparse_rows_blocks(d), steps = (int)(((long long)d.L + 255) / 256);
     const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx | (uintptr_t)v.weights | (uintptr_t)v.weight_m | (uintptr_t)v.weight_v) % 16 == 0);
     const AdamRows o{v.weights, v.weight_m, v.weight_v, v.bias, v.bias_m, v.bias_v, adam_coefficients(lr, beta_1, beta_2, eps, step),
                      reinterpret_cast<unsigned long long*>(tickets), slot->host, gradient_blocks};

@@ -164,6 +164,14 @@ def test_step_on_rows_with_and_without_gradient(ffi, shape, share):
         assert sparse == expected
 
 
+@pytest.mark.parametrize("shape,share", [((64, 30, 259, 5), 0.005), ((33, 20, 130, 6), 0.02), ((32, 40, 193, 13), 0.01), ((20, 30, 67, 4), 0.02),
+                                         ((16, 9, 1001, 2), 0.03), ((24, 9, 1001, 3), 0.02)])
+def test_step_on_rows_that_share_sixteen_bytes(ffi, shape, share):
+    # some of the rows have a gradient: sixteen bytes that lie in a row of either kind, at the end of a wavefront's 64 labels and of the layer,
+    # rows shorter than that
+    test_step_on_rows_with_and_without_gradient(ffi, shape, share)
+
+
 def test_fused_train_step_follows_the_unfused_loop(ffi):
     # layer.fused_train_step + optimizer.step() against forward_loss / backward / optimizer.step(), three steps
     B, N, L = 64, 128, 2000
