@@ -506,7 +506,7 @@ int ffi_backward_sparse_adam_f32(const float* features, const int32_t* lookup, f
             }
         }
         const AdamVariables v{weights, weight_m, weight_v, bias, bias_m, bias_v};
-        return launch_weight_grad_adam_sparse(features, lookup, out_grad, words, gw, gb, v, learning_rate, beta_1, beta_2, epsilon, (long long)step, d, s);
+        return launch_weight_grad_adam_sparse(features, lookup, out_grad, words, gw, gb, v, learning_rate, beta_1, beta_2, epsilon, (long long)step, d, set_bits, s);
     }
     // dense kernels: gradients into a workspace, then the Adam pass
     if (grad_is_partial) FFI_TRY(launch_zero_unmasked(out_grad, words, d.B, d.L, s));

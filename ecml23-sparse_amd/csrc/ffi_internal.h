@@ -226,14 +226,14 @@ bool nonzero_previous(int B, int L, hipStream_t s, unsigned long long* count_out
 int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw,
                               float* bias_grad, const Dims& d, hipStream_t s);
 // the same gradients, of which the rows without a set bit are not written, and the Adam step on the variables; leaves the number of
-// set bits for nonzero_previous.  Weights, moments and bias at any alignment of a
-// float (the entry point refuses a bias off 16 bytes, as the dense route has to); bias and its moments may be null.
+// set bits for nonzero_previous (set_bits: what is known of it, for the launch).  Weights, moments and bias at any alignment
+// of a float (the entry point refuses a bias off 16 bytes, as the dense route has to); bias and its moments may be null.
 struct AdamVariables {
     float *weights, *weight_m, *weight_v, *bias, *bias_m, *bias_v;
 };
 int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad,
                                    const AdamVariables& v, float lr, float beta_1, float beta_2, float eps, long long step, const Dims& d,
-                                   hipStream_t s);
+                                   unsigned long long set_bits, hipStream_t s);
 bool sparse_input_grad_fits(int N, int K);
 bool sparse_weight_grad_fits(int B, int N);   // x within 32-bit byte offsets
 // g[b,j] = 0 wherever the mask bit of (b,j) is clear

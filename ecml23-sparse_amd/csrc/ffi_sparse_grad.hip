@@ -786,7 +786,7 @@ int launch_weight_grad_sparse(const float* x, const int32_t* idx, const float* g
 
 int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const float* g, const unsigned* words, float* gw, float* bias_grad,
                                    const AdamVariables& v, float lr, float beta_1, float beta_2, float eps, long long step, const Dims& d,
-                                   hipStream_t s) {
+                                   unsigned long long set_bits, hipStream_t s) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     unsigned* tickets = nullptr;
@@ -794,11 +794,17 @@ int launch_weight_grad_adam_sparse(const float* x, const int32_t* idx, const flo
     std::lock_guard<std::mutex> lock(g_count_mutex);
     CountSlot* slot = nullptr;
     FFI_TRY(count_slot(dev, s, &slot));
-    const int gradient_blocks = sparse_rows_blocks(d), steps = (int)(((long long)d.L + 255) / 256);
+    // A CU holds four of the workgroups.  On layers of so many labels that the gradients' would take all these places first, and the steps
+    // begin when they end, they are fewer where few labels have a gradient: 8 x 400 x 1,000,000 x 5 with 1.6 % of the labels 95 us so many,
+    // 85 so; 32 x 400 x 1,000,000 and 6.4 %, fan-in 5 96 and 87, 32 263 and 259.  (64 samples, 13 % and fan-in 16: 193 and 200.  Little
+    // more than the limit is no good either, two rounds where there was one: 32 x 400 x 800,000 x 8 83 and 86.)
+    int gradient_blocks = sparse_rows_blocks(d);
+    const int cus = device_cu_count(), steps = (int)(((long long)d.L + 255) / 256);
+    if (4 * gradient_blocks >= 13 * cus && set_bits < (unsigned long long)d.L / 10) gradient_blocks = 11 * cus / 4;
     const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx | (uintptr_t)v.weights | (uintptr_t)v.weight_m | (uintptr_t)v.weight_v) % 16 == 0);
     const AdamRows o{v.weights, v.weight_m, v.weight_v, v.bias, v.bias_m, v.bias_v, adam_coefficients(lr, beta_1, beta_2, eps, step),
                      reinterpret_cast<unsigned long long*>(tickets), slot->host, gradient_blocks};
-    const int steppers = std::min(steps, device_cu_count() * 16);
+    const int steppers = std::min(steps, 16 * cus);
     hipLaunchKernelGGL((vec4 ? wgrad_adam_kernel<true> : wgrad_adam_kernel<false>), dim3(gradient_blocks + steppers), dim3(256), 0, s,
                        sparse_rows_of(x, idx, g, words, gw, bias_grad, d), o);
     FFI_HIP_TRY(hipGetLastError());

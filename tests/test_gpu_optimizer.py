@@ -165,10 +165,10 @@ def test_step_on_rows_with_and_without_gradient(ffi, shape, share):
 
 
 @pytest.mark.parametrize("shape,share", [((64, 30, 259, 5), 0.005), ((33, 20, 130, 6), 0.02), ((32, 40, 193, 13), 0.01), ((20, 30, 67, 4), 0.02),
-                                         ((16, 9, 1001, 2), 0.03), ((24, 9, 1001, 3), 0.02)])
+                                         ((16, 9, 1001, 2), 0.03), ((24, 9, 1001, 3), 0.02), ((8, 9, 900_001, 2), 0.005), ((8, 9, 900_001, 5), 0.005)])
 def test_step_on_rows_that_share_sixteen_bytes(ffi, shape, share):
     # some of the rows have a gradient: sixteen bytes that lie in a row of either kind, at the end of a wavefront's 64 labels and of the layer,
-    # rows shorter than that
+    # rows shorter than that, and layers of so many labels that the gradients' workgroups are limited
     test_step_on_rows_with_and_without_gradient(ffi, shape, share)
 
 
