@@ -241,6 +241,19 @@ __device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, flo
         }
     }
     xor_permute_groups(acc, lane & 7);
+    // A window's only stream has the sums (that many batch tiles leave one workgroup each: no ticket is drawn).
+    auto store4 = [&](int n, int b, const float4& v) {
+        const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (b + i < a.B) a.gx[TP ? (size_t)(col_lo + n) * a.B + b + i : (size_t)(b + i) * a.N + col_lo + n] = e[i];
+    };
+    if (a.s.streams == 1) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            if ((int)threadIdx.x < ncols) store4(threadIdx.x, b0 + 4 * c, make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]));
+        return;
+    }
     // The sums of kRedoTeam consecutive streams are added by the workgroup of theirs that finishes last, the teams' sums by the
     // last of those.  (All streams' by one workgroup: 1.4 ms for 256.)
     auto sums_of = [&](int st) { return a.partial + (((size_t)window * a.s.streams + st) * a.s.nbt + bt) * ((size_t)a.s.lower * kTileBatch); };
@@ -276,14 +289,8 @@ __device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, flo
     if (!last_of(tickets + team, in_team)) return;
     for (int q = threadIdx.x; q < quads; q += kRedoThreads) reinterpret_cast<float4*>(sums_of(lead))[q] = sum(q, in_team, 1);
     if (!last_of(tickets + teams, teams)) return;
-    for (int q = threadIdx.x; q < quads; q += kRedoThreads) {
-        const float4 v = sum(q, teams, kRedoTeam);
-        const int n = q / (kTileBatch / 4), b = b0 + q % (kTileBatch / 4) * 4;
-        const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (b + i < a.B) a.gx[TP ? (size_t)(col_lo + n) * a.B + b + i : (size_t)(b + i) * a.N + col_lo + n] = e[i];
-    }
+    for (int q = threadIdx.x; q < quads; q += kRedoThreads)
+        store4(q / (kTileBatch / 4), b0 + q % (kTileBatch / 4) * 4, sum(q, teams, kRedoTeam));
 }
 
 template <bool TP>
@@ -322,14 +329,14 @@ bool redo_shape(const Dims& d, RedoShape* s) {
     s->tiles = (d.L + tl - 1) / tl;
     s->streams = (s->tiles + s->tiles_per_stream - 1) / s->tiles_per_stream;
     s->lds = std::max(redo_lds_bytes(tl, d.K), tile_lds_bytes(d.N));
-    return (long long)s->nbt * s->windows * (redo_teams(s->streams) + 1) <= kTicketCount;
+    return s->streams == 1 || (long long)s->nbt * s->windows * (redo_teams(s->streams) + 1) <= kTicketCount;
 }
 
 }  // namespace
 
 size_t backward_if_outdated_workspace(const Dims& d) {
     RedoShape s;
-    return redo_shape(d, &s) ? (size_t)s.windows * s.streams * s.nbt * s.lower * kTileBatch * sizeof(float) : 0;
+    return redo_shape(d, &s) && s.streams > 1 ? (size_t)s.windows * s.streams * s.nbt * s.lower * kTileBatch * sizeof(float) : 0;
 }
 
 int backward_if_outdated_prepare(const Dims& d, hipStream_t s) {
@@ -352,8 +359,10 @@ int launch_backward_if_outdated(const unsigned long long* verdict, const float* 
         a.x = features; a.w = weights; a.g = out_grad; a.idx = lookup;
         a.gx = feature_grad; a.gw = gw; a.bias_grad = gb;
         a.B = d.B; a.N = d.N; a.L = d.L; a.K = d.K;
-        FFI_TRY(workspace_get(s, kWsPartials, backward_if_outdated_workspace(d), (void**)&a.partial));
-        FFI_TRY(tickets_get(s, (void**)&a.tickets));
+        if (a.s.streams > 1) {
+            FFI_TRY(workspace_get(s, kWsPartials, backward_if_outdated_workspace(d), (void**)&a.partial));
+            FFI_TRY(tickets_get(s, (void**)&a.tickets));
+        }
         const auto kernel = d.tp ? redo_backward_kernel<true> : redo_backward_kernel<false>;
         FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)a.s.lds));
         const int items = std::min(a.s.nbt * a.s.streams * a.s.windows, 4 * cus);

@@ -609,8 +609,9 @@ def test_in_place_rewiring_is_picked_up(ffi, shape):
 
 # What recomputes both gradients behind an outdated plan: one and several teams of label streams (16 each) and a team of one,
 # two windows of columns, a batch tile of one sample, fan-ins off the 16 connections of a unit, fewer units than threads and
-# several rounds of them
-@pytest.mark.parametrize("shape", [(33, 1200, 9001, 17), (7, 40, 30_000, 300), (1, 1216, 20_011, 33), (130, 64, 17_000, 15), (64, 768, 140_000, 32)])
+# several rounds of them, one stream only, and more batch tiles than there are counters for teams of streams
+@pytest.mark.parametrize("shape", [(33, 1200, 9001, 17), (7, 40, 30_000, 300), (1, 1216, 20_011, 33), (130, 64, 17_000, 15), (64, 768, 140_000, 32),
+                                   (5000, 900, 70, 3), (65_600, 80, 64, 4), (32_790, 1030, 40, 3)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_both_gradients_behind_an_outdated_plan(ffi, shape, transposed):
     B, N, L, K = shape
