@@ -704,7 +704,7 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
         // small layers walk no plan: one is built for the check of the ids
         if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
         // what recomputes the gradients behind an outdated plan
-        else if (backward_if_outdated_workspace(d) > 0) partial_slot = backward_if_outdated_workspace(d), total += kTicketCount * sizeof(unsigned);
+        else if (backward_if_outdated_workspace(d) > 0) total += backward_if_outdated_workspace(d) + kTicketCount * sizeof(unsigned);
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;
         if ((one_window || two_windows) && d.K <= 1024 && d.L < (1 << 25)) {
             // tiled plan: the geometry of ffi_plan.hip, the slot rows of a slice estimated for column ids drawn uniformly

@@ -54,23 +54,27 @@ __global__ __launch_bounds__(kFbBlock) void fallback_backward_kernel(const unsig
 // What is launched behind every backward pass and exits at once counts its launches: one of 256 workgroups, where a kernel per
 // gradient (and zeros by a third) took 3.8 us each.
 //
-// Weight gradient: the rows of one batch tile in LDS, a unit of (label, 32 connections) per thread, its sums in registers across
-// all batch tiles (ffi_weight_grad.hip).
+// Weight gradient: the rows of one batch tile in LDS, a unit of (label, 16 connections) per thread, its sums in registers across
+// all batch tiles (ffi_weight_grad.hip).  (32 connections: 54 spilled registers.)
 //
 // Input gradient: a workgroup takes a stream of label tiles for one batch tile and a window of the columns, a thread per column,
 // and sorts each tile's connections by column itself: counts per column (integer LDS atomics), an exclusive scan, then every
 // connection takes the next free place of its column's bucket.  Thread t then walks the bucket of column col_lo + t, gathering
 // rows of the tile's out_grad from LDS.  No slot balancing (rows lie in label order, so row parities are random and the reads
-// run at the 8-clock rate; a wavefront walks as long as its longest bucket), and the order inside a bucket is whatever the
-// atomics gave: sums are not reproducible bit for bit.  The workgroups that finish last add the streams' sums
-// up.  (670,091 labels x fan-in 32 over 768 columns, batch 128: float atomics into an LDS tile of gx -- ds_add_f32
-// retires a third of a lane per clock and CU here, integer atomics seven lanes -- took 14.3 ms.)
+// run at the 8-clock rate; a wavefront walks as long as its longest bucket), and the order inside a bucket and of the streams is
+// whatever the atomics gave: sums are not reproducible bit for bit.  (670,091 labels x fan-in 32 over 768 columns, batch 128: float
+// atomics into an LDS tile of gx -- ds_add_f32 retires a third of a lane per clock and CU here, integer atomics seven lanes -- took
+// 14.3 ms.)
+//
+// What bounds it: a CU holds one workgroup, so each of its phases has to have its loads in flight together -- ids and weights eight at
+// a time (one: 1,640 us for the pass behind an edit of that layer, 1,450 so), features of [B,N] by four columns of four samples (element
+// by element, all to one pair of LDS banks: 2,050) -- and the streams' sums must not wait for each other: atomics on memory with the
+// columns side by side (32 x 768 x 131,072 x 32 176 us; partial sums that the last workgroup of 16 and then the last of all added up,
+// each behind a device-scope fence, 400; the columns 32 samples apart in [N,B], as two kernels before, 435).
 // LDS: gs[tile_labels][32] | ws[tile_labels * K] | lst[tile_labels * K] | cursor[threads] | wave sums[16].
 constexpr int kRedoThreads = 1024;
+constexpr int kRedoInFlight = 8;      // loads of a thread, in loops that hand each value to LDS
 constexpr int kRedoChunk = 16;        // connections per unit of the weight gradient
-
-constexpr int kRedoTeam = 16;         // streams whose sums are added first
-__host__ __device__ constexpr int redo_teams(int streams) { return (streams + kRedoTeam - 1) / kRedoTeam; }
 
 struct RedoShape {
     int nbt, windows, lower;              // batch tiles; windows of the columns, the first one's size
@@ -82,8 +86,8 @@ struct RedoArgs {
     const float *x, *w, *g;
     const int32_t* idx;
     float *gx, *gw, *bias_grad;           // gx or gw may be null
-    float* partial;                       // [window][stream][batch tile][lower][32]
-    unsigned* tickets;                    // [window][batch tile][teams + 1], zero between launches
+    double* sums;                         // [window][batch tile][32][lower], zero between launches
+    unsigned* tickets;                    // [window][batch tile], zero between launches
     int B, N, L, K;
     RedoShape s;
 };
@@ -114,10 +118,7 @@ __device__ __forceinline__ void redo_weight_grad(const RedoArgs& a, float* xs) {
             if (TP) {
                 stage_rows32<kRedoThreads>(xs, a.x, a.N, a.B, b0);
             } else {
-                for (int e = threadIdx.x; e < a.N * kTileBatch; e += kRedoThreads) {
-                    const int b = e / a.N, n = e - b * a.N;
-                    xs[n * kTileBatch + b] = b0 + b < a.B ? a.x[(size_t)(b0 + b) * a.N + n] : 0.f;
-                }
+                stage_columns32<kRedoThreads>(xs, a.x, a.N, a.B, b0);
             }
             __syncthreads();
             unsigned skew = (unsigned)(size_t)(__attribute__((address_space(3))) float*)xs + (unsigned)(lane & 7) * 16u;
@@ -192,11 +193,28 @@ __device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, flo
             for (int c = 0; c < 8; ++c)
                 *reinterpret_cast<float4*>(rowp + ((c ^ r) << 4)) = make_float4(gb[4 * c], gb[4 * c + 1], gb[4 * c + 2], gb[4 * c + 3]);
         }
-        for (int q = threadIdx.x; q < total; q += kRedoThreads) ws[q] = a.w[(size_t)j0 * K + q];
+        for (int q0 = threadIdx.x; q0 < total; q0 += kRedoInFlight * kRedoThreads) {
+            float v[kRedoInFlight];
+#pragma unroll
+            for (int i = 0; i < kRedoInFlight; ++i) v[i] = a.w[(size_t)j0 * K + min(q0 + i * kRedoThreads, total - 1)];
+#pragma unroll
+            for (int i = 0; i < kRedoInFlight; ++i)
+                if (q0 + i * kRedoThreads < total) ws[q0 + i * kRedoThreads] = v[i];
+        }
         __syncthreads();
-        for (int e = threadIdx.x; e < total; e += kRedoThreads) {
-            const unsigned c = (unsigned)(src[e] - col_lo);             // (ids outside [0, N) or outside the window: skipped)
-            if (c < (unsigned)ncols) atomicAdd(&cursor[c], 1);
+        // the thread's entries e0 + i * kRedoThreads: column inside the window (ids outside [0, N) or outside the window: beyond it)
+        auto columns = [&](int e0, unsigned (&c)[kRedoInFlight]) {
+#pragma unroll
+            for (int i = 0; i < kRedoInFlight; ++i) c[i] = (unsigned)(src[min(e0 + i * kRedoThreads, total - 1)] - col_lo);
+#pragma unroll
+            for (int i = 0; i < kRedoInFlight; ++i) c[i] = e0 + i * kRedoThreads < total ? c[i] : ~0u;
+        };
+        for (int e0 = threadIdx.x; e0 < total; e0 += kRedoInFlight * kRedoThreads) {
+            unsigned c[kRedoInFlight];
+            columns(e0, c);
+#pragma unroll
+            for (int i = 0; i < kRedoInFlight; ++i)
+                if (c[i] < (unsigned)ncols) atomicAdd(&cursor[c[i]], 1);
         }
         __syncthreads();
         // exclusive scan of the counts over the workgroup
@@ -218,11 +236,15 @@ __device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, flo
             // (label of entry e without a division per entry: the thread's entries are kRedoThreads apart)
             int l = (int)threadIdx.x / K, k = (int)threadIdx.x - l * K;
             const int dl = kRedoThreads / K, dk = kRedoThreads - dl * K;
-            for (int e = threadIdx.x; e < total; e += kRedoThreads) {
-                const unsigned c = (unsigned)(src[e] - col_lo);
-                if (c < (unsigned)ncols) lst[atomicAdd(&cursor[c], 1)] = ((unsigned)e << 10) | (unsigned)l;
-                l += dl; k += dk;
-                if (k >= K) { k -= K; ++l; }
+            for (int e0 = threadIdx.x; e0 < total; e0 += kRedoInFlight * kRedoThreads) {
+                unsigned c[kRedoInFlight];
+                columns(e0, c);
+#pragma unroll
+                for (int i = 0; i < kRedoInFlight; ++i) {
+                    if (c[i] < (unsigned)ncols) lst[atomicAdd(&cursor[c[i]], 1)] = (unsigned)(e0 + i * kRedoThreads) << 10 | (unsigned)l;
+                    l += dl; k += dk;
+                    if (k >= K) { k -= K; ++l; }
+                }
             }
         }
         __syncthreads();
@@ -241,56 +263,32 @@ __device__ __forceinline__ void redo_input_grad(const RedoArgs& a, int item, flo
         }
     }
     xor_permute_groups(acc, lane & 7);
-    // A window's only stream has the sums (that many batch tiles leave one workgroup each: no ticket is drawn).
-    auto store4 = [&](int n, int b, const float4& v) {
-        const float e[4] = {v.x, v.y, v.z, v.w};
+    auto column = [&](int n, int b) -> float& { return a.gx[TP ? (size_t)(col_lo + n) * a.B + b0 + b : (size_t)(b0 + b) * a.N + col_lo + n]; };
+    const int nb = min(kTileBatch, a.B - b0);
+    if (a.s.streams == 1) {                                    // (few labels, or so many batch tiles that one workgroup each is all)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (b + i < a.B) a.gx[TP ? (size_t)(col_lo + n) * a.B + b + i : (size_t)(b + i) * a.N + col_lo + n] = e[i];
-    };
-    if (a.s.streams == 1) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if ((int)threadIdx.x < ncols) store4(threadIdx.x, b0 + 4 * c, make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]));
+        for (int b = 0; b < kTileBatch; ++b)
+            if ((int)threadIdx.x < ncols && b < nb) column(threadIdx.x, b) = acc[b];
         return;
     }
-    // The sums of kRedoTeam consecutive streams are added by the workgroup of theirs that finishes last, the teams' sums by the
-    // last of those.  (All streams' by one workgroup: 1.4 ms for 256.)
-    auto sums_of = [&](int st) { return a.partial + (((size_t)window * a.s.streams + st) * a.s.nbt + bt) * ((size_t)a.s.lower * kTileBatch); };
-    float* out = sums_of(stream) + threadIdx.x * kTileBatch;
+    // The streams add their sums up in memory that is zero between launches, the columns of a sample side by side, in 64 bits (up to 256
+    // streams in any order: 3.0e-7 of the result in 32, 1.4e-7 by teams of 16 and so); who adds last takes them from there.  All of that is done by atomics at device scope, which are waited for before the ticket is drawn.
+    double* const sums = a.sums + (size_t)(window * a.s.nbt + bt) * ((size_t)a.s.lower * kTileBatch);
 #pragma unroll
-    for (int c = 0; c < 8; ++c)
-        if ((int)threadIdx.x < ncols) *reinterpret_cast<float4*>(out + 4 * c) = make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]);
-    const int teams = redo_teams(a.s.streams), team = stream / kRedoTeam, lead = team * kRedoTeam;
-    unsigned* const tickets = a.tickets + (size_t)(window * a.s.nbt + bt) * (teams + 1);
-    auto last_of = [&](unsigned* ticket, int count) {
-        __threadfence();
-        __syncthreads();
-        if (threadIdx.x == 0) wave_sum[0] = atomicAdd(ticket, 1u) == (unsigned)count - 1u;
-        __syncthreads();
-        const bool last = wave_sum[0] != 0;
-        if (last) {
-            __threadfence();
-            if (threadIdx.x == 0) *ticket = 0u;
-        }
-        return last;
-    };
-    auto sum = [&](int q, int count, int step) {               // of quad q over `count` streams from `lead` or the first on
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        const int from = step == 1 ? lead : 0;
+    for (int b = 0; b < kTileBatch; ++b)
+        if ((int)threadIdx.x < ncols && b < nb) unsafeAtomicAdd(&sums[(size_t)b * a.s.lower + threadIdx.x], (double)acc[b]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned* const ticket = a.tickets + window * a.s.nbt + bt;
+    if (threadIdx.x == 0) wave_sum[0] = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)a.s.streams - 1u;
+    __syncthreads();
+    if (wave_sum[0] == 0) return;
 #pragma unroll 8
-        for (int i = 0; i < count; ++i) {
-            const float4 p = reinterpret_cast<const float4*>(sums_of(from + i * step))[q];
-            v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
-        }
-        return v;
-    };
-    const int quads = ncols * (kTileBatch / 4), in_team = min(kRedoTeam, a.s.streams - lead);
-    if (!last_of(tickets + team, in_team)) return;
-    for (int q = threadIdx.x; q < quads; q += kRedoThreads) reinterpret_cast<float4*>(sums_of(lead))[q] = sum(q, in_team, 1);
-    if (!last_of(tickets + teams, teams)) return;
-    for (int q = threadIdx.x; q < quads; q += kRedoThreads)
-        store4(q / (kTileBatch / 4), b0 + q % (kTileBatch / 4) * 4, sum(q, teams, kRedoTeam));
+    for (int e = threadIdx.x; e < nb * ncols; e += kRedoThreads) {
+        const int b = e / ncols, n = e - b * ncols;
+        column(n, b) = (float)__hip_atomic_exchange(&sums[(size_t)b * a.s.lower + n], 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <bool TP>
@@ -329,21 +327,21 @@ bool redo_shape(const Dims& d, RedoShape* s) {
     s->tiles = (d.L + tl - 1) / tl;
     s->streams = (s->tiles + s->tiles_per_stream - 1) / s->tiles_per_stream;
     s->lds = std::max(redo_lds_bytes(tl, d.K), tile_lds_bytes(d.N));
-    return s->streams == 1 || (long long)s->nbt * s->windows * (redo_teams(s->streams) + 1) <= kTicketCount;
+    return s->streams == 1 || (long long)s->nbt * s->windows <= kTicketCount;
 }
 
 }  // namespace
 
 size_t backward_if_outdated_workspace(const Dims& d) {
     RedoShape s;
-    return redo_shape(d, &s) && s.streams > 1 ? (size_t)s.windows * s.streams * s.nbt * s.lower * kTileBatch * sizeof(float) : 0;
+    return redo_shape(d, &s) && s.streams > 1 ? (size_t)s.windows * s.nbt * s.lower * kTileBatch * sizeof(double) : 0;
 }
 
 int backward_if_outdated_prepare(const Dims& d, hipStream_t s) {
     void* ws = nullptr;
     const size_t bytes = backward_if_outdated_workspace(d);
     if (bytes == 0) return FFI_OK;
-    FFI_TRY(workspace_get(s, kWsPartials, bytes, &ws));
+    FFI_TRY(zeroed_get(s, kWsSums, bytes, &ws));
     return tickets_get(s, &ws);
 }
 
@@ -360,7 +358,7 @@ int launch_backward_if_outdated(const unsigned long long* verdict, const float* 
         a.gx = feature_grad; a.gw = gw; a.bias_grad = gb;
         a.B = d.B; a.N = d.N; a.L = d.L; a.K = d.K;
         if (a.s.streams > 1) {
-            FFI_TRY(workspace_get(s, kWsPartials, backward_if_outdated_workspace(d), (void**)&a.partial));
+            FFI_TRY(zeroed_get(s, kWsSums, backward_if_outdated_workspace(d), (void**)&a.sums));
             FFI_TRY(tickets_get(s, (void**)&a.tickets));
         }
         const auto kernel = d.tp ? redo_backward_kernel<true> : redo_backward_kernel<false>;

@@ -67,11 +67,13 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11, kWsSums = 12 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 // 128 bytes of pinned host memory of the stream, for results that the host waits for
 int host_words_get(hipStream_t s, void** out);
-// 4,096 counters of the stream that are zero between launches (a kernel that counts in them puts them back)
+// The same, for memory that is zero between launches (a kernel that adds to it puts it back).
+int zeroed_get(hipStream_t s, int slot, size_t bytes, void** out);
+// 4,096 counters of that kind
 constexpr int kTicketCount = 4096;
 int tickets_get(hipStream_t s, void** out);
 void workspace_clear(int device);

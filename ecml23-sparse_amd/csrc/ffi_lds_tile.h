@@ -63,6 +63,34 @@ __device__ __forceinline__ void stage_rows32(float* __restrict__ xs, const float
     }
 }
 
+// xs[n][b] = src[(b0 + b) * ld + n] for b < 32 (zero beyond `rows`), n < ld: four columns of four rows per thread and step, eight
+// threads side by side for the 32 rows.
+template <int THREADS>
+__device__ __forceinline__ void stage_columns32(float* __restrict__ xs, const float* __restrict__ src, int ld, int rows, int b0) {
+    const int c = threadIdx.x & 7;
+#pragma unroll 1
+    for (int n = (threadIdx.x >> 3) * 4; n < ld; n += THREADS / 2) {
+        float v[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int b = b0 + 4 * c + i;
+            const float* from = src + (size_t)min(b, rows - 1) * ld + n;
+            if (n + 4 <= ld) {
+                const f32x4_unaligned q = *reinterpret_cast<const f32x4_unaligned*>(from);
+                v[i][0] = q.x; v[i][1] = q.y; v[i][2] = q.z; v[i][3] = q.w;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[i][k] = from[min(k, ld - 1 - n)];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[i][k] = b < rows ? v[i][k] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (n + k < ld) *reinterpret_cast<float4*>(xs + (size_t)(n + k) * kTileBatch + 4 * c) = make_float4(v[0][k], v[1][k], v[2][k], v[3][k]);
+    }
+}
+
 // Raw buffer resource over `bytes` bytes at p (gfx9 family: 32-bit data format word).  Loads
 // through it take a per-lane byte offset plus a wave-uniform (scalar) byte offset, and reads
 // beyond `bytes` return zero instead of faulting.

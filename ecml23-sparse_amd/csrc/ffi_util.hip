@@ -111,17 +111,22 @@ int workspace_get(hipStream_t s, int slot, size_t bytes, void** out) {
     return FFI_OK;
 }
 
-int tickets_get(hipStream_t s, void** out) {
+int zeroed_get(hipStream_t s, int slot, size_t bytes, void** out) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    for (WsEntry& e : g_ws) {
-        if (e.device == dev && e.stream == s && e.slot == kWsTickets) {
-            *out = e.ptr;
+    for (size_t i = 0; i < g_ws.size(); ++i) {
+        if (g_ws[i].device != dev || g_ws[i].stream != s || g_ws[i].slot != slot) continue;
+        if (g_ws[i].bytes >= bytes) {
+            *out = g_ws[i].ptr;
             return FFI_OK;
         }
+        FFI_HIP_TRY(hipStreamSynchronize(s));                     // (work queued on this stream may still use it)
+        (void)hipFree(g_ws[i].ptr);
+        g_ws.erase(g_ws.begin() + i);
+        break;
     }
-    WsEntry e{dev, s, kWsTickets, nullptr, kTicketCount * sizeof(unsigned)};
+    WsEntry e{dev, s, slot, nullptr, bytes};
     if (hipMalloc(&e.ptr, e.bytes) != hipSuccess) { (void)hipGetLastError(); return FFI_ERR_OUT_OF_MEMORY; }
     const hipError_t err = hipMemset(e.ptr, 0, e.bytes);          // (once, and waited for)
     if (err != hipSuccess || hipDeviceSynchronize() != hipSuccess) { (void)hipFree(e.ptr); return hip_fail(err); }
@@ -129,6 +134,8 @@ int tickets_get(hipStream_t s, void** out) {
     *out = e.ptr;
     return FFI_OK;
 }
+
+int tickets_get(hipStream_t s, void** out) { return zeroed_get(s, kWsTickets, kTicketCount * sizeof(unsigned), out); }
 
 int host_words_get(hipStream_t s, void** out) {
     int dev = -1;
