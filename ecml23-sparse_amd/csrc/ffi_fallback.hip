@@ -69,8 +69,8 @@ __global__ __launch_bounds__(kFbBlock) void fallback_backward_kernel(const unsig
 // What bounds it: a CU holds one workgroup, so each of its phases has to have its loads in flight together -- ids and weights eight at
 // a time (one: 1,640 us for the pass behind an edit of that layer, 1,450 so), features of [B,N] by four columns of four samples (element
 // by element, all to one pair of LDS banks: 2,050) -- and the streams' sums must not wait for each other: atomics on memory with the
-// columns side by side (32 x 768 x 131,072 x 32 176 us; partial sums that the last workgroup of 16 and then the last of all added up,
-// each behind a device-scope fence, 400; the columns 32 samples apart in [N,B], as two kernels before, 435).
+// columns side by side (32 x 768 x 131,072 x 32 in [B,N] 184 us; partial sums that the last workgroup of 16 and then the last of all added up,
+// each behind a device-scope fence, 400; in 32 bits 170; and with the columns 32 samples apart, in [N,B], 430).
 // LDS: gs[tile_labels][32] | ws[tile_labels * K] | lst[tile_labels * K] | cursor[threads] | wave sums[16].
 constexpr int kRedoThreads = 1024;
 constexpr int kRedoInFlight = 8;      // loads of a thread, in loops that hand each value to LDS

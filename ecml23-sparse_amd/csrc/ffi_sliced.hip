@@ -370,11 +370,14 @@ __global__ __launch_bounds__(kSlThreads) void fwd_sliced_kernel(const void* __re
 // 16 GL bytes per connection and lane group, and the lists) and the instructions around it.
 //   Scores leave from the registers: the lanes' low bits change places with the rounds (exchange_bit), which makes pieces of 32
 // labels without the tile in LDS that took them through it twice more; pieces of 32 bytes cost 140 us at 128 x 768 x 300,000 x 32
-// in bf16, the tile 112, these 89.  What a lane fetches is the same place of every chunk, so its divisions are done once.
+// in bf16, the tile 112, these 84.  What a lane fetches is the same place of every chunk, so its divisions are done once.
 //   A wavefront takes 32 labels at a time, the last ones in even shares; with fewer labels than that for all, the workgroups are
 // as many as give each wavefront one round (64 x 768 x 8,192 x 32 in bf16: 28.7 us with 32 labels each, 18.0 so).
 //   The slice comes in with four columns of a lane's four samples per step, lanes side by side holding a row of the slice: with
 // a column per lane, 32 lanes wrote to one pair of banks (the same shape: 18.0 -> 14.4 us, a first list already in flight).
+// COLUMNS: [B,N] of eight samples comes in by a column's samples per lane all the same, one way or the other and not both in one
+// kernel, whose first instructions are some of its 7 us.  From more than 512 columns on: top-k of 5 x 768 x 30,000 x 16 27.2 us by four
+// columns, 26.8 so; 400 columns 26.7 and 27.0, 300 and fewer the same.
 //   At 100 x 500 x 131,073 x 24 in bf16, all of it together: 45.6 -> 36.4 us.
 typedef unsigned lds_v4u __attribute__((ext_vector_type(4)));
 constexpr int kLdThreads = 1024;
@@ -401,7 +404,7 @@ template <int CTRL> __device__ __forceinline__ void exchange_bit(bool bit, float
     b = bit ? b : other;
 }
 
-template <int GL, bool BF16, bool QUADS>
+template <int GL, bool BF16, bool QUADS, bool COLUMNS = false>
 __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restrict__ features, const int32_t* __restrict__ idx,
                                                              const void* __restrict__ w, const float* __restrict__ bias,
                                                              float* __restrict__ out, int B, int N, int L, int K, int tp, int row_step,
@@ -440,6 +443,18 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
                 Quad<T> q = read4(n, b);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) q.v[i] = b + i < B ? q.v[i] : (T)0;
+                dst[n * kQ + c] = q;
+            }
+        } else if constexpr (COLUMNS) {
+#pragma unroll 4
+            for (int e = threadIdx.x; e < N * kQ; e += kLdThreads) {
+                const int n = e % N, c = e / N, b = slice * kSl + 4 * c;
+                Quad<T> q;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const T v = x[(size_t)min(b + i, B - 1) * N + n];
+                    q.v[i] = b + i < B ? v : (T)0;
+                }
                 dst[n * kQ + c] = q;
             }
         } else {
@@ -981,17 +996,16 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
     const size_t lds = lds_kernel_bytes<GL, BF16>(d.N) + (a.sink.tau != nullptr ? kLdThresholdBytes : 0);
     static_assert(2 * GL * LaneAcc<BF16>::kSamples * 4 <= kLdThresholdBytes, "thresholds of a slice");
     const dim3 grid((unsigned)(streams * a.slices)), block(kLdThreads);
-    if (a.quads) {
-        FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lds_kernel<GL, BF16, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((fwd_lds_kernel<GL, BF16, true>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0,
-                           a.row_step, a.slices, streams, chunk, a.sink);
-    } else {
-        FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lds_kernel<GL, BF16, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((fwd_lds_kernel<GL, BF16, false>), grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0,
-                           a.row_step, a.slices, streams, chunk, a.sink);
-    }
-    FFI_HIP_TRY(hipGetLastError());
-    return FFI_OK;
+    auto go = [&](auto kernel) -> int {
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0, a.row_step, a.slices,
+                           streams, chunk, a.sink);
+        FFI_HIP_TRY(hipGetLastError());
+        return FFI_OK;
+    };
+    if constexpr (GL == 2 && !BF16)
+        if (!d.tp && d.N > 512) return a.quads ? go(fwd_lds_kernel<GL, BF16, true, true>) : go(fwd_lds_kernel<GL, BF16, false, true>);
+    return a.quads ? go(fwd_lds_kernel<GL, BF16, true>) : go(fwd_lds_kernel<GL, BF16, false>);
 }
 
 // the ordered copy of the layer: [ids][weights], part by part

@@ -161,6 +161,12 @@ def test_forward_from_slices_in_lds_shares(ffi, bf16, B, N, L, K):
         assert (np.abs(out.cpu().numpy() - ref) <= (K + 2) * 2.0 ** -24 * size + 1e-30).all()
 
 
+# Slices of eight samples staged by four columns at a time and, of many columns, by one: samples missing, a second slice, columns off four
+@pytest.mark.parametrize("B,N,L,K", [(5, 512, 3000, 44), (5, 513, 3000, 44), (7, 1215, 9001, 13), (9, 700, 9000, 24)])
+def test_forward_from_slices_of_eight_samples(ffi, B, N, L, K):
+    test_forward_from_slices_in_lds_shares(ffi, False, B, N, L, K)
+
+
 # Wide inputs with few columns and few labels: more blocks than labels fill, lists of few connections, a last block of one label;
 # many blocks whose sums are added
 @pytest.mark.parametrize("B,N,L,K", [(5, 1_217, 130, 3), (33, 1_242, 3_201, 95), (64, 5_000, 129, 40), (17, 2_000, 13_331, 8), (3, 20_000, 700, 16)])
