@@ -199,8 +199,11 @@ SmallShape small_shape(const Dims& d) {
 // Layers of few labels give the larger paths few workgroups, each with all batch tiles one after the other.  Up to 1,024 labels,
 // backward: 128 x 1,000 x 1,000 x 64 61 us against 117, 256 x 300 x 1,024 x 40 73 against 85, 365 x 53 x 1,000 x 32 85 against 91 (12 M
 // visits; at 15 to 25 M 106 to 176 against 106 to 147); up to 512 and fan-ins up to 128: 365 x 53 x 549 x 45 67 against 119, 512 x 1,000
-// x 500 x 128 216 against 372 (fan-in 200 94 against 75).  Forward up to 512 labels and from fan-in 64 on: 128 x 300 x 256 x 200 15
-// against 119, 365 x 100 x 500 x 64 19 against 41, 128 x 768 x 500 x 128 18 against 30 (16 M products: 33 against 31).
+// x 500 x 128 216 against 372 (fan-in 200 94 against 75).  Of 818 backward passes of up to 512 labels and 10 to 33 M visits the small
+// path lost 30, all of more samples than CUs, where a workgroup has all connections of a sample (2.6 us a thousand), and of fan-ins of
+// 65 to 96: there the large ones take 10 us a batch tile from 513 to 768 columns and 11 to 12 up to some 330 (260 x 600 x 512 x 96 90 against
+// 127, 290 x 60 x 512 x 96 108 against 128; 380 x 60 x 480 x 90 118 against 114, 290 x 500 x 512 x 96 139 against 128).
+// Forward up to 512 labels and from fan-in 64 on: 128 x 300 x 256 x 200 15 against 119, 365 x 100 x 500 x 64 19 against 41, 128 x 768 x 500 x 128 18 against 30 (16 M products: 33 against 31).
 bool takes_small_forward(const Dims& d) {
     const long long sums = (long long)d.B * d.L * d.K;
     if (d.B > 65535 * kSmSamples) return false;            // (groups of samples are the grid's second dimension)
@@ -208,9 +211,13 @@ bool takes_small_forward(const Dims& d) {
     return sums <= (4ll << 20) || (d.L <= 512 && d.K >= 64 && sums <= 12'000'000);
 }
 bool takes_small_backward(const Dims& d) {
-    const long long visits = small_shape(d).units * d.L * d.K, cells = (long long)d.B * d.N;
+    const long long units = small_shape(d).units, visits = units * d.L * d.K, cells = (long long)d.B * d.N;
     if (g_options.small_path != 0) return g_options.small_path > 0 && visits < (1ll << 30) && cells < (1ll << 30);
-    const bool few_labels = (d.L <= 1024 && visits <= 12'000'000) || (d.L <= 512 && d.K <= 128 && visits <= (32ll << 20));
+    bool few_labels = (d.L <= 1024 && visits <= 12'000'000) || (d.L <= 512 && d.K <= 128 && visits <= (32ll << 20));
+    const long long tiles = (d.B + 31) / 32, connections = (long long)d.L * d.K;
+    if (d.K > 64 && d.K <= 96 && (d.N <= 330 || (d.N > 512 && d.N <= 768)) && connections > tiles * (d.N > 512 ? 3900 : d.N > 128 ? 4500 : 4200) &&
+        units > device_cu_count())
+        few_labels = false;
     return (visits <= (4ll << 20) || (few_labels && d.N <= 1216)) && cells <= (4ll << 20);
 }
 

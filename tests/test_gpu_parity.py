@@ -1086,7 +1086,8 @@ def test_plan_form_and_gradients_at_few_columns(ffi, N, B, L, K):
 
 
 @pytest.mark.parametrize("shape", [(365, 53, 512, 65), (365, 53, 513, 20), (128, 300, 256, 200), (90, 1000, 1024, 65), (90, 1216, 1025, 65),
-                                   (500, 200, 512, 128), (500, 200, 500, 129), (300, 1217, 512, 64)])
+                                   (500, 200, 512, 128), (500, 200, 500, 129), (300, 1217, 512, 64),
+                                   (257, 330, 512, 96), (257, 331, 512, 96), (290, 600, 420, 95), (256, 600, 512, 96)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_layers_of_few_labels(ffi, shape, transposed):
     # both sides of the lines up to which the launches for small layers take them
