@@ -792,8 +792,8 @@ int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds) 
         while (tw >= 64 && (long long)tw * K >= 32768) tw -= 2;
         // Tiles per workgroup come in whole numbers: the walking kernel runs cus / batch tiles label streams of
         // ceil(tiles / streams) tiles each, and the largest tile can leave the last stream nearly empty, or whole CUs
-        // without a stream (670,091 labels in 608-label tiles: 62 streams of 18 tiles on 64 CUs' worth of workgroups).
-        // The tile shrinks to what fills every stream with that same number of tiles (582 labels in that example: 64 x 18); a
+        // without a stream (670,091 labels in 618-label tiles: 1,085, of which the last of 64 streams gets 14 and the others 17).
+        // The tile shrinks to what fills every stream with that same number of tiles (616 labels in that example); a
         // smaller tile pads a little more per connection, which costs less than the idle streams.  (Workgroups that share
         // a CU are left alone: there the streams outnumber the CUs.)
         if (tw >= 64 && (threads > 256 || nbt_hint < 2)) {

@@ -789,9 +789,9 @@ __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __res
 // flight.  Twelve wavefronts and not sixteen: with 168 registers the sums of 704 labels fit a workgroup, and a slice is gone
 // through less often (misses of L2 77 -> 60 M lines in bf16).
 //
-// What bounds it: the L1's 64 bytes per clock, busy 88 % of the time.  670,091 labels, against sixteen wavefronts that bring
-// their own lists, 512 labels: 128 samples, 65,536 columns, fan-in 72 in fp32 1,215 -> 1,139 us (21.7 TB/s); 512 samples, 100,000
-// columns, fan-in 64 in bf16 2,112 -> 2,000 us.
+// What bounds it: the L1, whose address side is busy 89 % of the time in bf16 and 92 in fp32, its data side 96.  670,091 labels,
+// against sixteen wavefronts that bring their own lists, 512 labels: 128 samples, 65,536 columns, fan-in 72 in fp32 1,215 -> 1,145 us
+// (21.6 TB/s); 512 samples, 100,000 columns, fan-in 64 in bf16 2,112 -> 2,000 us.
 constexpr int kPhWaves = 11, kPhThreads = (kPhWaves + 1) * 64;    // wavefronts that walk, and one that brings their lists
 
 // `bytes` (a multiple of 1,024) from the resource's begin on into LDS, past the registers, by one wavefront
@@ -1036,10 +1036,8 @@ int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
     hipLaunchKernelGGL(rbr, dim3((unsigned)((d.L + 4 * kRbrRows - 1) / (4 * kRbrRows))), dim3(256), rbr_lds, s, a.idx, a.w, rows, row_w, d.L, d.K,
                        (unsigned)(((unsigned long long)ranges << 32) / (unsigned long long)d.N), ranges);
     FFI_HIP_TRY(hipGetLastError());
-    // (as many labels as the registers hold sums of: a slice is gone through as often as there are rounds; fewer where that
-    // leaves CUs idle)
     return phased_labels(d.L, a.slices) == 8 ? launch_phased_walk<BF16, 8>(a, rows, row_w, d, s)
-                                                                          : launch_phased_walk<BF16, 4>(a, rows, row_w, d, s);
+                                             : launch_phased_walk<BF16, 4>(a, rows, row_w, d, s);
 }
 
 // Rounds of workgroups, one per CU and each with its XCD's share of the work, times the labels of a lane group.
