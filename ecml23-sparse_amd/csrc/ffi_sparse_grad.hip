@@ -388,7 +388,7 @@ __global__ __launch_bounds__(256, 4) void wgrad_sparse_kernel(const SparseRows r
 // They also count the set bits, which the next call decides from (host_count; totals: a sum and a count of workgroups, zero between
 // launches).
 // (32 x 768 x 670,091 x 32, 0.2 % of the gradients not zero, late in training: two launches that count 9.6 us, the gradient 22, the
-// step on the weights 72 and on the bias 5.8; 93 so.  The whole step with its forward pass 183 -> 170.)
+// step on the weights 72 and on the bias 5.8; 92 so.  The whole step with its forward pass 183 -> 170.)
 //   A wavefront that steps looks at the masks of its labels first and leaves out the rows with a gradient, by accesses that the end of
 // a buffer keeps from memory: no branch parts the loads.  (All rows read beside the masks, 168 us for the whole step above, and this
 // 168; loads under branches 172.  What rows of other lengths share sixteen bytes of is read element by element, three a lane at most.)
