@@ -735,18 +735,15 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
             }
             if (tile_path_fits(d.N) && d.N < (1 << kArrIdBits)) total += arranged_words((long long)(L * ((K + 31) / 32))) * 2;   // idx16
         } else {
-            const size_t labels = (size_t)plan_block_labels(d.N, d.K, d.L), nblocks = (L + labels - 1) / labels, lists = nblocks * N;
-            const size_t slots = plan_expected_slots(d.N, d.K, d.L);
-            int gl, slices, m, streams, per_stream;
-            walk_shape(d.N, d.B, d.L, (int)nblocks, &gl, &slices, &m, &streams, &per_stream);
-            const size_t padded = (size_t)slices * gl * 4;                              // samples of the sliced copies
-            total += slots * 6 + (lists + 1) * 4 + L * K * 4;                           // slot_pos, slot_lab, oct_ptr, pos_slot
-            total += slots * 4 * 2;                                                     // weights and weight gradients in slot order
-            // out_grad in slices and the sums per stream; the lists' ends while the plan is built
-            partial_slot = std::max(partial_slot, lists * 4);
+            const GlobalShape f = global_shape(d.N, d.K, d.L, d.B);
+            const size_t sl = 256 / (size_t)f.members, padded = (B + sl - 1) / sl * sl, units = (size_t)f.segments * f.groups;
+            const size_t at_once = small_backward ? 1 : (size_t)walk_slices((long long)units, (int)(padded / sl));
+            total += f.max_slots * 4 * (2 + at_once);                                   // entries; weights and weight gradients in their order
+            total += L * K * 6 + (2 * units + 1) * 4;                                   // slot_of, tile_pos, chunk_ptr, chunk_count
+            // counts while the plan is built; out_grad in slices and the sums per segment
+            partial_slot = std::max(partial_slot, global_build_words(f, (int)(((long long)d.L * d.K + (1ll << f.tile_bits) - 1) >> f.tile_bits)) * 4);
             if (!small_backward) {
-                partial_slot = std::max(partial_slot, (L + N * (size_t)streams) * padded * 4);
-                features_slot = std::max(features_slot, N * padded * 4);
+                partial_slot = std::max(partial_slot, (L + (f.segments > 1 ? N * (size_t)f.segments : 0)) * padded * 4);
             }
         }
     }

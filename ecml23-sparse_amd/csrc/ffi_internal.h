@@ -269,10 +269,12 @@ int launch_rewire(int32_t* lookup, const float* w, float* const* arrays, int n_a
 // padding slots: a fixed order, but not the ascending-position order in which the reference's CPU
 // kernel accumulates (tfsparse/cc/kernels/backward.cpp:64-72).
 //
-// tiled == false (any shape): the connections grouped by (block of `block_labels` labels, column), positions ascending, every
-// list padded to whole octs of slots: list blk * N + n is octs oct_ptr[blk * N + n] .. oct_ptr[blk * N + n + 1] - 1.
-// slot_pos = flat position of the slot's connection (-1: padding), slot_lab = its label inside the block (kNoLabel: padding),
-// pos_slot = slot_pos the other way round.
+// tiled == false (any shape): a stream per (segment of `seg_labels` labels, group of kGroupColumns columns) lists the stream's
+// connections in steps of `members` connections of one column, in the order in which the steps' first members come in the lookup;
+// a column's last step may hold padding.  Steps fill chunks, entry_in_chunk() says where: stream u has chunk_count[u]
+// chunks from chunk_ptr[u] on.  entries = label inside the segment << 8 | column inside the group (kPadEntry and above: padding).
+// The connections again in the order of the lookup's tiles of 2^tile_bits flat positions, and inside a tile by stream: tile_pos =
+// position inside the tile, slot_of = the connection's entry.
 struct ffi_plan {
     int device = -1;
     int L = 0, K = 0, N = 0;
@@ -302,14 +304,14 @@ struct ffi_plan {
     // connections reordered so that even and odd columns alternate (see ffi_plan.hip); stored in blocks of 64 units,
     // quarter by quarter (ffi::arranged_quarter_offset), so that the 64 lanes of a wavefront load 1 KB in one piece
     unsigned short* idx16 = nullptr;
-    // blocked global form
-    int block_labels = 0;     // labels per block (<= 65535: bounds the part of out_grad that is live at a time)
-    int nblocks = 0;
-    long long slots = 0;
-    unsigned* oct_ptr = nullptr;         // [nblocks * N + 1]
-    int32_t* slot_pos = nullptr;
-    unsigned short* slot_lab = nullptr;
-    unsigned* pos_slot = nullptr;        // [L * K] slot of each flat position
+    // global form
+    int members = 0, groups = 0, segments = 0, seg_labels = 0, tile_bits = 0;
+    long long slots = 0;                 // entries, padding and room behind the streams' last chunks included
+    unsigned* chunk_ptr = nullptr;       // [segments * groups + 1]
+    unsigned* chunk_count = nullptr;     // [segments * groups]
+    unsigned* entries = nullptr;         // [slots]
+    unsigned* slot_of = nullptr;         // [L * K]
+    unsigned short* tile_pos = nullptr;  // [L * K]
     unsigned long long* d_scratch = nullptr;  // counters of the build, fingerprint partial sums (device)
     unsigned long long* h_scratch = nullptr;  // pinned mirror
     hipEvent_t fp_done = nullptr;             // recorded behind the fingerprint kernel and its copy to h_scratch
@@ -343,7 +345,16 @@ struct ffi_plan {
 };
 
 namespace ffi {
-constexpr unsigned short kNoLabel = 0xffff;  // slot_lab of a padding slot
+constexpr int kGroupColumns = 32;            // columns of a stream of the global form: those of a wavefront that walks it
+constexpr unsigned kPadEntry = 0xffffff00u;  // entries from here on are padding
+// A chunk holds sixteen steps, 64 entries for every four members: entry_in_chunk() = where member m of step i lies in it.  A wavefront
+// that walks the chunk holds entries 64 k + lane in its lanes; a step's 64 / members lanes per member sum the member's weight
+// gradient so that the lane is left with its own entries'.
+constexpr int kChunkSteps = 16;
+__host__ __device__ inline int entry_in_chunk(int members, int i, int m) {
+    const int lanes = 64 / members, v = (i & 1) << 2 | (i & 2) | (i >> 2 & 1), half = i >> 3;
+    return lanes == 16 ? m * 16 + v * 2 + half : half * 64 + m * 8 + v;
+}
 constexpr int kPlanTileLabels = 1024;     // a [1024+1][32] fp32 tile fits LDS
 constexpr unsigned kPadPos = 0xffffu;      // pos16 of a padding slot; real positions are below it (tile_labels * K <= 0xffff)
 // LDS of the kernel that walks the tiled form: the tile's rows of out_grad (per bank half: half the tile plus some room
@@ -393,9 +404,13 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
-constexpr int kWalkColumns = 128;          // columns of a workgroup that walks the global form, eight lanes each
-int plan_block_labels(int N, int K, int L);
-size_t plan_expected_slots(int N, int K, int L);
+// How the global form of a lookup is cut (`batch`: the batch size it is built for, 0 = unknown).
+struct GlobalShape {
+    int members, groups, segments, seg_labels, tile_bits;
+    size_t max_slots;
+};
+GlobalShape global_shape(int N, int K, int L, int batch);
+size_t global_build_words(const GlobalShape& f, int tiles);
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s);
 // Content fingerprint of `lookup` (and the count of ids outside [0,N)).  _begin enqueues the kernel
 // on `s` and returns; _end waits for that kernel only, not for what the caller enqueued on `s`
@@ -440,7 +455,7 @@ void plan_free(ffi_plan* p);
 int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp,
                       hipStream_t s, const LookupCheck* check = nullptr);
 // Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.
-void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, int* streams, int* blocks_per_stream);
+int walk_slices(long long units, int slices);
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
                          bool tp, hipStream_t s);
 }  // namespace ffi

@@ -13,9 +13,6 @@
 #include <cstring>
 #include <functional>
 
-#include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/types/double_buffer.hpp>
-
 namespace ffi {
 namespace {
 
@@ -623,48 +620,296 @@ inline size_t tile_fill_lds(int threads, int ncols, int tile_labels) {
     return (size_t)(threads / 64) * ncols * sizeof(unsigned) + (size_t)((tile_labels + 1) & ~1) * sizeof(unsigned short);
 }
 
-// ---- blocked global form ------------------------------------------------------------------------
+// ---- global form --------------------------------------------------------------------------------
 
-// ptr[n] = first position in the sorted key array whose key is >= n (n in [0,nkeys]), and the octs that the kListsPerBlock lists
-// of a workgroup take together
-constexpr int kListsPerBlock = kBlock - 1;
-__global__ __launch_bounds__(kBlock) void list_ptr_kernel(const unsigned* __restrict__ sorted_keys, int total, int nkeys,
-                                                          int32_t* __restrict__ ptr, unsigned* __restrict__ block_octs) {
-    __shared__ int begin[kBlock];
-    const int n = (int)min(blockIdx.x * (unsigned)kListsPerBlock + threadIdx.x, (unsigned)nkeys);
-    int lo = 0, hi = total;
-    while (lo < hi) {
-        const int mid = lo + ((hi - lo) >> 1);
-        if (sorted_keys[mid] < (unsigned)n) lo = mid + 1; else hi = mid;
+// A position's stream: one per segment of labels and group of columns.
+struct StreamOf {
+    int K, seg_labels, segments, groups;
+    __device__ __forceinline__ unsigned operator()(unsigned id, unsigned pos) const {
+        const unsigned group = id / kGroupColumns;
+        return segments == 1 ? group : pos / (unsigned)K / (unsigned)seg_labels * (unsigned)groups + group;
     }
-    ptr[n] = lo;
-    begin[threadIdx.x] = lo;
+};
+
+// counts[t][u] = connections of stream u in tile t, a workgroup per tile; so many streams at a time as the LDS has counters
+constexpr int kTileThreads = 1024, kCountWindow = 16384;
+__global__ __launch_bounds__(kTileThreads) void tile_streams_kernel(const int32_t* __restrict__ idx, int total, int tile_bits, int units,
+                                                                    const StreamOf stream_of, unsigned* __restrict__ counts) {
+    extern __shared__ __align__(16) unsigned tile_counts[];
+    constexpr int kInflight = 8;
+    const unsigned p0 = blockIdx.x << tile_bits, end = min(p0 + (1u << tile_bits), (unsigned)total);
+    for (int u0 = 0; u0 < units; u0 += kCountWindow) {
+        const int n = min(kCountWindow, units - u0);
+        for (int i = threadIdx.x; i < n; i += kTileThreads) tile_counts[i] = 0u;
+        __syncthreads();
+        for (unsigned p = p0 + threadIdx.x; p < end; p += kTileThreads * kInflight) {
+            unsigned id[kInflight];
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i) id[i] = (unsigned)idx[min(p + i * kTileThreads, end - 1)];
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i) {
+                const unsigned at = p + i * kTileThreads, u = stream_of(id[i], at) - (unsigned)u0;
+                if (at < end && u < (unsigned)n) atomicAdd(&tile_counts[u], 1u);
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += kTileThreads) counts[(size_t)blockIdx.x * units + u0 + i] = tile_counts[i];
+        __syncthreads();
+    }
+}
+
+// counts[t][u] -> connections of stream u in the tiles before t; and of all tiles, and the chunks that the stream is given: its steps
+// are at most one for every `members` connections and a partly filled one per column, and no more than its connections.
+// 64 streams per workgroup, each wavefront a stretch of the tiles.
+__global__ __launch_bounds__(kTileThreads) void stream_counts_kernel(unsigned* __restrict__ counts, int tiles, int units, int members,
+                                                                     unsigned* __restrict__ of_stream, unsigned* __restrict__ chunks) {
+    constexpr int kParts = kTileThreads / 64;
+    __shared__ unsigned sums[kParts][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6, u = blockIdx.x * 64 + lane;
+    const int per = (tiles + kParts - 1) / kParts, from = min(part * per, tiles), to = min(from + per, tiles);
+    unsigned sum = 0;
+    if (u < units) {
+#pragma unroll 8
+        for (int t = from; t < to; ++t) sum += counts[(size_t)t * units + u];
+    }
+    sums[part][lane] = sum;
     __syncthreads();
-    // (behind the last list begin and end are the same)
-    const unsigned octs = threadIdx.x < kListsPerBlock ? (unsigned)(begin[threadIdx.x + 1] - lo + 7) / 8u : 0u;
-    unsigned long long sum = 0;
-    (void)block_sum_below<kBlock>(octs, &sum);
-    if (threadIdx.x == 0) block_octs[blockIdx.x] = (unsigned)sum;
-}
-
-// oct_ptr[n] = octs of the lists before list n, from the octs before the list's workgroup of list_ptr_kernel
-__global__ __launch_bounds__(kBlock) void oct_ptr_kernel(const int32_t* __restrict__ ptr, int nkeys, const unsigned* __restrict__ octs_before,
-                                                         unsigned* __restrict__ oct_ptr) {
-    const unsigned n = blockIdx.x * (unsigned)kListsPerBlock + threadIdx.x;
-    const bool mine = threadIdx.x < kListsPerBlock && n < (unsigned)nkeys;
-    const unsigned octs = mine ? (unsigned)(ptr[n + 1] - ptr[n] + 7) / 8u : 0u;
-    unsigned long long sum = 0;
-    const unsigned at = octs_before[blockIdx.x] + (unsigned)block_sum_below<kBlock>(octs, &sum);
-    if (mine) {
-        oct_ptr[n] = at;
-        if (n == (unsigned)nkeys - 1u) oct_ptr[nkeys] = at + octs;
+    if (u >= units) return;
+    unsigned run = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) {
+        run += i < part ? sums[i][lane] : 0u;
+        all += sums[i][lane];
+    }
+    for (int t0 = from; t0 < to; t0 += 8) {
+        unsigned n[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) n[i] = counts[(size_t)min(t0 + i, to - 1) * units + u];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (t0 + i < to) {
+                counts[(size_t)(t0 + i) * units + u] = run;
+                run += n[i];
+            }
+    }
+    if (part == 0) {
+        const unsigned entries = (unsigned)(kChunkSteps * members);
+        of_stream[u] = all;
+        chunks[u] = min((all + (unsigned)(kGroupColumns * (members - 1)) + entries - 1u) / entries, (all + kChunkSteps - 1u) / kChunkSteps);
     }
 }
 
-int bits_for(unsigned max_value) {
-    int b = 1;
-    while (b < 32 && (max_value >> b) != 0) ++b;
-    return b;
+// A tile's connections by stream, in the order of the lookup inside a stream: tile_pos, and into the streams' lists (label inside the
+// segment << 8 | column inside the group); place_of = where in the lists.  One workgroup per tile, whose wavefronts take consecutive
+// stretches of it: they count their connections per stream, sums over streams and wavefronts turn the counts into places, and the
+// stretches are gone through again, 64 connections at a time, each of which takes the place it finds and leaves the next one there (of
+// several of one stream among the 64 the lanes' order decides, not the LDS's).  Places gather in LDS and leave by whole runs.
+// As many wavefronts as the counters of 16 bits leave room for.
+constexpr size_t kTileCounterBytes = 61440;
+__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const int32_t* __restrict__ idx, int total, int tile_bits, int units, const StreamOf stream_of,
+                                                                 const unsigned* __restrict__ before, const unsigned* __restrict__ begin,
+                                                                 unsigned short* __restrict__ tile_pos, unsigned* __restrict__ place_of,
+                                                                 unsigned* __restrict__ list, int window) {
+    extern __shared__ __align__(16) unsigned tile_lds[];
+    __shared__ unsigned wave_sums[kTileThreads / 64];
+    constexpr int kInflight = 8;
+    const int nthreads = blockDim.x, nwaves = nthreads >> 6, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned tile = 1u << tile_bits, p0 = blockIdx.x << tile_bits, n = min(tile, (unsigned)total - p0);
+    unsigned short* const stage_pos = reinterpret_cast<unsigned short*>(tile_lds);                       // [tile]
+    unsigned char* const stage_col = reinterpret_cast<unsigned char*>(tile_lds) + 2 * (size_t)tile;      // [tile]
+    unsigned* const counters = tile_lds + 3 * (size_t)tile / 4;                                          // [wave][window / 2] two streams a word
+    const int words = window / 2;
+    unsigned* const mine = counters + (size_t)wave * words;
+    const unsigned stretch = ((n + nwaves - 1) / nwaves + 63) & ~63u, from = min(wave * stretch, n), to = min(from + stretch, n);
+    unsigned placed = 0;                                                                                 // connections of the streams before the window
+    for (int u0 = 0; u0 < units; u0 += window) {
+        const unsigned streams = (unsigned)min(window, units - u0);
+        for (int i = threadIdx.x; i < nwaves * words; i += nthreads) counters[i] = 0u;
+        __syncthreads();
+        auto walk = [&](auto visit) {
+            unsigned next[kInflight];
+            auto fetch = [&](unsigned e0) {
+#pragma unroll
+                for (int i = 0; i < kInflight; ++i) next[i] = (unsigned)idx[p0 + min(e0 + 64 * i + lane, n - 1)];
+            };
+            fetch(from);
+            for (unsigned e0 = from; e0 < to; e0 += 64 * kInflight) {
+                unsigned id[kInflight], u[kInflight];
+#pragma unroll
+                for (int i = 0; i < kInflight; ++i) {
+                    const unsigned e = e0 + 64 * i + lane;
+                    id[i] = next[i];
+                    u[i] = stream_of(id[i], p0 + e) - (unsigned)u0;
+                    if (e >= to || u[i] >= streams) u[i] = ~0u;
+                }
+                fetch(e0 + 64 * kInflight);
+                visit(id, u, e0 + lane);
+            }
+        };
+        walk([&](const unsigned*, const unsigned* u, unsigned) {
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i)
+                if (u[i] != ~0u) atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
+        });
+        __syncthreads();
+        // each thread takes consecutive pairs of streams: their connections, those of the threads before it, and the places
+        const int per = (words + nthreads - 1) / nthreads, w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
+        unsigned sum = 0;
+        for (int w = w0; w < w1; ++w)
+            for (int v = 0; v < nwaves; ++v) {
+                const unsigned c = counters[(size_t)v * words + w];
+                sum += (c & 0xffffu) + (c >> 16);
+            }
+        unsigned upto = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned below = __shfl_up(upto, off, 64);
+            if (lane >= off) upto += below;
+        }
+        if (lane == 63) wave_sums[wave] = upto;
+        __syncthreads();
+        unsigned run = placed + upto - sum, all = 0;
+        for (int v = 0; v < nwaves; ++v) {
+            run += v < wave ? wave_sums[v] : 0u;
+            all += wave_sums[v];
+        }
+        for (int w = w0; w < w1; ++w) {
+            unsigned even = run, odd = 0;
+            for (int v = 0; v < nwaves; ++v) odd += counters[(size_t)v * words + w] & 0xffffu;
+            odd += run;
+            for (int v = 0; v < nwaves; ++v) {
+                const unsigned c = counters[(size_t)v * words + w];
+                counters[(size_t)v * words + w] = (even & 0xffffu) | odd << 16;
+                even += c & 0xffffu;
+                odd += c >> 16;
+            }
+            run = odd;
+        }
+        __syncthreads();
+        walk([&](const unsigned* id, const unsigned* u, unsigned e) {
+            unsigned found[kInflight], there[kInflight];
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i) {
+                there[i] = found[i] = 0u;
+                if (u[i] != ~0u) {
+                    there[i] = mine[u[i] >> 1];
+                    found[i] = atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kInflight; ++i) {
+                const unsigned shift = 16 * (u[i] & 1);
+                unsigned at = there[i] >> shift & 0xffffu;
+                for (unsigned long long left = __ballot(u[i] != ~0u && (found[i] >> shift & 0xffffu) != at); left != 0ull;) {
+                    const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)u[i], __builtin_ctzll(left));
+                    const unsigned long long same = __ballot(u[i] == k);
+                    if (u[i] == k) at += (unsigned)__popcll(same & ((1ull << lane) - 1ull));
+                    left &= ~same;
+                }
+                if (u[i] != ~0u) {
+                    stage_pos[at] = (unsigned short)(e + 64 * i);
+                    stage_col[at] = (unsigned char)(id[i] % kGroupColumns);
+                }
+            }
+        });
+        __syncthreads();
+        // eight lanes to a run; behind the walk the last wavefront's counter of a stream is the end of its run
+        const unsigned* const last = counters + (size_t)(nwaves - 1) * words;
+        auto end_of = [&](unsigned u) { return last[u >> 1] >> (16 * (u & 1)) & 0xffffu; };
+        for (unsigned u = threadIdx.x / 8; u < streams; u += nthreads / 8) {
+            const unsigned start = u > 0 ? end_of(u - 1) : placed, end = end_of(u), stream = (unsigned)u0 + u;
+            if (start == end) continue;
+            const unsigned base = begin[stream] + before[(size_t)blockIdx.x * units + stream] - start;
+            const int label0 = (int)(stream / (unsigned)stream_of.groups) * stream_of.seg_labels;
+            for (unsigned q = start + (threadIdx.x & 7); q < end; q += 8) {
+                const unsigned pos = stage_pos[q];
+                tile_pos[p0 + q] = (unsigned short)pos;
+                place_of[p0 + q] = base + q;
+                list[base + q] = (unsigned)((int)((p0 + pos) / (unsigned)stream_of.K) - label0) << 8 | stage_col[q];
+            }
+        }
+        placed += all;
+        __syncthreads();
+    }
+}
+
+// The steps of a stream, one wavefront per stream, 64 connections at a time in the order of the lookup: the connection of rank r
+// among its column's is member r % MEMBERS of that column's step r / MEMBERS, and steps are numbered as their first members come.
+// Writes the stream's entries, and for each connection of the list its slot.
+// Bound by the latency of a turn (ballots for the ranks, a round trip to LDS for the number of a step), four turns' loads in flight.
+constexpr int kStepWaves = 4, kStepRing = 32;            // (a turn opens at most 64 / MEMBERS steps of a column)
+template <int MEMBERS>
+__global__ __launch_bounds__(kStepWaves * 64) void stream_steps_kernel(const unsigned* __restrict__ list, const unsigned* __restrict__ begin,
+                                                                       const unsigned* __restrict__ chunk_ptr, int units, unsigned* __restrict__ entries,
+                                                                       unsigned* __restrict__ slot_at, unsigned* __restrict__ chunk_count) {
+    constexpr int kEntries = kChunkSteps * MEMBERS, kAhead = 4;
+    __shared__ unsigned opened[kStepWaves][kGroupColumns][kStepRing], counts[kStepWaves][kGroupColumns];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int u = blockIdx.x * kStepWaves + wave;
+    if (u >= units) return;
+    unsigned (*const open)[kStepRing] = opened[wave];
+    unsigned* const count = counts[wave];
+    if (lane < kGroupColumns) count[lane] = 0u;
+    const unsigned from = begin[u], end = begin[u + 1];
+    const size_t slot0 = (size_t)chunk_ptr[u] * kEntries;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    auto slot_of = [&](unsigned step, unsigned m) { return slot0 + (size_t)(step / kChunkSteps) * kEntries + entry_in_chunk(MEMBERS, (int)(step % kChunkSteps), (int)m); };
+    unsigned steps = 0;
+    unsigned next[kAhead];
+    auto fetch = [&](int i, unsigned at) { next[i] = list[min(at + lane, end - 1u)]; };
+    if (from < end) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) fetch(i, from + 64 * i);
+    }
+    for (unsigned e0 = from; e0 < end; e0 += 64 * kAhead) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const unsigned e = e0 + 64 * i + lane, entry = next[i], col = entry % kGroupColumns;
+            const bool on = e < end;
+            fetch(i, e0 + 64 * (i + kAhead));
+            unsigned long long same = __ballot(on);
+#pragma unroll
+            for (int bit = 0; bit < 5; ++bit) {
+                const unsigned long long set = __ballot((col >> bit & 1u) != 0u);
+                same &= (col >> bit & 1u) ? set : ~set;
+            }
+            const unsigned rank = count[col] + (unsigned)__popcll(same & below), m = rank % MEMBERS, place = rank / MEMBERS % kStepRing;
+            const unsigned long long firsts = __ballot(on && m == 0u);
+            if (on && m == 0u) open[col][place] = steps + (unsigned)__popcll(firsts & below);
+            if (on && (same & ~below & ~(1ull << lane)) == 0ull) count[col] = rank + 1u;       // (the column's last of this turn)
+            __builtin_amdgcn_wave_barrier();
+            if (on) {
+                const size_t slot = slot_of(open[col][place], m);
+                entries[slot] = entry;
+                slot_at[e] = (unsigned)slot;
+            }
+            steps += (unsigned)__popcll(firsts);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    // what is left of the columns' last steps, and of the last chunk
+    if (lane < kGroupColumns && count[lane] % MEMBERS != 0u) {
+        const unsigned step = open[lane][count[lane] / MEMBERS % kStepRing];
+        for (unsigned m = count[lane] % MEMBERS; m < MEMBERS; ++m) entries[slot_of(step, m)] = kPadEntry | (unsigned)lane;
+    }
+    const unsigned chunks = (steps + kChunkSteps - 1u) / kChunkSteps, rest = chunks * kChunkSteps - steps;
+    if ((unsigned)lane < rest)
+        for (unsigned m = 0; m < MEMBERS; ++m) entries[slot_of(steps + (unsigned)lane, m)] = kPadEntry;
+    if (lane == 0) chunk_count[u] = chunks;
+}
+
+// places in the streams' lists -> slots
+__global__ __launch_bounds__(kBlock) void slots_of_places_kernel(const unsigned* __restrict__ slot_at, unsigned* __restrict__ slot_of, int total) {
+    constexpr int kInflight = 4;
+    const int i0 = blockIdx.x * (kBlock * kInflight) + threadIdx.x;
+    unsigned v[kInflight];
+#pragma unroll
+    for (int i = 0; i < kInflight; ++i) v[i] = slot_of[min(i0 + i * kBlock, total - 1)];
+#pragma unroll
+    for (int i = 0; i < kInflight; ++i) v[i] = slot_at[v[i]];
+#pragma unroll
+    for (int i = 0; i < kInflight; ++i)
+        if (i0 + i * kBlock < total) slot_of[i0 + i * kBlock] = v[i];
 }
 
 // Detaches the arrays from the plan.  keep == true (a rebuild follows): their buffers go to the spare list.
@@ -684,7 +929,7 @@ void free_arrays(ffi_plan* p, bool keep = false) {
     }
     p->owned.clear();
     p->rowpos = nullptr;
-    p->oct_ptr = nullptr; p->slot_pos = nullptr; p->slot_lab = nullptr; p->pos_slot = nullptr; p->slots = 0; p->slice_off = nullptr; p->lab16 = nullptr; p->pos16 = nullptr; p->slot32 = nullptr; p->idx16 = nullptr; p->colperm = nullptr;
+    p->chunk_ptr = nullptr; p->chunk_count = nullptr; p->entries = nullptr; p->slot_of = nullptr; p->tile_pos = nullptr; p->slots = 0; p->slice_off = nullptr; p->lab16 = nullptr; p->pos16 = nullptr; p->slot32 = nullptr; p->idx16 = nullptr; p->colperm = nullptr;
     p->tiled = false; p->w_in_lds = false; p->total_rows = 0; p->bytes = 0;
 }
 
@@ -739,19 +984,38 @@ void dev_release(ffi_plan* p, void* ptr) {
 
 }  // namespace
 
-// Labels per block of the global form: the block's rows of one slice of out_grad (128 bytes each) take five eighths of an
-// XCD's L2 -- shared by as many blocks as the workgroups of that many columns leave room for at a time -- unless the
-// lists of a block's columns would then hold fewer than eight connections.  Few columns (kWalkColumns to a workgroup of the walk) and
-// few labels get as many blocks as the CUs have workgroups for in one go, as far as the lists keep twelve.  All passes at 126 x 1,242
-// x 15,823 x 95: 449 us with three blocks, 160 with 25; 128 x 2,000 x 13,330 x 32 197 and 97, 128 x 2,500 x 131,072 x 32 351 and 328.
-// (One block more, so that some CUs have two workgroups: 418 us at 128 x 1,300 x 131,072 x 32, where the former blocks took 345 and these 331.)
-int plan_block_labels(int N, int K, int L) {
-    const double resident = 20480.0 * std::min(1.0, (double)N / 4096.0), filled = 8.0 * (double)N / (double)K;
-    const int chunks = (N + kWalkColumns - 1) / kWalkColumns, wanted = std::max(1, device_cu_count() / chunks);
-    const double busy = std::max(std::max(128.0, 12.0 * N / K), std::ceil((double)L / wanted));
-    const int labels = (int)std::min(65535.0, std::max(std::min(busy, 1024.0), std::max(std::min(resident, busy), filled)));
-    return std::min(labels, L);
+// Steps of four connections where a row of 64 samples is gathered by sixteen lanes, of eight where 32 samples are enough (the
+// walking kernel takes 0.67 ms for 64 samples and 0.40 for 32 at 65,536 columns x 670,091 labels x 72).  Segments: as many as make the
+// walk shortest, in steps of a wavefront -- its share of the connections, half a step per column that the last connections do not
+// fill, and some forty for its beginning and end -- times the rounds that the CUs, eight wavefronts each, need for all streams and
+// slices.  128 samples and more, 1,300 to 2,500 columns want a segment on every CU; 2 samples, 22,133 columns, 200,058 labels, fan-in 8
+// two of them (walk 31 us; 40 with eight, whose three rounds are a little less of the connections).
+// Labels and rows of a segment stay within the entries and 32-bit offsets.
+GlobalShape global_shape(int N, int K, int L, int batch) {
+    GlobalShape f{};
+    f.members = batch > 0 && batch <= 32 ? 8 : 4;
+    f.groups = (N + kGroupColumns - 1) / kGroupColumns;
+    const double total = (double)L * K, waves = 8.0 * device_cu_count();
+    const int slices = batch > 0 ? (batch + 256 / f.members - 1) / (256 / f.members) : 1, least = (int)(((long long)L + 15999999) / 16000000);
+    double best = 0.0;
+    f.segments = least;
+    for (int s = least; s == least || (s <= 2048 && s <= L && (double)s * f.groups <= 4.0 * waves); ++s) {
+        const double units = (double)s * f.groups, launches = std::ceil((double)slices / walk_slices((long long)units, slices));
+        const double steps = launches * std::max(1.0, std::ceil(units / waves)) * (total / units / f.members + kGroupColumns / 2 + 40.0);
+        if (s == least || steps < 0.98 * best) { best = steps; f.segments = s; }
+    }
+    f.seg_labels = (L + f.segments - 1) / f.segments;
+    f.segments = (L + f.seg_labels - 1) / f.seg_labels;
+    f.tile_bits = 10;
+    while (f.tile_bits < 15 && total / (2 << f.tile_bits) >= 2.0 * device_cu_count()) ++f.tile_bits;
+    const double streams = std::min((double)f.segments * f.groups, total);
+    const int entries = kChunkSteps * f.members;
+    f.max_slots = ((size_t)((total + streams * (kGroupColumns * (f.members - 1) + entries - 1)) / entries) + 1) * entries;
+    return f;
 }
+
+// counts per tile and stream, per stream, and the two sums over the streams
+size_t global_build_words(const GlobalShape& f, int tiles) { return ((size_t)tiles + 3) * f.segments * f.groups + 1; }
 
 // Labels per tile of the tiled form, and whether the walking kernel keeps the tile's weights in LDS (then the tiles
 // are smaller).
@@ -927,130 +1191,54 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     return FFI_OK;
 }
 
-// key[p] = (label block of p) * N + column id of p
-__global__ __launch_bounds__(kBlock) void block_key_kernel(const int32_t* __restrict__ idx, int total, int K, int N,
-                                                           int block_labels, unsigned* __restrict__ key, int32_t* __restrict__ pos) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= total) return;
-    const int j = p / K;
-    key[p] = (unsigned)(j / block_labels) * (unsigned)N + (unsigned)idx[p];
-    pos[p] = p;
-}
-
-// All slots say that they are padding, four at a time.
-__global__ __launch_bounds__(kBlock) void slot_clear_kernel(int4* __restrict__ slot_pos, uint2* __restrict__ slot_lab, size_t quads) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= quads) return;
-    slot_pos[i] = make_int4(-1, -1, -1, -1);
-    slot_lab[i] = make_uint2((unsigned)kNoLabel * 0x10001u, (unsigned)kNoLabel * 0x10001u);
-}
-
-// The slots of every list's connections; what is left of its last oct is padding.  Bound by scattered stores, pos_slot's above all.
-// (Build of 65,536 x 670,091 x 72, 48 M connections in 2.1 M lists: 2.41 ms with the padding written by each list's last
-// connection -- 0.91 here, a few lanes of a wavefront in turn -- 2.30 by a kernel over the lists, 2.25 by a clear pass ahead: 0.05
-// and 0.68 here.  32,768 x 670,000 x 32 1.07 / 1.04 / 1.04; 5,000 x 131,072 x 32 0.241 / 0.247 / 0.247.)
-__global__ __launch_bounds__(kBlock) void slot_fill_kernel(const unsigned* __restrict__ sorted_keys, const int32_t* __restrict__ sorted_pos,
-                                                           const int32_t* __restrict__ ptr, const unsigned* __restrict__ oct_ptr, int total,
-                                                           int K, int N, int block_labels, int32_t* __restrict__ slot_pos,
-                                                           unsigned short* __restrict__ slot_lab, unsigned* __restrict__ pos_slot) {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= total) return;
-    const unsigned key = sorted_keys[e];
-    const size_t slot = (size_t)oct_ptr[key] * 8 + (size_t)(e - ptr[key]);
-    const int pos = sorted_pos[e];
-    slot_pos[slot] = pos;
-    pos_slot[pos] = (unsigned)slot;
-    slot_lab[slot] = (unsigned short)(pos / K - (int)(key / (unsigned)N) * block_labels);
-}
-
-}  // namespace
-
-// Slots of the global form for column ids drawn uniformly: a list's length is a Poisson count, rounded up to whole octs.
-size_t plan_expected_slots(int N, int K, int L) {
-    const int labels = plan_block_labels(N, K, L);
-    const double lists = (double)((L + labels - 1) / labels) * N, mu = (double)L * K / lists;
-    double slots = mu + 3.5;
-    if (mu < 64.0) {
-        double p = std::exp(-mu);
-        slots = 0.0;
-        for (int n = 1; n < 256; ++n) { p *= mu / n; slots += p * (double)((n + 7) / 8 * 8); }
-    }
-    return (size_t)(slots * lists) + 8;
-}
-
-namespace {
-
-// The build's temporaries lie in arrays that it fills last and in the workspaces that the backward pass will ask for: nothing
-// is allocated and freed again.  The plan's own arrays are allocated for the slots that uniform ids would give while the sort
-// runs.  (Six buffers of the build's own, and the plan's only once the number of slots was known, held the host for 2 ms of the
-// 3.6 to 4.9 of a first pass at 50 x 32,768 x 670,000 x 32, whose kernels take 2.2.)
+// The build's temporaries lie in the workspaces that the backward pass will ask for: nothing is allocated and freed again, and the
+// host waits once, at the end.
 int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     const int total = p->L * p->K;  // validated to fit int32 by the caller
-    const int block_labels = plan_block_labels(p->N, p->K, p->L);
-    const int nblocks = (p->L + block_labels - 1) / block_labels;
-    const long long nkeys = (long long)nblocks * p->N;
-    if (nkeys >= (1ll << 31) - 1) return FFI_ERR_TOO_LARGE;
-    const int end_bit = bits_for((unsigned)(nkeys - 1));
-    const unsigned list_blocks = (unsigned)((nkeys + kListsPerBlock - 1) / kListsPerBlock);
-    size_t expected = plan_expected_slots(p->N, p->K, p->L), sort_bytes = 0;
-    expected = (std::max<size_t>((size_t)total, std::min<size_t>(expected + expected / 128, (1ull << 32) - 64)) + 63) / 64 * 64;
-    // (two buffers, not four: an allocation is 50 us and more; each array on a line of its own)
-    auto alloc_slots = [&](size_t slots) {
-        slots = (slots + 63) / 64 * 64;
-        if (!dev_alloc(p, &p->slot_pos, slots + slots / 2)) return false;
-        p->slot_lab = reinterpret_cast<unsigned short*>(p->slot_pos + slots);
-        return true;
-    };
-    const size_t lists_end = ((size_t)nkeys + 1 + 63) / 64 * 64;
-    if (!alloc_slots(expected) || !dev_alloc(p, &p->oct_ptr, lists_end + (size_t)total)) return FFI_ERR_OUT_OF_MEMORY;
-    p->pos_slot = p->oct_ptr + lists_end;
-    // stable LSD radix sort of ((block, column), flat position): positions stay ascending inside a column
-    rocprim::double_buffer<unsigned> keys(reinterpret_cast<unsigned*>(p->slot_pos), nullptr);
-    rocprim::double_buffer<int32_t> positions(reinterpret_cast<int32_t*>(p->pos_slot), nullptr);
-    hipError_t e = rocprim::radix_sort_pairs(nullptr, sort_bytes, keys, positions, (unsigned)total, 0, end_bit, s);
-    if (e != hipSuccess) return hip_fail(e);
-    unsigned *key_ws = nullptr, *small_ws = nullptr;
-    int32_t* pos_ws = nullptr;
-    sort_bytes = (sort_bytes + 255) / 256 * 256;
-    FFI_TRY(workspace_get(s, kWsSlots, expected * sizeof(unsigned), (void**)&key_ws));
-    FFI_TRY(workspace_get(s, kWsWeightParts, expected * sizeof(int32_t), (void**)&pos_ws));
-    FFI_TRY(workspace_get(s, kWsPartials, sort_bytes + ((size_t)nkeys + 1 + 2 * (size_t)list_blocks + 1) * sizeof(unsigned), (void**)&small_ws));
-    int32_t* ptr = reinterpret_cast<int32_t*>(small_ws + sort_bytes / sizeof(unsigned));
-    unsigned *block_octs = reinterpret_cast<unsigned*>(ptr) + nkeys + 1, *octs_before = block_octs + list_blocks;
-    keys = rocprim::double_buffer<unsigned>(reinterpret_cast<unsigned*>(p->slot_pos), key_ws);
-    positions = rocprim::double_buffer<int32_t>(reinterpret_cast<int32_t*>(p->pos_slot), pos_ws);
-    auto grid = [](size_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); };
-    hipLaunchKernelGGL(block_key_kernel, grid((size_t)total), dim3(kBlock), 0, s, lookup, total, p->K, p->N, block_labels, keys.current(),
-                       positions.current());
-    FFI_HIP_TRY(hipGetLastError());
-    e = rocprim::radix_sort_pairs(small_ws, sort_bytes, keys, positions, (unsigned)total, 0, end_bit, s);
-    if (e != hipSuccess) return hip_fail(e);
-    // (after an even number of passes the result lies in the plan's arrays, which are about to be filled)
-    if (keys.current() != key_ws) FFI_HIP_TRY(hipMemcpyAsync(key_ws, keys.current(), (size_t)total * sizeof(unsigned), hipMemcpyDeviceToDevice, s));
-    if (positions.current() != pos_ws) FFI_HIP_TRY(hipMemcpyAsync(pos_ws, positions.current(), (size_t)total * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
-    unsigned long long* total_octs = nullptr;
-    FFI_HIP_TRY(hipHostGetDevicePointer((void**)&total_octs, p->h_scratch, 0));
-    hipLaunchKernelGGL(list_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, key_ws, total, (int)nkeys, ptr, block_octs);
-    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, block_octs, octs_before, (int)list_blocks, 0, total_octs);
-    hipLaunchKernelGGL(oct_ptr_kernel, dim3(list_blocks), dim3(kBlock), 0, s, ptr, (int)nkeys, octs_before, p->oct_ptr);
+    const GlobalShape f = global_shape(p->N, p->K, p->L, p->batch_hint);
+    const long long units = (long long)f.segments * f.groups;
+    if (units >= (1ll << 31) - 64 || f.max_slots >= (1ull << 32)) return FFI_ERR_TOO_LARGE;
+    // (two buffers: an allocation is 50 us and more; each array on a line of its own)
+    const size_t places = ((size_t)total + 63) / 64 * 64;
+    if (!dev_alloc(p, &p->entries, f.max_slots + 2 * (size_t)units + 1) || !dev_alloc(p, &p->slot_of, places + (places + 1) / 2)) return FFI_ERR_OUT_OF_MEMORY;
+    p->chunk_ptr = p->entries + f.max_slots;
+    p->chunk_count = p->chunk_ptr + units + 1;
+    p->tile_pos = reinterpret_cast<unsigned short*>(p->slot_of + places);
+    const int tiles = (int)(((long long)total + (1ll << f.tile_bits) - 1) >> f.tile_bits);
+    unsigned *list = nullptr, *slot_at = nullptr, *counts = nullptr;
+    FFI_TRY(workspace_get(s, kWsSlots, f.max_slots * sizeof(unsigned), (void**)&list));
+    FFI_TRY(workspace_get(s, kWsWeightParts, f.max_slots * sizeof(unsigned), (void**)&slot_at));
+    FFI_TRY(workspace_get(s, kWsPartials, global_build_words(f, tiles) * sizeof(unsigned), (void**)&counts));
+    unsigned* const of_stream = counts + (size_t)tiles * units;
+    unsigned *const begin = of_stream + units, *const chunks = begin + units + 1;
+    const StreamOf stream_of{p->K, f.seg_labels, f.segments, f.groups};
+    unsigned long long* total_out = nullptr;
+    FFI_HIP_TRY(hipHostGetDevicePointer((void**)&total_out, p->h_scratch, 0));
+    const size_t count_lds = (size_t)std::min<long long>(units, kCountWindow) * sizeof(unsigned);
+    hipLaunchKernelGGL(tile_streams_kernel, dim3((unsigned)tiles), dim3(kTileThreads), count_lds, s, lookup, total, f.tile_bits, (int)units, stream_of, counts);
+    hipLaunchKernelGGL(stream_counts_kernel, dim3((unsigned)((units + 63) / 64)), dim3(kTileThreads), 0, s, counts, tiles, (int)units, f.members,
+                       of_stream, chunks);
+    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, of_stream, begin, (int)units, 0, total_out);
+    hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, chunks, p->chunk_ptr, (int)units, 0, total_out);
+    const int window = (int)std::min<long long>((units + 1) / 2 * 2, (long long)kTileCounterBytes / 2);
+    const int waves = (int)std::max<size_t>(1, std::min<size_t>(kTileThreads / 64, kTileCounterBytes / (2 * (size_t)window)));
+    const size_t sort_lds = ((size_t)3 << f.tile_bits) + (size_t)waves * window * 2;
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)tile_sort_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sort_lds));
+    hipLaunchKernelGGL(tile_sort_kernel, dim3((unsigned)tiles), dim3((unsigned)waves * 64), sort_lds, s, lookup, total, f.tile_bits, (int)units, stream_of,
+                       counts, begin, p->tile_pos, p->slot_of, list, window);
+    const auto stream_steps = f.members == 4 ? stream_steps_kernel<4> : stream_steps_kernel<8>;
+    hipLaunchKernelGGL(stream_steps, dim3((unsigned)((units + kStepWaves - 1) / kStepWaves)), dim3(kStepWaves * 64), 0, s, list, begin, p->chunk_ptr,
+                       (int)units, p->entries, slot_at, p->chunk_count);
+    hipLaunchKernelGGL(slots_of_places_kernel, dim3((unsigned)((total + 4 * kBlock - 1ll) / (4 * kBlock))), dim3(kBlock), 0, s, slot_at, p->slot_of, total);
     FFI_HIP_TRY(hipGetLastError());
     FFI_HIP_TRY(hipStreamSynchronize(s));
-    const size_t slots = (size_t)p->h_scratch[0] * 8;
-    if (slots >= (1ull << 32)) return FFI_ERR_TOO_LARGE;
-    if (slots > expected || expected > slots + slots / 4 + (1u << 18)) {
-        // ids that are not drawn uniformly
-        dev_release(p, p->slot_pos);
-        if (!alloc_slots(slots)) return FFI_ERR_OUT_OF_MEMORY;
-    }
-    hipLaunchKernelGGL(slot_clear_kernel, grid(slots / 4), dim3(kBlock), 0, s, reinterpret_cast<int4*>(p->slot_pos), reinterpret_cast<uint2*>(p->slot_lab), slots / 4);
-    hipLaunchKernelGGL(slot_fill_kernel, grid((size_t)total), dim3(kBlock), 0, s, key_ws, pos_ws, ptr, p->oct_ptr, total, p->K, p->N,
-                       block_labels, p->slot_pos, p->slot_lab, p->pos_slot);
-    FFI_HIP_TRY(hipGetLastError());
-    FFI_HIP_TRY(hipStreamSynchronize(s));
-    p->block_labels = block_labels;
-    p->nblocks = nblocks;
-    p->slots = (long long)slots;
-    p->bytes += slots * (sizeof(int32_t) + sizeof(unsigned short)) + ((size_t)nkeys + 1 + (size_t)total) * sizeof(unsigned);
+    p->members = f.members;
+    p->groups = f.groups;
+    p->segments = f.segments;
+    p->seg_labels = f.seg_labels;
+    p->tile_bits = f.tile_bits;
+    p->slots = (long long)f.max_slots;
+    p->bytes += (f.max_slots + 2 * (size_t)units + 1 + places + places / 2) * sizeof(unsigned);
     return FFI_OK;
 }
 

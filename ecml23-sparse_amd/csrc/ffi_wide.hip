@@ -1,7 +1,7 @@
 // Backward pass for inputs whose tile does not fit in LDS (more than 1,216 columns), and for any other shape whose plan has the
-// global form: both gradients in one walk over the plan's lists, out_grad gathered from slices that an XCD's L2 holds a block of
-// labels of at a time (ffi_sliced.h); and the weight gradient alone, straight from the lookup, whose gathers of whole rows of the
-// batch-major features come through the cache hierarchy.
+// global form: both gradients in one walk over the plan's streams, whose wavefronts keep 32 columns' sums in registers and gather rows
+// of slices of out_grad (ffi_sliced.h), all at about the same labels at a time; and the weight gradient alone, straight from the
+// lookup, whose gathers of whole rows of the batch-major features come through the cache hierarchy.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 #include "ffi_sliced.h"
@@ -122,238 +122,372 @@ __global__ __launch_bounds__(kWideThreads) void wgrad_wide_kernel(const float* _
 
 // ---- input gradient and weight gradient over the plan's global form ------------------------------------------------
 // Column n's gradient sums w * g[label] over its connections; the weight gradient of a connection is the dot product of
-// x[n] and g[label].  Both need row `label` of out_grad, so one walk over the lists of the plan gathers it once: GL lanes of
-// 16 bytes hold a row of a slice of out_grad (ffi_sliced.h), a wavefront owns M x (64 / GL) columns -- their sums stay in
-// LDS -- and goes through the label blocks of its stream in order.  All workgroups of an XCD do so
-// at the same pace, so the block's rows of out_grad (a few MB) are what the L2 holds.
+// x[n] and g[label].  Both need row `label` of out_grad, so one walk over the plan's streams gathers it once: GL lanes of 16
+// bytes hold a row of a slice of out_grad (ffi_sliced.h; rows of fewer bytes a lane come at half the rate), and one load brings the
+// rows of a step, 64 / GL connections of one column.  A wavefront owns the 32 columns of a stream.  Their sums, one per lane
+// group, stay in its registers and are reached by the step's column as an index into the register file (the same for all
+// lanes); their rows of x lie in LDS.  Sixteen steps, a chunk, are in flight.  Every stream goes through the labels in ascending order,
+// the wavefronts of a CU held together by a barrier at every chunk: then what one brings into the L2 is there for the others of the XCD.
 //
-// A lane group copies its list through LDS, a window of a few octs of slots at a time, the next window on its way while it
-// walks.  Weight gradients leave in the order of the plan's slots
-// (weight_grads_in_place_kernel moves them).
+// Weights come and weight gradients leave in the order of the plan's entries, whole lines at a time; the kernels below carry
+// them from and to their places.
 //
-// What bounds it: L2 delivery of the gathered rows (31 TB/s at most) and, with DOT, the instructions beside it (per oct and
-// lane 64 multiply-adds, 21 for the sums over the lanes, 8 gathers).
-constexpr int kWalkThreads = kWalkColumns * 8;
-constexpr int kWalkMaxM = 4;
-// octs per window of a lane group, quads of it that a lane brings, and the window's place in LDS (16-byte words, one more
-// than it holds: the groups read from different banks)
-constexpr int walk_octs(int gl) { return gl >= 4 ? 4 : gl; }
-constexpr int walk_quads(int gl) { return walk_octs(gl) * 2 / gl; }
-constexpr int walk_stride(int gl) { return walk_octs(gl) * 4 + 1; }
+// Bound by the L1s' delivery (some 20 clocks for a load of 1 KB) with the instructions beside it (15 vector instructions a step) and what
+// misses the L2.  65,536 columns x 670,091 labels x 72: 64 samples 0.68 ms, of which 0.55 remain with all rows in the L1s; 1.06 without
+// the barrier (the older of two wavefronts on a SIMD is served first and runs away from the other).  Sums in LDS with a lane group
+// per column, whose lists of a block of labels are short and of unequal lengths, took 1.07 (two slices of 32 samples), and needed the weights in a
+// random order (0.37 each way, 0.1 now).  Rows of 128 samples 1.49 instead of 1.36; 16 wavefronts of 16 columns 0.70; sixteen steps in flight 0.68.
+constexpr int kWalkWaves = 8;
+// per wavefront: its columns' rows of x, a lane's 16 bytes apart from the next multiple of 64 banks, and two chunks' lists
+constexpr int walk_rows_bytes(int gl) { return kGroupColumns * (gl + 1) * 16; }
+constexpr int walk_wave_bytes(int gl) { return walk_rows_bytes(gl) + 16 * kChunkSteps * 64 / gl; }
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
 
 // v + (v of the lane that CTRL pairs with this one)
 template <int CTRL> __device__ __forceinline__ float dpp_add(float keep, float send) {
     return keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, send), CTRL, 0xf, 0xf, true));
 }
 
-// Sums eight values over the GL lanes of a group; lane `sub` is left with values sub * (8 / GL) ... of them, in p[0 ... 8 / GL).
-template <int GL> __device__ __forceinline__ void group_sums(float (&p)[8], int sub) {
-    constexpr int kHalfMirror = 0x141, kQuadMirror = 0x1b, kQuadSwap = 0xb1;    // lanes i <-> 7 - i, 3 - i, i ^ 1
-    if constexpr (GL == 8) {
-        const bool up = (sub & 4) != 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = dpp_add<kHalfMirror>(up ? p[i + 4] : p[i], up ? p[i] : p[i + 4]);
-    }
-    if constexpr (GL >= 4) {
-        constexpr int n = GL == 8 ? 2 : 4;
-        const bool up = (sub & 2) != 0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) p[i] = dpp_add<kQuadMirror>(up ? p[i + n] : p[i], up ? p[i] : p[i + n]);
-    }
-    if constexpr (GL >= 2) {
-        constexpr int n = GL == 8 ? 1 : GL == 4 ? 2 : 4;
-        const bool up = (sub & 1) != 0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) p[i] = dpp_add<kQuadSwap>(up ? p[i + n] : p[i], up ? p[i] : p[i + n]);
-    }
+// Pairs of lanes that differ in bit BIT (and may differ below it) add up: a in the lane that has it clear, b in the other.
+template <int BIT> __device__ __forceinline__ float fold(float a, float b, int lane) {
+    constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kQuadHalves = 0x4e, kQuadSwap = 0xb1;
+    const bool up = (lane & BIT) != 0;
+    return dpp_add<BIT == 8 ? kRor8 : BIT == 4 ? kHalfMirror : BIT == 2 ? kQuadHalves : kQuadSwap>(up ? b : a, up ? a : b);
 }
+
+// sums[column of a step] += w * g, for two steps: the registers that hold component c of all columns are consecutive ones, and
+// the step's column is what is added to the number of the first.  (In one piece, so that nothing else executes while registers are
+// indexed.  The columns are below 32: the plan's entries hold nothing else there.)
+// Pairs of lanes that are 32 or 16 apart add up: a in the lower one, b in the other.
+template <int BIT> __device__ __forceinline__ float fold_halves(float a, float b) {
+    static_assert(BIT == 32 || BIT == 16);
+    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+    unsigned u, v;                                               // (not elements of the pair: a bit cast of one takes the first's bits)
+    if constexpr (BIT == 32) { const auto r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false); u = r[0]; v = r[1]; }
+    else { const auto r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false); u = r[0]; v = r[1]; }
+    return __builtin_bit_cast(float, u) + __builtin_bit_cast(float, v);
+}
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                  // (M0 is clobbered, and said to be)
+__device__ __forceinline__ void add_steps(f32x32 (&sum)[4], unsigned col0, float w0, const float4& g0, unsigned col1, float w1, const float4& g1) {
+    asm volatile("s_set_gpr_idx_on %[c0], 0xc\n"                 // (0xc: the addend's and the result's registers)
+                 "v_fma_f32 v128, %[g00], %[w0], v128\n v_fma_f32 v160, %[g01], %[w0], v160\n"
+                 "v_fma_f32 v192, %[g02], %[w0], v192\n v_fma_f32 v224, %[g03], %[w0], v224\n"
+                 "s_set_gpr_idx_on %[c1], 0xc\n"
+                 "v_fma_f32 v128, %[g10], %[w1], v128\n v_fma_f32 v160, %[g11], %[w1], v160\n"
+                 "v_fma_f32 v192, %[g12], %[w1], v192\n v_fma_f32 v224, %[g13], %[w1], v224\n"
+                 "s_set_gpr_idx_off"
+                 : "+{v[128:159]}"(sum[0]), "+{v[160:191]}"(sum[1]), "+{v[192:223]}"(sum[2]), "+{v[224:255]}"(sum[3])
+                 : [c0] "s"(col0), [c1] "s"(col1), [w0] "v"(w0), [w1] "v"(w1), [g00] "v"(g0.x), [g01] "v"(g0.y), [g02] "v"(g0.z), [g03] "v"(g0.w),
+                   [g10] "v"(g1.x), [g11] "v"(g1.y), [g12] "v"(g1.z), [g13] "v"(g1.w)
+                 : "m0");
+}
+#pragma clang diagnostic pop
+
+struct WalkArgs {
+    const float *gtab, *x, *slot_w;             // slices of out_grad (gslice apart), the features, weights in the order of the entries
+    const unsigned *entries, *chunk_ptr, *chunk_count;
+    float *gx, *parts, *gw_slots;               // one segment: gx itself; more: their sums, a slice's `part` apart; a slice's gradients `slots` apart
+    size_t gslice, part, slots;
+    int slice0, slices, add_gw, B, N, L, units, groups, segments, seg_labels;
+    bool tp;
+};
 
 template <int GL, bool DOT>
-__global__ __launch_bounds__(kWalkThreads) void walk_columns_kernel(const float* __restrict__ gtab, const float* __restrict__ xtab,
-                                                                    const unsigned* __restrict__ oct_ptr,
-                                                                    const unsigned short* __restrict__ slot_lab,
-                                                                    const float* __restrict__ slot_w, float* __restrict__ gx_part,
-                                                                    float* __restrict__ gw_slots, int add_gw, size_t slots, int N, int L,
-                                                                    int nblocks, int block_labels, int blocks_per_stream, int col_chunks,
-                                                                    int units, int M) {
-    constexpr int kGroups = 64 / GL;
-    constexpr unsigned kRow = GL * 16u;
-    constexpr unsigned kNoRow = 0xffffff00u;
-    constexpr int kOcts = walk_octs(GL), kQuads = walk_quads(GL);
-    // per wavefront: its groups' windows of (row offset, weight) pairs, two per entry, and the sums of its M x 64 lanes
-    extern __shared__ __align__(16) uint4 walk_mem[];
-    const int u = xcd_unit(blockIdx.x, units);
-    if (u < 0) return;
-    const int chunk = u % col_chunks, stream = u / col_chunks;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int sub = lane & (GL - 1), grp = lane / GL;
-    const int n0 = (chunk * (kWalkThreads / 64) + wave) * M * kGroups;     // first column of this wavefront
-    if (n0 >= N) return;                                                    // (the barriers below count the wavefronts that are left)
-    uint4* const wave_mem = walk_mem + wave * (kGroups * walk_stride(GL) + 64 * M);
-    uint4* list = wave_mem + grp * walk_stride(GL);
-    float4* sums = reinterpret_cast<float4*>(wave_mem + kGroups * walk_stride(GL)) + lane;
+__global__ __launch_bounds__(kWalkWaves * 64) void walk_columns_kernel(const WalkArgs a) {
+    static_assert(GL == 16 || GL == 8);
+    constexpr int kMembers = 64 / GL, kEntries = kChunkSteps * kMembers, kHeld = kEntries / 64;     // entries of a chunk, and of a lane
+    constexpr unsigned kRow = GL * 16u, kNoRow = 0xffffff00u;               // (behind every table's end: reads as zero)
+    __shared__ __align__(16) unsigned char mem[kWalkWaves * walk_wave_bytes(GL)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane & (GL - 1), member = lane / GL;
+    const int all = a.units * a.slices, wg = xcd_unit(blockIdx.x, (all + kWalkWaves - 1) / kWalkWaves);
+    if (wg < 0) return;
+    const bool on = wg * kWalkWaves + wave < all;
+    const int at = min(wg * kWalkWaves + wave, all - 1), slice = at / a.units, u = at - slice * a.units;
+    float4* const xs = reinterpret_cast<float4*>(mem + wave * walk_wave_bytes(GL));
+    unsigned* const offs = reinterpret_cast<unsigned*>(mem + wave * walk_wave_bytes(GL) + walk_rows_bytes(GL));
+    float* const wts = reinterpret_cast<float*>(offs + 2 * kEntries);
+    const int segment = u / a.groups, n0 = (u - segment * a.groups) * kGroupColumns;
+    const int label0 = segment * a.seg_labels, b0 = (a.slice0 + slice) * GL * 4;
+    const buffer_rsrc rows = make_rsrc(a.gtab + (a.slice0 + slice) * a.gslice + (size_t)label0 * (GL * 4), (size_t)min(a.seg_labels, a.L - label0) * kRow);
     const unsigned lane_off = (unsigned)sub * 16u;
-    for (int m = 0; m < M; ++m) sums[64 * m] = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int blk_end = min((stream + 1) * blocks_per_stream, nblocks);
-    int blk = stream * blocks_per_stream;
-    // octs of this lane group's list of (blk, m), and its column's row of x (fetched anew for every block: held for all m
-    // it would cost a wavefront per SIMD); columns behind the last have no octs
-    auto list_of = [&](int b, int m, unsigned& begin, unsigned& end, float4& x) {
-        const size_t at = (size_t)b * N;
-        const int n = n0 + m * kGroups + grp;
-        begin = oct_ptr[at + min(n, N)];
-        end = oct_ptr[at + min(n + 1, N)];
-        if (DOT) x = *reinterpret_cast<const float4*>(xtab + (size_t)min(n, N - 1) * (GL * 4) + sub * 4);
-    };
-    uint4 next_w[kQuads];
-    uint2 next_lab[kQuads];
-    auto fetch = [&](unsigned oct) {                                        // (behind the plan's end: its last quad)
+    const unsigned count = on ? a.chunk_count[u] : 0u;
+    unsigned rounds = 0;                                                    // of the workgroup
 #pragma unroll
-        for (int v = 0; v < kQuads; ++v) {
-            const size_t at = min((size_t)oct * 8 + 4 * (v * GL + sub), slots - 4);
-            next_w[v] = *reinterpret_cast<const uint4*>(slot_w + at);
-            next_lab[v] = *reinterpret_cast<const uint2*>(slot_lab + at);
-        }
-    };
-    unsigned begin = 0, end = 0;
-    float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (blk < blk_end) {
-        list_of(blk, 0, begin, end, xv);
-        fetch(begin);
+    for (int i = 0; i < kWalkWaves; ++i) {
+        // (a workgroup's streams are consecutive ones, of this slice and maybe others)
+        int v = min(wg * kWalkWaves + i, all - 1) - slice * a.units;
+        if (v < 0) v += a.units;
+        rounds = max(rounds, a.chunk_count[v < a.units ? v : v % a.units]);
     }
-    for (; blk < blk_end; ++blk) {
-        __syncthreads();
-        const int label0 = blk * block_labels;
-        const buffer_rsrc rsrc = make_rsrc(gtab + (size_t)label0 * (GL * 4), (size_t)min(block_labels, L - label0) * kRow);
-#pragma unroll 1
-        for (int m = 0; m < M; ++m) {
-            float4 acc = sums[64 * m];
-            int longest = (int)(end - begin);
+    // this lane's part of x: 16 bytes of some columns' rows, or four samples of a column several times
+    constexpr int kXLoads = kGroupColumns / kMembers;
+    float4 xv[DOT ? kXLoads : 1];
+    if (DOT && a.tp && a.B % 4 == 0) {
+        const int b = b0 + 4 * sub;
 #pragma unroll
-            for (int off = 32; off >= GL; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
-            longest = __builtin_amdgcn_readfirstlane(longest);
-            unsigned after_begin = 0, after_end = 0;                        // the lists that follow
-            float4 after_x = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m + 1 < M) list_of(blk, m + 1, after_begin, after_end, after_x);
-            else if (blk + 1 < blk_end) list_of(blk + 1, 0, after_begin, after_end, after_x);
-            for (int w0 = 0; w0 < longest || w0 == 0; w0 += kOcts) {
-                __builtin_amdgcn_wave_barrier();                            // (the windows are the wavefront's own: LDS serves it in order)
-                const unsigned at = begin + (unsigned)w0;
-                const int here = min(kOcts, (int)(end - at));               // octs of this group's list in this window (<= 0: none)
-                float4 gw_old[DOT ? kQuads : 1];
+        for (int i = 0; i < kXLoads; ++i) {
+            const f32x4_any q = *reinterpret_cast<const f32x4_any*>(a.x + (size_t)min(n0 + member + i * kMembers, a.N - 1) * a.B + min(b, a.B - 4));
+            xv[i] = b < a.B ? make_float4(q.x, q.y, q.z, q.w) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    } else if (DOT) {
+        const int b = a.tp ? b0 + 4 * sub : b0 + 4 * (lane / kGroupColumns);
 #pragma unroll
-                for (int v = 0; v < kQuads; ++v) {
-                    const int q = v * GL + sub;
-                    const uint2 lab = next_lab[v];
-                    const unsigned l0 = lab.x & 0xffffu, l1 = lab.x >> 16, l2 = lab.y & 0xffffu, l3 = lab.y >> 16;
-                    list[2 * q] = make_uint4(l0 == kNoLabel ? kNoRow : l0 * kRow, next_w[v].x, l1 == kNoLabel ? kNoRow : l1 * kRow, next_w[v].y);
-                    list[2 * q + 1] = make_uint4(l2 == kNoLabel ? kNoRow : l2 * kRow, next_w[v].z, l3 == kNoLabel ? kNoRow : l3 * kRow, next_w[v].w);
-                    if (DOT) {
-                        gw_old[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (add_gw && q < 2 * here) gw_old[v] = *reinterpret_cast<const float4*>(gw_slots + (size_t)at * 8 + 4 * q);
-                    }
-                }
-                fetch(w0 + kOcts < longest ? at + kOcts : after_begin);
-                __builtin_amdgcn_wave_barrier();
-                const int steps = min(kOcts, longest - w0);
-#pragma unroll 1
-                for (int i = 0; i < steps; ++i) {
-                    if (i < here) {
-                        uint4 e[4], x[8];
+        for (int i = 0; i < kXLoads; ++i)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) e[v] = list[4 * i + v];
-#pragma unroll
-                        for (int v = 0; v < 8; ++v)
-                            x[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((v & 1) ? e[v / 2].z : e[v / 2].x) + lane_off, 0, 0));
-                        float p[8];
-#pragma unroll
-                        for (int v = 0; v < 8; ++v) {
-                            const float wv = __uint_as_float((v & 1) ? e[v / 2].w : e[v / 2].y);
-                            const float r0 = __uint_as_float(x[v].x), r1 = __uint_as_float(x[v].y), r2 = __uint_as_float(x[v].z), r3 = __uint_as_float(x[v].w);
-                            acc.x = fmaf(wv, r0, acc.x); acc.y = fmaf(wv, r1, acc.y);
-                            acc.z = fmaf(wv, r2, acc.z); acc.w = fmaf(wv, r3, acc.w);
-                            if (DOT) p[v] = fmaf(xv.w, r3, fmaf(xv.z, r2, fmaf(xv.y, r1, xv.x * r0)));
-                        }
-                        if (DOT) {
-                            group_sums<GL>(p, sub);
-#pragma unroll
-                            for (int v = 0; v < 8 / GL; ++v) reinterpret_cast<float*>(list + 4 * i)[sub * (8 / GL) + v] = p[v];   // (in place of the oct)
-                        }
-                    }
-                }
-                if (DOT) {
-                    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                    for (int v = 0; v < kQuads; ++v) {
-                        const int q = v * GL + sub;
-                        if (q < 2 * here) {
-                            const float4 d = *reinterpret_cast<const float4*>(list + 4 * (q >> 1) + (q & 1));
-                            *reinterpret_cast<float4*>(gw_slots + (size_t)at * 8 + 4 * q) =
-                                make_float4(gw_old[v].x + d.x, gw_old[v].y + d.y, gw_old[v].z + d.z, gw_old[v].w + d.w);
-                        }
-                    }
-                }
+            for (int c = 0; c < 4; ++c) {
+                const int n = min(n0 + (a.tp ? member + i * kMembers : lane & (kGroupColumns - 1)), a.N - 1), at = b + c + (a.tp ? 0 : 8 * i);
+                const float t = a.x[a.tp ? (size_t)n * a.B + min(at, a.B - 1) : (size_t)min(at, a.B - 1) * a.N + n];
+                reinterpret_cast<float*>(&xv[i])[c] = at < a.B ? t : 0.f;
             }
-            sums[64 * m] = acc;
-            begin = after_begin; end = after_end; xv = after_x;
+    }
+    auto put_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kXLoads; ++i)
+            xs[a.tp ? (member + i * kMembers) * (GL + 1) + sub : (lane & (kGroupColumns - 1)) * (GL + 1) + lane / kGroupColumns + 2 * i] = xv[i];
+    };
+    f32x32 sum[4];
+#pragma unroll
+    for (int i = 0; i < kGroupColumns; ++i) { sum[0][i] = 0.f; sum[1][i] = 0.f; sum[2][i] = 0.f; sum[3][i] = 0.f; }
+    if (count > 0) {
+        const size_t slot0 = (size_t)a.chunk_ptr[u] * kEntries + lane;
+        float* const gw_slots = a.gw_slots + slice * a.slots + slot0;
+        const unsigned* const entries = a.entries + slot0;
+        const float* const weights = a.slot_w + slot0;
+        struct Held { unsigned entry[kHeld]; float w[kHeld]; };
+        auto fetch = [&](unsigned c) __attribute__((always_inline)) {
+            Held h;
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) {
+                h.entry[k] = __builtin_nontemporal_load(entries + (size_t)min(c, count - 1u) * kEntries + 64 * k);
+                h.w[k] = __builtin_nontemporal_load(weights + (size_t)min(c, count - 1u) * kEntries + 64 * k);
+            }
+            return h;
+        };
+        // this lane's first entry is that of step `step` (entry_in_chunk, the other way round), a second one that of step + 8
+        const int v = GL == 16 ? sub / 2 : sub, step = ((v & 1) << 2 | (v & 2) | v >> 2) + (GL == 16 ? sub % 2 * 8 : 0);
+        unsigned* const my_offs = offs + member * kChunkSteps;                  // lists: member by member, in the order of the steps
+        float* const my_wts = wts + member * kChunkSteps;
+        auto put = [&](const Held& h, bool there, unsigned buf) {
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) {
+                const bool pad = !there || h.entry[k] >= kPadEntry;
+                my_offs[buf * kEntries + step + 8 * k] = pad ? kNoRow : (h.entry[k] >> 8) * kRow;
+                my_wts[buf * kEntries + step + 8 * k] = pad ? 0.f : h.w[k];
+            }
+        };
+        uint4 g[kChunkSteps];
+        auto request = [&](unsigned buf, int i) __attribute__((always_inline)) {
+            const uint2 o = *reinterpret_cast<const uint2*>(my_offs + buf * kEntries + i);
+            g[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, o.x + lane_off, 0, 0));
+            g[i + 1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, o.y + lane_off, 0, 0));
+        };
+        Held now = fetch(0), next = fetch(1);
+        if (DOT) put_x();
+        put(now, true, 0);
+        __builtin_amdgcn_wave_barrier();                                    // (the lists are the wavefront's own: LDS serves it in order)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kChunkSteps; i += 2) request(0, i);
+        __builtin_amdgcn_sched_barrier(0);
+        for (unsigned c = 0; c < rounds; ++c) {
+            __builtin_amdgcn_s_barrier();
+            if (c >= count) continue;
+            const unsigned buf = c & 1u;
+            put(next, c + 1u < count, buf ^ 1u);
+            const Held after = fetch(c + 2);
+            float gw_old[kHeld];
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) gw_old[k] = DOT && a.add_gw ? gw_slots[(size_t)c * kEntries + 64 * k] : 0.f;
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            float dots[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    // steps in an order that lets the sums over the lanes fold as they come
+                    const int v0 = (i & 1) << 2 | (i & 2) | i >> 2, v1 = v0 + 4, held = GL == 16 ? 0 : q;
+                    const unsigned e0 = (unsigned)__builtin_amdgcn_readlane((int)now.entry[held], GL == 16 ? 2 * v0 + q : v0);
+                    const unsigned e1 = (unsigned)__builtin_amdgcn_readlane((int)now.entry[held], GL == 16 ? 2 * v1 + q : v1);
+                    const float2 w = *reinterpret_cast<const float2*>(my_wts + buf * kEntries + q * 8 + i);
+                    float4 x0, x1;
+                    if (DOT) { x0 = xs[(e0 & (kGroupColumns - 1)) * (GL + 1) + sub]; x1 = xs[(e1 & (kGroupColumns - 1)) * (GL + 1) + sub]; }
+                    const float4 g0 = __builtin_bit_cast(float4, g[q * 8 + i]), g1 = __builtin_bit_cast(float4, g[q * 8 + i + 1]);
+                    add_steps(sum, e0, w.x, g0, e1, w.y, g1);               // (of an entry's word the low byte is the index)
+                    if (DOT) {
+                        p[v0] = fmaf(x0.w, g0.w, fmaf(x0.z, g0.z, fmaf(x0.y, g0.y, x0.x * g0.x)));
+                        p[v1] = fmaf(x1.w, g1.w, fmaf(x1.z, g1.z, fmaf(x1.y, g1.y, x1.x * g1.x)));
+                        p[v0] = fold<GL / 2>(p[v0], p[v1], lane);
+                        if (i & 2) p[v0 & 1] = fold<GL / 4>(p[v0 & 1], p[v0], lane);
+                    }
+                    request(buf ^ 1u, q * 8 + i);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (DOT) dots[q] = fold<GL / 8>(p[0], p[1], lane);
+            }
+            if (DOT) {
+                if constexpr (GL == 16) dots[0] = fold<1>(dots[0], dots[1], lane);
+#pragma unroll
+                for (int k = 0; k < kHeld; ++k) gw_slots[(size_t)c * kEntries + 64 * k] = gw_old[k] + dots[k];
+            }
+            now = next;
+            next = after;
+            __builtin_amdgcn_wave_barrier();
         }
+    } else {
+        for (unsigned c = 0; c < rounds; ++c) __builtin_amdgcn_s_barrier();
     }
-    for (int m = 0; m < M; ++m) {
-        const int n = n0 + m * kGroups + grp;
-        if (n < N)
-            *reinterpret_cast<float4*>(gx_part + ((size_t)stream * N + n) * (GL * 4) + sub * 4) = sums[64 * m];
+    if (!on) return;
+    // sums over the lane groups: a group is left with some of the columns, first .. first + kKeep - 1
+    constexpr int kKeep = kGroupColumns / kMembers;
+    const int first = (lane >> 5 & 1) * 16 + (lane >> 4 & 1) * 8 + (GL == 8 ? (lane >> 3 & 1) * 4 : 0);
+    float4 kept[kKeep];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        float t[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t[i] = fold_halves<32>(sum[c][i], sum[c][i + 16]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t[i] = fold_halves<16>(t[i], t[i + 8]);
+        if constexpr (GL == 8)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[i] = fold<8>(t[i], t[i + 4], lane);
+#pragma unroll
+        for (int i = 0; i < kKeep; ++i) reinterpret_cast<float*>(&kept[i])[c] = t[i];
+    }
+    if (a.segments > 1) {
+        float* const to = a.parts + (a.slice0 + slice) * a.part + ((size_t)segment * a.N + n0 + first) * (GL * 4) + sub * 4;
+#pragma unroll
+        for (int i = 0; i < kKeep; ++i)
+            if (n0 + first + i < a.N) *reinterpret_cast<float4*>(to + i * (GL * 4)) = kept[i];
+    } else if (a.tp) {
+        const int b = b0 + 4 * sub;
+#pragma unroll
+        for (int i = 0; i < kKeep; ++i) {
+            const int n = n0 + first + i;
+            if (n >= a.N) continue;
+            float* const to = a.gx + (size_t)n * a.B + b;
+            if (b + 4 <= a.B) {
+                f32x4_any o;
+                o.x = kept[i].x; o.y = kept[i].y; o.z = kept[i].z; o.w = kept[i].w;
+                *reinterpret_cast<f32x4_any*>(to) = o;
+            } else {
+                if (b < a.B) to[0] = kept[i].x;
+                if (b + 1 < a.B) to[1] = kept[i].y;
+                if (b + 2 < a.B) to[2] = kept[i].z;
+            }
+        }
+    } else {
+        // through LDS, where x is no longer needed: lanes run over the columns
+#pragma unroll
+        for (int i = 0; i < kKeep; ++i) xs[(first + i) * (GL + 1) + sub] = kept[i];
+        __builtin_amdgcn_wave_barrier();
+        const int i = lane & (kGroupColumns - 1), n = n0 + i;
+        const float* const from = reinterpret_cast<const float*>(xs + i * (GL + 1));
+        for (int q = lane / kGroupColumns; q < GL * 4 && b0 + q < a.B; q += 2)
+            if (n < a.N) a.gx[(size_t)(b0 + q) * a.N + n] = from[q];
     }
 }
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
+// Weights into the order of the plan's entries, and weight gradients from it: a workgroup takes a tile of consecutive flat positions
+// through LDS, so that memory sees them as they lie on this side, and runs of a stream's neighbouring entries on the other.
+// (Weight gradients of `slices` slices that were formed side by side are summed, in their order.)
+// Consecutive tiles go to one XCD, whose L2 gathers what several of them write to a line.
+constexpr int kTileMoveThreads = 1024, kTileMoveAhead = 8;
 
-// slot_w[slot] = the weight of the slot's connection (0 in padding).  Slots are dealt to the XCDs in eight consecutive
-// ranges: an XCD reads the weights of one label block after the other, which its L2 holds.
-__global__ __launch_bounds__(256) void slot_weights_kernel(const float* __restrict__ w, const int32_t* __restrict__ slot_pos,
-                                                           float* __restrict__ slot_w, size_t slots, int units) {
-    const int u = xcd_unit(blockIdx.x, units);
-    if (u < 0) return;
-    const size_t q = (size_t)u * 256 + threadIdx.x;
-    if (q * 4 >= slots) return;
-    // (what is touched once goes past the L2, which the gathered array needs: 395 -> 369 us at 670,091 labels x fan-in 72)
-    const v4i at = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(slot_pos) + q);
-    v4f v;
-    v.x = w[max(at.x, 0)]; v.y = w[max(at.y, 0)]; v.z = w[max(at.z, 0)]; v.w = w[max(at.w, 0)];
-    if (at.x < 0) v.x = 0.f;
-    if (at.y < 0) v.y = 0.f;
-    if (at.z < 0) v.z = 0.f;
-    if (at.w < 0) v.w = 0.f;
-    __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(slot_w) + q);
+__global__ __launch_bounds__(kTileMoveThreads) void weights_to_slots_kernel(const float* __restrict__ w, const unsigned short* __restrict__ tile_pos,
+                                                                            const unsigned* __restrict__ slot_of, float* __restrict__ slot_w,
+                                                                            size_t total, int tile_bits, int tiles) {
+    extern __shared__ __align__(16) float tile_mem[];
+    const int t = xcd_unit(blockIdx.x, tiles);
+    if (t < 0) return;
+    const size_t p0 = (size_t)t << tile_bits;
+    const int n = (int)min((size_t)1 << tile_bits, total - p0);
+    unsigned at[kTileMoveAhead], slot[kTileMoveAhead];
+    auto places = [&](int i) {
+#pragma unroll
+        for (int q = 0; q < kTileMoveAhead; ++q) {
+            const size_t e = p0 + min(i + q * kTileMoveThreads, n - 1);
+            at[q] = __builtin_nontemporal_load(tile_pos + e);
+            slot[q] = __builtin_nontemporal_load(slot_of + e);
+        }
+    };
+    places(threadIdx.x);
+    for (int i = 4 * threadIdx.x; i + 4 <= n; i += 4 * kTileMoveThreads) {
+        const f32x4_any q = *reinterpret_cast<const f32x4_any*>(w + p0 + i);
+        *reinterpret_cast<float4*>(tile_mem + i) = make_float4(q.x, q.y, q.z, q.w);
+    }
+    for (int i = (n & ~3) + (int)threadIdx.x; i < n; i += kTileMoveThreads) tile_mem[i] = w[p0 + i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kTileMoveThreads * kTileMoveAhead) {
+#pragma unroll
+        for (int q = 0; q < kTileMoveAhead; ++q)
+            if (i + q * kTileMoveThreads < n) slot_w[slot[q]] = tile_mem[at[q]];
+        places(i + kTileMoveThreads * kTileMoveAhead);
+    }
 }
 
-// gw[pos] = gw_slots[pos_slot[pos]]; positions are dealt to the XCDs like the slots above.  (Reads at random places: the same
-// permutation as scattered writes, from the slots' side, took twice as long.)
-__global__ __launch_bounds__(256) void weight_grads_in_place_kernel(const float* __restrict__ gw_slots, const unsigned* __restrict__ pos_slot,
-                                                                    float* __restrict__ gw, size_t count, int units) {
-    const int u = xcd_unit(blockIdx.x, units);
-    if (u < 0) return;
-    const size_t p0 = ((size_t)u * 256 + threadIdx.x / 64 * 64) * 4 + (threadIdx.x & 63);
-    float v[4];
+__global__ __launch_bounds__(kTileMoveThreads) void weight_grads_from_slots_kernel(const float* __restrict__ gw_slots, const unsigned short* __restrict__ tile_pos,
+                                                                                   const unsigned* __restrict__ slot_of, float* __restrict__ gw,
+                                                                                   size_t total, int tile_bits, int tiles, int slices, size_t slots) {
+    extern __shared__ __align__(16) float tile_mem[];
+    const int t = xcd_unit(blockIdx.x, tiles);
+    if (t < 0) return;
+    const size_t p0 = (size_t)t << tile_bits;
+    const int n = (int)min((size_t)1 << tile_bits, total - p0);
+    for (int i = threadIdx.x; i < n; i += kTileMoveThreads * kTileMoveAhead) {
+        unsigned at[kTileMoveAhead], slot[kTileMoveAhead];
+        float v[kTileMoveAhead];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = gw_slots[__builtin_nontemporal_load(pos_slot + min(p0 + 64 * i, count - 1))];
+        for (int q = 0; q < kTileMoveAhead; ++q) {
+            const size_t e = p0 + min(i + q * kTileMoveThreads, n - 1);
+            at[q] = __builtin_nontemporal_load(tile_pos + e);
+            slot[q] = __builtin_nontemporal_load(slot_of + e);
+        }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (p0 + 64 * i < count) __builtin_nontemporal_store(v[i], gw + p0 + 64 * i);
+        for (int q = 0; q < kTileMoveAhead; ++q) v[q] = gw_slots[slot[q]];
+        for (int t = 1; t < slices; ++t) {
+#pragma unroll
+            for (int q = 0; q < kTileMoveAhead; ++q) v[q] += gw_slots[t * slots + slot[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < kTileMoveAhead; ++q) tile_mem[at[q]] = v[q];    // (behind the end: the last one once more)
+    }
+    __syncthreads();
+    for (int i = 4 * threadIdx.x; i + 4 <= n; i += 4 * kTileMoveThreads) {
+        const float4 q = *reinterpret_cast<const float4*>(tile_mem + i);
+        f32x4_any o;
+        o.x = q.x; o.y = q.y; o.z = q.z; o.w = q.w;
+        *reinterpret_cast<f32x4_any*>(gw + p0 + i) = o;
+    }
+    for (int i = (n & ~3) + (int)threadIdx.x; i < n; i += kTileMoveThreads) gw[p0 + i] = tile_mem[i];
 }
 
-// gx ([N,B] or [B,N]) = sum over the streams of part[slice][stream][n][sl], ascending; 32 columns x 32 samples per workgroup
+// gx ([N,B] or [B,N]) = sum over the segments of part[slice][segment][n][sl], in a fixed order; 32 columns x 32 samples per workgroup
 template <bool TP>
 __global__ __launch_bounds__(256) void gather_gx_kernel(const float* __restrict__ part, float* __restrict__ gx, int N, int B, int sl,
-                                                        int streams) {
+                                                        int segments) {
     __shared__ float tile[32][33];
     const int n0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     for (int i = ty; i < 32; i += 8) {
         const int n = n0 + i, b = b0 + tx;
         float v = 0.f;
-        if (n < N && b < B)
-            for (int t = 0; t < streams; ++t) v += part[(((size_t)(b / sl) * streams + t) * N + n) * sl + b % sl];
+        if (n < N && b < B) {
+            // (eight sums side by side: loads in flight, and a shorter chain of roundings)
+            const float* const from = part + ((size_t)(b / sl) * segments * N + n) * sl + b % sl;
+            float q[8] = {};
+            for (int t = 0; t < segments; t += 8)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (t + e < segments) q[e] += from[(size_t)(t + e) * N * sl];
+            v = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+        }
         if (TP) {
             if (n < N && b < B) gx[(size_t)n * B + b] = v;
         } else {
@@ -381,32 +515,12 @@ __global__ __launch_bounds__(256) void column_sums_kernel(const float* __restric
     if (ty == 0 && j < L) bias_grad[j] = ((part[0][tx] + part[1][tx]) + part[2][tx]) + part[3][tx];
 }
 
-struct WalkArgs {
-    const float *gtab, *xtab, *slot_w;
-    float *gx_part, *gw_slots;
-    bool add_gw;
-    int streams, blocks_per_stream;
-};
-
 template <int GL, bool DOT>
-int launch_walk(int m, const ffi_plan* p, const WalkArgs& a, hipStream_t s) {
-    const int wg_cols = kWalkThreads / 64 * m * (64 / GL), col_chunks = (p->N + wg_cols - 1) / wg_cols;
-    const int units = col_chunks * a.streams;
-    const size_t lds = (size_t)(kWalkThreads / 64) * (64 / GL * walk_stride(GL) + 64 * m) * sizeof(uint4);
-    FFI_HIP_TRY(hipFuncSetAttribute((const void*)walk_columns_kernel<GL, DOT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((walk_columns_kernel<GL, DOT>), dim3(xcd_grid(units)), dim3(kWalkThreads), lds, s, a.gtab, a.xtab, p->oct_ptr,
-                       p->slot_lab, a.slot_w, a.gx_part, a.gw_slots, a.add_gw ? 1 : 0, (size_t)p->slots, p->N, p->L, p->nblocks,
-                       p->block_labels, a.blocks_per_stream, col_chunks, units, m);
+int launch_walk(const WalkArgs& a, hipStream_t s) {
+    const int workgroups = (a.units * a.slices + kWalkWaves - 1) / kWalkWaves;
+    hipLaunchKernelGGL((walk_columns_kernel<GL, DOT>), dim3(xcd_grid(workgroups)), dim3(kWalkWaves * 64), 0, s, a);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
-}
-
-template <bool DOT>
-int launch_walk_gl(int gl, int m, const ffi_plan* p, const WalkArgs& a, hipStream_t s) {
-    if (gl == 1) return launch_walk<1, DOT>(m, p, a, s);
-    if (gl == 2) return launch_walk<2, DOT>(m, p, a, s);
-    if (gl == 4) return launch_walk<4, DOT>(m, p, a, s);
-    return launch_walk<8, DOT>(m, p, a, s);
 }
 
 }  // namespace
@@ -458,66 +572,53 @@ int launch_weight_grad_wide(const float* x, const int32_t* idx, const float* g, 
     return FFI_OK;
 }
 
-// How the walk is cut: columns per lane group (m) and streams of label blocks, so that about 16 wavefronts per CU are in
-// flight: as many columns per group as that allows (a walk of all blocks each), else several streams whose sums are added.
-void walk_shape(int N, int B, int L, int nblocks, int* gl, int* slices, int* m, int* streams, int* blocks_per_stream) {
-    *gl = slice_lanes(B, 4);
-    *slices = (B + *gl * 4 - 1) / (*gl * 4);
-    const long long target = device_cu_count();                             // workgroups
-    const int group_cols = kWalkThreads / *gl;                              // columns per workgroup and m
-    *m = kWalkMaxM;
-    while (*m > 1 && (long long)(N + group_cols * *m - 1) / (group_cols * *m) < target) *m /= 2;
-    const long long wgs = (N + group_cols * *m - 1) / (group_cols * *m);
-    const int want = (int)std::min<long long>(nblocks, std::max<long long>(1, target / wgs));
-    *blocks_per_stream = (nblocks + want - 1) / want;
-    *streams = (nblocks + *blocks_per_stream - 1) / *blocks_per_stream;
+// Slices that one launch walks: as many as the CUs hold wavefronts for.
+int walk_slices(long long units, int slices) {
+    return (int)std::max<long long>(1, std::min<long long>(slices, (long long)kWalkWaves * device_cu_count() / units));
 }
 
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
                          bool tp, hipStream_t s) {
-    if (!p->oct_ptr || !p->slot_pos || !p->slot_lab) return FFI_ERR_BAD_ARGUMENT;
+    if (!p->entries || !p->slot_of || !p->tile_pos || !p->chunk_ptr) return FFI_ERR_BAD_ARGUMENT;
     // (before anything is enqueued: a refused call leaves its outputs alone)
+    if ((long long)p->segments * p->groups * ((B + 31) / 32) >= (1ll << 31)) return FFI_ERR_TOO_LARGE;
     const dim3 gx_grid((unsigned)((p->N + 31) / 32), (unsigned)(((long long)B + 31) / 32));
     if (gx_grid.y > 65535u) return FFI_ERR_TOO_LARGE;
     const bool dot = gw != nullptr;
-    int gl, slices, m;
-    WalkArgs a{};
-    walk_shape(p->N, B, p->L, p->nblocks, &gl, &slices, &m, &a.streams, &a.blocks_per_stream);
-    const int sl = gl * 4;
-    const size_t slots = (size_t)p->slots, count = (size_t)p->L * p->K, gslice = (size_t)p->L * sl, part = (size_t)p->N * sl * a.streams;
-    float* ws = nullptr;
+    const int sl = 256 / p->members, slices = (B + sl - 1) / sl, units = p->segments * p->groups, at_once = walk_slices(units, slices);
+    const size_t slots = (size_t)p->slots, count = (size_t)p->L * p->K, gslice = (size_t)p->L * sl, part = p->segments > 1 ? (size_t)p->N * sl * p->segments : 0;
+    float *ws = nullptr, *slot_w = nullptr, *gw_slots = nullptr;
     FFI_TRY(workspace_get(s, kWsPartials, (gslice + part) * slices * sizeof(float), (void**)&ws));
-    float* slot_w = nullptr;
     FFI_TRY(workspace_get(s, kWsSlots, slots * sizeof(float), (void**)&slot_w));
+    if (dot) FFI_TRY(workspace_get(s, kWsWeightParts, slots * at_once * sizeof(float), (void**)&gw_slots));
     FFI_TRY(launch_slices_f32(g, ws, p->L, B, sl, false, s));
     float* const parts = ws + gslice * slices;
-    float* xtab = nullptr;
-    if (dot) {
-        FFI_TRY(workspace_get(s, kWsFeaturesT, (size_t)p->N * sl * slices * sizeof(float), (void**)&xtab));
-        FFI_TRY(launch_slices_f32(x, xtab, p->N, B, sl, tp, s));
-        FFI_TRY(workspace_get(s, kWsWeightParts, slots * sizeof(float), (void**)&a.gw_slots));
-    }
-    const int slot_units = (int)((slots / 4 + 255) / 256);
-    hipLaunchKernelGGL(slot_weights_kernel, dim3(xcd_grid(slot_units)), dim3(256), 0, s, w, p->slot_pos, slot_w, slots, slot_units);
+    const int tiles = (int)((count + ((size_t)1 << p->tile_bits) - 1) >> p->tile_bits);
+    const size_t tile_bytes = sizeof(float) << p->tile_bits;
+    for (const void* k : {(const void*)weights_to_slots_kernel, (const void*)weight_grads_from_slots_kernel})
+        FFI_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile_bytes));
+    hipLaunchKernelGGL(weights_to_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, w, p->tile_pos, p->slot_of, slot_w, count,
+                       p->tile_bits, tiles);
     FFI_HIP_TRY(hipGetLastError());
-    // one slice after the other: their weight gradients add up in place
-    a.slot_w = slot_w;
-    for (int q = 0; q < slices; ++q) {
-        a.gtab = ws + gslice * q; a.gx_part = parts + part * q; a.add_gw = q > 0;
-        a.xtab = dot ? xtab + (size_t)p->N * sl * q : nullptr;
-        FFI_TRY(dot ? launch_walk_gl<true>(gl, m, p, a, s) : launch_walk_gl<false>(gl, m, p, a, s));
+    // one launch after the other: their weight gradients add up in place
+    for (int q = 0; q < slices; q += at_once) {
+        const WalkArgs a{ws, x, slot_w, p->entries, p->chunk_ptr, p->chunk_count, gx, parts, gw_slots, gslice, part, slots, q, std::min(at_once, slices - q),
+                         q > 0 ? 1 : 0, B, p->N, p->L, units, p->groups, p->segments, p->seg_labels, tp};
+        if (p->members == 4) FFI_TRY((dot ? launch_walk<16, true>(a, s) : launch_walk<16, false>(a, s)));
+        else FFI_TRY((dot ? launch_walk<8, true>(a, s) : launch_walk<8, false>(a, s)));
     }
     if (dot) {
-        const int units = (int)((count + 1023) / 1024);
-        hipLaunchKernelGGL(weight_grads_in_place_kernel, dim3(xcd_grid(units)), dim3(256), 0, s, a.gw_slots, p->pos_slot, gw, count, units);
+        hipLaunchKernelGGL(weight_grads_from_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, gw_slots, p->tile_pos, p->slot_of,
+                           gw, count, p->tile_bits, tiles, at_once, slots);
         FFI_HIP_TRY(hipGetLastError());
     }
     if (bias_grad != nullptr) {
         hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((p->L + 63) / 64)), dim3(256), 0, s, g, bias_grad, B, p->L);
         FFI_HIP_TRY(hipGetLastError());
     }
-    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
-    else hipLaunchKernelGGL(gather_gx_kernel<false>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, a.streams);
+    if (p->segments == 1) return FFI_OK;
+    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, p->segments);
+    else hipLaunchKernelGGL(gather_gx_kernel<false>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, p->segments);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }

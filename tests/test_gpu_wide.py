@@ -82,8 +82,7 @@ def test_forward_in_phases(ffi, spread):
         lib.ffi_set_option(b"wide_phases", 0)
 
 
-# (B, N, L, K): lane groups of 1, 2, 4 and 8; lists that are empty, shorter and longer than a window; several label blocks,
-# streams and slices; one column
+# (B, N, L, K): streams that are empty, shorter and longer than a chunk; several segments, streams and slices; one column
 BACKWARD_SHAPES = [(1, 1217, 900, 3), (4, 2000, 30_000, 9), (5, 1217, 129, 17), (8, 3000, 3000, 40), (9, 1300, 65, 33), (16, 2500, 5000, 64),
                    (17, 40_000, 63, 3), (33, 1300, 9000, 72), (100, 40_000, 200, 65), (130, 1500, 97, 130), (64, 30_000, 3000, 36)]
 
@@ -167,8 +166,7 @@ def test_forward_from_slices_of_eight_samples(ffi, B, N, L, K):
     test_forward_from_slices_in_lds_shares(ffi, False, B, N, L, K)
 
 
-# Wide inputs with few columns and few labels: more blocks than labels fill, lists of few connections, a last block of one label;
-# many blocks whose sums are added
+# Wide inputs with few columns and few labels: columns of few connections, segments whose sums are added
 @pytest.mark.parametrize("B,N,L,K", [(5, 1_217, 130, 3), (33, 1_242, 3_201, 95), (64, 5_000, 129, 40), (17, 2_000, 13_331, 8), (3, 20_000, 700, 16)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_backward_over_many_label_blocks(ffi, B, N, L, K, transposed):
@@ -180,6 +178,34 @@ def test_backward_over_many_label_blocks(ffi, B, N, L, K, transposed):
         gx, gw = call(xd, dev(lookup), dev(w), dev(g))
         gx = gx.t() if transposed else gx
         assert rel_err(gx.cpu().numpy(), o_gx) <= 2e-5 and rel_err(gw.cpu().numpy(), o_gw) <= 2e-5
+
+
+# The walk over streams of 32 columns: (batches of the calls in turn -- the first one's plan has steps of four or eight connections and
+# serves the others --, N, L, K).  One column behind whole groups; streams of no, one and several chunks; several segments, several
+# slices in a launch and several launches; tiles of exactly their positions and one more; more streams than the build counts at a time
+WALK_SHAPES = [((20, 70, 3), 1249, 5000, 7), ((70, 20, 200), 1248, 5000, 7), ((1, 130), 1300, 9000, 72), ((300, 33), 2500, 3001, 33),
+               ((64,), 1300, 1024, 1), ((32,), 1300, 1025, 1), ((65, 64), 40_000, 20_011, 12), ((3, 40), 1_000_000, 300, 4)]
+
+
+@pytest.mark.parametrize("shape", WALK_SHAPES, ids=str)
+def test_walk_over_streams(ffi, shape):
+    batches, N, L, K = shape
+    lib = ffi._lib.lib()
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        _, lookup, w, _ = reference_law_inputs(1, N, L, K, seed=L + K)
+        dl, dw = dev(lookup), dev(w)
+        for B in batches:
+            rng = np.random.default_rng(B)
+            x, g = rng.standard_normal((B, N), dtype=np.float32), rng.standard_normal((B, L), dtype=np.float32)
+            ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+            for tp in (False, True):
+                call = ffi.fan_in_sparse_matmul_grad_tp if tp else ffi.fan_in_sparse_matmul_grad
+                gx, gw = call(dev(x.T if tp else x), dl, dw, dev(g))
+                gx = gx.t() if tp else gx
+                assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-5, (B, tp)
+    finally:
+        lib.ffi_set_option(b"small_path", 0)
 
 
 # Up to four samples, scores and answer in one launch: fan-ins of one quad, off the quads and of several passes over a row; fewer
@@ -412,9 +438,8 @@ def test_subnormal_operands_and_sums(ffi, bf16, B, N, phases):
         lib.ffi_set_option(b"small_path", 0)
 
 
-# Plans of the global form: numbers of lists at the edges of the workgroups that count them (255 each), lists shorter than an oct,
-# of whole octs and longer, ids so uneven that the slots are far from what uniform ids would give; narrow layers too uneven for the
-# tiled form; sort keys of one, two and three digits
+# Plans of the global form: few and many streams, columns of fewer connections than a step and of many, ids so uneven that the slots are
+# far from what uniform ids would give; narrow layers too uneven for the tiled form
 @pytest.mark.parametrize("kind", ["uniform", "one column", "squared", "last column"])
 @pytest.mark.parametrize("N,L,K", [(1275, 40, 3), (1276, 2_000, 16), (1530, 9_000, 8), (1531, 30_000, 4), (70_000, 300, 2), (255, 5_000, 8), (256, 6_000, 9)])
 def test_plans_of_the_global_form(ffi, kind, N, L, K):
