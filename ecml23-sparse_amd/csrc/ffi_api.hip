@@ -145,7 +145,7 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     auto passes = [&](const LookupCheck* check) -> int {
         // (the global form's walk has both operands of a connection at hand: one walk for both gradients)
         if (!p->tiled && wg.features != nullptr)
-            return launch_backward_wide(p, wg.features, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d.B, d.tp, s);
+            return launch_backward_wide(p, wg.features, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d.B, d.tp, s, check);
         FFI_TRY(between(p));
         return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, check);
     };
@@ -179,16 +179,11 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         if (st != FFI_OK) { drop_cached_plan(p); return st; }
         return passes(nullptr);
     }
-    if (p->tiled) {
-        LookupCheck check;
-        FFI_TRY(plan_guard_begin(p, lookup, s, &check));
-        FFI_TRY(passes(&check));
-    } else {
-        FFI_TRY(plan_guard_enqueue(p, lookup, s));
-        FFI_TRY(passes(nullptr));
-    }
+    LookupCheck check;
+    FFI_TRY(plan_guard_begin(p, lookup, s, &check));
+    FFI_TRY(passes(&check));
     return launch_backward_if_outdated(p->d_guard + kGuardVerdict, wg.features, lookup, weights, out_grad, feature_grad,
-                                       wg.weight_grad, wg.bias_grad, d, s);
+                                       wg.weight_grad, wg.bias_grad, d, !p->tiled && wg.features != nullptr, s);
 }
 
 }  // namespace

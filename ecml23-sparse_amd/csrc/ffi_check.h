@@ -1,5 +1,5 @@
-// Check of a lookup's content against a plan's fingerprint, on the device: as a kernel of its own, or as workgroups of a
-// kernel that has other work too (gfx950).
+// Check of a lookup's content against a plan's fingerprint, on the device, as workgroups of a kernel that has other
+// work too (gfx950).
 #ifndef FFI_CHECK_H
 #define FFI_CHECK_H
 

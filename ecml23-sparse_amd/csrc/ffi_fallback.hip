@@ -347,7 +347,7 @@ int backward_if_outdated_prepare(const Dims& d, hipStream_t s) {
 
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,
                                 const float* weights, const float* out_grad, float* feature_grad, float* weight_grad,
-                                float* bias_grad, const Dims& d, hipStream_t s) {
+                                float* bias_grad, const Dims& d, bool zeroed, hipStream_t s) {
     const int cus = device_cu_count();
     float* gw = features != nullptr ? weight_grad : nullptr;
     float* gb = features != nullptr ? bias_grad : nullptr;
@@ -368,7 +368,7 @@ int launch_backward_if_outdated(const unsigned long long* verdict, const float* 
         FFI_HIP_TRY(hipGetLastError());
         return FFI_OK;
     }
-    if (feature_grad != nullptr) {
+    if (feature_grad != nullptr && !zeroed) {
         hipLaunchKernelGGL(fallback_zero_kernel, dim3(cus), dim3(kFbBlock), 0, s, verdict, feature_grad, (size_t)d.B * d.N);
         FFI_HIP_TRY(hipGetLastError());
     }

@@ -456,7 +456,7 @@ int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* 
         }
         return FFI_OK;
     }
-    return launch_backward_wide(p, nullptr, w, g, gx, nullptr, nullptr, B, tp, s);
+    return launch_backward_wide(p, nullptr, w, g, gx, nullptr, nullptr, B, tp, s, check);
 }
 
 }  // namespace ffi

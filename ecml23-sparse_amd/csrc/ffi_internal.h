@@ -422,8 +422,6 @@ int plan_fingerprint(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigned
 int plan_scratch_alloc(ffi_plan* p);
 // Makes a plan that nothing uses any more one of another lookup, to be built: its buffers serve the build where they fit.
 void plan_reuse(ffi_plan* p, int L, int K, int N);
-// Enqueues a check of `lookup` against the plan's fingerprint on `s`: the verdict lands in p->d_guard[kGuardVerdict]
-// (device) for the kernels enqueued behind it, and in the pinned mirror for a later call of the host.
 constexpr int kGuardVerdict = 4;
 constexpr int kCheckThreads = 1024;
 constexpr int kCheckBlocks = 256;                  // workgroups of a check (at most)
@@ -435,8 +433,9 @@ struct LookupCheck {                               // (ffi_check.h)
     int blocks;
     unsigned long long *guard, *host_mirror, seq;
 };
-int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s);
-// The same without the launch: for a kernel on `s` that has check.blocks workgroups of kCheckThreads threads run it.
+// A check of `lookup` against the plan's fingerprint, for a kernel on `s` that has check.blocks workgroups of kCheckThreads threads run
+// it: the verdict lands in p->d_guard[kGuardVerdict] (device) for the kernels enqueued behind that one, and in the pinned mirror for a
+// later call of the host.
 int plan_guard_begin(ffi_plan* p, const int32_t* lookup, hipStream_t s, LookupCheck* check);
 // What the last finished check found, if the host has not seen it yet: *seen = false when no check has finished
 // since the last poll.  Never waits.
@@ -447,17 +446,19 @@ int plan_guard_poll(ffi_plan* p, bool* seen, bool* current, unsigned long long* 
 // allocated by backward_if_outdated_prepare, ahead of the first kernel of the call.
 size_t backward_if_outdated_workspace(const Dims& d);
 int backward_if_outdated_prepare(const Dims& d, hipStream_t s);
+// (`zeroed`: where the verdict is 0 feature_grad is zero already)
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,
                                 const float* weights, const float* out_grad, float* feature_grad, float* weight_grad,
-                                float* bias_grad, const Dims& d, hipStream_t s);
+                                float* bias_grad, const Dims& d, bool zeroed, hipStream_t s);
 void plan_free(ffi_plan* p);
-// `check` (may be null; tiled form only): run by the last kernel, beside its own work
+// `check` (may be null): run by a kernel of the pass beside its own work
 int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp,
                       hipStream_t s, const LookupCheck* check = nullptr);
-// Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.
+// Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.  With a
+// check and gw, gx is zero where the check has found the plan outdated.
 int walk_slices(long long units, int slices);
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
-                         bool tp, hipStream_t s);
+                         bool tp, hipStream_t s, const LookupCheck* check);
 }  // namespace ffi
 
 #endif  // FFI_INTERNAL_H

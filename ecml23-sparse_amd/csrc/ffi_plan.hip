@@ -72,11 +72,6 @@ __global__ __launch_bounds__(64) void guard_init_kernel(unsigned long long* __re
     if (i < 8) guard[i] = i == 3 || i == 5 ? fingerprint : i == 4 ? 1ull : 0ull;
 }
 
-__global__ __launch_bounds__(kCheckThreads) void fingerprint_guard_kernel(const LookupCheck check) {
-    __shared__ CheckShared shared;
-    check_block(check, blockIdx.x, shared);
-}
-
 // ---- tiled form ---------------------------------------------------------------------------------
 
 // Order of a column's slots inside a tile.  The kernel that walks the plan reads, per slot, the
@@ -1584,14 +1579,6 @@ int plan_guard_begin(ffi_plan* p, const int32_t* lookup, hipStream_t s, LookupCh
                          p->d_guard, mirror, p->guard_seq + 1};
     p->guard_seq += 1;
     p->guard_stream = s;
-    return FFI_OK;
-}
-
-int plan_guard_enqueue(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
-    LookupCheck check;
-    FFI_TRY(plan_guard_begin(p, lookup, s, &check));
-    hipLaunchKernelGGL(fingerprint_guard_kernel, dim3((unsigned)check.blocks), dim3(kCheckThreads), 0, s, check);
-    FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 

@@ -3,6 +3,7 @@
 // of slices of out_grad (ffi_sliced.h), all at about the same labels at a time; and the weight gradient alone, straight from the
 // lookup, whose gathers of whole rows of the batch-major features come through the cache hierarchy.
 #include "ffi_internal.h"
+#include "ffi_check.h"
 #include "ffi_lds_tile.h"
 #include "ffi_sliced.h"
 
@@ -398,13 +399,23 @@ __global__ __launch_bounds__(kWalkWaves * 64) void walk_columns_kernel(const Wal
 // through LDS, so that memory sees them as they lie on this side, and runs of a stream's neighbouring entries on the other.
 // (Weight gradients of `slices` slices that were formed side by side are summed, in their order.)
 // Consecutive tiles go to one XCD, whose L2 gathers what several of them write to a line.
-constexpr int kTileMoveThreads = 1024, kTileMoveAhead = 8;
+//
+// The first check.blocks workgroups of the one check the lookup's content against the plan instead (ffi_check.h); where that found the plan
+// outdated, the other clears gx for the kernel that then forms the gradients anew.  (As kernels of their own the two were 9 of the 50 to 60
+// us of a backward pass of few connections, and the check 40 of 3,250 at 65,536 columns x 670,091 labels x 72.)
+constexpr int kTileMoveThreads = kCheckThreads, kTileMoveAhead = 8;
 
 __global__ __launch_bounds__(kTileMoveThreads) void weights_to_slots_kernel(const float* __restrict__ w, const unsigned short* __restrict__ tile_pos,
                                                                             const unsigned* __restrict__ slot_of, float* __restrict__ slot_w,
-                                                                            size_t total, int tile_bits, int tiles) {
+                                                                            size_t total, int tile_bits, int tiles, const LookupCheck check) {
     extern __shared__ __align__(16) float tile_mem[];
-    const int t = xcd_unit(blockIdx.x, tiles);
+    __shared__ CheckShared check_shared;
+    const int checks = (check.blocks + kXcds - 1) / kXcds * kXcds;
+    if ((int)blockIdx.x < checks) {
+        if ((int)blockIdx.x < check.blocks) check_block(check, blockIdx.x, check_shared);
+        return;
+    }
+    const int t = xcd_unit(blockIdx.x - checks, tiles);
     if (t < 0) return;
     const size_t p0 = (size_t)t << tile_bits;
     const int n = (int)min((size_t)1 << tile_bits, total - p0);
@@ -434,8 +445,11 @@ __global__ __launch_bounds__(kTileMoveThreads) void weights_to_slots_kernel(cons
 
 __global__ __launch_bounds__(kTileMoveThreads) void weight_grads_from_slots_kernel(const float* __restrict__ gw_slots, const unsigned short* __restrict__ tile_pos,
                                                                                    const unsigned* __restrict__ slot_of, float* __restrict__ gw,
-                                                                                   size_t total, int tile_bits, int tiles, int slices, size_t slots) {
+                                                                                   size_t total, int tile_bits, int tiles, int slices, size_t slots,
+                                                                                   const unsigned long long* __restrict__ verdict, float* __restrict__ gx, size_t gx_count) {
     extern __shared__ __align__(16) float tile_mem[];
+    if (verdict != nullptr && *verdict == 0)
+        for (size_t i = (size_t)blockIdx.x * kTileMoveThreads + threadIdx.x; i < gx_count; i += (size_t)gridDim.x * kTileMoveThreads) gx[i] = 0.f;
     const int t = xcd_unit(blockIdx.x, tiles);
     if (t < 0) return;
     const size_t p0 = (size_t)t << tile_bits;
@@ -468,38 +482,36 @@ __global__ __launch_bounds__(kTileMoveThreads) void weight_grads_from_slots_kern
     for (int i = (n & ~3) + (int)threadIdx.x; i < n; i += kTileMoveThreads) gw[p0 + i] = tile_mem[i];
 }
 
-// gx ([N,B] or [B,N]) = sum over the segments of part[slice][segment][n][sl], in a fixed order; 32 columns x 32 samples per workgroup
+// gx ([N,B] or [B,N]) = sum over the segments of part[slice][segment][n][sl], in a fixed order; 32 columns x 32 samples per workgroup, one
+// sum per thread (four: 22.8 us for 3,178 columns x 32 samples of 20 segments, 4.8 so)
 template <bool TP>
-__global__ __launch_bounds__(256) void gather_gx_kernel(const float* __restrict__ part, float* __restrict__ gx, int N, int B, int sl,
-                                                        int segments) {
+__global__ __launch_bounds__(1024) void gather_gx_kernel(const float* __restrict__ part, float* __restrict__ gx, int N, int B, int sl,
+                                                         int segments) {
     __shared__ float tile[32][33];
     const int n0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int i = ty; i < 32; i += 8) {
-        const int n = n0 + i, b = b0 + tx;
-        float v = 0.f;
-        if (n < N && b < B) {
-            // (eight sums side by side: loads in flight, and a shorter chain of roundings)
-            const float* const from = part + ((size_t)(b / sl) * segments * N + n) * sl + b % sl;
-            float q[8] = {};
-            for (int t = 0; t < segments; t += 8)
+    {
+        const int n = min(n0 + ty, N - 1), b = min(b0 + tx, B - 1);
+        // (eight sums side by side: loads in flight, and a shorter chain of roundings)
+        const float* const from = part + ((size_t)(b / sl) * segments * N + n) * sl + b % sl;
+        float q[8] = {};
+        for (int t = 0; t < segments; t += 8) {
+            float v[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (t + e < segments) q[e] += from[(size_t)(t + e) * N * sl];
-            v = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+            for (int e = 0; e < 8; ++e) v[e] = from[(size_t)min(t + e, segments - 1) * N * sl];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] += t + e < segments ? v[e] : 0.f;
         }
+        const float v = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
         if (TP) {
-            if (n < N && b < B) gx[(size_t)n * B + b] = v;
-        } else {
-            tile[i][tx] = v;
+            if (n0 + ty < N && b0 + tx < B) gx[(size_t)n * B + b] = v;
+            return;
         }
+        tile[ty][tx] = v;
     }
-    if (TP) return;
     __syncthreads();
-    for (int i = ty; i < 32; i += 8) {
-        const int n = n0 + tx, b = b0 + i;
-        if (n < N && b < B) gx[(size_t)b * N + n] = tile[tx][i];
-    }
+    const int n = n0 + tx, b = b0 + ty;
+    if (n < N && b < B) gx[(size_t)b * N + n] = tile[tx][ty];
 }
 
 // bias_grad[j] = sum over the samples of g[b, j]: 64 labels per workgroup, four partial sums added in order
@@ -578,7 +590,7 @@ int walk_slices(long long units, int slices) {
 }
 
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
-                         bool tp, hipStream_t s) {
+                         bool tp, hipStream_t s, const LookupCheck* check) {
     if (!p->entries || !p->slot_of || !p->tile_pos || !p->chunk_ptr) return FFI_ERR_BAD_ARGUMENT;
     // (before anything is enqueued: a refused call leaves its outputs alone)
     if ((long long)p->segments * p->groups * ((B + 31) / 32) >= (1ll << 31)) return FFI_ERR_TOO_LARGE;
@@ -597,8 +609,9 @@ int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, cons
     const size_t tile_bytes = sizeof(float) << p->tile_bits;
     for (const void* k : {(const void*)weights_to_slots_kernel, (const void*)weight_grads_from_slots_kernel})
         FFI_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile_bytes));
-    hipLaunchKernelGGL(weights_to_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, w, p->tile_pos, p->slot_of, slot_w, count,
-                       p->tile_bits, tiles);
+    const LookupCheck with = check != nullptr ? *check : LookupCheck{};
+    hipLaunchKernelGGL(weights_to_slots_kernel, dim3(xcd_grid(with.blocks) + xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, w, p->tile_pos,
+                       p->slot_of, slot_w, count, p->tile_bits, tiles, with);
     FFI_HIP_TRY(hipGetLastError());
     // one launch after the other: their weight gradients add up in place
     for (int q = 0; q < slices; q += at_once) {
@@ -607,19 +620,21 @@ int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, cons
         if (p->members == 4) FFI_TRY((dot ? launch_walk<16, true>(a, s) : launch_walk<16, false>(a, s)));
         else FFI_TRY((dot ? launch_walk<8, true>(a, s) : launch_walk<8, false>(a, s)));
     }
-    if (dot) {
-        hipLaunchKernelGGL(weight_grads_from_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, gw_slots, p->tile_pos, p->slot_of,
-                           gw, count, p->tile_bits, tiles, at_once, slots);
-        FFI_HIP_TRY(hipGetLastError());
-    }
     if (bias_grad != nullptr) {
         hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((p->L + 63) / 64)), dim3(256), 0, s, g, bias_grad, B, p->L);
         FFI_HIP_TRY(hipGetLastError());
     }
-    if (p->segments == 1) return FFI_OK;
-    if (tp) hipLaunchKernelGGL(gather_gx_kernel<true>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, p->segments);
-    else hipLaunchKernelGGL(gather_gx_kernel<false>, gx_grid, dim3(256), 0, s, parts, gx, p->N, B, sl, p->segments);
-    FFI_HIP_TRY(hipGetLastError());
+    if (p->segments > 1) {
+        const auto gather_gx = tp ? gather_gx_kernel<true> : gather_gx_kernel<false>;
+        hipLaunchKernelGGL(gather_gx, gx_grid, dim3(1024), 0, s, parts, gx, p->N, B, sl, p->segments);
+        FFI_HIP_TRY(hipGetLastError());
+    }
+    // (last: it clears gx behind an outdated plan)
+    if (dot) {
+        hipLaunchKernelGGL(weight_grads_from_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, gw_slots, p->tile_pos, p->slot_of,
+                           gw, count, p->tile_bits, tiles, at_once, slots, check != nullptr ? check->guard + kGuardVerdict : nullptr, gx, (size_t)p->N * B);
+        FFI_HIP_TRY(hipGetLastError());
+    }
     return FFI_OK;
 }
 

@@ -208,6 +208,40 @@ def test_walk_over_streams(ffi, shape):
         lib.ffi_set_option(b"small_path", 0)
 
 
+# Behind an outdated plan of the global form: gx is cleared by the kernel that moves the weight gradients, or, without them, by one of its
+# own; one segment and several, more and less of gx than workgroups have threads
+@pytest.mark.parametrize("shape", [(33, 1300, 3000, 9), (70, 40_000, 2000, 5)], ids=str)
+@pytest.mark.parametrize("input_only", [False, True])
+def test_wide_gradients_behind_an_outdated_plan(ffi, shape, input_only):
+    B, N, L, K = shape
+    lib = ffi._lib.lib()
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B + K)
+    dx, dl, dw, dg = dev(x), dev(lookup), dev(w), dev(g)
+
+    def call():
+        if not input_only:
+            return ffi.fan_in_sparse_matmul_grad(dx, dl, dw, dg)
+        gx = torch.full((B, N), float("nan"), device="cuda")
+        ffi._lib.check(lib.ffi_input_grad_f32(dl.data_ptr(), dw.data_ptr(), dg.data_ptr(), gx.data_ptr(), B, N, L, K, 0,
+                                              torch.cuda.current_stream().cuda_stream))
+        return gx, None
+
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        call()
+        rng = np.random.default_rng(8)
+        for _ in range(2):
+            lookup = lookup.copy()
+            lookup[rng.integers(0, L, 400), rng.integers(0, K, 400)] = rng.integers(0, N, 400)
+            dl.copy_(dev(lookup))
+            gx, gw = call()
+            ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4
+            assert gw is None or rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4
+    finally:
+        lib.ffi_set_option(b"small_path", 0)
+
+
 # Up to four samples, scores and answer in one launch: fan-ins of one quad, off the quads and of several passes over a row; fewer
 # labels than asked for, a label per lane and four, more workgroups than CUs; features that just fit
 @pytest.mark.parametrize("bf16", [False, True])
