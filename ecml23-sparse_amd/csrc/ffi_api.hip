@@ -68,8 +68,8 @@ ffi_plan* find_cached_plan(const int32_t* lookup, const Dims& d, int dev) {
     return nullptr;
 }
 
-// Builds a plan for a lookup that has none and adds it to the cache.  Caller holds g_cache_mutex.
-int create_cached_plan(const int32_t* lookup, const Dims& d, int dev, hipStream_t s, ffi_plan** out) {
+// Builds a plan for a lookup that has none (`ids_only`: only checks its ids) and adds it to the cache.  Caller holds g_cache_mutex.
+int create_cached_plan(const int32_t* lookup, const Dims& d, int dev, bool ids_only, hipStream_t s, ffi_plan** out) {
     ffi_plan* p = nullptr;
     if (g_cache.size() >= kMaxCachedPlans) {
         // the least recently used plan of this device makes room, and hands on its buffers (a program that goes from lookup to
@@ -86,7 +86,7 @@ int create_cached_plan(const int32_t* lookup, const Dims& d, int dev, hipStream_
     }
     if (p == nullptr) FFI_TRY(plan_alloc(d.L, d.K, d.N, &p));
     p->batch_hint = d.B;
-    int st = plan_build(p, lookup, s);
+    int st = ids_only ? plan_check_ids(p, lookup, s) : plan_build(p, lookup, s);
     if (st != FFI_OK) { plan_free(p); delete p; return st; }
     g_cache.push_back(p);
     *out = p;
@@ -149,7 +149,9 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         FFI_TRY(between(p));
         return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, check);
     };
-    // small layers read the lookup itself: of the plan they need that its build has found every id in range
+    // small layers read the lookup itself: of a plan they need only that every id was found in range, so none is laid out for them.
+    // (A rewiring and the pass behind it with a plan built for its check of the ids and without: 22 x 1,198 x 12,291 x 7 627 -> 206 us,
+    // 17 x 64 x 10,000 x 4 301 -> 208.)
     const bool small = takes_small_backward(d);
     auto small_pass = [&]() -> int {
         unsigned long long* bad = nullptr;
@@ -159,12 +161,12 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     };
     if (!small) FFI_TRY(backward_if_outdated_prepare(d, s));
     if (!p) {
-        FFI_TRY(create_cached_plan(lookup, d, dev, s, &p));
+        FFI_TRY(create_cached_plan(lookup, d, dev, small, s, &p));
         return small ? small_pass() : passes(nullptr);
     }
     if (small) {
         if (p->edited_by_library || __atomic_exchange_n(p->h_guard + kGuardHostBadIds, 0ull, __ATOMIC_ACQ_REL) != 0) {
-            const int st = plan_build(p, lookup, s);
+            const int st = plan_check_ids(p, lookup, s);
             if (st != FFI_OK) { drop_cached_plan(p); return st; }
         }
         return small_pass();
@@ -172,8 +174,9 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     bool seen = false, current = true;
     unsigned long long bad = 0;
     FFI_TRY(plan_guard_poll(p, &seen, &current, &bad));
-    if (p->edited_by_library || (seen && !current)) {
-        // the lookup changed under the plan (the calls since then were served by the recomputing kernels);
+    if (p->ids_only || p->edited_by_library || (seen && !current)) {
+        // the lookup changed under the plan (the calls since then were served by the recomputing kernels), or only passes that walk
+        // no plan have met it in this content;
         // the build fingerprints the present content, so this call needs no check
         const int st = plan_build(p, lookup, s);
         if (st != FFI_OK) { drop_cached_plan(p); return st; }
@@ -696,12 +699,14 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
         total += rows;
     }
     if (passes & FFI_PASS_BACKWARD) {
-        // small layers walk no plan: one is built for the check of the ids
+        // small layers walk no plan: their ids are checked
         if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
         // what recomputes the gradients behind an outdated plan
         else if (backward_if_outdated_workspace(d) > 0) total += backward_if_outdated_workspace(d) + kTicketCount * sizeof(unsigned);
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;
-        if ((one_window || two_windows) && d.K <= 1024 && d.L < (1 << 25)) {
+        if (small_backward) {
+            // (nothing else)
+        } else if ((one_window || two_windows) && d.K <= 1024 && d.L < (1 << 25)) {
             // tiled plan: the geometry of ffi_plan.hip, the slot rows of a slice estimated for column ids drawn uniformly
             // (longest of 64 columns whose lengths scatter like Poisson counts around tile_labels * fan_in / num_features);
             // inputs wider than 1,024 columns have one such form per half of the columns, walked one after the other
@@ -719,7 +724,6 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
                 const size_t slots = tiles * slices * rows * 64;
                 total += slots * 2 * 2 + (tiles * slices + 1) * 4 + L * 2;              // 4 bytes per slot (lab16 + pos16, or slot32), slice_off, rowpos
                 if (sorted) total += tiles * threads * 2;                               // the column of each thread in each tile
-                if (small_backward) continue;
                 if (!w_in_lds) features_slot = std::max(features_slot, slots * 4);     // weights in slot order
                 const size_t nbt = (B + 31) / 32;
                 const size_t per_cu = (size_t)tiled_workgroups_per_cu((int)threads, (int)TL, d.K, w_in_lds, (int)((B + 31) / 32));
@@ -732,14 +736,12 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
         } else {
             const GlobalShape f = global_shape(d.N, d.K, d.L, d.B);
             const size_t sl = 256 / (size_t)f.members, padded = (B + sl - 1) / sl * sl, units = (size_t)f.segments * f.groups;
-            const size_t at_once = small_backward ? 1 : (size_t)walk_slices((long long)units, (int)(padded / sl));
+            const size_t at_once = (size_t)walk_slices((long long)units, (int)(padded / sl));
             total += f.max_slots * 4 * (2 + at_once);                                   // entries; weights and weight gradients in their order
             total += L * K * 6 + (2 * units + 1) * 4;                                   // slot_of, tile_pos, chunk_ptr, chunk_count
             // counts while the plan is built; out_grad in slices and the sums per segment
             partial_slot = std::max(partial_slot, global_build_words(f, (int)(((long long)d.L * d.K + (1ll << f.tile_bits) - 1) >> f.tile_bits)) * 4);
-            if (!small_backward) {
-                partial_slot = std::max(partial_slot, (L + (f.segments > 1 ? N * (size_t)f.segments : 0)) * padded * 4);
-            }
+            partial_slot = std::max(partial_slot, (L + (f.segments > 1 ? N * (size_t)f.segments : 0)) * padded * 4);
         }
     }
     return total + features_slot + partial_slot;

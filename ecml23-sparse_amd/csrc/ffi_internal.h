@@ -326,6 +326,7 @@ struct ffi_plan {
     unsigned long long guard_seen = 0;        // number of the last check whose result the host has looked at
     bool guard_stale = false;                 // such a look found the plan outdated and nobody has acted on it yet
     bool edited_by_library = false;           // the library itself has enqueued an in-place edit of `lookup` since the plan was built
+    bool ids_only = false;                    // the ids were found in range, and nothing is laid out for them (plan_check_ids)
     hipStream_t guard_stream = nullptr;       // the stream of that check
     size_t bytes = 0;
     // Device buffers behind the arrays above (`owned`) and buffers of an earlier build kept for the next one (`spare`):
@@ -403,6 +404,7 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 }
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
+int plan_check_ids(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
 // How the global form of a lookup is cut (`batch`: the batch size it is built for, 0 = unknown).
 struct GlobalShape {

@@ -1442,6 +1442,20 @@ int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     p->guard_seen = p->guard_seq;
     p->guard_stale = false;
     p->edited_by_library = false;
+    p->ids_only = false;
+    return FFI_OK;
+}
+
+// Takes the place of a build for passes that read the lookup itself: finds every id in range, waiting for `s`, and lays nothing
+// out.  What an earlier build laid out is of no content that counts any more; it goes when the next build replaces it.
+int plan_check_ids(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
+    unsigned long long fp = 0, bad = 0;
+    p->ids_only = true;
+    free_spares(p);                            // (those of a plan that made room for this one)
+    FFI_TRY(plan_fingerprint(p, lookup, s, &fp, &bad));
+    if (bad != 0) return FFI_ERR_BAD_LOOKUP;
+    p->lookup = lookup;
+    p->edited_by_library = false;
     return FFI_OK;
 }
 

@@ -56,3 +56,25 @@ def test_an_id_out_of_range_is_reported_by_the_next_call():
         ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
     lookup[3, 2] = 49
     ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
+
+
+def test_a_lookup_whose_ids_only_were_checked_gets_its_plan_when_a_pass_walks_one():
+    # 2 samples read the lookup itself, 700 walk a plan; edits that the library is told of lie between them, at one address
+    ffi = load_package()
+    lib = ffi._lib.lib()
+    N, L, K = 300, 5000, 16
+    cases = {B: reference_law_inputs(B, N, L, K, seed=B) for B in (2, 700)}
+    lookup = torch.empty((L, K), dtype=torch.int32, device="cuda")
+    for turn, B in enumerate((2, 700, 2, 2, 700, 700, 2)):
+        x, ids, w, g = cases[B]
+        ids = (ids + 7 * turn) % N
+        lookup.copy_(torch.from_numpy(ids))
+        ffi._lib.check(lib.ffi_lookup_edited(lookup.data_ptr()))
+        gx, gw = ffi.fan_in_sparse_matmul_grad(*(torch.from_numpy(a).cuda() for a in (x,)), lookup, *(torch.from_numpy(a).cuda() for a in (w, g)))
+        ref_gx, ref_gw = oracle.backward(x, ids, w, g, transposed=False)
+        assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4, (turn, B)
+    lookup[3, 2] = N
+    ffi._lib.check(lib.ffi_lookup_edited(lookup.data_ptr()))
+    x, ids, w, g = (torch.from_numpy(a).cuda() for a in cases[2])
+    with pytest.raises(ffi._lib.FfiError):
+        ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
