@@ -87,17 +87,127 @@ __device__ __forceinline__ unsigned column_slots(unsigned thread, unsigned even,
     return max(first ? 2u * first - 1u : 0u, 2u * second);
 }
 
-// The sum of v over each LANES consecutive lanes (32 or 64), in all of them.
+// The sum of v over each LANES consecutive lanes (8, 32 or 64), in all of them.
 template <int LANES> __device__ __forceinline__ int lanes_total(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);         // lane ^ 1
     v += __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);         // lane ^ 2
     v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);        // 7 - lane within eight
+    if (LANES == 8) return v;
     v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);        // 15 - lane within sixteen
     const auto rows = __builtin_amdgcn_permlane16_swap(v, v, false, false);
     v = (int)(rows[0] + rows[1]);
     if (LANES == 32) return v;
     const auto halves = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return (int)(halves[0] + halves[1]);
+}
+
+constexpr int kPastLabels = 16;         // a sweep's steps end up to seven labels behind the last one and look one step ahead
+// What a sweep over a tile's labels works on, in LDS (see tile_color_kernel).
+struct TileLabels {
+    int* imb;                          // [ncols + 1] even minus odd labels per column
+    const unsigned* ids3;              // [nl][W] column ids, three to a word
+    const unsigned char* wt;           // [ncols + 1] weight of a column's balance; 0 at the end
+    unsigned char* half;               // [nl + kPastLabels] the half each label goes to
+    int nl, K, W, ncols, cap;
+};
+
+// One sweep, by one wavefront: 64 / LANES labels a step, PER connections of each in a lane's registers (MORE: the rest of the fan-in one by
+// one).  AGAIN: every label is taken out and put back.  placed: labels in even and odd rows so far.
+template <int LANES, int PER, bool MORE, bool AGAIN>
+__device__ __forceinline__ void sweep_labels(const TileLabels& t, int (&placed)[2]) {
+    constexpr int kAbreast = 64 / LANES;
+    constexpr unsigned long long kFirst = LANES == 8 ? 0x0101010101010101ull : LANES == 32 ? 0x0000000100000001ull : 1ull;   // a label's first lane
+    const int lane = threadIdx.x & 63, sub = lane & (LANES - 1), abreast = lane / LANES;
+    int word_at[PER], shift[PER], col[PER], w[PER];
+    unsigned word[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int k = min(sub + LANES * i, t.K - 1);
+        word_at[i] = k / 3;
+        shift[i] = 10 * (k % 3);
+    }
+    const int last = (t.nl - 1) * t.W;
+    int label = abreast, row = min(abreast * t.W, last), row1 = row;       // of the step; first words of its label and of the next one asked for
+    int next = abreast, next_half = 0;                                     // the label that advance() goes to
+    // To `next`, whose words are here; those of the label behind it and the columns' weights are asked for.
+    auto advance = [&]() {
+        row1 = min(row1 + kAbreast * t.W, last);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            // (behind the fan-in and behind the last label: the entry of weight 0)
+            col[i] = sub + LANES * i < t.K && next < t.nl ? (int)((word[i] >> shift[i]) & 1023u) : t.ncols;
+            word[i] = t.ids3[row1 + word_at[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) w[i] = (int)t.wt[col[i]];
+        if (AGAIN) next_half = t.half[next];
+        next += kAbreast;
+    };
+    auto rest = [&](auto visit) {
+        if (!MORE) return;
+        for (int k = sub + LANES * PER; k < t.K; k += LANES) {
+            const int c = (int)((t.ids3[row + k / 3] >> (10 * (k % 3))) & 1023u);
+            visit(label < t.nl ? c : t.ncols);
+        }
+    };
+    auto add = [&](const int (&c)[PER], int delta) {                       // (a column may occur twice in a label)
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (sub + LANES * i < t.K) atomicAdd(&t.imb[c[i]], delta);
+        rest([&](int q) { atomicAdd(&t.imb[q], delta); });
+    };
+#pragma unroll
+    for (int i = 0; i < PER; ++i) word[i] = t.ids3[row + word_at[i]];
+    advance();
+    const int steps = (t.nl + kAbreast - 1) / kAbreast, tie = (abreast & 1) ? -1 : 1;
+    for (int g = 0; g < steps; ++g) {
+        int c[PER], sum = 0;
+        // (1 or -1: the half taken where the columns ask for neither -- the label's own, or the emptier one, by turns)
+        const int lean = AGAIN ? (next_half ? 1 : -1) : placed[1] < placed[0] ? tie : -tie;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) c[i] = col[i];
+        if (AGAIN) add(c, lean);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) sum += __mul24(w[i], t.imb[c[i]]);
+        advance();
+        rest([&](int q) { sum += t.wt[q] * t.imb[q]; });
+        bool odd = 2 * lanes_total<LANES>(sum) + lean > 0;
+        if (__builtin_expect(max(placed[0], placed[1]) + kAbreast > t.cap, 0)) {               // (uniform)
+            // the halves may be full: where a label asks to go as far as there is room; labels that stay keep their places, theirs first
+            const unsigned long long there = __ballot(label < t.nl) & kFirst, was = AGAIN ? __ballot(lean > 0) & there : 0ull;
+            unsigned long long to = __ballot(odd) & there;
+            const unsigned long long asked = to;
+            int room[2] = {t.cap - placed[0], t.cap - placed[1]};
+            if (AGAIN) {
+                room[1] += __popcll(was);
+                room[0] += __popcll(there & ~was);
+            }
+            for (int pass = 0; pass < 2; ++pass)
+                for (int h = 0; h < kAbreast; ++h) {
+                    const unsigned long long bit = 1ull << (h * LANES);
+                    if (!(there & bit) || (AGAIN && ((asked ^ was) & bit)) != (pass == 1)) continue;
+                    if (room[(to & bit) ? 1 : 0] <= 0) to ^= bit;
+                    --room[(to & bit) ? 1 : 0];
+                }
+            placed[0] = t.cap - room[0];
+            placed[1] = t.cap - room[1];
+            odd = (to >> (abreast * LANES) & 1ull) != 0;
+        } else if (AGAIN) {
+            // (what is not there, behind the last label, stays as it was)
+            const int more = ((int)__popcll(__ballot(odd)) - (int)__popcll(__ballot(lean > 0))) / LANES;
+            placed[1] += more;
+            placed[0] -= more;
+        } else {
+            const unsigned long long there = __ballot(label < t.nl) & kFirst;
+            const int more = (int)__popcll(__ballot(odd) & there);
+            placed[1] += more;
+            placed[0] += (int)__popcll(there) - more;
+        }
+        add(c, odd ? -1 : 1);
+        t.half[label] = odd ? 1 : 0;                                       // (all lanes of a label, one value)
+        label += kAbreast;
+        row = min(row + kAbreast * t.W, last);
+    }
 }
 
 // Which LDS row of the walking kernel's tile each label is staged into (rowpos[j], inside the label's tile).
@@ -107,25 +217,25 @@ template <int LANES> __device__ __forceinline__ int lanes_total(int v) {
 // and each goes to the half that the columns it feeds have used less so far (weighted sum over its connections
 // of even-count minus odd-count of the column), which keeps the columns that matter close to an even split.
 // Rows of a half are handed out in ascending order, at most `cap` per half.  One workgroup per tile; the tile's
-// column ids are staged in LDS, one wavefront then decides label after label (lane <-> connection), or two at a time where 32 lanes
-// hold a fan-in; beyond a fan-in of 64 a lane has several connections.
+// column ids are staged in LDS, one wavefront then decides a few labels at a time (sweep_labels).
 // (`col_lo`: the plan covers the columns [col_lo, col_lo + ncols) only; connections into other columns are left out)
 // (`all_columns_count`: plans that hand the columns to threads by length -- there every column is about as long as the
 // longest of its slice, so every column's balance weighs the same)
-template <int LANES, bool MORE>              // (MORE: fan-ins above LANES = 64)
+template <int LANES, int PER, bool MORE>     // of the second sweep: lanes per label, connections per lane (MORE: fan-ins beyond them)
 __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restrict__ idx, int L, int K, int tile_labels, int cap,
                                                          int ncols, unsigned short* __restrict__ rowpos, int col_lo,
                                                          int all_columns_count, unsigned* __restrict__ counts) {
     extern __shared__ int color_lds[];
     // (entry `ncols` of both: where connections into columns outside the window go -- weight 0, so they never count)
     int* imb = color_lds;                                                        // [ncols + 1] even minus odd labels per column
-    // The tile's column ids, three 10-bit ids per word, a label's ids in W = ceil(K / 3) words of its own, and the weights as
-    // 16-bit numbers: with 16-bit ids and 32-bit weights a tile of 582 labels x fan-in 32 took 44 KB of LDS, three workgroups per
+    // The tile's column ids, three 10-bit ids per word, a label's ids in W = ceil(K / 3) words of its own, and the weights
+    // and the halves in bytes: with 16-bit ids and 32-bit weights a tile of 582 labels x fan-in 32 took 44 KB of LDS, three workgroups per
     // CU and two rounds for 1,152 tiles; now 30 KB, five workgroups per CU, all tiles at once (the work of a tile is one
-    // wavefront's sequential loop).
+    // wavefront's sequential loop; 32,000 bytes are the most of which five fit, a tile of 616 labels takes 31.6 KB).
     const int W = (K + 2) / 3;
     unsigned* ids3 = reinterpret_cast<unsigned*>(color_lds + ncols + 1);         // [tile_labels * W]
-    unsigned short* wt = reinterpret_cast<unsigned short*>(ids3 + (size_t)tile_labels * W);   // [ncols + 1] weight of the column's balance (at most 256)
+    unsigned char* wt = reinterpret_cast<unsigned char*>(ids3 + (size_t)tile_labels * W);   // [ncols + 1] weight of the column's balance
+    unsigned char* half = wt + ncols + 1;                                        // [tile_labels + kPastLabels] the half each label goes to
     const int t = blockIdx.x;
     const int j0 = t * tile_labels;
     const int nl = min(tile_labels, L - j0);
@@ -133,25 +243,36 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     const unsigned outside = (unsigned)min(ncols, 1023);                          // (windows are at most 640 columns wide; a single window has no ids outside)
     for (int i = threadIdx.x; i <= ncols; i += 256) { imb[i] = 0; wt[i] = 0; }
     __syncthreads();
-    for (int wi = threadIdx.x; wi < nl * W; wi += 256) {
-        const int jl = wi / W, k0 = 3 * (wi - jl * W);
-        unsigned word = 0;
+    constexpr int kTogether = 4;                                                 // words whose ids are asked for together
+    for (int w0 = threadIdx.x; w0 < nl * W; w0 += 256 * kTogether) {
+        unsigned v[kTogether][3];
+        int k0[kTogether];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            unsigned c = outside;
-            if (k0 + i < K) {
-                const unsigned v = (unsigned)(src[jl * K + k0 + i] - col_lo);
-                if (v < (unsigned)ncols) { c = v; atomicAdd(&imb[v], 1); }       // column lengths first (in imb: the LDS adds whole words)
-            } else {
-                c = (unsigned)min(ncols, 1023);                                  // (behind the label's last id: never read)
-            }
-            word |= c << (10 * i);
+        for (int u = 0; u < kTogether; ++u) {
+            const int wi = min(w0 + 256 * u, nl * W - 1), jl = wi / W;
+            k0[u] = 3 * (wi - jl * W);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) v[u][i] = (unsigned)(src[jl * K + min(k0[u] + i, K - 1)] - col_lo);
         }
-        ids3[wi] = word;
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u) {
+            if (w0 + 256 * u >= nl * W) break;
+            unsigned word = 0;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                unsigned c = outside;                                            // (also behind the label's last id, where it is never read)
+                if (k0[u] + i < K && v[u][i] < (unsigned)ncols) {
+                    c = v[u][i];
+                    atomicAdd(&imb[c], 1);                                       // column lengths first (in imb: the LDS adds whole words)
+                }
+                word |= c << (10 * i);
+            }
+            ids3[w0 + 256 * u] = word;
+        }
     }
     __syncthreads();
     // Only the longest columns of a slice (64 columns, one wavefront of the walking kernel) set its number of slot
-    // rows, so their balance counts most: weight = 256 * (length / longest of the slice)^8.
+    // rows, so their balance counts most: weight = 255 * (length / longest of the slice)^8.
     for (int c = threadIdx.x; c < ncols; c += 256) {
         const int len = imb[c];
         imb[c] = 0;
@@ -160,109 +281,29 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
         for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off, 64));
         float r = longest > 0 ? (float)len / (float)longest : 0.f;
         r *= r; r *= r; r *= r;
-        wt[c] = (unsigned short)(all_columns_count ? (len > 0 ? 256 : 0) : (int)(256.f * r));
+        wt[c] = (unsigned char)(all_columns_count ? (len > 0 ? 1 : 0) : (int)(255.f * r));
     }
     __syncthreads();
-    // the half a label goes to: bit 30 of its first word
-    auto half_of = [&](int jl) { return (int)(ids3[jl * W] >> 30 & 1u); };
     const int lane = threadIdx.x & 63;
     auto decide_all = [&]() {
-    constexpr int kAbreast = 64 / LANES;                                         // labels decided together
-    const int groups = (nl + kAbreast - 1) / kAbreast, k_mine = lane & (LANES - 1), abreast = lane / LANES;
-    int placed[2] = {0, 0};
     // What bounds the kernel is the chain from one step's adds to the next step's decision: an LDS round trip, the sum over the
-    // lanes by DPP and lane swaps, a comparison in every lane; what it does to the counts of placed labels is beside the chain.  Of
-    // two labels decided together the second does not see what the first just did: 670,091 labels x fan-in 32 over 768 columns
-    // 322 -> 181 us, 200,000 x 8 over 300 143 -> 81, with slot rows per connection 1.1522 -> 1.1523, 2.0510 -> 2.0514.  (Four
-    // together: 0.1 to 0.4 % more slot rows, which every walk pays for.  Two of a fan-in of 64, two connections a lane: 528 -> 455
-    // us at 501,070 labels, for 0.16 % more.)
-    // A lane's column is asked for two steps ahead, the column's weight one.
-    auto place_of = [&](int k) { return make_int2(k / 3, 10 * (k % 3)); };
-    const int2 place = place_of(min(k_mine, K - 1));
-    auto label_of = [&](int g) { return g * kAbreast + abreast; };
-    auto word_of = [&](int g) { return ids3[min(label_of(g), nl - 1) * W + place.x]; };
-    const bool on = k_mine < K;
-    int col1 = 0, w1 = 0;                                                        // the next label's
-    unsigned word2 = 0;
-    auto advance = [&](int g) {                                                  // to label_of(g), whose word is here
-        col1 = (int)((word2 >> place.y) & 1023u);
-        if (kAbreast > 1 && label_of(g) >= nl) col1 = ncols;                     // (behind the last label: weight 0)
-        word2 = word_of(g + 1);
-        const int w = (int)wt[col1];
-        w1 = on ? w : 0;
-    };
-    // connections behind the first of a lane (fan-ins above 64)
-    auto rest = [&](int g, auto visit) {
-        if (!MORE) return;
-        for (int k = lane + 64; k < K; k += 64) {
-            const int2 at = place_of(k);
-            visit((int)((ids3[label_of(g) * W + at.x] >> at.y) & 1023u));
-        }
-    };
-    // the balance that a lane's label asks for, after `back` (0: nothing) is added to its columns; then `decide` says which half
-    auto step = [&](int g, int had, int back, auto decide) {
-        const int c = col1, w = w1;
-        if (back != 0) {
-            if (__builtin_expect(on, 1)) atomicAdd(&imb[c], back);
-            rest(g, [&](int q) { atomicAdd(&imb[q], back); });
-        }
-        int sum = __mul24(w, imb[c]);
-        advance(g + 1);
-        rest(g, [&](int q) { sum += wt[q] * imb[q]; });
-        const int color = decide(lanes_total<LANES>(sum)), delta = color ? -1 : 1;
-        if (__builtin_expect(on, 1)) atomicAdd(&imb[c], delta);                                          // (a column may occur twice in a label)
-        rest(g, [&](int q) { atomicAdd(&imb[q], delta); });
-        if (k_mine == 0 && label_of(g) < nl && color != had) atomicXor(&ids3[label_of(g) * W], 1u << 30);
-    };
-    // where the labels of a step go once the halves may be full: `color` as far as there is room, else `other`
-    auto settle = [&](int g, int color, int other, bool again) {
-        const unsigned long long first = kAbreast == 1 ? 1ull : 1ull | 1ull << LANES;            // a label's first lane
-        const unsigned long long there = first & (g * kAbreast + kAbreast > nl ? 1ull : ~0ull);
-        unsigned long long to = __ballot(color != 0) & there;
-        const unsigned long long was = __ballot(other != 0) & there;
-        if (again) {
-            placed[1] -= __popcll(was);
-            placed[0] -= __popcll(there & ~was);
-        }
-        if (__builtin_expect(max(placed[0], placed[1]) + kAbreast > cap, 0)) {                          // (uniform)
-            int room[2] = {cap - placed[0], cap - placed[1]};
-            // (labels that stay keep their places: theirs first)
-#pragma unroll
-            for (int pass = 0; pass < 2; ++pass)
-#pragma unroll
-                for (int h = 0; h < kAbreast; ++h) {
-                    const unsigned long long bit = 1ull << (h * LANES);
-                    if (!(there & bit) || (again && ((to ^ was) & bit)) != (pass == 1)) continue;
-                    if (room[(to & bit) ? 1 : 0] <= 0) to ^= bit;
-                    --room[(to & bit) ? 1 : 0];
-                }
-            color = (int)(to >> (abreast * LANES) & 1ull);
-        }
-        placed[1] += __popcll(to);
-        placed[0] += __popcll(there & ~to);
-        return color;
-    };
-    word2 = word_of(0);
-    advance(0);
-    for (int g = 0; g < groups; ++g) {
-        const int even = placed[1] < placed[0] ? 1 : 0;
-        step(g, 0, 0, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : even ^ abreast), 0, false); });
-    }
+    // lanes by DPP and lane swaps, a comparison in every lane, some 60 instructions of one wavefront.  Labels decided together do not see
+    // what the others of the step just did.  In the first sweep that is mended by the second: eight a step.  In the second it stays: two
+    // (one beyond a fan-in of 32).  Slot rows per connection, 582-label tiles of fan-in 32 over 768 columns: 1.5267 with two in both, 1.5279 so,
+    // 1.5309 with four in the second; sorted columns 1.1542, 1.1549, 1.1559.  670,091 labels of fan-in 32 196 -> 126 us,
+    // 14 of them ids asked for twelve at a time; 131,072 labels a whole build 248 -> 195, 50,000 of fan-in 100 897 -> 517.  (The first sweep by
+    // four wavefronts, a quarter of the labels each, and their sums put together: 1.5347, 1.1586.)
+    int placed[2] = {0, 0};
+    const TileLabels labels{imb, ids3, wt, half, nl, K, W, ncols, cap};
+    sweep_labels<8, LANES / 8 * PER, MORE, false>(labels, placed);
     // Second sweep: every label is taken out and put back into the half its columns now ask for -- the first sweep placed
     // the early labels knowing nothing of the later ones.  (Measured on uniformly drawn ids, 586-label tiles of fan-in 32
     // over 768 columns: slot rows 1.528 -> 1.514 per connection, where columns of unconstrained order would need 1.490.)
-    word2 = word_of(0);
-    advance(0);
-    int next_old = half_of(min(label_of(0), nl - 1));       // (written by this wavefront above, whose LDS accesses are in order)
-    for (int g = 0; g < groups; ++g) {
-        const int old = next_old;
-        next_old = half_of(min(label_of(g + 1), nl - 1));
-        step(g, old, old ? 1 : -1, [&](int sum) { return settle(g, sum > 0 ? 1 : (sum < 0 ? 0 : old), old, true); });
-    }
+    sweep_labels<LANES, PER, MORE, true>(labels, placed);
     // rows of a half are handed out in ascending label order
     int next[2] = {0, 0};
     for (int l0 = 0; l0 < nl; l0 += 64) {
-        const bool on = l0 + lane < nl, odd = on && half_of(min(l0 + lane, nl - 1)) != 0;
+        const bool on = l0 + lane < nl, odd = on && half[min(l0 + lane, nl - 1)] != 0;
         const unsigned long long odds = __ballot(odd), evens = __ballot(on && !odd), before = (1ull << lane) - 1ull;
         if (on) rowpos[j0 + l0 + lane] = (unsigned short)(2 * (next[odd] + __popcll((odd ? odds : evens) & before)) + (odd ? 1 : 0));
         next[0] += __popcll(evens);
@@ -277,7 +318,7 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     for (int wi = threadIdx.x; wi < nl * W; wi += 256) {
         const int jl = wi / W, k0 = 3 * (wi - jl * W);
         const unsigned word = ids3[wi];
-        const int one = half_of(jl) ? 0x10000 : 1;
+        const int one = half[jl] ? 0x10000 : 1;
 #pragma unroll
         for (int i = 0; i < 3; ++i)
             if (k0 + i < K) atomicAdd(&imb[(word >> (10 * i)) & 1023u], one);
@@ -1110,8 +1151,9 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     const int cap = tiled_rows_per_half(TL);
     if (!dev_alloc(p, &p->rowpos, (size_t)p->L)) return FFI_ERR_OUT_OF_MEMORY;
     {
-        const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + ((size_t)threads + 2) * sizeof(unsigned short);
-        const auto color = p->K <= 32 ? tile_color_kernel<32, false> : p->K <= 64 ? tile_color_kernel<64, false> : tile_color_kernel<64, true>;
+        const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + (size_t)threads + 1 + (size_t)TL + kPastLabels;
+        const auto color = p->K <= 32 ? tile_color_kernel<32, 1, false> : p->K <= 64 ? tile_color_kernel<64, 1, false>
+                                    : p->K <= 128 ? tile_color_kernel<64, 2, false> : tile_color_kernel<64, 2, true>;
         hipError_t ea = hipFuncSetAttribute((const void*)color, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (ea != hipSuccess) return hip_fail(ea);
         hipLaunchKernelGGL(color, dim3(tiles), dim3(256), lds, s, lookup, p->L, p->K, TL, cap, threads, p->rowpos, p->col_lo,
