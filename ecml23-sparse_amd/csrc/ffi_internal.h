@@ -67,7 +67,7 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11, kWsSums = 12 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11, kWsSums = 12, kWsSelect = 13 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 // 128 bytes of pinned host memory of the stream, for results that the host waits for
 int host_words_get(hipStream_t s, void** out);

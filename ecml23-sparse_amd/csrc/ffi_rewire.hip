@@ -3,9 +3,9 @@
 //
 //   threshold selection  the k-th smallest |w| (FixedFractionSelector: tf.nn.top_k(-|w|, k), last value) by a
 //                        three-pass radix select over the 31-bit patterns of |w| (11 + 11 + 9 bits): each pass
-//                        histograms one digit of the values that match the digits found so far
-//                        (select_hist_kernel), a one-block kernel picks the bin that holds the k-th value
-//                        (select_pick_kernel).  Integer atomics only: the result does not depend on their order.
+//                        histograms one digit of the values that match the digits found so far, and its last
+//                        workgroup picks the bin that holds the k-th value (select_pass_kernel).  Integer atomics only:
+//                        the result does not depend on their order.
 //   rewire_kernel        every position p with |w[p]| < threshold: lookup[p] = a source drawn uniformly from
 //                        [0, num_features) by a counter-based generator keyed on (seed, p); arrays[i][p] = 0.
 #include "ffi_internal.h"
@@ -16,94 +16,142 @@
 namespace ffi {
 namespace {
 
-constexpr int kSelThreads = 256;
+constexpr int kSelThreads = 1024;
 constexpr int kSelBins = 2048;
 
+// Zero between selections but for `prefix` and `k`, which each pass leaves for the next.
 struct SelectState {
     unsigned prefix;              // digits found so far (the high bits of the answer)
+    unsigned ticket;
     unsigned long long k;         // rank still to find among the values matching the prefix (1-based)
+    unsigned long long listed;    // values that match the first digit: those in the list, or more than it holds
+    unsigned long long rewired;   // rewire_kernel: connections changed, and the workgroups that have said so << 40
 };
 
 __device__ __forceinline__ unsigned magnitude_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 
-// hist[bin] += number of values whose bits above (shift + nbits) equal state->prefix and whose digit is bin
+// Workgroup-local bins are hist[bin] += number of values whose bits above (shift + nbits) equal the prefix and whose digit is bin.
 // Weights have few exponents, so in the first pass a wavefront's lanes meet in some twenty bins: its lanes count in four copies of
 // the histogram, side by side in the banks, and the workgroups add to kHistTotals totals.  (21 M normal values: 58 us in one
-// copy, 31 in four or eight that all go to one total, 25 so; the other passes, which few values match, 18, what it takes to
+// copy, 31 in four or eight that all go to one total, 25 so; the second pass, which few values match, 18, what it takes to
 // read them.)
-constexpr int kHistThreads = 1024, kHistCopies = 4, kHistTotals = 8;
-__global__ __launch_bounds__(kHistThreads) void select_hist_kernel(const float* __restrict__ w, size_t count, int shift, int nbits,
-                                                                    const SelectState* __restrict__ state,
-                                                                    unsigned* __restrict__ hist) {
+// The second pass also puts the values that match the first digit in a list, and the third reads the list instead of all values
+// where they fitted into it, which takes values that crowd within an eighth of an octave to fail.  The workgroup that adds its
+// bins last picks the bin in which the cumulative count reaches k, appends it to the prefix, reduces k by the count of the bins
+// below it and clears the bins: all read-modify-writes at device scope whose results are waited for before the ticket is drawn.
+// (A launch for each pick and one to clear, and all values read in the third pass: 81 us in seven launches, 62 so in three; 12,291 x 7: 187 us of a rewiring and its pass against 206.)
+constexpr int kHistThreads = 1024, kHistCopies = 4, kHistTotals = 8, kSelLocalList = 2048;
+template <int PASS>
+__global__ __launch_bounds__(kHistThreads) void select_pass_kernel(const float* __restrict__ w, size_t count, unsigned long long k0,
+                                                                    SelectState* __restrict__ state, unsigned* __restrict__ hist,
+                                                                    unsigned* __restrict__ list, unsigned long long capacity, float* __restrict__ threshold) {
+    constexpr int kShift = PASS == 0 ? 20 : PASS == 1 ? 9 : 0, kBits = PASS == 2 ? 9 : 11, kEach = kSelBins / kHistThreads;
+    constexpr unsigned kMask = (1u << kBits) - 1u;
     __shared__ __align__(16) unsigned local[kSelBins * kHistCopies];
+    __shared__ unsigned mine[PASS == 1 ? kSelLocalList : 1], n_mine, is_last;
+    __shared__ unsigned long long list_at;
+    const unsigned prefix = PASS == 0 ? 0u : state->prefix, copy = threadIdx.x % kHistCopies;
+    const bool from_list = PASS == 2 && state->listed <= capacity;
+    const size_t n = from_list ? (size_t)state->listed : count;
+    // (a list has work for few workgroups: the others leave, and no ticket is expected of them)
+    const unsigned parts = from_list ? (unsigned)min((size_t)gridDim.x, max((n + kHistThreads - 1) / kHistThreads, (size_t)1)) : gridDim.x;
+    if (blockIdx.x >= parts) return;
     for (int i = threadIdx.x; i < kSelBins * kHistCopies; i += kHistThreads) local[i] = 0;
+    if (threadIdx.x == 0) n_mine = 0u;
     __syncthreads();
-    const unsigned prefix = state->prefix;
-    const int above = shift + nbits;                       // 31 in the first pass: nothing to match
-    const unsigned mask = (1u << nbits) - 1u, copy = threadIdx.x % kHistCopies;
-    for (size_t i = (size_t)blockIdx.x * kHistThreads + threadIdx.x; i < count; i += (size_t)gridDim.x * kHistThreads) {
-        const unsigned key = magnitude_bits(w[i]);
-        if (above >= 31 || (key >> above) == prefix) atomicAdd(&local[((key >> shift) & mask) * kHistCopies + copy], 1u);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < kSelBins; i += kHistThreads) {
-        unsigned n = 0;
+    constexpr int kTogether = 4;                                          // values asked for together
+    constexpr unsigned kNone = ~0u;                                       // (no magnitude)
+    const size_t stride = (size_t)parts * kHistThreads;
+    for (size_t i0 = (size_t)blockIdx.x * kHistThreads + threadIdx.x; i0 < n; i0 += kTogether * stride) {
+        unsigned keys[kTogether];
 #pragma unroll
-        for (int c = 0; c < kHistCopies; c += 4) {
-            const uint4 q = *reinterpret_cast<const uint4*>(local + i * kHistCopies + c);
-            n += (q.x + q.y) + (q.z + q.w);
+        for (int u = 0; u < kTogether; ++u) {
+            const size_t i = min(i0 + u * stride, n - 1);
+            const unsigned key = from_list ? list[i] : magnitude_bits(w[i]);
+            keys[u] = i0 + u * stride < n ? key : kNone;
         }
-        if (n) atomicAdd(&hist[(blockIdx.x % kHistTotals) * kSelBins + i], n);
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u) {
+            const unsigned key = keys[u];
+            const bool match = key != kNone && (PASS == 0 || (key >> (kShift + kBits)) == prefix);
+            if (match) atomicAdd(&local[((key >> kShift) & kMask) * kHistCopies + copy], 1u);
+            if (PASS == 1) {
+                const unsigned long long matches = __ballot(match);
+                if (matches != 0ull) {                                        // (one add of a wavefront)
+                    const int lane = threadIdx.x & 63, first = __ffsll((long long)matches) - 1;
+                    unsigned at = 0;
+                    if (lane == first) at = atomicAdd(&n_mine, (unsigned)__popcll(matches));
+                    at = (unsigned)__builtin_amdgcn_readlane((int)at, first) + (unsigned)__popcll(matches & ((1ull << lane) - 1ull));
+                    if (match && at < (unsigned)kSelLocalList) mine[at] = key;
+                }
+            }
+        }
     }
-}
-
-// One block: the bin in which the cumulative count reaches state->k; appends it to the prefix, reduces k by the
-// count of the bins below it, clears the histogram for the next pass.
-// (Walked by one thread, 2,048 bins took 22 us, all of it LDS latency; 4.8 so.)
-constexpr int kPickThreads = 1024;
-__global__ __launch_bounds__(kPickThreads) void select_pick_kernel(unsigned* __restrict__ hist, int nbits, SelectState* __restrict__ state,
-                                                                   int last, float* __restrict__ threshold) {
-    constexpr int kEach = kSelBins / kPickThreads;
-    const int bins = 1 << nbits, first = threadIdx.x * kEach;
-    unsigned count[kEach];
-    unsigned long long mine = 0;
+    __syncthreads();
+    if (PASS == 1) {
+        if (threadIdx.x == 0)
+            list_at = n_mine ? __hip_atomic_fetch_add(&state->listed, n_mine > (unsigned)kSelLocalList ? capacity + 1ull : (unsigned long long)n_mine, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        __syncthreads();
+        for (unsigned i = threadIdx.x; i < min(n_mine, (unsigned)kSelLocalList); i += kHistThreads)
+            if (list_at + i < capacity) list[list_at + i] = mine[i];
+    }
+    unsigned old = 0;
+    for (int i = threadIdx.x; i < kSelBins; i += kHistThreads) {
+        unsigned c = 0;
+#pragma unroll
+        for (int q = 0; q < kHistCopies; q += 4) {
+            const uint4 v = *reinterpret_cast<const uint4*>(local + i * kHistCopies + q);
+            c += (v.x + v.y) + (v.z + v.w);
+        }
+        if (c) old |= __hip_atomic_fetch_add(&hist[(blockIdx.x % kHistTotals) * kSelBins + i], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("" :: "v"(old));                                         // (the adds have returned)
+    __syncthreads();
+    if (threadIdx.x == 0) is_last = __hip_atomic_fetch_add(&state->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1u;
+    __syncthreads();
+    if (!is_last) return;
+    // (walked by one thread, 2,048 bins took 22 us, all of it latency)
+    const int first = threadIdx.x * kEach;
+    unsigned bins[kEach][kHistTotals], bin_count[kEach];
+    unsigned long long sum = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i)
+#pragma unroll
+        for (int t = 0; t < kHistTotals; ++t)
+            bins[i][t] = __hip_atomic_exchange(&hist[t * kSelBins + first + i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int i = 0; i < kEach; ++i) {
-        count[i] = 0u;
+        bin_count[i] = 0u;                                                // (behind the last bin: nothing was added)
 #pragma unroll
-        for (int t = 0; t < kHistTotals; ++t) count[i] += hist[t * kSelBins + first + i];     // (behind the last bin: nothing was added)
-        mine += count[i];
+        for (int t = 0; t < kHistTotals; ++t) bin_count[i] += bins[i][t];
+        sum += bin_count[i];
     }
-    const unsigned long long k = state->k;
-    const unsigned prefix = state->prefix;
-    unsigned long long total = 0, below = block_sum_below<kPickThreads>(mine, &total);      // (its barrier: all is read before any is written)
+    const unsigned long long k = PASS == 0 ? k0 : state->k;
+    unsigned long long below = block_sum_below<kHistThreads>(sum, &total);       // (its barrier: state is read before it is written)
     int pick = -1;
-    if (below < k && below + mine >= k) {
+    if (below < k && below + sum >= k) {
         pick = first;
 #pragma unroll
         for (int i = 0; i + 1 < kEach; ++i)
-            if (pick == first + i && below + count[i] < k) { below += count[i]; ++pick; }
+            if (pick == first + i && below + bin_count[i] < k) { below += bin_count[i]; ++pick; }
     } else if (total < k && threadIdx.x == 0) {
-        pick = bins - 1;
+        pick = (1 << kBits) - 1;
         below = total;
     }
     if (pick >= 0) {
-        const unsigned value = (prefix << nbits) | (unsigned)pick;
+        const unsigned value = (prefix << kBits) | (unsigned)pick;
         state->prefix = value;
         state->k = k - below;
-        if (last) *threshold = __uint_as_float(value);
+        if (PASS == 2) *threshold = __uint_as_float(value);
     }
-    for (int i = threadIdx.x; i < kSelBins * kHistTotals; i += kPickThreads) hist[i] = 0;
+    if (threadIdx.x == 0) {
+        state->ticket = 0u;
+        if (PASS == 2) state->listed = 0ull;
+    }
 }
 
-__global__ void select_init_kernel(SelectState* state, unsigned* hist, unsigned long long k, float* threshold) {
-    for (int i = threadIdx.x; i < kSelBins * kHistTotals; i += blockDim.x) hist[i] = 0;
-    if (threadIdx.x == 0) {
-        state->prefix = 0;
-        state->k = k;
-        if (k == 0) *threshold = 0.f;            // nothing is below 0 in magnitude: an empty selection
-    }
-}
+__global__ void select_none_kernel(float* threshold) { *threshold = 0.f; }    // nothing is below 0 in magnitude: an empty selection
 
 // splitmix64 finaliser over (seed, position): a counter-based generator, so the draw of a position does not
 // depend on how the launch is shaped
@@ -121,7 +169,8 @@ struct ArrayList {
 __global__ __launch_bounds__(kSelThreads) void rewire_kernel(int32_t* __restrict__ lookup, const float* __restrict__ w,
                                                               ArrayList arrays, int n_arrays, size_t count,
                                                               unsigned num_features, const float* __restrict__ threshold,
-                                                              unsigned long long seed, unsigned long long* __restrict__ block_counts) {
+                                                              unsigned long long seed, unsigned long long* __restrict__ counted,
+                                                              long long* __restrict__ rewired) {
     __shared__ unsigned red[kSelThreads / 64];
     const float thr = *threshold;
     unsigned changed = 0;
@@ -140,38 +189,41 @@ __global__ __launch_bounds__(kSelThreads) void rewire_kernel(int32_t* __restrict
     if (threadIdx.x == 0) {
         unsigned long long t = 0;
         for (int i = 0; i < kSelThreads / 64; ++i) t += red[i];
-        block_counts[blockIdx.x] = t;
+        // (fewer than 2^40 connections and 2^24 workgroups; who adds last has the sum.  Adds to one address take turns: of 2,048
+        // workgroups of 256 threads they were 12 us of the kernel's 49, so it has 512 of 1,024.)
+        const unsigned long long one = 1ull << 40, all = __hip_atomic_fetch_add(counted, t + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + t + one;
+        if (all >> 40 == gridDim.x) {
+            if (rewired != nullptr) *rewired = (long long)(all & (one - 1ull));
+            __hip_atomic_store(counted, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
-__global__ __launch_bounds__(1024) void rewire_count_kernel(const unsigned long long* __restrict__ block_counts, int n,
-                                                            long long* __restrict__ out) {
-    unsigned long long t = 0, all = 0;
-    for (int i = threadIdx.x; i < n; i += 1024) t += block_counts[i];
-    (void)block_sum_below<1024>(t, &all);
-    if (threadIdx.x == 0) *out = (long long)all;
-}
+constexpr size_t kSelectBytes = 256 + kSelBins * kHistTotals * sizeof(unsigned);     // the state, then the bins
+static_assert(sizeof(SelectState) <= 256, "the bins lie behind it");
 
 int stream_blocks(size_t count) {
-    return (int)std::max<size_t>(1, std::min<size_t>((count + kSelThreads - 1) / kSelThreads, (size_t)device_cu_count() * 8));
+    return (int)std::max<size_t>(1, std::min<size_t>((count + kSelThreads - 1) / kSelThreads, (size_t)device_cu_count() * 2));
 }
 
 }  // namespace
 
 int launch_select_threshold(const float* w, size_t count, unsigned long long k, float* threshold, hipStream_t s) {
+    if (k == 0) {
+        hipLaunchKernelGGL(select_none_kernel, dim3(1), dim3(1), 0, s, threshold);
+        FFI_HIP_TRY(hipGetLastError());
+        return FFI_OK;
+    }
     unsigned char* ws = nullptr;
-    FFI_TRY(workspace_get(s, kWsRewire, 256 + kSelBins * kHistTotals * sizeof(unsigned), (void**)&ws));
+    FFI_TRY(zeroed_get(s, kWsSelect, kSelectBytes, (void**)&ws));
+    const size_t capacity = std::max<size_t>(count / 32, 1024);
+    unsigned* list = nullptr;
+    FFI_TRY(workspace_get(s, kWsRewire, capacity * sizeof(unsigned), (void**)&list));
     SelectState* state = reinterpret_cast<SelectState*>(ws);
     unsigned* hist = reinterpret_cast<unsigned*>(ws + 256);
-    hipLaunchKernelGGL(select_init_kernel, dim3(1), dim3(kPickThreads), 0, s, state, hist, k, threshold);
-    if (k > 0) {
-        const int blocks = (int)std::max<size_t>(1, std::min<size_t>((count + kHistThreads - 1) / kHistThreads, (size_t)device_cu_count() * 2));
-        const int shifts[3] = {20, 9, 0}, bits[3] = {11, 11, 9};
-        for (int pass = 0; pass < 3; ++pass) {
-            hipLaunchKernelGGL(select_hist_kernel, dim3(blocks), dim3(kHistThreads), 0, s, w, count, shifts[pass], bits[pass], state, hist);
-            hipLaunchKernelGGL(select_pick_kernel, dim3(1), dim3(kPickThreads), 0, s, hist, bits[pass], state, pass == 2 ? 1 : 0, threshold);
-        }
-    }
+    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((count + kHistThreads - 1) / kHistThreads, (size_t)device_cu_count() * 2));
+    for (const auto pass : {select_pass_kernel<0>, select_pass_kernel<1>, select_pass_kernel<2>})
+        hipLaunchKernelGGL(pass, dim3(blocks), dim3(kHistThreads), 0, s, w, count, k, state, hist, list, (unsigned long long)capacity, threshold);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
@@ -180,14 +232,10 @@ int launch_rewire(int32_t* lookup, const float* w, float* const* arrays, int n_a
                   const float* threshold, unsigned long long seed, long long* rewired, hipStream_t s) {
     ArrayList list{};
     for (int i = 0; i < n_arrays; ++i) list.p[i] = arrays[i];
-    const int blocks = stream_blocks(count);
-    unsigned long long* block_counts = nullptr;
-    FFI_TRY(workspace_get(s, kWsRewire, 256 + std::max<size_t>(kSelBins * sizeof(unsigned), (size_t)blocks * sizeof(unsigned long long)),
-                          (void**)&block_counts));
-    block_counts = reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(block_counts) + 256);
-    hipLaunchKernelGGL(rewire_kernel, dim3(blocks), dim3(kSelThreads), 0, s, lookup, w, list, n_arrays, count, num_features, threshold,
-                       seed, block_counts);
-    if (rewired != nullptr) hipLaunchKernelGGL(rewire_count_kernel, dim3(1), dim3(1024), 0, s, block_counts, blocks, rewired);
+    unsigned char* ws = nullptr;
+    FFI_TRY(zeroed_get(s, kWsSelect, kSelectBytes, (void**)&ws));
+    hipLaunchKernelGGL(rewire_kernel, dim3(stream_blocks(count)), dim3(kSelThreads), 0, s, lookup, w, list, n_arrays, count, num_features, threshold,
+                       seed, &reinterpret_cast<SelectState*>(ws)->rewired, rewired);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }

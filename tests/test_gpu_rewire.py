@@ -41,6 +41,21 @@ def test_threshold_is_the_kth_smallest_magnitude(ffi, n):
         assert thr.cpu().numpy()[0] == oracle.select_threshold(w, k), (n, k)
 
 
+@pytest.mark.parametrize("n", [1024, 32 * 2048, (1 << 21) + 17])
+def test_threshold_where_the_values_crowd(ffi, n):
+    # the list of the values that match the first digit: empty but for one, beyond a workgroup's share, beyond its own size, all values
+    rng = np.random.default_rng(n)
+    near = (1.0 + rng.random(n) * 0.06).astype(np.float32)               # one first digit (eighths of an octave)
+    for share in (0.0, 0.02, 0.04, 0.5, 1.0):
+        w = np.where(rng.random(n) < share, near, rng.normal(size=n).astype(np.float32) * 100.0).astype(np.float32)
+        w[0] = 1.03
+        wt = torch.from_numpy(w).cuda()
+        rank = int((np.abs(w) < 1.03).sum())
+        for k in (rank + 1, max(rank, 1), 1, n):
+            thr = ffi.fixed_fan_in_ops.select_threshold(wt, k)
+            assert thr.cpu().numpy()[0] == oracle.select_threshold(w, k), (n, share, k)
+
+
 def test_threshold_argument_errors(ffi):
     lib = ffi._lib.lib()
     w = torch.zeros(8, device="cuda")
