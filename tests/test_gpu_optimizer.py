@@ -225,3 +225,113 @@ def test_moments_are_rewired_in_place_or_through_an_override(ffi):
         results.append((layer.kernel_indices, layer.kernel_weights.detach(), m, v))
     assert layer.rewires_in_place() is False
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def _training(ffi, *, batch=20, features=40, labels=500, fan_in=6, loss=None, values=True, rewire=0, layer_class=None, ks=(1, 3, 5), optimizer=None):
+    gen = torch.Generator(device="cuda").manual_seed(batch + labels)
+    layer = (layer_class or ffi.StratifiedRewireLayerV2)(labels, features, connections=labels * fan_in, generator=gen,
+                                                         rewire_selector=ffi.FixedFractionSelector(0.1))
+    wrapper = ffi.SparseOptWrapper(rewire, layer)
+    adam = ffi.SparseAdam(layer.parameters(), learning_rate=0.01)
+    wrapper.compile(optimizer(layer, adam) if optimizer else adam, loss or ffi.SparseSquaredHingeLoss(), [ffi.PrecisionAtK(k) for k in ks])
+    x = torch.rand((batch, features), device="cuda", generator=gen)
+    flat = torch.randperm(batch * labels, device="cuda", generator=gen)[:3 * batch]
+    y = (torch.stack([flat // labels, flat % labels], dim=1), torch.rand(3 * batch, device="cuda", generator=gen) if values else None)
+    return wrapper, layer, adam, x, y
+
+
+def _after_steps(wrapper, layer, adam, x, y, steps=4):
+    results = [wrapper.train_step((x, y)) for _ in range(steps)]
+    state = [layer.kernel_weights.data, layer.bias.data, layer.kernel_weights.grad, layer.bias.grad, layer.kernel_indices, *adam._momentums, *adam._velocities]
+    return results, [t.clone() for t in state]
+
+
+@pytest.mark.parametrize("case", [dict(), dict(batch=1, labels=33, fan_in=3), dict(batch=129, features=1300, labels=700, fan_in=33), dict(values=False),
+                                  dict(batch=70, features=1217, labels=240_000, fan_in=1),        # (scores, gradients and ranks in one kernel)
+                                  dict(batch=64, labels=262_144, fan_in=4), dict(rewire=2), dict(rewire=2, layer_class="StratifiedRewireLayer"),
+                                  dict(loss="SparseBinaryCrossEntropyLoss"), dict(loss="SparseHingeLoss", ks=(8,)),
+                                  dict(optimizer=lambda layer, adam: [torch.optim.SGD([layer.bias], lr=0.1), adam])])
+def test_a_step_without_a_graph_is_the_step_with_one(ffi, case):
+    case = {**case, **({"loss": getattr(ffi, case["loss"])()} if "loss" in case else {})}
+    case = {**case, **({"layer_class": getattr(ffi, case["layer_class"])} if "layer_class" in case else {})}
+    direct, general = _training(ffi, **case), _training(ffi, **case)
+    assert direct[0]._steps_directly(direct[3])
+    seen = []
+    general[1].register_forward_hook(lambda *_: seen.append(1) and None)
+    got, want = _after_steps(*direct), _after_steps(*general)
+    assert len(seen) == 4
+    for a, b in zip(got[0], want[0]):
+        assert a.keys() == b.keys() and all(abs(a[key] - b[key]) <= 1e-6 * abs(b[key]) for key in a), (a, b)
+    one_kernel = case.get("batch", 20) * case.get("labels", 500) >= 1 << 24
+    for a, b in zip(got[1], want[1]):
+        assert torch.equal(a, b) or (one_kernel and rel_err(a.cpu().numpy(), b.cpu().numpy()) <= 1e-5)      # (sums in another order)
+
+
+def test_what_a_caller_put_into_a_step_still_runs(ffi):
+    calls = []
+    note = lambda *_: calls.append(1) and None
+
+    class OwnLoss(type(ffi.SparseSquaredHingeLoss())):
+        def __call__(self, y_true, y_pred):
+            calls.append(1)
+            return super().__call__(y_true, y_pred) * 2
+
+    class OwnLayer(ffi.StratifiedRewireLayerV2):
+        def forward(self, inputs):
+            calls.append(1)
+            return super().forward(inputs)
+
+    class OwnMetric(ffi.PrecisionAtK):
+        def update_state(self, y_true, y_pred, sample_weight=None):
+            calls.append(tuple(y_pred.shape))
+
+    def own_forward(wrapper, layer, x):
+        plain = layer.forward
+        layer.forward = lambda inputs: (calls.append(1), plain(inputs))[1]
+
+    puts = [lambda wrapper, layer, x: layer.register_forward_pre_hook(note), lambda wrapper, layer, x: layer.register_forward_hook(note),
+            lambda wrapper, layer, x: layer.register_full_backward_hook(note), lambda wrapper, layer, x: layer.kernel_weights.register_hook(note),
+            lambda wrapper, layer, x: layer.bias.register_post_accumulate_grad_hook(note), own_forward,
+            lambda wrapper, layer, x: wrapper.metrics.append(OwnMetric(1))]
+    for put in puts:
+        wrapper, layer, _, x, y = _training(ffi)
+        put(wrapper, layer, x)
+        calls.clear()
+        wrapper.train_step((x, y))
+        assert calls, put
+    for more in (dict(loss=OwnLoss()), dict(layer_class=OwnLayer)):
+        wrapper, _, _, x, y = _training(ffi, **more)
+        calls.clear()
+        wrapper.train_step((x, y))
+        assert calls, more
+    wrapper, _, _, x, y = _training(ffi)
+    calls.clear()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (calls.append(1), t)[1], lambda t: t):
+        wrapper.train_step((x, y))
+    assert calls
+    hook = torch.nn.modules.module.register_module_forward_hook(note)
+    try:
+        calls.clear()
+        wrapper.train_step((x, y))
+        assert calls
+    finally:
+        hook.remove()
+    # the gradient of the input, a variable that is held fixed, gradients that add up; what is refused
+    x.requires_grad_(True)
+    wrapper.train_step((x, y))
+    assert x.grad is not None
+    wrapper, layer, _, x, y = _training(ffi)
+    layer.bias.requires_grad_(False)
+    wrapper.train_step((x, y))
+    assert layer.bias.grad is None and not layer.bias.any()
+    wrapper, layer, adam, x, y = _training(ffi)
+    adam.zero_grad = lambda: None
+    wrapper.train_step((x, y))
+    first = layer.bias.grad.clone()
+    layer.bias.grad.fill_(1.0)
+    wrapper.train_step((x, y))
+    assert float((layer.bias.grad - 1.0).abs().max()) <= 10 * float(first.abs().max())
+    with pytest.raises(ValueError):
+        wrapper.train_step((x[:, 1:], y))
+    with pytest.raises(RuntimeError), torch.no_grad():
+        wrapper.train_step((x, y))
