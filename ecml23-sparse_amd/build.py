@@ -27,6 +27,7 @@ SOURCES = [
     "ffi_wide.hip",
     "ffi_sliced.hip",
     "ffi_small.hip",
+    "ffi_dense.hip",
     "ffi_topk.hip",
     "ffi_loss.hip",
     "ffi_sparse_grad.hip",

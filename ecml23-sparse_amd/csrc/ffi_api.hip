@@ -149,14 +149,15 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
         FFI_TRY(between(p));
         return launch_input_grad(p, weights, out_grad, feature_grad, d.B, d.tp, s, check);
     };
-    // small layers read the lookup itself: of a plan they need only that every id was found in range, so none is laid out for them.
+    // small layers and layers of few columns read the lookup itself: of a plan they need only that every id was found in range, so none is laid out for them.
     // (A rewiring and the pass behind it with a plan built for its check of the ids and without: 22 x 1,198 x 12,291 x 7 627 -> 206 us,
     // 17 x 64 x 10,000 x 4 301 -> 208.)
-    const bool small = takes_small_backward(d);
+    const bool dense = !takes_small_backward(d) && takes_dense_backward(d), small = dense || takes_small_backward(d);
     auto small_pass = [&]() -> int {
         unsigned long long* bad = nullptr;
         FFI_HIP_TRY(hipHostGetDevicePointer((void**)&bad, p->h_guard + kGuardHostBadIds, 0));
         if (wg.features == nullptr) FFI_TRY(between(p));       // (nothing, or a weight gradient formed without the plan)
+        if (dense) return launch_backward_dense(wg.features, lookup, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d, s, bad);
         return launch_backward_small(wg.features, lookup, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d, s, bad);
     };
     if (!small) FFI_TRY(backward_if_outdated_prepare(d, s));
@@ -659,6 +660,7 @@ int ffi_set_option(const char* name, int value) {
         {"plan_sorted_columns", &ffi::Options::plan_sorted_columns, -1, 1},
         {"small_path", &ffi::Options::small_path, -1, 1},
         {"wide_phases", &ffi::Options::wide_phases, -1, 1},
+        {"dense_rows", &ffi::Options::dense_rows, -1, 1},
     };
     for (const auto& t : table) {
         if (std::strcmp(name, t.name) != 0) continue;
@@ -688,7 +690,8 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
     if (check_dims(batch, num_features, num_units, fan_in, transposed, &d) != FFI_OK) return 0;
     const size_t B = (size_t)d.B, N = (size_t)d.N, L = (size_t)d.L, K = (size_t)d.K;
     const bool narrow = tile_path_fits(d.N) && d.L < (1 << 25);
-    const bool forward = (passes & FFI_PASS_FORWARD) && !takes_small_forward(d), small_backward = takes_small_backward(d);
+    const bool forward = (passes & FFI_PASS_FORWARD) && !takes_small_forward(d) && !takes_dense_forward(d);
+    const bool dense_backward = !takes_small_backward(d) && takes_dense_backward(d), small_backward = dense_backward || takes_small_backward(d);
     // a copy of the features (one slot, shared by the passes and by the permuted weights below): batch-major, or in slices
     size_t total = 0, partial_slot = 0, features_slot = 0;
     const bool copies = (forward && !few_samples(d)) || ((passes & FFI_PASS_BACKWARD) && !small_backward);
@@ -699,8 +702,9 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
         total += rows;
     }
     if (passes & FFI_PASS_BACKWARD) {
-        // small layers walk no plan: their ids are checked
-        if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
+        // small layers and layers of few columns walk no plan: their ids are checked
+        if (dense_backward) partial_slot = dense_backward_workspace(d), total += dense_backward_zeroed(d);
+        else if (small_backward) partial_slot = small_backward_workspace(d), total += kTicketCount * sizeof(unsigned);
         // what recomputes the gradients behind an outdated plan
         else if (backward_if_outdated_workspace(d) > 0) total += backward_if_outdated_workspace(d) + kTicketCount * sizeof(unsigned);
         const bool one_window = d.N <= 1024, two_windows = !one_window && tile_path_fits(d.N) && d.N <= 2048;

@@ -673,6 +673,7 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
 int launch_forward(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d,
                    hipStream_t s) {
     if (takes_small_forward(d)) return launch_forward_small(x, idx, w, bias, out, d, s);
+    if (takes_dense_forward(d)) return launch_forward_dense(x, idx, w, bias, out, d, s);
     // (the kernel reaches the 32 rows of out of a batch tile through 32-bit byte offsets)
     if (tile_path_fits(d.N) && d.L < (1 << 25) && !few_samples(d)) return forward_tiles(x, idx, w, bias, out, nullptr, kEpiScores, nullptr, nullptr, d, s);
     return launch_forward_wide(x, idx, w, bias, out, d, s);

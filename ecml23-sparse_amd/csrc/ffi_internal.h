@@ -32,6 +32,7 @@ struct Options {
     int workgroups_per_cu = 0;      // upper limit for the kernel that walks a tiled plan
     int wide_phases = 0;            // -1: never / 1: wherever it can: the forward kernel in phases for wide inputs
     int small_path = 0;             // -1: never / 1: wherever they can: the two launches for small layers
+    int dense_rows = 0;             // -1: never / 1: wherever they can: the kernels for few columns
     int plan_sorted_columns = 0;    // -1: never / 1: always (in the weights-in-LDS form) the plans that hand the columns to the walking kernel's threads tile by tile, by length
 };
 extern Options g_options;
@@ -67,7 +68,7 @@ private:
 
 // Library-owned device scratch, one buffer per (device, stream, slot), grown on demand and kept.
 // Work that uses a buffer is ordered by the stream it belongs to.
-enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11, kWsSums = 12, kWsSelect = 13 };
+enum WorkspaceSlot { kWsFeaturesT = 0, kWsPartials = 1, kWsSlots = 2, kWsLoss = 3, kWsNonzero = 4, kWsGradients = 5, kWsRewire = 6, kWsTopk = 7, kWsRows = 8, kWsWeightParts = 9, kWsHostWords = 10, kWsTickets = 11, kWsSums = 12, kWsSelect = 13, kWsDense = 14 };
 int workspace_get(hipStream_t s, int slot, size_t bytes, void** out);
 // 128 bytes of pinned host memory of the stream, for results that the host waits for
 int host_words_get(hipStream_t s, void** out);
@@ -142,6 +143,16 @@ struct TopkArgs {
 bool takes_small_forward(const Dims& d);
 bool takes_small_backward(const Dims& d);
 size_t small_backward_workspace(const Dims& d);
+
+// Few columns (ffi_dense.hip); the ids, and what is null, as for small layers.
+bool takes_dense_forward(const Dims& d);
+bool takes_dense_backward(const Dims& d);
+bool takes_dense_weight_grad(const Dims& d);
+size_t dense_backward_workspace(const Dims& d);
+size_t dense_backward_zeroed(const Dims& d);
+int launch_forward_dense(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s);
+int launch_backward_dense(const float* x, const int32_t* idx, const float* w, const float* g, float* gx, float* gw, float* gb, const Dims& d, hipStream_t s,
+                          unsigned long long* bad);
 int launch_forward_small(const float* x, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s);
 int launch_backward_small(const float* x, const int32_t* idx, const float* w, const float* g, float* gx, float* gw, float* gb, const Dims& d,
                           hipStream_t s, unsigned long long* bad);

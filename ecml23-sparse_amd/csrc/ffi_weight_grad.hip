@@ -575,6 +575,7 @@ bool three_units_cheaper(long long units, int N, int cus) {
 int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
                        hipStream_t s, const ffi_plan* plan) {
     if (takes_small_backward(d)) return launch_backward_small(x, idx, nullptr, g, nullptr, gw, bias_grad, d, s, nullptr);
+    if (plan == nullptr && takes_dense_weight_grad(d)) return launch_backward_dense(x, idx, nullptr, g, nullptr, gw, bias_grad, d, s, nullptr);
     // (32 rows of out_grad must be reachable through 32-bit byte offsets)
     if (tile_path_fits(d.N) && d.L < (1 << 25)) {
         const float* xT = x;

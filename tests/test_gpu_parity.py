@@ -879,7 +879,8 @@ def test_plan_layouts_serve_any_batch_size(ffi, shape):
                                    (160, 128, 40_000, 16, True), (300, 200, 40_000, 16, False),     # (several input-gradient workgroups per CU)
                                    (128, 768, 160_000, 32, True), (64, 1100, 200_000, 16, True),    # (plans that sort a tile's columns by length; two column windows)
                                    (96, 65_536, 40_000, 40, True), (20, 30_000, 200_000, 24, False), (3, 150_000, 20_000, 8, True),    # (forward in phases, several slices; short lists)
-                                   (17, 4000, 3000, 44, False), (8, 700, 9000, 24, False), (12, 600, 60_000, 8, False)])            # (small layers; few samples)
+                                   (17, 4000, 3000, 44, False), (8, 700, 9000, 24, False), (12, 600, 60_000, 8, False),
+                                   (100, 20, 90_000, 20, False), (30, 60, 90_000, 50, True)])            # (small layers; few samples; few columns)
 def test_workspace_estimate_brackets_what_the_library_holds(ffi, shape):
     # ffi_workspace_bytes() is asked before anything is allocated; ffi_cache_bytes() says what forward + backward then
     # hold (plans + workspaces).  The estimate models the padding of the plan for uniformly drawn ids.
