@@ -737,6 +737,7 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
                 partial_slot = std::max(partial_slot, streams * threads * nbt * 32 * 4);
             }
             if (tile_path_fits(d.N) && d.N < (1 << kArrIdBits)) total += arranged_words((long long)(L * ((K + 31) / 32))) * 2;   // idx16
+            total += weight_grad_parts_bytes(d);
         } else {
             const GlobalShape f = global_shape(d.N, d.K, d.L, d.B);
             const size_t sl = 256 / (size_t)f.members, padded = (B + sl - 1) / sl * sl, units = (size_t)f.segments * f.groups;

@@ -144,6 +144,8 @@ bool takes_small_forward(const Dims& d);
 bool takes_small_backward(const Dims& d);
 size_t small_backward_workspace(const Dims& d);
 
+// What a weight gradient over a plan keeps of partial sums (0: nothing).
+size_t weight_grad_parts_bytes(const Dims& d);
 // Few columns (ffi_dense.hip); the ids, and what is null, as for small layers.
 bool takes_dense_forward(const Dims& d);
 bool takes_dense_backward(const Dims& d);

@@ -29,6 +29,36 @@ constexpr int kWgChunk = 32;        // connections per unit
 constexpr int kResThreads = 512;
 constexpr int kResUnits = 4;        // units per thread
 
+// Where a launch has too few units to give every wavefront some, its workgroups take more units each and `tiles` of the batch tiles:
+// row y of the grid leaves its sums at y times `stride` floats (the weights' and the labels'), and sum_parts_kernel adds them up.
+struct BatchParts {
+    int tiles;
+    size_t stride;
+};
+
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ part, size_t stride, int parts, size_t weights, size_t bias_at,
+                                                        float* __restrict__ gw, float* __restrict__ bias_grad, int L) {
+    const size_t quads = bias_at / 4, total = quads + (bias_grad != nullptr ? (size_t)(L + 3) / 4 : 0);
+    const bool aligned = ((uintptr_t)gw & 15) == 0;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int q = 0; q < parts; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(part + q * stride + 4 * i);
+            sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+        }
+        const bool weight = i < quads;
+        float* const to = weight ? gw + 4 * i : bias_grad + 4 * (i - quads);
+        const size_t left = weight ? (weights > 4 * i ? weights - 4 * i : 0) : (size_t)L - 4 * (i - quads);
+        if (weight && aligned && left >= 4) {
+            *reinterpret_cast<float4*>(to) = sum;
+        } else {
+            const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+            for (size_t e = 0; e < 4 && e < left; ++e) to[e] = v[e];
+        }
+    }
+}
+
 template <bool VEC4>
 __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float* __restrict__ xT,
                                                                      const int32_t* __restrict__ idx,
@@ -36,14 +66,16 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
                                                                      float* __restrict__ gw,
                                                                      float* __restrict__ bias_grad, int B, int N,
                                                                      int L, int K, int nchunks, int n1, int upb1,
-                                                                     int upb2) {
+                                                                     int upb2, BatchParts parts) {
     extern __shared__ __align__(16) float xs[];
     const int lane = threadIdx.x & 63;
     const int blk = blockIdx.x;
     const long long total_units = (long long)L * nchunks;
     const long long u_begin = blk < n1 ? (long long)blk * upb1 : (long long)n1 * upb1 + (long long)(blk - n1) * upb2;
     const long long u_end = min(u_begin + (blk < n1 ? upb1 : upb2), total_units);
-    const int nbt = (B + kTileBatch - 1) / kTileBatch;
+    const int bt0 = blockIdx.y * parts.tiles, nbt = min(bt0 + parts.tiles, (B + kTileBatch - 1) / kTileBatch);
+    gw += blockIdx.y * parts.stride;
+    if (bias_grad != nullptr) bias_grad += blockIdx.y * parts.stride;
 
     float res[kResUnits][kWgChunk];
 #pragma unroll
@@ -54,7 +86,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
 #pragma unroll
     for (int q = 0; q < kResUnits; ++q) gsum[q] = 0.f;
 
-    for (int bt = 0; bt < nbt; ++bt) {
+    for (int bt = bt0; bt < nbt; ++bt) {
         const int b0 = bt * kTileBatch;
         __syncthreads();                                   // everyone is done with the previous tile
         stage_rows32<kResThreads, 8>(xs, xT, N, B, b0);
@@ -151,7 +183,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_arranged_kernel(const float
                                                                      float* __restrict__ gw,
                                                                      float* __restrict__ bias_grad, int B, int N,
                                                                      int L, int K, int nchunks, int n1, int ipb1,
-                                                                     int ipb2) {
+                                                                     int ipb2, BatchParts parts) {
     extern __shared__ __align__(16) float xs[];
     const int lane = threadIdx.x & 63;
     const int blk = blockIdx.x;
@@ -164,7 +196,9 @@ __global__ __launch_bounds__(kResThreads) void wgrad_arranged_kernel(const float
     const long long total_items = NCH == 1 ? (long long)L * nchunks : (long long)L;
     const long long i_begin = blk < n1 ? (long long)blk * ipb1 : (long long)n1 * ipb1 + (long long)(blk - n1) * ipb2;
     const long long i_end = min(i_begin + (blk < n1 ? ipb1 : ipb2), total_items);
-    const int nbt = (B + kTileBatch - 1) / kTileBatch;
+    const int bt0 = blockIdx.y * parts.tiles, nbt = min(bt0 + parts.tiles, (B + kTileBatch - 1) / kTileBatch);
+    gw += blockIdx.y * parts.stride;
+    if (bias_grad != nullptr) bias_grad += blockIdx.y * parts.stride;
 
     float res[UNITS][kWgChunk];
 #pragma unroll
@@ -175,7 +209,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_arranged_kernel(const float
 #pragma unroll
     for (int q = 0; q < kItems; ++q) gsum[q] = 0.f;
 
-    for (int bt = 0; bt < nbt; ++bt) {
+    for (int bt = bt0; bt < nbt; ++bt) {
         const int b0 = bt * kTileBatch;
         __syncthreads();                                   // everyone is done with the previous tile
         stage_rows32<kResThreads, 8>(xs, xT, N, B, b0);
@@ -319,7 +353,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* 
                                                                    float* __restrict__ gw,
                                                                    float* __restrict__ bias_grad, int B, int N,
                                                                    int L, int K, int nchunks, int n1, int ipb1,
-                                                                   int ipb2) {
+                                                                   int ipb2, BatchParts parts) {
     extern __shared__ __align__(16) float xs[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -330,7 +364,9 @@ __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* 
     const long long total_items = NCH == 1 ? (long long)L * nchunks : (long long)L;
     const long long i_begin = blk < n1 ? (long long)blk * ipb1 : (long long)n1 * ipb1 + (long long)(blk - n1) * ipb2;
     const long long i_end = min(i_begin + (blk < n1 ? ipb1 : ipb2), total_items);
-    const int nbt = (B + kTileBatch - 1) / kTileBatch;
+    const int bt0 = blockIdx.y * parts.tiles, nbt = min(bt0 + parts.tiles, (B + kTileBatch - 1) / kTileBatch);
+    gw += blockIdx.y * parts.stride;
+    if (bias_grad != nullptr) bias_grad += blockIdx.y * parts.stride;
 
     float res[UNITS][kWgChunk];
 #pragma unroll
@@ -390,14 +426,14 @@ __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* 
     };
     unsigned idn[kWgChunk / 2];                            // ids of the next chunk, in flight
     if (act[0]) {
-        const buffer_rsrc r0 = g_rows(0);
+        const buffer_rsrc r0 = g_rows(bt0);
         if constexpr (QUADS) static_for<kTileBatch / 4>([&](auto mc) { fetch_g_rows4(r0, (unsigned)__builtin_amdgcn_readfirstlane((int)jq[0]), mc); });
         else static_for<kTileBatch>([&](auto bc) { fetch_g_row(r0, jq[0], bc); });
 #pragma unroll
         for (int t = 0; t < kWgChunk / 8; ++t) fetch_ids_quarter(item[0], 0, t, idn);
     }
     const bool direct = (B % 4 == 0) && (N % 8 == 0) && (((uintptr_t)xT & 15) == 0);
-    for (int bt = 0; bt < nbt; ++bt) {
+    for (int bt = bt0; bt < nbt; ++bt) {
         const int b0 = bt * kTileBatch;
         __syncthreads();                                   // everyone is done with the previous tile
         if (direct && b0 + kTileBatch <= B) {
@@ -572,6 +608,82 @@ bool three_units_cheaper(long long units, int N, int cus) {
     return cost(3, 0.93) < 0.95 * cost(4, 1.0);
 }
 
+namespace {
+
+// How many rows of workgroups share the batch tiles, and how many CUs are a row's.  In units of a full round as above (8 us): a batch
+// tile costs a workgroup its staging and its rounds; the rows' sums cost a launch and their way to memory and back.  (One row: 419 x
+// 998 x 22,834 x 32 had 90 units in a workgroup of 512 threads, fourteen times behind 128 KB of staging.  Both passes, us: there 223 -> 153, 264 x
+// 1,042 x 1,146 x 104 290 -> 145, 512 x 1,200 x 2,000 x 120 391 -> 127, 500 x 300 x 5,000 x 60 232 -> 122; what the model puts above 0.85
+// went both ways.)
+struct BatchSplit {
+    int rows, tiles, cus;
+};
+BatchSplit batch_split(long long items, long long cap, double walks, const Dims& d, int cus) {
+    const int nbt = (d.B + kTileBatch - 1) / kTileBatch;
+    const double stage = 0.36 * (double)d.N / 768.0, sums = ((double)d.L * d.K + d.L) * 8.0 / 2.5e6 / 8.0;
+    auto cost = [&](int rows) {
+        const long long own = std::max(1, cus / rows), full = items / (cap * own), rest = items - full * cap * own;
+        double c = (double)full * (stage + (double)(cap / kResThreads) * walks);
+        if (rest > 0) {
+            const long long wgs = std::min<long long>(own, (rest + 63) / 64), per = (rest + wgs - 1) / wgs, last = per % kResThreads;
+            c += stage + walks * ((double)(per / kResThreads) + (last ? 0.33 + 0.084 * (double)((last + 63) / 64) : 0.0));
+        }
+        return c * ((nbt + rows - 1) / rows) + (rows > 1 ? 0.7 + rows * sums : 0.0);
+    };
+    BatchSplit best{1, nbt, cus};
+    double least = 0.85 * cost(1);                      // (the model is no better than that)
+    for (int rows = 2; rows <= std::min(nbt, 16); ++rows) {
+        const int tiles = (nbt + rows - 1) / rows;
+        if ((nbt + tiles - 1) / tiles != rows) continue;
+        const double c = cost(rows);
+        if (c < least) { least = c; best = BatchSplit{rows, tiles, std::max(1, cus / rows)}; }
+    }
+    return best;
+}
+
+size_t part_floats(const Dims& d) { return ((size_t)d.L * d.K + 63) / 64 * 64 + ((size_t)d.L + 63) / 64 * 64; }     // weights' sums, then the labels'
+
+// How a launch over a plan's arranged ids is made.
+struct ArrangedForm {
+    bool stream;          // the streaming kernel
+    int nch, units;       // chunks of a label in one thread (1: units are dealt one by one), units of a thread
+    int last_walk;        // connections in a label's last chunk, rounded up to the eights the walk is cut in
+    BatchSplit split;
+};
+ArrangedForm arranged_form(const Dims& d) {
+    ArrangedForm f;
+    const int nchunks = (d.K + kWgChunk - 1) / kWgChunk, cus = device_cu_count();
+    // with room for the wavefronts' out_grad slices behind the tile of x: the streaming kernel
+    // (and rows of out_grad of at least 256 bytes: the LDS-direct loads take their destination's offset inside the
+    // slice back out of the scalar offset of the row, which must not become negative)
+    f.stream = tile_lds_bytes(d.N) + (size_t)(kResThreads / 64) * kSliceFloats * sizeof(float) <= kLdsPerWorkgroup && d.L >= 64 && g_options.wgrad_stream >= 0;
+    f.last_walk = (d.K - (nchunks - 1) * kWgChunk + 7) / 8 * 8;
+    // (two chunks per label: one label per thread, 64 sums, measured 2-4 % under two labels per thread, whose 128 sums
+    // leave the streaming kernel 92 bytes of spills per lane)
+    if (nchunks == 2 || nchunks == 4) {
+        f.nch = nchunks;
+        f.units = nchunks == 2 && f.stream && g_options.wgrad_units != 4 ? 2 : 4;
+    } else {
+        // the streaming kernel: three units per thread wherever measured (4,000 to 3,000,000 labels, batch 32-512, 64-768
+        // columns, fan-in 8-32 and 96: 3-15 % under four units); the kernel without slices: by the model above
+        f.nch = 1;
+        f.units = g_options.wgrad_units == 3 ||
+                  (g_options.wgrad_units != 4 && (f.stream || three_units_cheaper((long long)d.L * nchunks, d.N, cus))) ? 3 : 4;
+    }
+    const bool short_walk = f.stream && (f.nch > 1 || nchunks == 1);
+    const double walks = f.nch - (short_walk ? 1.0 - f.last_walk / (double)kWgChunk : 0.0);
+    f.split = batch_split(f.nch == 1 ? (long long)d.L * nchunks : (long long)d.L, (long long)(f.units / f.nch) * kResThreads, walks, d, cus);
+    return f;
+}
+
+}  // namespace
+
+size_t weight_grad_parts_bytes(const Dims& d) {
+    if (!tile_path_fits(d.N) || d.N >= (1 << kArrIdBits) || d.L >= (1 << 25)) return 0;
+    const int rows = arranged_form(d).split.rows;
+    return rows > 1 ? rows * part_floats(d) * sizeof(float) : 0;
+}
+
 int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float* gw, float* bias_grad, const Dims& d,
                        hipStream_t s, const ffi_plan* plan) {
     if (takes_small_backward(d)) return launch_backward_small(x, idx, nullptr, g, nullptr, gw, bias_grad, d, s, nullptr);
@@ -589,41 +701,55 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
         // A first round of full workgroups (kResUnits units per thread), one per CU, as long as whole rounds
         // fit; what is left is shared evenly by a second set of workgroups in the same launch.
         const int nchunks = (d.K + kWgChunk - 1) / kWgChunk;
-        int n1 = 0, n2 = 0, ipb = 0, ipb2 = 0;
-        auto split = [&](long long items, long long cap) {             // cap: items a workgroup can hold
-            n1 = (int)(items / (cap * cus)) * cus;
+        int n1 = 0, n2 = 0, ipb = 0, ipb2 = 0, rows = 1;
+        BatchParts parts{1 << 26, 0};
+        float *to_w = gw, *to_b = bias_grad;
+        const size_t weights = (size_t)d.L * d.K, bias_at = (weights + 63) / 64 * 64;
+        auto split = [&](long long items, long long cap, const BatchSplit& b) -> int {      // cap: items a workgroup can hold
+            rows = b.rows;
+            n1 = (int)(items / (cap * b.cus)) * b.cus;
             const long long rest = items - (long long)n1 * cap;
             n2 = 0; ipb2 = 0;
             if (rest > 0) {
-                const long long rounds = (rest + cap * cus - 1) / (cap * cus);
-                n2 = (int)std::min<long long>(rounds * cus, (rest + 63) / 64);
+                const long long rounds = (rest + cap * b.cus - 1) / (cap * b.cus);
+                n2 = (int)std::min<long long>(rounds * b.cus, (rest + 63) / 64);
                 ipb2 = (int)((rest + n2 - 1) / n2);
                 n2 = (int)((rest + ipb2 - 1) / ipb2);
             }
             ipb = (int)cap;
+            if (rows == 1) return FFI_OK;
+            parts = BatchParts{b.tiles, part_floats(d)};
+            FFI_TRY(workspace_get(s, kWsWeightParts, parts.stride * rows * sizeof(float), (void**)&to_w));
+            if (bias_grad != nullptr) to_b = to_w + bias_at;
+            return FFI_OK;
+        };
+        auto sum_parts = [&]() -> int {
+            if (rows > 1) {
+                const size_t quads = bias_at / 4 + (size_t)(d.L + 3) / 4;
+                hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)std::min<size_t>((quads + 255) / 256, (size_t)cus * 8)), dim3(256), 0, s, to_w, parts.stride,
+                                   rows, weights, bias_at, gw, bias_grad, d.L);
+            }
+            FFI_HIP_TRY(hipGetLastError());
+            return FFI_OK;
         };
         if (plan != nullptr && plan->idx16 != nullptr) {
             // the unit slots of the final reordering need 144 bytes per thread
-            // with room for the wavefronts' out_grad slices behind the tile of x: the streaming kernel
-            // (and rows of out_grad of at least 256 bytes: the LDS-direct loads take their destination's offset inside the
-            // slice back out of the scalar offset of the row, which must not become negative)
-            const bool stream = tile_lds_bytes(d.N) + (size_t)(kResThreads / 64) * kSliceFloats * sizeof(float) <= kLdsPerWorkgroup &&
-                                d.L >= 64 && g_options.wgrad_stream >= 0;
+            const ArrangedForm form = arranged_form(d);
+            const bool stream = form.stream;
             const size_t lds = std::max(tile_lds_bytes(d.N) + (stream ? (size_t)(kResThreads / 64) * kSliceFloats * sizeof(float) : 0),
                                         (size_t)kResThreads * kSlotPitch * sizeof(float));
             // a label of two or four chunks: all its units in one thread (its out_grad values are loaded once per
             // batch tile instead of once per chunk); the work is then split by labels, not by units
-            // connections in a label's last chunk, rounded up to the eights the walk is cut in
-            const int last_walk = (d.K - (nchunks - 1) * kWgChunk + 7) / 8 * 8;
+            const int last_walk = form.last_walk;
 #define FFI_LAUNCH_STREAM_WALK(NCH, UNITS, WALK)                                                                                       \
             do {                                                                                                                       \
                 FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_stream_kernel<NCH, UNITS, true, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-                hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, true, WALK>), dim3((unsigned)(n1 + n2)), dim3(kResThreads), lds, s, xT, plan->idx16, g, gw, \
-                                   bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2);                                             \
+                hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, true, WALK>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
+                                   to_b, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2, parts);                                          \
             } while (0)
 #define FFI_LAUNCH_ARRANGED(NCH, UNITS)                                                                                                \
             do {                                                                                                                       \
-                split(NCH == 1 ? (long long)d.L * nchunks : (long long)d.L, (long long)(UNITS / NCH) * kResThreads);                   \
+                FFI_TRY(split(NCH == 1 ? (long long)d.L * nchunks : (long long)d.L, (long long)(UNITS / NCH) * kResThreads, form.split)); \
                 if (stream) {                                                                                                          \
                     constexpr bool kQuads = NCH > 1;   /* a wavefront's lanes hold consecutive labels */                               \
                     if ((kQuads || nchunks == 1) && last_walk < kWgChunk) {                                                            \
@@ -633,48 +759,41 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
                         else FFI_LAUNCH_STREAM_WALK(NCH, UNITS, 24);                                                                   \
                     } else if (kQuads || nchunks == 1) {                                                                               \
                         FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_stream_kernel<NCH, UNITS, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-                        hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, true>), dim3((unsigned)(n1 + n2)), dim3(kResThreads), lds, s, xT, plan->idx16, g, gw, \
-                                           bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2);                                     \
+                        hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, true>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
+                                           to_b, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2, parts);                                  \
                     } else {                                                                                                           \
                         FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_stream_kernel<NCH, UNITS, kQuads>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-                        hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, kQuads>), dim3((unsigned)(n1 + n2)), dim3(kResThreads), lds, s, xT, plan->idx16, g, gw, \
-                                           bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2);                                     \
+                        hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, kQuads>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
+                                           to_b, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2, parts);                                  \
                     }                                                                                                                  \
                 } else {                                                                                                               \
                     FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_arranged_kernel<NCH, UNITS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-                    hipLaunchKernelGGL((wgrad_arranged_kernel<NCH, UNITS>), dim3((unsigned)(n1 + n2)), dim3(kResThreads), lds, s, xT, plan->idx16, g, gw, \
-                                       bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2);                                         \
+                    hipLaunchKernelGGL((wgrad_arranged_kernel<NCH, UNITS>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
+                                       to_b, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2, parts);                                      \
                 }                                                                                                                      \
             } while (0)
-            // (two chunks per label: one label per thread, 64 sums, measured 2-4 % under two labels per thread, whose 128 sums
-            // leave the streaming kernel 92 bytes of spills per lane)
-            if (nchunks == 2 && (g_options.wgrad_units == 4 || !stream)) FFI_LAUNCH_ARRANGED(2, 4);
-            else if (nchunks == 2) FFI_LAUNCH_ARRANGED(2, 2);
-            else if (nchunks == 4) FFI_LAUNCH_ARRANGED(4, 4);
-            // the streaming kernel: three units per thread wherever measured (4,000 to 3,000,000 labels, batch 32-512, 64-768
-            // columns, fan-in 8-32 and 96: 3-15 % under four units); the kernel without slices: by the model above
-            else if (g_options.wgrad_units == 3 ||
-                     (g_options.wgrad_units != 4 && (stream || three_units_cheaper((long long)d.L * nchunks, d.N, cus)))) FFI_LAUNCH_ARRANGED(1, 3);
+            if (form.nch == 2 && form.units == 4) FFI_LAUNCH_ARRANGED(2, 4);
+            else if (form.nch == 2) FFI_LAUNCH_ARRANGED(2, 2);
+            else if (form.nch == 4) FFI_LAUNCH_ARRANGED(4, 4);
+            else if (form.units == 3) FFI_LAUNCH_ARRANGED(1, 3);
             else FFI_LAUNCH_ARRANGED(1, 4);
 #undef FFI_LAUNCH_ARRANGED
 #undef FFI_LAUNCH_STREAM_WALK
-            FFI_HIP_TRY(hipGetLastError());
-            return FFI_OK;
+            return sum_parts();
         }
-        split((long long)d.L * nchunks, (long long)kResUnits * kResThreads);
+        FFI_TRY(split((long long)d.L * nchunks, (long long)kResUnits * kResThreads, batch_split((long long)d.L * nchunks, (long long)kResUnits * kResThreads, 1.0, d, cus)));
         const unsigned blocks = (unsigned)(n1 + n2);
         const int upb = ipb, upb2 = ipb2;
         const size_t lds = tile_lds_bytes(d.N);
         const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx) % 16 == 0);
         if (vec4) {
             FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<true>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2);
+            hipLaunchKernelGGL(wgrad_resident_kernel<true>, dim3(blocks, (unsigned)rows), dim3(kResThreads), lds, s, xT, idx, g, to_w, to_b, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, parts);
         } else {
             FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<false>, dim3(blocks), dim3(kResThreads), lds, s, xT, idx, g, gw, bias_grad, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2);
+            hipLaunchKernelGGL(wgrad_resident_kernel<false>, dim3(blocks, (unsigned)rows), dim3(kResThreads), lds, s, xT, idx, g, to_w, to_b, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, parts);
         }
-        FFI_HIP_TRY(hipGetLastError());
-        return FFI_OK;
+        return sum_parts();
     }
     return launch_weight_grad_wide(x, idx, g, gw, bias_grad, d, s);
 }

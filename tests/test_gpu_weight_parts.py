@@ -1,0 +1,39 @@
+"""Weight gradients of few labels and many samples, whose sums come from several rows of workgroups, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from conftest import load_package, reference_law_inputs, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+# (B, N, L, K): one, two, three and four chunks of connections with full and part-filled last ones; rows whose share of the batch tiles
+# is uneven or ends within a tile; sizes off four; inputs with and without room for the streaming kernel's slices
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("shape", [(264, 1042, 1146, 104), (419, 998, 2283, 32), (500, 300, 1301, 61), (512, 1200, 601, 120), (333, 768, 4097, 33), (200, 80, 1500, 70),
+                                   (161, 700, 90, 128), (225, 900, 5003, 7)])
+def test_gradients_of_few_labels(shape, transposed):
+    ffi = load_package()
+    lib = ffi._lib.lib()
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=L)
+    xt = np.ascontiguousarray(x.T if transposed else x)
+    ref_gx, ref_gw = oracle.backward(xt, lookup, w, g, transposed=transposed)
+    ref_gb = g.astype(np.float64).sum(0)
+    dx, dl, dw, dg = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (xt, lookup, w, g))
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        for need_x in (True, False):                       # (over a plan and from the lookup itself)
+            gx, gb = torch.full_like(dx, float("nan")), torch.full((L,), float("nan"), device="cuda")
+            storage = torch.full((L * K + 1,), float("nan"), device="cuda")
+            for gw in (storage[:-1], storage[1:]):         # (at sixteen bytes and off them)
+                for _ in range(2):
+                    ffi._lib.check(lib.ffi_backward_bias_f32(dx.data_ptr(), dl.data_ptr(), dw.data_ptr(), dg.data_ptr(), gx.data_ptr() if need_x else None,
+                                                             gw.data_ptr(), gb.data_ptr(), B, N, L, K, int(transposed), stream))
+                    assert rel_err(gw.cpu().numpy().reshape(L, K), ref_gw) <= 1e-5 and rel_err(gb.cpu().numpy(), ref_gb) <= 1e-5
+            assert not need_x or rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5
+    finally:
+        assert lib.ffi_set_option(b"small_path", 0) == 0
