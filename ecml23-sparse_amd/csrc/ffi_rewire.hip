@@ -19,13 +19,34 @@ namespace {
 constexpr int kSelThreads = 1024;
 constexpr int kSelBins = 2048;
 
-// Zero between selections but for `prefix` and `k`, which each pass leaves for the next.
+// Read-modify-writes of one address take turns, some 10 ns each where their results are waited for: 512 workgroups that draw from
+// one counter are 5 us.  So they draw from one of eight, each on a line of its own, and who draws last there draws from the last.
+// Zero between launches.
+constexpr int kDrawWays = 8;
+struct Draw {
+    struct __attribute__((aligned(64))) Way { unsigned long long n; } way[kDrawWays + 1];
+};
+// Adds `v`, below 2^40, of a workgroup (of the `parts` that call this, one thread each) to the others'; true in the one that comes last,
+// which has the sum, and all that the others' had waited for before is done then.
+__device__ __forceinline__ bool draw_last(Draw* d, unsigned parts, unsigned long long v, unsigned long long* sum) {
+    constexpr unsigned long long one = 1ull << 40;
+    const unsigned way = blockIdx.x % kDrawWays, of_way = (parts - way + kDrawWays - 1) / kDrawWays;
+    unsigned long long all = __hip_atomic_fetch_add(&d->way[way].n, v + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v + one;
+    if (all >> 40 != of_way) return false;
+    __hip_atomic_store(&d->way[way].n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = all & (one - 1ull);
+    all = __hip_atomic_fetch_add(&d->way[kDrawWays].n, v + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v + one;
+    if (all >> 40 != min(parts, (unsigned)kDrawWays)) return false;
+    __hip_atomic_store(&d->way[kDrawWays].n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *sum = all & (one - 1ull);
+    return true;
+}
+
+// `prefix` and `k` are what each pass leaves for the next.
 struct SelectState {
+    Draw draw;
     unsigned prefix;              // digits found so far (the high bits of the answer)
-    unsigned ticket;
     unsigned long long k;         // rank still to find among the values matching the prefix (1-based)
-    unsigned long long listed;    // values that match the first digit: those in the list, or more than it holds
-    unsigned long long rewired;   // rewire_kernel: connections changed, and the workgroups that have said so << 40
 };
 
 __device__ __forceinline__ unsigned magnitude_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
@@ -35,66 +56,74 @@ __device__ __forceinline__ unsigned magnitude_bits(float v) { return __float_as_
 // the histogram, side by side in the banks, and the workgroups add to kHistTotals totals.  (21 M normal values: 58 us in one
 // copy, 31 in four or eight that all go to one total, 25 so; the second pass, which few values match, 18, what it takes to
 // read them.)
-// The second pass also puts the values that match the first digit in a list, and the third reads the list instead of all values
-// where they fitted into it, which takes values that crowd within an eighth of an octave to fail.  The workgroup that adds its
-// bins last picks the bin in which the cumulative count reaches k, appends it to the prefix, reduces k by the count of the bins
+// The second pass also lists the values that match the first digit, a workgroup's in a piece of its own, and the third reads the lists
+// instead of all values where they all fitted, which takes values that crowd within an eighth of an octave to fail.  The workgroup
+// that adds its bins last picks the bin in which the cumulative count reaches k, appends it to the prefix, reduces k by the count of the bins
 // below it and clears the bins: all read-modify-writes at device scope whose results are waited for before the ticket is drawn.
-// (A launch for each pick and one to clear, and all values read in the third pass: 81 us in seven launches, 62 so in three; 12,291 x 7: 187 us of a rewiring and its pass against 206.)
-constexpr int kHistThreads = 1024, kHistCopies = 4, kHistTotals = 8, kSelLocalList = 2048;
+// (A launch for each pick and one to clear, and all values read in the third pass: 81 us in seven launches, 56 so in three; 3.5 M 29 and 32, in four launches fewer.)
+constexpr int kHistThreads = 1024, kHistCopies = 4, kHistTotals = 8, kSelLocalList = 2048, kListParts = 32;
+// lists: [n_lists] counts, then n_lists pieces of kSelLocalList values (n_lists: workgroups of the second pass, at most kHistThreads)
 template <int PASS>
 __global__ __launch_bounds__(kHistThreads) void select_pass_kernel(const float* __restrict__ w, size_t count, unsigned long long k0,
                                                                     SelectState* __restrict__ state, unsigned* __restrict__ hist,
-                                                                    unsigned* __restrict__ list, unsigned long long capacity, float* __restrict__ threshold) {
+                                                                    unsigned* __restrict__ lists, int n_lists, float* __restrict__ threshold) {
     constexpr int kShift = PASS == 0 ? 20 : PASS == 1 ? 9 : 0, kBits = PASS == 2 ? 9 : 11, kEach = kSelBins / kHistThreads;
     constexpr unsigned kMask = (1u << kBits) - 1u;
     __shared__ __align__(16) unsigned local[kSelBins * kHistCopies];
     __shared__ unsigned mine[PASS == 1 ? kSelLocalList : 1], n_mine, is_last;
-    __shared__ unsigned long long list_at;
     const unsigned prefix = PASS == 0 ? 0u : state->prefix, copy = threadIdx.x % kHistCopies;
-    const bool from_list = PASS == 2 && state->listed <= capacity;
-    const size_t n = from_list ? (size_t)state->listed : count;
-    // (a list has work for few workgroups: the others leave, and no ticket is expected of them)
-    const unsigned parts = from_list ? (unsigned)min((size_t)gridDim.x, max((n + kHistThreads - 1) / kHistThreads, (size_t)1)) : gridDim.x;
+    bool from_lists = false;
+    if (PASS == 2) from_lists = !__syncthreads_or((int)threadIdx.x < n_lists && lists[threadIdx.x] > (unsigned)kSelLocalList);
+    // (lists have work for few workgroups: the others leave, and no ticket is expected of them)
+    const unsigned parts = from_lists ? min(gridDim.x, (unsigned)kListParts) : gridDim.x;
     if (blockIdx.x >= parts) return;
     for (int i = threadIdx.x; i < kSelBins * kHistCopies; i += kHistThreads) local[i] = 0;
     if (threadIdx.x == 0) n_mine = 0u;
     __syncthreads();
-    constexpr int kTogether = 4;                                          // values asked for together
-    constexpr unsigned kNone = ~0u;                                       // (no magnitude)
-    const size_t stride = (size_t)parts * kHistThreads;
-    for (size_t i0 = (size_t)blockIdx.x * kHistThreads + threadIdx.x; i0 < n; i0 += kTogether * stride) {
-        unsigned keys[kTogether];
-#pragma unroll
-        for (int u = 0; u < kTogether; ++u) {
-            const size_t i = min(i0 + u * stride, n - 1);
-            const unsigned key = from_list ? list[i] : magnitude_bits(w[i]);
-            keys[u] = i0 + u * stride < n ? key : kNone;
+    auto add = [&](unsigned key) { atomicAdd(&local[((key >> kShift) & kMask) * kHistCopies + copy], 1u); };
+    if (from_lists) {
+        const int lane = threadIdx.x & 63;
+        for (int q = blockIdx.x + (int)parts * (threadIdx.x >> 6); q < n_lists; q += (int)parts * (kHistThreads / 64)) {
+            const unsigned n = lists[q];
+            const unsigned* from = lists + n_lists + (size_t)q * kSelLocalList;
+            for (unsigned i = lane; i < n; i += 64)
+                if (from[i] >> kBits == prefix) add(from[i]);
         }
+    } else {
+        constexpr int kTogether = 4;                                      // values asked for together
+        constexpr unsigned kNone = ~0u;                                   // (no magnitude)
+        const size_t stride = (size_t)gridDim.x * kHistThreads;
+        for (size_t i0 = (size_t)blockIdx.x * kHistThreads + threadIdx.x; i0 < count; i0 += kTogether * stride) {
+            unsigned keys[kTogether];
 #pragma unroll
-        for (int u = 0; u < kTogether; ++u) {
-            const unsigned key = keys[u];
-            const bool match = key != kNone && (PASS == 0 || (key >> (kShift + kBits)) == prefix);
-            if (match) atomicAdd(&local[((key >> kShift) & kMask) * kHistCopies + copy], 1u);
-            if (PASS == 1) {
-                const unsigned long long matches = __ballot(match);
-                if (matches != 0ull) {                                        // (one add of a wavefront)
-                    const int lane = threadIdx.x & 63, first = __ffsll((long long)matches) - 1;
-                    unsigned at = 0;
-                    if (lane == first) at = atomicAdd(&n_mine, (unsigned)__popcll(matches));
-                    at = (unsigned)__builtin_amdgcn_readlane((int)at, first) + (unsigned)__popcll(matches & ((1ull << lane) - 1ull));
-                    if (match && at < (unsigned)kSelLocalList) mine[at] = key;
+            for (int u = 0; u < kTogether; ++u) {
+                const size_t i = i0 + u * stride;
+                const unsigned key = magnitude_bits(w[min(i, count - 1)]);
+                keys[u] = i < count ? key : kNone;
+            }
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) {
+                const unsigned key = keys[u];
+                const bool match = key != kNone && (PASS == 0 || (key >> (kShift + kBits)) == prefix);
+                if (match) add(key);
+                if (PASS == 1) {
+                    const unsigned long long matches = __ballot(match);
+                    if (matches != 0ull) {                                // (one add of a wavefront)
+                        const int lane = threadIdx.x & 63, first = __ffsll((long long)matches) - 1;
+                        unsigned at = 0;
+                        if (lane == first) at = atomicAdd(&n_mine, (unsigned)__popcll(matches));
+                        at = (unsigned)__builtin_amdgcn_readlane((int)at, first) + (unsigned)__popcll(matches & ((1ull << lane) - 1ull));
+                        if (match && at < (unsigned)kSelLocalList) mine[at] = key;
+                    }
                 }
             }
         }
     }
     __syncthreads();
     if (PASS == 1) {
-        if (threadIdx.x == 0)
-            list_at = n_mine ? __hip_atomic_fetch_add(&state->listed, n_mine > (unsigned)kSelLocalList ? capacity + 1ull : (unsigned long long)n_mine, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-        __syncthreads();
-        for (unsigned i = threadIdx.x; i < min(n_mine, (unsigned)kSelLocalList); i += kHistThreads)
-            if (list_at + i < capacity) list[list_at + i] = mine[i];
+        if (threadIdx.x == 0) lists[blockIdx.x] = n_mine;
+        unsigned* const to = lists + n_lists + (size_t)blockIdx.x * kSelLocalList;
+        for (unsigned i = threadIdx.x; i < min(n_mine, (unsigned)kSelLocalList); i += kHistThreads) to[i] = mine[i];
     }
     unsigned old = 0;
     for (int i = threadIdx.x; i < kSelBins; i += kHistThreads) {
@@ -108,7 +137,10 @@ __global__ __launch_bounds__(kHistThreads) void select_pass_kernel(const float* 
     }
     asm volatile("" :: "v"(old));                                         // (the adds have returned)
     __syncthreads();
-    if (threadIdx.x == 0) is_last = __hip_atomic_fetch_add(&state->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1u;
+    if (threadIdx.x == 0) {
+        unsigned long long none;
+        is_last = draw_last(&state->draw, parts, 0ull, &none);
+    }
     __syncthreads();
     if (!is_last) return;
     // (walked by one thread, 2,048 bins took 22 us, all of it latency)
@@ -145,10 +177,6 @@ __global__ __launch_bounds__(kHistThreads) void select_pass_kernel(const float* 
         state->k = k - below;
         if (PASS == 2) *threshold = __uint_as_float(value);
     }
-    if (threadIdx.x == 0) {
-        state->ticket = 0u;
-        if (PASS == 2) state->listed = 0ull;
-    }
 }
 
 __global__ void select_none_kernel(float* threshold) { *threshold = 0.f; }    // nothing is below 0 in magnitude: an empty selection
@@ -169,7 +197,7 @@ struct ArrayList {
 __global__ __launch_bounds__(kSelThreads) void rewire_kernel(int32_t* __restrict__ lookup, const float* __restrict__ w,
                                                               ArrayList arrays, int n_arrays, size_t count,
                                                               unsigned num_features, const float* __restrict__ threshold,
-                                                              unsigned long long seed, unsigned long long* __restrict__ counted,
+                                                              unsigned long long seed, Draw* __restrict__ counted,
                                                               long long* __restrict__ rewired) {
     __shared__ unsigned red[kSelThreads / 64];
     const float thr = *threshold;
@@ -189,18 +217,13 @@ __global__ __launch_bounds__(kSelThreads) void rewire_kernel(int32_t* __restrict
     if (threadIdx.x == 0) {
         unsigned long long t = 0;
         for (int i = 0; i < kSelThreads / 64; ++i) t += red[i];
-        // (fewer than 2^40 connections and 2^24 workgroups; who adds last has the sum.  Adds to one address take turns: of 2,048
-        // workgroups of 256 threads they were 12 us of the kernel's 49, so it has 512 of 1,024.)
-        const unsigned long long one = 1ull << 40, all = __hip_atomic_fetch_add(counted, t + one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + t + one;
-        if (all >> 40 == gridDim.x) {
-            if (rewired != nullptr) *rewired = (long long)(all & (one - 1ull));
-            __hip_atomic_store(counted, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        unsigned long long all;
+        if (draw_last(counted, gridDim.x, t, &all) && rewired != nullptr) *rewired = (long long)all;
     }
 }
 
-constexpr size_t kSelectBytes = 256 + kSelBins * kHistTotals * sizeof(unsigned);     // the state, then the bins
-static_assert(sizeof(SelectState) <= 256, "the bins lie behind it");
+constexpr size_t kSelectHead = 1024, kSelectBytes = kSelectHead + kSelBins * kHistTotals * sizeof(unsigned);     // the state, then the bins
+static_assert(sizeof(SelectState) <= kSelectHead, "the bins lie behind it");
 
 int stream_blocks(size_t count) {
     return (int)std::max<size_t>(1, std::min<size_t>((count + kSelThreads - 1) / kSelThreads, (size_t)device_cu_count() * 2));
@@ -216,14 +239,13 @@ int launch_select_threshold(const float* w, size_t count, unsigned long long k, 
     }
     unsigned char* ws = nullptr;
     FFI_TRY(zeroed_get(s, kWsSelect, kSelectBytes, (void**)&ws));
-    const size_t capacity = std::max<size_t>(count / 32, 1024);
-    unsigned* list = nullptr;
-    FFI_TRY(workspace_get(s, kWsRewire, capacity * sizeof(unsigned), (void**)&list));
     SelectState* state = reinterpret_cast<SelectState*>(ws);
-    unsigned* hist = reinterpret_cast<unsigned*>(ws + 256);
-    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((count + kHistThreads - 1) / kHistThreads, (size_t)device_cu_count() * 2));
+    unsigned* hist = reinterpret_cast<unsigned*>(ws + kSelectHead);
+    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>({(count + kHistThreads - 1) / kHistThreads, (size_t)device_cu_count() * 2, (size_t)kHistThreads}));
+    unsigned* lists = nullptr;
+    FFI_TRY(workspace_get(s, kWsRewire, (size_t)blocks * (1 + kSelLocalList) * sizeof(unsigned), (void**)&lists));
     for (const auto pass : {select_pass_kernel<0>, select_pass_kernel<1>, select_pass_kernel<2>})
-        hipLaunchKernelGGL(pass, dim3(blocks), dim3(kHistThreads), 0, s, w, count, k, state, hist, list, (unsigned long long)capacity, threshold);
+        hipLaunchKernelGGL(pass, dim3(blocks), dim3(kHistThreads), 0, s, w, count, k, state, hist, lists, (int)blocks, threshold);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
@@ -235,7 +257,7 @@ int launch_rewire(int32_t* lookup, const float* w, float* const* arrays, int n_a
     unsigned char* ws = nullptr;
     FFI_TRY(zeroed_get(s, kWsSelect, kSelectBytes, (void**)&ws));
     hipLaunchKernelGGL(rewire_kernel, dim3(stream_blocks(count)), dim3(kSelThreads), 0, s, lookup, w, list, n_arrays, count, num_features, threshold,
-                       seed, &reinterpret_cast<SelectState*>(ws)->rewired, rewired);
+                       seed, &reinterpret_cast<SelectState*>(ws)->draw, rewired);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
