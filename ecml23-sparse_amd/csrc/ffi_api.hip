@@ -143,6 +143,7 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     ffi_plan* p = find_cached_plan(lookup, d, dev);
     auto passes = [&](const LookupCheck* check) -> int {
+        FFI_TRY(plan_wait_built(p, s));
         // (the global form's walk has both operands of a connection at hand: one walk for both gradients)
         if (!p->tiled && wg.features != nullptr)
             return launch_backward_wide(p, wg.features, weights, out_grad, feature_grad, wg.weight_grad, wg.bias_grad, d.B, d.tp, s, check);
@@ -541,6 +542,11 @@ int ffi_rewire_f32(int32_t* lookup, const float* weights, float* const* arrays, 
                          (unsigned long long)seed, (long long*)rewired_count, (hipStream_t)stream);
 }
 
+static int wait_for(hipStream_t s) {
+    FFI_HIP_TRY(hipStreamSynchronize(s));
+    return FFI_OK;
+}
+
 int ffi_plan_create(const int32_t* lookup, int64_t num_units, int64_t fan_in, int64_t num_features,
                     int64_t batch_hint, ffi_stream_t stream, ffi_plan** plan) {
     StreamCall call_lock((hipStream_t)stream);
@@ -552,6 +558,7 @@ int ffi_plan_create(const int32_t* lookup, int64_t num_units, int64_t fan_in, in
     FFI_TRY(plan_alloc(d.L, d.K, d.N, &p));
     p->batch_hint = batch_hint > 0 ? d.B : 0;
     int st = plan_build(p, lookup, (hipStream_t)stream);
+    if (st == FFI_OK) st = wait_for((hipStream_t)stream);            // (the caller's own plan: complete when it is handed out)
     if (st != FFI_OK) { plan_free(p); delete p; return st; }
     *plan = p;
     return FFI_OK;
@@ -563,7 +570,8 @@ int ffi_plan_refresh(ffi_plan* plan, const int32_t* lookup, ffi_stream_t stream)
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     if (dev != plan->device) return FFI_ERR_BAD_ARGUMENT;
-    return plan_build(plan, lookup, (hipStream_t)stream);
+    FFI_TRY(plan_build(plan, lookup, (hipStream_t)stream));
+    return wait_for((hipStream_t)stream);
 }
 
 int ffi_plan_destroy(ffi_plan* plan) {
@@ -595,6 +603,7 @@ int ffi_input_grad_planned_f32(const ffi_plan* plan, const float* weights, const
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return FFI_ERR_NO_DEVICE;
     if (dev != plan->device) return FFI_ERR_BAD_ARGUMENT;
+    FFI_TRY(plan_wait_built(plan, (hipStream_t)stream));
     return launch_input_grad(plan, weights, out_grad, feature_grad, (int)batch, transposed != 0, (hipStream_t)stream);
 }
 
@@ -608,6 +617,7 @@ int ffi_weight_grad_planned_f32(const ffi_plan* plan, const float* features, con
     if (dev != plan->device) return FFI_ERR_BAD_ARGUMENT;
     Dims d;
     FFI_TRY(check_dims(batch, plan->N, plan->L, plan->K, transposed, &d));
+    FFI_TRY(plan_wait_built(plan, (hipStream_t)stream));
     return launch_weight_grad(features, lookup, out_grad, weight_grad, nullptr, d, (hipStream_t)stream, plan);
 }
 
@@ -728,6 +738,7 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
                 const size_t slots = tiles * slices * rows * 64;
                 total += slots * 2 * 2 + (tiles * slices + 1) * 4 + L * 2;              // 4 bytes per slot (lab16 + pos16, or slot32), slice_off, rowpos
                 if (sorted) total += tiles * threads * 2;                               // the column of each thread in each tile
+                partial_slot = std::max(partial_slot, (tiles * threads + tiles * slices) * 4);      // counts while the plan is built
                 if (!w_in_lds) features_slot = std::max(features_slot, slots * 4);     // weights in slot order
                 const size_t nbt = (B + 31) / 32;
                 const size_t per_cu = (size_t)tiled_workgroups_per_cu((int)threads, (int)TL, d.K, w_in_lds, (int)((B + 31) / 32));

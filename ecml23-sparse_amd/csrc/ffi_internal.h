@@ -3,6 +3,7 @@
 #define FFI_INTERNAL_H
 
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdint>
 #include <cstddef>
 #include <vector>
@@ -327,6 +328,8 @@ struct ffi_plan {
     unsigned short* tile_pos = nullptr;  // [L * K]
     unsigned long long* d_scratch = nullptr;  // counters of the build, fingerprint partial sums (device)
     unsigned long long* h_scratch = nullptr;  // pinned mirror
+    hipEvent_t built = nullptr;               // recorded behind the kernels that lay the plan out
+    mutable std::atomic<bool> built_pending{false};   // nobody has seen that event done yet (plan_wait_built)
     hipEvent_t fp_done = nullptr;             // recorded behind the fingerprint kernel and its copy to h_scratch
     int fp_blocks = 0;                        // workgroups of the fingerprint kernel in flight: that many pairs of partial sums
     // Check of the lookup's content on the device, without a host wait (plan_guard_*): device words
@@ -417,6 +420,8 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 }
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
+// Makes `s` wait for the kernels that lay the plan out, where they may still be running.
+int plan_wait_built(const ffi_plan* p, hipStream_t s);
 int plan_check_ids(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
 // How the global form of a lookup is cut (`batch`: the batch size it is built for, 0 = unknown).

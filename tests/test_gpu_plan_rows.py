@@ -33,3 +33,30 @@ def test_any_fan_in(fan_in, features, labels, skewed):
         assert rel_err(gx.cpu().numpy(), oracle.input_grad(x, lookup, w, g, transposed=False)) <= 1e-5
     finally:
         ffi._lib.check(lib.ffi_plan_destroy(plan))
+
+
+@pytest.mark.parametrize("features", [768, 1100, 5000])
+def test_a_plan_that_is_being_laid_out_serves_other_streams(features):
+    # the call that builds the plan does not wait for it: calls on other streams come right behind, and the next edit too
+    ffi = load_package()
+    B, L, K = 40, 60_000, 16
+    x, lookup, w, g = reference_law_inputs(B, features, L, K, seed=features)
+    dx, dw, dg = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, w, g))
+    shifted = [((lookup + 11 * turn) % features).astype(np.int32) for turn in range(3)]
+    on_device = [torch.from_numpy(a).cuda() for a in shifted]
+    dl = torch.empty_like(on_device[0])
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    ffi._lib.check(ffi._lib.lib().ffi_cache_clear())
+    for turn in range(3):
+        torch.cuda.synchronize()
+        dl.copy_(on_device[turn])
+        ffi._lib.check(ffi._lib.lib().ffi_lookup_edited(dl.data_ptr()))
+        torch.cuda.synchronize()
+        results = []
+        for i in range(6):
+            with torch.cuda.stream(streams[(turn + i) % 3]):
+                results.append(ffi.fan_in_sparse_matmul_grad(dx, dl, dw, dg))
+        torch.cuda.synchronize()
+        ref_gx, ref_gw = oracle.backward(x, shifted[turn], w, g, transposed=False)
+        for gx, gw in results:
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-5
