@@ -1107,9 +1107,10 @@ int make_table(const void* x, const Dims& d, hipStream_t s, const void** table) 
     return launch_slices((const float*)x, (float*)ws, d.N, d.B, f.sl, d.tp, s);
 }
 
+// (`like`, where not 0: the number of labels whose kernel is taken -- a label's score is then the same number)
 template <bool BF16>
 int forward_wide(const void* table, const int32_t* idx, const void* w, const float* bias, float* out, const TopkSink& sink, const Dims& d,
-                 hipStream_t s, int row_step = 1) {
+                 hipStream_t s, int row_step = 1, int like = 0) {
     const SlicedForm f = sliced_form<BF16>(d.B, d.N);
     const size_t slice_bytes = (size_t)d.N * f.gl * 16;
     const bool quads = d.K % 4 == 0 && ((uintptr_t)idx & 15) == 0 && ((uintptr_t)w & (BF16 ? 7 : 15)) == 0;
@@ -1122,7 +1123,7 @@ int forward_wide(const void* table, const int32_t* idx, const void* w, const flo
             default: return launch_fwd_lds<8, BF16>(a, d, s);
         }
     }
-    if (takes_phases(slice_bytes, f.gl, f.slices, d.L, d.K, BF16 ? 2 : 4)) return launch_fwd_phased<BF16>(a, d, s);
+    if (takes_phases(slice_bytes, f.gl, f.slices, like > 0 ? like : d.L, d.K, BF16 ? 2 : 4)) return launch_fwd_phased<BF16>(a, d, s);
     return launch_fwd_sliced_lanes<BF16>(f.gl, a, d, s);
 }
 
@@ -1159,7 +1160,10 @@ bool few_samples(const Dims& d) { return d.B <= 16; }
 // ---- top-k without the scores -------------------------------------------------------------------------------------
 namespace {
 
-constexpr int kTopkSampleLabels = 16384;
+// Every step-th label is in the sample: a sixteenth, whose threshold some 16 k labels reach, but some 2,000 labels at least and 16,384 at
+// most.  (16,384 labels of every layer and so, us for the pass: 200 x 30,000 x 30,000 x 30 fp32 128 and 86, 512 x 700 x 20,000 x 30 bf16 86 and 69,
+// 8 x 48,006 x 80,864 x 76 fp32 76 and 72, 20 x 349 x 38,198 x 19 bf16 30 and 29.)
+constexpr int kTopkSampleMost = 16384, kTopkSampleLeast = 2048, kTopkSampleStep = 16;
 
 // the rows of every step-th label
 template <typename T>
@@ -1180,7 +1184,7 @@ __global__ __launch_bounds__(256) void sample_rows_kernel(const int32_t* __restr
 template <bool BF16>
 int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, const TopkArgs& tk, const Dims& d, hipStream_t s) {
     using T = typename LaneAcc<BF16>::Element;
-    const int step = std::max(1, d.L / kTopkSampleLabels), S = std::min(d.L, (d.L + step - 1) / step);
+    const int step = std::max({1, d.L / kTopkSampleMost, std::min(kTopkSampleStep, d.L / kTopkSampleLeast)}), S = std::min(d.L, (d.L + step - 1) / step);
     const size_t rows = (size_t)S * d.K, rows_bytes = (rows * (4 + sizeof(T)) + (size_t)S * 4 + 32) / 16 * 16;
     const bool in_lds = sliced_form<BF16>(d.B, d.N).in_lds;
     unsigned char* ws = nullptr;
@@ -1191,7 +1195,7 @@ int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const 
     Dims ds = d;
     ds.L = S;
     if (in_lds) {
-        FFI_TRY(forward_wide<BF16>(table, idx, w, bias, c.sample, TopkSink{}, ds, s, step));
+        FFI_TRY(forward_wide<BF16>(table, idx, w, bias, c.sample, TopkSink{}, ds, s, step, d.L));
     } else {
         int32_t* sample_idx = reinterpret_cast<int32_t*>(ws + (topk_candidate_bytes(d.B, S) + 15) / 16 * 16);
         T* sample_w = reinterpret_cast<T*>(sample_idx + (rows + 3) / 4 * 4);
@@ -1199,7 +1203,7 @@ int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const 
         hipLaunchKernelGGL(sample_rows_kernel<T>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, idx, (const T*)w, bias, sample_idx,
                            sample_w, sample_bias, step, d.K, S);
         FFI_HIP_TRY(hipGetLastError());
-        FFI_TRY(forward_wide<BF16>(table, sample_idx, sample_w, bias ? sample_bias : nullptr, c.sample, TopkSink{}, ds, s));
+        FFI_TRY(forward_wide<BF16>(table, sample_idx, sample_w, bias ? sample_bias : nullptr, c.sample, TopkSink{}, ds, s, 1, d.L));
     }
     FFI_TRY(launch_topk_threshold(c.sample, (size_t)S, 1, S, TopkSampleLabels{step, 0}, tk.k, c, d.B, s));
     FFI_TRY(forward_wide<BF16>(table, idx, w, bias, nullptr, TopkSink{c.tau, c.tie, c.count, c.val, c.idx, kTopkCap}, d, s));

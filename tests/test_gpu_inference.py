@@ -293,3 +293,25 @@ def test_inference_config_full_size(ffi):
     assert rel_err(got, oracle.forward(xs, ls, ws, transposed=True)) <= SAME_INPUT_RTOL
     x32 = t["features"].cpu().numpy()
     assert rel_err(got, oracle.forward(x32, ls, t["weights"][sl].cpu().numpy(), transposed=True)) <= FP32_INPUT_RTOL
+
+
+# a sample of every 2nd to 18th label; wide inputs whose whole layer goes in phases and whose sample alone would not; few samples, some
+# rows of equal scores
+@pytest.mark.parametrize("shape", [(70, 60_000, 50_000, 20), (200, 30_000, 4_099, 12), (40, 131_072, 33_000, 30), (9, 40_000, 70_001, 9), (20, 349, 38_198, 19), (12, 700, 300_000, 6)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_topk_from_a_sample_of_few_labels(ffi, shape, bf16):
+    B, N, L, K = shape
+    gen = torch.Generator(device="cuda").manual_seed(L)
+    x = torch.relu(torch.randn((B, N), generator=gen, device="cuda"))
+    x[B // 2] = 0.0
+    lookup = torch.randint(0, N, (L, K), generator=gen, device="cuda", dtype=torch.int32)
+    w = torch.randn((L, K), generator=gen, device="cuda")
+    for k in (1, 8):
+        if bf16:
+            values, labels = ffi.fan_in_sparse_topk_bf16(x.bfloat16(), lookup, w.bfloat16(), k=k)
+            scores = ffi.fan_in_sparse_matmul_bf16(x.bfloat16(), lookup, w.bfloat16())
+        else:
+            values, labels = ffi.fan_in_sparse_topk(x, lookup, w, k=k)
+            _, _, scores = ffi.fan_in_sparse_topk(x, lookup, w, k=k, want_scores=True)
+        ref_v, ref_i = oracle.topk(scores.cpu().numpy(), k)
+        assert np.array_equal(labels.cpu().numpy(), ref_i) and np.array_equal(values.cpu().numpy(), ref_v), k
