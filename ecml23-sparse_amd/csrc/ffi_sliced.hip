@@ -778,16 +778,21 @@ __global__ __launch_bounds__(256) void rows_by_range_kernel(const int32_t* __res
 
 // ---- forward in phases --------------------------------------------------------------------------------------------
 // For slices that do not fit an XCD's L2: a workgroup takes 88 M labels -- their sums stay in registers -- and goes through the
-// parts of their rows (above: one oct of connections per label and part) in order, a barrier behind each.  All workgroups of
+// parts of their rows (above: one oct of connections per label and part) in order, the first quads of all labels and then the second, a
+// barrier behind either.  All workgroups of
 // an XCD begin at the same time and do the same work, so the gathers of a phase hit the few MB of the slice that its part of
 // the rows names.
 //
 // One wavefront brings the lists of all others, two parts ahead and past the registers; the others have nothing but gathers in
 // flight.  Loads return in order, and lists that each wavefront asked for itself held its gathers up for the time of the fabric
 // once a phase (with their lines marked for one use, which takes longer, the pass went from 2.1 to 2.9 ms).  The gathers of a
-// step (eight labels, an oct each) are issued before the sums of the step before them, so that a wavefront always has eight in
+// step (sixteen labels, a quad each) are issued before the sums of the step before them, so that a wavefront always has eight in
 // flight.  Twelve wavefronts and not sixteen: with 168 registers the sums of 704 labels fit a workgroup, and a slice is gone
 // through less often (misses of L2 77 -> 60 M lines in bf16).
+//
+// A phase of quads, of rows ordered by twice as many ranges as they have octs, names a narrower part of the slice than one of octs
+// and one range an oct, and L2 holds more of it: top-5 of 512 samples, 100,000 columns, 670,091 labels of fan-in 64 in bf16 2,258 -> 2,227 us,
+// scores of 64 samples, 131,072 columns, 300,000 labels of fan-in 40 166 -> 159, of 190, 60,791, 157,519 and 20 154 -> 153.
 //
 // What bounds it: the L1, whose address side is busy 89 % of the time in bf16 and 92 in fp32, its data side 96.  670,091 labels,
 // against sixteen wavefronts that bring their own lists, 512 labels: 128 samples, 65,536 columns, fan-in 72 in fp32 1,215 -> 1,145 us
@@ -845,6 +850,7 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
         pace();
         for (int r = 0; r < octs; ++r) {
             if (r + 2 < octs) bring(r + 2);
+            pace();                                                                     // (behind the first quads)
             __builtin_amdgcn_s_waitcnt(0x0f70);
             pace();
         }
@@ -866,19 +872,24 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
     // (entries of no connection hold ~0: behind the slice's end, where a load returns zero without touching memory)
     auto gather = [&](int r, int m, uint4 (&xs)[8], unsigned (&wv)[kWt]) {
         const unsigned char* part = smem + (size_t)(r % S::kBuffers) * S::kPartBytes;
-        const int label = wave * S::kWaveLabels + m * 8 + grp;
-        const uint4* ids = reinterpret_cast<const uint4*>(part + label * 32);
-        const uint4* ws = reinterpret_cast<const uint4*>(part + S::kIdBytes + label * (kWt * 4));
+        const int label = wave * S::kWaveLabels + 2 * (m % (M / 2)) * 8 + grp, half = m / (M / 2);
 #pragma unroll
-        for (int v = 0; v < kWt / 4; ++v) {
-            const uint4 e = ws[v];
-            wv[4 * v] = e.x; wv[4 * v + 1] = e.y; wv[4 * v + 2] = e.z; wv[4 * v + 3] = e.w;
+        for (int p = 0; p < 2; ++p) {
+            const uint4* ids = reinterpret_cast<const uint4*>(part + (label + 8 * p) * 32);
+            const unsigned char* ws = part + S::kIdBytes + (label + 8 * p) * (kWt * 4);
+            if (BF16) {
+                const uint2 e = reinterpret_cast<const uint2*>(ws)[half];
+                wv[2 * p] = e.x; wv[2 * p + 1] = e.y;
+            } else {
+                const uint4 e = reinterpret_cast<const uint4*>(ws)[half];
+                wv[kWt / 2 * p] = e.x; wv[kWt / 2 * p + 1] = e.y; wv[kWt / 2 * p + 2] = e.z; wv[kWt / 2 * p + 3] = e.w;
+            }
+            const uint4 a = ids[half];
+            const unsigned at[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                xs[4 * p + v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, at[v] * kRow + lane_off, 0, 0));
         }
-        const uint4 a = ids[0], b = ids[1];
-        const unsigned at[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int v = 0; v < 8; ++v)
-            xs[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, at[v] * kRow + lane_off, 0, 0));
     };
     pace();
     gather(0, 0, x[0], wt[0]);
@@ -889,8 +900,9 @@ __global__ __launch_bounds__(kPhThreads) void fwd_phased_kernel(const void* __re
             else gather(min(r + 1, octs - 1), 0, x[(m + 1) & 1], wt[(m + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[m].add_pair(x[m & 1][2 * v], x[m & 1][2 * v + 1], &wt[m & 1][v * (kWt / 4)]);
+            for (int v = 0; v < 4; ++v) acc[2 * (m % (M / 2)) + v / 2].add_pair(x[m & 1][2 * v], x[m & 1][2 * v + 1], &wt[m & 1][v * (kWt / 4)]);
             __builtin_amdgcn_sched_barrier(0);
+            if (m == M / 2 - 1) pace();
         }
         pace();
     }
@@ -1026,7 +1038,7 @@ int phased_labels(int L, int slices);
 
 template <bool BF16>
 int launch_fwd_phased(const FwdSliced& a, const Dims& d, hipStream_t s) {
-    const int octs = (d.K + 7) / 8, ranges = std::min(kMaxRanges, octs);
+    const int octs = (d.K + 7) / 8, ranges = std::min(kMaxRanges, 2 * octs);
     unsigned* rows = nullptr;
     FFI_TRY(workspace_get(s, kWsRows, phased_rows_bytes<BF16>(d.L, d.K), (void**)&rows));
     void* row_w = rows + (size_t)d.L * octs * 8;
