@@ -289,9 +289,11 @@ __global__ __launch_bounds__(256) void tile_color_kernel(const int32_t* __restri
     // What bounds the kernel is the chain from one step's adds to the next step's decision: an LDS round trip, the sum over the
     // lanes by DPP and lane swaps, a comparison in every lane, some 60 instructions of one wavefront.  Labels decided together do not see
     // what the others of the step just did.  In the first sweep that is mended by the second: eight a step.  In the second it stays: two
-    // (one beyond a fan-in of 32).  Slot rows per connection, 582-label tiles of fan-in 32 over 768 columns: 1.5267 with two in both, 1.5279 so,
+    // (one beyond a fan-in of 64).  Slot rows per connection, 582-label tiles of fan-in 32 over 768 columns: 1.5267 with two in both, 1.5279 so,
     // 1.5309 with four in the second; sorted columns 1.1542, 1.1549, 1.1559.  670,091 labels of fan-in 32 196 -> 126 us,
-    // 14 of them ids asked for twelve at a time; 131,072 labels a whole build 248 -> 195, 50,000 of fan-in 100 897 -> 517.  (The first sweep by
+    // 14 of them ids asked for twelve at a time; 131,072 labels a whole build 248 -> 195, 50,000 of fan-in 100 897 -> 517.  Fan-ins of 33 to 64, two against one in the second: 1.3290
+    // and 1.3269 (512 labels of 64 over 512 columns), 1.1888 and 1.1888 (567 of 38 over 584, sorted); builds at 501,070 x 64 and
+    // 181,536 x 38 609 -> 503 us and 187 -> 125.  (The first sweep by
     // four wavefronts, a quarter of the labels each, and their sums put together: 1.5347, 1.1586.)
     int placed[2] = {0, 0};
     const TileLabels labels{imb, ids3, wt, half, nl, K, W, ncols, cap};
@@ -1154,7 +1156,7 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     if (!dev_alloc(p, &p->rowpos, (size_t)p->L)) return FFI_ERR_OUT_OF_MEMORY;
     {
         const size_t lds = ((size_t)threads + 1) * sizeof(int) + (size_t)TL * ((p->K + 2) / 3) * sizeof(unsigned) + (size_t)threads + 1 + (size_t)TL + kPastLabels;
-        const auto color = p->K <= 32 ? tile_color_kernel<32, 1, false> : p->K <= 64 ? tile_color_kernel<64, 1, false>
+        const auto color = p->K <= 32 ? tile_color_kernel<32, 1, false> : p->K <= 64 ? tile_color_kernel<32, 2, false>
                                     : p->K <= 128 ? tile_color_kernel<64, 2, false> : tile_color_kernel<64, 2, true>;
         hipError_t ea = hipFuncSetAttribute((const void*)color, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (ea != hipSuccess) return hip_fail(ea);
