@@ -167,6 +167,7 @@ int launch_forward_topk(const float* x, const int32_t* idx, const float* w, cons
                         const Dims& d, hipStream_t s);
 // Top-k by a threshold (ffi_topk.hip): scores of a sample of the labels, the threshold of every sample of the batch, and the
 // candidates that reach it.  In a workspace of topk_candidate_bytes.
+constexpr int kTopkShortRow = 65536;    // rows of scores up to here are scanned without a threshold
 constexpr int kTopkCap = 8192;          // candidate slots per sample
 constexpr int kTopkCountStep = 32;      // ints between the samples' counters: a cache line each
 struct TopkCandidates {

@@ -1191,10 +1191,29 @@ __global__ __launch_bounds__(256) void sample_rows_kernel(const int32_t* __restr
     if (bias != nullptr && t == i * K) bias_out[i] = bias[j];
 }
 
+// Few scores in short rows: written out and scanned.  The threshold costs the sample's pass, its own launch and a list of candidates
+// that many labels of a short row reach; the scan reads each score once (10 MB at most, out of the caches) in two launches.  us for the
+// pass by threshold and by scan: 1 x 40,000 x 10,000 x 90 fp32 65 and 36, 16 x 2,000 x 10,000 x 90 bf16 57 and 35, 128 x 2,000 x 10,000 x 90
+// fp32 97 and 54, 40 x 2,000 x 65,000 x 40 bf16 50 and 43.  From some four million scores on, or in longer rows, which launch_topk_f32 itself
+// takes by a threshold, the scores' way through memory costs more: 128 x 30,000 labels bf16 up to 17 % slower, 12 x 300,000 x 6 32 and 38.
+constexpr long long kTopkFewScores = 5LL << 19;
+
+inline bool topk_scans_scores(const Dims& d) {
+    return d.L <= kTopkShortRow && (long long)d.B * d.L <= kTopkFewScores && d.B <= 65535;      // (a row of the scan's grid for every sample)
+}
+
 // The k-th best of a sample of the labels is a threshold that k labels reach; the same kernel scores the sample and all
 // labels, so that a label's score is the same number in both.
 template <bool BF16>
 int forward_topk_sliced(const void* x, const int32_t* idx, const void* w, const float* bias, const TopkArgs& tk, const Dims& d, hipStream_t s) {
+    if (topk_scans_scores(d)) {
+        float* scores = nullptr;
+        const void* table = nullptr;
+        FFI_TRY(workspace_get(s, kWsTopk, (size_t)d.B * d.L * sizeof(float), (void**)&scores));
+        FFI_TRY(make_table<BF16>(x, d, s, &table));
+        FFI_TRY(forward_wide<BF16>(table, idx, w, bias, scores, TopkSink{}, d, s));
+        return launch_topk_f32(scores, d.B, d.L, tk.k, tk.values, tk.indices, s);      // (its lists lie in a slot of their own)
+    }
     using T = typename LaneAcc<BF16>::Element;
     const int step = std::max({1, d.L / kTopkSampleMost, std::min(kTopkSampleStep, d.L / kTopkSampleLeast)}), S = std::min(d.L, (d.L + step - 1) / step);
     const size_t rows = (size_t)S * d.K, rows_bytes = (rows * (4 + sizeof(T)) + (size_t)S * 4 + 32) / 16 * 16;

@@ -745,7 +745,7 @@ int launch_topk_f32(const float* scores, int B, int L, int k, float* values, int
     const int per = (L + splits - 1) / splits;
     splits = (L + per - 1) / per;
     const TopkArgs tk{k, values, indices};
-    if (L <= 16 * kTopkRowSample) {
+    if (L <= kTopkShortRow) {
         // rows too short to be worth a threshold: every thread keeps a list, the wavefronts reduce them
         const int entries = splits * 4 * kTopMax;
         char* part = nullptr;

@@ -315,3 +315,37 @@ def test_topk_from_a_sample_of_few_labels(ffi, shape, bf16):
             _, _, scores = ffi.fan_in_sparse_topk(x, lookup, w, k=k, want_scores=True)
         ref_v, ref_i = oracle.topk(scores.cpu().numpy(), k)
         assert np.array_equal(labels.cpu().numpy(), ref_i) and np.array_equal(values.cpu().numpy(), ref_v), k
+
+
+# rows that are scored and scanned, the last shape of each side of the rule among them: 65,536 and 65,537 labels, 2,621,440 scores and a
+# few more, more samples than a grid's rows; NaN (no score), rows of one score and of -inf (fewer labels than k, too: empty places)
+@pytest.mark.parametrize("shape", [(5, 40_000, 65_536, 4), (5, 40_000, 65_537, 4), (40, 2_000, 65_536, 3), (640, 3_000, 4_096, 5), (641, 3_000, 4_096, 5),
+                                   (9, 1_217, 3, 2), (65_536, 40, 30, 3), (5, 70_000, 20_001, 33)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_topk_of_rows_that_are_scanned(ffi, shape, bf16):
+    B, N, L, K = shape
+    gen = torch.Generator(device="cuda").manual_seed(L + B)
+    x = torch.relu(torch.randn((B, N), generator=gen, device="cuda"))
+    lookup = torch.randint(0, N, (L, K), generator=gen, device="cuda", dtype=torch.int32)
+    w = torch.randn((L, K), generator=gen, device="cuda")
+    x[1] = 0.0
+    x[2] = float("nan")
+    w[0] = float("nan")                                                # label 0 has no score in any row
+    if bf16:
+        x, w = x.bfloat16(), w.bfloat16()
+    k = min(8, L)
+    topk, layer = (ffi.fan_in_sparse_topk_bf16, ffi.fan_in_sparse_matmul_bf16) if bf16 else (ffi.fan_in_sparse_topk, ffi.fan_in_sparse_matmul)
+    values, labels = (t.cpu().numpy() for t in topk(x, lookup, w, k=k))
+    scores = layer(x, lookup, w).cpu().numpy()
+    rows = np.r_[0:1, 3:B]
+    rows = rows if B <= 1000 else rows[:: len(rows) // 500]
+    clean = np.where(np.isnan(scores), -np.inf, scores)                # (label 0: below every finite score)
+    places = min(k, L - 1)
+    ref_v, ref_i = oracle.topk(clean[rows], places)
+    assert np.array_equal(labels[rows][:, :places], ref_i)
+    picked = np.take_along_axis(scores[rows], ref_i.astype(np.int64), axis=1)
+    assert np.array_equal(values[rows][:, :places], picked) or rel_err(values[rows][:, :places], ref_v) <= SAME_INPUT_RTOL
+    assert np.array_equal(labels[1][:places], np.arange(1, places + 1)) and not values[1][:places].any()      # a row of one score: ids ascend
+    assert (labels[2] == -1).all() and (values[2] == -np.inf).all()
+    if places < k:
+        assert (labels[rows][:, places:] == -1).all()
