@@ -1174,7 +1174,7 @@ namespace {
 
 // Every step-th label is in the sample: a sixteenth, whose threshold some 16 k labels reach, but some 2,000 labels at least and 16,384 at
 // most.  (16,384 labels of every layer and so, us for the pass: 200 x 30,000 x 30,000 x 30 fp32 128 and 86, 512 x 700 x 20,000 x 30 bf16 86 and 69,
-// 8 x 48,006 x 80,864 x 76 fp32 76 and 72, 20 x 349 x 38,198 x 19 bf16 30 and 29.)
+// 8 x 48,006 x 80,864 x 76 fp32 76 and 72.)
 constexpr int kTopkSampleMost = 16384, kTopkSampleLeast = 2048, kTopkSampleStep = 16;
 
 // the rows of every step-th label
