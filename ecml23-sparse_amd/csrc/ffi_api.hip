@@ -187,6 +187,12 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     LookupCheck check;
     FFI_TRY(plan_guard_begin(p, lookup, s, &check));
     FFI_TRY(passes(&check));
+    if (takes_outdated_wide(p, d)) {
+        // (the walk's slices of out_grad lie at the front of their slot; nothing has used it since)
+        float* slices = nullptr;
+        FFI_TRY(workspace_get(s, kWsPartials, (size_t)d.L * sizeof(float), (void**)&slices));
+        return launch_outdated_wide(p, wg.features, lookup, weights, slices, feature_grad, wg.weight_grad, d, s);
+    }
     return launch_backward_if_outdated(p->d_guard + kGuardVerdict, wg.features, lookup, weights, out_grad, feature_grad,
                                        wg.weight_grad, wg.bias_grad, d, !p->tiled && wg.features != nullptr, s);
 }

@@ -3,8 +3,8 @@
 // device-side check of the lookup (ffi_check.h) found that the cached plan is outdated -- the one call after an
 // in-place rewiring (sparse/custom_layer.py:32-43) -- and return at once otherwise.  Semantics:
 // tfsparse/cc/kernels/backward.cpp:8-36 (weight gradient) and :39-73 (input gradient).  Ids outside [0, num_features) are
-// skipped.  Narrow inputs take one kernel for both gradients; others plain ones whose input gradient scatters with float
-// atomics, as the reference's GPU kernels do (backward.cu.h:119,139,161,182).
+// skipped.  Narrow inputs take one kernel for both gradients and so do wide ones; few samples of many columns, and fan-ins beyond the LDS, plain
+// ones whose input gradient scatters with float atomics, as the reference's GPU kernels do (backward.cu.h:119,139,161,182).
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
 
@@ -304,6 +304,178 @@ __global__ __launch_bounds__(kRedoThreads) void redo_backward_kernel(const RedoA
     }
 }
 
+// ---- wide inputs: both gradients in one kernel ---------------------------------------------------------------------
+// An item is a range of columns and a slice of the samples, whose rows of the features and of their gradient lie in LDS.  Its workgroup reads
+// all ids, 32 a thread and step, keeps those of its columns in short lists, a list for every wavefront's ids, and every wavefront takes
+// the connections of its own columns (every sixteenth) from all lists: the lanes are the samples, so that no add meets another one.  A
+// connection's row of out_grad comes from the slices that the passes over the plan left in their slot; eight are fetched at once.
+// Bound by the steps of 32,768 ids, some 15 us each: what 16 wavefronts pick out of the lists, two barriers and a round trip for rows.
+// One thread a connection, its samples one by one and its input gradient by atomics in memory (the kernel above), the whole call at
+// 128 x 65,536 x 670,091 x 72: 313 ms, 47 so (16 ids a thread, all eight rows fetched also where fewer are left: 64); at
+// 50 x 32,768 x 670,000 x 32 51 and 10.7, at 128 x 1,300 x 100,000 x 32 14.9 and 2.9.
+constexpr int kOutIds = 32, kOutWaves = 16, kOutThreads = 64 * kOutWaves, kOutList = 256, kOutFetch = 8;
+constexpr int kOutTile = 16384;                // floats of a tile
+constexpr unsigned kOutStep = kOutIds * kOutThreads, kOutNone = ~0u;
+typedef int i32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
+
+struct OutdatedWide {
+    const unsigned long long* verdict;
+    const float *x, *w, *g;                    // g: slices [slice][L][sl]
+    const int32_t* idx;
+    float *gx, *gw;                            // gw (may be null, and x with it): zeros where the verdict is 0
+    int B, N, L, K, sl, slices, cols, ranges;
+    unsigned inverse_k;                        // 2^32 / K, and one more
+};
+
+template <bool TP>
+__global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const OutdatedWide a) {
+    if (*a.verdict != 0) return;
+    extern __shared__ __align__(16) float out_mem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float* const gxt = out_mem;
+    float* const xt = out_mem + a.cols * a.sl;
+    unsigned* const list = reinterpret_cast<unsigned*>(xt + a.cols * a.sl);
+    int* const len = reinterpret_cast<int*>(list + kOutWaves * kOutList);
+    const unsigned total = (unsigned)a.L * (unsigned)a.K;
+    for (int item = blockIdx.x; item < a.ranges * a.slices; item += gridDim.x) {
+        const int slice = item / a.ranges, c0 = (item - slice * a.ranges) * a.cols, ncols = min(a.cols, a.N - c0);
+        if (ncols <= 0) continue;
+        const int b0 = slice * a.sl, nb = min(a.sl, a.B - b0);
+        auto cell = [&](int n, int b) { return TP ? (size_t)(c0 + n) * a.B + b0 + b : (size_t)(b0 + b) * a.N + c0 + n; };
+        auto each = [&](auto f) {              // every column and sample of the item, side by side as they lie in memory
+            const int inner = TP ? a.sl : ncols, count = ncols * a.sl;
+            for (int e = threadIdx.x; e < count; e += kOutThreads) {
+                const int outer = e / inner, in = e - outer * inner;
+                f(TP ? outer : in, TP ? in : outer);
+            }
+        };
+        __syncthreads();                       // (the item before this one)
+        each([&](int n, int b) {
+            gxt[n * a.sl + b] = 0.f;
+            xt[n * a.sl + b] = a.gw != nullptr && b < nb ? a.x[cell(n, b)] : 0.f;
+        });
+        const float* const rows = a.g + (size_t)slice * a.L * a.sl + min(lane, a.sl - 1);
+        int ids[kOutIds], next[kOutIds];
+        auto fetch = [&](unsigned first, int (&v)[kOutIds]) {
+#pragma unroll
+            for (int q = 0; q < kOutIds / 4; ++q) {
+                const unsigned at = first + (unsigned)wave * (64u * kOutIds) + (unsigned)q * 256u + (unsigned)lane * 4u;
+                if (at + 4u <= total) {
+                    const i32x4_unaligned four = *reinterpret_cast<const i32x4_unaligned*>(a.idx + at);
+                    v[4 * q] = four.x; v[4 * q + 1] = four.y; v[4 * q + 2] = four.z; v[4 * q + 3] = four.w;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[4 * q + i] = at + i < total ? a.idx[at + i] : -1;
+                }
+            }
+        };
+        fetch(0, ids);
+        __syncthreads();
+        for (unsigned first = 0; first < total; first += kOutStep) {
+            if (first + kOutStep < total) fetch(first + kOutStep, next);
+            int from = 0;
+            bool more;
+            do {
+                // a list takes the ids of four rows at least; what it has no room for goes into the next round
+                int n = 0, to = from;
+#pragma unroll
+                for (int u = 0; u < kOutIds; ++u) {
+                    if (u < from || n > kOutList - 64) continue;
+                    const unsigned col = (unsigned)ids[u] - (unsigned)c0;
+                    const bool hit = ids[u] >= 0 && col < (unsigned)ncols;
+                    const unsigned long long hits = __ballot(hit);
+                    to = u + 1;
+                    if (hits == 0) continue;
+                    const int at = n + __builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0));
+                    if (hit) list[wave * kOutList + at] = col << 15 | (unsigned)wave << 11 | (unsigned)((u >> 2) * 256 + lane * 4 + (u & 3));
+                    n += (int)__popcll(hits);
+                }
+                from = to;
+                if (lane == 0) len[wave] = n;
+                more = __syncthreads_or(from < kOutIds) != 0;
+                // sixteen entries of every list at a time
+                for (int t = 0;; t += 16) {
+                    unsigned e[4];
+                    unsigned long long mine[4];
+                    bool left = false;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int l = i * 4 + (lane >> 4), at = t + (lane & 15), entries = len[l];
+                        e[i] = at < entries ? list[l * kOutList + at] : kOutNone;
+                        mine[i] = __ballot(e[i] != kOutNone && (int)((e[i] >> 15) & (kOutWaves - 1)) == wave);
+                        left |= entries > t + 16;
+                    }
+                    while ((mine[0] | mine[1] | mine[2] | mine[3]) != 0) {
+                        unsigned at[kOutFetch], p[kOutFetch];
+                        float gv[kOutFetch], wv[kOutFetch];
+#pragma unroll
+                        for (int h = 0; h < kOutFetch; ++h) {
+                            unsigned v = kOutNone;
+#pragma unroll
+                            for (int i = 3; i >= 0; --i)
+                                if (mine[i] != 0) v = (unsigned)__builtin_amdgcn_readlane((int)e[i], (int)__builtin_ctzll(mine[i]));
+                            bool taken = false;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                if (!taken && mine[i] != 0) {
+                                    mine[i] &= mine[i] - 1;
+                                    taken = true;
+                                }
+                            }
+                            p[h] = kOutNone;
+                            if (v == kOutNone) continue;
+                            p[h] = first + (v & 32767u);
+                            at[h] = (v >> 15) * (unsigned)a.sl;
+                            unsigned label = a.K > 1 ? __umulhi(p[h], a.inverse_k) : p[h];         // p / K, or one more
+                            label -= label * (unsigned)a.K > p[h] ? 1u : 0u;
+                            gv[h] = rows[(size_t)label * a.sl];
+                            wv[h] = a.w[p[h]];
+                        }
+                        float dot = 0.f;
+                        unsigned where = kOutNone;
+#pragma unroll
+                        for (int h = 0; h < kOutFetch; ++h) {
+                            if (p[h] == kOutNone) continue;
+                            float d = 0.f;
+                            if (lane < a.sl) {
+                                const unsigned o = at[h] + (unsigned)lane;
+                                gxt[o] = fmaf(wv[h], gv[h], gxt[o]);
+                                d = xt[o] * gv[h];
+                            }
+                            if (a.gw == nullptr) continue;
+#pragma unroll
+                            for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
+                            if (lane == h) { dot = d; where = p[h]; }
+                        }
+                        if (where != kOutNone) unsafeAtomicAdd(a.gw + where, dot);      // (the other slices' sums)
+                    }
+                    if (!__any(left)) break;
+                }
+                __syncthreads();
+            } while (more);
+#pragma unroll
+            for (int u = 0; u < kOutIds; ++u) ids[u] = next[u];
+        }
+        if (a.gx != nullptr)
+            each([&](int n, int b) {
+                if (b < nb) a.gx[cell(n, b)] = gxt[n * a.sl + b];
+            });
+    }
+}
+
+// Items so that the rounds of all CUs are full, a tile's room permitting.  Every item reads all ids, whatever the samples: few samples
+// of many columns keep the kernel above.  ms for the call by that and by this one, of one round: 4 x 131,072 x 300,000 x 40 2.7 and 5.8,
+// 8 of them 5.0 and 5.9, 32 x 131,072 x 100,000 x 30 4.8 and 1.6; 512 x 100,000 x 4,000 x 30, thirteen rounds, 3.6 and 1.3.
+bool outdated_wide_shape(const ffi_plan* p, const Dims& d, OutdatedWide* a) {
+    a->sl = 256 / p->members;
+    a->slices = (d.B + a->sl - 1) / a->sl;
+    const int cus = device_cu_count(), most = kOutTile / a->sl;
+    const long long rounds = ((long long)((d.N + most - 1) / most) * a->slices + cus - 1) / cus;
+    a->ranges = (int)std::min<long long>(d.N, std::max<long long>((d.N + most - 1) / most, rounds * cus / a->slices));
+    a->cols = (d.N + a->ranges - 1) / a->ranges;
+    return (long long)a->ranges * a->slices < (1ll << 31) && 12 * rounds <= d.B;
+}
+
 size_t redo_lds_bytes(int tile_labels, int K) {
     return (size_t)tile_labels * (kTileBatch * sizeof(float) + 8u * (size_t)K) + (size_t)kRedoThreads * 4u + 64u;
 }
@@ -343,6 +515,28 @@ int backward_if_outdated_prepare(const Dims& d, hipStream_t s) {
     if (bytes == 0) return FFI_OK;
     FFI_TRY(zeroed_get(s, kWsSums, bytes, &ws));
     return tickets_get(s, &ws);
+}
+
+bool takes_outdated_wide(const ffi_plan* p, const Dims& d) {
+    OutdatedWide a;
+    RedoShape r;
+    return !p->tiled && !redo_shape(d, &r) && outdated_wide_shape(p, d, &a);
+}
+
+int launch_outdated_wide(const ffi_plan* p, const float* x, const int32_t* idx, const float* w, const float* g_slices, float* gx, float* gw,
+                         const Dims& d, hipStream_t s) {
+    OutdatedWide a{};
+    if (!outdated_wide_shape(p, d, &a)) return FFI_ERR_BAD_ARGUMENT;
+    a.verdict = p->d_guard + kGuardVerdict;
+    a.x = x; a.w = w; a.g = g_slices; a.idx = idx; a.gx = gx; a.gw = x != nullptr ? gw : nullptr;
+    a.B = d.B; a.N = d.N; a.L = d.L; a.K = d.K;
+    a.inverse_k = d.K > 1 ? (unsigned)((1ull << 32) / (unsigned)d.K) + 1u : 0u;
+    const size_t lds = ((size_t)2 * a.cols * a.sl + kOutWaves * kOutList + kOutWaves) * sizeof(float);
+    const auto kernel = d.tp ? outdated_wide_kernel<true> : outdated_wide_kernel<false>;
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(device_cu_count(), a.ranges * a.slices)), dim3(kOutThreads), lds, s, a);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
 }
 
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,

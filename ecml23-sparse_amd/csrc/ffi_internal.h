@@ -467,6 +467,10 @@ int plan_guard_poll(ffi_plan* p, bool* seen, bool* current, unsigned long long* 
 // allocated by backward_if_outdated_prepare, ahead of the first kernel of the call.
 size_t backward_if_outdated_workspace(const Dims& d);
 int backward_if_outdated_prepare(const Dims& d, hipStream_t s);
+// The same behind a walk of a plan's global form (ffi_wide.hip), which left out_grad in slices; gw is zero where the verdict is 0.
+bool takes_outdated_wide(const ffi_plan* p, const Dims& d);
+int launch_outdated_wide(const ffi_plan* p, const float* x, const int32_t* idx, const float* w, const float* g_slices, float* gx, float* gw,
+                         const Dims& d, hipStream_t s);
 // (`zeroed`: where the verdict is 0 feature_grad is zero already)
 int launch_backward_if_outdated(const unsigned long long* verdict, const float* features, const int32_t* lookup,
                                 const float* weights, const float* out_grad, float* feature_grad, float* weight_grad,
@@ -476,7 +480,7 @@ void plan_free(ffi_plan* p);
 int launch_input_grad(const ffi_plan* p, const float* w, const float* g, float* gx, int B, bool tp,
                       hipStream_t s, const LookupCheck* check = nullptr);
 // Global form: the input gradient and, with gw given (then x too), the weight gradient (and bias gradient) in the same walk.  With a
-// check and gw, gx is zero where the check has found the plan outdated.
+// check and gw, gx is zero where the check has found the plan outdated -- gw instead where takes_outdated_wide().
 int walk_slices(long long units, int slices);
 int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, const float* g, float* gx, float* gw, float* bias_grad, int B,
                          bool tp, hipStream_t s, const LookupCheck* check);

@@ -446,10 +446,12 @@ __global__ __launch_bounds__(kTileMoveThreads) void weights_to_slots_kernel(cons
 __global__ __launch_bounds__(kTileMoveThreads) void weight_grads_from_slots_kernel(const float* __restrict__ gw_slots, const unsigned short* __restrict__ tile_pos,
                                                                                    const unsigned* __restrict__ slot_of, float* __restrict__ gw,
                                                                                    size_t total, int tile_bits, int tiles, int slices, size_t slots,
-                                                                                   const unsigned long long* __restrict__ verdict, float* __restrict__ gx, size_t gx_count) {
+                                                                                   const unsigned long long* __restrict__ verdict, float* __restrict__ clear, size_t clear_count) {
     extern __shared__ __align__(16) float tile_mem[];
-    if (verdict != nullptr && *verdict == 0)
-        for (size_t i = (size_t)blockIdx.x * kTileMoveThreads + threadIdx.x; i < gx_count; i += (size_t)gridDim.x * kTileMoveThreads) gx[i] = 0.f;
+    const bool outdated = verdict != nullptr && *verdict == 0;
+    if (outdated)
+        for (size_t i = (size_t)blockIdx.x * kTileMoveThreads + threadIdx.x; i < clear_count; i += (size_t)gridDim.x * kTileMoveThreads) clear[i] = 0.f;
+    if (outdated && clear == gw) return;
     const int t = xcd_unit(blockIdx.x, tiles);
     if (t < 0) return;
     const size_t p0 = (size_t)t << tile_bits;
@@ -629,10 +631,11 @@ int launch_backward_wide(const ffi_plan* p, const float* x, const float* w, cons
         hipLaunchKernelGGL(gather_gx, gx_grid, dim3(1024), 0, s, parts, gx, p->N, B, sl, p->segments);
         FFI_HIP_TRY(hipGetLastError());
     }
-    // (last: it clears gx behind an outdated plan)
+    // (last: behind an outdated plan it clears what the recomputing kernel adds up in memory)
     if (dot) {
+        const bool clears_gw = check != nullptr && takes_outdated_wide(p, Dims{B, p->N, p->L, p->K, tp});
         hipLaunchKernelGGL(weight_grads_from_slots_kernel, dim3(xcd_grid(tiles)), dim3(kTileMoveThreads), tile_bytes, s, gw_slots, p->tile_pos, p->slot_of,
-                           gw, count, p->tile_bits, tiles, at_once, slots, check != nullptr ? check->guard + kGuardVerdict : nullptr, gx, (size_t)p->N * B);
+                           gw, count, p->tile_bits, tiles, at_once, slots, check != nullptr ? check->guard + kGuardVerdict : nullptr, clears_gw ? gw : gx, clears_gw ? count : (size_t)p->N * B);
         FFI_HIP_TRY(hipGetLastError());
     }
     return FFI_OK;

@@ -633,6 +633,39 @@ def test_both_gradients_behind_an_outdated_plan(ffi, shape, transposed):
         assert rel_err(gw.cpu().numpy(), ref_gw) <= GRAD_RTOL
 
 
+# The same for inputs that do not fit on chip: ranges of columns and slices of 32 and 64 samples in full and in part, several rounds of
+# items, fewer ids than a step and one more, a layer whose ids crowd in one column (lists that overflow in every step),
+# and few samples of many columns, which the plain kernel takes
+@pytest.mark.parametrize("shape", [(40, 2000, 700, 12), (7, 1217, 16_384, 1), (33, 1300, 10_923, 3), (12, 1400, 32_768, 1), (64, 65_536, 9001, 17), (130, 40_000, 3000, 40),
+                                   (20, 30_001, 129, 127), (65, 1500, 20_000, 9), (1, 400_000, 3000, 7)])
+@pytest.mark.parametrize("crowded", [False, True])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_both_gradients_of_wide_inputs_behind_an_outdated_plan(ffi, shape, crowded, transposed):
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B + K)
+    xin = np.ascontiguousarray(x.T) if transposed else x
+    dx, dl, dw, dg = dev(xin), dev(lookup), dev(w), dev(g)
+    bwd = ffi.fan_in_sparse_matmul_grad_tp if transposed else ffi.fan_in_sparse_matmul_grad
+    grad = torch.empty_like(dx)
+    lib = ffi._lib.lib()
+    bwd(dx, dl, dw, dg)
+    rng = np.random.default_rng(8)
+    outs = []
+    for _ in range(2):                                  # two edits, both served before the host has seen a verdict
+        lookup = lookup.copy()
+        if crowded:
+            lookup[:] = np.where(rng.random(lookup.shape) < 0.9, N - 1, lookup)
+        lookup[rng.integers(0, L, 400), rng.integers(0, K, 400)] = rng.integers(0, N, 400)
+        dl.copy_(dev(lookup))
+        outs.append((lookup, *bwd(dx, dl, dw, dg)))
+    ffi._lib.check(lib.ffi_input_grad_f32(dl.data_ptr(), dw.data_ptr(), dg.data_ptr(), grad.data_ptr(), B, N, L, K, int(transposed), stream()))
+    outs.append((lookup, grad, outs[-1][2]))
+    for edited, gx, gw in outs:
+        ref_gx, ref_gw = oracle.backward(xin, edited, w, g, transposed=transposed)
+        assert rel_err(gx.cpu().numpy(), ref_gx) <= GRAD_RTOL
+        assert rel_err(gw.cpu().numpy(), ref_gw) <= GRAD_RTOL
+
+
 def _label_sample_errors(lookup, w, g, x, gx, gw, B, N, K, labels):
     """weight gradient of a label sample and the full input gradient against the oracle ([N,B] features)"""
     o_gw = oracle.weight_grad(x, lookup[labels], w[labels], np.ascontiguousarray(g[:, labels]), transposed=True)
