@@ -311,8 +311,8 @@ __global__ __launch_bounds__(kRedoThreads) void redo_backward_kernel(const RedoA
 // connection's row of out_grad comes from the slices that the passes over the plan left in their slot; eight are fetched at once.
 // Bound by the steps of 32,768 ids, some 15 us each: what 16 wavefronts pick out of the lists, two barriers and a round trip for rows.
 // One thread a connection, its samples one by one and its input gradient by atomics in memory (the kernel above), the whole call at
-// 128 x 65,536 x 670,091 x 72: 313 ms, 47 so (16 ids a thread, all eight rows fetched also where fewer are left: 64); at
-// 50 x 32,768 x 670,000 x 32 51 and 10.7, at 128 x 1,300 x 100,000 x 32 14.9 and 2.9.
+// 128 x 65,536 x 670,091 x 72: 313 ms, 45 so (16 ids a thread, all eight rows fetched also where fewer are left: 64; the next ids
+// in registers of their own, 152 bytes of spills: 47); at 50 x 32,768 x 670,000 x 32 51 and 10.2, at 128 x 1,300 x 100,000 x 32 14.9 and 2.8.
 constexpr int kOutIds = 32, kOutWaves = 16, kOutThreads = 64 * kOutWaves, kOutList = 256, kOutFetch = 8;
 constexpr int kOutTile = 16384;                // floats of a tile
 constexpr unsigned kOutStep = kOutIds * kOutThreads, kOutNone = ~0u;
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const Outdat
             xt[n * a.sl + b] = a.gw != nullptr && b < nb ? a.x[cell(n, b)] : 0.f;
         });
         const float* const rows = a.g + (size_t)slice * a.L * a.sl + min(lane, a.sl - 1);
-        int ids[kOutIds], next[kOutIds];
+        int ids[kOutIds];
         auto fetch = [&](unsigned first, int (&v)[kOutIds]) {
 #pragma unroll
             for (int q = 0; q < kOutIds / 4; ++q) {
@@ -372,7 +372,6 @@ __global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const Outdat
         fetch(0, ids);
         __syncthreads();
         for (unsigned first = 0; first < total; first += kOutStep) {
-            if (first + kOutStep < total) fetch(first + kOutStep, next);
             int from = 0;
             bool more;
             do {
@@ -390,6 +389,7 @@ __global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const Outdat
                     if (hit) list[wave * kOutList + at] = col << 15 | (unsigned)wave << 11 | (unsigned)((u >> 2) * 256 + lane * 4 + (u & 3));
                     n += (int)__popcll(hits);
                 }
+                if (from < kOutIds && to == kOutIds && first + kOutStep < total) fetch(first + kOutStep, ids);      // (on their way through the rest of the step)
                 from = to;
                 if (lane == 0) len[wave] = n;
                 more = __syncthreads_or(from < kOutIds) != 0;
@@ -453,8 +453,6 @@ __global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const Outdat
                 }
                 __syncthreads();
             } while (more);
-#pragma unroll
-            for (int u = 0; u < kOutIds; ++u) ids[u] = next[u];
         }
         if (a.gx != nullptr)
             each([&](int n, int b) {
@@ -465,7 +463,7 @@ __global__ __launch_bounds__(kOutThreads) void outdated_wide_kernel(const Outdat
 
 // Items so that the rounds of all CUs are full, a tile's room permitting.  Every item reads all ids, whatever the samples: few samples
 // of many columns keep the kernel above.  ms for the call by that and by this one, of one round: 4 x 131,072 x 300,000 x 40 2.7 and 5.8,
-// 8 of them 5.0 and 5.9, 32 x 131,072 x 100,000 x 30 4.8 and 1.6; 512 x 100,000 x 4,000 x 30, thirteen rounds, 3.6 and 1.3.
+// 8 of them 5.0 and 5.9, 32 x 131,072 x 100,000 x 30 4.8 and 1.5; 512 x 100,000 x 4,000 x 30, thirteen rounds, 3.6 and 1.3.
 bool outdated_wide_shape(const ffi_plan* p, const Dims& d, OutdatedWide* a) {
     a->sl = 256 / p->members;
     a->slices = (d.B + a->sl - 1) / a->sl;
