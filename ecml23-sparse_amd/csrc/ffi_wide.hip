@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void walk_columns_kernel(const Wal
 // Consecutive tiles go to one XCD, whose L2 gathers what several of them write to a line.
 //
 // The first check.blocks workgroups of the one check the lookup's content against the plan instead (ffi_check.h); where that found the plan
-// outdated, the other clears gx for the kernel that then forms the gradients anew.  (As kernels of their own the two were 9 of the 50 to 60
+// outdated, the other clears what the kernel that then forms the gradients anew adds up in memory: gw, or gx (takes_outdated_wide()).  (As kernels of their own the two were 9 of the 50 to 60
 // us of a backward pass of few connections, and the check 40 of 3,250 at 65,536 columns x 670,091 labels x 72.)
 constexpr int kTileMoveThreads = kCheckThreads, kTileMoveAhead = 8;
 

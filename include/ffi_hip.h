@@ -206,6 +206,7 @@ int ffi_lookup_edited(const int32_t* lookup);
  *   "plan_sorted_columns"  -1: never / 1: whenever the weights-in-LDS form is taken: plans that hand a tile's columns to the
  *                          walking kernel's threads sorted by length (fewer padded slots; the sums pass through LDS after every tile)
  *   "small_path"           -1: never / 1: wherever they can: the two launches that serve small layers
+ *   "dense_rows"           -1: never / 1: wherever they can: the kernels that write a label's row out over a few columns
  *   "wide_phases"          -1: never / 1: wherever it can: the kernel of wide forward passes that takes the columns in phases
  * Drops the cached plans and workspaces of the current device first (as ffi_cache_clear, with its rule about calls in
  * flight).  Unknown names and values outside the ranges above return FFI_ERR_BAD_ARGUMENT and change nothing.
