@@ -6,6 +6,7 @@
 #include "ffi_check.h"
 #include "ffi_lds_tile.h"
 #include "ffi_sliced.h"
+#include "ffi_walk.h"
 
 #include <algorithm>
 
@@ -138,7 +139,6 @@ __global__ __launch_bounds__(kWideThreads) void wgrad_wide_kernel(const float* _
 // the barrier (the older of two wavefronts on a SIMD is served first and runs away from the other).  Sums in LDS with a lane group
 // per column, whose lists of a block of labels are short and of unequal lengths, took 1.07 (two slices of 32 samples), and needed the weights in a
 // random order (0.37 each way, 0.1 now).  Rows of 128 samples 1.49 instead of 1.36; 16 wavefronts of 16 columns 0.70; sixteen steps in flight 0.68.
-constexpr int kWalkWaves = 8;
 // per wavefront: its columns' rows of x, a lane's 16 bytes apart from the next multiple of 64 banks, and two chunks' lists
 constexpr int walk_rows_bytes(int gl) { return kGroupColumns * (gl + 1) * 16; }
 constexpr int walk_wave_bytes(int gl) { return walk_rows_bytes(gl) + 16 * kChunkSteps * 64 / gl; }
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void walk_columns_kernel(const Wal
     const int all = a.units * a.slices, wg = xcd_unit(blockIdx.x, (all + kWalkWaves - 1) / kWalkWaves);
     if (wg < 0) return;
     const bool on = wg * kWalkWaves + wave < all;
-    const int at = min(wg * kWalkWaves + wave, all - 1), slice = at / a.units, u = at - slice * a.units;
+    const int at = walk_place(wg, wave, all), slice = at / a.units, u = at - slice * a.units;
     float4* const xs = reinterpret_cast<float4*>(mem + wave * walk_wave_bytes(GL));
     unsigned* const offs = reinterpret_cast<unsigned*>(mem + wave * walk_wave_bytes(GL) + walk_rows_bytes(GL));
     float* const wts = reinterpret_cast<float*>(offs + 2 * kEntries);
@@ -216,14 +216,9 @@ __global__ __launch_bounds__(kWalkWaves * 64) void walk_columns_kernel(const Wal
     const buffer_rsrc rows = make_rsrc(a.gtab + (a.slice0 + slice) * a.gslice + (size_t)label0 * (GL * 4), (size_t)min(a.seg_labels, a.L - label0) * kRow);
     const unsigned lane_off = (unsigned)sub * 16u;
     const unsigned count = on ? a.chunk_count[u] : 0u;
-    unsigned rounds = 0;                                                    // of the workgroup
+    unsigned rounds = 0;                                                    // of the workgroup, in all its wavefronts: they meet at as many barriers
 #pragma unroll
-    for (int i = 0; i < kWalkWaves; ++i) {
-        // (a workgroup's streams are consecutive ones, of this slice and maybe others)
-        int v = min(wg * kWalkWaves + i, all - 1) - slice * a.units;
-        if (v < 0) v += a.units;
-        rounds = max(rounds, a.chunk_count[v < a.units ? v : v % a.units]);
-    }
+    for (int i = 0; i < kWalkWaves; ++i) rounds = max(rounds, a.chunk_count[walk_stream(wg, i, a.units, all)]);
     // this lane's part of x: 16 bytes of some columns' rows, or four samples of a column several times
     constexpr int kXLoads = kGroupColumns / kMembers;
     float4 xv[DOT ? kXLoads : 1];

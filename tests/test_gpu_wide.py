@@ -1,5 +1,7 @@
 """Inputs whose tile does not fit in LDS (more than 1,216 columns): the kernels that gather from sample-sliced tables, at
 the sizes where they change form, against the CPU oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -496,6 +498,37 @@ def test_plans_of_the_global_form(ffi, kind, N, L, K):
             assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-4 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4
     finally:
         lib.ffi_set_option(b"small_path", 0)
+
+
+# Plans of one stream to seven, which put several slices of the samples into one workgroup of the walk: one label of more connections than the tiled form
+# takes, steps of four and of eight connections; samples for fewer slices than a workgroup has wavefronts, as many and more
+@pytest.mark.parametrize("streams", [1, 2, 3, 4, 5, 7])
+@pytest.mark.parametrize("hint,B", [(0, 193), (0, 641), (32, 193), (32, 481)])
+def test_walks_of_few_streams(ffi, streams, hint, B):
+    N, L, K = 32 * streams - 3, 1, 1100
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=streams + B)
+    ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+    dx, dl, dw, dg = dev(x), dev(lookup), dev(w), dev(g)
+    lib, stream = ffi._lib.lib(), torch.cuda.current_stream().cuda_stream
+    plan = ctypes.c_void_p()
+    ffi._lib.check(lib.ffi_plan_create(dl.data_ptr(), L, K, N, hint, stream, ctypes.byref(plan)))
+    try:
+        for transposed in (0, 1):
+            gx = torch.full((N, B) if transposed else (B, N), float("nan"), device="cuda")
+            ffi._lib.check(lib.ffi_input_grad_planned_f32(plan, dw.data_ptr(), dg.data_ptr(), gx.data_ptr(), B, transposed, stream))
+            got = gx.cpu().numpy()
+            # some K / N products of one gradient and a weight each, at most 128 of them: 128 2^-24 of the largest sum
+            assert rel_err(got.T if transposed else got, ref_gx) <= 1e-5
+    finally:
+        ffi._lib.check(lib.ffi_plan_destroy(plan))
+    # both gradients in one walk
+    assert lib.ffi_set_option(b"small_path", -1) == 0 and lib.ffi_set_option(b"dense_rows", -1) == 0
+    try:
+        for _ in range(2):
+            gx, gw = ffi.fan_in_sparse_matmul_grad(dx, dl, dw, dg)
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-4
+    finally:
+        assert lib.ffi_set_option(b"small_path", 0) == 0 and lib.ffi_set_option(b"dense_rows", 0) == 0
 
 
 def test_more_lookups_than_the_cache_holds(ffi):

@@ -188,3 +188,41 @@ def test_host_kernels_match_the_oracle():
     assert lib.ffi_host_forward_f32(one, one, one, one, 1, 1, 1, 1, 0, 0, 2) == -8
     bad = np.array([[3]], dtype=np.int32); f1 = np.ones((1, 1), dtype=np.float32)
     assert lib.ffi_host_forward_f32(ptr(f1), ptr(bad), ptr(f1), ptr(f1.copy()), 1, 1, 1, 1, 0, 0, 1) == -6
+
+
+def test_streams_that_the_wavefronts_of_a_walk_take(tmp_path):
+    # csrc/ffi_walk.h, on the host: every stream of every slice has one wavefront, and what a workgroup's wavefronts look up of one another's streams is in
+    # range and the same for all, also where few streams put several slices into one workgroup
+    import os
+    import shutil
+    import subprocess
+
+    from conftest import ROOT
+    source = tmp_path / "walk.cc"
+    source.write_text(r"""
+#include "ffi_walk.h"
+#include <cstdio>
+#include <vector>
+using namespace ffi;
+int main() {
+    for (int units = 1; units <= 64; ++units)
+        for (int slices = 1; slices <= 64; ++slices) {
+            const int all = units * slices;
+            std::vector<int> taken(all, 0);
+            for (int workgroup = 0; workgroup * kWalkWaves < all; ++workgroup)
+                for (int wave = 0; wave < kWalkWaves; ++wave) {
+                    const int place = walk_place(workgroup, wave, all), stream = walk_stream(workgroup, wave, units, all);
+                    if (place < 0 || place >= all || stream < 0 || stream >= units || stream != place - place / units * units)
+                        return std::printf("%d streams, %d slices: wavefront %d of %d looks up %d\n", units, slices, wave, workgroup, stream), 1;
+                    if (workgroup * kWalkWaves + wave < all) ++taken[place];
+                }
+            for (int place = 0; place < all; ++place)
+                if (taken[place] != 1) return std::printf("%d streams, %d slices: %d taken %d times\n", units, slices, place, taken[place]), 1;
+        }
+    return 0;
+}
+""")
+    compiler = shutil.which("g++") or shutil.which("c++")
+    subprocess.run([compiler, "-std=c++17", "-O1", "-I", os.path.join(ROOT, "ecml23-sparse_amd", "csrc"), str(source), "-o", str(tmp_path / "walk")], check=True)
+    done = subprocess.run([str(tmp_path / "walk")], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout
