@@ -421,7 +421,7 @@ __host__ __device__ inline size_t arranged_quarter_offset(long long u, int t) {
 }
 inline size_t arranged_words(long long units) { return (size_t)((units + 63) / 64) * 64 * 32; }
 int plan_build(ffi_plan* p, const int32_t* lookup, hipStream_t s);
-// Makes `s` wait for the kernels that lay the plan out, where they may still be running.
+// Makes `s`, or the host where `s` is being captured, wait for the kernels that lay the plan out, where they may still be running.
 int plan_wait_built(const ffi_plan* p, hipStream_t s);
 int plan_check_ids(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);

@@ -1630,18 +1630,34 @@ int plan_build_arrays(ffi_plan* p, const int32_t* lookup, hipStream_t s, unsigne
 }
 }  // namespace
 
+namespace {
+// The calls below may be made while this thread or another one captures a stream: none of them has to do with a capture.
+class UncapturedCalls {
+public:
+    UncapturedCalls() { known_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+    ~UncapturedCalls() { if (known_) (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool known_;
+};
+}  // namespace
+
 int plan_wait_built(const ffi_plan* p, hipStream_t s) {
     if (!p->built_pending.load(std::memory_order_acquire)) return FFI_OK;
-    // (under capture the plan is one of before, and a graph is replayed behind what its owner waited for)
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     FFI_HIP_TRY(hipStreamIsCapturing(s, &capture));
-    if (capture != hipStreamCaptureStatusNone) return FFI_OK;
-    const hipError_t e = hipEventQuery(p->built);
+    // (a graph cannot wait for an event of before its capture, and may be replayed at once and on any stream: there the host waits)
+    const bool captured = capture != hipStreamCaptureStatusNone;
+    hipError_t e;
+    {
+        const UncapturedCalls calls;
+        e = captured ? hipEventSynchronize(p->built) : hipEventQuery(p->built);
+    }
     if (e == hipSuccess) {
         p->built_pending.store(false, std::memory_order_release);
         return FFI_OK;
     }
-    if (e != hipErrorNotReady) return hip_fail(e);
+    if (captured || e != hipErrorNotReady) return hip_fail(e);
     (void)hipGetLastError();
     FFI_HIP_TRY(hipStreamWaitEvent(s, p->built, 0));
     return FFI_OK;

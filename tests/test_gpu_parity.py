@@ -826,6 +826,56 @@ def test_one_lookup_used_from_two_streams_in_turn(ffi):
             assert rel_err(gw[i].cpu().numpy(), ref_gw) <= GRAD_RTOL, (rnd, i)
 
 
+@pytest.mark.parametrize("shape", [(64, 300, 60_000, 16), (40, 1300, 300_000, 24), (33, 1150, 30_000, 9)])
+def test_a_call_captured_behind_the_build_of_its_plan(ffi, shape):
+    # a plan that one stream has just built, in a graph that another stream captures and replays with nothing in between; the workspaces
+    # of that stream are there from a call with another lookup of more connections
+    B, N, L, K = shape
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=B)
+    ref_gx, ref_gw = oracle.backward(x, lookup, w, g, transposed=False)
+    dx, dl, dw, dg = dev(x), dev(lookup), dev(w), dev(g)
+    lib = ffi._lib.lib()
+
+    def call(lookup, grads, stream, labels=L):
+        ffi._lib.check(lib.ffi_backward_f32(dx.data_ptr(), lookup.data_ptr(), dw.data_ptr(), dg.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(),
+                                            B, N, labels, K, 0, stream.cuda_stream))
+
+    one, other = torch.cuda.Stream(), torch.cuda.Stream()
+    first, captured = ([torch.empty((B, N), device="cuda"), torch.empty((L, K), device="cuda")] for _ in range(2))
+    more = 9 * L // 8
+    x2, lookup2, w2, g2 = (dev(a) for a in reference_law_inputs(B, N, more, K, seed=B + 1))
+    gx2, gw2 = torch.empty((B, N), device="cuda"), torch.empty((more, K), device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(2):
+        ffi._lib.check(lib.ffi_backward_f32(x2.data_ptr(), lookup2.data_ptr(), w2.data_ptr(), g2.data_ptr(), gx2.data_ptr(), gw2.data_ptr(), B, N, more, K, 0,
+                                            other.cuda_stream))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    call(dl, first, one)                                   # (builds; the kernels that lay the plan out are still running)
+    with torch.cuda.stream(other):
+        graph.capture_begin()
+        call(dl, captured, other)
+        graph.capture_end()
+        graph.replay()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for gx, gw in (first, captured):
+            assert rel_err(gx.cpu().numpy(), ref_gx) <= GRAD_RTOL and rel_err(gw.cpu().numpy(), ref_gw) <= GRAD_RTOL
+        assert torch.equal(first[0], captured[0])
+        for t in captured:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graph.replay()
+        torch.cuda.synchronize()
+    # the same lookup in a plain call again
+    call(dl, first, one)
+    torch.cuda.synchronize()
+    assert torch.equal(first[0], captured[0])
+    del graph
+    ffi._lib.check(lib.ffi_cache_clear())
+
+
 def test_plan_is_unusable_after_a_failed_refresh(ffi):
     # a rebuild that fails (here: an id out of range) leaves a plan without arrays; calls through it are refused
     # with a status instead of walking freed memory
