@@ -28,6 +28,20 @@ _has_global_hook = torch.nn.modules.module._has_any_global_hook
 _saved_tensor_hooks = torch._C._autograd._top_saved_tensors_default_hooks
 
 
+_MARK = "ecml23-sparse: held"
+
+
+def _accumulation_node(variable):
+    return variable.view_as(variable).grad_fn.next_functions[0][0]
+
+
+def _is_held(variable):
+    """Whether anybody holds the node of autograd's that adds to ``variable.grad``: libraries that exchange gradients put hooks
+    on it.  A node that nobody holds goes away, and with it its hooks and the mark put on it here."""
+    _accumulation_node(variable).metadata[_MARK] = True
+    return _accumulation_node(variable).metadata.pop(_MARK, False)
+
+
 def adam_step(variable, m, v, gradient, learning_rate, beta_1, beta_2, epsilon, step):
     """One in-place Adam step on contiguous float32 device tensors of equal size; ``step`` counts from 1."""
     for name, t in (("variable", variable), ("m", m), ("v", v), ("gradient", gradient)):
@@ -191,8 +205,15 @@ class SparseOptWrapper(torch.nn.Module):
         else:
             scores = _forward_bias(x, lookup, by_label, bias, False)
             out_grad, loss_sum = metrics_mod.sparse_loss_grad(scores, labels, self.loss.kind)
-        _, weight_grad, bias.grad = _backward_bias(x, lookup, by_label, out_grad, False, need_feature_grad=False)
-        weights.grad = weight_grad.view(-1)
+        _, weight_grad, bias_grad = _backward_bias(x, lookup, by_label, out_grad, False, need_feature_grad=False)
+        weight_grad = weight_grad.view(-1)
+        # (looked for here, where the GPU has work and the host has time: it takes some 15 us)
+        with torch.enable_grad():
+            held = _is_held(weights) or _is_held(bias)
+        if held:
+            torch.autograd.backward((weights, bias), (weight_grad, bias_grad))
+        else:
+            weights.grad, bias.grad = weight_grad, bias_grad
         for o in self.optimizers:
             o.step()
         self.handle_sparse_layers()

@@ -335,3 +335,31 @@ def test_what_a_caller_put_into_a_step_still_runs(ffi):
         wrapper.train_step((x[:, 1:], y))
     with pytest.raises(RuntimeError), torch.no_grad():
         wrapper.train_step((x, y))
+
+
+def _accumulation_node(variable):
+    return variable.expand_as(variable).grad_fn.next_functions[0][0]
+
+
+@pytest.mark.parametrize("variable", ["kernel_weights", "bias"])
+@pytest.mark.parametrize("before", [False, True])
+def test_hooks_on_the_node_that_adds_a_gradient_up_run(ffi, variable, before):
+    # where libraries that exchange gradients hang theirs: behind the sum, and ahead of it with a gradient to change
+    kept, plain = _training(ffi), _training(ffi)
+    node, seen = _accumulation_node(getattr(kept[1], variable)), []
+    if before:
+        node.register_prehook(lambda grads: (seen.append(1), tuple(2.0 * g for g in grads))[1])
+    else:
+        node.register_hook(lambda *_: seen.append(1) and None)
+    for steps in (1, 2):
+        results = [run[0].train_step((run[3], run[4])) for run in (kept, plain)]
+        assert len(seen) == steps
+        if steps == 1:
+            assert results[0] == results[1]
+            for name in ("kernel_weights", "bias"):
+                a, b = (getattr(run[1], name).grad for run in (kept, plain))
+                assert torch.equal(a, 2.0 * b if before and name == variable else b)
+    assert not node.metadata                                            # (nothing of the step's is left there)
+    del node
+    kept[0].train_step((kept[3], kept[4]))                              # (a node that nobody keeps goes, and its hooks with it)
+    assert len(seen) == 2
