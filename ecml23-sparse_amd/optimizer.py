@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from . import metrics as metrics_mod
@@ -168,7 +169,7 @@ class SparseOptWrapper(torch.nn.Module):
         """Whether the step is the layer, one of the library's losses and their gradients with respect to the layer's two
         variables, with nobody to see the graph in between: ``_direct_step`` then calls the library without one.  Everything a
         caller may have put there -- another model or loss, hooks on modules, variables or saved tensors, modes, transforms,
-        anomaly detection, tracing -- and everything that is refused takes the general way."""
+        forward derivatives, anomaly detection, tracing -- and everything that is refused takes the general way."""
         layer = self.base_model
         if (type(layer) not in _DIRECT_LAYERS or type(self.loss) not in _DIRECT_LOSSES or type(x) is not torch.Tensor
                 or x.requires_grad or x.dtype != torch.float32 or not x.is_cuda or x.dim() != 2 or x.shape[1] != layer.input_dim
@@ -177,7 +178,7 @@ class SparseOptWrapper(torch.nn.Module):
         if (not torch.is_grad_enabled() or torch.is_inference_mode_enabled() or torch.is_anomaly_enabled()
                 or torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
                 or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()
-                or torch._C._len_torch_function_stack() or _saved_tensor_hooks(False) is not None):
+                or torch._C._len_torch_function_stack() or _saved_tensor_hooks(False) is not None or forward_ad._current_level >= 0):
             return False
         if _has_global_hook() or any(layer.__dict__[name] for name in _MODULE_HOOKS) or not _OVERRIDABLE.isdisjoint(layer.__dict__):
             return False

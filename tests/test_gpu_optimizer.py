@@ -363,3 +363,12 @@ def test_hooks_on_the_node_that_adds_a_gradient_up_run(ffi, variable, before):
     del node
     kept[0].train_step((kept[3], kept[4]))                              # (a node that nobody keeps goes, and its hooks with it)
     assert len(seen) == 2
+
+
+def test_a_forward_derivative_of_a_step_is_refused(ffi):
+    # as by the layer's op, which has none
+    wrapper, _, _, x, y = _training(ffi)
+    with torch.autograd.forward_ad.dual_level():
+        with pytest.raises(RuntimeError):
+            wrapper.train_step((torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), y))
+    wrapper.train_step((x, y))
