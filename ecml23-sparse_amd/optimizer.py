@@ -20,13 +20,21 @@ from .fixed_fan_in_ops import _backward_bias, _forward_bias, _on, _stream_handle
 _DIRECT_LAYERS = (StratifiedRewireLayerV2, StratifiedRewireLayer)
 _DIRECT_LOSSES = (metrics_mod.SparseHingeLoss, metrics_mod.SparseSquaredHingeLoss, metrics_mod.SparseBinaryCrossEntropyLoss)
 _MODULE_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
-_OVERRIDABLE = frozenset(("forward", "__call__"))
+# (as the classes define them: what replaces one on a class or on the layer is to be called)
+_MODULE_CALLS = ("forward", "__call__", "_wrapped_call_impl", "_call_impl")
+_OVERRIDABLE = frozenset((*_MODULE_CALLS, "_compiled_call_impl"))
+_CALLS = {cls: tuple((name, getattr(cls, name)) for name in names)
+          for classes, names in ((_DIRECT_LAYERS, _MODULE_CALLS), (_DIRECT_LOSSES, ("__call__",))) for cls in classes}
 # From here on the scores are formed, turned into gradients and ranked in one kernel; below, a kernel each is faster: the one kernel's
 # ranks cost more than the scores' way through the caches.  us a step, one kernel and several: 128 x 300 x 300,000 x 4 240 and
 # 333, 128 x 1,100 x 200,000 x 20 293 and 318, 31 x 45 x 290,420 x 75 514 and 510, 32 x 768 x 131,072 x 32 179 and 151.
 _SCORES_IN_ONE_KERNEL = 1 << 24
 _has_global_hook = torch.nn.modules.module._has_any_global_hook
 _saved_tensor_hooks = torch._C._autograd._top_saved_tensors_default_hooks
+
+
+def _as_defined(cls):
+    return all(getattr(cls, name) is call for name, call in _CALLS[cls])
 
 
 _MARK = "ecml23-sparse: held"
@@ -168,7 +176,7 @@ class SparseOptWrapper(torch.nn.Module):
     def _steps_directly(self, x):
         """Whether the step is the layer, one of the library's losses and their gradients with respect to the layer's two
         variables, with nobody to see the graph in between: ``_direct_step`` then calls the library without one.  Everything a
-        caller may have put there -- another model or loss, hooks on modules, variables or saved tensors, modes, transforms,
+        caller may have put there -- another model or loss, other calls on their classes, hooks on modules, variables or saved tensors, modes, transforms,
         forward derivatives, anomaly detection, tracing -- and everything that is refused takes the general way."""
         layer = self.base_model
         if (type(layer) not in _DIRECT_LAYERS or type(self.loss) not in _DIRECT_LOSSES or type(x) is not torch.Tensor
@@ -179,6 +187,8 @@ class SparseOptWrapper(torch.nn.Module):
                 or torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
                 or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()
                 or torch._C._len_torch_function_stack() or _saved_tensor_hooks(False) is not None or forward_ad._current_level >= 0):
+            return False
+        if not _as_defined(type(layer)) or not _as_defined(type(self.loss)):
             return False
         if _has_global_hook() or any(layer.__dict__[name] for name in _MODULE_HOOKS) or not _OVERRIDABLE.isdisjoint(layer.__dict__):
             return False

@@ -372,3 +372,26 @@ def test_a_forward_derivative_of_a_step_is_refused(ffi):
         with pytest.raises(RuntimeError):
             wrapper.train_step((torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), y))
     wrapper.train_step((x, y))
+
+
+def test_calls_replaced_on_a_class_are_made(ffi, monkeypatch):
+    calls = []
+
+    def counted(call):
+        return lambda *args, **kwargs: (calls.append(1), call(*args, **kwargs))[1]
+
+    for owner, name in ((ffi.StratifiedRewireLayerV2, "forward"), (ffi.StratifiedRewireLayerV2, "__call__"), (torch.nn.Module, "_call_impl"),
+                        (ffi.metrics.SparseLossBase, "__call__"), (ffi.SparseSquaredHingeLoss, "__call__")):
+        wrapper, _, _, x, y = _training(ffi)
+        with monkeypatch.context() as patch:
+            patch.setattr(owner, name, counted(getattr(owner, name)))
+            calls.clear()
+            wrapper.train_step((x, y))
+            assert calls, (owner, name)
+    wrapper, layer, _, x, y = _training(ffi)
+    for name in ("_call_impl", "_compiled_call_impl"):                  # (the second is what Module.compile sets)
+        layer.__dict__[name] = counted(layer._call_impl)
+        calls.clear()
+        wrapper.train_step((x, y))
+        assert calls, name
+        del layer.__dict__[name]
