@@ -192,7 +192,7 @@ class SparseOptWrapper(torch.nn.Module):
             return False
         if _has_global_hook() or any(layer.__dict__[name] for name in _MODULE_HOOKS) or not _OVERRIDABLE.isdisjoint(layer.__dict__):
             return False
-        for variable in (layer._parameters["kernel_weights"], layer._parameters["bias"]):
+        for variable in (layer._parameters.get("kernel_weights"), layer._parameters.get("bias")):
             if (type(variable) is not torch.nn.Parameter or not variable.requires_grad or variable.grad is not None
                     or variable._backward_hooks or getattr(variable, "_post_accumulate_grad_hooks", None)
                     or variable.device != x.device or variable.dtype != torch.float32 or not variable.is_contiguous()):

@@ -395,3 +395,15 @@ def test_calls_replaced_on_a_class_are_made(ffi, monkeypatch):
         wrapper.train_step((x, y))
         assert calls, name
         del layer.__dict__[name]
+
+
+def test_a_variable_that_is_no_parameter_of_the_layer(ffi):
+    # computed from another one: the step trains that
+    wrapper, layer, adam, x, y = _training(ffi)
+    raw = torch.nn.Parameter(layer.kernel_weights.detach().clone())
+    del layer.kernel_weights
+    layer.kernel_weights = 1.0 * raw
+    wrapper.compile(ffi.SparseAdam([raw, layer.bias]), wrapper.loss, wrapper.metrics)
+    before = raw.detach().clone()
+    assert wrapper.train_step((x, y))["loss"] > 0.0
+    assert raw.grad is not None and not torch.equal(before, raw.detach())
