@@ -179,7 +179,9 @@ int input_grad_cached(const int32_t* lookup, const float* weights, const float* 
     if (p->ids_only || p->edited_by_library || (seen && !current)) {
         // the lookup changed under the plan (the calls since then were served by the recomputing kernels), or only passes that walk
         // no plan have met it in this content;
-        // the build fingerprints the present content, so this call needs no check
+        // the build fingerprints the present content, so this call needs no check.  The plan is laid out for this call's batch, not for the one
+        // that the lookup was first met with.
+        p->batch_hint = d.B;
         const int st = plan_build(p, lookup, s);
         if (st != FFI_OK) { drop_cached_plan(p); return st; }
         return passes(nullptr);

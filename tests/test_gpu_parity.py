@@ -876,6 +876,28 @@ def test_a_call_captured_behind_the_build_of_its_plan(ffi, shape):
     ffi._lib.check(lib.ffi_cache_clear())
 
 
+# (N, L, K), batches: a lookup met first by a few samples -- on a wide layer, on a narrow one, and on one whose few samples need no plan -- and edited
+@pytest.mark.parametrize("shape,few,many", [((3000, 5000, 40), 2, 130), ((500, 40_000, 40), 20, 300), ((300, 6000, 12), 2, 700), ((64, 30_000, 9), 30, 200)])
+def test_a_plan_built_anew_is_laid_out_for_the_batch_at_hand(ffi, shape, few, many):
+    N, L, K = shape
+    lib = ffi._lib.lib()
+    x, lookup, w, g = (dev(a) for a in reference_law_inputs(many, N, L, K, seed=L))
+    call = lambda B: ffi.fan_in_sparse_matmul_grad(x[:B].contiguous(), lookup, w, g[:B].contiguous())      # noqa: E731
+    ffi._lib.check(lib.ffi_cache_clear())
+    want = call(many)                                      # (what a first call gets)
+    ffi._lib.check(lib.ffi_cache_clear())
+    call(few)
+    ffi._lib.check(lib.ffi_lookup_edited(lookup.data_ptr()))
+    got = call(many)
+    # one layout, one order of sums
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    ffi._lib.check(lib.ffi_lookup_edited(lookup.data_ptr()))
+    want = call(few)
+    ffi._lib.check(lib.ffi_cache_clear())
+    got = call(few)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_plan_is_unusable_after_a_failed_refresh(ffi):
     # a rebuild that fails (here: an id out of range) leaves a plan without arrays; calls through it are refused
     # with a status instead of walking freed memory
