@@ -406,11 +406,18 @@ int launch_backward_dense_any(const float* x, const int32_t* idx, const float* w
 //   forward, up to 32 columns, fan-in from 16 on 1.1 to 3.5; of 8 to 15 up to 128 samples 1.0 to 1.5, above 0.9 to 1.4; of 4 and 5 0.6 to 1.4.  Up to
 //   16 samples the slices in LDS are faster (0.6 to 1.0).  33 to 64 columns: fan-in from 48 on 1.0 to 2.8; below, up to 64 samples 1.1 to 1.5 up to
 //   60,000 labels and 0.6 to 0.95 at 250,000; more samples 0.5 to 1.2.
-//   Both gradients, up to 32 columns: one group 1.2 to 15; two 0.87 (fan-in 5, 15,000 labels) to 4; four 0.55 at a fan-in of 4, 0.75 to 1.5 at 16, 1.0 to 3 at
-//   32.  33 to 64 columns: up to 32 samples 1.0 to 4.2; up to 64 1.1 to 2.2, 0.8 to 1.1 at 250,000 labels and fan-ins below 16; up to 128 0.6 to 1.3 at fan-ins below 20, 1.05 to 2.7
-//   from 28 on; more as the fan-in is to the groups (400 x 64 x 30,000 x 90 0.81), few labels excepted (256 x 64 x 2,000 x 90 0.87).
-//   Weight gradient alone: 1.0 to 3.6, but 0.6 to 1.0 for fan-ins from 40 on at 5,000 labels, where a wavefront has all connections of a tile, and 0.93 for
-//   400 samples, 33 to 64 columns and a fan-in of 5.
+//   Both gradients, one group: up to 32 columns 0.9 to 15; 33 to 64 up to 32 samples 1.0 to 4.2; up to 64 1.1 to 2.2, 0.8 to 1.1 at 250,000 labels and
+//   fan-ins below 16; up to 128 0.6 to 1.3 at fan-ins below 20, 1.05 to 2.7 from 28 on.
+// Each group more is another launch, of no more workgroups than there are tiles, where the others take all samples in one and spread few labels'
+// samples over the CUs.  Of 1,600 points more (130 to 200,000 samples, 64 to 200,000 labels):
+//   Both gradients, up to 32 columns: two groups 1.0 to 3.3, but 0.87 to 0.93 below 4,000 labels at fan-ins of 20 to 29 and 0.87 at 15,000 and 5; more 0.32
+//   (1,433 samples, 852 labels) to 0.8 below 8,192 labels, from there on 0.82 to 1.0 where there are fewer than 180,000 connections to a group and
+//   1.03 to 3.1 where there are more; three groups from 8,192 labels and a fan-in of 30 on 1.03 to 1.7.  33 to 64 columns: two groups 1.0 to 2.3 where the fan-in is
+//   50; more 0.83 to 0.96 up to 24,000 labels, 0.96 to 1.5 above.
+//   Weight gradient alone, one group: 1.0 to 3.9, but 0.6 to 1.0 for fan-ins from 40 on at 5,000 labels, where a wavefront has all connections of a tile.
+//   More of few labels 0.06 (171,000 samples, 378 labels: 2.3 ms and 36) to 0.7.  Up to 32 columns: two and three groups 1.1 to 1.7 from 16,384 labels
+//   on, but 0.6 to 0.8 at fan-ins below 8; more 0.4 to 0.95, from 80,000 labels (four groups: 50,000) or a million connections on 0.9 to 1.9.  33 to 64 columns:
+//   0.4 to 0.95, from 20,000 labels and 0.9 million (more than three groups: 2.2) connections on 0.89 to 2.2.
 bool takes_dense_forward(const Dims& d) {
     if (d.N > 64 || d.L >= (1 << 25) || d.B > 65535 * kDnSamples) return false;
     if (g_options.dense_rows != 0) return g_options.dense_rows > 0;
@@ -422,15 +429,21 @@ bool takes_dense_backward(const Dims& d) {
     if (d.N > 64 || d.L >= (1 << 25)) return false;
     if (g_options.dense_rows != 0) return g_options.dense_rows > 0;
     const int groups = (d.B + kDnSamples - 1) / kDnSamples;
-    if (d.N <= 32) return groups == 1 || d.K >= (d.L >= 16384 ? 5 : 10) * groups || (groups == 2 && d.L >= 32768);
-    if (groups > 1) return d.K >= 25 * groups && d.L >= 16384;
-    return d.B <= 32 || d.K >= 24 || (d.B <= 64 && (d.K >= 16 || d.L <= 100000));
+    if (groups == 1) return d.N <= 32 || d.B <= 32 || d.K >= 24 || (d.B <= 64 && (d.K >= 16 || d.L <= 100000));
+    if (d.N > 32) return d.K >= 25 * groups && d.L >= (groups == 2 ? 16384 : 24000);
+    if (groups == 2) return d.L >= 32768 || d.K >= (d.L >= 16384 ? 10 : d.L >= 4096 ? 20 : 32);
+    if (groups == 3 && d.L >= 8192 && d.K >= 30) return true;
+    return d.L >= 16384 && d.K >= 5 * groups && (long long)d.L * d.K >= 180000ll * groups;
 }
 bool takes_dense_weight_grad(const Dims& d) {
     if (d.N > 64 || d.L >= (1 << 25)) return false;
     if (g_options.dense_rows != 0) return g_options.dense_rows > 0;
-    if (d.N > 32 && d.B > 2 * kDnSamples && d.K < 16) return false;
-    return d.L >= 16384 || d.K <= 32;
+    const int groups = (d.B + kDnSamples - 1) / kDnSamples;
+    if (groups == 1) return d.L >= 16384 || d.K <= 32;
+    const long long connections = (long long)d.L * d.K;
+    if (d.N > 32) return d.L >= 20000 && connections >= (groups <= 3 ? 900000 : 2200000);
+    if (groups <= 3) return d.L >= 16384 && (d.K >= 8 || d.L >= 32768);
+    return d.L >= (groups == 4 ? 50000 : 80000) || (d.L >= 24000 && connections >= 1000000);
 }
 
 size_t dense_backward_workspace(const Dims& d) {

@@ -113,3 +113,32 @@ def test_an_id_out_of_range_is_reported_by_the_next_call(ffi):
         ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
     lookup[3, 2] = 49
     ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
+
+
+# More than one group of 128 samples: few labels' samples are spread over the CUs by the other kernels
+@pytest.mark.parametrize("shape", [(641, 32, 1035, 94), (1433, 32, 852, 126), (391, 32, 16_682, 40), (271, 64, 20_608, 92)])
+def test_many_samples_of_few_labels_take_the_other_kernels(shape):
+    _default_and_others(shape, True)
+
+
+@pytest.mark.parametrize("shape", [(20_000, 32, 1300, 14), (3000, 64, 1300, 30), (250, 43, 12_000, 20), (1200, 32, 12_000, 20), (2500, 32, 33_000, 6)])
+def test_weight_gradients_of_many_samples_take_the_other_kernels(shape):
+    _default_and_others(shape, False)
+
+
+def _default_and_others(shape, input_gradient):
+    # (the same kernels add in the same order)
+    B, N, L, K = shape
+    lib, stream = load_package()._lib.lib(), torch.cuda.current_stream().cuda_stream
+    x, lookup, w, g = (torch.from_numpy(a).cuda() for a in reference_law_inputs(B, N, L, K, seed=L))
+    results = []
+    try:
+        for dense in (0, -1):
+            assert lib.ffi_set_option(b"dense_rows", dense) == 0
+            gx, gw = torch.zeros_like(x), torch.empty_like(w)
+            assert lib.ffi_backward_f32(x.data_ptr(), lookup.data_ptr(), w.data_ptr(), g.data_ptr(), gx.data_ptr() if input_gradient else None, gw.data_ptr(),
+                                        B, N, L, K, 0, stream) == 0
+            results.append((gx, gw))
+    finally:
+        assert lib.ffi_set_option(b"dense_rows", 0) == 0
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
