@@ -8,7 +8,7 @@
 // move the scores, and no plan is built.
 // Semantics: tfsparse/cc/kernels/forward.cpp:9-44, backward.cpp:8-73 in the reference.  Connections of a label into one column are
 // added up before they meet the operand.  A column without a connection is a zero that meets the operand all the same, so
-// operands that are not finite are taken out and their products formed connection by connection.
+// operands that are not finite, and sums of weights that are not, are taken out and their products formed connection by connection.
 #include "ffi_internal.h"
 
 #include <algorithm>
@@ -66,12 +66,13 @@ __device__ __forceinline__ bool stage_features(const float* __restrict__ x, floa
     return odd;
 }
 
-// rows[lane][n] = the sum of the weights of label l0 + lane into column n; all zero behind the last label.  True where an id is out
-// of range (CLAMP: it counts as the last column, else not at all).
+// rows[lane][n] = the sum of the weights of label l0 + lane into column n; zero behind the last label, and where it is not finite: the
+// label's connections into such a column (a bit of *apart) are taken one by one, as what meets the sum may be zero or not finite itself, or it
+// is only the sum that overflows.  True where an id is out of range (CLAMP: it counts as the last column, else not at all).
 // A lane reads and writes its own row, one connection after the other.  Rows come in pieces of 16 bytes: with the 64 lanes on as many
 // lines, a piece costs the L1 what a word does.  (Forward 31 x 45 x 290,420 x 75: 196 us word by word, 85 so.)
 template <int NT, bool CLAMP>
-__device__ __forceinline__ bool write_rows(const int32_t* __restrict__ idx, const float* __restrict__ w, float* rows, int l0, int L, int N, int K) {
+__device__ __forceinline__ bool write_rows(const int32_t* __restrict__ idx, const float* __restrict__ w, float* rows, int l0, int L, int N, int K, unsigned long long* apart) {
     using S = DenseShape<NT>;
     const int lane = threadIdx.x & 63;
     float* mine = rows + lane * S::kPitch;
@@ -79,14 +80,24 @@ __device__ __forceinline__ bool write_rows(const int32_t* __restrict__ idx, cons
     const bool there = l0 + lane < L;
     const size_t row = (size_t)min(l0 + lane, L - 1) * K;
     bool bad = false;
+    float finite = 0.f;                                                   // NaN where a sum is not finite
     auto put = [&](unsigned id, float wv) {
         bad |= there && id >= (unsigned)N;
         const unsigned n = !there ? (unsigned)S::kColumns : CLAMP ? min(id, (unsigned)N - 1u) : min(id, id < (unsigned)N ? id : (unsigned)S::kColumns);
-        mine[n] += wv;
+        const float sum = mine[n] + wv;
+        finite = fmaf(sum, 0.f, finite);
+        mine[n] = sum;
+    };
+    auto done = [&]() {
+        *apart = 0ull;
+        if (there && !(finite == 0.f))
+            for (int n = 0; n < S::kColumns; ++n)
+                if (not_finite(mine[n])) { mine[n] = 0.f; *apart |= 1ull << n; }
+        return bad;
     };
     if (K < 4) {
         for (int k = 0; k < K; ++k) put((unsigned)idx[row + k], w[row + k]);
-        return bad;
+        return done();
     }
     constexpr int kQuads = 4;
     for (int k0 = 0; k0 < K; k0 += 4 * kQuads) {
@@ -106,12 +117,20 @@ __device__ __forceinline__ bool write_rows(const int32_t* __restrict__ idx, cons
                 if (v >= again) put(id[i].v[v], wv[i].v[v]);
         }
     }
-    return bad;
+    return done();
 }
 
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// *to += v, unless it is an infinity or a NaN that stays what it is: where no value is finite any more, all connections would add up in
+// N x B places.
+__device__ __forceinline__ void add_apart(float* to, float v) {
+    const float there = __hip_atomic_load(to, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (there != there || (not_finite(there) && (there == v || !not_finite(v)))) return;
+    unsafeAtomicAdd(to, v);
 }
 
 // Tile t of a wavefront: workgroups side by side first, so that few tiles spread over all CUs.
@@ -129,19 +148,24 @@ __global__ __launch_bounds__(64 * DenseShape<NT>::kForwardWaves) void fwd_dense_
     const bool odd = __syncthreads_or(stage_features<NT>(x, xs, B, N, b0, nb, width, tp));
     for (int t = blockIdx.x + gridDim.x * wave; t < tiles; t += gridDim.x * S::kForwardWaves) {
         const int l0 = t * kDnTile;
-        if (odd) {
-            // connection by connection
+        auto by_connections = [&]() {
+            const int l = l0 + lane;
             for (int b = 0; b < nb; ++b) {
-                const int l = min(l0 + lane, L - 1);
                 float sum = 0.f;
                 for (int k = 0; k < K; ++k) sum = fmaf(w[(size_t)l * K + k], xs[min((unsigned)idx[(size_t)l * K + k], (unsigned)N - 1u) * (width + 1) + b], sum);
-                if (l0 + lane < L) out[(size_t)(b0 + b) * L + l] = bias != nullptr ? sum + bias[l] : sum;
+                out[(size_t)(b0 + b) * L + l] = bias != nullptr ? sum + bias[l] : sum;
             }
+        };
+        if (odd) {
+            if (l0 + lane < L) by_connections();
             continue;
         }
+        unsigned long long apart;
         wave_lds_fence();
-        (void)write_rows<NT, true>(idx, w, rows, l0, L, N, K);
+        (void)write_rows<NT, true>(idx, w, rows, l0, L, N, K, &apart);
         wave_lds_fence();
+        const unsigned long long aparts = __ballot(apart != 0ull);
+        if (apart != 0ull) by_connections();
         float bj[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) bj[h] = bias != nullptr ? bias[min(l0 + 32 * h + low, L - 1)] : 0.f;
@@ -157,11 +181,12 @@ __global__ __launch_bounds__(64 * DenseShape<NT>::kForwardWaves) void fwd_dense_
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int l = l0 + 32 * h + low;
+                const bool stores = l < L && (aparts >> (32 * h + low) & 1ull) == 0ull;
                 float* to = out + (size_t)(b0 + bt) * L + l;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int b = product_row(r, lane);
-                    if (bt + b < nb && l < L) to[(size_t)b * L] = bias != nullptr ? acc[h][r] + bj[h] : acc[h][r];
+                    if (bt + b < nb && stores) to[(size_t)b * L] = bias != nullptr ? acc[h][r] + bj[h] : acc[h][r];
                 }
             }
         }
@@ -173,7 +198,7 @@ __global__ __launch_bounds__(64 * DenseShape<NT>::kForwardWaves) void fwd_dense_
 // read both ways -- as labels x samples for the weights' products with the features, as samples x labels for the columns' products
 // with the rows.  The columns' sums stay in registers for all tiles; at the end the workgroup adds its wavefronts' and leaves
 // them in part[workgroup][n][b].  The weights' products end up in the rows' place, from where each connection picks its column's.
-// A gradient that is not finite goes to `odd_sums` [N][B] connection by connection (zero between launches).
+// A gradient that is not finite, and a label's columns whose sums are not, go to `odd_sums` [N][B] connection by connection (zero between launches).
 template <int NT, int NB, bool GX, bool GW>
 __global__ __launch_bounds__((64 * DenseBackwardShape<NT, NB, GX, GW>::kWaves)) void bwd_dense_kernel(const float* __restrict__ x, const int32_t* __restrict__ idx,
                                                                              const float* __restrict__ w, const float* __restrict__ g,
@@ -205,9 +230,10 @@ __global__ __launch_bounds__((64 * DenseBackwardShape<NT, NB, GX, GW>::kWaves)) 
         };
         constexpr bool kAhead = !(NT == 2 && NB == 4 && GX && GW);         // (no registers left for it there)
         if (kAhead) ask(0);
+        unsigned long long apart = 0ull;
         if (GX) {
             wave_lds_fence();
-            seen_bad |= write_rows<NT, false>(idx, w, rows, l0, L, N, K);
+            seen_bad |= write_rows<NT, false>(idx, w, rows, l0, L, N, K, &apart);
         }
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
@@ -238,15 +264,16 @@ __global__ __launch_bounds__((64 * DenseBackwardShape<NT, NB, GX, GW>::kWaves)) 
                 }
             }
             if (GX) {
-                if (__ballot(!(finite == 0.f)) != 0ull) {
+                if (__ballot(apart != 0ull || !(finite == 0.f)) != 0ull) {
                     wave_lds_fence();
-                    for (int i = 0; i < 32; ++i) {
+                    for (int i = 0; i < min(32, nb - bt); ++i) {
                         const float v = gt[i * kDnGPitch + lane];
-                        if (!not_finite(v)) continue;
-                        gt[i * kDnGPitch + lane] = 0.f;
+                        const bool odd = not_finite(v);
+                        if (apart == 0ull && !odd) continue;
+                        if (odd) gt[i * kDnGPitch + lane] = 0.f;
                         for (int k = 0; k < K; ++k) {
                             const unsigned id = (unsigned)idx[(size_t)mine * K + k];
-                            if (id < (unsigned)N) atomicAdd(&odd_sums[(size_t)id * B + b0 + bt + i], w[(size_t)mine * K + k] * v);
+                            if (id < (unsigned)N && (odd || (apart >> id & 1ull) != 0ull)) add_apart(&odd_sums[(size_t)id * B + b0 + bt + i], w[(size_t)mine * K + k] * v);
                         }
                     }
                     wave_lds_fence();

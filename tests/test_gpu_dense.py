@@ -90,6 +90,56 @@ def test_what_is_not_finite_stays_with_its_connections(ffi, transposed):
     assert bool(torch.isfinite(gx).all())
 
 
+@pytest.mark.parametrize("B,N", [(40, 20), (130, 50)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_weights_that_add_up_to_no_finite_number(ffi, transposed, B, N):
+    # an infinite weight under an infinite gradient; weights of one column whose sum overflows and whose products with what they meet, zeros among
+    # that, do not; infinities that cancel; all of it beside other connections of the label, and in the last label
+    L, K = 200, 6
+    x, lookup, w, g = reference_law_inputs(B, N, L, K, seed=5)
+    x *= 0.1
+    g *= 0.1
+    lookup[70], w[70, 2], g[6, 70], g[7, 70] = np.arange(K), np.inf, -np.inf, np.inf
+    for l in (30, L - 1):
+        lookup[l] = [4, 9, 4, 9, 11, 12]
+        w[l, 0] = w[l, 2] = 3e38
+        w[l, 1] = w[l, 3] = -2.5e38
+    x[3, 4] = x[5, 9] = g[2, 30] = g[8, L - 1] = 0.0
+    lookup[100], w[100, 0], w[100, 3] = [15, 1, 2, 15, 3, 3], np.inf, -np.inf
+    g[9, 100] = np.nan
+    ref = np.zeros((B, L), np.float64)
+    gx_ref, gw_ref = np.zeros((B, N), np.float64), np.zeros((L, K), np.float64)
+    with np.errstate(invalid="ignore"):
+        for k in range(K):
+            ref += w[:, k].astype(np.float64) * x[:, lookup[:, k]]
+            gw_ref[:, k] = (g.astype(np.float64) * x[:, lookup[:, k]]).sum(0)
+            for l in range(L):
+                gx_ref[:, lookup[l, k]] += g[:, l].astype(np.float64) * w[l, k]
+    args = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x.T if transposed else x, lookup, w, g)]
+    forward, grad = (ffi.fan_in_sparse_matmul_tp, ffi.fan_in_sparse_matmul_grad_tp) if transposed else (ffi.fan_in_sparse_matmul, ffi.fan_in_sparse_matmul_grad)
+    for _ in range(2):
+        out = forward(*args[:3]).cpu().numpy()
+        gx, gw = (t.cpu().numpy() for t in grad(*args))
+        for got, want in ((out, ref), (gx.T if transposed else gx, gx_ref), (gw, gw_ref)):
+            np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+            np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+            np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+            ok = np.isfinite(want)
+            # (products of 3e38 and 0.1, a few of them, each rounded once: their sums may be off by 2^-22 of the largest)
+            np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-5 if np.abs(want[ok]).max() < 1e30 else 1e32)
+
+
+def test_nothing_finite(ffi):
+    B, N, L, K = 128, 32, 3000, 16
+    x, lookup, w, g = (torch.from_numpy(a).cuda() for a in reference_law_inputs(B, N, L, K, seed=9))
+    nan = float("nan")
+    for xs, ws, gs in ((x, torch.full_like(w, nan), torch.full_like(g, nan)), (x, w, torch.full_like(g, nan)), (x, torch.full_like(w, nan), g)):
+        gx, gw = ffi.fan_in_sparse_matmul_grad(xs, lookup, ws, gs)
+        assert bool(gx.isnan().all()) and bool(gw.isnan().all()) == bool(gs.isnan().all())
+    gx, gw = ffi.fan_in_sparse_matmul_grad(x, lookup, w, g)
+    assert bool(gx.isfinite().all()) and bool(gw.isfinite().all())
+
+
 def test_tiny_numbers_are_not_lost(ffi):
     # products and operands below the smallest normal number
     N, L, K = 8, 64, 2
