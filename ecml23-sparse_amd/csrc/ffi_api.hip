@@ -764,7 +764,7 @@ size_t ffi_workspace_bytes(int64_t batch, int64_t num_features, int64_t num_unit
             total += f.max_slots * 4 * (2 + at_once);                                   // entries; weights and weight gradients in their order
             total += L * K * 6 + (2 * units + 1) * 4;                                   // slot_of, tile_pos, chunk_ptr, chunk_count
             // counts while the plan is built; out_grad in slices and the sums per segment
-            partial_slot = std::max(partial_slot, global_build_words(f, (int)(((long long)d.L * d.K + (1ll << f.tile_bits) - 1) >> f.tile_bits)) * 4);
+            partial_slot = std::max(partial_slot, global_build_words(f, (long long)d.L * d.K) * 4);
             partial_slot = std::max(partial_slot, (L + (f.segments > 1 ? N * (size_t)f.segments : 0)) * padded * 4);
         }
     }

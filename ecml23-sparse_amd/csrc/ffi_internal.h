@@ -427,11 +427,11 @@ int plan_check_ids(ffi_plan* p, const int32_t* lookup, hipStream_t s);
 int plan_tile_labels(int N, int K, int L, int batch_hint, bool* weights_in_lds);
 // How the global form of a lookup is cut (`batch`: the batch size it is built for, 0 = unknown).
 struct GlobalShape {
-    int members, groups, segments, seg_labels, tile_bits;
+    int members, groups, segments, seg_labels, tile_bits, row_bits;      // (row_bits: positions of a row of tiles that the build counts together)
     size_t max_slots;
 };
 GlobalShape global_shape(int N, int K, int L, int batch);
-size_t global_build_words(const GlobalShape& f, int tiles);
+size_t global_build_words(const GlobalShape& f, long long total);
 int launch_arrange_in_place(int32_t* lookup, float* const* arrays, int n_arrays, int L, int K, hipStream_t s);
 // Content fingerprint of `lookup` (and the count of ids outside [0,N)).  _begin enqueues the kernel
 // on `s` and returns; _end waits for that kernel only, not for what the caller enqueued on `s`

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <type_traits>
 
 namespace ffi {
 namespace {
@@ -444,25 +445,54 @@ __global__ __launch_bounds__(1024) void slice_scan_kernel(const unsigned* __rest
                                                            int n, int group, unsigned long long* __restrict__ total_out) {
     constexpr int kAtOnce = 16;
     const int per = (n + 1023) / 1024;
-    const int b = min((int)threadIdx.x * per, n), e = min(b + per, n);
-    unsigned long long sum = 0, total = 0;
-    unsigned v[kAtOnce];                                                  // (the last ones asked for stay)
-    auto ask = [&](int i0) {
-#pragma unroll
-        for (int i = 0; i < kAtOnce; ++i) v[i] = i0 + i < e ? len[i0 + i] : 0u;
-    };
-    for (int i0 = b; i0 < e; i0 += kAtOnce) {
-        ask(i0);
-#pragma unroll
-        for (int i = 0; i < kAtOnce; ++i) sum += v[i];
-    }
-    unsigned long long run = block_sum_below<1024>(sum, &total);
-    for (int i0 = b; i0 < e; i0 += kAtOnce) {
-        if (per > kAtOnce) ask(i0);
+    unsigned long long total = 0;
+    if (per <= kAtOnce) {
+        const int b = min((int)threadIdx.x * per, n), e = min(b + per, n);
+        unsigned long long sum = 0;
+        unsigned v[kAtOnce];
 #pragma unroll
         for (int i = 0; i < kAtOnce; ++i) {
-            if (i0 + i < e) off[i0 + i] = (unsigned)run;
+            v[i] = b + i < e ? len[b + i] : 0u;
+            sum += v[i];
+        }
+        unsigned long long run = block_sum_below<1024>(sum, &total);
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            if (b + i < e) off[b + i] = (unsigned)run;
             run += v[i];
+        }
+    } else {
+        // (very many columns: a stretch at a time, whose values come and go by whole lines)
+        constexpr int kEach = 8, kStretch = 1024 * kEach;
+        __shared__ unsigned stage[kStretch + kStretch / kEach];
+        auto place = [](int i) { return i + i / kEach; };
+        for (int n0 = 0; n0 < n; n0 += kStretch) {
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                const int at = i * 1024 + (int)threadIdx.x;
+                stage[place(at)] = n0 + at < n ? len[n0 + at] : 0u;
+            }
+            __syncthreads();
+            unsigned long long sum = 0, all = 0;
+            unsigned v[kEach];
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                v[i] = stage[place((int)threadIdx.x * kEach + i)];
+                sum += v[i];
+            }
+            unsigned long long run = total + block_sum_below<1024>(sum, &all);
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                stage[place((int)threadIdx.x * kEach + i)] = (unsigned)run;
+                run += v[i];
+            }
+            total += all;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                const int at = i * 1024 + (int)threadIdx.x;
+                if (n0 + at < n) off[n0 + at] = stage[place(at)];
+            }
         }
     }
     if (threadIdx.x == 1023) {
@@ -669,7 +699,7 @@ struct StreamOf {
     }
 };
 
-// counts[t][u] = connections of stream u in tile t, a workgroup per tile; so many streams at a time as the LDS has counters
+// counts[t][u] = connections of stream u in tile t (or row of tiles: `tile_bits` is theirs), a workgroup per tile; so many streams at a time as the LDS has counters
 constexpr int kTileThreads = 1024, kCountWindow = 16384;
 __global__ __launch_bounds__(kTileThreads) void tile_streams_kernel(const int32_t* __restrict__ idx, int total, int tile_bits, int units,
                                                                     const StreamOf stream_of, unsigned* __restrict__ counts) {
@@ -742,132 +772,167 @@ __global__ __launch_bounds__(kTileThreads) void stream_counts_kernel(unsigned* _
 // stretches of it: they count their connections per stream, sums over streams and wavefronts turn the counts into places, and the
 // stretches are gone through again, 64 connections at a time, each of which takes the place it finds and leaves the next one there (of
 // several of one stream among the 64 the lanes' order decides, not the LDS's).  Places gather in LDS and leave by whole runs.
-// As many wavefronts as the counters of 16 bits leave room for.
+// As many wavefronts walk as the counters of 16 bits leave room for; the others help with the counters and the runs, which are all
+// there is to do where a tile has fewer connections than there are streams.  A workgroup takes the tiles of a row of `before` in turn and moves
+// the row on (one tile, unless the rows of single tiles would take too much memory).
 constexpr size_t kTileCounterBytes = 61440;
-__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const int32_t* __restrict__ idx, int total, int tile_bits, int units, const StreamOf stream_of,
-                                                                 const unsigned* __restrict__ before, const unsigned* __restrict__ begin,
+__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const int32_t* __restrict__ idx, int total, int tile_bits, int row_tiles, int units, const StreamOf stream_of,
+                                                                 unsigned* __restrict__ before, const unsigned* __restrict__ begin,
                                                                  unsigned short* __restrict__ tile_pos, unsigned* __restrict__ place_of,
-                                                                 unsigned* __restrict__ list, int window) {
+                                                                 unsigned* __restrict__ list, int window, int walkers) {
     extern __shared__ __align__(16) unsigned tile_lds[];
     __shared__ unsigned wave_sums[kTileThreads / 64];
     constexpr int kInflight = 8;
-    const int nthreads = blockDim.x, nwaves = nthreads >> 6, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned tile = 1u << tile_bits, p0 = blockIdx.x << tile_bits, n = min(tile, (unsigned)total - p0);
+    constexpr int nthreads = kTileThreads;
+    const int nwaves = walkers, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned tile = 1u << tile_bits;
     unsigned short* const stage_pos = reinterpret_cast<unsigned short*>(tile_lds);                       // [tile]
     unsigned char* const stage_col = reinterpret_cast<unsigned char*>(tile_lds) + 2 * (size_t)tile;      // [tile]
     unsigned* const counters = tile_lds + 3 * (size_t)tile / 4;                                          // [wave][window / 2] two streams a word
     const int words = window / 2;
     unsigned* const mine = counters + (size_t)wave * words;
-    const unsigned stretch = ((n + nwaves - 1) / nwaves + 63) & ~63u, from = min(wave * stretch, n), to = min(from + stretch, n);
-    unsigned placed = 0;                                                                                 // connections of the streams before the window
-    for (int u0 = 0; u0 < units; u0 += window) {
-        const unsigned streams = (unsigned)min(window, units - u0);
-        for (int i = threadIdx.x; i < nwaves * words; i += nthreads) counters[i] = 0u;
-        __syncthreads();
-        auto walk = [&](auto visit) {
-            unsigned next[kInflight];
-            auto fetch = [&](unsigned e0) {
+    before += (size_t)blockIdx.x * units;
+    for (int t = 0; t < row_tiles; ++t) {
+        const unsigned p0 = (blockIdx.x * (unsigned)row_tiles + t) << tile_bits;
+        if (p0 >= (unsigned)total) break;
+        const unsigned n = min(tile, (unsigned)total - p0), stretch = ((n + nwaves - 1) / nwaves + 63) & ~63u;
+        const unsigned from = wave < nwaves ? min(wave * stretch, n) : n, to = min(from + stretch, n);
+        unsigned placed = 0;                                                                                 // connections of the streams before the window
+        for (int u0 = 0; u0 < units; u0 += window) {
+            const unsigned streams = (unsigned)min(window, units - u0);
+            for (int i = threadIdx.x; i < nwaves * words; i += nthreads) counters[i] = 0u;
+            __syncthreads();
+            auto walk = [&](auto visit) {
+                if (from >= to) return;
+                unsigned next[kInflight];
+                auto fetch = [&](unsigned e0) {
 #pragma unroll
-                for (int i = 0; i < kInflight; ++i) next[i] = (unsigned)idx[p0 + min(e0 + 64 * i + lane, n - 1)];
+                    for (int i = 0; i < kInflight; ++i) next[i] = (unsigned)idx[p0 + min(e0 + 64 * i + lane, n - 1)];
+                };
+                fetch(from);
+                for (unsigned e0 = from; e0 < to; e0 += 64 * kInflight) {
+                    unsigned id[kInflight], u[kInflight];
+#pragma unroll
+                    for (int i = 0; i < kInflight; ++i) {
+                        const unsigned e = e0 + 64 * i + lane;
+                        id[i] = next[i];
+                        u[i] = stream_of(id[i], p0 + e) - (unsigned)u0;
+                        if (e >= to || u[i] >= streams) u[i] = ~0u;
+                    }
+                    fetch(e0 + 64 * kInflight);
+                    visit(id, u, e0 + lane);
+                }
             };
-            fetch(from);
-            for (unsigned e0 = from; e0 < to; e0 += 64 * kInflight) {
-                unsigned id[kInflight], u[kInflight];
+            walk([&](const unsigned*, const unsigned* u, unsigned) {
+#pragma unroll
+                for (int i = 0; i < kInflight; ++i)
+                    if (u[i] != ~0u) atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
+            });
+            __syncthreads();
+            // each thread takes consecutive pairs of streams: their connections, those of the threads before it, and the places
+            const int per = (words + nthreads - 1) / nthreads, w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
+            unsigned sum = 0;
+            for (int w = w0; w < w1; ++w)
+                for (int v = 0; v < nwaves; ++v) {
+                    const unsigned c = counters[(size_t)v * words + w];
+                    sum += (c & 0xffffu) + (c >> 16);
+                }
+            unsigned upto = sum;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned below = __shfl_up(upto, off, 64);
+                if (lane >= off) upto += below;
+            }
+            if (lane == 63) wave_sums[wave] = upto;
+            __syncthreads();
+            unsigned run = placed + upto - sum, all = 0;
+#pragma unroll
+            for (int v = 0; v < nthreads / 64; ++v) {
+                run += v < wave ? wave_sums[v] : 0u;
+                all += wave_sums[v];
+            }
+            for (int w = w0; w < w1; ++w) {
+                unsigned even = run, odd = 0;
+                for (int v = 0; v < nwaves; ++v) odd += counters[(size_t)v * words + w] & 0xffffu;
+                odd += run;
+                for (int v = 0; v < nwaves; ++v) {
+                    const unsigned c = counters[(size_t)v * words + w];
+                    counters[(size_t)v * words + w] = (even & 0xffffu) | odd << 16;
+                    even += c & 0xffffu;
+                    odd += c >> 16;
+                }
+                run = odd;
+            }
+            __syncthreads();
+            walk([&](const unsigned* id, const unsigned* u, unsigned e) {
+                unsigned found[kInflight], there[kInflight];
 #pragma unroll
                 for (int i = 0; i < kInflight; ++i) {
-                    const unsigned e = e0 + 64 * i + lane;
-                    id[i] = next[i];
-                    u[i] = stream_of(id[i], p0 + e) - (unsigned)u0;
-                    if (e >= to || u[i] >= streams) u[i] = ~0u;
+                    there[i] = found[i] = 0u;
+                    if (u[i] != ~0u) {
+                        there[i] = mine[u[i] >> 1];
+                        found[i] = atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
+                    }
                 }
-                fetch(e0 + 64 * kInflight);
-                visit(id, u, e0 + lane);
-            }
-        };
-        walk([&](const unsigned*, const unsigned* u, unsigned) {
 #pragma unroll
-            for (int i = 0; i < kInflight; ++i)
-                if (u[i] != ~0u) atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
-        });
-        __syncthreads();
-        // each thread takes consecutive pairs of streams: their connections, those of the threads before it, and the places
-        const int per = (words + nthreads - 1) / nthreads, w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
-        unsigned sum = 0;
-        for (int w = w0; w < w1; ++w)
-            for (int v = 0; v < nwaves; ++v) {
-                const unsigned c = counters[(size_t)v * words + w];
-                sum += (c & 0xffffu) + (c >> 16);
-            }
-        unsigned upto = sum;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned below = __shfl_up(upto, off, 64);
-            if (lane >= off) upto += below;
-        }
-        if (lane == 63) wave_sums[wave] = upto;
-        __syncthreads();
-        unsigned run = placed + upto - sum, all = 0;
-        for (int v = 0; v < nwaves; ++v) {
-            run += v < wave ? wave_sums[v] : 0u;
-            all += wave_sums[v];
-        }
-        for (int w = w0; w < w1; ++w) {
-            unsigned even = run, odd = 0;
-            for (int v = 0; v < nwaves; ++v) odd += counters[(size_t)v * words + w] & 0xffffu;
-            odd += run;
-            for (int v = 0; v < nwaves; ++v) {
-                const unsigned c = counters[(size_t)v * words + w];
-                counters[(size_t)v * words + w] = (even & 0xffffu) | odd << 16;
-                even += c & 0xffffu;
-                odd += c >> 16;
-            }
-            run = odd;
-        }
-        __syncthreads();
-        walk([&](const unsigned* id, const unsigned* u, unsigned e) {
-            unsigned found[kInflight], there[kInflight];
-#pragma unroll
-            for (int i = 0; i < kInflight; ++i) {
-                there[i] = found[i] = 0u;
-                if (u[i] != ~0u) {
-                    there[i] = mine[u[i] >> 1];
-                    found[i] = atomicAdd(&mine[u[i] >> 1], 1u << (16 * (u[i] & 1)));
+                for (int i = 0; i < kInflight; ++i) {
+                    const unsigned shift = 16 * (u[i] & 1);
+                    unsigned at = there[i] >> shift & 0xffffu;
+                    for (unsigned long long left = __ballot(u[i] != ~0u && (found[i] >> shift & 0xffffu) != at); left != 0ull;) {
+                        const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)u[i], __builtin_ctzll(left));
+                        const unsigned long long same = __ballot(u[i] == k);
+                        if (u[i] == k) at += (unsigned)__popcll(same & ((1ull << lane) - 1ull));
+                        left &= ~same;
+                    }
+                    if (u[i] != ~0u) {
+                        stage_pos[at] = (unsigned short)(e + 64 * i);
+                        stage_col[at] = (unsigned char)(id[i] % kGroupColumns);
+                    }
                 }
-            }
+            });
+            __syncthreads();
+            // eight lanes to a run, or one, whose places are asked for four runs at a time; behind the walk the last wavefront's counter of a stream is
+            // the end of its run
+            const unsigned* const last = counters + (size_t)(nwaves - 1) * words;
+            auto end_of = [&](unsigned u) { return last[u >> 1] >> (16 * (u & 1)) & 0xffffu; };
+            auto leave = [&](auto lanes) {
+                constexpr int kRuns = 4, kLanes = decltype(lanes)::value;
+                for (unsigned u = threadIdx.x / kLanes; u < streams; u += kRuns * nthreads / kLanes) {
+                    unsigned start[kRuns], end[kRuns], there[kRuns], first[kRuns];
 #pragma unroll
-            for (int i = 0; i < kInflight; ++i) {
-                const unsigned shift = 16 * (u[i] & 1);
-                unsigned at = there[i] >> shift & 0xffffu;
-                for (unsigned long long left = __ballot(u[i] != ~0u && (found[i] >> shift & 0xffffu) != at); left != 0ull;) {
-                    const unsigned k = (unsigned)__builtin_amdgcn_readlane((int)u[i], __builtin_ctzll(left));
-                    const unsigned long long same = __ballot(u[i] == k);
-                    if (u[i] == k) at += (unsigned)__popcll(same & ((1ull << lane) - 1ull));
-                    left &= ~same;
+                    for (int i = 0; i < kRuns; ++i) {
+                        const unsigned v = u + i * (nthreads / kLanes);
+                        start[i] = end[i] = there[i] = first[i] = 0u;
+                        if (v < streams) {
+                            start[i] = v > 0 ? end_of(v - 1) : placed;
+                            end[i] = end_of(v);
+                        }
+                        if (start[i] != end[i]) {
+                            there[i] = before[(unsigned)u0 + v];
+                            first[i] = begin[(unsigned)u0 + v];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < kRuns; ++i) {
+                        if (start[i] == end[i]) continue;
+                        const unsigned stream = (unsigned)u0 + u + i * (nthreads / kLanes), base = first[i] + there[i] - start[i];
+                        const int label0 = (int)(stream / (unsigned)stream_of.groups) * stream_of.seg_labels;
+                        for (unsigned q = start[i] + threadIdx.x % kLanes; q < end[i]; q += kLanes) {
+                            const unsigned pos = stage_pos[q];
+                            tile_pos[p0 + q] = (unsigned short)pos;
+                            place_of[p0 + q] = base + q;
+                            list[base + q] = (unsigned)((int)((p0 + pos) / (unsigned)stream_of.K) - label0) << 8 | stage_col[q];
+                        }
+                        if (row_tiles > 1 && threadIdx.x % kLanes == 0) before[stream] = there[i] + end[i] - start[i];
+                    }
                 }
-                if (u[i] != ~0u) {
-                    stage_pos[at] = (unsigned short)(e + 64 * i);
-                    stage_col[at] = (unsigned char)(id[i] % kGroupColumns);
-                }
-            }
-        });
-        __syncthreads();
-        // eight lanes to a run; behind the walk the last wavefront's counter of a stream is the end of its run
-        const unsigned* const last = counters + (size_t)(nwaves - 1) * words;
-        auto end_of = [&](unsigned u) { return last[u >> 1] >> (16 * (u & 1)) & 0xffffu; };
-        for (unsigned u = threadIdx.x / 8; u < streams; u += nthreads / 8) {
-            const unsigned start = u > 0 ? end_of(u - 1) : placed, end = end_of(u), stream = (unsigned)u0 + u;
-            if (start == end) continue;
-            const unsigned base = begin[stream] + before[(size_t)blockIdx.x * units + stream] - start;
-            const int label0 = (int)(stream / (unsigned)stream_of.groups) * stream_of.seg_labels;
-            for (unsigned q = start + (threadIdx.x & 7); q < end; q += 8) {
-                const unsigned pos = stage_pos[q];
-                tile_pos[p0 + q] = (unsigned short)pos;
-                place_of[p0 + q] = base + q;
-                list[base + q] = (unsigned)((int)((p0 + pos) / (unsigned)stream_of.K) - label0) << 8 | stage_col[q];
-            }
+            };
+            // (short runs: a lane to each)
+            if (n < (unsigned)units) leave(std::integral_constant<int, 1>{});
+            else leave(std::integral_constant<int, 8>{});
+            placed += all;
+            __syncthreads();
         }
-        placed += all;
-        __syncthreads();
     }
 }
 
@@ -1029,6 +1094,8 @@ void dev_release(ffi_plan* p, void* ptr) {
 // slices.  128 samples and more, 1,300 to 2,500 columns want a segment on every CU; 2 samples, 22,133 columns, 200,058 labels, fan-in 8
 // two of them (walk 31 us; 40 with eight, whose three rounds are a little less of the connections).
 // Labels and rows of a segment stay within the entries and 32-bit offsets.
+// Counts per tile and stream: at most kMostCounts of them, 1 GB, and rows of several tiles where that is not enough.
+constexpr long long kMostCounts = 1ll << 28;
 GlobalShape global_shape(int N, int K, int L, int batch) {
     GlobalShape f{};
     f.members = batch > 0 && batch <= 32 ? 8 : 4;
@@ -1046,14 +1113,18 @@ GlobalShape global_shape(int N, int K, int L, int batch) {
     f.segments = (L + f.seg_labels - 1) / f.seg_labels;
     f.tile_bits = 10;
     while (f.tile_bits < 15 && total / (2 << f.tile_bits) >= 2.0 * device_cu_count()) ++f.tile_bits;
+    // (many streams: their counts, four bytes for every tile and stream, are written once and read three times)
+    while (f.tile_bits < 15 && total / (2 << f.tile_bits) >= device_cu_count() && total / (1 << f.tile_bits) * f.segments * f.groups > (double)(1 << 26)) ++f.tile_bits;
+    f.row_bits = f.tile_bits;
+    while (std::ceil(total / std::ldexp(1.0, f.row_bits)) * f.segments * f.groups > (double)kMostCounts && f.row_bits < 31) ++f.row_bits;
     const double streams = std::min((double)f.segments * f.groups, total);
     const int entries = kChunkSteps * f.members;
     f.max_slots = ((size_t)((total + streams * (kGroupColumns * (f.members - 1) + entries - 1)) / entries) + 1) * entries;
     return f;
 }
 
-// counts per tile and stream, per stream, and the two sums over the streams
-size_t global_build_words(const GlobalShape& f, int tiles) { return ((size_t)tiles + 3) * f.segments * f.groups + 1; }
+// counts per row of tiles and stream, per stream, and the two sums over the streams
+size_t global_build_words(const GlobalShape& f, long long total) { return ((size_t)((total + (1ll << f.row_bits) - 1) >> f.row_bits) + 3) * f.segments * f.groups + 1; }
 
 // Labels per tile of the tiled form, and whether the walking kernel keeps the tile's weights in LDS (then the tiles
 // are smaller).
@@ -1241,19 +1312,19 @@ int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     p->chunk_ptr = p->entries + f.max_slots;
     p->chunk_count = p->chunk_ptr + units + 1;
     p->tile_pos = reinterpret_cast<unsigned short*>(p->slot_of + places);
-    const int tiles = (int)(((long long)total + (1ll << f.tile_bits) - 1) >> f.tile_bits);
+    const int rows = (int)(((long long)total + (1ll << f.row_bits) - 1) >> f.row_bits);
     unsigned *list = nullptr, *slot_at = nullptr, *counts = nullptr;
     FFI_TRY(workspace_get(s, kWsSlots, f.max_slots * sizeof(unsigned), (void**)&list));
     FFI_TRY(workspace_get(s, kWsWeightParts, f.max_slots * sizeof(unsigned), (void**)&slot_at));
-    FFI_TRY(workspace_get(s, kWsPartials, global_build_words(f, tiles) * sizeof(unsigned), (void**)&counts));
-    unsigned* const of_stream = counts + (size_t)tiles * units;
+    FFI_TRY(workspace_get(s, kWsPartials, global_build_words(f, total) * sizeof(unsigned), (void**)&counts));
+    unsigned* const of_stream = counts + (size_t)rows * units;
     unsigned *const begin = of_stream + units, *const chunks = begin + units + 1;
     const StreamOf stream_of{p->K, f.seg_labels, f.segments, f.groups};
     unsigned long long* total_out = nullptr;
     FFI_HIP_TRY(hipHostGetDevicePointer((void**)&total_out, p->h_scratch, 0));
     const size_t count_lds = (size_t)std::min<long long>(units, kCountWindow) * sizeof(unsigned);
-    hipLaunchKernelGGL(tile_streams_kernel, dim3((unsigned)tiles), dim3(kTileThreads), count_lds, s, lookup, total, f.tile_bits, (int)units, stream_of, counts);
-    hipLaunchKernelGGL(stream_counts_kernel, dim3((unsigned)((units + 63) / 64)), dim3(kTileThreads), 0, s, counts, tiles, (int)units, f.members,
+    hipLaunchKernelGGL(tile_streams_kernel, dim3((unsigned)rows), dim3(kTileThreads), count_lds, s, lookup, total, f.row_bits, (int)units, stream_of, counts);
+    hipLaunchKernelGGL(stream_counts_kernel, dim3((unsigned)((units + 63) / 64)), dim3(kTileThreads), 0, s, counts, rows, (int)units, f.members,
                        of_stream, chunks);
     hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, of_stream, begin, (int)units, 0, total_out);
     hipLaunchKernelGGL(slice_scan_kernel, dim3(1), dim3(1024), 0, s, chunks, p->chunk_ptr, (int)units, 0, total_out);
@@ -1261,8 +1332,8 @@ int build_global(ffi_plan* p, const int32_t* lookup, hipStream_t s) {
     const int waves = (int)std::max<size_t>(1, std::min<size_t>(kTileThreads / 64, kTileCounterBytes / (2 * (size_t)window)));
     const size_t sort_lds = ((size_t)3 << f.tile_bits) + (size_t)waves * window * 2;
     FFI_HIP_TRY(hipFuncSetAttribute((const void*)tile_sort_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sort_lds));
-    hipLaunchKernelGGL(tile_sort_kernel, dim3((unsigned)tiles), dim3((unsigned)waves * 64), sort_lds, s, lookup, total, f.tile_bits, (int)units, stream_of,
-                       counts, begin, p->tile_pos, p->slot_of, list, window);
+    hipLaunchKernelGGL(tile_sort_kernel, dim3((unsigned)rows), dim3(kTileThreads), sort_lds, s, lookup, total, f.tile_bits, 1 << (f.row_bits - f.tile_bits), (int)units, stream_of,
+                       counts, begin, p->tile_pos, p->slot_of, list, window, waves);
     const auto stream_steps = f.members == 4 ? stream_steps_kernel<4> : stream_steps_kernel<8>;
     hipLaunchKernelGGL(stream_steps, dim3((unsigned)((units + kStepWaves - 1) / kStepWaves)), dim3(kStepWaves * 64), 0, s, list, begin, p->chunk_ptr,
                        (int)units, p->entries, slot_at, p->chunk_count);

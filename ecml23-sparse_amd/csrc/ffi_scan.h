@@ -8,7 +8,7 @@ namespace ffi {
 
 #if defined(__HIPCC__)
 // The sum of `v` over the threads below this one, and over all THREADS of them in *total; THREADS a multiple of 64.  Called by the
-// whole workgroup, once per kernel.
+// whole workgroup; a barrier comes between two calls of it.
 template <int THREADS>
 __device__ __forceinline__ unsigned long long block_sum_below(unsigned long long v, unsigned long long* total) {
     __shared__ unsigned long long of_wave[THREADS / 64];

@@ -74,3 +74,12 @@ def test_option_names_and_ranges_are_checked():
                         (b"workgroups_per_cu", 2), (b"plan_sorted_columns", -1), (b"plan_sorted_columns", 1)):
         assert lib.ffi_set_option(name, value) == 0
         assert lib.ffi_set_option(name, 0) == 0
+
+
+def test_a_layer_of_very_many_columns_asks_for_memory_that_a_gpu_has():
+    # what the backward pass holds grows with the connections and with the columns, not with their product
+    lib = load_package()._lib.lib()
+    for columns, labels, fan_in in ((100_000_000, 10_000_000, 100), (17_000_000, 522_240, 4), (1_000_000, 1_000_000, 64)):
+        held = lib.ffi_workspace_bytes(1, columns, labels, fan_in, 0, 2)
+        # 27 bytes a connection, and a column's share of its stream: 4 chunk words and 2 chunks of 128 entries of 12 bytes; 1 GB of counts
+        assert 0 < held <= 27 * labels * fan_in + columns // 32 * (16 + 2 * 128 * 12) + (5 << 28)

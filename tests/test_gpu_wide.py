@@ -184,9 +184,11 @@ def test_backward_over_many_label_blocks(ffi, B, N, L, K, transposed):
 
 # The walk over streams of 32 columns: (batches of the calls in turn -- the first one's plan has steps of four or eight connections and
 # serves the others --, N, L, K).  One column behind whole groups; streams of no, one and several chunks; several segments, several
-# slices in a launch and several launches; tiles of exactly their positions and one more; more streams than the build counts at a time
+# slices in a launch and several launches; tiles of exactly their positions and one more; more streams than the build counts at a time, and
+# so many that its tiles grow and their counts come in rows
 WALK_SHAPES = [((20, 70, 3), 1249, 5000, 7), ((70, 20, 200), 1248, 5000, 7), ((1, 130), 1300, 9000, 72), ((300, 33), 2500, 3001, 33),
-               ((64,), 1300, 1024, 1), ((32,), 1300, 1025, 1), ((65, 64), 40_000, 20_011, 12), ((3, 40), 1_000_000, 300, 4)]
+               ((64,), 1300, 1024, 1), ((32,), 1300, 1025, 1), ((65, 64), 40_000, 20_011, 12), ((3, 40), 1_000_000, 300, 4),
+               ((5,), 2_400_000, 70_001, 15), ((2,), 17_000_000, 522_240, 4)]
 
 
 @pytest.mark.parametrize("shape", WALK_SHAPES, ids=str)
