@@ -130,11 +130,11 @@ void drop_cached_plan(ffi_plan* p) {
 // Input gradient through the plan cache, with `between(plan)` (the weight-gradient launch, or
 // nothing) enqueued ahead of it.  The host never waits in the steady state (the reference's op only
 // enqueues, tfsparse/cc/kernels/backward.cu:59-64): the lookup's content is checked against the cached
-// plan by workgroups of the last plan-driven kernel, which leave their verdict on the device -- those kernels read the
-// plan, never the lookup, so they are safe whatever the lookup holds now -- and behind them comes what
+// plan by workgroups of a plan-driven kernel (the tiled form's last one, the global form's first), which leave their verdict on the
+// device -- those kernels read the plan, never the lookup, so they are safe whatever the lookup holds now -- and behind them comes what
 // recomputes both gradients straight from the lookup if the verdict says the plan is outdated (a rewire),
 // and returns at once otherwise.  The host looks at the verdict of an earlier call when that has arrived
-// (a poll, not a wait) and only then rebuilds the plan, which does synchronise.
+// (a poll, not a wait) and only then rebuilds the plan, whose ids it waits for.
 template <class Between>
 int input_grad_cached(const int32_t* lookup, const float* weights, const float* out_grad, float* feature_grad,
                       const Dims& d, hipStream_t s, Between between, const PlannedWeightGrad& wg = PlannedWeightGrad()) {

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kRedoThreads) void redo_backward_kernel(const RedoA
 // connection's row of out_grad comes from the slices that the passes over the plan left in their slot; eight are fetched at once.
 // Bound by the steps of 32,768 ids, some 15 us each: what 16 wavefronts pick out of the lists, two barriers and a round trip for rows.
 // One thread a connection, its samples one by one and its input gradient by atomics in memory (the kernel above), the whole call at
-// 128 x 65,536 x 670,091 x 72: 313 ms, 45 so (16 ids a thread, all eight rows fetched also where fewer are left: 64; the next ids
+// 128 x 65,536 x 670,091 x 72: 313 ms, 45 so, with 84 to 108 bytes of spills (16 ids a thread, all eight rows fetched also where fewer are left: 64; the next ids
 // in registers of their own, 152 bytes of spills: 47); at 50 x 32,768 x 670,000 x 32 51 and 10.2, at 128 x 1,300 x 100,000 x 32 14.9 and 2.8.
 constexpr int kOutIds = 32, kOutWaves = 16, kOutThreads = 64 * kOutWaves, kOutList = 256, kOutFetch = 8;
 constexpr int kOutTile = 16384;                // floats of a tile

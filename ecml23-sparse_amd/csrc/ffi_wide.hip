@@ -157,9 +157,6 @@ template <int BIT> __device__ __forceinline__ float fold(float a, float b, int l
     return dpp_add<BIT == 8 ? kRor8 : BIT == 4 ? kHalfMirror : BIT == 2 ? kQuadHalves : kQuadSwap>(up ? b : a, up ? a : b);
 }
 
-// sums[column of a step] += w * g, for two steps: the registers that hold component c of all columns are consecutive ones, and
-// the step's column is what is added to the number of the first.  (In one piece, so that nothing else executes while registers are
-// indexed.  The columns are below 32: the plan's entries hold nothing else there.)
 // Pairs of lanes that are 32 or 16 apart add up: a in the lower one, b in the other.
 template <int BIT> __device__ __forceinline__ float fold_halves(float a, float b) {
     static_assert(BIT == 32 || BIT == 16);
@@ -170,6 +167,9 @@ template <int BIT> __device__ __forceinline__ float fold_halves(float a, float b
     return __builtin_bit_cast(float, u) + __builtin_bit_cast(float, v);
 }
 
+// sums[column of a step] += w * g, for two steps: the registers that hold component c of all columns are consecutive ones, and
+// the step's column is what is added to the number of the first.  (In one piece, so that nothing else executes while registers are
+// indexed.  The columns are below 32: the plan's entries hold nothing else there.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"                  // (M0 is clobbered, and said to be)
 __device__ __forceinline__ void add_steps(f32x32 (&sum)[4], unsigned col0, float w0, const float4& g0, unsigned col1, float w1, const float4& g1) {

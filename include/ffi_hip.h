@@ -107,9 +107,10 @@ int ffi_forward_noalloc_f32(const float* features, const int32_t* lookup, const 
  * which is built on the device on first use and cached inside the library, keyed on the lookup
  * pointer and shape, so in-place edits of lookup (rewiring, sparse/custom_layer.py:32-43) must be picked up:
  *   - edits made through this library (ffi_rewire_f32, ffi_arrange_connections_f32) mark the cached view outdated
- *     on the host, and the next backward call rebuilds it before it enqueues anything (that call synchronises
- *     `stream` and takes the time of a plan build, 0.75 ms at 768 columns and 670,091 x 32 connections; results stay
- *     bit-reproducible);
+ *     on the host, and the next backward call rebuilds it before it enqueues anything, for the batch of that call (the
+ *     host waits until the ids are checked, behind the work that `stream` holds; the kernels that lay the view out, 0.34 ms at
+ *     768 columns and 670,091 x 32 connections, run ahead of the call's own, and calls on other streams, captured ones
+ *     among them, wait for them; results stay bit-reproducible);
  *   - edits by foreign code are caught by a content fingerprint that a kernel re-checks on every call, on the
  *     device, without a host wait: every call enqueued before the host has seen the verdict -- the first call after
  *     the edit and as many more as the host runs ahead of the GPU -- computes correct results by kernels that read
@@ -225,8 +226,9 @@ size_t ffi_cache_bytes(void);
  * tfsparse/cc/kernels/register.cpp:29,59-60); this lets a caller budget for what this library adds.  The plan's size
  * depends on the lookup's content: the figure assumes column ids drawn uniformly (as the reference draws them,
  * sparse/custom_layer.py:15,38) and is an estimate; ffi_cache_bytes() reports the actual amount afterwards.  Other entry
- * points keep workspaces of their own beside it: top-k calls 64 KiB of candidates per sample and the scores of up to 32,767
- * sampled labels for each (wide inputs: those labels' rows too), the fused loss and optimizer calls a weight gradient.  Needs a
+ * points keep workspaces of their own beside it: top-k calls 64 KiB of candidates per sample and the scores of up to 17,408
+ * sampled labels for each (wide inputs: those labels' rows too) or, of rows of up to 65,536 labels, all scores (up to 10.5 MB), the
+ * fused loss and optimizer calls a weight gradient.  Needs a
  * current device only for the number of compute units; returns 0 for shapes the entry points reject.
  */
 enum ffi_pass_flags { FFI_PASS_FORWARD = 1, FFI_PASS_BACKWARD = 2 };
