@@ -407,7 +407,7 @@ __device__ __forceinline__ void fwd_lane64_step(unsigned base, float wv, float (
 
 // v[4c+i] <-> v[4(c ^ r)+i] for r in [0,16): its own inverse; four stages of conditional swaps.
 __device__ __forceinline__ void xor_permute_groups64(float (&v)[64], int r) {
-    const bool b8 = r & 8, b4 = r & 4, b2 = r & 2, b1 = r & 1;
+    const unsigned b8 = all_if(r & 8), b4 = all_if(r & 4), b2 = all_if(r & 2), b1 = all_if(r & 1);
 #pragma unroll
     for (int e = 0; e < 64; ++e)
         if (!(e & 32)) cond_swap(b8, v[e], v[e + 32]);

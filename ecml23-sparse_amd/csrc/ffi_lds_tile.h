@@ -132,15 +132,19 @@ __device__ __forceinline__ void load_rows32(const float* __restrict__ m, int ld,
 // arrange that; the forward pass and the weight gradient take rows in the order of the lookup
 // matrix and run at the 8-clock rate.
 
-__device__ __forceinline__ void cond_swap(bool p, float& a, float& b) {
-    const float t = p ? b : a;
-    b = p ? a : b;
-    a = t;
+// Swaps a and b where `mask` has all bits set, and leaves them where it has none.
+__device__ __forceinline__ void cond_swap(unsigned mask, float& a, float& b) {
+    float s, t;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xca" : "=v"(s) : "v"(mask), "v"(b), "v"(a));
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xca" : "=v"(t) : "v"(mask), "v"(a), "v"(b));
+    a = s;
+    b = t;
 }
+__device__ __forceinline__ unsigned all_if(bool p) { return p ? ~0u : 0u; }
 
 // v[4c+i] <-> v[4(c ^ r)+i] for r in [0,8): its own inverse; three stages of conditional swaps.
 __device__ __forceinline__ void xor_permute_groups(float (&v)[32], int r) {
-    const bool b4 = r & 4, b2 = r & 2, b1 = r & 1;
+    const unsigned b4 = all_if(r & 4), b2 = all_if(r & 2), b1 = all_if(r & 1);
 #pragma unroll
     for (int e = 0; e < 32; ++e)
         if (!(e & 16)) cond_swap(b4, v[e], v[e + 16]);
