@@ -28,17 +28,6 @@ namespace {
 // ------------------------------------------------------------------------------------------------
 // `base` is a raw LDS address: (address of the tile + (lane & 7) * 16) + row * 128.  The tile is 128-byte aligned, so the
 // chunk bits can be flipped with XOR after the add: one add and seven XORs per row instead of an add per read.
-typedef float lds_v4f __attribute__((ext_vector_type(4)));
-typedef const lds_v4f __attribute__((address_space(3)))* lds_v4f_ptr;
-template <int C>
-__device__ __forceinline__ void fwd_lane_step(unsigned base, float wv, float (&acc)[32]) {
-    const lds_v4f v = *(lds_v4f_ptr)(size_t)(skew_addr<C>(base));
-    acc[4 * C + 0] = fmaf(wv, v.x, acc[4 * C + 0]);
-    acc[4 * C + 1] = fmaf(wv, v.y, acc[4 * C + 1]);
-    acc[4 * C + 2] = fmaf(wv, v.z, acc[4 * C + 2]);
-    acc[4 * C + 3] = fmaf(wv, v.w, acc[4 * C + 3]);
-}
-
 // One connection of the lane's label: the eight 16-byte reads of row `rb` (chunk order skewed per lane) and their 32
 // multiply-adds, in a pinned order -- two reads in flight; a read's registers are refilled as soon as its four values
 // are used, under the multiply-adds of the other read.  Left to itself the scheduler finds this order or one that
@@ -359,6 +348,11 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
 // the 32 lanes the LDS serves together hit every bank exactly twice whatever rows they read (128-byte rows sit in
 // one half of the banks and the random parities of the rows cost about 1.7x), and W/idx are read once per 64
 // batch rows instead of once per 32.  Plain scores only.
+//
+// Bound by the issue of its instructions (81 to 82 for a connection's 64 multiply-adds: 289 us of them at 256 samples x 512 columns x
+// 501,070 labels x 64) and by the wait for a read wherever none is in flight.  Each read waited for in turn, as the compiler ordered it,
+// that layer took 394 to 435 us; a chunk's 256 reads as one pinned stream, two in flight, issued and used two at a time, 319 to 343
+// (one at a time 328 to 338, four in flight 318 to 333, eight spill).
 // ------------------------------------------------------------------------------------------------
 constexpr int kLane64Batch = 64;
 constexpr int kLane64MaxN = 608;        // 152 KB of LDS
@@ -395,10 +389,8 @@ __device__ __forceinline__ void stage_rows64(float* __restrict__ xs, const float
     }
 }
 
-// base = address of the row + (lane & 15) * 16 (the tile is 256-byte aligned: the chunk bits are flipped with XOR)
 template <int C>
-__device__ __forceinline__ void fwd_lane64_step(unsigned base, float wv, float (&acc)[64]) {
-    const lds_v4f v = *(lds_v4f_ptr)(size_t)(C == 0 ? base : (base ^ (unsigned)(C * 16)));
+__device__ __forceinline__ void fwd_lane64_chunk(const lds_v4f& v, float wv, float (&acc)[64]) {
     acc[4 * C + 0] = fmaf(wv, v.x, acc[4 * C + 0]);
     acc[4 * C + 1] = fmaf(wv, v.y, acc[4 * C + 1]);
     acc[4 * C + 2] = fmaf(wv, v.z, acc[4 * C + 2]);
@@ -407,7 +399,7 @@ __device__ __forceinline__ void fwd_lane64_step(unsigned base, float wv, float (
 
 // v[4c+i] <-> v[4(c ^ r)+i] for r in [0,16): its own inverse; four stages of conditional swaps.
 __device__ __forceinline__ void xor_permute_groups64(float (&v)[64], int r) {
-    const unsigned b8 = all_if(r & 8), b4 = all_if(r & 4), b2 = all_if(r & 2), b1 = all_if(r & 1);
+    const bool b8 = r & 8, b4 = r & 4, b2 = r & 2, b1 = r & 1;
 #pragma unroll
     for (int e = 0; e < 64; ++e)
         if (!(e & 32)) cond_swap(b8, v[e], v[e + 32]);
@@ -451,45 +443,36 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* _
         float acc[64];
 #pragma unroll
         for (int i = 0; i < 64; ++i) acc[i] = 0.f;
-        for (int k0 = 0; k0 < K; k0 += 16) {
-            const bool full = VEC4 && k0 + 16 <= K;
-            unsigned idp[8];
-            float wv[16];
-            if (full) {
+        unsigned idp[8];
+        float wv[16];
+        auto row = [&](auto k) {
+            const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
+            return (id << 8) + skewbase;
+        };
+        auto fmas = [&](auto k, auto c, const lds_v4f& v) { fwd_lane64_chunk<c>(v, wv[k], acc); };
+        int k0 = 0;
+        for (; VEC4 && k0 + 16 <= K; k0 += 16) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int4 v = *reinterpret_cast<const int4*>(irow + k0 + 4 * q);
-                    idp[2 * q + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
-                    idp[2 * q + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
-                    const float4 f = *reinterpret_cast<const float4*>(wrow + k0 + 4 * q);
-                    wv[4 * q] = f.x; wv[4 * q + 1] = f.y; wv[4 * q + 2] = f.z; wv[4 * q + 3] = f.w;
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const unsigned a = (k0 + 2 * q < K) ? (unsigned)irow[k0 + 2 * q] : 0u;
-                    const unsigned b = (k0 + 2 * q + 1 < K) ? (unsigned)irow[k0 + 2 * q + 1] : 0u;
-                    idp[q] = a | (b << 16);
-                }
-#pragma unroll
-                for (int k = 0; k < 16; ++k) wv[k] = (k0 + k < K) ? wrow[k0 + k] : 0.f;
+            for (int q = 0; q < 4; ++q) {
+                const int4 v = *reinterpret_cast<const int4*>(irow + k0 + 4 * q);
+                idp[2 * q + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
+                idp[2 * q + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
+                const float4 f = *reinterpret_cast<const float4*>(wrow + k0 + 4 * q);
+                wv[4 * q] = f.x; wv[4 * q + 1] = f.y; wv[4 * q + 2] = f.z; wv[4 * q + 3] = f.w;
             }
+            stream_rows<16, 16, 2, 2>(row, fmas);
+        }
+        for (; k0 < K; k0 += 16) {
+            // (what is no full chunk: the connections past the row's end load its last one again and are skipped)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) idp[q] = (unsigned)irow[min(k0 + 2 * q, K - 1)] | ((unsigned)irow[min(k0 + 2 * q + 1, K - 1)] << 16);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) wv[k] = wrow[min(k0 + k, K - 1)];
             const int kn = min(16, K - k0);
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                if (full || k < kn) {
-                    const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
-                    const unsigned rb = (id << 8) + skewbase;
-                    fwd_lane64_step<0>(rb, wv[k], acc); fwd_lane64_step<1>(rb, wv[k], acc);
-                    fwd_lane64_step<2>(rb, wv[k], acc); fwd_lane64_step<3>(rb, wv[k], acc);
-                    fwd_lane64_step<4>(rb, wv[k], acc); fwd_lane64_step<5>(rb, wv[k], acc);
-                    fwd_lane64_step<6>(rb, wv[k], acc); fwd_lane64_step<7>(rb, wv[k], acc);
-                    fwd_lane64_step<8>(rb, wv[k], acc); fwd_lane64_step<9>(rb, wv[k], acc);
-                    fwd_lane64_step<10>(rb, wv[k], acc); fwd_lane64_step<11>(rb, wv[k], acc);
-                    fwd_lane64_step<12>(rb, wv[k], acc); fwd_lane64_step<13>(rb, wv[k], acc);
-                    fwd_lane64_step<14>(rb, wv[k], acc); fwd_lane64_step<15>(rb, wv[k], acc);
-                }
-            }
+            static_for<16>([&](auto k) {
+                if (k < kn)
+                    stream_rows<1, 16, 2, 2>([&](auto) { return row(k); }, [&](auto, auto c, const lds_v4f& v) { fmas(k, c, v); });
+            });
         }
         xor_permute_groups64(acc, lane & 15);              // back to natural batch order
         if (bias != nullptr) {                             // added after the sum, as a separate bias_add would
@@ -499,10 +482,15 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* _
         }
         if (valid) {
             const unsigned lane_off = (unsigned)j * 4u;
-            const unsigned stride = (unsigned)L * 4u;
+            unsigned stride = (unsigned)L * 4u;
+            // (the rows' offsets are formed one after the other: all 64 do not fit the scalar registers, and came back from vector lanes)
+            asm volatile("" : "+s"(stride));
+            unsigned off = 0;
 #pragma unroll
-            for (int b = 0; b < 64; ++b)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, lane_off, (unsigned)b * stride, 0);
+            for (int b = 0; b < 64; ++b) {
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, lane_off, off, 0);
+                off += stride;
+            }
         }
     }
 }

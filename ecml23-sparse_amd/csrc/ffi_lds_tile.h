@@ -6,6 +6,9 @@
 
 #include "ffi_internal.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace ffi {
 
 constexpr int kTileBatch = 32;        // batch entries per LDS row: 128 bytes = one pass over the banks
@@ -132,19 +135,15 @@ __device__ __forceinline__ void load_rows32(const float* __restrict__ m, int ld,
 // arrange that; the forward pass and the weight gradient take rows in the order of the lookup
 // matrix and run at the 8-clock rate.
 
-// Swaps a and b where `mask` has all bits set, and leaves them where it has none.
-__device__ __forceinline__ void cond_swap(unsigned mask, float& a, float& b) {
-    float s, t;
-    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xca" : "=v"(s) : "v"(mask), "v"(b), "v"(a));
-    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xca" : "=v"(t) : "v"(mask), "v"(a), "v"(b));
-    a = s;
-    b = t;
+__device__ __forceinline__ void cond_swap(bool p, float& a, float& b) {
+    const float t = p ? b : a;
+    b = p ? a : b;
+    a = t;
 }
-__device__ __forceinline__ unsigned all_if(bool p) { return p ? ~0u : 0u; }
 
 // v[4c+i] <-> v[4(c ^ r)+i] for r in [0,8): its own inverse; three stages of conditional swaps.
 __device__ __forceinline__ void xor_permute_groups(float (&v)[32], int r) {
-    const unsigned b4 = all_if(r & 4), b2 = all_if(r & 2), b1 = all_if(r & 1);
+    const bool b4 = r & 4, b2 = r & 2, b1 = r & 1;
 #pragma unroll
     for (int e = 0; e < 32; ++e)
         if (!(e & 16)) cond_swap(b4, v[e], v[e + 16]);
@@ -205,6 +204,40 @@ __device__ __forceinline__ void row_fmas(const float4 (&v)[8], float wv, float (
         acc[4 * c + 2] = fmaf(wv, v[c].z, acc[4 * c + 2]);
         acc[4 * c + 3] = fmaf(wv, v[c].w, acc[4 * c + 3]);
     }
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
+template <class F, int... Is>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) { (f(std::integral_constant<int, Is>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+
+// The rows of ROWS connections as one stream of 16-byte reads, DEPTH of them in flight from the first to the last: `row(k)`
+// is the base address of connection k's row (as above), of which CHUNKS reads are taken, `use(k, c, v)` what becomes of
+// read c.  The order is pinned: GROUP reads, whose registers were used just before, then the next GROUP uses.
+template <int ROWS, int CHUNKS, int DEPTH, int GROUP, class Row, class Use>
+__device__ __forceinline__ void stream_rows(Row&& row, Use&& use) {
+    static_assert(DEPTH % GROUP == 0 && CHUNKS % GROUP == 0, "whole groups");
+    constexpr int kReads = ROWS * CHUNKS, kFirst = DEPTH < kReads ? DEPTH : kReads;
+    lds_v4f v[kFirst];
+    unsigned at = 0;
+    auto read = [&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        if constexpr (s % CHUNKS == 0) at = row(std::integral_constant<int, s / CHUNKS>{});
+        v[s % kFirst] = *(lds_v4f_ptr)(size_t)(at ^ (unsigned)(s % CHUNKS * 16));
+    };
+    static_for<kFirst>(read);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<kReads / GROUP>([&](auto gc) {
+        constexpr int g = decltype(gc)::value * GROUP;
+        static_for<GROUP>([&](auto i) {
+            constexpr int s = g + decltype(i)::value;
+            use(std::integral_constant<int, s / CHUNKS>{}, std::integral_constant<int, s % CHUNKS>{}, v[s % kFirst]);
+        });
+        if constexpr (GROUP > 1) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (g + kFirst < kReads) static_for<GROUP>([&](auto i) { read(std::integral_constant<int, g + kFirst + decltype(i)::value>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+    });
 }
 
 #endif  // __HIPCC__

@@ -5,8 +5,6 @@
 #include "ffi_lds_tile.h"
 
 #include <algorithm>
-#include <type_traits>
-#include <utility>
 
 namespace ffi {
 namespace {
@@ -304,12 +302,6 @@ __global__ __launch_bounds__(kResThreads) void wgrad_arranged_kernel(const float
 // ------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) float* lds_f32_ptr;
 constexpr int kSliceFloats = kTileBatch * 64;               // one wavefront's slice of out_grad
-
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
-template <class F, int... Is>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) { (f(std::integral_constant<int, Is>{}), ...); }
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
 
 // LDS-direct buffer loads put lane i's value at M0 + immediate + i * size, and an M0 that changes between two of them
 // costs about 30 ns (measured: 32 loads with one M0 each 0.53 us, with an M0 per 16 of them 0.22 us).  So the
