@@ -21,9 +21,12 @@ inline bool tile_path_fits(int rows) { return tile_lds_bytes(rows) <= kTileLdsBu
 #if defined(__HIPCC__)
 
 // Workgroups are dealt round-robin to the 8 XCDs; this renumbers them so that consecutive logical
-// ids share an XCD (and its L2).
+// ids share an XCD (and its L2), however many there are (left in round-robin order where their number is no multiple of eight, the
+// 255 workgroups of 160 or 192 samples fetched every label's ids and weights in each of three batch tiles' XCDs: 192 x 600 x 200,000 x 40,
+// forward by tiles of 64 198 us, 104 so, by tiles of 32 144 and 98).
 __device__ __forceinline__ int xcd_contiguous_block(int block, int nblocks) {
-    return (nblocks & 7) == 0 ? (block & 7) * (nblocks >> 3) + (block >> 3) : block;
+    const int xcd = block & 7, per = nblocks >> 3, more = nblocks & 7;
+    return xcd * per + min(xcd, more) + (block >> 3);
 }
 
 // xs[r][c] = src[r*ld + c0 + c] for c < 32 (zero beyond column `ld`), r < rows.  src rows are read
