@@ -2,10 +2,12 @@
 //   out[b,j] = sum_k w[j,k] * x[b, idx[j,k]]
 // (semantics of tfsparse/cc/kernels/forward.cpp:9-44 in the reference).
 //
-//   fwd_lane32_kernel  narrow inputs (a [N][32] fp32 tile of x fits in LDS): every multiply-add
-//                      takes its x operand from LDS; the LDS delivers 128 bytes per clock per CU,
-//                      which bounds the kernel (4 bytes per multiply-add), so the layout is chosen
-//                      to keep the gathers free of bank conflicts and the instruction count low.
+//   fwd_lane32_kernel    narrow inputs (a [N][32] fp32 tile of x fits in LDS): every multiply-add
+//                        takes its x operand from LDS; the LDS delivers 128 bytes per clock per CU,
+//                        which bounds the kernel (4 bytes per multiply-add), so the layout is chosen
+//                        to keep the gathers free of bank conflicts and the instruction count low.
+//                        Scores go into a loss or a top-k as they are formed.
+//   fwd_stream32_kernel  the same for plain scores; fwd_lane64_kernel by tiles of 64 samples.
 // Batches of at most 16 samples and wide inputs go to the kernels of ffi_sliced.hip.
 #include "ffi_internal.h"
 #include "ffi_lds_tile.h"
@@ -343,6 +345,162 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
 }
 
 // ------------------------------------------------------------------------------------------------
+// A label's row of connections against a tile of W samples in LDS, for plain scores: the reads of a chunk of connections as one pinned
+// stream, two in flight (the kernel above drains them after each connection), ids and weights by quads whatever the fan-in.  LAST says what the
+// row ends in: 0 whole chunks; C > 0 up to C connections behind at least one chunk, loaded as the last C of the row, of which those that are
+// new are walked; -C no whole chunk, at most C connections.  A build for each: under run-time branches the registers of the loads count as
+// live throughout, and 20 to 100 of them spill.
+//
+// Time with the connections drained one after the other and a part-filled chunk loaded one by one -> so, us, at 32 x 768 x 131,072, 128 x 768 x
+// 670,091 and 100 x 1,000 x 300,000: fan-in 8 12.4 -> 11.2, 156 -> 123, 36 -> 33; 13 15.4 -> 13.0, 188 -> 151, 50 -> 42; 31 32 -> 20.5, 376 -> 230,
+// 167 -> 86; 32 20.2 -> 18.4, 191 -> 188, 81 -> 77; 40 25.2 -> 21.8, 259 -> 233, 101 -> 97; 63 44 -> 32, 590 -> 369, 240 -> 153; 64 29 -> 26,
+// 333 -> 330, 147 -> 145.  20 x 700 x 20,000, a tenth of a round of labels: 1.2 to 1.5 times as fast from fan-in 13 on.
+// ------------------------------------------------------------------------------------------------
+template <int C>
+struct RowChunk {
+    unsigned idp[C / 2];                   // two 16-bit ids per register
+    float wv[C];
+    __device__ __forceinline__ unsigned id(int k) const { return (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu); }
+    // Quad q is that from element at(q) of the row: a lane's 16 bytes are a gather of its own, which the memory system serves at any alignment.
+    // The quads of a line one after the other: the lines of 16 wavefronts do not stay in the L1 between them (mixed with the weights', 9.3 million
+    // requests reached the L2 at 128 samples x 670,091 labels x 32, so 6.5).
+    template <class At>
+    __device__ __forceinline__ void load(const int32_t* __restrict__ irow, const float* __restrict__ wrow, At&& at) {
+        int4 v[C / 4];
+        float4 f[C / 4];
+        static_for<C / 4>([&](auto q) { v[q] = *reinterpret_cast<const int4*>(irow + at(q)); __builtin_amdgcn_sched_barrier(0); });
+        static_for<C / 4>([&](auto q) { f[q] = *reinterpret_cast<const float4*>(wrow + at(q)); __builtin_amdgcn_sched_barrier(0); });
+#pragma unroll
+        for (int q = 0; q < C / 4; ++q) {
+            idp[2 * q + 0] = (unsigned)v[q].x | ((unsigned)v[q].y << 16);
+            idp[2 * q + 1] = (unsigned)v[q].z | ((unsigned)v[q].w << 16);
+            wv[4 * q] = f[q].x; wv[4 * q + 1] = f[q].y; wv[4 * q + 2] = f[q].z; wv[4 * q + 3] = f[q].w;
+        }
+    }
+};
+
+// N connections from the FIRST of a chunk on: `skewbase` is the tile's address plus 16 (lane % (W / 4)).
+template <int W, int FIRST, int N, int C>
+__device__ __forceinline__ void walk_chunk(const RowChunk<C>& chunk, unsigned skewbase, float (&acc)[W]) {
+    stream_rows<N, W / 4, 2, W == 64 ? 2 : 1>([&](auto k) { return chunk.id(FIRST + k) * (unsigned)(W * 4) + skewbase; },
+                                              [&](auto k, auto c, const lds_v4f& v) {
+                                                  const float wv = chunk.wv[FIRST + k];
+                                                  acc[4 * c + 0] = fmaf(wv, v.x, acc[4 * c + 0]);
+                                                  acc[4 * c + 1] = fmaf(wv, v.y, acc[4 * c + 1]);
+                                                  acc[4 * c + 2] = fmaf(wv, v.z, acc[4 * c + 2]);
+                                                  acc[4 * c + 3] = fmaf(wv, v.w, acc[4 * c + 3]);
+                                              });
+}
+
+template <int LAST>
+__device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const float* __restrict__ wrow, int K, unsigned skewbase, float (&acc)[32]) {
+    if constexpr (LAST < 0) {
+        // (whole quads, those behind the last one read it again; then up to three connections one by one)
+        RowChunk<-LAST> chunk;
+        RowChunk<4> end;
+        if (K >= 4) chunk.load(irow, wrow, [&](int q) { return min(4 * q, K - 4); });
+        if (K & 3) {
+            unsigned id[3];
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                const int at = min((K & ~3) + e, K - 1);
+                id[e] = (unsigned)irow[at];
+                end.wv[e] = wrow[at];
+            }
+            end.idp[0] = id[0] | (id[1] << 16);
+            end.idp[1] = id[2];
+        }
+        static_for<-LAST / 4>([&](auto q) {
+            if (4 * q + 4 <= K) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
+        });
+        static_for<3>([&](auto e) {
+            if (e < (K & 3)) walk_chunk<32, e, 1>(end, skewbase, acc);
+        });
+    } else {
+        int k0 = 0;
+        for (; k0 + 32 <= K; k0 += 32) {
+            RowChunk<32> chunk;
+            chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
+            walk_chunk<32, 0, 32>(chunk, skewbase, acc);
+        }
+        if constexpr (LAST > 0) {
+            RowChunk<LAST> chunk;
+            chunk.load(irow, wrow, [&](int q) { return K - LAST + 4 * q; });
+            const int seen = LAST - (K - k0);
+            static_for<LAST / 4>([&](auto q) {
+                if (4 * q >= seen) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
+                else
+                    static_for<3>([&](auto i) {
+                        constexpr int k = 4 * q + 1 + i;
+                        if (k >= seen) walk_chunk<32, k, 1>(chunk, skewbase, acc);
+                    });
+            });
+        }
+    }
+}
+
+// What a row of K connections ends in, for walk_row: whole quads of the few sizes that are worth a build.
+template <class Launch>
+int for_row_end(int K, Launch&& launch) {
+    const int last = K % 32;
+    if (K < 32) {
+        if (K <= 4) return launch(std::integral_constant<int, -4>{});
+        if (K <= 8) return launch(std::integral_constant<int, -8>{});
+        if (K <= 16) return launch(std::integral_constant<int, -16>{});
+        return launch(std::integral_constant<int, -32>{});
+    }
+    if (last == 0) return launch(std::integral_constant<int, 0>{});
+    if (last <= 4) return launch(std::integral_constant<int, 4>{});
+    if (last <= 8) return launch(std::integral_constant<int, 8>{});
+    if (last <= 16) return launch(std::integral_constant<int, 16>{});
+    return launch(std::integral_constant<int, 32>{});
+}
+
+// The kernel above for plain scores.
+template <int LAST>
+__global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
+                                                                    const float* __restrict__ w, const float* __restrict__ bias,
+                                                                    float* __restrict__ out, int B, int N, int L, int K, int nbt, int labels_per_stream) {
+    extern __shared__ __align__(128) float xs[];
+    const int u = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int bt = u % nbt, stream = u / nbt;
+    const int b0 = bt * kTileBatch;
+    const int lane = threadIdx.x & 63;
+    const int l_begin = stream * labels_per_stream, l_end = min(l_begin + labels_per_stream, L);
+    stage_rows32<kTileThreads, 8>(xs, xT, N, B, b0);
+    __syncthreads();
+    const unsigned skewbase = (unsigned)(size_t)(__attribute__((address_space(3))) float*)xs + (unsigned)(lane & 7) * 16u;
+    // rows of out for this batch tile, reached through a scalar row offset plus the lane's label; rows past the batch
+    // lie beyond the resource's size and their stores are dropped
+    const buffer_rsrc orsrc = make_rsrc(out + (size_t)b0 * (size_t)L, (size_t)min(kTileBatch, B - b0) * (size_t)L * sizeof(float));
+    for (int base = l_begin; base + (int)(threadIdx.x & ~63u) < l_end; base += kTileThreads) {
+        const int j = base + (int)threadIdx.x;
+        const bool valid = j < l_end;
+        const int32_t* irow = idx + (size_t)min(j, l_end - 1) * K;
+        const float* wrow = w + (size_t)min(j, l_end - 1) * K;
+        float acc[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+        walk_row<LAST>(irow, wrow, K, skewbase, acc);
+        xor_permute_groups(acc, lane & 7);                 // back to natural batch order
+        if (bias != nullptr) {                             // added after the sum, as a separate bias_add would
+            const float bj = bias[min(j, l_end - 1)];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) acc[i] += bj;
+        }
+        if (valid) {
+            unsigned stride = (unsigned)L * 4u, off = 0;
+            asm volatile("" : "+s"(stride));               // (see fwd_lane64_kernel)
+#pragma unroll
+            for (int b = 0; b < 32; ++b) {
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, (unsigned)j * 4u, off, 0);
+                off += stride;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // The same kernel over batch tiles of 64 for inputs narrow enough that an [N][64] fp32 tile of x fits in LDS
 // (N <= kLane64MaxN): a row is 256 bytes and covers all 64 banks, so with the chunk order skewed by (lane & 15)
 // the 32 lanes the LDS serves together hit every bank exactly twice whatever rows they read (128-byte rows sit in
@@ -389,14 +547,6 @@ __device__ __forceinline__ void stage_rows64(float* __restrict__ xs, const float
     }
 }
 
-template <int C>
-__device__ __forceinline__ void fwd_lane64_chunk(const lds_v4f& v, float wv, float (&acc)[64]) {
-    acc[4 * C + 0] = fmaf(wv, v.x, acc[4 * C + 0]);
-    acc[4 * C + 1] = fmaf(wv, v.y, acc[4 * C + 1]);
-    acc[4 * C + 2] = fmaf(wv, v.z, acc[4 * C + 2]);
-    acc[4 * C + 3] = fmaf(wv, v.w, acc[4 * C + 3]);
-}
-
 // v[4c+i] <-> v[4(c ^ r)+i] for r in [0,16): its own inverse; four stages of conditional swaps.
 __device__ __forceinline__ void xor_permute_groups64(float (&v)[64], int r) {
     const bool b8 = r & 8, b4 = r & 4, b2 = r & 2, b1 = r & 1;
@@ -414,7 +564,6 @@ __device__ __forceinline__ void xor_permute_groups64(float (&v)[64], int r) {
         if (!(e & 4)) cond_swap(b1, v[e], v[e + 4]);
 }
 
-template <bool VEC4>
 __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
                                                                   const float* __restrict__ w, const float* __restrict__ bias,
                                                                   float* __restrict__ out, int B, int N, int L, int K, int nbt,
@@ -443,35 +592,22 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* _
         float acc[64];
 #pragma unroll
         for (int i = 0; i < 64; ++i) acc[i] = 0.f;
-        unsigned idp[8];
-        float wv[16];
-        auto row = [&](auto k) {
-            const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
-            return (id << 8) + skewbase;
-        };
-        auto fmas = [&](auto k, auto c, const lds_v4f& v) { fwd_lane64_chunk<c>(v, wv[k], acc); };
         int k0 = 0;
-        for (; VEC4 && k0 + 16 <= K; k0 += 16) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int4 v = *reinterpret_cast<const int4*>(irow + k0 + 4 * q);
-                idp[2 * q + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
-                idp[2 * q + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
-                const float4 f = *reinterpret_cast<const float4*>(wrow + k0 + 4 * q);
-                wv[4 * q] = f.x; wv[4 * q + 1] = f.y; wv[4 * q + 2] = f.z; wv[4 * q + 3] = f.w;
-            }
-            stream_rows<16, 16, 2, 2>(row, fmas);
+        for (; k0 + 16 <= K; k0 += 16) {
+            RowChunk<16> chunk;
+            chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
+            walk_chunk<64, 0, 16>(chunk, skewbase, acc);
         }
-        for (; k0 < K; k0 += 16) {
-            // (what is no full chunk: the connections past the row's end load its last one again and are skipped)
+        if (k0 < K) {
+            // (what is no whole chunk: the connections past the row's end load its last one again and are skipped)
+            RowChunk<16> chunk;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) idp[q] = (unsigned)irow[min(k0 + 2 * q, K - 1)] | ((unsigned)irow[min(k0 + 2 * q + 1, K - 1)] << 16);
+            for (int q = 0; q < 8; ++q) chunk.idp[q] = (unsigned)irow[min(k0 + 2 * q, K - 1)] | ((unsigned)irow[min(k0 + 2 * q + 1, K - 1)] << 16);
 #pragma unroll
-            for (int k = 0; k < 16; ++k) wv[k] = wrow[min(k0 + k, K - 1)];
-            const int kn = min(16, K - k0);
+            for (int k = 0; k < 16; ++k) chunk.wv[k] = wrow[min(k0 + k, K - 1)];
+            const int kn = K - k0;
             static_for<16>([&](auto k) {
-                if (k < kn)
-                    stream_rows<1, 16, 2, 2>([&](auto) { return row(k); }, [&](auto, auto c, const lds_v4f& v) { fmas(k, c, v); });
+                if (k < kn) walk_chunk<64, k, 1>(chunk, skewbase, acc);
             });
         }
         xor_permute_groups64(acc, lane & 15);              // back to natural batch order
@@ -495,7 +631,6 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* _
     }
 }
 
-template <bool VEC4>
 int launch_lane64(const float* xT, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, hipStream_t s) {
     const int cus = device_cu_count();
     const int nbt = (d.B + kLane64Batch - 1) / kLane64Batch;
@@ -503,21 +638,25 @@ int launch_lane64(const float* xT, const int32_t* idx, const float* w, const flo
     const int per_stream = (d.L + streams - 1) / streams;
     streams = (d.L + per_stream - 1) / per_stream;
     const size_t lds = (size_t)d.N * kLane64Batch * sizeof(float);
-    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lane64_kernel<VEC4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((fwd_lane64_kernel<VEC4>), dim3(streams * nbt), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N,
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lane64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(fwd_lane64_kernel, dim3(streams * nbt), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N,
                        d.L, d.K, nbt, per_stream);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
 
 // (64 rows of out of a batch tile are reached through 32-bit byte offsets)
-// Where the tile of 64 samples fits, and where it pays.  Measured against the 32-sample kernel at 501,070 labels, 256-608
-// columns: +2...+10 % from 192 samples up at every fan-in, -3...-14 % at 64-160 samples with a fan-in up to 40; +5...+12 %
-// from 128 samples up with a fan-in of 64 or more; +20...+37 % at fan-in 48 at every batch size (a last chunk of 16
-// connections is a full chunk here, and loaded one by one there).
+// Where the tile of 64 samples fits, and where it pays: it walks twice the multiply-adds per address and reads ids and weights half as often,
+// and leaves half as many workgroups.  Time of the tiles of 32 over its own, 128 and 600 columns x 200,000 labels and 400 x 600,000: whole chunks of 16
+// from 128 samples and fan-in 32 on 1.07...1.42, from 192 samples 1.10...1.28 at fan-in 16; fan-ins 33 and 100 1.07...1.36 from 192
+// samples on, fan-in 40 (eight connections behind the last chunk, loaded one by one) 0.75...1.0; 160 samples, the last tile half empty, 0.89...1.09 at
+// fan-in 32 and 1.03...1.17 from 48 on; fan-ins up to 13 0.6...1.0.  20,000 labels, 80 to 470 a workgroup: 0.4...1.0 throughout.
 bool lane64_fits(const Dims& d) {
     if (d.N > kLane64MaxN || d.B <= kTileBatch || d.L >= (1 << 24) || g_options.fwd_lane64 < 0) return false;
-    return d.B >= 192 || (d.K >= 64 && d.B >= 128) || (d.K > 32 && d.K % 32 != 0 && d.K % 16 == 0);
+    const int tiles = (d.B + kLane64Batch - 1) / kLane64Batch, rest = d.B % kLane64Batch, behind = d.K % 16;
+    if (behind > 4 || (behind > 0 && d.K < 32) || (long long)d.L * tiles < 768ll * device_cu_count()) return false;
+    if (rest != 0 && rest <= kTileBatch) return d.K >= 48 && d.B >= 2 * kLane64Batch;
+    return (d.K >= 16 && d.B >= 192) || (d.K >= 32 && d.B >= 2 * kLane64Batch) || (d.K >= 48 && behind == 0);
 }
 
 }  // namespace
@@ -560,6 +699,15 @@ int launch_lane32(const float* xT, const int32_t* idx, const float* w, const flo
     return FFI_OK;
 }
 
+template <int LAST>
+int launch_stream32(const float* xT, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, int nbt, int per_stream, int blocks,
+                    size_t lds, hipStream_t s) {
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_stream32_kernel<LAST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(fwd_stream32_kernel<LAST>, dim3(blocks), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N, d.L, d.K, nbt, per_stream);
+    FFI_HIP_TRY(hipGetLastError());
+    return FFI_OK;
+}
+
 template <int EPI>
 int launch_lane32_any(bool vec4, bool topk, const float* xT, const int32_t* idx, const float* w, const float* bias, float* out,
                       const Dims& d, int nbt, int per_stream, int blocks, size_t lds, const FwdLoss& fl, const FwdTopk& ft,
@@ -573,9 +721,9 @@ int launch_lane32_any(bool vec4, bool topk, const float* xT, const int32_t* idx,
     if constexpr (EPI != kEpiLossGradSkewed) {              // (that epilogue has no top-k form)
         if (topk) return vec == 2 ? FFI_LANE32(2, EPI, true) : vec == 1 ? FFI_LANE32(1, EPI, true) : FFI_LANE32(0, EPI, true);
     }
-    if (EPI == kEpiNone) return FFI_OK;                     // nothing to compute
-    constexpr int E = EPI == kEpiNone ? kEpiScores : EPI;
-    return vec == 2 ? FFI_LANE32(2, E, false) : vec == 1 ? FFI_LANE32(1, E, false) : FFI_LANE32(0, E, false);
+    if constexpr (EPI != kEpiNone && EPI != kEpiScores)     // (plain scores: fwd_stream32_kernel)
+        return vec == 2 ? FFI_LANE32(2, EPI, false) : vec == 1 ? FFI_LANE32(1, EPI, false) : FFI_LANE32(0, EPI, false);
+    else return FFI_ERR_BAD_ARGUMENT;
 #undef FFI_LANE32
 }
 
@@ -594,11 +742,7 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
     }
     const size_t lds = tile_lds_bytes(d.N);
     const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)w | (uintptr_t)idx) % 16 == 0);
-    if (epi == kEpiScores && tk == nullptr && lane64_fits(d)) {
-        // (16-byte loads for the full chunks of 16 also where rows are only 4-byte aligned: see launch_lane32_any)
-        const bool quads = vec4 || ((((uintptr_t)w | (uintptr_t)idx) % 4 == 0) && d.K >= 16);
-        return quads ? launch_lane64<true>(xT, idx, w, bias, out, d, s) : launch_lane64<false>(xT, idx, w, bias, out, d, s);
-    }
+    if (epi == kEpiScores && tk == nullptr && lane64_fits(d)) return launch_lane64(xT, idx, w, bias, out, d, s);
     const int cus = device_cu_count();
     const int nbt = (d.B + kTileBatch - 1) / kTileBatch;
     int streams = std::max(1, cus / nbt);
@@ -624,6 +768,8 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         ft = FwdTopk{tc.tau, tc.tie, tc.count, tc.val, tc.idx, kTopkCap};
         lds_topk = lds + (size_t)kTileBatch * kTopkPark * sizeof(int2);
     }
+    if (epi == kEpiScores && !topk)
+        return for_row_end(d.K, [&](auto last) { return launch_stream32<last>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, s); });
     int npartial = 0;
     double* corr = nullptr;
     if (epi == kEpiLossGrad || epi == kEpiLossGradAndScores) {

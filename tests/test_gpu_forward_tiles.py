@@ -10,10 +10,10 @@ from conftest import load_package, reference_law_inputs, rel_err
 pytestmark = pytest.mark.gpu
 
 
-# fan-ins around the chunks of 16 and of 32; batches that fill, start and end within a tile; the most columns that fit; labels that leave
+# fan-ins around the chunks of 16 and of 32 and the quads behind them; batches that fill, start and end within a tile; the most columns that fit; labels that leave
 # a wavefront, a workgroup and a round part empty
-@pytest.mark.parametrize("fan_in", [1, 3, 4, 15, 16, 17, 24, 31, 32, 33, 47, 48, 64, 65, 127])
-@pytest.mark.parametrize("batch,features,labels", [(192, 608, 1500), (255, 77, 70_001), (321, 300, 65)])
+@pytest.mark.parametrize("fan_in", [1, 3, 4, 5, 8, 9, 15, 16, 17, 24, 31, 32, 33, 36, 37, 41, 47, 48, 49, 63, 64, 65, 127])
+@pytest.mark.parametrize("batch,features,labels", [(192, 608, 1500), (192, 608, 66_001), (255, 77, 70_001), (321, 300, 65)])
 def test_tiles_of_64_samples_and_of_32_agree(fan_in, batch, features, labels):
     ffi = load_package()
     lib = ffi._lib.lib()
