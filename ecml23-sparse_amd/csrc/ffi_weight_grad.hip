@@ -561,6 +561,20 @@ __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* 
                         const lds_v4f v = *(lds_v4f_ptr)(size_t)(srow + (((unsigned)t ^ sw) << 4));
                         if (mine && k0 + 4 * t < K) *reinterpret_cast<float4*>(grow + 4 * t) = make_float4(v.x, v.y, v.z, v.w);
                     }
+                } else if (QUADS && K > 6) {
+                    // (rows off 16 bytes: instruction t stores the rows of lanes 2 t and 2 t + 1, a float per lane.  A row per lane, float by float,
+                    // touches 64 rows with each store: the kernel at 32 samples x 768 x 131,072 x 31 33 us, 18 so, x 47 45 and 24; x 5 all passes 44 and 45)
+                    const long long it0 = __builtin_amdgcn_readfirstlane((int)(it - lane));
+                    const int j0 = NCH == 1 ? (int)(it0 % L) : (int)it0;
+                    const unsigned half = (unsigned)lane >> 5, q = (unsigned)lane & 31u;
+                    const bool there = (int)q < K - k0;
+                    float* to = gw + (size_t)(j0 + (int)half) * K + k0 + q;
+#pragma unroll
+                    for (int t = 0; t < 32; ++t) {
+                        const unsigned r = (unsigned)(2 * t) + half;
+                        const float v = *(lds_f32_ptr)(size_t)((unsigned)(size_t)gslice + r * 128u + ((q ^ ((unsigned)(t & 7) << 2)) << 2));
+                        if (there && it0 + (long long)r < i_end) to[(size_t)(2 * t) * K] = v;
+                    }
                 } else {
                     for (int k = 0; k < kWgChunk; ++k) {
                         const float v = *(lds_f32_ptr)(size_t)(srow + (((unsigned)k ^ (sw << 2)) << 2));

@@ -37,3 +37,30 @@ def test_gradients_of_few_labels(shape, transposed):
             assert not need_x or rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5
     finally:
         assert lib.ffi_set_option(b"small_path", 0) == 0
+
+
+# every fan-in around the quads and chunks that rows are loaded, walked and stored by, with a label count that leaves wavefronts and
+# workgroups part empty: over a plan and from the lookup itself, results at sixteen bytes and off them
+@pytest.mark.parametrize("fan_in", [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 23, 24, 25, 28, 29, 31, 32, 33, 36, 47, 63, 64, 65, 95, 97, 127])
+@pytest.mark.parametrize("batch,features,labels", [(33, 300, 1301), (64, 768, 517)])
+def test_gradients_of_any_fan_in(batch, features, labels, fan_in):
+    ffi = load_package()
+    lib = ffi._lib.lib()
+    x, lookup, w, g = reference_law_inputs(batch, features, labels, fan_in, seed=fan_in + labels)
+    _, ref_gw = oracle.backward(x, lookup, w, g)
+    ref_gb = g.astype(np.float64).sum(0)
+    dx, dl, dw, dg = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, lookup, w, g))
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        for need_x in (True, False):
+            storage = torch.full((labels * fan_in + 2,), float("nan"), device="cuda")
+            for gw in (storage[:-2], storage[1:-1]):
+                storage.fill_(float("nan"))
+                gx, gb = torch.empty_like(dx), torch.empty((labels,), device="cuda")
+                ffi._lib.check(lib.ffi_backward_bias_f32(dx.data_ptr(), dl.data_ptr(), dw.data_ptr(), dg.data_ptr(), gx.data_ptr() if need_x else None,
+                                                         gw.data_ptr(), gb.data_ptr(), batch, features, labels, fan_in, 0, stream))
+                assert rel_err(gw.cpu().numpy().reshape(labels, fan_in), ref_gw) <= 1e-5 and rel_err(gb.cpu().numpy(), ref_gb) <= 1e-5
+                assert int(torch.isnan(storage).sum()) == 2        # (nothing beside the gradient is written)
+    finally:
+        assert lib.ffi_set_option(b"small_path", 0) == 0
