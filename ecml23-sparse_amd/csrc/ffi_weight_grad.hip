@@ -57,7 +57,13 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
     }
 }
 
-template <bool VEC4>
+// WALK: connections a unit walks; ids and sums move by quads at any alignment.  WHOLE, a fan-in of 32 or more: 32, a label's last unit taking its last
+// (those that it shares with the unit before are formed twice, to the same bits).  Else the fan-in rounded up to eight, the quads behind its last one
+// being that quad again; 4: fan-ins below four, one by one.
+// Units of 32 whatever the fan-in, the ids and sums of part-filled ones one by one -> so, both launches, us, at 32 samples x 768 x 131,072 and 100 x 500 x
+// 200,000: fan-in 8 22.5 -> 14.8, 80 -> 38; 16 31.7 -> 18.5, 104 -> 53; 31 46 -> 28, 139 -> 85; 32 26.6 -> 25.9, 84 -> 82; 33 51 -> 34, 173 -> 120;
+// 48 48 -> 37, 174 -> 127; 63 81 -> 38, 236 -> 130.
+template <int WALK, bool WHOLE>
 __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float* __restrict__ xT,
                                                                      const int32_t* __restrict__ idx,
                                                                      const float* __restrict__ g,
@@ -74,12 +80,16 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
     const int bt0 = blockIdx.y * parts.tiles, nbt = min(bt0 + parts.tiles, (B + kTileBatch - 1) / kTileBatch);
     gw += blockIdx.y * parts.stride;
     if (bias_grad != nullptr) bias_grad += blockIdx.y * parts.stride;
+    // a unit's label and the place of its first connection; quad q of a row that is shorter than a unit
+    auto label_of = [&](long long u) { return (int)(u / nchunks); };
+    auto first_of = [&](long long u, int j) { return WHOLE ? min((int)(u - (long long)j * nchunks) * kWgChunk, K - kWgChunk) : 0; };
+    auto quad_at = [&](int q) { return WHOLE ? 4 * q : min(4 * q, K - 4); };
 
-    float res[kResUnits][kWgChunk];
+    float res[kResUnits][WALK];
 #pragma unroll
     for (int q = 0; q < kResUnits; ++q)
 #pragma unroll
-        for (int k = 0; k < kWgChunk; ++k) res[q][k] = 0.f;
+        for (int k = 0; k < WALK; ++k) res[q][k] = 0.f;
     float gsum[kResUnits];                                 // column sums of out_grad (the bias gradient)
 #pragma unroll
     for (int q = 0; q < kResUnits; ++q) gsum[q] = 0.f;
@@ -97,8 +107,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
             const long long ubase = u_begin + (long long)q * kResThreads;
             if (ubase + (long long)(threadIdx.x & ~63u) < u_end) {          // the wavefront has units in this round
                 const long long u = min(ubase + (long long)threadIdx.x, u_end - 1);   // clamped: loads stay in bounds
-                const int j = (int)(u / nchunks);
-                const int k0 = (int)(u - (long long)j * nchunks) * kWgChunk;
+                const int j = label_of(u), k0 = first_of(u, j);
                 const int32_t* irow = idx + (size_t)j * K + k0;
                 // out_grad of this label for the tile's 32 batch rows: coalesced across lanes
                 float gb[32];
@@ -110,25 +119,24 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
                     gsum[q] = t;
                 }
                 // column ids of the unit, two 16-bit ids per register (ids < 2^16 on this path)
-                unsigned idp[kWgChunk / 2];
-                if (VEC4 && k0 + kWgChunk <= K) {
+                unsigned idp[WALK / 2];
+                if (WALK == 4) {
 #pragma unroll
-                    for (int t = 0; t < kWgChunk / 4; ++t) {
-                        const int4 v = *reinterpret_cast<const int4*>(irow + 4 * t);
+                    for (int t = 0; t < WALK / 2; ++t) idp[t] = (unsigned)irow[min(2 * t, K - 1)] | ((unsigned)irow[min(2 * t + 1, K - 1)] << 16);
+                } else if (K >= (WHOLE ? kWgChunk : 4)) {         // (always: a block of their own, or their 32 registers are wanted beside out_grad's)
+#pragma unroll
+                    for (int t = 0; t < WALK / 4; ++t) {
+                        const int4 v = *reinterpret_cast<const int4*>(irow + quad_at(t));
                         idp[2 * t + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
                         idp[2 * t + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
                     }
                 } else {
 #pragma unroll
-                    for (int t = 0; t < kWgChunk / 2; ++t) {
-                        const unsigned a = (k0 + 2 * t < K) ? (unsigned)irow[2 * t] : 0u;
-                        const unsigned b = (k0 + 2 * t + 1 < K) ? (unsigned)irow[2 * t + 1] : 0u;
-                        idp[t] = a | (b << 16);
-                    }
+                    for (int t = 0; t < WALK / 2; ++t) idp[t] = 0u;
                 }
                 xor_permute_groups(gb, lane & 7);          // match the skewed chunk order of the gathers
 #pragma unroll
-                for (int k = 0; k < kWgChunk; ++k) {
+                for (int k = 0; k < WALK; ++k) {
                     const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
                     float4 xv[8];
                     read_row((id << 7) + skew, xv);
@@ -143,18 +151,17 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
     for (int q = 0; q < kResUnits; ++q) {
         const long long u = u_begin + (long long)q * kResThreads + threadIdx.x;
         if (u < u_end) {
-            const int j = (int)(u / nchunks);
-            const int k0 = (int)(u - (long long)j * nchunks) * kWgChunk;
+            const int j = label_of(u), k0 = first_of(u, j);
             float* grow = gw + (size_t)j * K + k0;
-            if (bias_grad != nullptr && k0 == 0) bias_grad[j] = gsum[q];
-            if (VEC4 && k0 + kWgChunk <= K) {
+            if (bias_grad != nullptr && u - (long long)j * nchunks == 0) bias_grad[j] = gsum[q];
+            if (WALK == 4) {
 #pragma unroll
-                for (int t = 0; t < kWgChunk / 4; ++t)
-                    *reinterpret_cast<float4*>(grow + 4 * t) = make_float4(res[q][4 * t], res[q][4 * t + 1], res[q][4 * t + 2], res[q][4 * t + 3]);
+                for (int k = 0; k < WALK; ++k)
+                    if (k < K) grow[k] = res[q][k];
             } else {
 #pragma unroll
-                for (int k = 0; k < kWgChunk; ++k)
-                    if (k0 + k < K) grow[k] = res[q][k];
+                for (int t = 0; t < WALK / 4; ++t)
+                    *reinterpret_cast<f32x4_unaligned*>(grow + quad_at(t)) = f32x4_unaligned{res[q][4 * t], res[q][4 * t + 1], res[q][4 * t + 2], res[q][4 * t + 3]};
             }
         }
     }
@@ -791,14 +798,10 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
         const unsigned blocks = (unsigned)(n1 + n2);
         const int upb = ipb, upb2 = ipb2;
         const size_t lds = tile_lds_bytes(d.N);
-        const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)gw | (uintptr_t)idx) % 16 == 0);
-        if (vec4) {
-            FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<true>, dim3(blocks, (unsigned)rows), dim3(kResThreads), lds, s, xT, idx, g, to_w, to_b, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, parts);
-        } else {
-            FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_resident_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(wgrad_resident_kernel<false>, dim3(blocks, (unsigned)rows), dim3(kResThreads), lds, s, xT, idx, g, to_w, to_b, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, parts);
-        }
+        const auto kernel = d.K < 4 ? wgrad_resident_kernel<4, false> : d.K <= 8 ? wgrad_resident_kernel<8, false> : d.K <= 16 ? wgrad_resident_kernel<16, false> :
+                            d.K <= 24 ? wgrad_resident_kernel<24, false> : d.K < kWgChunk ? wgrad_resident_kernel<32, false> : wgrad_resident_kernel<32, true>;
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)rows), dim3(kResThreads), lds, s, xT, idx, g, to_w, to_b, d.B, d.N, d.L, d.K, nchunks, n1, upb, upb2, parts);
         return sum_parts();
     }
     return launch_weight_grad_wide(x, idx, g, gw, bias_grad, d, s);
