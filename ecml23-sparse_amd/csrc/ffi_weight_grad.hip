@@ -673,9 +673,12 @@ ArrangedForm arranged_form(const Dims& d) {
     f.last_walk = (d.K - (nchunks - 1) * kWgChunk + 7) / 8 * 8;
     // (two chunks per label: one label per thread, 64 sums, measured 2-4 % under two labels per thread, whose 128 sums
     // leave the streaming kernel 92 bytes of spills per lane)
-    if (nchunks == 2 || nchunks == 4) {
+    // (three chunks per label, 96 sums, with the slices and where labels alone keep most wavefronts busy or the last chunk is mostly empty: all passes by
+    // units and by labels 32 x 768 x 131,072 x 65 133 and 92 us, x 80 105 and 94, x 95 155 and 110, 128 x 500 x 200,000 x 65 355 and 291; 256 x 300 x
+    // 60,000 x 96 255 and 268, x 72 230 and 217)
+    if (nchunks == 2 || nchunks == 4 || (nchunks == 3 && f.stream && (d.L >= 320ll * cus || f.last_walk <= 16))) {
         f.nch = nchunks;
-        f.units = nchunks == 2 && f.stream && g_options.wgrad_units != 4 ? 2 : 4;
+        f.units = nchunks == 3 ? 3 : nchunks == 2 && f.stream && g_options.wgrad_units != 4 ? 2 : 4;
     } else {
         // the streaming kernel: three units per thread wherever measured (4,000 to 3,000,000 labels, batch 32-512, 64-768
         // columns, fan-in 8-32 and 96: 3-15 % under four units); the kernel without slices: by the model above
@@ -787,6 +790,7 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
             } while (0)
             if (form.nch == 2 && form.units == 4) FFI_LAUNCH_ARRANGED(2, 4);
             else if (form.nch == 2) FFI_LAUNCH_ARRANGED(2, 2);
+            else if (form.nch == 3) FFI_LAUNCH_ARRANGED(3, 3);
             else if (form.nch == 4) FFI_LAUNCH_ARRANGED(4, 4);
             else if (form.units == 3) FFI_LAUNCH_ARRANGED(1, 3);
             else FFI_LAUNCH_ARRANGED(1, 4);

@@ -41,7 +41,7 @@ def test_gradients_of_few_labels(shape, transposed):
 
 # every fan-in around the quads and chunks that rows are loaded, walked and stored by, with a label count that leaves wavefronts and
 # workgroups part empty: over a plan and from the lookup itself, results at sixteen bytes and off them
-@pytest.mark.parametrize("fan_in", [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 23, 24, 25, 28, 29, 31, 32, 33, 36, 47, 63, 64, 65, 95, 97, 127])
+@pytest.mark.parametrize("fan_in", [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 23, 24, 25, 28, 29, 31, 32, 33, 36, 47, 63, 64, 65, 73, 95, 97, 127])
 @pytest.mark.parametrize("batch,features,labels", [(33, 300, 1301), (64, 768, 517)])
 def test_gradients_of_any_fan_in(batch, features, labels, fan_in):
     ffi = load_package()
@@ -64,3 +64,8 @@ def test_gradients_of_any_fan_in(batch, features, labels, fan_in):
                 assert int(torch.isnan(storage).sum()) == 2        # (nothing beside the gradient is written)
     finally:
         assert lib.ffi_set_option(b"small_path", 0) == 0
+
+
+@pytest.mark.parametrize("fan_in", [72, 81, 89, 95, 96])
+def test_gradients_of_three_chunks_and_many_labels(fan_in):
+    test_gradients_of_any_fan_in(33, 70, 82_001, fan_in)
