@@ -404,12 +404,22 @@ template <int CTRL> __device__ __forceinline__ void exchange_bit(bool bit, float
     b = bit ? b : other;
 }
 
-template <int GL, bool BF16, bool QUADS, bool COLUMNS = false>
+typedef unsigned u32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned u32x2_unaligned __attribute__((ext_vector_type(2), aligned(2)));
+
+// How ids and weights are read: one by one; by quads, of rows of whole quads on 16-byte boundaries; by quads of any rows, the quad that a row
+// ends in being its last four connections.  Of the latter the odd fan-ins take their time, 300,000 labels of 8 samples x 768 by ones and by quads:
+// fan-in 7 16.4 and 11.0 us, 23 25 and 20.5, 33 38 and 32, but 47 52 and 61 (16 samples 34 and 32, bf16 64 and 58), 65 73 and 90 (44 and 42, 78 and 72).
+enum LdsRows { kOneByOne = 0, kQuads = 1, kAnyQuads = 2 };
+template <int GL> constexpr bool any_quads_pay(int K) { return K >= 4 && (GL >= 4 || K <= 33); }
+
+template <int GL, bool BF16, int ROWS, bool COLUMNS = false>
 __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restrict__ features, const int32_t* __restrict__ idx,
                                                              const void* __restrict__ w, const float* __restrict__ bias,
                                                              float* __restrict__ out, int B, int N, int L, int K, int tp, int row_step,
                                                              int slices, int streams, int chunk, const TopkSink sink) {
     using S = LdsShape<GL, BF16>;
+    constexpr bool QUADS = ROWS != kOneByOne;
     constexpr int kPer = LaneAcc<BF16>::kSamples, kSl = GL * kPer, kWaves = kLdThreads / 64;
     constexpr unsigned kRow = GL * 16u;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -504,13 +514,27 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
             int l, k;
             if (QUADS) {
                 place((unsigned)(64 * v + lane), chunk / 4, l, k);
-                const unsigned at = (unsigned)min(j + min(l, S::kGroups - 1), L - 1) * row_pitch + (unsigned)(k0 + (4 * k < kc ? 4 * k : 0));
-                ids[v] = *reinterpret_cast<const uint4*>(idx + at);
-                if (BF16) {
-                    const uint2 h = *reinterpret_cast<const uint2*>(w16 + at);
-                    ws[v].x = h.x; ws[v].y = h.y;
+                const int row = min(j + min(l, S::kGroups - 1), L - 1), off = 4 * k < kc ? 4 * k : 0;
+                if constexpr (ROWS == kAnyQuads) {
+                    const unsigned at = (unsigned)row * row_pitch + (unsigned)(k0 + min(off, kc - 4));
+                    const u32x4_unaligned id = *reinterpret_cast<const u32x4_unaligned*>(idx + at);
+                    ids[v] = make_uint4(id.x, id.y, id.z, id.w);
+                    if (BF16) {
+                        const u32x2_unaligned h = *reinterpret_cast<const u32x2_unaligned*>(w16 + at);
+                        ws[v].x = h.x; ws[v].y = h.y;
+                    } else {
+                        const u32x4_unaligned f = *reinterpret_cast<const u32x4_unaligned*>(w32 + at);
+                        ws[v] = make_uint4(f.x, f.y, f.z, f.w);
+                    }
                 } else {
-                    ws[v] = *reinterpret_cast<const uint4*>(w32 + at);
+                    const unsigned at = (unsigned)row * row_pitch + (unsigned)(k0 + off);
+                    ids[v] = *reinterpret_cast<const uint4*>(idx + at);
+                    if (BF16) {
+                        const uint2 h = *reinterpret_cast<const uint2*>(w16 + at);
+                        ws[v].x = h.x; ws[v].y = h.y;
+                    } else {
+                        ws[v] = *reinterpret_cast<const uint4*>(w32 + at);
+                    }
                 }
             } else {
                 unsigned* id4 = &ids[v].x;
@@ -533,6 +557,17 @@ __global__ __launch_bounds__(kLdThreads) void fwd_lds_kernel(const void* __restr
             if (QUADS) {
                 place((unsigned)(64 * v + lane), chunk / 4, l, k);
                 if (l < S::kGroups && 4 * k < kc) {
+                    if (ROWS == kAnyQuads && (kc & 3)) {                  // (of the quad that the row ends in, the quad before holds the first)
+                        const int seen = 4 * k + 4 - kc;
+                        const uint4 was = ids[v], wt = ws[v];
+                        ids[v].x = seen > 0 ? (unsigned)N : was.x; ids[v].y = seen > 1 ? (unsigned)N : was.y; ids[v].z = seen > 2 ? (unsigned)N : was.z;
+                        if (BF16) {
+                            ws[v].x = seen > 1 ? 0u : seen > 0 ? wt.x & 0xffff0000u : wt.x;
+                            ws[v].y = seen > 2 ? wt.y & 0xffff0000u : wt.y;
+                        } else {
+                            ws[v].x = seen > 0 ? 0u : wt.x; ws[v].y = seen > 1 ? 0u : wt.y; ws[v].z = seen > 2 ? 0u : wt.z;
+                        }
+                    }
                     if (BF16) {
                         *reinterpret_cast<uint4*>(list + l * S::kPitch + 4 * k) = make_uint4(ids[v].x * kRow, ids[v].y * kRow, ids[v].z * kRow, ids[v].w * kRow);
                         *reinterpret_cast<uint2*>(list_w + l * S::kWeightPitch + 2 * k) = make_uint2(ws[v].x, ws[v].y);
@@ -1008,6 +1043,7 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
     const size_t lds = lds_kernel_bytes<GL, BF16>(d.N) + (a.sink.tau != nullptr ? kLdThresholdBytes : 0);
     static_assert(2 * GL * LaneAcc<BF16>::kSamples * 4 <= kLdThresholdBytes, "thresholds of a slice");
     const dim3 grid((unsigned)(streams * a.slices)), block(kLdThreads);
+    const int how = a.quads ? kQuads : any_quads_pay<GL>(d.K) ? kAnyQuads : kOneByOne;
     auto go = [&](auto kernel) -> int {
         FFI_HIP_TRY(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(kernel, grid, block, lds, s, a.table, a.idx, a.w, a.bias, a.out, d.B, d.N, d.L, d.K, d.tp ? 1 : 0, a.row_step, a.slices,
@@ -1016,8 +1052,11 @@ int launch_fwd_lds(const FwdSliced& a, const Dims& d, hipStream_t s) {
         return FFI_OK;
     };
     if constexpr (GL == 2 && !BF16)
-        if (!d.tp && d.N > 512) return a.quads ? go(fwd_lds_kernel<GL, BF16, true, true>) : go(fwd_lds_kernel<GL, BF16, false, true>);
-    return a.quads ? go(fwd_lds_kernel<GL, BF16, true>) : go(fwd_lds_kernel<GL, BF16, false>);
+        if (!d.tp && d.N > 512)
+            return how == kQuads ? go(fwd_lds_kernel<GL, BF16, kQuads, true>) : how == kAnyQuads ? go(fwd_lds_kernel<GL, BF16, kAnyQuads, true>) :
+                                   go(fwd_lds_kernel<GL, BF16, kOneByOne, true>);
+    return how == kQuads ? go(fwd_lds_kernel<GL, BF16, kQuads>) : how == kAnyQuads ? go(fwd_lds_kernel<GL, BF16, kAnyQuads>) :
+                           go(fwd_lds_kernel<GL, BF16, kOneByOne>);
 }
 
 // the ordered copy of the layer: [ids][weights], part by part
