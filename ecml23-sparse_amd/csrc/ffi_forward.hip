@@ -30,31 +30,125 @@ namespace {
 // ------------------------------------------------------------------------------------------------
 // `base` is a raw LDS address: (address of the tile + (lane & 7) * 16) + row * 128.  The tile is 128-byte aligned, so the
 // chunk bits can be flipped with XOR after the add: one add and seven XORs per row instead of an add per read.
-// One connection of the lane's label: the eight 16-byte reads of row `rb` (chunk order skewed per lane) and their 32
-// multiply-adds, in a pinned order -- two reads in flight; a read's registers are refilled as soon as its four values
-// are used, under the multiply-adds of the other read.  Left to itself the scheduler finds this order or one that
-// waits for each read in turn (13 % slower over the whole kernel), depending on code far away from here.
-__device__ __forceinline__ void fwd_lane_connection(unsigned rb, float wv, float (&acc)[32]) {
-    lds_v4f a = *(lds_v4f_ptr)(size_t)rb;
-    lds_v4f b = *(lds_v4f_ptr)(size_t)(rb ^ 16u);
-    __builtin_amdgcn_sched_barrier(0);
+// ------------------------------------------------------------------------------------------------
+// A label's row of connections against a tile of W samples in LDS: the reads of a chunk of connections as one pinned stream, two in flight from its
+// first to its last (left to itself the scheduler finds that order or one that waits for each read in turn, depending on code far away from
+// here; 13 % slower over the whole kernel at 32 samples a tile, 19 at 64), ids and weights by quads whatever the fan-in.  LAST says what the row ends
+// in: 0 whole chunks; C > 0 up to C connections behind at least one chunk, loaded as the last ones of the row, of which those that are new are
+// walked; -C no whole chunk, at most C connections.  A build for each: under run-time branches the registers of the loads count as live
+// throughout, and 20 to 100 of them spill.
+//
+// Time with the connections drained one after the other and a part-filled chunk loaded one by one -> so, us.  Plain scores at 32 x 768 x 131,072, 128 x
+// 768 x 670,091 and 100 x 1,000 x 300,000: fan-in 8 12.4 -> 11.2, 156 -> 123, 36 -> 33; 13 15.4 -> 13.0, 188 -> 151, 50 -> 42; 31 32 -> 20.5,
+// 376 -> 230, 167 -> 86; 32 20.2 -> 18.4, 191 -> 188, 81 -> 77; 40 25.2 -> 21.8, 259 -> 233, 101 -> 97; 63 44 -> 32, 590 -> 369, 240 -> 153; 64 29 -> 26,
+// 333 -> 330, 147 -> 145.  20 x 700 x 20,000, a tenth of a round of labels: 1.2 to 1.5 times as fast from fan-in 13 on.  The fused training step of 32 x
+// 768 x 670,091: fan-in 8 79 -> 74, 31 263 -> 219, 32 171 -> 161, 63 529 -> 398; top-k of 200 x 300 x 100,000: 31 153 -> 95, 32 95 -> 90, 63 281 -> 142.
+// ------------------------------------------------------------------------------------------------
+template <int C>
+struct RowChunk {
+    unsigned idp[C / 2];                   // two 16-bit ids per register
+    float wv[C];
+    __device__ __forceinline__ unsigned id(int k) const { return (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu); }
+    // Quad q is that from element at(q) of the row: a lane's 16 bytes are a gather of its own, which the memory system serves at any alignment.
+    // The quads of a line one after the other: the lines of 16 wavefronts do not stay in the L1 between them (mixed with the weights', 9.3 million
+    // requests reached the L2 at 128 samples x 670,091 labels x 32, so 6.5).
+    template <class At>
+    __device__ __forceinline__ void load(const int32_t* __restrict__ irow, const float* __restrict__ wrow, At&& at) {
+        int4 v[C / 4];
+        float4 f[C / 4];
+        static_for<C / 4>([&](auto q) { v[q] = *reinterpret_cast<const int4*>(irow + at(q)); __builtin_amdgcn_sched_barrier(0); });
+        static_for<C / 4>([&](auto q) { f[q] = *reinterpret_cast<const float4*>(wrow + at(q)); __builtin_amdgcn_sched_barrier(0); });
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        acc[8 * p + 0] = fmaf(wv, a.x, acc[8 * p + 0]);
-        acc[8 * p + 4] = fmaf(wv, b.x, acc[8 * p + 4]);
-        acc[8 * p + 1] = fmaf(wv, a.y, acc[8 * p + 1]);
-        acc[8 * p + 2] = fmaf(wv, a.z, acc[8 * p + 2]);
-        acc[8 * p + 3] = fmaf(wv, a.w, acc[8 * p + 3]);
-        acc[8 * p + 5] = fmaf(wv, b.y, acc[8 * p + 5]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (p < 3) a = *(lds_v4f_ptr)(size_t)(rb ^ (unsigned)(32 * p + 32));
-        __builtin_amdgcn_sched_barrier(0);
-        acc[8 * p + 6] = fmaf(wv, b.z, acc[8 * p + 6]);
-        acc[8 * p + 7] = fmaf(wv, b.w, acc[8 * p + 7]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (p < 3) b = *(lds_v4f_ptr)(size_t)(rb ^ (unsigned)(32 * p + 48));
-        __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < C / 4; ++q) {
+            idp[2 * q + 0] = (unsigned)v[q].x | ((unsigned)v[q].y << 16);
+            idp[2 * q + 1] = (unsigned)v[q].z | ((unsigned)v[q].w << 16);
+            wv[4 * q] = f[q].x; wv[4 * q + 1] = f[q].y; wv[4 * q + 2] = f[q].z; wv[4 * q + 3] = f[q].w;
+        }
     }
+};
+
+// N connections from the FIRST of a chunk on: `skewbase` is the tile's address plus 16 (lane % (W / 4)).
+template <int W, int FIRST, int N, int C>
+__device__ __forceinline__ void walk_chunk(const RowChunk<C>& chunk, unsigned skewbase, float (&acc)[W]) {
+    stream_rows<N, W / 4, 2, W == 64 ? 2 : 1>([&](auto k) { return chunk.id(FIRST + k) * (unsigned)(W * 4) + skewbase; },
+                                              [&](auto k, auto c, const lds_v4f& v) {
+                                                  const float wv = chunk.wv[FIRST + k];
+                                                  acc[4 * c + 0] = fmaf(wv, v.x, acc[4 * c + 0]);
+                                                  acc[4 * c + 1] = fmaf(wv, v.y, acc[4 * c + 1]);
+                                                  acc[4 * c + 2] = fmaf(wv, v.z, acc[4 * c + 2]);
+                                                  acc[4 * c + 3] = fmaf(wv, v.w, acc[4 * c + 3]);
+                                              });
+}
+
+template <int LAST>
+__device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const float* __restrict__ wrow, int K, unsigned skewbase, float (&acc)[32]) {
+    if constexpr (LAST < 0) {
+        // (whole quads, those behind the last one read it again; then up to three connections one by one)
+        RowChunk<-LAST> chunk;
+        RowChunk<4> end;
+        if (K >= 4) chunk.load(irow, wrow, [&](int q) { return min(4 * q, K - 4); });
+        if (K & 3) {
+            unsigned id[3];
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                const int at = min((K & ~3) + e, K - 1);
+                id[e] = (unsigned)irow[at];
+                end.wv[e] = wrow[at];
+            }
+            end.idp[0] = id[0] | (id[1] << 16);
+            end.idp[1] = id[2];
+        }
+        static_for<-LAST / 4>([&](auto q) {
+            if (4 * q + 4 <= K) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
+        });
+        static_for<3>([&](auto e) {
+            if (e < (K & 3)) walk_chunk<32, e, 1>(end, skewbase, acc);
+        });
+    } else {
+        int k0 = 0;
+        for (; k0 + 32 <= K; k0 += 32) {
+            RowChunk<32> chunk;
+            chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
+            walk_chunk<32, 0, 32>(chunk, skewbase, acc);
+        }
+        if constexpr (LAST == 32) {                        // (in two steps: the registers of one spill)
+            RowChunk<16> chunk;
+            chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
+            walk_chunk<32, 0, 16>(chunk, skewbase, acc);
+            k0 += 16;
+        }
+        if constexpr (LAST > 0) {
+            constexpr int kLast = LAST == 32 ? 16 : LAST;
+            RowChunk<kLast> chunk;
+            chunk.load(irow, wrow, [&](int q) { return K - kLast + 4 * q; });
+            const int seen = kLast - (K - k0);
+            static_for<kLast / 4>([&](auto q) {
+                if (4 * q >= seen) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
+                else
+                    static_for<3>([&](auto i) {
+                        constexpr int k = 4 * q + 1 + i;
+                        if (k >= seen) walk_chunk<32, k, 1>(chunk, skewbase, acc);
+                    });
+            });
+        }
+    }
+}
+
+// What a row of K connections ends in, for walk_row: the few sizes that are worth a build.
+template <class Launch>
+int for_row_end(int K, Launch&& launch) {
+    const int last = K % 32;
+    if (K < 32) {
+        if (K <= 4) return launch(std::integral_constant<int, -4>{});
+        if (K <= 8) return launch(std::integral_constant<int, -8>{});
+        if (K <= 16) return launch(std::integral_constant<int, -16>{});
+        return launch(std::integral_constant<int, -32>{});
+    }
+    if (last == 0) return launch(std::integral_constant<int, 0>{});
+    if (last <= 4) return launch(std::integral_constant<int, 4>{});
+    if (last <= 8) return launch(std::integral_constant<int, 8>{});
+    if (last <= 16) return launch(std::integral_constant<int, 16>{});
+    return launch(std::integral_constant<int, 32>{});
 }
 
 // What the kernel does with a finished score s (after the bias):
@@ -126,10 +220,8 @@ __device__ __forceinline__ void loss_epilogue(float (&acc)[32], bool all_rows, u
     mask = m;
 }
 
-// VEC: how a label's column ids and weights are loaded.  0: one by one (any fan-in, any alignment); 1: by 16-byte quads
-// (fan-in a multiple of four, 16-byte aligned arrays), a partly filled last chunk one by one; 2: by quads, for a fan-in
-// below one chunk of 32 (a build of its own: the same code inside the general loop costs the full chunks 25 %).
-template <int VEC, int EPI, bool TOPK>
+// LAST: what a row ends in, see walk_row.
+template <int LAST, int EPI, bool TOPK>
 __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* __restrict__ xT,
                                                                   const int32_t* __restrict__ idx,
                                                                   const float* __restrict__ w,
@@ -154,7 +246,6 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     const unsigned skewbase = (unsigned)(size_t)(__attribute__((address_space(3))) float*)xs + (unsigned)(lane & 7) * 16u;
     const int l_begin = stream * labels_per_stream;
     const int l_end = min(l_begin + labels_per_stream, L);
-    const int nchunks = (K + 31) / 32;
     // rows of out for this batch tile, reached through a scalar row offset plus the lane's label
     const int nrows = min(kTileBatch, B - b0);
     float* obase = out + (size_t)b0 * (size_t)L;
@@ -163,8 +254,6 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     if (EPI == kEpiLossGradAndScores) grsrc = make_rsrc(fl.gout + (size_t)b0 * (size_t)L, (size_t)nrows * (size_t)L * sizeof(float));
     float lsum = 0.f;
 
-    constexpr bool VEC4 = VEC >= 1;
-    constexpr bool SHORT = VEC == 2;
     constexpr bool SKEW = EPI == kEpiLossGradSkewed;
     constexpr bool LOSS = EPI == kEpiLossGrad || EPI == kEpiLossGradAndScores || SKEW;
     static_assert(!(SKEW && TOPK), "the top-k tests need the natural order");
@@ -182,53 +271,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
         float acc[32];
 #pragma unroll
         for (int i = 0; i < 32; ++i) acc[i] = 0.f;
-        for (int ch = 0; ch < nchunks; ++ch) {
-            const int k0 = ch * 32;
-            const bool full = VEC4 && !SHORT && k0 + 32 <= K;
-            unsigned idp[16];
-            float wv[32];
-            if (SHORT) {
-                // the one, partly filled chunk: the quads behind its end re-read its first quad, so that the loads stay
-                // unconditional; their connections are skipped below
-                const int quads = K >> 2;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int at = 4 * (q < quads ? q : 0);
-                    const int4 v = *reinterpret_cast<const int4*>(irow + at);
-                    idp[2 * q + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
-                    idp[2 * q + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
-                    const float4 f = *reinterpret_cast<const float4*>(wrow + at);
-                    wv[4 * q] = f.x; wv[4 * q + 1] = f.y; wv[4 * q + 2] = f.z; wv[4 * q + 3] = f.w;
-                }
-            } else if (full) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int4 v = *reinterpret_cast<const int4*>(irow + k0 + 4 * q);
-                    idp[2 * q + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
-                    idp[2 * q + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
-                    const float4 f = *reinterpret_cast<const float4*>(wrow + k0 + 4 * q);
-                    wv[4 * q] = f.x; wv[4 * q + 1] = f.y; wv[4 * q + 2] = f.z; wv[4 * q + 3] = f.w;
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const unsigned a = (k0 + 2 * q < K) ? (unsigned)irow[k0 + 2 * q] : 0u;
-                    const unsigned b = (k0 + 2 * q + 1 < K) ? (unsigned)irow[k0 + 2 * q + 1] : 0u;
-                    idp[q] = a | (b << 16);
-                }
-#pragma unroll
-                for (int k = 0; k < 32; ++k) wv[k] = (k0 + k < K) ? wrow[k0 + k] : 0.f;
-            }
-            const int kn = min(32, K - k0);
-#pragma unroll
-            for (int k = 0; k < 32; ++k) {
-                if (full || k < kn) {
-                    const unsigned id = (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu);
-                    const unsigned rb = (id << 7) + skewbase;
-                    fwd_lane_connection(rb, wv[k], acc);
-                }
-            }
-        }
+        walk_row<LAST>(irow, wrow, K, skewbase, acc);
         if (!SKEW) xor_permute_groups(acc, lane & 7);      // back to natural batch order
         if (bias != nullptr) {                             // added after the sum, as a separate bias_add would
             const float bj = bias[jj];
@@ -344,119 +387,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     }
 }
 
-// ------------------------------------------------------------------------------------------------
-// A label's row of connections against a tile of W samples in LDS, for plain scores: the reads of a chunk of connections as one pinned
-// stream, two in flight (the kernel above drains them after each connection), ids and weights by quads whatever the fan-in.  LAST says what the
-// row ends in: 0 whole chunks; C > 0 up to C connections behind at least one chunk, loaded as the last C of the row, of which those that are
-// new are walked; -C no whole chunk, at most C connections.  A build for each: under run-time branches the registers of the loads count as
-// live throughout, and 20 to 100 of them spill.
-//
-// Time with the connections drained one after the other and a part-filled chunk loaded one by one -> so, us, at 32 x 768 x 131,072, 128 x 768 x
-// 670,091 and 100 x 1,000 x 300,000: fan-in 8 12.4 -> 11.2, 156 -> 123, 36 -> 33; 13 15.4 -> 13.0, 188 -> 151, 50 -> 42; 31 32 -> 20.5, 376 -> 230,
-// 167 -> 86; 32 20.2 -> 18.4, 191 -> 188, 81 -> 77; 40 25.2 -> 21.8, 259 -> 233, 101 -> 97; 63 44 -> 32, 590 -> 369, 240 -> 153; 64 29 -> 26,
-// 333 -> 330, 147 -> 145.  20 x 700 x 20,000, a tenth of a round of labels: 1.2 to 1.5 times as fast from fan-in 13 on.
-// ------------------------------------------------------------------------------------------------
-template <int C>
-struct RowChunk {
-    unsigned idp[C / 2];                   // two 16-bit ids per register
-    float wv[C];
-    __device__ __forceinline__ unsigned id(int k) const { return (k & 1) ? (idp[k >> 1] >> 16) : (idp[k >> 1] & 0xffffu); }
-    // Quad q is that from element at(q) of the row: a lane's 16 bytes are a gather of its own, which the memory system serves at any alignment.
-    // The quads of a line one after the other: the lines of 16 wavefronts do not stay in the L1 between them (mixed with the weights', 9.3 million
-    // requests reached the L2 at 128 samples x 670,091 labels x 32, so 6.5).
-    template <class At>
-    __device__ __forceinline__ void load(const int32_t* __restrict__ irow, const float* __restrict__ wrow, At&& at) {
-        int4 v[C / 4];
-        float4 f[C / 4];
-        static_for<C / 4>([&](auto q) { v[q] = *reinterpret_cast<const int4*>(irow + at(q)); __builtin_amdgcn_sched_barrier(0); });
-        static_for<C / 4>([&](auto q) { f[q] = *reinterpret_cast<const float4*>(wrow + at(q)); __builtin_amdgcn_sched_barrier(0); });
-#pragma unroll
-        for (int q = 0; q < C / 4; ++q) {
-            idp[2 * q + 0] = (unsigned)v[q].x | ((unsigned)v[q].y << 16);
-            idp[2 * q + 1] = (unsigned)v[q].z | ((unsigned)v[q].w << 16);
-            wv[4 * q] = f[q].x; wv[4 * q + 1] = f[q].y; wv[4 * q + 2] = f[q].z; wv[4 * q + 3] = f[q].w;
-        }
-    }
-};
-
-// N connections from the FIRST of a chunk on: `skewbase` is the tile's address plus 16 (lane % (W / 4)).
-template <int W, int FIRST, int N, int C>
-__device__ __forceinline__ void walk_chunk(const RowChunk<C>& chunk, unsigned skewbase, float (&acc)[W]) {
-    stream_rows<N, W / 4, 2, W == 64 ? 2 : 1>([&](auto k) { return chunk.id(FIRST + k) * (unsigned)(W * 4) + skewbase; },
-                                              [&](auto k, auto c, const lds_v4f& v) {
-                                                  const float wv = chunk.wv[FIRST + k];
-                                                  acc[4 * c + 0] = fmaf(wv, v.x, acc[4 * c + 0]);
-                                                  acc[4 * c + 1] = fmaf(wv, v.y, acc[4 * c + 1]);
-                                                  acc[4 * c + 2] = fmaf(wv, v.z, acc[4 * c + 2]);
-                                                  acc[4 * c + 3] = fmaf(wv, v.w, acc[4 * c + 3]);
-                                              });
-}
-
-template <int LAST>
-__device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const float* __restrict__ wrow, int K, unsigned skewbase, float (&acc)[32]) {
-    if constexpr (LAST < 0) {
-        // (whole quads, those behind the last one read it again; then up to three connections one by one)
-        RowChunk<-LAST> chunk;
-        RowChunk<4> end;
-        if (K >= 4) chunk.load(irow, wrow, [&](int q) { return min(4 * q, K - 4); });
-        if (K & 3) {
-            unsigned id[3];
-#pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                const int at = min((K & ~3) + e, K - 1);
-                id[e] = (unsigned)irow[at];
-                end.wv[e] = wrow[at];
-            }
-            end.idp[0] = id[0] | (id[1] << 16);
-            end.idp[1] = id[2];
-        }
-        static_for<-LAST / 4>([&](auto q) {
-            if (4 * q + 4 <= K) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
-        });
-        static_for<3>([&](auto e) {
-            if (e < (K & 3)) walk_chunk<32, e, 1>(end, skewbase, acc);
-        });
-    } else {
-        int k0 = 0;
-        for (; k0 + 32 <= K; k0 += 32) {
-            RowChunk<32> chunk;
-            chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
-            walk_chunk<32, 0, 32>(chunk, skewbase, acc);
-        }
-        if constexpr (LAST > 0) {
-            RowChunk<LAST> chunk;
-            chunk.load(irow, wrow, [&](int q) { return K - LAST + 4 * q; });
-            const int seen = LAST - (K - k0);
-            static_for<LAST / 4>([&](auto q) {
-                if (4 * q >= seen) walk_chunk<32, 4 * q, 4>(chunk, skewbase, acc);
-                else
-                    static_for<3>([&](auto i) {
-                        constexpr int k = 4 * q + 1 + i;
-                        if (k >= seen) walk_chunk<32, k, 1>(chunk, skewbase, acc);
-                    });
-            });
-        }
-    }
-}
-
-// What a row of K connections ends in, for walk_row: whole quads of the few sizes that are worth a build.
-template <class Launch>
-int for_row_end(int K, Launch&& launch) {
-    const int last = K % 32;
-    if (K < 32) {
-        if (K <= 4) return launch(std::integral_constant<int, -4>{});
-        if (K <= 8) return launch(std::integral_constant<int, -8>{});
-        if (K <= 16) return launch(std::integral_constant<int, -16>{});
-        return launch(std::integral_constant<int, -32>{});
-    }
-    if (last == 0) return launch(std::integral_constant<int, 0>{});
-    if (last <= 4) return launch(std::integral_constant<int, 4>{});
-    if (last <= 8) return launch(std::integral_constant<int, 8>{});
-    if (last <= 16) return launch(std::integral_constant<int, 16>{});
-    return launch(std::integral_constant<int, 32>{});
-}
-
-// The kernel above for plain scores.
+// The kernel above for plain scores, which leave as soon as they are in order: fewer registers, and a build for every way a row ends.
 template <int LAST>
 __global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
                                                                     const float* __restrict__ w, const float* __restrict__ bias,
@@ -689,11 +620,11 @@ __global__ __launch_bounds__(256) void fwd_sample_kernel(const float* __restrict
     }
 }
 
-template <int VEC, int EPI, bool TOPK>
+template <int LAST, int EPI, bool TOPK>
 int launch_lane32(const float* xT, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, int nbt,
                   int per_stream, int blocks, size_t lds, const FwdLoss& fl, const FwdTopk& ft, hipStream_t s) {
-    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lane32_kernel<VEC, EPI, TOPK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((fwd_lane32_kernel<VEC, EPI, TOPK>), dim3(blocks), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N,
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_lane32_kernel<LAST, EPI, TOPK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((fwd_lane32_kernel<LAST, EPI, TOPK>), dim3(blocks), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N,
                        d.L, d.K, nbt, per_stream, fl, ft);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
@@ -709,22 +640,22 @@ int launch_stream32(const float* xT, const int32_t* idx, const float* w, const f
 }
 
 template <int EPI>
-int launch_lane32_any(bool vec4, bool topk, const float* xT, const int32_t* idx, const float* w, const float* bias, float* out,
+int launch_lane32_any(bool topk, const float* xT, const int32_t* idx, const float* w, const float* bias, float* out,
                       const Dims& d, int nbt, int per_stream, int blocks, size_t lds, const FwdLoss& fl, const FwdTopk& ft,
                       hipStream_t s) {
-    // (see fwd_lane32_kernel: 2 = quads, fan-in below one chunk)
-    // Rows that are not 16-byte aligned (a fan-in that is no multiple of four, or unaligned arrays) still take build 1
-    // when they hold a full chunk: its 16-byte loads are per-lane gathers of 4-byte-aligned addresses, which the
-    // memory system serves, and only the last, partly filled chunk is loaded one by one (fan-in 33: 412 -> 215 us, fan-in 63: 1.10 -> 0.58 ms).
-    const int vec = vec4 ? (d.K < 32 ? 2 : 1) : ((((uintptr_t)w | (uintptr_t)idx) % 4 == 0 && d.K >= 32) ? 1 : 0);
-#define FFI_LANE32(VEC, E, T) launch_lane32<VEC, E, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s)
+    auto go = [&](auto top) -> int {
+        constexpr bool T = decltype(top)::value;
+        if (d.K < 32) return launch_lane32<-32, EPI, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s);
+        if (d.K % 32 == 0) return launch_lane32<0, EPI, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s);
+        if (d.K % 32 <= 8) return launch_lane32<8, EPI, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s);
+        if (d.K % 32 <= 16) return launch_lane32<16, EPI, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s);
+        return launch_lane32<32, EPI, T>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, fl, ft, s);
+    };
     if constexpr (EPI != kEpiLossGradSkewed) {              // (that epilogue has no top-k form)
-        if (topk) return vec == 2 ? FFI_LANE32(2, EPI, true) : vec == 1 ? FFI_LANE32(1, EPI, true) : FFI_LANE32(0, EPI, true);
+        if (topk) return go(std::true_type{});
     }
-    if constexpr (EPI != kEpiNone && EPI != kEpiScores)     // (plain scores: fwd_stream32_kernel)
-        return vec == 2 ? FFI_LANE32(2, EPI, false) : vec == 1 ? FFI_LANE32(1, EPI, false) : FFI_LANE32(0, EPI, false);
+    if constexpr (EPI != kEpiNone && EPI != kEpiScores) return go(std::false_type{});      // (plain scores: fwd_stream32_kernel)
     else return FFI_ERR_BAD_ARGUMENT;
-#undef FFI_LANE32
 }
 
 // Narrow-input forward pass with the given epilogue; `la` is needed for the loss epilogues only, `tk` (may be
@@ -741,7 +672,6 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         xT = ws;
     }
     const size_t lds = tile_lds_bytes(d.N);
-    const bool vec4 = (d.K % 4 == 0) && (((uintptr_t)w | (uintptr_t)idx) % 16 == 0);
     if (epi == kEpiScores && tk == nullptr && lane64_fits(d)) return launch_lane64(xT, idx, w, bias, out, d, s);
     const int cus = device_cu_count();
     const int nbt = (d.B + kTileBatch - 1) / kTileBatch;
@@ -780,12 +710,12 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         fl.words = la->nz_words;
         fl.skip_zero_stores = la->skip_zero_stores ? 1 : 0;
     }
-    if (epi == kEpiScores) FFI_TRY(launch_lane32_any<kEpiScores>(vec4, topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
+    if (epi == kEpiScores) FFI_TRY(launch_lane32_any<kEpiScores>(topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
     else if (epi == kEpiLossGrad && !topk && fl.skip_zero_stores)
-        FFI_TRY(launch_lane32_any<kEpiLossGradSkewed>(vec4, false, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
-    else if (epi == kEpiLossGrad) FFI_TRY(launch_lane32_any<kEpiLossGrad>(vec4, topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
-    else if (epi == kEpiLossGradAndScores) FFI_TRY(launch_lane32_any<kEpiLossGradAndScores>(vec4, topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
-    else FFI_TRY(launch_lane32_any<kEpiNone>(vec4, topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
+        FFI_TRY(launch_lane32_any<kEpiLossGradSkewed>(false, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
+    else if (epi == kEpiLossGrad) FFI_TRY(launch_lane32_any<kEpiLossGrad>(topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
+    else if (epi == kEpiLossGradAndScores) FFI_TRY(launch_lane32_any<kEpiLossGradAndScores>(topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
+    else FFI_TRY(launch_lane32_any<kEpiNone>(topk, xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds_topk, fl, ft, s));
     if (topk) {
         // (a sample with more candidates than its list holds: its row once more, from the score matrix if there is one)
         TopkRowSource src;
