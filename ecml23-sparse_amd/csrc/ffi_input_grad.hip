@@ -89,11 +89,12 @@ __global__ __launch_bounds__(1024) void igrad_permute_weights_kernel(
 // block of the weights << 17) | (LDS row << 7), in place of lab16:
 // the tile's weights are staged in LDS behind the rows of out_grad (with a zero word at tile_labels * K that
 // padding slots read) and every slot fetches its weight from there, so no slot-ordered copy of the weights exists.
-// PERM (with WLDS and LPT == 1): `colperm` names, per tile, the column each thread walks -- the plan sorts a tile's columns by
-// length so that the 64 columns of a wavefront are about equally long.  The thread's sums over one tile then belong to
-// another thread's column: after every tile they pass through LDS (the tile's rows and weights are dead by then; row n of
-// the exchange = column n, chunks skewed like every other row) to the column's own thread, which adds them to the
-// sums it keeps over the whole label stream.
+// PERM (with LPT == 1): `colperm` names, per tile, the column each thread walks -- the plan sorts a tile's columns by
+// length so that the 64 columns of a wavefront are about equally long.  The thread's sums then belong to another thread's
+// column: after every tile they pass through LDS (the tile's rows and weights are dead by then; row n of
+// the exchange = column n, chunks skewed like every other row).  With WLDS a tile's sums go to the column's own thread, which adds them to those it
+// keeps over the whole label stream; without, where nobody keeps sums of its own and the registers are half as many, the
+// sums over all tiles so far go to the thread that walks the column next.
 template <int MAXT, int LPT, bool WLDS, bool PERM = false>
 __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* __restrict__ lab16, const float* __restrict__ wp,
                                   const unsigned* __restrict__ slice_off,
@@ -101,7 +102,8 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
                                   int tile_labels, int tiles, int tiles_per_stream, int nbt, unsigned total_rows,
                                   const unsigned short* __restrict__ rowpos, int zero_row,
                                   const unsigned* __restrict__ slot32, int K, const unsigned short* __restrict__ colperm = nullptr) {
-    static_assert(!PERM || (WLDS && LPT == 1), "the exchange of sums is built for the weights-in-LDS form");
+    static_assert(!PERM || LPT == 1, "the exchange of sums takes a row per thread");
+    constexpr bool KEEP = PERM && WLDS;                    // (each tile's sums are added to those before; else the sums move on with their column)
     extern __shared__ __align__(16) float gs[];
     char* gs_bytes = reinterpret_cast<char*>(gs);
     const int nthreads = blockDim.x;
@@ -128,29 +130,36 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
     for (int i = 0; i < 32; ++i) acc[i] = 0.f;
     // (PERM) the sums of the thread's own column over the tiles so far; `acc` holds one tile's sums of whatever column
     // the thread walks in it
-    float home[PERM ? 32 : 1];
+    float home[KEEP ? 32 : 1];
 #pragma unroll
-    for (int i = 0; i < (PERM ? 32 : 1); ++i) home[i] = 0.f;
+    for (int i = 0; i < (KEEP ? 32 : 1); ++i) home[i] = 0.f;
     unsigned walked = 0;                                   // (PERM) the column of the tile just walked
     // acc -> row `walked` of the exchange; a barrier; row threadIdx.x -> home.  Called between two barriers that keep
     // the tile's rows from being read or written meanwhile.
-    auto hand_over = [&]() __attribute__((always_inline)) {
+    // (without KEEP: -> acc, from the row of the column that the thread walks next)
+    auto hand_over = [&](unsigned next) __attribute__((always_inline)) {
         char* rowp = gs_bytes + ((size_t)walked << 7);
         const int r = lane & 7;
 #pragma unroll
         for (int c = 0; c < 8; ++c)
             *reinterpret_cast<float4*>(rowp + ((c ^ r) << 4)) = make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]);
         __syncthreads();
-        const char* mine = gs_bytes + ((size_t)threadIdx.x << 7);
+        const char* mine = gs_bytes + ((size_t)(KEEP ? threadIdx.x : next) << 7);
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const float4 v = *reinterpret_cast<const float4*>(mine + ((c ^ r) << 4));
+            if constexpr (!KEEP) {
+                acc[4 * c] = v.x; acc[4 * c + 1] = v.y; acc[4 * c + 2] = v.z; acc[4 * c + 3] = v.w;
+                continue;
+            }
             // (group c of `home`, like group c of `acc`, holds batch entries 4 (c ^ r) ...: undone once, at the end)
-            home[PERM ? 4 * c : 0] += v.x; home[PERM ? 4 * c + 1 : 0] += v.y;
-            home[PERM ? 4 * c + 2 : 0] += v.z; home[PERM ? 4 * c + 3 : 0] += v.w;
+            home[KEEP ? 4 * c : 0] += v.x; home[KEEP ? 4 * c + 1 : 0] += v.y;
+            home[KEEP ? 4 * c + 2 : 0] += v.z; home[KEEP ? 4 * c + 3 : 0] += v.w;
         }
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+            for (int i = 0; i < 32; ++i) acc[i] = 0.f;
+        }
     };
 
     for (int t = t_begin; t < t_end; ++t) {
@@ -223,12 +232,12 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
         const unsigned wpieces = (nw + 255u) / 256u;
         if (PERM) {
             if (t > t_begin) {
-                hand_over();
+                hand_over(next_walked);
                 __syncthreads();               // the exchange has been read: the tile may be staged over it
             }
             // (requested only now that the exchange is over: asked for in front of it, the pieces that land behind the
             // exchange's rows made the kernel 4 % slower)
-            if (wvec) weights_to_lds(0u, wpieces);
+            if (WLDS && wvec) weights_to_lds(0u, wpieces);
             walked = next_walked;
         }
         // rows `zero_row` (even) and `zero_row + 1` (odd) are all zero: the targets of padding slots
@@ -267,7 +276,7 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
                         make_float4(gbn[p][4 * c], gbn[p][4 * c + 1], gbn[p][4 * c + 2], gbn[p][4 * c + 3]);
             }
         }
-        if (PERM) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the weights have arrived in LDS
+        if (KEEP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the weights have arrived in LDS
         __syncthreads();
         if (rows == 0) continue;               // wave-uniform: no column of this slice is used in the tile
         for (unsigned i = 0; i < rows; i += kAhead) {
@@ -309,9 +318,11 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
     }
     if (PERM) {
         __syncthreads();                       // the last tile is no longer being read
-        if (t_begin < t_end) hand_over();
+        if (t_begin < t_end) hand_over(threadIdx.x);
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) acc[i] = home[PERM ? i : 0];
+            for (int i = 0; i < 32; ++i) acc[i] = home[KEEP ? i : 0];
+        }
     }
     // back to natural batch order, then one 128-byte row per thread
     xor_permute_groups(acc, lane & 7);
@@ -396,27 +407,29 @@ int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, i
     // the tile's rows + the two all-zero rows (+ the tile's weights)
     const size_t lds = tiled_lds_bytes(p->tile_labels, p->K, p->w_in_lds);
     const dim3 grid(streams * nbt), block(p->threads);
-#define FFI_LAUNCH_TILE(MAXT, LPT, WLDS)                                                                                \
+#define FFI_LAUNCH_TILE_AS(MAXT, LPT, WLDS, PERM, BYTES)                                                                \
     do {                                                                                                                \
-        FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_tile_kernel<MAXT, LPT, WLDS>,                                \
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                        \
-        hipLaunchKernelGGL((igrad_tile_kernel<MAXT, LPT, WLDS>), grid, block, lds, s, p->lab16, WLDS ? w : wp, p->slice_off, g, \
+        FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_tile_kernel<MAXT, LPT, WLDS, PERM>,                          \
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(BYTES)));                    \
+        hipLaunchKernelGGL((igrad_tile_kernel<MAXT, LPT, WLDS, PERM>), grid, block, BYTES, s, p->lab16, WLDS ? w : wp, p->slice_off, g, \
                            partial, B, p->L, p->tile_labels, p->tiles, tps, nbt, (unsigned)p->total_rows, p->rowpos, p->zero_row, \
-                           p->slot32, p->K);                                                                             \
+                           p->slot32, p->K, p->colperm);                                                                 \
     } while (0)
+#define FFI_LAUNCH_TILE(MAXT, LPT, WLDS) FFI_LAUNCH_TILE_AS(MAXT, LPT, WLDS, false, lds)
+    // (the exchange of sums between the threads takes a 128-byte row per thread, wherever the tile ends)
+    const size_t lds_x = std::max(lds, (size_t)p->threads * kTileBatch * sizeof(float));
     // the plan sizes its tiles so that one of these fits: tile_labels <= LPT * threads
     if (p->w_in_lds) {
         // (plans take that form only with workgroups of at most 768 threads that stage one label each)
         if (p->threads > 768 || p->tile_labels > p->threads) return FFI_ERR_BAD_ARGUMENT;
         if (p->colperm != nullptr) {
-            // (the exchange of sums between the threads takes a 128-byte row per thread, wherever the tile ends)
-            const size_t lds_x = std::max(lds, (size_t)p->threads * kTileBatch * sizeof(float));
-            FFI_HIP_TRY(hipFuncSetAttribute((const void*)igrad_tile_kernel<768, 1, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_x));
-            hipLaunchKernelGGL((igrad_tile_kernel<768, 1, true, true>), grid, block, lds_x, s, p->lab16, w, p->slice_off, g, partial, B, p->L,
-                               p->tile_labels, p->tiles, tps, nbt, (unsigned)p->total_rows, p->rowpos, p->zero_row, p->slot32, p->K, p->colperm);
+            FFI_LAUNCH_TILE_AS(768, 1, true, true, lds_x);
         } else {
             FFI_LAUNCH_TILE(768, 1, true);
         }
+    } else if (p->colperm != nullptr) {
+        if (p->tile_labels > p->threads) return FFI_ERR_BAD_ARGUMENT;
+        if (per_cu > 1 || p->threads > 768) FFI_LAUNCH_TILE_AS(1024, 1, false, true, lds_x); else FFI_LAUNCH_TILE_AS(768, 1, false, true, lds_x);
     } else if (per_cu > 1) {
         FFI_LAUNCH_TILE(1024, 1, false);                 // (the instantiation of at most 128 registers)
     } else if (p->threads <= 768) {
@@ -425,6 +438,7 @@ int launch_tiled(const ffi_plan* p, const float* w, const float* g, float* gx, i
         FFI_LAUNCH_TILE(1024, 1, false);
     }
 #undef FFI_LAUNCH_TILE
+#undef FFI_LAUNCH_TILE_AS
     // (64 streams of 128 samples: 6.2 us by one thread per sum, 6.9 by two)
     const int width = B <= 32 ? 32 : B <= 64 ? 64 : B <= 128 ? 128 : 256, groups = streams >= 128 && B <= 128 ? std::min(8, streams / 32) : 1;
     const int ncols = p->col_n ? p->col_n : p->N, btiles = (B + width - 1) / width;

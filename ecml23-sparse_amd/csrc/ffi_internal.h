@@ -34,7 +34,7 @@ struct Options {
     int wide_phases = 0;            // -1: never / 1: wherever it can: the forward kernel in phases for wide inputs
     int small_path = 0;             // -1: never / 1: wherever they can: the two launches for small layers
     int dense_rows = 0;             // -1: never / 1: wherever they can: the kernels for few columns
-    int plan_sorted_columns = 0;    // -1: never / 1: always (in the weights-in-LDS form) the plans that hand the columns to the walking kernel's threads tile by tile, by length
+    int plan_sorted_columns = 0;    // -1: never / 1: always (with a label per thread to stage) the plans that hand the columns to the walking kernel's threads tile by tile, by length
 };
 extern Options g_options;
 
@@ -404,13 +404,16 @@ inline int tiled_workgroups_per_cu(int threads, int tile_labels, int K, bool wit
     return n < 1 ? 1 : n;
 }
 // Whether a tiled plan hands its columns to the walking kernel's threads tile by tile, sorted by length (ffi_plan.hip,
-// tile_perm_kernel): the weights-in-LDS form with six or more slices, where every workgroup walks two tiles or more.
+// tile_perm_kernel): forms that stage a label per thread, with six or more slices, where every workgroup walks two tiles or more.
 inline bool plan_sorts_columns(int threads, int tile_labels, int K, bool weights_in_lds, int tiles, int batch_hint) {
-    if (!weights_in_lds || g_options.plan_sorted_columns < 0) return false;
+    if (g_options.plan_sorted_columns < 0 || tile_labels > threads) return false;
     if (g_options.plan_sorted_columns > 0) return true;                 // (tests: whenever the form allows)
     if (threads < 384) return false;
+    // (weights in slot order: 256 x 512 x 501,070 x 64 1.30 -> 1.06 slot rows a connection, the gradient's kernel 500 -> 462 us and the weights' 103 -> 95, forward
+    // and backward's gradients 1,080 -> 1,022; fan-in 48 923 -> 853, 32 697 -> 686, 24 605 -> 622; 300 x 900 x 100,000 x 64 373 -> 346; 512 x 700 x 60,000 x 40 204 -> 212)
+    if (!weights_in_lds && (K < 32 || (threads > 512 && threads <= 768))) return false;
     const int nbt = batch_hint > 32 ? (batch_hint + 31) / 32 : 1;
-    const int per_stream = tiled_workgroups_per_cu(threads, tile_labels, K, true, nbt) * device_cu_count() / nbt;
+    const int per_stream = tiled_workgroups_per_cu(threads, tile_labels, K, weights_in_lds, nbt) * device_cu_count() / nbt;
     return tiles >= 2 * (per_stream > 1 ? per_stream : 1);
 }
 constexpr int kArrIdBits = 11;            // column-id field of an arranged entry (narrow inputs: ids < 1216)

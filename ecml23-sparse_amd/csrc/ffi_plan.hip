@@ -1209,8 +1209,7 @@ int build_tiled(ffi_plan* p, const int32_t* lookup, hipStream_t s, const std::fu
     const int slices = threads / 64;
     const int tiles = (p->L + TL - 1) / TL;
     const size_t nslices = (size_t)tiles * slices;
-    // (the walking kernel hands its sums from the tile's thread to the column's own thread through LDS: built for the
-    // weights-in-LDS form, whose workgroup has the registers for both sets of sums)
+    // (the walking kernel hands its sums from the tile's thread to the column's own thread, or to its next, through LDS)
     // Measured (input gradient, weights-in-LDS form, sorted against thread t <-> column t): 768 columns x fan-in 32, batch 128:
     // 1.517 -> 1.150 slot rows per connection, 251 -> 239 us; batch 64: 151 -> 141; fan-in 16: 178 -> 170; fan-in 64 (300,000
     // labels): 207 -> 190; 512 columns: 261 -> 251; 640 columns, batch 256: 226 -> 215; no gain at 256 columns and fewer (few

@@ -60,3 +60,39 @@ def test_a_plan_that_is_being_laid_out_serves_other_streams(features):
         ref_gx, ref_gw = oracle.backward(x, shifted[turn], w, g, transposed=False)
         for gx, gw in results:
             assert rel_err(gx.cpu().numpy(), ref_gx) <= 1e-5 and rel_err(gw.cpu().numpy(), ref_gw) <= 1e-5
+
+
+@pytest.mark.parametrize("batch,features,labels,fan_in", [(256, 512, 140_001, 40), (300, 900, 33_003, 33), (161, 385, 90_000, 65), (200, 448, 70_001, 100)])
+def test_columns_sorted_tile_by_tile_with_weights_in_slot_order(batch, features, labels, fan_in):
+    # the sums move with their column from thread to thread between the tiles
+    ffi = load_package()
+    lib = ffi._lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(labels)
+    lookup = torch.randint(0, features, (labels, fan_in), generator=gen, device="cuda", dtype=torch.int32)
+    lookup[::7, : fan_in // 2] = 3                             # (a column far longer than the others)
+    w = torch.randn((labels, fan_in), generator=gen, device="cuda")
+    g = torch.randn((batch, labels), generator=gen, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    results = []
+    for value in (1, -1, 0):
+        assert lib.ffi_set_option(b"plan_sorted_columns", value) == 0 and lib.ffi_set_option(b"plan_weights_in_lds", -1) == 0
+        try:
+            plan = ctypes.c_void_p()
+            ffi._lib.check(lib.ffi_plan_create(lookup.data_ptr(), labels, fan_in, features, batch, stream, ctypes.byref(plan)))
+            gx = torch.full((batch, features), float("nan"), device="cuda")
+            ffi._lib.check(lib.ffi_input_grad_planned_f32(plan, w.data_ptr(), g.data_ptr(), gx.data_ptr(), batch, 0, stream))
+            torch.cuda.synchronize()
+            ffi._lib.check(lib.ffi_plan_destroy(plan))
+        finally:
+            assert lib.ffi_set_option(b"plan_sorted_columns", 0) == 0 and lib.ffi_set_option(b"plan_weights_in_lds", 0) == 0
+        results.append(gx)
+    exact = torch.zeros((batch, features), dtype=torch.float64, device="cuda")
+    magnitude = torch.zeros_like(exact)
+    for k in range(fan_in):
+        term = g.double() * w[:, k].double()
+        exact.index_add_(1, lookup[:, k].long(), term)
+        magnitude.index_add_(1, lookup[:, k].long(), term.abs())
+    for gx in results:
+        # (sums of some thousand terms a stream, in order: far below 2^-24 times their number and magnitude)
+        assert bool(((gx.double() - exact).abs() <= 1e-5 * magnitude + 1e-6).all())
+        assert rel_err(gx.cpu().numpy(), exact.cpu().numpy()) <= 1e-5
