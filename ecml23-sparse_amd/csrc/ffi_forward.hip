@@ -28,9 +28,6 @@ namespace {
 // the chunk order skewed by its lane id; the accumulators are brought back to natural batch order
 // before the stores, which are then full 256-byte rows of out per wavefront.
 // ------------------------------------------------------------------------------------------------
-// `base` is a raw LDS address: (address of the tile + (lane & 7) * 16) + row * 128.  The tile is 128-byte aligned, so the
-// chunk bits can be flipped with XOR after the add: one add and seven XORs per row instead of an add per read.
-// ------------------------------------------------------------------------------------------------
 // A label's row of connections against a tile of W samples in LDS: the reads of a chunk of connections as one pinned stream, two in flight from its
 // first to its last (left to itself the scheduler finds that order or one that waits for each read in turn, depending on code far away from
 // here; 13 % slower over the whole kernel at 32 samples a tile, 19 at 64), ids and weights by quads whatever the fan-in.  LAST says what the row ends
@@ -68,9 +65,9 @@ struct RowChunk {
 };
 
 // N connections from the FIRST of a chunk on: `skewbase` is the tile's address plus 16 (lane % (W / 4)).
-template <int W, int FIRST, int N, int C>
+template <int W, int FIRST, int N, int GROUP = W == 64 ? 2 : 1, int C>
 __device__ __forceinline__ void walk_chunk(const RowChunk<C>& chunk, unsigned skewbase, float (&acc)[W]) {
-    stream_rows<N, W / 4, 2, W == 64 ? 2 : 1>([&](auto k) { return chunk.id(FIRST + k) * (unsigned)(W * 4) + skewbase; },
+    stream_rows<N, W / 4, 2, GROUP>([&](auto k) { return chunk.id(FIRST + k) * (unsigned)(W * 4) + skewbase; },
                                               [&](auto k, auto c, const lds_v4f& v) {
                                                   const float wv = chunk.wv[FIRST + k];
                                                   acc[4 * c + 0] = fmaf(wv, v.x, acc[4 * c + 0]);
@@ -80,7 +77,7 @@ __device__ __forceinline__ void walk_chunk(const RowChunk<C>& chunk, unsigned sk
                                               });
 }
 
-template <int LAST>
+template <int LAST, int GROUP = 1>
 __device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const float* __restrict__ wrow, int K, unsigned skewbase, float (&acc)[32]) {
     if constexpr (LAST < 0) {
         // (whole quads, those behind the last one read it again; then up to three connections one by one)
@@ -109,7 +106,7 @@ __device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const
         for (; k0 + 32 <= K; k0 += 32) {
             RowChunk<32> chunk;
             chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
-            walk_chunk<32, 0, 32>(chunk, skewbase, acc);
+            walk_chunk<32, 0, 32, GROUP>(chunk, skewbase, acc);
         }
         if constexpr (LAST == 32) {                        // (in two steps: the registers of one spill)
             RowChunk<16> chunk;
@@ -388,7 +385,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
 }
 
 // The kernel above for plain scores, which leave as soon as they are in order: fewer registers, and a build for every way a row ends.
-template <int LAST>
+template <int LAST, int GROUP>
 __global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
                                                                     const float* __restrict__ w, const float* __restrict__ bias,
                                                                     float* __restrict__ out, int B, int N, int L, int K, int nbt, int labels_per_stream) {
@@ -412,7 +409,7 @@ __global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float*
         float acc[32];
 #pragma unroll
         for (int i = 0; i < 32; ++i) acc[i] = 0.f;
-        walk_row<LAST>(irow, wrow, K, skewbase, acc);
+        walk_row<LAST, GROUP>(irow, wrow, K, skewbase, acc);
         xor_permute_groups(acc, lane & 7);                 // back to natural batch order
         if (bias != nullptr) {                             // added after the sum, as a separate bias_add would
             const float bj = bias[min(j, l_end - 1)];
@@ -630,11 +627,11 @@ int launch_lane32(const float* xT, const int32_t* idx, const float* w, const flo
     return FFI_OK;
 }
 
-template <int LAST>
+template <int LAST, int GROUP = 1>
 int launch_stream32(const float* xT, const int32_t* idx, const float* w, const float* bias, float* out, const Dims& d, int nbt, int per_stream, int blocks,
                     size_t lds, hipStream_t s) {
-    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_stream32_kernel<LAST>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(fwd_stream32_kernel<LAST>, dim3(blocks), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N, d.L, d.K, nbt, per_stream);
+    FFI_HIP_TRY(hipFuncSetAttribute((const void*)fwd_stream32_kernel<LAST, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((fwd_stream32_kernel<LAST, GROUP>), dim3(blocks), dim3(kTileThreads), lds, s, xT, idx, w, bias, out, d.B, d.N, d.L, d.K, nbt, per_stream);
     FFI_HIP_TRY(hipGetLastError());
     return FFI_OK;
 }
@@ -698,6 +695,10 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         ft = FwdTopk{tc.tau, tc.tie, tc.count, tc.val, tc.idx, kTopkCap};
         lds_topk = lds + (size_t)kTileBatch * kTopkPark * sizeof(int2);
     }
+    // (whole chunks, and labels for many rounds: reads and their uses two at a time.  The kernel at 128 x 768 x 670,091 x 32, ten rounds, 186 us, one at a time 190;
+    // at 32 x 768 x 131,072 x 32, half a round, 18.8 and 17.2)
+    if (epi == kEpiScores && !topk && d.K % 32 == 0 && per_stream >= 8 * kTileThreads)
+        return launch_stream32<0, 2>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, s);
     if (epi == kEpiScores && !topk)
         return for_row_end(d.K, [&](auto last) { return launch_stream32<last>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, s); });
     int npartial = 0;
