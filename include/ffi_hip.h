@@ -204,7 +204,7 @@ int ffi_lookup_edited(const int32_t* lookup);
  *   "fwd_lane64"           -1: never the forward kernel that holds 64 samples per workgroup
  *   "plan_weights_in_lds"  -1: never / 1: whenever it fits: the input-gradient form that keeps a tile's weights in LDS
  *   "workgroups_per_cu"    n > 0: at most n workgroups per CU for the kernel that walks a tiled plan
- *   "plan_sorted_columns"  -1: never / 1: whenever the weights-in-LDS form is taken: plans that hand a tile's columns to the
+ *   "plan_sorted_columns"  -1: never / 1: whenever a tile has no more labels than threads: plans that hand a tile's columns to the
  *                          walking kernel's threads sorted by length (fewer padded slots; the sums pass through LDS after every tile)
  *   "small_path"           -1: never / 1: wherever they can: the two launches that serve small layers
  *   "dense_rows"           -1: never / 1: wherever they can: the kernels that write a label's row out over a few columns
