@@ -58,8 +58,9 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
 }
 
 // WALK: connections a unit walks; ids and sums move by quads at any alignment.  WHOLE, a fan-in of 32 or more: 32, a label's last unit taking its last
-// (those that it shares with the unit before are formed twice, to the same bits).  Else the fan-in rounded up to eight, the quads behind its last one
-// being that quad again; 4: fan-ins below four, one by one.
+// and storing only those that the unit before has not: each sum has one writer (neighbouring lanes add the samples up in unlike orders, so the sums
+// that both form differ in their last bits).  Else the fan-in rounded up to eight, the quads behind its last one being that quad again; 4: fan-ins
+// below four, one by one.
 // Units of 32 whatever the fan-in, the ids and sums of part-filled ones one by one -> so, both launches, us, at 32 samples x 768 x 131,072 and 100 x 500 x
 // 200,000: fan-in 8 22.5 -> 14.8, 80 -> 38; 16 31.7 -> 18.5, 104 -> 53; 31 46 -> 28, 139 -> 85; 32 26.6 -> 25.9, 84 -> 82; 33 51 -> 34, 173 -> 120;
 // 48 48 -> 37, 174 -> 127; 63 81 -> 38, 236 -> 130.
@@ -152,16 +153,24 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
         const long long u = u_begin + (long long)q * kResThreads + threadIdx.x;
         if (u < u_end) {
             const int j = label_of(u), k0 = first_of(u, j);
+            const int chunk = (int)(u - (long long)j * nchunks), seen = WHOLE ? chunk * kWgChunk - k0 : 0;       // (its first ones are the unit before's)
             float* grow = gw + (size_t)j * K + k0;
-            if (bias_grad != nullptr && u - (long long)j * nchunks == 0) bias_grad[j] = gsum[q];
+            if (bias_grad != nullptr && chunk == 0) bias_grad[j] = gsum[q];
             if (WALK == 4) {
 #pragma unroll
                 for (int k = 0; k < WALK; ++k)
                     if (k < K) grow[k] = res[q][k];
             } else {
 #pragma unroll
-                for (int t = 0; t < WALK / 4; ++t)
-                    *reinterpret_cast<f32x4_unaligned*>(grow + quad_at(t)) = f32x4_unaligned{res[q][4 * t], res[q][4 * t + 1], res[q][4 * t + 2], res[q][4 * t + 3]};
+                for (int t = 0; t < WALK / 4; ++t) {
+                    if (4 * t >= seen) {
+                        *reinterpret_cast<f32x4_unaligned*>(grow + quad_at(t)) = f32x4_unaligned{res[q][4 * t], res[q][4 * t + 1], res[q][4 * t + 2], res[q][4 * t + 3]};
+                    } else {
+#pragma unroll
+                        for (int k = 4 * t + 1; k < 4 * t + 4; ++k)
+                            if (k >= seen) grow[k] = res[q][k];
+                    }
+                }
             }
         }
     }

@@ -69,3 +69,34 @@ def test_gradients_of_any_fan_in(batch, features, labels, fan_in):
 @pytest.mark.parametrize("fan_in", [72, 81, 89, 95, 96])
 def test_gradients_of_three_chunks_and_many_labels(fan_in):
     test_gradients_of_any_fan_in(33, 70, 82_001, fan_in)
+
+
+# Every sum has one writer.  With features of ones the sums of a unit (32 connections of a label) are the same bits, and those of the next unit, whose
+# lane adds the samples up in another order, mostly are not: sums that another unit left show.  Labels for many workgroups, whose first units are
+# odd ones too; batch tiles shared between rows of workgroups, and not.
+@pytest.mark.parametrize("fan_in", [33, 34, 35, 36, 47, 63, 65, 67, 95, 97, 127, 128])
+@pytest.mark.parametrize("batch,features,labels", [(33, 300, 40_003), (419, 998, 2283), (31, 96, 1001)])
+def test_sums_of_the_lookup_itself_have_one_writer(batch, features, labels, fan_in):
+    ffi = load_package()
+    lib = ffi._lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(fan_in)
+    lookup = torch.randint(0, features, (labels, fan_in), generator=gen, device="cuda", dtype=torch.int32)
+    x = torch.ones((batch, features), device="cuda")
+    g = torch.randn((batch, labels), generator=gen, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.ffi_set_option(b"small_path", -1) == 0
+    try:
+        first = None
+        for _ in range(4):
+            gw = torch.full((labels, fan_in), float("nan"), device="cuda")
+            ffi._lib.check(lib.ffi_weight_grad_f32(x.data_ptr(), lookup.data_ptr(), g.data_ptr(), gw.data_ptr(), batch, features, labels, fan_in, 0, stream))
+            first = gw if first is None else first
+            assert torch.equal(gw, first)
+            for k0 in range(0, fan_in, 32):
+                unit = gw[:, k0:k0 + 32]
+                assert torch.equal(unit, unit[:, :1].expand_as(unit))
+        # (sums of `batch` terms, each rounded to 24 bits, in any order)
+        exact, magnitude = g.double().sum(0, keepdim=True).t(), g.double().abs().sum(0, keepdim=True).t()
+        assert bool(((first.double() - exact).abs() <= batch * 2.0 ** -24 * magnitude).all())
+    finally:
+        assert lib.ffi_set_option(b"small_path", 0) == 0
