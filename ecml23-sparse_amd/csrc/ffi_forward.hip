@@ -384,6 +384,26 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane32_kernel(const float* _
     }
 }
 
+// A lane's scores of W samples, one row of out each, through a resource of those rows.  The rows' offsets are formed one after the other (the caller
+// hides the stride from the compiler: hoisted, all of them do not fit the scalar registers and come back from vector lanes).
+// PAUSE: clocks between two stores.  Back to back, a wavefront's stores fill the CU's path to memory, and the wavefronts that ask for ids and
+// weights wait behind them: 16 clocks pay where many rounds of labels overlap, and cost their own time and more in a launch of few.  Forward pass of
+// plain scores with what the caches hold cold, back to back and with 16 clocks: 128 x 768 x 670,091 x 32, ten rounds, 212 and 200 us (in the
+// passes of a benchmark step 180 and 172), x 8 126 and 115, x 31 260 and 251; 512 x 1,024 x 140,000 x 32, nine rounds, 163 and 143; 128 x 768 x 300,000 x 32, under five,
+// 91 and 92, warm 82 and 88; 32 x 768 x 670,091 x 32, under three, 99 and 99, warm 56 and 57.  (Tiles of 64: 256 x 512 x 501,070 x 64 370 and
+// 384, 192 x 300 x 66,001 x 32 35.5 and 36.2, but 192 x 600 x 300,000 x 16 97 and 88; without.)
+template <int PAUSE, int W>
+__device__ __forceinline__ void store_paced(const float (&acc)[W], const buffer_rsrc& orsrc, unsigned lane_off, unsigned stride) {
+    unsigned off = 0;
+#pragma unroll
+    for (int b = 0; b < W; ++b) {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, lane_off, off, 0);
+        if constexpr (PAUSE > 0) asm volatile("s_nop %0" ::"n"(PAUSE - 1));
+        off += stride;
+    }
+}
+inline __host__ __device__ bool many_rounds(int labels_per_stream) { return labels_per_stream >= 8 * kTileThreads; }
+
 // The kernel above for plain scores, which leave as soon as they are in order: fewer registers, and a build for every way a row ends.
 template <int LAST, int GROUP>
 __global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float* __restrict__ xT, const int32_t* __restrict__ idx,
@@ -417,13 +437,10 @@ __global__ __launch_bounds__(kTileThreads) void fwd_stream32_kernel(const float*
             for (int i = 0; i < 32; ++i) acc[i] += bj;
         }
         if (valid) {
-            unsigned stride = (unsigned)L * 4u, off = 0;
-            asm volatile("" : "+s"(stride));               // (see fwd_lane64_kernel)
-#pragma unroll
-            for (int b = 0; b < 32; ++b) {
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, (unsigned)j * 4u, off, 0);
-                off += stride;
-            }
+            unsigned stride = (unsigned)L * 4u;
+            asm volatile("" : "+s"(stride));               // (see store_paced)
+            if (many_rounds(labels_per_stream)) store_paced<16>(acc, orsrc, (unsigned)j * 4u, stride);
+            else store_paced<2>(acc, orsrc, (unsigned)j * 4u, stride);
         }
     }
 }
@@ -547,14 +564,8 @@ __global__ __launch_bounds__(kTileThreads) void fwd_lane64_kernel(const float* _
         if (valid) {
             const unsigned lane_off = (unsigned)j * 4u;
             unsigned stride = (unsigned)L * 4u;
-            // (the rows' offsets are formed one after the other: all 64 do not fit the scalar registers, and came back from vector lanes)
             asm volatile("" : "+s"(stride));
-            unsigned off = 0;
-#pragma unroll
-            for (int b = 0; b < 64; ++b) {
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[b]), orsrc, lane_off, off, 0);
-                off += stride;
-            }
+            store_paced<0>(acc, orsrc, lane_off, stride);
         }
     }
 }
@@ -695,9 +706,10 @@ int forward_tiles(const float* x, const int32_t* idx, const float* w, const floa
         ft = FwdTopk{tc.tau, tc.tie, tc.count, tc.val, tc.idx, kTopkCap};
         lds_topk = lds + (size_t)kTileBatch * kTopkPark * sizeof(int2);
     }
-    // (whole chunks, and labels for many rounds: reads and their uses two at a time.  The kernel at 128 x 768 x 670,091 x 32, ten rounds, 186 us, one at a time 190;
-    // at 32 x 768 x 131,072 x 32, half a round, 18.8 and 17.2)
-    if (epi == kEpiScores && !topk && d.K % 32 == 0 && per_stream >= 8 * kTileThreads)
+    // (whole chunks, and labels for many rounds: reads and their uses two at a time.  The kernel with cold caches, two and one at a time: 128 x 768 x 670,091 x 32, ten
+    // rounds, 200 and 205 us, 512 x 1,024 x 140,000 x 32, nine, 143 and 151; 64 x 768 x 900,000 x 32, seven, 154 and 152, 64 x 768 x 670,091 x 32, five, 125
+    // and 122; 32 x 768 x 131,072 x 32, half a round, 26 and 25)
+    if (epi == kEpiScores && !topk && d.K % 32 == 0 && many_rounds(per_stream))
         return launch_stream32<0, 2>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, s);
     if (epi == kEpiScores && !topk)
         return for_row_end(d.K, [&](auto last) { return launch_stream32<last>(xT, idx, w, bias, out, d, nbt, per_stream, blocks, lds, s); });
