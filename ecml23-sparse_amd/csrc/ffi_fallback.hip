@@ -316,7 +316,6 @@ __global__ __launch_bounds__(kRedoThreads) void redo_backward_kernel(const RedoA
 constexpr int kOutIds = 32, kOutWaves = 16, kOutThreads = 64 * kOutWaves, kOutList = 256, kOutFetch = 8;
 constexpr int kOutTile = 16384;                // floats of a tile
 constexpr unsigned kOutStep = kOutIds * kOutThreads, kOutNone = ~0u;
-typedef int i32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 
 struct OutdatedWide {
     const unsigned long long* verdict;

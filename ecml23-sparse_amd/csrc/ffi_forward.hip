@@ -51,10 +51,10 @@ struct RowChunk {
     // requests reached the L2 at 128 samples x 670,091 labels x 32, so 6.5).
     template <class At>
     __device__ __forceinline__ void load(const int32_t* __restrict__ irow, const float* __restrict__ wrow, At&& at) {
-        int4 v[C / 4];
-        float4 f[C / 4];
-        static_for<C / 4>([&](auto q) { v[q] = *reinterpret_cast<const int4*>(irow + at(q)); __builtin_amdgcn_sched_barrier(0); });
-        static_for<C / 4>([&](auto q) { f[q] = *reinterpret_cast<const float4*>(wrow + at(q)); __builtin_amdgcn_sched_barrier(0); });
+        i32x4_unaligned v[C / 4];
+        f32x4_unaligned f[C / 4];
+        static_for<C / 4>([&](auto q) { v[q] = *reinterpret_cast<const i32x4_unaligned*>(irow + at(q)); __builtin_amdgcn_sched_barrier(0); });
+        static_for<C / 4>([&](auto q) { f[q] = *reinterpret_cast<const f32x4_unaligned*>(wrow + at(q)); __builtin_amdgcn_sched_barrier(0); });
 #pragma unroll
         for (int q = 0; q < C / 4; ++q) {
             idp[2 * q + 0] = (unsigned)v[q].x | ((unsigned)v[q].y << 16);

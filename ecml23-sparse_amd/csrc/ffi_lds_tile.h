@@ -36,6 +36,7 @@ __device__ __forceinline__ int xcd_contiguous_block(int block, int nblocks) {
 // element, one in flight, a tile of 768 rows took some 12 us instead of 2: all passes at 127 x 768 x 131,072 x 32 208 us, at 127 x 767 x
 // 131,072 x 4 130, at 163 x 797 x 10,774 x 4 114; 165, 87 and 82 so).
 typedef float f32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
+typedef int i32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 template <int THREADS, int INFLIGHT = 4>
 __device__ __forceinline__ void stage_rows32(float* __restrict__ xs, const float* __restrict__ src, int rows,
                                              int ld, int c0) {

@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float
                 } else if (K >= (WHOLE ? kWgChunk : 4)) {         // (always: a block of their own, or their 32 registers are wanted beside out_grad's)
 #pragma unroll
                     for (int t = 0; t < WALK / 4; ++t) {
-                        const int4 v = *reinterpret_cast<const int4*>(irow + quad_at(t));
+                        const i32x4_unaligned v = *reinterpret_cast<const i32x4_unaligned*>(irow + quad_at(t));
                         idp[2 * t + 0] = (unsigned)v.x | ((unsigned)v.y << 16);
                         idp[2 * t + 1] = (unsigned)v.z | ((unsigned)v.w << 16);
                     }
