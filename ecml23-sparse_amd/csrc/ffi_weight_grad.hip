@@ -353,7 +353,7 @@ __device__ __forceinline__ void stage_rows32_direct(float* xs, const float* __re
 
 // WALK: connections walked in a label's last chunk.  A fan-in that is not a multiple of 32 leaves that chunk partly
 // filled, and the arranged order puts the real connections first: such launches walk its first 8, 16 or 24 entries only
-// (labels of one, two or four chunks, i.e. the launches in which a thread holds whole labels).
+// (labels of one to four chunks, i.e. the launches in which a thread holds whole labels).
 template <int NCH, int UNITS, bool QUADS, int WALK = kWgChunk>
 __global__ __launch_bounds__(kResThreads) void wgrad_stream_kernel(const float* __restrict__ xT,
                                                                    const unsigned short* __restrict__ idx16,
@@ -763,7 +763,7 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
             const bool stream = form.stream;
             const size_t lds = std::max(tile_lds_bytes(d.N) + (stream ? (size_t)(kResThreads / 64) * kSliceFloats * sizeof(float) : 0),
                                         (size_t)kResThreads * kSlotPitch * sizeof(float));
-            // a label of two or four chunks: all its units in one thread (its out_grad values are loaded once per
+            // a label of two to four chunks: all its units in one thread (its out_grad values are loaded once per
             // batch tile instead of once per chunk); the work is then split by labels, not by units
             const int last_walk = form.last_walk;
 #define FFI_LAUNCH_STREAM_WALK(NCH, UNITS, WALK)                                                                                       \
@@ -791,6 +791,8 @@ int launch_weight_grad(const float* x, const int32_t* idx, const float* g, float
                         hipLaunchKernelGGL((wgrad_stream_kernel<NCH, UNITS, kQuads>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
                                            to_b, d.B, d.N, d.L, d.K, nchunks, n1, ipb, ipb2, parts);                                  \
                     }                                                                                                                  \
+                } else if constexpr (NCH == 3 || (NCH == 2 && UNITS == 2)) {                                                           \
+                    return FFI_ERR_BAD_ARGUMENT;       /* (arranged_form takes these with the slices only) */                          \
                 } else {                                                                                                               \
                     FFI_HIP_TRY(hipFuncSetAttribute((const void*)wgrad_arranged_kernel<NCH, UNITS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
                     hipLaunchKernelGGL((wgrad_arranged_kernel<NCH, UNITS>), dim3((unsigned)(n1 + n2), (unsigned)rows), dim3(kResThreads), lds, s, xT, plan->idx16, g, to_w, \
