@@ -155,15 +155,15 @@ PATH_SHAPES = [
     (160, 256, 9000, 16),      # five batch tiles, weights in LDS (fan-in below 32): three workgroups of 256 threads
     (160, 256, 9000, 32),      # five batch tiles, weights in slot order: four workgroups of 256 threads
     (288, 64, 20000, 8),       # nine batch tiles, weights in slot order: sixteen workgroups of 64 threads
-    # forward over batch tiles of 64 (N <= 608; from 192 samples, from 128 with a fan-in of 64 or more, fan-in 48 / 80 / 112):
+    # narrow inputs whose batch ends within a tile of 64 samples, and fan-ins off the chunks (too few labels for the tiles of 64, see test_gpu_forward_tiles.py):
     (256, 512, 5000, 64),      # whole tiles, vector loads
-    (200, 608, 3100, 21),      # the widest input of that path, fourth tile partly filled, odd fan-in (scalar loads)
-    (33, 40, 2100, 48),        # one sample beyond a 32-tile; three half chunks of 16
-    (193, 300, 1500, 8),       # one sample in the fourth 64-tile; fan-in below a half chunk
-    (130, 256, 2000, 72),      # fan-in with a tail of 8 behind four half chunks
-    # full chunks loaded by quads from rows that are only 4-byte aligned (fan-in no multiple of four), last chunk one by one:
+    (200, 608, 3100, 21),      # a last tile of eight samples, odd fan-in below one chunk
+    (33, 40, 2100, 48),        # one sample beyond a 32-tile; a chunk and sixteen connections
+    (193, 300, 1500, 8),       # one sample in the last tile; two quads
+    (130, 256, 2000, 72),      # two chunks and eight connections
+    # rows that are only 4-byte aligned (fan-in no multiple of four), by quads throughout:
     (64, 768, 3000, 33), (40, 512, 2000, 63), (200, 300, 1500, 35), (130, 256, 2000, 67),
-    # the 32-sample kernel's build for a fan-in below one chunk (loads by quads):
+    # the builds for a fan-in below one chunk:
     (100, 608, 3100, 24), (65, 300, 1500, 8), (128, 768, 5000, 16), (50, 1000, 700, 28), (40, 640, 900, 4),
 ]
 
@@ -183,9 +183,9 @@ def test_code_paths(ffi, shape, transposed):
     assert rel_err(gx, o_gx) <= GRAD_RTOL
 
 
-@pytest.mark.parametrize("shape", [(100, 608, 3100, 21),     # 32-sample tiles, the fourth holds 4 samples; loads one by one
-                                   (100, 608, 3100, 24),     # the same with loads by quads (fan-in below one chunk)
-                                   (200, 608, 3100, 21),     # 64-sample tiles, the fourth holds 8 samples
+@pytest.mark.parametrize("shape", [(100, 608, 3100, 21),     # the fourth tile of 32 holds 4 samples; quads and a connection behind them
+                                   (100, 608, 3100, 24),     # the same, whole quads
+                                   (200, 608, 3100, 21),     # the last tile holds 8 samples
                                    (70, 768, 2000, 32),      # 32-sample tiles, full chunks
                                    (70, 2000, 900, 32)])     # wide input
 @pytest.mark.parametrize("transposed", [False, True])
