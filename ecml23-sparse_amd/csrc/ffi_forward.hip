@@ -108,7 +108,7 @@ __device__ __forceinline__ void walk_row(const int32_t* __restrict__ irow, const
             chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
             walk_chunk<32, 0, 32, GROUP>(chunk, skewbase, acc);
         }
-        if constexpr (LAST == 32) {                        // (in two steps: the registers of one spill)
+        if constexpr (LAST == 32) {                        // (in two steps of 16: fewer registers)
             RowChunk<16> chunk;
             chunk.load(irow, wrow, [&](int q) { return k0 + 4 * q; });
             walk_chunk<32, 0, 16>(chunk, skewbase, acc);

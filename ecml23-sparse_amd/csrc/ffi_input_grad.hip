@@ -128,15 +128,15 @@ __global__ __launch_bounds__(MAXT) void igrad_tile_kernel(const unsigned short* 
     float acc[32];
 #pragma unroll
     for (int i = 0; i < 32; ++i) acc[i] = 0.f;
-    // (PERM) the sums of the thread's own column over the tiles so far; `acc` holds one tile's sums of whatever column
-    // the thread walks in it
+    // (KEEP) the sums of the thread's own column over the tiles so far; `acc` holds one tile's sums of whatever column
+    // the thread walks in it.  (PERM without KEEP) `acc` holds the sums over the tiles so far of the column walked in this one
     float home[KEEP ? 32 : 1];
 #pragma unroll
     for (int i = 0; i < (KEEP ? 32 : 1); ++i) home[i] = 0.f;
     unsigned walked = 0;                                   // (PERM) the column of the tile just walked
-    // acc -> row `walked` of the exchange; a barrier; row threadIdx.x -> home.  Called between two barriers that keep
-    // the tile's rows from being read or written meanwhile.
-    // (without KEEP: -> acc, from the row of the column that the thread walks next)
+    // acc -> row `walked` of the exchange; a barrier; then with KEEP row threadIdx.x is added to home, without it row `next`, the column that the
+    // thread walks in the next tile (at the end its own), becomes acc.  Called between two barriers that keep the tile's rows from being
+    // read or written meanwhile.
     auto hand_over = [&](unsigned next) __attribute__((always_inline)) {
         char* rowp = gs_bytes + ((size_t)walked << 7);
         const int r = lane & 7;

@@ -408,8 +408,9 @@ typedef unsigned u32x4_unaligned __attribute__((ext_vector_type(4), aligned(4)))
 typedef unsigned u32x2_unaligned __attribute__((ext_vector_type(2), aligned(2)));
 
 // How ids and weights are read: one by one; by quads, of rows of whole quads on 16-byte boundaries; by quads of any rows, the quad that a row
-// ends in being its last four connections.  Of the latter the odd fan-ins take their time, 300,000 labels of 8 samples x 768 by ones and by quads:
-// fan-in 7 16.4 and 11.0 us, 23 25 and 20.5, 33 38 and 32, but 47 52 and 61 (16 samples 34 and 32, bf16 64 and 58), 65 73 and 90 (44 and 42, 78 and 72).
+// ends in being its last four connections.  300,000 labels of 8 samples x 768 by ones and by quads: fan-in 7 17.1 and 12.0 us, 10 15.5 and 13.1, 22 23.0
+// and 20.2, 33 34.8 and 32.2, 34 35.6 and 34.0, but 38 38.8 and 42.6, 46 46.8 and 58.5, 47 48.6 and 59.5 (16 samples 34 and 32, bf16 64 and 58), 62 60 and
+// 76, 65 69 and 88 (44 and 42, 78 and 72), 126 108 and 135; with cold caches, one sample x 670,091 and four samples x 300,000 the line is the same.
 enum LdsRows { kOneByOne = 0, kQuads = 1, kAnyQuads = 2 };
 template <int GL> constexpr bool any_quads_pay(int K) { return K >= 4 && (GL >= 4 || K <= 33); }
 
