@@ -30,7 +30,7 @@ PROFILE_DIR = os.path.join(ROOT, "profiles")
 
 # GPU kernels behind each pass (one C-ABI call)
 PASS_KERNELS = {
-    "forward": "fwd_lane32_kernel",
+    "forward": "fwd_stream32_kernel",
     "weight_grad": "wgrad_stream_kernel",
     "input_grad": "igrad_permute_weights_kernel + igrad_tile_kernel + igrad_reduce_kernel",
 }
@@ -39,6 +39,16 @@ WIDE_PASS_KERNELS = {
     "weight_grad": "wgrad_wide_kernel alone, walk_columns_kernel<DOT> + weight_grads_in_place_kernel in a whole backward pass",
     "input_grad": "slices_from_*_kernel + slot_weights_kernel + walk_columns_kernel + gather_gx_kernel",
 }
+
+
+def takes_tiles_of_64(B, N, L, K, cus):
+    """The library's choice between its two forward kernels for plain scores of narrow inputs (lane64_fits in csrc/ffi_forward.hip)."""
+    tiles, rest, behind = -(-B // 64), B % 64, K % 16
+    if N > 608 or B <= 32 or behind > 4 or (behind and K < 32) or L * tiles < 768 * cus:
+        return False
+    if 0 < rest <= 32:
+        return K >= 48 and B >= 128
+    return (K >= 16 and B >= 192) or (K >= 32 and B >= 128) or (K >= 48 and behind == 0)
 
 
 def measured_traffic(config_name):
@@ -709,7 +719,7 @@ def main():
     traffic, traffic_source = measured_traffic(cfg.name)
     narrow = N <= 1216
     pass_kernels = dict(PASS_KERNELS if narrow else WIDE_PASS_KERNELS)
-    if N <= 608 and B > 32 and (B >= 192 or (K >= 64 and B >= 128) or (K > 32 and K % 32 != 0 and K % 16 == 0)):
+    if takes_tiles_of_64(B, N, L, K, torch.cuda.get_device_properties(0).multi_processor_count):
         pass_kernels["forward"] = "fwd_lane64_kernel"       # batch tiles of 64 where the [N][64] tile fits in LDS and pays
     if narrow and plan_info[0] and plan_info[1]:
         # the plan's tiles are small enough for the walking kernel to keep the tile's weights in LDS: no permutation kernel

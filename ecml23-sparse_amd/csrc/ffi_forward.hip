@@ -36,9 +36,9 @@ namespace {
 // throughout, and 20 to 100 of them spill.
 //
 // Time with the connections drained one after the other and a part-filled chunk loaded one by one -> so, us.  Plain scores at 32 x 768 x 131,072, 128 x
-// 768 x 670,091 and 100 x 1,000 x 300,000: fan-in 8 12.4 -> 11.2, 156 -> 123, 36 -> 33; 13 15.4 -> 13.0, 188 -> 151, 50 -> 42; 31 32 -> 20.5,
-// 376 -> 230, 167 -> 86; 32 20.2 -> 18.4, 191 -> 188, 81 -> 77; 40 25.2 -> 21.8, 259 -> 233, 101 -> 97; 63 44 -> 32, 590 -> 369, 240 -> 153; 64 29 -> 26,
-// 333 -> 330, 147 -> 145.  20 x 700 x 20,000, a tenth of a round of labels: 1.2 to 1.5 times as fast from fan-in 13 on.  The fused training step of 32 x
+// 768 x 670,091 and 100 x 1,000 x 300,000: fan-in 8 12.9 -> 11.9, 156 -> 121, 37 -> 33; 13 15.5 -> 13.6, 190 -> 141, 52 -> 43; 31 32 -> 22,
+// 377 -> 243, 167 -> 97; 32 20.3 -> 18.0, 193 -> 190, 81 -> 78; 40 25.2 -> 21.3, 261 -> 243, 101 -> 94; 63 44 -> 33, 588 -> 368, 239 -> 143; 64 29 -> 26,
+// 339 -> 336, 143 -> 143 (those of many rounds with the pause between stores, see store_paced).  20 x 700 x 20,000, a tenth of a round of labels: 1.2 to 1.5 times as fast from fan-in 13 on.  The fused training step of 32 x
 // 768 x 670,091: fan-in 8 79 -> 74, 31 263 -> 219, 32 171 -> 161, 63 529 -> 398; top-k of 200 x 300 x 100,000: 31 153 -> 95, 32 95 -> 90, 63 281 -> 142.
 // ------------------------------------------------------------------------------------------------
 template <int C>

@@ -63,7 +63,8 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
 // below four, one by one.
 // Units of 32 whatever the fan-in, the ids and sums of part-filled ones one by one -> so, both launches, us, at 32 samples x 768 x 131,072 and 100 x 500 x
 // 200,000: fan-in 8 22.5 -> 14.8, 80 -> 38; 16 31.7 -> 18.5, 104 -> 53; 31 46 -> 28, 139 -> 85; 32 26.6 -> 25.9, 84 -> 82; 33 51 -> 34, 173 -> 120;
-// 48 48 -> 37, 174 -> 127; 63 81 -> 38, 236 -> 130.
+// 48 48 -> 37, 174 -> 127; 63 81 -> 38, 236 -> 130 (sums shared by two units stored by both; by one of them the same: the kernel 31, 32 and 36 at 33, 48
+// and 63, where a fan-in of 32 takes 22, and 118, 117 and 126).
 template <int WALK, bool WHOLE>
 __global__ __launch_bounds__(kResThreads) void wgrad_resident_kernel(const float* __restrict__ xT,
                                                                      const int32_t* __restrict__ idx,
